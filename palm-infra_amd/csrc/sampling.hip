@@ -119,6 +119,22 @@ PALM_API int palm_apply_penalties(hipStream_t stream, float* logits, int V, cons
     return 0;
 }
 
+// ---- the uniform numbers ----------------------------------------------------------------------------
+// out[i] = hash(seed, streams[i], draws[i]) as a float32 in [0, 1), on the host, in host memory: splitmix64's finaliser three
+// times, its top 24 bits (the sampler's own uniform() says the same for one number).
+static uint64_t splitmix(uint64_t z) {
+    z += 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+PALM_API int palm_uniforms(unsigned long long seed, const uint64_t* streams, const uint64_t* draws, int n, float* out) {
+    PALM_CHECK(n >= 0 && streams && draws && out, "uniforms: n=%d", n);
+    const uint64_t of_seed = splitmix(seed);
+    for (int i = 0; i < n; ++i) out[i] = (float)(splitmix(splitmix(of_seed ^ streams[i]) ^ draws[i]) >> 40) / 16777216.0f;
+    return 0;
+}
+
 // ---- sampling -------------------------------------------------------------------------------------
 // One block of 16 waves for each row.  Wave w owns the contiguous range [w * per, (w + 1) * per) of the row and
 // walks it 64 elements at a time, a lane an element: reads are contiguous, and "index order" is the order
@@ -325,23 +341,19 @@ __device__ void write_probabilities(const float* __restrict__ row, int V, float 
     });
 }
 
-// One block per row.  out[row] = the token; probs_out (optional, [rows, V]) = the distribution drawn from.
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
-    const float* __restrict__ logits, int V, const float* __restrict__ uniforms, float temperature, int top_k,
-    float top_p, float min_p, int* __restrict__ out, float* __restrict__ probs_all) {
-    __shared__ SampleShared sh;
-    const float* row = logits + (size_t)blockIdx.x * V;
-    float* probs_out = probs_all ? probs_all + (size_t)blockIdx.x * V : nullptr;
+// One row by the whole block.  *out = the token; probs_out (optional, [V]) = the distribution drawn from.
+__device__ __forceinline__ void sample_row(const float* __restrict__ row, int V, const float* __restrict__ uniform, float temperature, int top_k,
+                                           float top_p, float min_p, int* __restrict__ out, float* __restrict__ probs_out, SampleShared& sh) {
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const BestPair best = block_argmax(row, V, sh.best);
     if (temperature <= 0.f || top_k == 1) {
         if (probs_out) for (int i = threadIdx.x; i < V; i += blockDim.x) probs_out[i] = i == best.i ? 1.f : 0.f;
-        if (threadIdx.x == 0) out[blockIdx.x] = best.i;
+        if (threadIdx.x == 0) *out = best.i;
         return;
     }
     const float l_max = best.v, inv_t = 1.0f / temperature;
     const float min_w = min_p > 0.f ? min_p : 0.f;          // w_best = exp(0) = 1
-    const float u = uniforms[blockIdx.x];
+    const float u = *uniform;
     const bool use_top_p = top_p > 0.f && top_p < 1.f;
     const Range mine = wave_range(V);
 
@@ -368,7 +380,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         }
         if (total == 0ull) {                                 // nothing has weight (a row of -inf or NaN): the first maximum
             if (probs_out) for (int i = threadIdx.x; i < V; i += blockDim.x) probs_out[i] = i == best.i ? 1.f : 0.f;
-            if (threadIdx.x == 0) out[blockIdx.x] = best.i;
+            if (threadIdx.x == 0) *out = best.i;
             return;
         }
         uint32_t tau = 0u;
@@ -503,7 +515,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                         });
                     }
                     __syncthreads();
-                    if (threadIdx.x == 0) out[blockIdx.x] = sh.result >= 0 ? sh.result : best.i;
+                    if (threadIdx.x == 0) *out = sh.result >= 0 ? sh.result : best.i;
                     return;
                 }
             }
@@ -562,7 +574,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         if (target >= total) target = total - 1ull;
         if (probs_out) write_probabilities(row, V, l_max, inv_t, min_w, tau, all, n_ties, total, sh, probs_out);
         const int tok = draw_index_order(row, V, l_max, inv_t, min_w, tau, all, n_ties, w_tau, target, sh);
-        if (threadIdx.x == 0) out[blockIdx.x] = tok >= 0 ? tok : best.i;
+        if (threadIdx.x == 0) *out = tok >= 0 ? tok : best.i;
         return;
     }
 
@@ -738,7 +750,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             cum += sh.cand_w[i];
             if (target <= cum) { pick = sh.cand_i[i]; break; }
         }
-        out[blockIdx.x] = pick;
+        *out = pick;
         sh.remaining = active;
         sh.total = sum;
     }
@@ -747,6 +759,247 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         __threadfence_block();
         for (int i = threadIdx.x; i < sh.remaining; i += blockDim.x) probs_out[sh.cand_i[i]] = sh.cand_w[i] / sh.total;
     }
+}
+
+// One block per row; probs_all (optional): [rows, V].
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
+    const float* __restrict__ logits, int V, const float* __restrict__ uniforms, float temperature, int top_k,
+    float top_p, float min_p, int* __restrict__ out, float* __restrict__ probs_all) {
+    __shared__ SampleShared sh;
+    sample_row(logits + (size_t)blockIdx.x * V, V, uniforms + blockIdx.x, temperature, top_k, top_p, min_p, out + blockIdx.x,
+               probs_all ? probs_all + (size_t)blockIdx.x * V : nullptr, sh);
+}
+
+// ---- top-k of a large vocabulary: many blocks a row -----------------------------------------------------------------
+// One block reads a row at what one compute unit gets of memory, three times over, and its counting takes turns in LDS:
+// 110 us for 151,936 logits whatever the batch.  Here the row is cut into slices of up to SLICE elements, a block each,
+// which stay in registers: a slice hands on what may belong to the row's k largest, and a second kernel (a block a row)
+// takes the exact k of the slices' candidates, sorts them and draws as sample_row does, in the same order of operations.
+// A slice's cut is the k-th largest of its threads' maxima (the least that fewer than k of them exceed): k elements of the slice are at least that large, so no element
+// below it belongs to the k; for k = 50 some 55 of 4,096 elements are not below it.  The second kernel narrows the 2,000
+// candidates of a row down the same way before it ranks what is left, each against each.  A row that does not go this way (a NaN
+// in it, a slice or a row with more candidates than there is room for: many equal logits) is done by sample_row.
+// Measured with k = 50 and 151,936 logits, both kernels: 21 us for one row (110 as one block), 26 us for 33 (117).  What is left
+// is latency: two launches, and in the second a chain of two trips to memory, five barriers and the k dependent additions.
+constexpr int SLICE_THREADS = 256;
+constexpr int SLICE_QUADS = 4;                                       // 16-byte pieces of a slice that a thread holds
+constexpr int SLICE = SLICE_THREADS * SLICE_QUADS * 4;
+constexpr int SLICE_CAP = 256;                                       // candidates that a slice can hand on
+constexpr int SLICED_TOPK_MAX = 128;                                 // half a slice's threads: the cut stays a tail of the slice
+constexpr int SLICED_MIN_VOCAB = 16384;                              // (below, the row is a few slices: one block does as well)
+constexpr int SURVIVORS = 1024;
+
+static int slices_of(int V) { return (V / 4 + SLICE / 4 - 1) / (SLICE / 4); }
+
+// how many of the 256 keys are larger
+__device__ inline int larger_keys(const uint32_t* keys, uint32_t own) {
+    int n = 0;
+    const uint4* four = reinterpret_cast<const uint4*>(keys);
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+        const uint4 q = four[j];
+        n += (q.x > own) + (q.y > own) + (q.z > own) + (q.w > own);
+    }
+    return n;
+}
+
+// counts [rows, slices]: how many candidates (-1: the row does not go this way); cands [rows, slices, SLICE_CAP]: key, index
+__global__ __launch_bounds__(SLICE_THREADS) void topk_slice_kernel(const float* __restrict__ logits, int V, int k, int* __restrict__ counts,
+                                                                   uint2* __restrict__ cands) {
+    __shared__ __attribute__((aligned(16))) uint32_t top[SLICE_THREADS];
+    __shared__ uint32_t cut;
+    __shared__ int n, bad;
+    const int slices = gridDim.x, tid = threadIdx.x;
+    const float4* row = reinterpret_cast<const float4*>(logits + (size_t)blockIdx.y * V);
+    const int per = (V / 4 + slices - 1) / slices;                   // the slices are of one length, or nearly
+    const int begin = blockIdx.x * per, end = min(V / 4, begin + per);
+    if (tid == 0) { n = 0; bad = 0; cut = 0xffffffffu; }
+    float e[SLICE_QUADS * 4];
+#pragma unroll
+    for (int u = 0; u < SLICE_QUADS; ++u) {
+        const int i = begin + u * SLICE_THREADS + tid;
+        const float4 q = i < end ? row[i] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        e[4 * u] = q.x; e[4 * u + 1] = q.y; e[4 * u + 2] = q.z; e[4 * u + 3] = q.w;
+    }
+    uint32_t best = 0u;
+    bool nan = false;
+#pragma unroll
+    for (int u = 0; u < SLICE_QUADS * 4; ++u) {
+        nan |= e[u] != e[u];
+        best = max(best, ordered_key(e[u]));
+    }
+    top[tid] = best;
+    __syncthreads();
+    if (nan) bad = 1;
+    if (larger_keys(top, best) < k) atomicMin(&cut, best);           // the k-th largest is the least of those
+    __syncthreads();
+    const uint32_t least = cut;
+    uint2* mine = cands + ((size_t)blockIdx.y * slices + blockIdx.x) * SLICE_CAP;
+    int hits = 0;
+#pragma unroll
+    for (int u = 0; u < SLICE_QUADS * 4; ++u) hits += begin + (u / 4) * SLICE_THREADS + tid < end && ordered_key(e[u]) >= least;
+    int upto = hits;                                                 // with those of the lanes before
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) { const int o = __shfl_up(upto, off, WAVE); if (tid % WAVE >= off) upto += o; }
+    int at = 0;
+    if (tid % WAVE == WAVE - 1) at = atomicAdd(&n, upto);
+    at = __shfl(at, WAVE - 1, WAVE) + upto - hits;
+    if (hits) {
+#pragma unroll
+        for (int u = 0; u < SLICE_QUADS * 4; ++u) {
+            const int i = begin + (u / 4) * SLICE_THREADS + tid;
+            const uint32_t key = ordered_key(e[u]);
+            if (i < end && key >= least) {
+                if (at < SLICE_CAP) mine[at] = make_uint2(key, 4u * i + u % 4);
+                ++at;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) counts[(size_t)blockIdx.y * slices + blockIdx.x] = bad || n > SLICE_CAP ? -1 : n;
+}
+
+struct DrawShared {
+    __attribute__((aligned(16))) uint32_t top[256];
+    uint32_t cut;
+    int n, bad, zeros;
+    uint2 survivor[SURVIVORS];
+    float v[SLICED_TOPK_MAX];
+    int i[SLICED_TOPK_MAX];
+};
+
+__global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
+    const float* __restrict__ logits, int V, const float* __restrict__ uniforms, float temperature, int k, float top_p, float min_p,
+    const int* __restrict__ counts, const uint2* __restrict__ cands, int slices, int* __restrict__ out) {
+    __shared__ union { SampleShared row; DrawShared draw; } shared;
+    DrawShared& sh = shared.draw;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    counts += (size_t)blockIdx.x * slices;
+    cands += (size_t)blockIdx.x * slices * SLICE_CAP;
+    if (tid == 0) { sh.n = 0; sh.bad = 0; sh.zeros = 0; sh.cut = 0xffffffffu; }
+    __syncthreads();
+    // the counts of the first slices a wave takes and the first places a lane takes are asked for together and kept (a place
+    // beyond its slice's count holds nothing, and nothing is made of it)
+    constexpr int HELD = 3, ROUNDS = 2;
+    int held_n[HELD];
+    uint2 held[HELD][ROUNDS];
+#pragma unroll
+    for (int h = 0; h < HELD; ++h) {
+        const int s = min(wave + h * SAMPLE_WAVES, slices - 1);
+        held_n[h] = counts[s];
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) held[h][r] = cands[(size_t)s * SLICE_CAP + lane + r * WAVE];
+    }
+#pragma unroll
+    for (int h = 0; h < HELD; ++h) {
+        if (wave + h * SAMPLE_WAVES >= slices) held_n[h] = 0;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r)
+            if (lane + r * WAVE >= held_n[h]) held[h][r] = make_uint2(0u, 0u);
+    }
+    // f(key, index) for the others: few, or a vocabulary of more than HELD x SAMPLE_WAVES slices
+    auto rest = [&](auto&& f) {
+        auto slice = [&](int s, int c, int first) {
+            if (c < 0) sh.bad = 1;
+            for (int j = first; j < c; j += WAVE) f(cands[(size_t)s * SLICE_CAP + j]);
+        };
+#pragma unroll
+        for (int h = 0; h < HELD; ++h) slice(wave + h * SAMPLE_WAVES, held_n[h], lane + ROUNDS * WAVE);
+        for (int s = wave + HELD * SAMPLE_WAVES; s < slices; s += SAMPLE_WAVES) slice(s, counts[s], lane);
+    };
+    uint32_t best = 0u;                                              // of this thread's candidates (0 is no float's key)
+#pragma unroll
+    for (int h = 0; h < HELD; ++h)
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) best = max(best, held[h][r].x);
+    rest([&](uint2 one) { best = max(best, one.x); });
+    best = max(best, (uint32_t)__shfl_xor((int)best, 1, WAVE));
+    best = max(best, (uint32_t)__shfl_xor((int)best, 2, WAVE));
+    if (tid % 4 == 0) sh.top[tid / 4] = best;
+    __syncthreads();
+    if (tid < 256 && larger_keys(sh.top, sh.top[tid]) < k) atomicMin(&sh.cut, sh.top[tid]);
+    __syncthreads();
+    const uint32_t least = max(sh.cut, 1u);
+    auto survives = [&](uint2 one) {
+        if (one.x < least) return;
+        const int at = atomicAdd(&sh.n, 1);
+        if (at < SURVIVORS) sh.survivor[at] = one;
+    };
+#pragma unroll
+    for (int h = 0; h < HELD; ++h)
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) survives(held[h][r]);
+    rest(survives);
+    __syncthreads();
+    const int n = sh.n;
+    if (sh.bad || n > SURVIVORS || n < k) {                          // (n < k: fewer than k elements in the row; not with k < V)
+        __syncthreads();
+        sample_row(logits + (size_t)blockIdx.x * V, V, uniforms + blockIdx.x, temperature, k, top_p, min_p, out + blockIdx.x, nullptr, shared.row);
+        return;
+    }
+    // the k largest by key, ties to the lower index, each to the place that its rank names
+    if (tid < n) {
+        const uint2 own = sh.survivor[tid];
+        int rank = 0;
+#pragma unroll 8
+        for (int j = 0; j < n; ++j) {
+            const uint2 o = sh.survivor[j];
+            rank += o.x > own.x || (o.x == own.x && o.y < own.y);
+        }
+        if (rank < k) {
+            sh.v[rank] = key_value(own.x);
+            sh.i[rank] = (int)own.y;
+            if (key_value(own.x) == 0.f) sh.zeros = 1;
+        }
+    }
+    __syncthreads();
+    // sorted by value, ties to the lower index: the same, but that the keys tell -0 from 0 and the values do not
+    if (sh.zeros) {
+        const float v = sh.v[min(tid, k - 1)];
+        const int i = sh.i[min(tid, k - 1)];
+        int rank = 0;
+        for (int j = 0; j < k; ++j) rank += sh.v[j] > v || (sh.v[j] == v && sh.i[j] < i);
+        __syncthreads();
+        if (tid < k) { sh.v[rank] = v; sh.i[rank] = i; }
+        __syncthreads();
+    }
+    if (wave > 0) return;
+    // sample_row's walk.  Its three sums are prefixes of one, added up in the same order: a place each, lane l of this wave
+    // holds the weights and the prefix sums l and 64 + l.
+    const float l_max = sh.v[0], inv_t = 1.0f / temperature;
+    float w[2], sum_to[2];
+    float run = 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        w[h] = lane + h * WAVE < k ? expf((sh.v[min(lane + h * WAVE, k - 1)] - l_max) * inv_t) : 0.f;
+        sum_to[h] = 0.f;
+#pragma unroll 8
+        for (int i = 0; i < min(k - h * WAVE, WAVE); ++i) {
+            run += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[h]), i));
+            if (lane == i) sum_to[h] = run;
+        }
+    }
+    // the first of the `active` places for which the flag is set, `otherwise` if there is none
+    auto first_place = [&](auto&& flag, int active, int otherwise) {
+        const unsigned long long low = __ballot(lane < active && flag(0)), high = __ballot(lane + WAVE < active && flag(1));
+        return low ? __ffsll((long long)low) - 1 : high ? WAVE + __ffsll((long long)high) - 1 : otherwise;
+    };
+    auto prefix = [&](int i) { return __shfl(i < WAVE ? sum_to[0] : sum_to[1], i % WAVE, WAVE); };
+    int active = k;
+    if (min_p > 0.f) {
+        const float threshold = min_p * __shfl(w[0], 0, WAVE);
+        active = first_place([&](int h) { return lane + h > 0 && !(w[h] >= threshold); }, k, k);
+    }
+    float sum = prefix(active - 1);
+    if (!(sum > 0.f) || !isfinite(sum)) { sum_to[0] = 1.f; active = 1; sum = 1.f; }
+    if (top_p > 0.f && top_p < 1.f) {
+        const float cutoff = top_p * sum;
+        const int last = first_place([&](int h) { return sum_to[h] >= cutoff; }, active, -1);
+        if (last >= 0) { active = last + 1; sum = prefix(last); }
+    }
+    const float target = uniforms[blockIdx.x] * sum;
+    const int pick = first_place([&](int h) { return target <= sum_to[h]; }, active, active - 1);
+    if (lane == 0) out[blockIdx.x] = sh.i[pick];
 }
 
 PALM_API int palm_sample(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms,
@@ -762,6 +1015,32 @@ PALM_API int palm_sample(hipStream_t stream, const float* logits, int n_rows, in
     if (n_rows == 0) return 0;
     sample_kernel<<<n_rows, SAMPLE_THREADS, 0, stream>>>(logits, V, uniforms, temperature, top_k, top_p, min_p, out,
                                                         probs_out);
+    PALM_LAUNCHED();
+    return 0;
+}
+
+// Whether palm_sample_sliced serves these rows: one to SLICED_TOPK_MAX candidates of a large vocabulary, rows of whole 16-byte
+// pieces; and the bytes of workspace that it needs then (0: it does not).  From SLICED_MIN_VOCAB on the slices win at any batch.
+PALM_API long long palm_sample_sliced_work(int n_rows, int V, float temperature, int top_k) {
+    if (temperature <= 0.f || top_k <= 1 || top_k > SLICED_TOPK_MAX || V < SLICED_MIN_VOCAB || V % 4 != 0 || n_rows < 1 || n_rows > 65535) return 0;
+    return (long long)n_rows * slices_of(V) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int));
+}
+
+PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, float temperature,
+                                int top_k, float top_p, float min_p, int* out, void* work, long long work_bytes) {
+    const long long needed = palm_sample_sliced_work(n_rows, V, temperature, top_k);
+    PALM_CHECK(needed > 0 && (uintptr_t)logits % 16 == 0, "sample: %d rows of %d logits with top_k = %d do not go in slices", n_rows, V, top_k);
+    PALM_CHECK(work_bytes >= needed && (uintptr_t)work % 8 == 0, "sample: %lld bytes of workspace where %lld are needed", work_bytes, needed);
+    PALM_CHECK(temperature <= 2.f, "sample: temperature must be between 0 and 2");
+    PALM_CHECK(top_p >= 0.f && top_p <= 1.f, "sample: top_p must be between 0 and 1");
+    PALM_CHECK(min_p >= 0.f && min_p <= 1.f, "sample: min_p must be between 0 and 1");
+    PALM_CHECK(uniforms, "sample: a draw needs the uniform numbers");
+    const int slices = slices_of(V);
+    uint2* cands = (uint2*)work;
+    int* counts = (int*)(cands + (size_t)n_rows * slices * SLICE_CAP);
+    topk_slice_kernel<<<dim3(slices, n_rows), SLICE_THREADS, 0, stream>>>(logits, V, top_k, counts, cands);
+    PALM_LAUNCHED();
+    topk_draw_kernel<<<n_rows, SAMPLE_THREADS, 0, stream>>>(logits, V, uniforms, temperature, top_k, top_p, min_p, counts, cands, slices, out);
     PALM_LAUNCHED();
     return 0;
 }

@@ -7,6 +7,7 @@ are memory here; the one computation that torch does on the product path is the 
 """
 from __future__ import annotations
 
+from array import array
 from ctypes import c_float, c_int, c_longlong, c_ulonglong, c_void_p
 from dataclasses import dataclass
 
@@ -49,7 +50,10 @@ _SIGNATURES = {
     "palm_linear_tile_parts": [c_int, c_int, c_int],
     "palm_argmax": [c_void_p, c_void_p, c_int, c_int, c_void_p],
     "palm_apply_penalties": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_float, c_float, c_float],
+    "palm_uniforms": [c_ulonglong, c_void_p, c_void_p, c_int, c_void_p],
     "palm_sample": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_float, c_int, c_float, c_float, c_void_p, c_void_p],
+    "palm_sample_sliced": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_float, c_int, c_float, c_float, c_void_p, c_void_p, c_longlong],
+    "palm_sample_sliced_work": [c_int, c_int, c_float, c_int],
 }
 
 _core = None
@@ -63,6 +67,7 @@ def core():
         for name, argtypes in _SIGNATURES.items():
             fn = getattr(lib, name)
             fn.argtypes, fn.restype = argtypes, c_int      # (the *_parts and *_blocks functions return a count, not a status)
+        lib.palm_sample_sliced_work.restype = c_longlong
         if lib.palm_page_tokens() != PAGE_TOKENS:
             raise KernelError(f"the kernels were built for pages of {lib.palm_page_tokens()} tokens, "
                               f"the cache uses {PAGE_TOKENS}")
@@ -326,6 +331,25 @@ def apply_penalties(logits: torch.Tensor, rows, tokens, counts, repeat_penalty: 
                  rows.shape[0], float(repeat_penalty), float(presence), float(frequency))
 
 
+def uniforms_into(out: torch.Tensor, seed: int, streams, draws) -> None:
+    """out[i], a float32 in host memory, = the uniform number of (seed, streams[i], draws[i]), as ``sampling.uniform`` makes one
+    (one by one in Python 33 of them took some 60 us, longer than the draw itself)."""
+    s, d = _u64(streams), _u64(draws)
+    _need(out.device.type == "cpu" and out.dtype == F32 and out.is_contiguous() and out.shape == (len(s),) and len(s) == len(d),
+          f"uniforms: {out.dtype} {tuple(out.shape)} on {out.device} for {len(s)} streams and {len(d)} draws")
+    library.call(core(), "palm_uniforms", int(seed) & _U64, s.buffer_info()[0], d.buffer_info()[0], len(s), out.data_ptr())
+
+
+_U64 = (1 << 64) - 1
+
+
+def _u64(numbers) -> array:
+    try:
+        return array("Q", numbers)
+    except OverflowError:                                       # below zero or beyond 64 bits: modulo 2^64
+        return array("Q", [n & _U64 for n in numbers])
+
+
 def sample(logits: torch.Tensor, uniforms: torch.Tensor | None, temperature: float, top_k: int = 0, top_p: float = 0.0,
            min_p: float = 0.0, want_probs: bool = False):
     """One token for each row.  ``uniforms`` [rows] float32 in [0, 1).  With want_probs also the
@@ -335,6 +359,13 @@ def sample(logits: torch.Tensor, uniforms: torch.Tensor | None, temperature: flo
     n, V = logits.shape
     _need(uniforms is None or (uniforms.shape == (n,) and uniforms.dtype == F32), "sample: uniforms must be float32 [rows]")
     out = torch.empty((n,), dtype=torch.int32, device=logits.device)
+    if not want_probs and uniforms is not None and logits.data_ptr() % 16 == 0:
+        needed = core().palm_sample_sliced_work(n, V, float(temperature), int(top_k))
+        if needed:
+            work = torch.empty((needed,), dtype=torch.uint8, device=logits.device)
+            library.call(core(), "palm_sample_sliced", _stream(), _p(logits), n, V, _p(uniforms), float(temperature), int(top_k),
+                         float(top_p), float(min_p), _p(out), _p(work), needed)
+            return out
     probs = torch.empty((n, V), dtype=F32, device=logits.device) if want_probs else None
     library.call(core(), "palm_sample", _stream(), _p(logits), n, V, _p(uniforms), float(temperature), int(top_k), float(top_p),
                  float(min_p), _p(out), _p(probs))

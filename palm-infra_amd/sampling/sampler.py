@@ -93,8 +93,9 @@ class DeviceSampler:
         if p.greedy:
             return ops.argmax(logits)
         # through pinned memory: the host does not wait for the device here
-        u = torch.tensor([uniform(p.seed, st.stream, st.draws) for st in states], dtype=torch.float32).pin_memory().to(
-            logits.device, non_blocking=True)
+        u = torch.empty((len(states),), dtype=torch.float32, pin_memory=True)
+        ops.uniforms_into(u, p.seed, [st.stream for st in states], [st.draws for st in states])
+        u = u.to(logits.device, non_blocking=True)
         for st in states:
             st.draws += 1
         top_k = p.top_k if 0 < p.top_k < V else 0

@@ -638,6 +638,31 @@ def test_top_k_where_the_candidates_do_not_stand_out(ops):
                 assert tok == P.draw(lg.double().numpy(), u, temperature=0.9, top_k=k), (k, u)
 
 
+@pytest.mark.parametrize("V,k", [(16384, 2), (16388, 128), (65536, 50), (151936, 1), (151936, 50), (151936, 128), (151936, 129), (151937, 50)])
+def test_top_k_in_slices_draws_what_one_block_draws(ops, V, k):
+    """Rows cut into slices against the kernel that takes a row whole (which the tests above hold to the plain sampler):
+    the same tokens, also where a row's candidates do not fit (equal logits) and in rows with NaN, infinities and both zeros."""
+    from palm_infra_amd.kernels import library
+    grid = torch.round(rand(1, V, seed=V + 1, scale=2.0) * 4) / 4
+    masked = torch.full((1, V), float("-inf"))
+    masked[0, ::V // 40] = rand(1, V, seed=V + 2)[0, ::V // 40]
+    zeros = -rand(1, V, seed=V + 3).abs() - 1.0
+    zeros[0, 5::V // 70], zeros[0, 9::V // 70] = 0.0, -0.0
+    inf, nan = rand(2, V, seed=V + 4).split(1)
+    inf, nan = inf.clone(), nan.clone()
+    inf[0, V - 2], inf[0, 7] = float("inf"), float("-inf")
+    nan[0, V // 3] = float("nan")
+    rising = torch.linspace(-8.0, 8.0, V)[None]
+    lg = torch.cat([rand(3, V, seed=V, scale=3.0), grid, masked, zeros, inf, nan, rising, rising.flip(1)]).to(DEV)
+    n = lg.shape[0]
+    for T, top_p, min_p, seed in ((0.6, 0.9, 0.0, 1), (1.0, 1.0, 0.05, 2), (1.7, 0.0, 0.0, 3)):
+        u = torch.rand(n, generator=torch.Generator().manual_seed(seed)).to(DEV)
+        u[0], u[1] = 0.0, 0.99999994
+        want = torch.empty(n, dtype=torch.int32, device=DEV)
+        library.call(ops.core(), "palm_sample", ops._stream(), lg.data_ptr(), n, V, u.data_ptr(), T, k, top_p, min_p, want.data_ptr(), None)
+        assert ops.sample(lg, u, T, k, top_p, min_p).tolist() == want.tolist(), (T, top_p, min_p)
+
+
 def test_rows_are_sampled_independently(ops):
     lg = rand(4, 2000, seed=8)
     u = torch.tensor([0.1, 0.5, 0.9, 0.3])

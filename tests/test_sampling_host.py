@@ -34,6 +34,16 @@ def test_uniform_numbers_depend_on_seed_stream_and_draw_only():
     assert 0.4 < sum(a) / len(a) < 0.6 and len(set(a)) > 190
 
 
+@pytest.mark.parametrize("seed", [0, 42, (1 << 64) - 1, (1 << 64) + 3])
+def test_a_batch_of_uniform_numbers_is_the_single_ones(seed):
+    import torch
+    from palm_infra_amd.kernels import ops
+    pairs = [(0, 0), (3, 199), (-5, 1), (1 << 63, 7), (11, (1 << 40) + 1)]
+    out = torch.empty(len(pairs))
+    ops.uniforms_into(out, seed, [s for s, _ in pairs], [d for _, d in pairs])
+    assert out.tolist() == [uniform(seed, s, d) for s, d in pairs]
+
+
 def test_history_window_counts_match_the_plain_penalties():
     hist = [4, 9, 4, 4, 2, 300, -1]
     assert penalty_counts(hist, 3, 100) == {2: 1}              # 300 and -1 are not tokens of a 100-vocabulary
