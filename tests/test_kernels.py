@@ -215,6 +215,22 @@ def test_linear_exact_result_of_a_row_does_not_depend_on_the_other_rows(ops):
         assert torch.equal(alone[0], whole[r])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (1, 4096, 4096), (16, 40, 96), (17, 100, 160), (33, 515, 1056), (81, 64, 512), (157, 1030, 4096), (300, 257, 2048)])
+def test_float32_products_on_the_matrix_cores(ops, M, N, K):
+    """Tiles' edges in every direction, waves with and without a stage of K, runs that end inside and at the end; the rows of
+    a product alone, and added to what is there."""
+    a, w, c = rand(M, K, seed=M), rand(N, K, seed=N + 1), rand(M, N, seed=K)
+    got = ops.linear_exact(a.to(DEV), w.to(DEV)).cpu()
+    # one product's rounding is 2^-24 of it; sums of K terms of unit variance are off by at most some sqrt(K) of those
+    bound = 8 * 2.0 ** -24 * K ** 0.5 * 4
+    assert (got.double() - P.linear(a, w)).abs().max() < bound
+    for r in {0, M // 2, M - 1}:
+        assert torch.equal(ops.linear_exact(a[r:r + 1].contiguous().to(DEV), w.to(DEV)).cpu()[0], got[r])
+    out = c.to(DEV)
+    ops.linear_exact(a.to(DEV), w.to(DEV), out=out, accumulate=True)
+    assert torch.equal(out.cpu(), got + c)
+
+
 def test_linear_refuses_what_does_not_fit(ops):
     from palm_infra_amd.kernels import KernelError
     with pytest.raises(KernelError, match="inner size"):
