@@ -845,7 +845,8 @@ _LATENT_SIGNATURES = {
 _RECURRENT_SIGNATURES = {
     "palm_retention": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p,
                        c_float, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
-                       c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
+                       c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int],
+    "palm_retention_matrix_chunk": [c_int, c_int, c_int],
     "palm_retention_pad": [c_int],
     "palm_joined_norm_gate": [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
 }
@@ -1043,18 +1044,22 @@ def retention(qkvg: torch.Tensor, heads: int, dim: int, vdim: int, decay: torch.
         raw = torch.empty((n, heads * vdim), dtype=F32, device=qkvg.device)
     else:
         _need(not gate_sigmoid, "retention: the per-head unit norm comes with a silu gate")
-    chunk = retention_chunk(ctx.n_seqs, heads, ctx.max_new) if chunk is None else int(chunk)
+    # runs in chunks on the matrix cores where the sizes and the rows' alignment allow, else walked over token by token
+    matrix = 0
+    if chunk is None and col0 % 8 == 0 and qkvg.shape[1] % 8 == 0 and (qkvg.data_ptr() | state.data_ptr()) % 16 == 0:
+        matrix = recurrent().palm_retention_matrix_chunk(dim, vdim, ctx.max_new)
+    chunk = matrix or (retention_chunk(ctx.n_seqs, heads, ctx.max_new) if chunk is None else int(chunk))
     # q and k after the rotation, 32-bit, in rows padded to the key size that the kernel is compiled for
     rotated = torch.empty((n, heads, 2, recurrent().palm_retention_pad(dim)), dtype=F32, device=qkvg.device)
     starts = None
     if chunk:
-        max_chunks = -(-ctx.max_new // chunk)
-        starts = torch.empty((ctx.n_seqs * max_chunks, heads, dim, vdim), dtype=F32, device=qkvg.device)
+        places = n // chunk + ctx.n_seqs if matrix else ctx.n_seqs * -(-ctx.max_new // chunk)
+        starts = torch.empty((places, heads, dim, vdim), dtype=F32, device=qkvg.device)
     g_off = col0 + 2 * heads * dim + heads * vdim
     library.call(recurrent(), "palm_retention", _stream(), _p(qkvg), _code(qkvg, "retention"), qkvg.shape[1], col0, col0 + heads * dim,
                  col0 + 2 * heads * dim, g_off, _p(cos), _p(sin), int(rot), _p(decay), float(k_scale), float(eps),
                  _p(state), _p(ctx.seq_slot), _p(ctx.seq_new), _p(ctx.cu_new), ctx.n_seqs, heads, dim, vdim, _p(out),
-                 int(ctx.max_new), chunk, _p(starts), n, _p(rotated), int(input_silu), int(raw is not None), _p(raw))
+                 int(ctx.max_new), chunk, _p(starts), n, _p(rotated), int(input_silu), int(raw is not None), _p(raw), int(bool(matrix)))
     if raw is not None:
         library.call(recurrent(), "palm_joined_norm_gate", _stream(), _p(raw), _p(joined_norm), float(eps),
                      qkvg.data_ptr() + g_off * qkvg.element_size(), _code(qkvg, "retention"), qkvg.shape[1], int(gate_sigmoid), n,

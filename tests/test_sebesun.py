@@ -281,6 +281,50 @@ def test_retention_kernel_keeps_a_far_token_and_forgets_at_its_decay(dtype):
 
 
 @gpu
+@pytest.mark.parametrize("dk,dv", [(64, 128), (64, 256), (128, 128), (128, 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_retention_in_chunks_on_the_matrix_cores(dtype, dk, dv):
+    """Runs of tokens around the borders of tiles and chunks, side by side in one step on states that hold something, against
+    the recurrence in 64 bits and against the walk token by token: outputs with the per-head norm, outputs joined, the states."""
+    from palm_infra_amd.kernels import ops
+    torch.manual_seed(dk + dv)
+    H, lengths = 3, [1, 16, 17, 64, 65, 130, 8]
+    T, width = sum(lengths), 2 * dk + 2 * dv
+    rows = (torch.randn(T, H * width + 8) * 0.5).to(dtype)
+    decay = torch.tensor([0.97, 0.9, 0.999])
+    state0 = torch.randn(len(lengths), H, dk, dv)
+    weight = torch.rand(H * dv) + 0.5
+    r64 = rows.double()[:, 8:]
+    q, k = r64[:, :H * dk].view(T, H, dk), r64[:, H * dk:2 * H * dk].view(T, H, dk) * dk ** -0.5
+    v, g = r64[:, 2 * H * dk:2 * H * dk + H * dv].view(T, H, dv), r64[:, 2 * H * dk + H * dv:]
+    o, left, at = torch.zeros(T, H, dv, dtype=P.F64), [], 0
+    for b, n in enumerate(lengths):
+        S = state0[b].double()
+        for t in range(at, at + n):
+            S = decay.double()[:, None, None] * S + k[t][:, :, None] * v[t][:, None, :]
+            o[t] = (S * q[t][:, :, None]).sum(1)
+        left.append(S)
+        at += n
+    flat = o.reshape(T, H * dv)
+    want = {"head": P.unit_rms(o, 1e-6).reshape(T, H * dv) * P.silu(g), "joined": P.unit_rms(flat, 1e-6) * weight.double() * torch.sigmoid(g)}
+    # outputs of unit scale: 32-bit sums of up to 130 * dk terms, then one rounding to the type
+    tol = 1e-4 if dtype == torch.float32 else 3e-2
+    assert ops.recurrent().palm_retention_matrix_chunk(dk, dv, max(lengths)) == 64
+    for kind in ("head", "joined"):
+        results = []
+        for chunk in (None, 0):
+            state = state0.clone().cuda()
+            ctx = _step_context([0] * len(lengths), lengths)
+            got = ops.retention(rows.cuda(), H, dk, dv, decay.cuda(), dk ** -0.5, 1e-6, state, ctx, chunk=chunk, col0=8,
+                                joined_norm=weight.cuda() if kind == "joined" else None, gate_sigmoid=kind == "joined")
+            error = (got.double().cpu() - want[kind]).abs().max()
+            assert error < tol * max(1.0, float(want[kind].abs().max())), f"{kind}, chunk {chunk}: {error}"
+            assert (state.double().cpu() - torch.stack(left)).abs().max() < 1e-4, f"{kind}, chunk {chunk}: the state"
+            results.append(got)
+        assert (results[0].float() - results[1].float()).abs().max() < tol * max(1.0, float(want[kind].abs().max()))
+
+
+@gpu
 @pytest.mark.parametrize("dk,dv", [(12, 28), (40, 72)])      # the second pair is one that the matrix-core kernel takes in bfloat16
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge(dtype, dk, dv):
