@@ -46,6 +46,9 @@ _SIGNATURES = {
     "palm_linear_mid": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int],
     "palm_linear_mid_parts": [c_int, c_int, c_int, c_int],
     "palm_linear_mid_blocks": [c_int, c_int, c_int, c_int, c_int],
+    "palm_linear_big": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_longlong],
+    "palm_linear_big_work": [c_int, c_int, c_int, c_int],
+    "palm_linear_big_takes": [c_int, c_int, c_int, c_int],
     "palm_linear_tile": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int],
     "palm_linear_tile_parts": [c_int, c_int, c_int],
     "palm_argmax": [c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -67,7 +70,7 @@ def core():
         for name, argtypes in _SIGNATURES.items():
             fn = getattr(lib, name)
             fn.argtypes, fn.restype = argtypes, c_int      # (the *_parts and *_blocks functions return a count, not a status)
-        lib.palm_sample_sliced_work.restype = c_longlong
+        lib.palm_sample_sliced_work.restype = lib.palm_linear_big_work.restype = c_longlong
         if lib.palm_page_tokens() != PAGE_TOKENS:
             raise KernelError(f"the kernels were built for pages of {lib.palm_page_tokens()} tokens, "
                               f"the cache uses {PAGE_TOKENS}")
@@ -477,6 +480,45 @@ def linear_mid(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: 
         out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=a.device)
     library.call(core(), "palm_linear_mid", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_mid out"), M, N, K,
                  1 if gated else 0, planes)
+    return out
+
+
+BIG_FROM = 320              # rows from which the kernel of large tiles may serve a product
+BIG_GATED_FROM = 500
+BIG_LONG_K = 8192
+BIG_REST = 90               # tiles
+
+
+def big_pays(M: int, N: int, K: int, gated: bool = False) -> bool:
+    """Whether a prompt's product of bfloat16 operands goes through the kernel of large tiles (linear_big.hip) instead of the
+    library.  Measured from 260 to 13,331 rows at the shapes of the named models (the kernel some 1.35 PFLOP/s where the chip is full,
+    the library 0.7 to 1.5):
+
+    gated (the activation in the kernel, against the library and the activation's pass): from 500 rows on, 0.95 to 1.40 times as
+    fast, 1.08 in the geometric mean; below 0.88 to 0.96.
+    inner sizes from 8,192 on: 0.94 to 1.97 times as fast, 1.17 in the mean (4,309 x 4,096, K = 12,288: 316 us and 623): the
+    library's choice of tile is often a poor one there.  (At 260 rows 0.81 to 1.54.)
+    other products: 0.89 to 1.40, 0.99 in the mean, so the library keeps them, but where tiles of 256 x 256 would fill the chip once
+    or more and then leave up to a third of it busy: those last tiles are cut along K here (7,000 x 7,168, K = 5,120: 372 us and
+    494; 1.08 in the mean of such sizes)."""
+    if M < (BIG_GATED_FROM if gated else BIG_FROM) or not core().palm_linear_big_takes(M, N, K, int(gated)):
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    return gated or K >= BIG_LONG_K or (tiles > COMPUTE_UNITS and 0 < tiles % COMPUTE_UNITS <= BIG_REST)
+
+
+def linear_big(a: torch.Tensor, w: torch.Tensor, gated: bool = False) -> torch.Tensor:
+    """bfloat16 a [M, K] . w [N, K]^T for a prompt's rows in tiles of up to 256 x 256; [M, N] in bfloat16, or with ``gated`` (w: gate
+    rows over up rows) silu(gate) * up, [M, N / 2]."""
+    _dev("linear_big", a, w)
+    _need(a.dtype == BF16 and w.dtype == BF16 and a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1],
+          f"linear_big: a {tuple(a.shape)} {a.dtype} and w {tuple(w.shape)} {w.dtype} (bfloat16, one inner size)")
+    M, K = a.shape
+    N = w.shape[0]
+    out = torch.empty((M, N // 2 if gated else N), dtype=BF16, device=a.device)
+    needed = core().palm_linear_big_work(M, N, K, int(gated))
+    work = torch.empty((needed,), dtype=torch.uint8, device=a.device) if needed else None
+    library.call(core(), "palm_linear_big", _stream(), _p(a), _p(w), _p(out), M, N, K, int(gated), _p(work), needed)
     return out
 
 

@@ -9,8 +9,9 @@
                                                                 rows), up to 128 rows, the kernel that shares the
                                                                 rows through LDS, a strip of weights in each wave's
                                                                 registers
-  bfloat16 x bfloat16, many rows (prompts)                      the BLAS library, as the reference's GPU path
-                                                                does for its products (engine/cuda_matmul.cu:245-260)
+  bfloat16 x bfloat16, many rows (prompts)                      the kernel of large tiles where it beats the BLAS library
+                                                                (ops.big_pays), else the library, as the reference's GPU
+                                                                path does for its products (engine/cuda_matmul.cu:245-260)
 
 A bias (none of Qwen3's projections has one) is added by a pass of its own to the product's 32-bit result, which
 then comes whole (no planes, no norm folded in) and is rounded once, after the add: correct for any part that needs
@@ -76,8 +77,16 @@ class Linear:
             if (rows <= THIN_ROWS or out_dtype != torch.bfloat16
                     or (ops.thin_serves(x, w) and ops.wide_pays(rows, self.out_features, self.in_features, planes_ok=planes_ok))):
                 return ops.linear_thin(x, w, out_dtype, planes_ok=planes_ok)
+            if self._big(x):
+                return ops.linear_big(x, w)
             return ops.linear_library(x, w)
         return ops.linear_exact(x, w, out_dtype)
+
+    def _big(self, x, gated: bool = False) -> bool:
+        """Whether the kernel of large tiles serves these rows (its reads are of 16 bytes)."""
+        return (x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and x.is_contiguous() and self.weight.is_contiguous()
+                and (x.data_ptr() | self.weight.data_ptr()) % 16 == 0
+                and ops.big_pays(x.shape[0], self.out_features, self.in_features, gated=gated))
 
     def _folds(self, rows: torch.Tensor) -> bool:
         """Whether the kernel that folds a norm into the product serves these rows."""
@@ -107,4 +116,6 @@ class Linear:
         if ops.thin_serves(x, self.weight) and (
                 x.shape[0] <= THIN_ROWS or ops.wide_pays(x.shape[0], self.out_features, self.in_features, gated=True)):
             return ops.linear_thin(x, self.weight, x.dtype, gated=True)
+        if self._big(x, gated=True):
+            return ops.linear_big(x, self.weight, gated=True)
         return ops.swiglu(self(x))

@@ -304,6 +304,31 @@ def test_linear_tile_against_the_plain_product(ops, M, N, K):
     assert torch.equal(ops.linear_thin(a.to(DEV), w.to(DEV), F32).cpu(), got32)
 
 
+# tiles of 128, 192 and 256 tokens, whole and cut along K; odd and even numbers of stages, the fewest; rows, weight rows and
+# features that end inside a tile; grids that are no multiple of the dies
+@pytest.mark.parametrize("M,N,K,gated", [
+    (1, 8, 128, False), (300, 136, 192, False), (257, 264, 320, False), (70, 1040, 1088, False), (190, 520, 4160, False), (250, 2400, 8192, False),
+    (570, 4096, 8192, False), (2500, 8200, 192, False), (4096, 4096, 192, False), (4309, 4104, 4160, False),
+    (300, 160, 192, True), (900, 160, 8192, True), (520, 4000, 2048, True), (3000, 5504, 320, True), (4096, 8192, 128, True), (4309, 8208, 4160, True)])
+def test_products_in_large_tiles_against_the_plain_product(ops, M, N, K, gated):
+    a, w = rand(M, K, seed=M + K).to(DEV), rand(N, K, seed=N, scale=K ** -0.5).to(DEV)
+    ref = a.double() @ w.double().t()
+    if gated:
+        ref = torch.nn.functional.silu(ref[:, :N // 2]) * ref[:, N // 2:]
+    got = ops.linear_big(a, w, gated=gated)
+    # exact products of bfloat16 values, added in 32-bit (K roundings of 2^-24 of sums of unit scale at most), one rounding to 8 bits
+    bound = 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * 8
+    assert got.shape == ref.shape and bool(((got.double() - ref).abs() <= bound).all()), float((got.double() - ref).abs().max())
+
+
+def test_products_in_large_tiles_refuse_what_does_not_fit(ops):
+    from palm_infra_amd.kernels import KernelError
+    for M, N, K, gated in ((300, 136, 160, False), (300, 100, 192, False), (300, 136, 192, True), (300, 136, 64, False)):
+        assert not ops.core().palm_linear_big_takes(M, N, K, int(gated)) and not ops.big_pays(M, N, K, gated)
+        with pytest.raises(KernelError, match="linear_big"):
+            ops.linear_big(rand(M, K).to(DEV), rand(N, K).to(DEV), gated=gated)
+
+
 @pytest.mark.parametrize("M", [70, 256, 300])
 @pytest.mark.parametrize("N,K,cut", [(4096, 12288, True), (4096, 4096, True), (1000, 3072, True), (24576, 4096, False),
                                      (4096, 1024, False)])
