@@ -5,15 +5,14 @@
 //             runs one after the other; place every pair in its run, in no particular order (a slot is a column of the
 //             products by itself: no result depends on where in its run a pair lies); the slots that pad a run hold -1
 //   grouped   for every tile (its expert comes from the plan): mid = silu(G_e x) * (U_e x) for the tile's rows x, then
-//             y = D_e mid.  The weights are the first operand of the matrix instruction, so that a lane ends with four
-//             neighbouring features of one row.  Sizes in whole cache lines with enough rows an expert: blocks of 128 rows x 256
-//             features through a ring of stages in LDS (moe_tile_kernel).  Otherwise a wave owns 32 features x 64 rows and reads its
-//             fragments from memory itself (a weight fragment feeds four products, a row fragment two or four)
+//             y = D_e mid.  The weights are the first operand of the matrix instruction, so that a lane ends with
+//             neighbouring features of one row.  Sizes in whole cache lines: blocks of 64 to 256 rows x 256 weight rows through
+//             LDS (moe_big_kernel).  Otherwise a wave owns 32 features x 64 rows and reads its fragments from memory itself (a
+//             weight fragment feeds four products, a row fragment two or four)
 //   combine   out[t] = sum_c weight[t, c] * y[place of pair (t, c)], in the order of c, 32-bit, plus up to two rows that other
 //             branches made
-#include "mfma.h"
+#include "big_walk.h"
 #include "expert_form.h"
-#include "lds_stage.h"
 
 constexpr int GT_TOKENS = 64;                     // rows of a tile whose fragments come from memory
 constexpr int GT_RUNS = GT_TOKENS / 16;           // runs of 16 rows: what one matrix instruction takes
@@ -35,7 +34,7 @@ __device__ inline bf16x8 grouped_row8(const bf16_t* row, int col, int dim) {
 __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int* __restrict__ chosen, const int* __restrict__ ids, int vocab, int top,
                                                                 int n_pairs, int experts, int max_tiles, int tile,
                                                                 int* __restrict__ tile_expert, int* __restrict__ slot_pair,
-                                                                int* __restrict__ pair_slot) {
+                                                                int* __restrict__ pair_slot, int* __restrict__ used) {
     __shared__ int start_s[PLAN_MAX_EXPERTS + 1], cursor_s[PLAN_MAX_EXPERTS];
     const int lane = threadIdx.x % WAVE;
     auto choice = [&](int p) { return ids ? chosen[(size_t)min(max(ids[p / top], 0), vocab - 1) * top + p % top] : chosen[p]; };
@@ -65,7 +64,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int* __res
             if (e < experts) start_s[e] = at;
             at += padded[i];
         }
-        if (lane == WAVE - 1) start_s[experts] = up_to;
+        if (lane == WAVE - 1) {
+            start_s[experts] = up_to;
+            *used = up_to / tile;
+        }
     }
     __syncthreads();
     for (int i = threadIdx.x; i < max_tiles; i += PLAN_THREADS) tile_expert[i] = -1;
@@ -163,137 +165,59 @@ __global__ __launch_bounds__(GT_WAVES * WAVE) void moe_grouped_kernel(const bf16
         }
 }
 
-// The same products with both operands crossing LDS.  A block of eight waves owns TILE_ROWS slots x TILE_W_ROWS rows of an
-// expert's matrix and walks over K in stages of 64 (a row of a stage is one cache line of 128 bytes), the stages in a ring
-// that global_load_lds fills; a row's eight 16-byte chunks are permuted by the row's number so that an operand's reads spread
-// over the banks (the lane that fills a place fetches the chunk that belongs there).  MFMA 32x32x16: 32 weight rows x 32 slots, a wave
-// owns 64 weight rows x 64 slots.  Gated forms: of every 64 weight rows of a tile the first 32 are gate rows and the others
-// their up rows.  FORM as above.  The tiles of an expert that lies in the plan follow each other, features innermost, and each
-// die gets a run of neighbouring tiles.
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-constexpr int TILE_ROWS = 128, TILE_W_ROWS = 256, TILE_K = 64, TILE_WAVES = 8, TILE_WAVES_F = 4;
-constexpr int TILE_LINE = TILE_K * 2, TILE_CHUNKS = TILE_LINE / 16, TILE_RING = 3;
-constexpr int TILE_STAGE = (TILE_ROWS + TILE_W_ROWS) * TILE_LINE;
-constexpr int TILE_LOADS = TILE_STAGE / 1024 / TILE_WAVES;            // instructions a wave and stage
-constexpr int TILE_DIES = 8;
-
-template <int FORM>
-__global__ __launch_bounds__(TILE_WAVES * WAVE) void moe_tile_kernel(const bf16_t* __restrict__ a, const int* __restrict__ slot_pair, int top,
-                                                                     const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
-                                                                     int max_tiles, int feature_tiles, int n_features, int k_dim,
-                                                                     ExpertCap cap, bf16_t* __restrict__ out) {
+// The same products in tiles of 64 NT slots x 256 weight rows through the walk of a prompt's plain products (big_walk.h; gated
+// forms: of every 128 weight rows the first 64 are gate rows and the others their up rows).  FORM as above.
+//
+// What bounds it up to some 200 rows an expert is the weights' way from memory (32 experts of 2,048 x 4,096, 352 rows of four
+// choices: 1.07 GB in 212 us with the plan and the sum, 5 TB/s), from there on the number of stages.  So
+//   - the tiles in use, not as many as there could be, are shared out evenly over the dies (each gets a run of neighbouring
+//     tiles, features innermost: an expert's weights and a tile's rows are read into one L2); by the number there could be,
+//     three of eight dies stood idle at 852 rows
+//   - an expert's features begin their walk at stages of their own: rows lie 4 or 8 KB apart, and blocks that walk in step ask
+//     all for the same few of memory's channels (352 rows: 288 us in step, 234 so, tiles of 128 rows)
+//   - the tile is as high as an expert's rows need, as long as that spares another tile (see big_tile_of).
+// Us with plan and sum, squared relu, rows of four choices over 32 experts: 130 rows 484 -> 211 (fragments from memory before),
+// 352: 347 -> 212, 852: 372 -> 262, 2,048: 590 -> 440 (a ring of three stages of 32 x 32 x 16 instructions before).
+template <int NT, int FORM>
+__global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_big_kernel(
+    const bf16_t* __restrict__ a, const int* __restrict__ slot_pair, int top, const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
+    const int* __restrict__ used, int feature_tiles, int n_features, int k_dim, ExpertCap cap, bf16_t* __restrict__ out) {
     constexpr bool GATED = FORM == 1 || FORM == 3;
-    constexpr int TILE_FEATURES = GATED ? TILE_W_ROWS / 2 : TILE_W_ROWS;
-    __shared__ __attribute__((aligned(1024))) char lds[TILE_RING * TILE_STAGE];
-    const int total = max_tiles * feature_tiles, per_die = (total + TILE_DIES - 1) / TILE_DIES;
-    const int pid = (blockIdx.x % TILE_DIES) * per_die + blockIdx.x / TILE_DIES;
-    if (pid >= total) return;
-    const int tile = pid / feature_tiles, f0 = pid % feature_tiles * TILE_FEATURES;
-    const int e = tile_expert[tile];
-    if (e < 0) return;
-    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int wave_f = wave % TILE_WAVES_F, wave_t = wave / TILE_WAVES_F;
-    const bf16_t* we = w + (size_t)e * (GATED ? 2 : 1) * n_features * k_dim;
-
-    // the rows this lane brings in: instruction q of this wave fills the stage's rows (q * 8 + wave) * 8 .. + 7, weights first
-    const char* src[TILE_LOADS];
+    __shared__ __attribute__((aligned(1024))) char lds[2 * (BIG_FEAT + 64 * NT) * BIG_ROW];
+    const int total = *used * feature_tiles, per_die = (total + BIG_DIES - 1) / BIG_DIES;
+    const int pid = (blockIdx.x % BIG_DIES) * per_die + blockIdx.x / BIG_DIES;
+    if ((int)blockIdx.x / BIG_DIES >= per_die || pid >= total) return;
+    const int tile = pid / feature_tiles, ft = pid % feature_tiles;
+    const int e = __builtin_amdgcn_readfirstlane(tile_expert[tile]);
+    const int stages = k_dim / BIG_K;
+    f32x4 acc[8][NT];
+    big_walk<NT, true>(lds, a, w + (size_t)e * (GATED ? 2 : 1) * n_features * k_dim, (uint32_t)(k_dim * 2), stages, (5 * e + 2 * ft) % stages,
+                       [&](int row) {
+                           const int slot = tile * 64 * NT + row;
+                           return slot_pair ? max(slot_pair[slot], 0) / top : slot;      // a slot that pads the run reads row 0; nobody reads its result
+                       },
+                       [&](int row) {
+                           return GATED ? (row & 64 ? n_features : 0) + min(ft * 128 + row / 128 * 64 + row % 64, n_features - 1)
+                                        : min(ft * 256 + row, n_features - 1);
+                       },
+                       acc);
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, wave_f = wave % 2, wave_t = wave / 2;
 #pragma unroll
-    for (int q = 0; q < TILE_LOADS; ++q) {
-        const int R = (q * TILE_WAVES + wave) * 8 + lane / TILE_CHUNKS;
-        const int chunk = (lane % TILE_CHUNKS) ^ ((R >> 1) & (TILE_CHUNKS - 1));
-        const bf16_t* row;
-        if (R < TILE_W_ROWS) {
-            const int f = GATED ? f0 + R / 64 * 32 + R % 32 : f0 + R;
-            row = we + ((size_t)min(f, n_features - 1) + (GATED && R / 32 % 2 ? n_features : 0)) * k_dim;
-        } else {
-            const int slot = tile * TILE_ROWS + R - TILE_W_ROWS;
-            // a slot that pads the run reads row 0; nobody reads its result
-            row = a + (size_t)(slot_pair ? max(slot_pair[slot], 0) / top : slot) * k_dim;
-        }
-        src[q] = reinterpret_cast<const char*>(row) + chunk * 16;
-    }
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds);
-    auto bring = [&](int kt, int place) {
+    for (int t = 0; t < NT; ++t) {
+        bf16_t* row = out + ((size_t)tile * 64 * NT + wave_t * 16 * NT + 16 * t + lane % 16) * n_features;
 #pragma unroll
-        for (int q = 0; q < TILE_LOADS; ++q)
-            row_chunk_into_lds(src[q] + (size_t)kt * TILE_LINE, lds0 + place * TILE_STAGE + (q * TILE_WAVES + wave) * 1024);
-    };
-    int w_off[2], x_off[2], cs[TILE_K / 16];
+        for (int half = 0; half < (GATED ? 1 : 2); ++half) {
+            float v[16];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        w_off[i] = (wave_f * 64 + i * 32 + lane % 32) * TILE_LINE;
-        x_off[i] = (TILE_W_ROWS + wave_t * 64 + i * 32 + lane % 32) * TILE_LINE;
-    }
-#pragma unroll
-    for (int s = 0; s < TILE_K / 16; ++s) cs[s] = ((2 * s + lane / 32) ^ ((lane >> 1) & (TILE_CHUNKS - 1))) * 16;
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[f][t][v] = 0.f;
-
-    const int stages = k_dim / TILE_K;
-    constexpr int AHEAD = TILE_RING - 1;
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i)
-        if (i < stages) bring(i, i);
-    int place = 0;
-    for (int kt = 0; kt < stages; ++kt) {
-        if (kt + AHEAD <= stages) all_but_the_youngest_have_arrived<(AHEAD - 1) * TILE_LOADS>();
-        else all_but_the_youngest_have_arrived<0>();
-        __syncthreads();                                       // every wave's share of the stage; and everyone is done with the one before
-        if (kt + AHEAD < stages) bring(kt + AHEAD, place == 0 ? TILE_RING - 1 : place - 1);
-        const char* stage = lds + place * TILE_STAGE;
-        bf16x8 wf[2][2], xf[2][2];
-        auto read_operands = [&](int s) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                wf[s & 1][i] = *reinterpret_cast<const bf16x8*>(stage + w_off[i] + cs[s]);
-                xf[s & 1][i] = *reinterpret_cast<const bf16x8*>(stage + x_off[i] + cs[s]);
-            }
-        };
-        read_operands(0);
-#pragma unroll
-        for (int s = 0; s < TILE_K / 16; ++s) {
-            if (s + 1 < TILE_K / 16) read_operands(s + 1);
-#pragma unroll
-            for (int f = 0; f < 2; ++f)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    acc[f][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s & 1][f], xf[s & 1][t], acc[f][t], 0, 0, 0);
-            if (s + 1 < TILE_K / 16) {
+            for (int f = 0; f < 4; ++f)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // one matrix instruction
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // one LDS read
+                    const float z = acc[4 * half + f][t][i];
+                    v[4 * f + i] = FORM == 1 ? expert_silu_gated(z, acc[4 + f][t][i]) : FORM == 3 ? expert_capped(z, acc[4 + f][t][i], cap)
+                                   : FORM == 2 ? expert_gelu(z) : FORM == 4 ? expert_relu_squared(z) : z;
                 }
-            }
+            big_store(row, (GATED ? ft * 128 + wave_f * 64 : ft * 256 + wave_f * 128 + half * 64) + 16 * (lane / 16), n_features, v);
         }
-        place = place + 1 == TILE_RING ? 0 : place + 1;
-    }
-
-    // element v of a result tile: slot lane % 32, weight row 8 (v / 4) + 4 (lane / 32) + v % 4
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const size_t slot = (size_t)tile * TILE_ROWS + wave_t * 64 + t * 32 + lane % 32;
-#pragma unroll
-        for (int f = 0; f < (GATED ? 1 : 2); ++f)
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const int feat = f0 + (GATED ? wave_f * 32 : wave_f * 64 + f * 32) + 8 * q4 + 4 * (lane / 32);
-                if (feat >= n_features) continue;              // n_features is a multiple of four
-                bf16_t v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float z = acc[f][t][4 * q4 + i];
-                    v[i] = f32_to_bf16(FORM == 1 ? expert_silu_gated(z, acc[1][t][4 * q4 + i]) : FORM == 3 ? expert_capped(z, acc[1][t][4 * q4 + i], cap)
-                                       : FORM == 2 ? expert_gelu(z) : FORM == 4 ? expert_relu_squared(z) : z);
-                }
-                *reinterpret_cast<uint2*>(out + slot * n_features + feat) = make_uint2((uint32_t)v[0].bits | ((uint32_t)v[1].bits << 16),
-                                                                                       (uint32_t)v[2].bits | ((uint32_t)v[3].bits << 16));
-            }
     }
 }
 
@@ -320,17 +244,38 @@ __global__ void moe_combine_kernel(const bf16_t* __restrict__ y, const int* __re
     }
 }
 
-// Rows of a tile: the kernel whose operands cross LDS takes sizes in whole lines and pays from some 40 rows an expert on.
-static int tile_of(long long n_pairs, int experts, int width, int ff) {
-    return width % TILE_K == 0 && ff % TILE_K == 0 && n_pairs >= 40ll * experts ? TILE_ROWS : GT_TOKENS;
+// Rows of a tile for experts with n_pairs / experts rows each: what takes the fewest stages' time (0.75, 0.87, 1.13 and 1.42 us
+// for 64 to 256 rows, a full chip) for an expert with somewhat more rows than the mean, a second tile for a few experts costing
+// almost a whole round.  Measured, us, 32 experts of 2,048 x 4,096, tiles of 64 / 128 / 192 / 256 rows: mean 25: 212 / 230 / 272 /
+// 317, 75: 288 / 231 / 244 / 275, 106: - / 308 / 262 / 312, 187: - / 363 / 378 / 303, 256: - / 484 / 440 / 454, 625: 1,247 / 909 /
+// 849 / 831.
+static int big_tile_of(long long n_pairs, int experts) {
+    const double mean = (double)n_pairs / experts, rows = mean + 2.25 * sqrt(mean);
+    const double stage_us[4] = {0.75, 0.87, 1.13, 1.42};
+    int best = 64;
+    double best_cost = 1e300;
+    for (int nt = 1; nt <= 4; ++nt) {
+        const double cost = ceil(rows / (64 * nt)) * stage_us[nt - 1];
+        if (cost < best_cost) { best_cost = cost; best = 64 * nt; }
+    }
+    return best;
 }
-PALM_API int palm_moe_tile_tokens(int n_pairs, int experts, int width, int ff) { return tile_of(n_pairs, experts, width, ff); }
+// Whether the tiles cross LDS: rows in whole stages that start on 16 bytes, offsets from a matrix's first row of 32 bits.
+static bool big_tiles(long long n_pairs, int experts, int width, int ff, bool aligned) {
+    const long long rows = n_pairs + 256ll * (experts + 1), inner = max(width, ff);
+    return aligned && width % BIG_K == 0 && ff % BIG_K == 0 && rows * inner < (1ll << 31) && 2ll * ff * width < (1ll << 31);
+}
+static int tile_of(long long n_pairs, int experts, int width, int ff, bool aligned) {
+    return big_tiles(n_pairs, experts, width, ff, aligned) ? big_tile_of(n_pairs, experts) : GT_TOKENS;
+}
+// aligned: h, gate_up and down start on 16 bytes
+PALM_API int palm_moe_tile_tokens(int n_pairs, int experts, int width, int ff, int aligned) { return tile_of(n_pairs, experts, width, ff, aligned != 0); }
 
 // chosen, weight [n, top]; h bfloat16 [n, width]; gate_up bfloat16 [experts, 2 ff, width] (the plain forms: [experts, ff, width], up
 // rows alone); add0, add1: null or bfloat16 rows [n, width]; down bfloat16 [experts, width, ff].
 // With ids [n] chosen is a table [vocab, top] of which every token takes its id's row, and weight may be null (1 / top).
-// Room, with tile = palm_moe_tile_tokens(n top, experts, width, ff), max_tiles = ceil(n top / tile) + experts and slots = max_tiles * tile: plan: (max_tiles + slots
-// + n top) ints; mid: slots * ff bfloat16; y: slots * width bfloat16.  out float32 [n, width].
+// Room, with tile = palm_moe_tile_tokens(n top, experts, width, ff, aligned), max_tiles = ceil(n top / tile) + experts and
+// slots = max_tiles * tile: plan: (max_tiles + slots + n top + 1) ints; mid: slots * ff bfloat16; y: slots * width bfloat16.  out float32 [n, width].
 PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gate_up, const void* down, const int* chosen,
                               const float* weight, int n_tokens, int top, int experts, int width, int ff, int* plan, void* mid, void* y,
                               float* out, int form, float limit, float slope, float shift, const void* add0, const void* add1,
@@ -346,28 +291,36 @@ PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gat
     if (n_tokens == 0) return 0;
     const long long n_pairs = (long long)n_tokens * top;
     PALM_CHECK(n_pairs < (1ll << 30), "moe_grouped: %lld pairs are more than one launch takes", n_pairs);
-    const int tile = tile_of(n_pairs, experts, width, ff);
+    const bool aligned = ((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down) % 16 == 0, big = big_tiles(n_pairs, experts, width, ff, aligned);
+    const int tile = tile_of(n_pairs, experts, width, ff, aligned);
     const int max_tiles = (int)((n_pairs + tile - 1) / tile) + experts;
     int* tile_expert = plan;
     int* slot_pair = tile_expert + max_tiles;
     int* pair_slot = slot_pair + (size_t)max_tiles * tile;
-    moe_plan_kernel<<<1, PLAN_THREADS, 0, stream>>>(chosen, ids, vocab, top, (int)n_pairs, experts, max_tiles, tile, tile_expert, slot_pair, pair_slot);
+    int* used = pair_slot + n_pairs;
+    moe_plan_kernel<<<1, PLAN_THREADS, 0, stream>>>(chosen, ids, vocab, top, (int)n_pairs, experts, max_tiles, tile, tile_expert, slot_pair, pair_slot, used);
     const int combine_threads = width >= 2048 ? 256 : 128;
     const ExpertCap cap{limit, slope, shift};
-    if (tile == TILE_ROWS) {
-        auto blocks = [&](int feature_tiles) { return dim3((max_tiles * feature_tiles + TILE_DIES - 1) / TILE_DIES * TILE_DIES); };
-        const int up_features = expert_is_gated(form) ? TILE_W_ROWS / 2 : TILE_W_ROWS;
-        const int up_tiles = (ff + up_features - 1) / up_features, down_tiles = (width + TILE_W_ROWS - 1) / TILE_W_ROWS;
+    if (big) {
+        auto blocks = [&](int feature_tiles) { return dim3((max_tiles * feature_tiles + BIG_DIES - 1) / BIG_DIES * BIG_DIES); };
+        const int up_features = expert_is_gated(form) ? BIG_FEAT / 2 : BIG_FEAT;
+        const int up_tiles = (ff + up_features - 1) / up_features, down_tiles = (width + BIG_FEAT - 1) / BIG_FEAT;
         PALM_CHECK((long long)max_tiles * max(up_tiles, down_tiles) < (1ll << 30), "moe_grouped: %d tiles of rows are more than one launch takes", max_tiles);
-#define MOE_TILE_UP(FORM) moe_tile_kernel<FORM><<<blocks(up_tiles), TILE_WAVES * WAVE, 0, stream>>>((const bf16_t*)h, slot_pair, top, \
-            (const bf16_t*)gate_up, tile_expert, max_tiles, up_tiles, ff, width, cap, (bf16_t*)mid)
-        if (form == EXPERT_GATED_SILU) MOE_TILE_UP(1);
-        else if (form == EXPERT_GELU) MOE_TILE_UP(2);
-        else if (form == EXPERT_CAPPED) MOE_TILE_UP(3);
-        else MOE_TILE_UP(4);
-#undef MOE_TILE_UP
-        moe_tile_kernel<0><<<blocks(down_tiles), TILE_WAVES * WAVE, 0, stream>>>((const bf16_t*)mid, nullptr, top, (const bf16_t*)down, tile_expert,
-                                                                                 max_tiles, down_tiles, width, ff, cap, (bf16_t*)y);
+#define MOE_BIG_UP(NT, FORM) moe_big_kernel<NT, FORM><<<blocks(up_tiles), BIG_THREADS, 0, stream>>>((const bf16_t*)h, slot_pair, top, \
+            (const bf16_t*)gate_up, tile_expert, used, up_tiles, ff, width, cap, (bf16_t*)mid)
+#define MOE_BIG(NT) { \
+        if (form == EXPERT_GATED_SILU) MOE_BIG_UP(NT, 1); \
+        else if (form == EXPERT_GELU) MOE_BIG_UP(NT, 2); \
+        else if (form == EXPERT_CAPPED) MOE_BIG_UP(NT, 3); \
+        else MOE_BIG_UP(NT, 4); \
+        moe_big_kernel<NT, 0><<<blocks(down_tiles), BIG_THREADS, 0, stream>>>((const bf16_t*)mid, nullptr, top, (const bf16_t*)down, tile_expert, \
+                                                                              used, down_tiles, width, ff, cap, (bf16_t*)y); }
+        if (tile == 64) MOE_BIG(1)
+        else if (tile == 128) MOE_BIG(2)
+        else if (tile == 192) MOE_BIG(3)
+        else MOE_BIG(4)
+#undef MOE_BIG
+#undef MOE_BIG_UP
         moe_combine_kernel<<<n_tokens, combine_threads, 0, stream>>>((const bf16_t*)y, pair_slot, weight, top, width, (const bf16_t*)add0, (const bf16_t*)add1, out);
         PALM_LAUNCHED();
         return 0;

@@ -910,7 +910,7 @@ _FEEDFORWARD_SIGNATURES = {
                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "palm_moe_few_planes": [c_int],
     "palm_moe_route_table": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p],
-    "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int],
+    "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int, c_int],
     "palm_moe_grouped": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                          c_void_p, c_void_p, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int],
     "palm_gather_rows": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
@@ -1978,10 +1978,11 @@ def moe_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chos
     top = chosen.shape[1]
     experts = _check_experts(what, h, gate_up, down, chosen, weight, ff, form, ids, None)[0]
     _need(moe_grouped_serves(h, gate_up, ff) and down.dtype == BF16, f"{what}: bfloat16 rows and weights, sizes in multiples of eight")
-    tile = feedforward().palm_moe_tile_tokens(n * top, experts, width, ff)
+    aligned = (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0
+    tile = feedforward().palm_moe_tile_tokens(n * top, experts, width, ff, aligned)
     max_tiles = (n * top + tile - 1) // tile + experts
     slots = max_tiles * tile
-    plan = torch.empty((max_tiles + slots + n * top,), dtype=torch.int32, device=h.device)
+    plan = torch.empty((max_tiles + slots + n * top + 1,), dtype=torch.int32, device=h.device)
     mid = torch.empty((slots, ff), dtype=BF16, device=h.device)
     y = torch.empty((slots, width), dtype=BF16, device=h.device)
     out = torch.empty((n, width), dtype=F32, device=h.device)

@@ -69,6 +69,25 @@ def test_grouped_products(form, E, top, W, F, n, uneven):
 
 
 @gpu
+@pytest.mark.parametrize("form", ["gated_silu", "relu_squared"])
+@pytest.mark.parametrize("E,top,W,F,n,uneven", [(7, 3, 64, 128, 1, False), (4, 1, 1088, 64, 129, True), (3, 1, 192, 320, 200, False), (2, 2, 640, 576, 97, False),
+                                                (2, 1, 128, 704, 290, True), (2, 1, 256, 64, 430, False)])
+def test_grouped_tiles(form, E, top, W, F, n, uneven):
+    """Tiles of 64 to 256 rows, with one stage and many, part tiles of features and of rows, and rows that start on no 16 bytes
+    (which take the fragments' kernel): 32-bit sums of the same products, one rounding of the inner rows and one of the experts'."""
+    from palm_infra_amd.kernels import ops
+    h, up, down, chosen, weight = case(form, E, top, W, F, n, uneven, E * n + F, torch.bfloat16)
+    want = plain_mixture(form, h, up, down, chosen, weight, F)
+    tol = 0.02 * float(want.abs().max())
+    args = [t.cuda() for t in (h, up, down, chosen, weight)]
+    first = ops.moe_grouped(*args, F, form)
+    assert float((first.cpu().double() - want).abs().max()) <= tol
+    assert torch.equal(ops.moe_grouped(*args, F, form), first)
+    odd = torch.empty(n * W + 1, dtype=torch.bfloat16, device="cuda")[1:].view(n, W).copy_(args[0])
+    assert float((ops.moe_grouped(odd, *args[1:], F, form).cpu().double() - want).abs().max()) <= tol
+
+
+@gpu
 @pytest.mark.parametrize("form", ["gated_silu", "gelu", "capped_gated", "relu_squared"])
 @pytest.mark.parametrize("E,top,W,F,shared", [(4, 2, 64, 64, 40), (3, 1, 72, 24, None), (33, 4, 320, 264, 264), (5, 5, 8, 8, 16), (512, 3, 48, 16, None), (6, 2, 2056, 520, 1032)])
 def test_few_rows(form, E, top, W, F, shared):
