@@ -1968,6 +1968,18 @@ def moe_grouped_serves(h: torch.Tensor, gate_up: torch.Tensor, ff: int) -> bool:
     return h.dtype == BF16 and gate_up.dtype == BF16 and h.shape[1] % 8 == 0 and ff % 8 == 0
 
 
+# Above so many rows the grouped products' tiles of 64 rows are faster than the kernels for few rows, shared expert and all: a
+# layer of 32 experts of 2,048 x 4,096, four a row, and a shared one of twice the size, 16 rows 226 us by the kernels for few
+# rows, 190 + 33 by the grouped ones and the plain products; 32 rows 318 and 206 + 33, 64: 392, 206 + 35, 128: 587, 207 + 38.
+GROUPED_FROM = 16
+
+
+def moe_grouped_pays(h: torch.Tensor, gate_up: torch.Tensor, ff: int) -> bool:
+    """Whether a step's rows go through the grouped products although the kernels for few rows would take them: enough rows, and
+    sizes in whole stages, so that the matrices come through LDS."""
+    return h.shape[0] > GROUPED_FROM and moe_grouped_serves(h, gate_up, ff) and h.shape[1] % 64 == 0 and ff % 64 == 0
+
+
 def moe_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor | None, ff: int,
                 form: str = "gated_silu", cap=NO_CAP, add=(), ids: torch.Tensor | None = None) -> torch.Tensor:
     """Every row through its chosen experts, for many rows, planned on the device: the (row, choice) pairs grouped by expert,

@@ -140,6 +140,10 @@ class RoutedExperts:
         z = self.expert_first[e](xs)
         return ops.capped_gate(z, *self.cap) if self.form == "capped_gated" else ops.activation(z, ops.PLAIN_EXPERTS[self.form])
 
+    def takes_few(self, h):
+        """Whether the kernels for few rows take these: up to DIRECT_ROWS, unless the grouped products are the better ones."""
+        return h.shape[0] <= self.DIRECT_ROWS and not ops.moe_grouped_pays(h, self.first, self.inter)
+
     def run_few(self, h, chosen, weight, add=(), ids=None, shared=None, planes_ok=False):
         """``run_experts`` for at most DIRECT_ROWS rows, planned nowhere: the matrix cores, or the kernels that each (row, choice)
         reads its expert in.  ``ids``, ``shared``: see ``ops.moe_experts``; ``planes_ok``: float32 planes may come back."""
@@ -151,7 +155,7 @@ class RoutedExperts:
     def run_experts(self, h, chosen, weight, add=()):
         """float32 [n, hidden]: sum_c weight[t, c] * expert chosen[t, c] of h[t], plus the rows ``add`` (up to two)."""
         top = chosen.shape[1]
-        if h.shape[0] <= self.DIRECT_ROWS:
+        if self.takes_few(h):
             return self.run_few(h, chosen, weight, add)
         if ops.moe_grouped_serves(h, self.first, self.inter):
             return ops.moe_grouped(h, self.first, self.down_all, chosen, weight, self.inter, self.form, self.cap, add)
@@ -306,13 +310,14 @@ class RoutedTableFeedForward(RoutedExperts):
     def _run(self, h, ctx, planes_ok):
         n, shared = h.shape[0], tuple(s.weight for s in self.shared) if self.shared is not None else None
         # in a step of few rows the shared expert rides in the experts' own kernels
-        rides = shared is not None and n <= self.DIRECT_ROWS and (
+        few = self.takes_few(h)
+        rides = shared is not None and few and (
             ops.moe_few_serves(h, self.first, self.inter, self.experts, self.top, shared) or (n <= self.SHARED_DIRECT_ROWS and self.shared_fits))
         add = []
         if shared is not None and not rides:
             up, down = self.shared
             add.append(down(ops.activation(up(h), ops.PLAIN_EXPERTS[self.form])))
-        if n <= self.DIRECT_ROWS:
+        if few:
             return self.run_few(h, self.table, None, add, ids=ctx.token_ids, shared=shared if rides else None, planes_ok=planes_ok)
         if ops.moe_grouped_serves(h, self.first, self.inter):
             return ops.moe_grouped(h, self.first, self.down_all, self.table, None, self.inter, self.form, self.cap, add, ids=ctx.token_ids)

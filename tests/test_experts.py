@@ -118,3 +118,10 @@ def test_few_rows(form, E, top, W, F, shared):
         y = [torch.randn(n, W).to(torch.bfloat16).cuda() for _ in range(2)]
         more = ops.moe_few(*args, F, form, cap, add=y, shared=extra)
         assert torch.allclose(more, got + y[0].float() + y[1].float(), atol=1e-3, rtol=1e-4)
+
+
+def test_which_steps_go_through_the_grouped_products():
+    from palm_infra_amd.kernels import ops
+    pays = lambda n, W, F, dt=torch.bfloat16: ops.moe_grouped_pays(torch.empty(n, W, dtype=dt), torch.empty(F, W, dtype=dt), F)
+    assert pays(17, 64, 128) and pays(128, 4096, 64)
+    assert not pays(16, 64, 128) and not pays(17, 72, 128) and not pays(17, 64, 40) and not pays(17, 64, 128, torch.float32)
