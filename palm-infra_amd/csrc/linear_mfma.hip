@@ -327,7 +327,7 @@ static int stream_steps(int n_super, int parts) {
     return (per_part + nw - 1) / nw;
 }
 
-// The steps the kernel variants make for a wish of `steps`: 2, 4, 6 or 8 with the activations in registers
+// The steps the kernel variants make for a wish of `steps` (linear_ring.hip's the odd ones too): 2, 4, 6 or 8 with the activations in registers
 // (K up to 8192), else a multiple of 4 with the activations read beside the weights, which for more than a few
 // rows is much the slower way (2 against 5 TB/s at 16 rows).
 constexpr int STREAM_MAX_REG_STEPS = 8;
