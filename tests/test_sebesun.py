@@ -217,6 +217,48 @@ def test_stream_kernel_norms_adds_and_averages_over_depth(W):
 
 
 @gpu
+@pytest.mark.parametrize("W,J", [(4096, 0), (4096, 4), (4100, 5), (8192, 8), (12288, 7), (16384, 1)])
+def test_averages_over_many_planes(W, J):
+    """One to four groups of four a thread, and planes that fill the reads under way together or leave some over."""
+    from palm_infra_amd.kernels import ops
+    torch.manual_seed(W + J)
+    n = 3
+    x, y, w = torch.randn(n, W, device="cuda"), torch.randn(n, W, device="cuda") * 3, torch.rand(W, device="cuda") + 0.5
+    results, mix = torch.randn(J + 2, n, W, device="cuda"), torch.randn(J + 1, device="cuda")
+    summed = x.double() + P.rms_norm(y.double(), w.double(), 1e-5)
+    want = sum((mix[j].double() * results[j].double() for j in range(J)), mix[J].double() * summed)
+    xs, rs = x.clone(), results.clone()
+    h = ops.add_normed(xs, y, w, 1e-5, torch.bfloat16, results=rs, mix=mix)
+    assert torch.allclose(xs.double(), want, atol=1e-5) and torch.allclose(rs[J].double(), summed, atol=1e-5)
+    assert torch.equal(rs[J + 1], results[J + 1]) and torch.equal(rs[:J], results[:J]) and torch.equal(h, xs.bfloat16())
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [2, 3, 4, 5])
+@pytest.mark.parametrize("lens,C,wide", [([16], 64, 64), ([1, 15, 47], 1028, 2060), ([33, 2, 130], 260, 264), ([40, 3], 66, 66), ([20, 16], 64, 67)])
+def test_causal_conv_in_runs_is_the_convolution_token_by_token(dtype, taps, lens, C, wide):
+    """Runs of tokens a thread, their remainders, and the sizes that go a token a thread: bit for bit the steps of one token each."""
+    from palm_infra_amd.kernels import ops
+    from palm_infra_amd.parts import make_context
+    torch.manual_seed(taps * C + wide)
+    x = torch.randn(sum(lens), wide, device="cuda").to(dtype)
+    w, bias = torch.randn(C, taps, device="cuda"), torch.randn(C, device="cuda") if C % 64 == 0 else None
+    before = torch.randn(len(lens), taps - 1, C, device="cuda")
+    slots = list(range(len(lens)))[::-1]
+    state = before.clone()
+    got = ops.causal_conv(x, C, w, bias, state, make_context(slots, [0] * len(lens), [[0] * n for n in lens], dtype, "cuda"))
+    ends = [sum(lens[:b + 1]) for b in range(len(lens))]
+    for b, n in enumerate(lens):
+        one = before.clone()
+        ctx = make_context([slots[b]], [0], [[0]], dtype, "cuda")
+        for t in range(n):
+            row = ends[b] - n + t
+            assert torch.equal(ops.causal_conv(x[row:row + 1], C, w, bias, one, ctx)[0], got[row]), (b, t)
+        assert torch.equal(one[slots[b]], state[slots[b]])
+
+
+@gpu
 def test_xielu_on_both_sides_of_zero():
     from palm_infra_amd.kernels import ops
     z = torch.linspace(-12, 12, 1001, device="cuda")
