@@ -142,6 +142,12 @@ PALM_API int palm_causal_conv(hipStream_t stream, const void* x, int dtype, int 
 //   scan   for every token a lane updates its states from LDS and the group adds up its part of y with shuffles;
 //          nothing but the multiply-add on S waits for the token before it, so the exponentials of a tile overlap
 //   out    all threads add the skip term, gate with silu(z_t) and store the tile's outputs row by row
+// Up to 16 states the next tile's inputs are asked for before the scan and wait in registers (with more states a thread has more of
+// them to hold, and fewer blocks fit: 64 states, many sequences, 10 to 20 % slower).  A part tile goes token by token: unrolled, it
+// costs the registers of another wave a SIMD.  What bounds it is the vector unit (some 30 instructions a token and state) and, once
+// the short sequences are done, the chain of tiles.  8,192 channels x 16 states, us, before (each tile's inputs waited for, the
+// library's exponential, three barriers a tile) and now: 2,603 tokens 580 and 415, 717 + 572 + 1,314 405 and 335, 8 x 300 264 and
+// 235, one token each of 64 sequences 51 and 41.
 constexpr int SCAN_TILE = 16;
 
 // Sum over groups of G consecutive lanes (G a power of two), every lane gets its group's sum.  Within a row of 16
@@ -160,6 +166,24 @@ template <int G> __device__ inline float group_sum(float y) {
     if constexpr (G >= 64) y += __shfl_xor(y, 32, WAVE);
     return y;
 }
+// exp(dt A) for an A that stays: 2^(dt A log2 e) with the product's rounding and that of A log2 e made up for in first order, so that
+// the error is the exponential unit's own and not that of a rounded argument.  Below 2^-150: 0, as any 32-bit exponential.
+struct ScanDecay {
+    float hi, lo;                                       // A log2 e and, times ln 2, what hi leaves of it
+    __device__ static ScanDecay of(float a) {
+        constexpr float LOG2E = 1.44269504f, LOG2E_REST = 1.92596299e-8f, LN2 = 0.693147181f;
+        a = fmaxf(a, -1e30f);                           // (finite: an A beyond the range is forgotten at once all the same)
+        ScanDecay d;
+        d.hi = a * LOG2E;
+        d.lo = (fmaf(a, LOG2E, -d.hi) + a * LOG2E_REST) * LN2;
+        return d;
+    }
+    __device__ float over(float dt) const {
+        constexpr float LN2 = 0.693147181f;
+        const float p = dt * hi, rest = fmaf(fmaf(dt, hi, -p), LN2, dt * lo), e = __builtin_amdgcn_exp2f(p);
+        return p < -150.f ? 0.f : fmaf(e, rest, e);
+    }
+};
 constexpr int SCAN_WAVES = 4;
 constexpr int SCAN_THREADS = SCAN_WAVES * WAVE;
 
@@ -169,8 +193,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     const float* __restrict__ dtl, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
     const float* __restrict__ d_skip, float* __restrict__ state, const int* __restrict__ seq_slot,
     const int* __restrict__ seq_new, const int* __restrict__ cu_new, int channels, int n_state, T* __restrict__ out) {
+    constexpr bool AHEAD = G <= 16;
     constexpr int CH = SCAN_THREADS / G;               // channels of a block
     constexpr int NP = G * PER;                        // the state size, padded
+    constexpr int NB = (SCAN_TILE * NP + SCAN_THREADS - 1) / SCAN_THREADS, NC = (SCAN_TILE * CH + SCAN_THREADS - 1) / SCAN_THREADS;
     __shared__ float b_s[SCAN_TILE][NP], c_s[SCAN_TILE][NP];
     __shared__ float dt_s[SCAN_TILE][CH], u_s[SCAN_TILE][CH], y_s[SCAN_TILE][CH];
     const int j = threadIdx.x % G, ch = threadIdx.x / G;
@@ -181,36 +207,73 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     const int n_new = seq_new[b];
     const size_t row0 = (size_t)cu_new[b];
     float* sp = state + ((size_t)seq_slot[b] * channels + cc) * n_state;
-    float S[PER], A[PER];
+    float S[PER];
+    ScanDecay A[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int n = j + k * G;
         S[k] = n < n_state ? sp[n] : 0.f;
-        A[k] = n < n_state ? -expf(a_log[(size_t)cc * n_state + n]) : 0.f;
+        A[k] = ScanDecay::of(n < n_state ? -expf(a_log[(size_t)cc * n_state + n]) : 0.f);
     }
+    // this thread's elements of a tile: idx = threadIdx + i SCAN_THREADS is token idx / NP (idx / CH), state (channel) the rest
+    T b_r[NB], c_r[NB], u_r[NC], z_r[NC];              // (as they lie in memory: a conversion would wait for each)
+    float dt_r[NC], skip[NC], bias[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int idx = threadIdx.x + i * SCAN_THREADS, ck = min(c0 + idx % CH, channels - 1);
+        skip[i] = bias[i] = 0.f;
+        if (idx / CH >= n_new) continue;
+        skip[i] = d_skip[ck];
+        bias[i] = dt_bias[ck];
+    }
+    auto ask = [&](int t0) {                           // (tokens beyond the sequence are not read and not used)
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int idx = threadIdx.x + i * SCAN_THREADS, n = idx % NP;
+            b_r[i] = c_r[i] = T{};
+            if (n >= n_state || t0 + idx / NP >= n_new) continue;
+            const T* r = bc + (row0 + t0 + idx / NP) * bc_stride;
+            b_r[i] = r[b_off + n];
+            c_r[i] = r[c_off + n];
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int idx = threadIdx.x + i * SCAN_THREADS, ck = min(c0 + idx % CH, channels - 1);
+            dt_r[i] = 0.f;
+            u_r[i] = z_r[i] = T{};
+            if (t0 + idx / CH >= n_new) continue;
+            const size_t row = row0 + t0 + idx / CH;
+            dt_r[i] = dtl[row * channels + ck];
+            u_r[i] = u[row * channels + ck];
+            z_r[i] = z[row * z_stride + ck];
+        }
+    };
+    if (AHEAD) ask(0);
     for (int t0 = 0; t0 < n_new; t0 += SCAN_TILE) {
         const int tt = min(SCAN_TILE, n_new - t0);
-        for (int idx = threadIdx.x; idx < tt * NP; idx += SCAN_THREADS) {
-            const int ti = idx / NP, n = idx % NP;
-            const T* r = bc + (row0 + t0 + ti) * bc_stride;
-            b_s[ti][n] = n < n_state ? to_float(r[b_off + n]) : 0.f;
-            c_s[ti][n] = n < n_state ? to_float(r[c_off + n]) : 0.f;
+        if (!AHEAD) ask(t0);
+        float u_t[NC], z_t[NC];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int idx = threadIdx.x + i * SCAN_THREADS;
+            if (idx / NP < tt) { b_s[idx / NP][idx % NP] = to_float(b_r[i]); c_s[idx / NP][idx % NP] = to_float(c_r[i]); }
         }
-        for (int idx = threadIdx.x; idx < tt * CH; idx += SCAN_THREADS) {
-            const int ti = idx / CH, k = idx % CH;
-            const int ck = min(c0 + k, channels - 1);
-            const size_t row = row0 + t0 + ti;
-            dt_s[ti][k] = softplus_dt(dtl[row * channels + ck] + dt_bias[ck]);
-            u_s[ti][k] = to_float(u[row * channels + ck]);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int idx = threadIdx.x + i * SCAN_THREADS;
+            if (idx / CH < tt) { dt_s[idx / CH][idx % CH] = softplus_dt(dt_r[i] + bias[i]); u_s[idx / CH][idx % CH] = to_float(u_r[i]); }
+            u_t[i] = to_float(u_r[i]);
+            z_t[i] = to_float(z_r[i]);
         }
         __syncthreads();
+        if (AHEAD && t0 + SCAN_TILE < n_new) ask(t0 + SCAN_TILE);        // on their way while this tile is scanned
 #define SCAN_TOKEN(ti) { \
             const float dt = dt_s[ti][ch]; \
             const float du = dt * u_s[ti][ch]; \
             float y = 0.f; \
             _Pragma("unroll") for (int k = 0; k < PER; ++k) { \
                 const int n = j + k * G; \
-                S[k] = fmaf(expf(dt * A[k]), S[k], du * b_s[ti][n]);        /* beyond the state size A, B and C are zero */ \
+                S[k] = fmaf(A[k].over(dt), S[k], du * b_s[ti][n]);          /* beyond the state size A, B and C are zero */ \
                 y = fmaf(S[k], c_s[ti][n], y); \
             } \
             y = group_sum<G>(y); \
@@ -219,21 +282,20 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 #pragma unroll
             for (int ti = 0; ti < SCAN_TILE; ++ti) SCAN_TOKEN(ti)
         } else {
-#pragma unroll
-            for (int ti = 0; ti < SCAN_TILE; ++ti)
-                if (ti < tt) SCAN_TOKEN(ti)
+#pragma unroll 1
+            for (int ti = 0; ti < tt; ++ti) SCAN_TOKEN(ti)
         }
 #undef SCAN_TOKEN
         __syncthreads();
-        for (int idx = threadIdx.x; idx < tt * CH; idx += SCAN_THREADS) {
-            const int ti = idx / CH, k = idx % CH;
-            if (c0 + k < channels) {
-                const size_t row = row0 + t0 + ti;
-                const float y = fmaf(d_skip[c0 + k], u_s[ti][k], y_s[ti][k]);
-                out[row * channels + c0 + k] = from_float<T>(y * silu_f(to_float(z[row * z_stride + c0 + k])));
+        // the next tile's elements may go to LDS while these are read: y_s is written behind the next barrier only
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int idx = threadIdx.x + i * SCAN_THREADS, ti = idx / CH, k = idx % CH;
+            if (ti < tt && c0 + k < channels) {
+                const float y = fmaf(skip[i], u_t[i], y_s[ti][k]);
+                out[(row0 + t0 + ti) * channels + c0 + k] = from_float<T>(y * silu_f(z_t[i]));
             }
         }
-        __syncthreads();
     }
     if (mine && n_new > 0) {
 #pragma unroll
