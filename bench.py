@@ -216,8 +216,8 @@ def kernel_table(engine, cfg, slots, batch: int, context: int) -> dict:
 
 def prefill_kernel_table(engine, cfg, tokens: int) -> dict:
     """The prompt step's dominant kernels one by one at `tokens` rows, as kernel_table does it: the four products
-    of a layer (the library's), the prompt attention, the norm with the residual add and the gated activation;
-    flops (or bytes) each has to do, the time of one launch and the fraction of the peak that makes."""
+    of a layer (as the parts choose their kernels; gate and up without the activation), the prompt attention, the norm
+    with the residual add and the gated activation; flops (or bytes) each has to do, the time of one launch and the fraction of the peak that makes."""
     import torch
     from palm_infra_amd.engine import StepEntry
     from palm_infra_amd.kernels import ops

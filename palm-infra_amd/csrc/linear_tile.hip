@@ -1,9 +1,7 @@
 // C[M, N] = X[M, K] . W[N, K]^T for many rows: bfloat16 operands on the matrix cores, 32-bit accumulation.  The
 // product is the reference's matmul (kernels/matmul_dense.cpp:939-953), which its GPU path hands to a library
-// (engine/cuda_matmul.cu:245-260), and so does this engine for a prompt's products.  This kernel is here for what
-// that library call cannot give: a float32 result from bfloat16 operands, the logits at many places of a prompt.
-// (It once had epilogues that applied the gated activation or added the product to the residual stream; for many
-// rows the library's kernel with a pass of its own after it was the faster way, and they are gone.)
+// (engine/cuda_matmul.cu:245-260).  This kernel is here for float32 results from bfloat16 operands, the logits at
+// many places of a prompt; a prompt's bfloat16 products are linear_big.hip's or the library's.
 //
 // Tiling.  A block of eight waves owns TOK tokens x FEAT features and walks over K (or, with K cut into ranges, over
 // its range) in stages of 64.  A stage of both operands lies in LDS as rows of 128 bytes (64 k-values: a whole
@@ -16,9 +14,8 @@
 // What bounds it: a compute unit reads at most some 45 GB/s of what its die's L2 does not hold (measured with the
 // products and the LDS reads taken out, through registers or straight into LDS, with one, two or three stages in
 // flight; a long prompt's operands are far larger than L2), 11 to 12 TB/s for the chip; a tile of 256 x 256 needs 128 KB for every 64 k-values, which is 270 us for the gate/up product of
-// 2,048 rows, about what the library's kernel of the same tile takes in all.  This kernel overlaps its products
-// and its reads less well (360 us), so prompts keep the library; it serves where a library call cannot: float32
-// results of many rows (logits at many places).
+// 2,048 rows.  This kernel overlaps its products and its reads less well (360 us; linear_big.hip's waves, half a
+// step apart, do better, with bfloat16 results); it serves float32 results of many rows (logits at many places).
 // MFMA 32x32x16: the A operand is 32 weight rows (features), the B operand 32 activation rows (tokens); a lane
 // of the result holds one token and 16 features in runs of four, so results leave as 8-byte (bfloat16) or
 // 16-byte (float32) pieces of a token's row.

@@ -3,7 +3,7 @@
 Every function checks on the host what its kernel assumes (device, element types, contiguity, shapes
 that fit each other) before it launches anything, and launches on torch's current stream.  Tensors
 are memory here; the one computation that torch does on the product path is the library matrix product of
-``linear_library`` (bfloat16 products of more rows than the kernels here stream weights past).
+``linear_library`` (bfloat16 products of more rows than the kernels here stream weights past, where ``big_pays`` says no).
 """
 from __future__ import annotations
 
