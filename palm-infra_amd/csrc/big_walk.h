@@ -51,6 +51,17 @@ __device__ __forceinline__ void big_store(bf16_t* __restrict__ row, int at, int 
     }
 }
 
+__device__ __forceinline__ void big_store(float* __restrict__ row, int at, int width, const float (&v)[16]) {
+    if (at + 16 <= width) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) *reinterpret_cast<float4*>(row + at + 4 * h) = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (at + i < width) row[at + i] = v[i];
+    }
+}
+
 // x, w: the matrices' first rows and first column of the walk; x_row(i), w_row(i): the rows that are row i of the tile (of 64 NT
 // and of 256); row_bytes from row to row in both.  acc[4 half + f][t][v], lane (r, g) of wave (wave_f, wave_t): token
 // wave_t * 16 NT + 16 t + r, tile row 128 wave_f + 64 half + 16 g + 4 f + v.  TURNED: the walk begins at stage `turn` and wraps.

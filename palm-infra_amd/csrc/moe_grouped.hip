@@ -10,7 +10,8 @@
 //             LDS (moe_big_kernel).  Otherwise a wave owns 32 features x 64 rows and reads its fragments from memory itself (a
 //             weight fragment feeds four products, a row fragment two or four)
 //   combine   out[t] = sum_c weight[t, c] * y[place of pair (t, c)], in the order of c, 32-bit, plus up to two rows that other
-//             branches made
+//             branches made and float32 planes of another (a shared expert's).  y is bfloat16, or float32 where the caller asks
+//             for results that are rounded nowhere before the sum, as those of the kernels for few rows are
 #include "big_walk.h"
 #include "expert_form.h"
 
@@ -178,10 +179,10 @@ __global__ __launch_bounds__(GT_WAVES * WAVE) void moe_grouped_kernel(const bf16
 //   - the tile is as high as an expert's rows need, as long as that spares another tile (see big_tile_of).
 // Us with plan and sum, squared relu, rows of four choices over 32 experts: 130 rows 484 -> 211 (fragments from memory before),
 // 352: 347 -> 212, 852: 372 -> 262, 2,048: 590 -> 440 (a ring of three stages of 32 x 32 x 16 instructions before).
-template <int NT, int FORM>
+template <int NT, int FORM, typename TO>
 __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_big_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ slot_pair, int top, const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
-    const int* __restrict__ used, int feature_tiles, int n_features, int k_dim, ExpertCap cap, bf16_t* __restrict__ out) {
+    const int* __restrict__ used, int feature_tiles, int n_features, int k_dim, ExpertCap cap, TO* __restrict__ out) {
     constexpr bool GATED = FORM == 1 || FORM == 3;
     __shared__ __attribute__((aligned(1024))) char lds[2 * (BIG_FEAT + 64 * NT) * BIG_ROW];
     const int total = *used * feature_tiles, per_die = (total + BIG_DIES - 1) / BIG_DIES;
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
     big_walk<NT, true>(lds, a, w + (size_t)e * (GATED ? 2 : 1) * n_features * k_dim, (uint32_t)(k_dim * 2), stages, (5 * e + 2 * ft) % stages,
                        [&](int row) {
                            const int slot = tile * 64 * NT + row;
-                           return slot_pair ? max(slot_pair[slot], 0) / top : slot;      // a slot that pads the run reads row 0; nobody reads its result
+                           return FORM == 0 ? slot : max(slot_pair[slot], 0) / top;      // a slot that pads the run reads row 0; nobody reads its result
                        },
                        [&](int row) {
                            return GATED ? (row & 64 ? n_features : 0) + min(ft * 128 + row / 128 * 64 + row % 64, n_features - 1)
@@ -204,7 +205,9 @@ __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, wave_f = wave % 2, wave_t = wave / 2;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        bf16_t* row = out + ((size_t)tile * 64 * NT + wave_t * 16 * NT + 16 * t + lane % 16) * n_features;
+        const int slot = tile * 64 * NT + wave_t * 16 * NT + 16 * t + lane % 16;
+        if (sizeof(TO) == 4 && slot_pair[slot] < 0) continue;          // (few rows: most of a tile pads its run)
+        TO* row = out + (size_t)slot * n_features;
 #pragma unroll
         for (int half = 0; half < (GATED ? 1 : 2); ++half) {
             float v[16];
@@ -221,24 +224,39 @@ __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
     }
 }
 
+__device__ inline void combine_load8(const bf16_t* p, float (&v)[8]) {
+    const bf16x8 q = load_bf16x8(p);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (float)q[i];
+}
+__device__ inline void combine_load8(const float* p, float (&v)[8]) {
+    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
 // One block per token; eight neighbouring columns a thread (width is a multiple of eight).  weight: null, or [n, top] (null: 1 / top).
-__global__ void moe_combine_kernel(const bf16_t* __restrict__ y, const int* __restrict__ pair_slot, const float* __restrict__ weight, int top,
-                                   int width, const bf16_t* __restrict__ add0, const bf16_t* __restrict__ add1, float* __restrict__ out) {
+// planes: n_planes float32 [n, width] to be added.
+template <typename TY>
+__global__ void moe_combine_kernel(const TY* __restrict__ y, const int* __restrict__ pair_slot, const float* __restrict__ weight, int top,
+                                   int width, const bf16_t* __restrict__ add0, const bf16_t* __restrict__ add1, const float* __restrict__ planes,
+                                   int n_planes, float* __restrict__ out) {
     const size_t t = blockIdx.x;
     for (int d = threadIdx.x * 8; d < width; d += blockDim.x * 8) {
         float total[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) total[i] = 0.f;
-        auto add = [&](const bf16_t* row, float f) {
-            const bf16x8 v = load_bf16x8(row + d);
+        auto add = [&](const auto* row, float f) {
+            float v[8];
+            combine_load8(row + d, v);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) total[i] = fmaf(f, (float)v[i], total[i]);
+            for (int i = 0; i < 8; ++i) total[i] = fmaf(f, v[i], total[i]);
         };
 #pragma unroll 4
         for (int c = 0; c < top; ++c)
             add(y + (size_t)pair_slot[t * top + c] * width, weight ? weight[t * top + c] : 1.0f / (float)top);
         if (add0) add(add0 + t * width, 1.0f);
         if (add1) add(add1 + t * width, 1.0f);
+        for (int p = 0; p < n_planes; ++p) add(planes + ((size_t)p * gridDim.x + t) * width, 1.0f);
         *reinterpret_cast<float4*>(out + t * width + d) = make_float4(total[0], total[1], total[2], total[3]);
         *reinterpret_cast<float4*>(out + t * width + d + 4) = make_float4(total[4], total[5], total[6], total[7]);
     }
@@ -275,11 +293,15 @@ PALM_API int palm_moe_tile_tokens(int n_pairs, int experts, int width, int ff, i
 // rows alone); add0, add1: null or bfloat16 rows [n, width]; down bfloat16 [experts, width, ff].
 // With ids [n] chosen is a table [vocab, top] of which every token takes its id's row, and weight may be null (1 / top).
 // Room, with tile = palm_moe_tile_tokens(n top, experts, width, ff, aligned), max_tiles = ceil(n top / tile) + experts and
-// slots = max_tiles * tile: plan: (max_tiles + slots + n top + 1) ints; mid: slots * ff bfloat16; y: slots * width bfloat16.  out float32 [n, width].
+// slots = max_tiles * tile: plan: (max_tiles + slots + n top + 1) ints; mid: slots * ff bfloat16; y: slots * width, bfloat16 or with y32
+// (for tiles that cross LDS) float32.  planes: n_planes float32 rows [n, width] to add.  out float32 [n, width].
+PALM_API int palm_moe_grouped_in_tiles(long long n_pairs, int experts, int width, int ff, int aligned) {
+    return experts <= PLAN_MAX_EXPERTS && big_tiles(n_pairs, experts, width, ff, aligned != 0);
+}
 PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gate_up, const void* down, const int* chosen,
                               const float* weight, int n_tokens, int top, int experts, int width, int ff, int* plan, void* mid, void* y,
                               float* out, int form, float limit, float slope, float shift, const void* add0, const void* add1,
-                              const int* ids, int vocab) {
+                              const int* ids, int vocab, int y32, const float* planes, int n_planes) {
     PALM_CHECK(ids ? vocab > 0 : weight != nullptr, "moe_grouped: choices come with weights, or from a table of %d ids", vocab);
     PALM_CHECK(experts <= PLAN_MAX_EXPERTS, "moe_grouped: %d experts exceed %d", experts, PLAN_MAX_EXPERTS);
     PALM_CHECK(form >= EXPERT_GATED_SILU && form <= EXPERT_RELU_SQUARED, "moe_grouped: form %d is neither gated silu (0) nor plain gelu (1) nor capped "
@@ -292,6 +314,8 @@ PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gat
     const long long n_pairs = (long long)n_tokens * top;
     PALM_CHECK(n_pairs < (1ll << 30), "moe_grouped: %lld pairs are more than one launch takes", n_pairs);
     const bool aligned = ((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down) % 16 == 0, big = big_tiles(n_pairs, experts, width, ff, aligned);
+    PALM_CHECK(big || !y32, "moe_grouped: 32-bit results come from tiles that cross LDS (sizes of whole stages, rows that start on 16 bytes)");
+    PALM_CHECK(n_planes == 0 || (n_planes > 0 && planes && (uintptr_t)planes % 16 == 0), "moe_grouped: %d planes to add", n_planes);
     const int tile = tile_of(n_pairs, experts, width, ff, aligned);
     const int max_tiles = (int)((n_pairs + tile - 1) / tile) + experts;
     int* tile_expert = plan;
@@ -300,28 +324,32 @@ PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gat
     int* used = pair_slot + n_pairs;
     moe_plan_kernel<<<1, PLAN_THREADS, 0, stream>>>(chosen, ids, vocab, top, (int)n_pairs, experts, max_tiles, tile, tile_expert, slot_pair, pair_slot, used);
     const int combine_threads = width >= 2048 ? 256 : 128;
+#define MOE_COMBINE(TY) moe_combine_kernel<TY><<<n_tokens, combine_threads, 0, stream>>>((const TY*)y, pair_slot, weight, top, width, \
+        (const bf16_t*)add0, (const bf16_t*)add1, planes, n_planes, out)
     const ExpertCap cap{limit, slope, shift};
     if (big) {
         auto blocks = [&](int feature_tiles) { return dim3((max_tiles * feature_tiles + BIG_DIES - 1) / BIG_DIES * BIG_DIES); };
         const int up_features = expert_is_gated(form) ? BIG_FEAT / 2 : BIG_FEAT;
         const int up_tiles = (ff + up_features - 1) / up_features, down_tiles = (width + BIG_FEAT - 1) / BIG_FEAT;
         PALM_CHECK((long long)max_tiles * max(up_tiles, down_tiles) < (1ll << 30), "moe_grouped: %d tiles of rows are more than one launch takes", max_tiles);
-#define MOE_BIG_UP(NT, FORM) moe_big_kernel<NT, FORM><<<blocks(up_tiles), BIG_THREADS, 0, stream>>>((const bf16_t*)h, slot_pair, top, \
+#define MOE_BIG_UP(NT, FORM) moe_big_kernel<NT, FORM, bf16_t><<<blocks(up_tiles), BIG_THREADS, 0, stream>>>((const bf16_t*)h, slot_pair, top, \
             (const bf16_t*)gate_up, tile_expert, used, up_tiles, ff, width, cap, (bf16_t*)mid)
 #define MOE_BIG(NT) { \
         if (form == EXPERT_GATED_SILU) MOE_BIG_UP(NT, 1); \
         else if (form == EXPERT_GELU) MOE_BIG_UP(NT, 2); \
         else if (form == EXPERT_CAPPED) MOE_BIG_UP(NT, 3); \
         else MOE_BIG_UP(NT, 4); \
-        moe_big_kernel<NT, 0><<<blocks(down_tiles), BIG_THREADS, 0, stream>>>((const bf16_t*)mid, nullptr, top, (const bf16_t*)down, tile_expert, \
-                                                                              used, down_tiles, width, ff, cap, (bf16_t*)y); }
+        if (y32) MOE_BIG_DOWN(NT, float); else MOE_BIG_DOWN(NT, bf16_t); }
+#define MOE_BIG_DOWN(NT, TO) moe_big_kernel<NT, 0, TO><<<blocks(down_tiles), BIG_THREADS, 0, stream>>>((const bf16_t*)mid, slot_pair, top, \
+            (const bf16_t*)down, tile_expert, used, down_tiles, width, ff, cap, (TO*)y)
         if (tile == 64) MOE_BIG(1)
         else if (tile == 128) MOE_BIG(2)
         else if (tile == 192) MOE_BIG(3)
         else MOE_BIG(4)
 #undef MOE_BIG
 #undef MOE_BIG_UP
-        moe_combine_kernel<<<n_tokens, combine_threads, 0, stream>>>((const bf16_t*)y, pair_slot, weight, top, width, (const bf16_t*)add0, (const bf16_t*)add1, out);
+#undef MOE_BIG_DOWN
+        if (y32) MOE_COMBINE(float); else MOE_COMBINE(bf16_t);
         PALM_LAUNCHED();
         return 0;
     }
@@ -335,7 +363,8 @@ PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gat
 #undef MOE_UP
     moe_grouped_kernel<0><<<dim3(max_tiles, (width + GT_FEATURES - 1) / GT_FEATURES), GT_WAVES * WAVE, 0, stream>>>(
         (const bf16_t*)mid, nullptr, top, (const bf16_t*)down, tile_expert, width, ff, cap, (bf16_t*)y);
-    moe_combine_kernel<<<n_tokens, combine_threads, 0, stream>>>((const bf16_t*)y, pair_slot, weight, top, width, (const bf16_t*)add0, (const bf16_t*)add1, out);
+    MOE_COMBINE(bf16_t);
+#undef MOE_COMBINE
     PALM_LAUNCHED();
     return 0;
 }

@@ -912,10 +912,12 @@ _FEEDFORWARD_SIGNATURES = {
     "palm_moe_route_table": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p],
     "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int, c_int],
     "palm_moe_grouped": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
-                         c_void_p, c_void_p, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int],
+                         c_void_p, c_void_p, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int],
+    "palm_moe_grouped_in_tiles": [c_longlong, c_int, c_int, c_int, c_int],
     "palm_gather_rows": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
     "palm_scatter_add": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "palm_activation": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_longlong],
+    "palm_activation_planes": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_longlong],
 }
 _STREAMS_SIGNATURES = {
     "palm_streams_spread": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
@@ -1882,6 +1884,17 @@ def activation(z: torch.Tensor, kind: str) -> torch.Tensor:
     return out
 
 
+def activation_of_planes(z: torch.Tensor, kind: str, out_dtype: torch.dtype) -> torch.Tensor:
+    """``activation`` of a product in float32, [n, m] or planes [P, n, m] of partial sums (see ``linear_thin``); rounded once, to ``out_dtype``."""
+    _dev("activation", z)
+    _need(kind in ACTIVATIONS, f"activation: {kind!r} is not one of {sorted(ACTIVATIONS)}")
+    _need(z.dtype == F32 and z.dim() in (2, 3) and z.is_contiguous(), f"activation: {z.dtype} {tuple(z.shape)} are no float32 planes")
+    out = torch.empty(z.shape[-2:], dtype=out_dtype, device=z.device)
+    library.call(feedforward(), "palm_activation_planes", _stream(), _p(z), z.shape[0] if z.dim() == 3 else 1, _p(out), _code(out, "activation"),
+                 ACTIVATIONS[kind], out.numel())
+    return out
+
+
 def moe_route_table(ids: torch.Tensor, table: torch.Tensor):
     """ids int32 [n], table int32 [vocab, top] -> (chosen int32 [n, top], weight float32 [n, top]): every token's row of the table,
     and 1 / top for each choice.  (An id outside the table takes its nearest row: such a token's logits are no numbers anyway.)"""
@@ -1969,38 +1982,55 @@ def moe_grouped_serves(h: torch.Tensor, gate_up: torch.Tensor, ff: int) -> bool:
 
 
 # Above so many rows the grouped products' tiles of 64 rows are faster than the kernels for few rows, shared expert and all: a
-# layer of 32 experts of 2,048 x 4,096, four a row, and a shared one of twice the size, 16 rows 226 us by the kernels for few
-# rows, 190 + 33 by the grouped ones and the plain products; 32 rows 318 and 206 + 33, 64: 392, 206 + 35, 128: 587, 207 + 38.
+# layer of 32 experts of 2,048 x 4,096, four a row, and a shared one of twice the size, us, in a recorded step: 17 rows 273 by the
+# kernels for few rows and 197 by the grouped ones and the shared expert's three launches, 32 rows 330 and 217, 64: 390 and 228,
+# 128: 582 and 244.
 GROUPED_FROM = 16
 
 
-def moe_grouped_pays(h: torch.Tensor, gate_up: torch.Tensor, ff: int) -> bool:
+def moe_grouped_pays(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ff: int, top: int) -> bool:
     """Whether a step's rows go through the grouped products although the kernels for few rows would take them: enough rows, and
     sizes in whole stages, so that the matrices come through LDS."""
-    return h.shape[0] > GROUPED_FROM and moe_grouped_serves(h, gate_up, ff) and h.shape[1] % 64 == 0 and ff % 64 == 0
+    n, width = h.shape
+    if n <= GROUPED_FROM or not moe_grouped_serves(h, gate_up, ff) or down.dtype != BF16:
+        return False
+    experts = down.shape[0] // width
+    return bool(feedforward().palm_moe_grouped_in_tiles(n * top, experts, width, ff, _starts_on_16(h, gate_up, down)))
+
+
+def _starts_on_16(*tensors) -> bool:
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
 def moe_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor | None, ff: int,
-                form: str = "gated_silu", cap=NO_CAP, add=(), ids: torch.Tensor | None = None) -> torch.Tensor:
+                form: str = "gated_silu", cap=NO_CAP, add=(), ids: torch.Tensor | None = None, exact: bool = False,
+                planes: torch.Tensor | None = None) -> torch.Tensor:
     """Every row through its chosen experts, for many rows, planned on the device: the (row, choice) pairs grouped by expert,
     two grouped products on the matrix cores, the weighted sum in the order of the choices.  Shapes as ``moe_experts``;
-    returns float32 [n, width]."""
+    returns float32 [n, width].  The experts' results are bfloat16 between the second product and the sum, or float32 with
+    ``exact`` (operands in whole stages of 64 that start on 16 bytes).  ``planes``: float32 [n, width] or [P, n, width] of another branch to be added."""
     what = "moe_grouped"
     n, width = h.shape
     top = chosen.shape[1]
     experts = _check_experts(what, h, gate_up, down, chosen, weight, ff, form, ids, None)[0]
     _need(moe_grouped_serves(h, gate_up, ff) and down.dtype == BF16, f"{what}: bfloat16 rows and weights, sizes in multiples of eight")
-    aligned = (h.data_ptr() | gate_up.data_ptr() | down.data_ptr()) % 16 == 0
+    aligned = _starts_on_16(h, gate_up, down)
+    n_planes = 0
+    if planes is not None:
+        _dev(what, planes)
+        n_planes = planes.shape[0] if planes.dim() == 3 else 1
+        _need(planes.shape[-2:] == h.shape and planes.dim() in (2, 3) and planes.dtype == F32 and planes.is_contiguous(), f"{what}: planes {planes.dtype} "
+              f"{tuple(planes.shape)} for rows {tuple(h.shape)}")
     tile = feedforward().palm_moe_tile_tokens(n * top, experts, width, ff, aligned)
     max_tiles = (n * top + tile - 1) // tile + experts
     slots = max_tiles * tile
     plan = torch.empty((max_tiles + slots + n * top + 1,), dtype=torch.int32, device=h.device)
     mid = torch.empty((slots, ff), dtype=BF16, device=h.device)
-    y = torch.empty((slots, width), dtype=BF16, device=h.device)
+    y = torch.empty((slots, width), dtype=F32 if exact else BF16, device=h.device)
     out = torch.empty((n, width), dtype=F32, device=h.device)
     library.call(feedforward(), "palm_moe_grouped", _stream(), _p(h), _p(gate_up), _p(down), _p(chosen), _p(weight), n, top, experts, width, ff,
                  _p(plan), _p(mid), _p(y), _p(out), EXPERT_FORMS[form], *(float(c) for c in cap), *_addends(what, add, h), _p(ids),
-                 chosen.shape[0] if ids is not None else 0)
+                 chosen.shape[0] if ids is not None else 0, int(exact), _p(planes), n_planes)
     return out
 
 

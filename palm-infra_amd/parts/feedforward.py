@@ -141,8 +141,13 @@ class RoutedExperts:
         return ops.capped_gate(z, *self.cap) if self.form == "capped_gated" else ops.activation(z, ops.PLAIN_EXPERTS[self.form])
 
     def takes_few(self, h):
-        """Whether the kernels for few rows take these: up to DIRECT_ROWS, unless the grouped products are the better ones."""
-        return h.shape[0] <= self.DIRECT_ROWS and not ops.moe_grouped_pays(h, self.first, self.inter)
+        """Whether the kernels for few rows take these: up to DIRECT_ROWS, unless the grouped products are the better ones.  (Those
+        then keep the experts' results in 32 bits up to the sum, as the kernels for few rows do.)"""
+        return h.shape[0] <= self.DIRECT_ROWS and not ops.moe_grouped_pays(h, self.first, self.down_all, self.inter, self.top)
+
+    def run_grouped(self, h, chosen, weight, add=(), ids=None, planes=None):
+        return ops.moe_grouped(h, self.first, self.down_all, chosen, weight, self.inter, self.form, self.cap, add, ids=ids,
+                               exact=h.shape[0] <= self.DIRECT_ROWS, planes=planes)
 
     def run_few(self, h, chosen, weight, add=(), ids=None, shared=None, planes_ok=False):
         """``run_experts`` for at most DIRECT_ROWS rows, planned nowhere: the matrix cores, or the kernels that each (row, choice)
@@ -158,7 +163,7 @@ class RoutedExperts:
         if self.takes_few(h):
             return self.run_few(h, chosen, weight, add)
         if ops.moe_grouped_serves(h, self.first, self.inter):
-            return ops.moe_grouped(h, self.first, self.down_all, chosen, weight, self.inter, self.form, self.cap, add)
+            return self.run_grouped(h, chosen, weight, add)
         # group the (token, choice) pairs by expert; within an expert in the order of the tokens
         flat = chosen.to("cpu").numpy().reshape(-1)
         order = np.argsort(flat, kind="stable").astype(np.int32)
@@ -309,17 +314,22 @@ class RoutedTableFeedForward(RoutedExperts):
 
     def _run(self, h, ctx, planes_ok):
         n, shared = h.shape[0], tuple(s.weight for s in self.shared) if self.shared is not None else None
-        # in a step of few rows the shared expert rides in the experts' own kernels
+        # in a step of few rows the shared expert rides in the experts' own kernels, or beside the grouped products runs through the
+        # kernels for thin products, its sums in 32 bits up to the activation and up to the experts' sum
         few = self.takes_few(h)
         rides = shared is not None and few and (
             ops.moe_few_serves(h, self.first, self.inter, self.experts, self.top, shared) or (n <= self.SHARED_DIRECT_ROWS and self.shared_fits))
-        add = []
+        add, planes = [], None
         if shared is not None and not rides:
-            up, down = self.shared
-            add.append(down(ops.activation(up(h), ops.PLAIN_EXPERTS[self.form])))
+            (up, down), kind = self.shared, ops.PLAIN_EXPERTS[self.form]
+            if n <= self.DIRECT_ROWS and not few:
+                mid = ops.activation_of_planes(up(h, out_dtype=torch.float32, planes_ok=True), kind, h.dtype)
+                planes = down(mid, out_dtype=torch.float32, planes_ok=True)
+            else:
+                add.append(down(ops.activation(up(h), kind)))
         if few:
             return self.run_few(h, self.table, None, add, ids=ctx.token_ids, shared=shared if rides else None, planes_ok=planes_ok)
         if ops.moe_grouped_serves(h, self.first, self.inter):
-            return ops.moe_grouped(h, self.first, self.down_all, self.table, None, self.inter, self.form, self.cap, add, ids=ctx.token_ids)
+            return self.run_grouped(h, self.table, None, add, ids=ctx.token_ids, planes=planes)
         chosen, weight = ops.moe_route_table(ctx.token_ids, self.table)
         return self.run_experts(h, chosen, weight, add)

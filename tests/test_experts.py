@@ -120,8 +120,52 @@ def test_few_rows(form, E, top, W, F, shared):
         assert torch.allclose(more, got + y[0].float() + y[1].float(), atol=1e-3, rtol=1e-4)
 
 
+@gpu
+@pytest.mark.parametrize("form,E,top,W,F", [("relu_squared", 6, 2, 256, 128), ("gated_silu", 4, 3, 1088, 64), ("capped_gated", 33, 4, 320, 192), ("gelu", 2, 1, 64, 704)])
+def test_grouped_products_in_32_bits_are_as_near_as_the_kernels_for_few_rows(form, E, top, W, F):
+    """A step of few rows may take either way: both round the inner rows to bfloat16 and nothing behind them, so their errors against
+    64 bits are alike (the sums' order apart: 2^-24 against the inner rows' 2^-9); results in bfloat16 before the sum add two
+    fifths.  With planes of another branch to add."""
+    from palm_infra_amd.kernels import ops
+    cap = CAP if form == "capped_gated" else ops.NO_CAP
+    for n in (17, 40, 128):
+        h, up, down, chosen, weight = case(form, E, top, W, F, n, False, E + F + n, torch.bfloat16)
+        want = plain_mixture(form, h, up, down, chosen, weight, F)
+        args = [t.cuda() for t in (h, up, down, chosen, weight)]
+        error = lambda got: float((got.cpu().double() - want).norm() / want.norm())
+        got = ops.moe_grouped(*args, F, form, cap, exact=True)
+        assert error(got) <= 1.05 * error(ops.moe_few(*args, F, form, cap)), (n, error(got))
+        assert torch.equal(ops.moe_grouped(*args, F, form, cap, exact=True), got)
+        planes = torch.randn(3, n, W).cuda()
+        more = ops.moe_grouped(*args, F, form, cap, exact=True, planes=planes)
+        assert torch.allclose(more, got + planes.sum(0), atol=1e-5 * float(want.abs().max()), rtol=1e-5)
+        assert torch.equal(ops.moe_grouped(*args, F, form, cap, exact=True, planes=planes[0]), ops.moe_grouped(*args, F, form, cap, exact=True, planes=planes[:1]))
+    from palm_infra_amd.kernels import KernelError
+    odd = torch.empty(n * W + 1, dtype=torch.bfloat16, device="cuda")[1:].view(n, W).copy_(args[0])
+    with pytest.raises(KernelError, match="32-bit results"):
+        ops.moe_grouped(odd, *args[1:], F, form, cap, exact=True)
+
+
+@gpu
+@pytest.mark.parametrize("planes,n,m", [(1, 3, 7), (2, 17, 64), (4, 128, 1030)])
+def test_activation_of_a_product_in_planes(planes, n, m):
+    from palm_infra_amd.kernels import ops
+    z = torch.randn(planes, n, m)
+    total = z.double().sum(0)
+    for kind, want in (("relu_squared", torch.clamp(total, min=0.0) ** 2), ("gelu_erf", plain_expert("gelu", total, m))):
+        exact = ops.activation_of_planes(z.cuda(), kind, torch.float32).cpu()
+        assert torch.allclose(exact.double(), want, atol=1e-5, rtol=1e-5)
+        assert torch.equal(ops.activation_of_planes(z.cuda(), kind, torch.bfloat16).cpu(), exact.to(torch.bfloat16))
+
+
 def test_which_steps_go_through_the_grouped_products():
     from palm_infra_amd.kernels import ops
-    pays = lambda n, W, F, dt=torch.bfloat16: ops.moe_grouped_pays(torch.empty(n, W, dtype=dt), torch.empty(F, W, dtype=dt), F)
+
+    def pays(n, W, F, E=1, top=1, dt=torch.bfloat16, offset=0):
+        h = torch.empty(n * W + 8, dtype=dt)[offset:offset + n * W].view(n, W)
+        return ops.moe_grouped_pays(h, torch.empty(E * F, W, dtype=dt), torch.empty(E * W, F, dtype=dt), F, top)
     assert pays(17, 64, 128) and pays(128, 4096, 64)
-    assert not pays(16, 64, 128) and not pays(17, 72, 128) and not pays(17, 64, 40) and not pays(17, 64, 128, torch.float32)
+    assert not pays(16, 64, 128) and not pays(17, 72, 128) and not pays(17, 64, 40) and not pays(17, 64, 128, dt=torch.float32)
+    # what the grouped products refuse or do from memory stays with the kernels for few rows: more experts, rows that start on no 16 bytes
+    assert pays(17, 64, 64, E=512, top=4) and not pays(17, 64, 64, E=513, top=4)
+    assert not pays(17, 64, 128, offset=1) and pays(17, 64, 128, offset=8)

@@ -585,7 +585,8 @@ def test_direct_queries_through_the_key_matrix_and_cache_rows_in_one_launch(dtyp
 
 @gpu
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("E,top,W,F,shared", [(6, 2, 48, 24, 40), (5, 1, 64, 32, 32), (4, 4, 40, 16, None), (9, 5, 50, 7, 11), (33, 3, 72, 40, 8), (7, 2, 264, 136, 64)])
+@pytest.mark.parametrize("E,top,W,F,shared", [(6, 2, 48, 24, 40), (5, 1, 64, 32, 32), (4, 4, 40, 16, None), (9, 5, 50, 7, 11), (33, 3, 72, 40, 8), (7, 2, 264, 136, 64),
+                                             (6, 2, 64, 128, 192), (36, 4, 2048, 64, 128)])
 def test_table_experts_for_few_rows_and_many(dtype, E, top, W, F, shared):
     """The part alone, with the step's token ids choosing: one row, a few (the shared expert rides along), a decode batch's
     and a prompt's; also when all tokens choose the same experts and when an expert is chosen by nobody."""
@@ -615,6 +616,7 @@ def test_table_experts_for_few_rows_and_many(dtype, E, top, W, F, shared):
     f = {"router": {"experts": E, "top": top}, **({"shared": {"ff": shared}} if shared else {})}
     # (squares of bfloat16 numbers summed over few inner values: outputs of several units)
     tol = dict(atol=1e-4, rtol=1e-4) if dtype == "float32" else dict(atol=8e-2, rtol=3e-2)
+    grouped = []
     for n, same in ((1, False), (9, False), (16, True), (17, False), (128, False), (128, True), (129, True), (200, False)):
         ids = [5] * n if same else torch.randint(0, V, (n,), generator=g).tolist()
         h = torch.randn(n, W, generator=g).to(dt)
@@ -622,6 +624,15 @@ def test_table_experts_for_few_rows_and_many(dtype, E, top, W, F, shared):
         ctx = _step_context([0], [n], ids=[ids])
         got = part.forward(h.cuda(), ctx)
         assert torch.allclose(got.cpu().double(), want, **tol), (n, same, float((got.cpu().double() - want).abs().max()))
+        if dtype == "bfloat16" and n <= 128 and not part.takes_few(h.cuda()):
+            # the grouped products and the shared expert beside them round what the kernels for few rows round, and nothing else
+            few = ops.moe_few(h.cuda(), part.first, part.down_all, part.table, None, F, part.form, ids=ctx.token_ids,
+                              shared=tuple(s.weight for s in part.shared))
+            error, of_few = (float((o.cpu().double() - want).norm() / want.norm()) for o in (got, few))
+            assert error <= 1.05 * of_few, (n, error, of_few)
+            grouped.append(n)
+    # sizes in whole stages take the grouped products below a prompt's rows
+    assert grouped == ({64: [17, 128, 128], 2048: [17, 128, 128]}.get(W, []) if dtype == "bfloat16" and F % 64 == 0 else [])
     chosen, weight = ops.moe_route_table(torch.tensor([3, 36, 0], dtype=torch.int32).cuda(), t["table"].cuda())
     assert torch.equal(chosen.cpu(), t["table"][[3, 36, 0]]) and torch.allclose(weight.cpu(), torch.full((3, top), 1.0 / top))
     t["table"][2, 0] = E
@@ -799,6 +810,30 @@ def test_a_padded_recorded_step_of_many_sequences(tmp_path_factory, dtype):
     got = eng.step([StepEntry(s, [r[-1]], [0]) for s, r in zip(slots[:7], reqs)])
     assert_close(got, torch.stack([r[-1] for r in refs[:7]]), dtype, "seven of them")
     for s in slots[:7]:
+        eng.close(s)
+
+
+@gpu
+def test_a_recorded_step_whose_experts_are_grouped(tmp_path):
+    """Nineteen sequences decode together, padded to twenty-four rows, through experts whose tiles take the grouped products in a
+    recorded step, the shared expert beside them: several replays, with other work between them, against the plain implementation."""
+    from palm_infra_amd.engine import Engine, StepEntry
+    raw = S.model(97, 2048, 1e-5, [S.layer(S.attention(4, 2, 32, 32, 0.2, window=37, rot=(16, 500.0)), S.moe(36, 4, 64, shared=128)),
+                                   S.layer(S.attention(2, 2, 32, 32, 0.2), S.moe(40, 2, 64))])
+    eng = Engine.from_dir(S.write_model(raw, 31, tmp_path, "bfloat16"), dtype="bfloat16", max_tokens=4096)
+    rows = torch.empty((24, 2048), dtype=torch.bfloat16, device="cuda")
+    assert not any(b.feed_forward.takes_few(rows) for b in eng.model.layers)
+    cfg, w = P.read_model(tmp_path)
+    reqs = S.prompts(raw, [6 + 2 * i for i in range(19)], seed=18)
+    refs = [P.forward(cfg, w, r) for r in reqs]
+    slots = [eng.open() for _ in reqs]
+    eng.step([StepEntry(s, r[:-5], []) for s, r in zip(slots, reqs)])
+    for t in range(5, 0, -1):
+        got = eng.step([StepEntry(s, [r[-t]], [0]) for s, r in zip(slots, reqs)])
+        torch.randn(300, 300, device="cuda").sum()
+        torch.cuda.synchronize()
+        assert_close(got, torch.stack([r[-t] for r in refs]), "bfloat16", f"nineteen, {t} to go")
+    for s in slots:
         eng.close(s)
 
 
