@@ -9,7 +9,8 @@
 //          values of the experts in use are dealt to the planes' waves in turn; a piece's products go, weighted, into the wave's
 //          own sums [row, 16 features] in LDS, and the waves' sums are added in their order
 //
-// Both kernels are made for up to 16 rows (one column tile) and for more (up to four that share every matrix fragment).
+// Both kernels are made for up to 16 rows (one column tile) and for more (up to four that share every matrix fragment): the steps
+// of more rows that the grouped products (moe_grouped.hip) do not serve, or whose few tiles there leave the chip idle.
 //
 // A shared expert that every row goes through (weight one, an inner size of its own) runs as one more expert.  Result: float32
 // planes [planes, n, width] for a reader that adds them, the first with the rows of other branches.
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(FEW_UP_WAVES * WAVE) void moe_few_up_kernel(const b
             // the first chunk's matrix rows are on their way while the activations go to LDS
             constexpr int CHUNK = 32 * FEW_STEPS;
             // blocks begin at chunks of their own: in step they meet on a few of memory's channels (16 rows, 32 experts of 2,048 x
-            // 4,096, a layer: 206 -> 196 us; 64 rows: 331 -> 267)
+            // 4,096, a layer: 206 -> 196 us)
             const int chunks = (len + CHUNK - 1) / CHUNK, turn = (3 * e + blockIdx.y + 2 * wave) % chunks;
             auto chunk_at = [&](int i) { i += turn; return k0 + (i < chunks ? i : i - chunks) * CHUNK; };
             bf16x8 wf[MATS][FEW_STEPS];

@@ -1981,21 +1981,35 @@ def moe_grouped_serves(h: torch.Tensor, gate_up: torch.Tensor, ff: int) -> bool:
     return h.dtype == BF16 and gate_up.dtype == BF16 and h.shape[1] % 8 == 0 and ff % 8 == 0
 
 
-# Above so many rows the grouped products' tiles of 64 rows are faster than the kernels for few rows, shared expert and all: a
-# layer of 32 experts of 2,048 x 4,096, four a row, and a shared one of twice the size, us, in a recorded step: 17 rows 273 by the
-# kernels for few rows and 197 by the grouped ones and the shared expert's three launches, 32 rows 330 and 217, 64: 390 and 228,
-# 128: 582 and 244.
+# Up to so many rows every step goes through the kernels for few rows; above, through the grouped products where their tiles keep the
+# chip busy: a tile of 64 rows walks over its stages at about a microsecond each, whatever the rows.  Us, kernels for few rows and
+# grouped products with 32-bit results, 17 / 64 / 128 rows (both alone, in a recorded step):
+#   32 experts of 2,048 x 4,096, four a row (768 tiles)       234 264 382   168 196 201
+#   32 capped experts of 1,536 x 4,096, four a row (896)      220 255 345   220 231 237
+#   16 gated experts of 1,408 x 2,048, four a row (304)        95 140 173    73  70  72
+#   64 gated experts of 256 x 512, eight a row (256)           32  41  65    27  28  29
+#   32 experts of 512 x 1,024, four a row (192)                38  46  72    38  38  39
+#   8 gated experts of 1,024 x 2,048, one a row (128)          45  51  69    51  52  53
+#   8 experts of 1,024 x 2,048, two a row (96)                 43  67  86    53  54  56
+#   16 experts of 256 x 512, two a row (48)                    18  20  28    25  25  26
+# A shared expert rides in the kernels for few rows and is three launches beside the grouped products: 32 experts of 1,024 x 2,048 with one
+# of 2,048 (384 tiles) 99 129 204 and 76 83 90, of 512 x 1,024 with one of 512 (192 tiles) 37 51 85 and 51 56 56.
 GROUPED_FROM = 16
+GROUPED_SURELY_FROM = 96
+GROUPED_TILES, GROUPED_TILES_SHARED = 192, 320
 
 
-def moe_grouped_pays(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ff: int, top: int) -> bool:
-    """Whether a step's rows go through the grouped products although the kernels for few rows would take them: enough rows, and
-    sizes in whole stages, so that the matrices come through LDS."""
+def moe_grouped_pays(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, ff: int, top: int, form: str, shared: bool = False) -> bool:
+    """Whether a step's rows go through the grouped products although the kernels for few rows would take them: sizes in whole stages,
+    so that the matrices come through LDS, and tiles enough for the number of rows."""
     n, width = h.shape
     if n <= GROUPED_FROM or not moe_grouped_serves(h, gate_up, ff) or down.dtype != BF16:
         return False
     experts = down.shape[0] // width
-    return bool(feedforward().palm_moe_grouped_in_tiles(n * top, experts, width, ff, _starts_on_16(h, gate_up, down)))
+    if not feedforward().palm_moe_grouped_in_tiles(n * top, experts, width, ff, _starts_on_16(h, gate_up, down)):
+        return False
+    tiles = min(experts, n * top) * (-(-expert_rows(form) * ff // 256) + -(-width // 256))
+    return n > GROUPED_SURELY_FROM or tiles >= (GROUPED_TILES_SHARED if shared else GROUPED_TILES)
 
 
 def _starts_on_16(*tensors) -> bool:

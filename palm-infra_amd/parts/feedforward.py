@@ -140,10 +140,10 @@ class RoutedExperts:
         z = self.expert_first[e](xs)
         return ops.capped_gate(z, *self.cap) if self.form == "capped_gated" else ops.activation(z, ops.PLAIN_EXPERTS[self.form])
 
-    def takes_few(self, h):
+    def takes_few(self, h, shared: bool = False):
         """Whether the kernels for few rows take these: up to DIRECT_ROWS, unless the grouped products are the better ones.  (Those
         then keep the experts' results in 32 bits up to the sum, as the kernels for few rows do.)"""
-        return h.shape[0] <= self.DIRECT_ROWS and not ops.moe_grouped_pays(h, self.first, self.down_all, self.inter, self.top)
+        return h.shape[0] <= self.DIRECT_ROWS and not ops.moe_grouped_pays(h, self.first, self.down_all, self.inter, self.top, self.form, shared)
 
     def run_grouped(self, h, chosen, weight, add=(), ids=None, planes=None):
         return ops.moe_grouped(h, self.first, self.down_all, chosen, weight, self.inter, self.form, self.cap, add, ids=ids,
@@ -316,7 +316,7 @@ class RoutedTableFeedForward(RoutedExperts):
         n, shared = h.shape[0], tuple(s.weight for s in self.shared) if self.shared is not None else None
         # in a step of few rows the shared expert rides in the experts' own kernels, or beside the grouped products runs through the
         # kernels for thin products, its sums in 32 bits up to the activation and up to the experts' sum
-        few = self.takes_few(h)
+        few = self.takes_few(h, shared is not None)
         rides = shared is not None and few and (
             ops.moe_few_serves(h, self.first, self.inter, self.experts, self.top, shared) or (n <= self.SHARED_DIRECT_ROWS and self.shared_fits))
         add, planes = [], None

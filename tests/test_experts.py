@@ -161,11 +161,15 @@ def test_activation_of_a_product_in_planes(planes, n, m):
 def test_which_steps_go_through_the_grouped_products():
     from palm_infra_amd.kernels import ops
 
-    def pays(n, W, F, E=1, top=1, dt=torch.bfloat16, offset=0):
+    def pays(n, W, F, E=1, top=1, dt=torch.bfloat16, form="gelu", shared=False, offset=0):
         h = torch.empty(n * W + 8, dtype=dt)[offset:offset + n * W].view(n, W)
-        return ops.moe_grouped_pays(h, torch.empty(E * F, W, dtype=dt), torch.empty(E * W, F, dtype=dt), F, top)
-    assert pays(17, 64, 128) and pays(128, 4096, 64)
-    assert not pays(16, 64, 128) and not pays(17, 72, 128) and not pays(17, 64, 40) and not pays(17, 64, 128, dt=torch.float32)
+        return ops.moe_grouped_pays(h, torch.empty(E * ops.expert_rows(form) * F, W, dtype=dt), torch.empty(E * W, F, dtype=dt), F, top, form, shared)
+    assert pays(97, 64, 128) and pays(128, 4096, 64) and not pays(96, 64, 128)
+    assert pays(17, 2048, 64, E=22, top=4) and not pays(17, 2048, 64, E=21, top=4)          # 198 and 189 tiles
+    assert not pays(17, 2048, 64, E=22, top=1)                                               # at most seventeen experts in use
+    assert not pays(17, 2048, 64, E=22, top=4, shared=True) and pays(17, 2048, 64, E=36, top=4, shared=True)
+    assert pays(17, 1024, 512, E=32, top=4) and pays(17, 1024, 512, E=32, top=4, form="gated_silu")
+    assert not pays(16, 2048, 64, E=22, top=4) and not pays(97, 72, 128) and not pays(97, 64, 40) and not pays(97, 64, 128, dt=torch.float32)
     # what the grouped products refuse or do from memory stays with the kernels for few rows: more experts, rows that start on no 16 bytes
-    assert pays(17, 64, 64, E=512, top=4) and not pays(17, 64, 64, E=513, top=4)
-    assert not pays(17, 64, 128, offset=1) and pays(17, 64, 128, offset=8)
+    assert pays(97, 64, 64, E=512, top=4) and not pays(97, 64, 64, E=513, top=4)
+    assert not pays(97, 64, 128, offset=1) and pays(97, 64, 128, offset=8)
