@@ -134,11 +134,12 @@ __global__ __launch_bounds__(256) void retention_local_kernel(const T* __restric
 #pragma unroll 4
     for (int s = 0; s < (n + 3) / 4; ++s) {
         const int t = 4 * s + g, row = chunk.row0 + min(t, n - 1);
-        const float w = t < n ? power[max(n - 1 - t, 0)] : 0.f;
+        const float w = power[max(n - 1 - t, 0)];
         RetRun<VT> vv = ret_run<VT>(rows + (size_t)row * row_stride + v_off + h * VDIM + v0 + VT * r);
-        if (act) {
 #pragma unroll
-            for (int ve = 0; ve < VT; ++ve) vv.v[ve] = rec_silu(vv.v[ve]);
+        for (int ve = 0; ve < VT; ++ve) {                // (a token beyond the chunk: zeros on both sides, as zero times infinity is none)
+            if (act) vv.v[ve] = rec_silu(vv.v[ve]);
+            vv.v[ve] = t < n ? vv.v[ve] : 0.f;
         }
         const float* kr = qk + ((size_t)row * heads + h) * 2 * DIM + DIM + 4 * r;
 #pragma unroll
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(256) void retention_local_kernel(const T* __restric
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int ve = 0; ve < VT; ++ve) acc[q][e][ve] = ret_mfma(vv.v[ve], kv.v[e] * w, acc[q][e][ve]);
+                for (int ve = 0; ve < VT; ++ve) acc[q][e][ve] = ret_mfma(vv.v[ve], t < n ? kv.v[e] * w : 0.f, acc[q][e][ve]);
         }
     }
     float* out = starts + (chunk.place * heads + h) * DIM * VDIM + v0 + 4 * VT * g;
@@ -273,10 +274,30 @@ __global__ __launch_bounds__(256) void retention_out_kernel(const T* __restrict_
                 for (int ve = 0; ve < VT; ++ve) vv[e].v[ve] = rec_silu(vv[e].v[ve]);
             }
         }
+        float odd = 0.f;                                 // a number unless one of the values is none, or infinite
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int ve = 0; ve < VT; ++ve) odd = fmaf(vv[e].v[ve], 0.f, odd);
+        const bool finite = __ballot(odd != odd) == 0;
 #pragma unroll
         for (int i = sb; i < TT; ++i) {                  // the tokens before the block see none of it
             if (16 * i >= n) continue;
             const RetRun<4> p = ret_run<4>(&P[16 * i + r][16 * sb + 4 * g]);
+            if (i == sb && !finite) {
+                // within the block zeros stand for what a token does not see, and zero times infinity is no number: a token at a
+                // time, and only the tokens that see it take it in
+#pragma unroll 1
+                for (int from = 0; from < 4; ++from)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int ve = 0; ve < VT; ++ve) {
+                            const f32x4 one = ret_mfma(g == from ? vv[e].v[ve] : 0.f, g == from ? p.v[e] : 0.f, f32x4{0.f, 0.f, 0.f, 0.f});
+                            if (r >= 4 * from + e) o[i][ve] += one;
+                        }
+                continue;
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll

@@ -367,6 +367,43 @@ def test_retention_in_chunks_on_the_matrix_cores(dtype, dk, dv):
 
 
 @gpu
+@pytest.mark.parametrize("dk,dv", [(64, 128), (128, 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("input_silu", [False, True])
+def test_retention_chunks_keep_infinities_where_they_are(dtype, dk, dv, input_silu):
+    """An infinite or no number in a token's values or keys reaches that token and later ones of its sequence, in its own value
+    dimensions (or rows of the state) and no others, as when the tokens are walked over one by one; with the inputs through silu too."""
+    from palm_infra_amd.kernels import ops
+    torch.manual_seed(dk)
+    H, lengths = 2, [40, 17, 70, 33]
+    T = sum(lengths)
+    rows = (torch.randn(T, H * (2 * dk + 2 * dv)) * 0.5).to(dtype)
+    v0, inf = 2 * H * dk, float("inf")
+    rows[21, v0 + 5] = inf                                   # sequence 0, token 21 (the middle of a block of sixteen), head 0
+    rows[56, v0 + dv + 9] = float("nan")                     # sequence 1, its last token (the chunk ends there), head 1
+    rows[57 + 66, v0 + 3] = inf                              # sequence 2, the second chunk
+    rows[T - 1, H * dk + 7] = inf                            # sequence 3: a key of its last token, head 0
+    decay, state0 = torch.tensor([0.97, 0.9]), torch.randn(len(lengths), H, dk, dv)
+    results = []
+    for chunk in (None, 0):
+        state = state0.clone().cuda()
+        ctx = _step_context([0] * len(lengths), lengths)
+        raw = ops.retention(rows.cuda(), H, dk, dv, decay.cuda(), dk ** -0.5, 1e-6, state, ctx, chunk=chunk, input_silu=input_silu)
+        results.append((raw.float().cpu(), state.cpu()))
+    (got, left), (want, walked) = results
+    # (the norm over a head's outputs spreads one of them over its head: a token's head is finite or it is not)
+    whole = lambda y: torch.isfinite(y.view(T, H, dv)).all(-1)
+    assert torch.equal(whole(got), whole(want)) and not whole(want).all()
+    assert whole(got)[:21].all() and whole(got)[40:56].all() and whole(got)[57:57 + 66].all() and whole(got)[-33:-1].all()
+    tol = 1e-4 if dtype == torch.float32 else 3e-2
+    keep = whole(want)
+    a, b = got.view(T, H, dv)[keep], want.view(T, H, dv)[keep]
+    assert (a - b).abs().max() < tol * max(1.0, float(b.abs().max()))
+    assert torch.equal(torch.isfinite(left), torch.isfinite(walked)) and not torch.isfinite(walked).all()
+    assert (left[torch.isfinite(left)] - walked[torch.isfinite(walked)]).abs().max() < 1e-4
+
+
+@gpu
 @pytest.mark.parametrize("dk,dv", [(12, 28), (40, 72)])      # the second pair is one that the matrix-core kernel takes in bfloat16
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge(dtype, dk, dv):
