@@ -172,7 +172,7 @@ struct ScanDecay {
     float hi, lo;                                       // A log2 e and, times ln 2, what hi leaves of it
     __device__ static ScanDecay of(float a) {
         constexpr float LOG2E = 1.44269504f, LOG2E_REST = 1.92596299e-8f, LN2 = 0.693147181f;
-        a = fmaxf(a, -1e30f);                           // (finite: an A beyond the range is forgotten at once all the same)
+        if (a < -2e38f) a = -2e38f;                     // (hi stays finite; no number stays none)
         ScanDecay d;
         d.hi = a * LOG2E;
         d.lo = (fmaf(a, LOG2E, -d.hi) + a * LOG2E_REST) * LN2;

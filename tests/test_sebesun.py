@@ -404,6 +404,43 @@ def test_retention_chunks_keep_infinities_where_they_are(dtype, dk, dv, input_si
 
 
 @gpu
+@pytest.mark.parametrize("C,N", [(130, 3), (65, 8), (200, 16), (70, 20), (37, 64), (9, 100), (6, 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_selective_scan_alone(dtype, C, N):
+    """Every build of the kernel by state size, around the borders of its tiles of sixteen tokens, on states that hold something, against
+    the recurrence in 64 bits; a decay so fast that nothing stays, and an A that is no number, which its channel shows."""
+    from palm_infra_amd.kernels import ops
+    g = torch.Generator().manual_seed(C + N)
+    lengths = [1, 15, 16, 17, 49, 2]
+    T = sum(lengths)
+    R = lambda *s: torch.randn(*s, generator=g)
+    u, xz, bc = (R(T, c).to(dtype) for c in (C, 2 * C, 2 * N + 3))
+    dtl, bias, skip, state0 = R(T, C), R(C) - 2.0, R(C), R(len(lengths), C, N)
+    a_log = torch.log(torch.arange(1, N + 1).float()).repeat(C, 1) + 0.1 * R(C, N)
+    a_log[1, 1], a_log[2, 2], a_log[4, 0] = 75.0, 88.7, float("nan")
+    A, dt = -torch.exp(a_log.double()), torch.nn.functional.softplus((dtl + bias).double())
+    z, B, Cm = xz[:, C:].double(), bc[:, 1:1 + N].double(), bc[:, 2 + N:2 + 2 * N].double()
+    want, left, at = torch.zeros(T, C, dtype=P.F64), [], 0
+    for b, n in enumerate(lengths):
+        S = state0[b].double()
+        for t in range(at, at + n):
+            S = torch.exp(dt[t][:, None] * A) * S + (dt[t] * u[t].double())[:, None] * B[t]
+            want[t] = ((S * Cm[t]).sum(1) + skip.double() * u[t].double()) * P.silu(z[t])
+        left.append(S)
+        at += n
+    left = torch.stack(left)
+    state = state0.clone().cuda()
+    got = ops.selective_scan(u.cuda(), xz.cuda(), bc.cuda(), 1, 2 + N, dtl.cuda(), bias.cuda(), a_log.cuda(), skip.cuda(), state,
+                             _step_context([0] * len(lengths), lengths)).double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isnan(got[:, 4]).all() and torch.isnan(got).sum() == T
+    assert torch.equal(torch.isnan(state.cpu()), torch.isnan(left))
+    # 32-bit sums of up to 256 terms over up to 49 tokens, then one rounding to the type
+    keep, tol = torch.arange(C) != 4, 1e-5 if dtype == torch.float32 else 4e-3
+    assert (got - want)[:, keep].abs().max() < tol * float(want[:, keep].abs().max())
+    assert (state.cpu().double() - left)[:, keep].abs().max() < 1e-5 * float(left[:, keep].abs().max())
+
+
+@gpu
 @pytest.mark.parametrize("dk,dv", [(12, 28), (40, 72)])      # the second pair is one that the matrix-core kernel takes in bfloat16
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge(dtype, dk, dv):
