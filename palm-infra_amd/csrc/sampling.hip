@@ -129,7 +129,7 @@ static uint64_t splitmix(uint64_t z) {
     return z ^ (z >> 31);
 }
 PALM_API int palm_uniforms(unsigned long long seed, const uint64_t* streams, const uint64_t* draws, int n, float* out) {
-    PALM_CHECK(n >= 0 && streams && draws && out, "uniforms: n=%d", n);
+    PALM_CHECK(n >= 0 && (n == 0 || (streams && draws && out)), "uniforms: n=%d", n);        // (nothing has no address)
     const uint64_t of_seed = splitmix(seed);
     for (int i = 0; i < n; ++i) out[i] = (float)(splitmix(splitmix(of_seed ^ streams[i]) ^ draws[i]) >> 40) / 16777216.0f;
     return 0;

@@ -44,6 +44,14 @@ def test_a_batch_of_uniform_numbers_is_the_single_ones(seed):
     assert out.tolist() == [uniform(seed, s, d) for s, d in pairs]
 
 
+def test_an_empty_batch_takes_no_uniform_numbers():
+    import torch
+    from palm_infra_amd.kernels import ops
+    out = torch.empty(0)
+    ops.uniforms_into(out, 42, [], [])
+    assert out.shape == (0,)
+
+
 def test_history_window_counts_match_the_plain_penalties():
     hist = [4, 9, 4, 4, 2, 300, -1]
     assert penalty_counts(hist, 3, 100) == {2: 1}              # 300 and -1 are not tokens of a 100-vocabulary
