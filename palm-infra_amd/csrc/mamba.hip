@@ -197,6 +197,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     constexpr int CH = SCAN_THREADS / G;               // channels of a block
     constexpr int NP = G * PER;                        // the state size, padded
     constexpr int NB = (SCAN_TILE * NP + SCAN_THREADS - 1) / SCAN_THREADS, NC = (SCAN_TILE * CH + SCAN_THREADS - 1) / SCAN_THREADS;
+    // of B and C at a time: all, but where that costs blocks a compute unit (128 states, eight at a time: 88 registers and five waves a
+    // SIMD; 2,048 channels, 717 + 572 + 1,314 tokens 694 us, in halves 617; one token each of 64 sequences 84 and 65).  (256 states:
+    // LDS sets the number of blocks.)
+    constexpr int HELD = PER == 2 ? 4 : NB;
     __shared__ float b_s[SCAN_TILE][NP], c_s[SCAN_TILE][NP];
     __shared__ float dt_s[SCAN_TILE][CH], u_s[SCAN_TILE][CH], y_s[SCAN_TILE][CH];
     const int j = threadIdx.x % G, ch = threadIdx.x / G;
@@ -216,7 +220,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
         A[k] = ScanDecay::of(n < n_state ? -expf(a_log[(size_t)cc * n_state + n]) : 0.f);
     }
     // this thread's elements of a tile: idx = threadIdx + i SCAN_THREADS is token idx / NP (idx / CH), state (channel) the rest
-    T b_r[NB], c_r[NB], u_r[NC], z_r[NC];              // (as they lie in memory: a conversion would wait for each)
+    T b_r[HELD], c_r[HELD], u_r[NC], z_r[NC];          // (as they lie in memory: a conversion would wait for each)
     float dt_r[NC], skip[NC], bias[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
@@ -226,16 +230,27 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
         skip[i] = d_skip[ck];
         bias[i] = dt_bias[ck];
     }
-    auto ask = [&](int t0) {                           // (tokens beyond the sequence are not read and not used)
+    auto ask_states = [&](int t0, int first) {         // (tokens beyond the sequence are not read and not used)
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const int idx = threadIdx.x + i * SCAN_THREADS, n = idx % NP;
+        for (int i = 0; i < HELD; ++i) {
+            const int idx = threadIdx.x + (first + i) * SCAN_THREADS, n = idx % NP;
             b_r[i] = c_r[i] = T{};
             if (n >= n_state || t0 + idx / NP >= n_new) continue;
             const T* r = bc + (row0 + t0 + idx / NP) * bc_stride;
             b_r[i] = r[b_off + n];
             c_r[i] = r[c_off + n];
         }
+    };
+    auto keep_states = [&](int tt, int first) {
+#pragma unroll
+        for (int i = 0; i < HELD; ++i) {
+            const int idx = threadIdx.x + (first + i) * SCAN_THREADS;
+            if (idx / NP < tt) { b_s[idx / NP][idx % NP] = to_float(b_r[i]); c_s[idx / NP][idx % NP] = to_float(c_r[i]); }
+        }
+    };
+    // (where a tile has fewer elements than the block threads, the threads beyond it read the next tiles': nearer when their turn
+    // comes.  Leaving them out was 7 to 9 % slower for 64 and 128 states.)
+    auto ask_channels = [&](int t0) {
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
             const int idx = threadIdx.x + i * SCAN_THREADS, ck = min(c0 + idx % CH, channels - 1);
@@ -248,15 +263,15 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
             z_r[i] = z[row * z_stride + ck];
         }
     };
-    if (AHEAD) ask(0);
+    if (AHEAD) { ask_states(0, 0); ask_channels(0); }
     for (int t0 = 0; t0 < n_new; t0 += SCAN_TILE) {
         const int tt = min(SCAN_TILE, n_new - t0);
-        if (!AHEAD) ask(t0);
+        if (!AHEAD) ask_channels(t0);
         float u_t[NC], z_t[NC];
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const int idx = threadIdx.x + i * SCAN_THREADS;
-            if (idx / NP < tt) { b_s[idx / NP][idx % NP] = to_float(b_r[i]); c_s[idx / NP][idx % NP] = to_float(c_r[i]); }
+#pragma unroll 1
+        for (int first = 0; first < NB; first += HELD) {
+            if (!AHEAD) ask_states(t0, first);
+            keep_states(tt, first);
         }
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
@@ -266,7 +281,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
             z_t[i] = to_float(z_r[i]);
         }
         __syncthreads();
-        if (AHEAD && t0 + SCAN_TILE < n_new) ask(t0 + SCAN_TILE);        // on their way while this tile is scanned
+        if (AHEAD && t0 + SCAN_TILE < n_new) { ask_states(t0 + SCAN_TILE, 0); ask_channels(t0 + SCAN_TILE); }        // on their way while this tile is scanned
 #define SCAN_TOKEN(ti) { \
             const float dt = dt_s[ti][ch]; \
             const float du = dt * u_s[ti][ch]; \
