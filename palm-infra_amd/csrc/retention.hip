@@ -65,10 +65,13 @@ __global__ void retention_rotate_kernel(const T* __restrict__ qkvg, int row_stri
 // instructions, element e of every lane each), VT neighbouring value dimensions of V and S (tile e is made of dimensions
 // VT r + e).  A lane of a result then holds 4 VT neighbouring value dimensions of one token, or of one row of S.
 // A block of four waves serves a (head, chunk, sequence), wave w the value dimensions 16 VT w .. : sizes of 64 VT.
-// Chunk c of sequence b lies at place cu_new[b] / C + b + c of the starts: no two share one, and they are at most
-// n_tokens / C + n_seqs.
+// Chunk c of sequence b has place cu_new[b] / C + b + c: no two share one, a sequence's lie side by side, and they are at most
+// n_tokens / C + n_seqs.  The starts have room for a window of RET_ROOM bytes of them, and the three kernels take one window of
+// places after the other (16 heads of 128 x 256: 64 places, 4,096 tokens; a window is then 1,024 blocks, so the cuts cost nothing:
+// 8,192 tokens 585 us with room for all, 566 in windows).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int RET_CHUNK = 64;
+constexpr long long RET_ROOM = 128ll << 20;
 
 __device__ inline f32x4 ret_mfma(float a, float b, f32x4 acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
 template <int N> struct RetRun { float v[N]; };
@@ -105,20 +108,30 @@ __device__ inline void ret_store_run4(bf16_t* p, float a, float b, float c, floa
 }
 
 struct RetChunk {
-    int row0, n;                 // the chunk's first row and how many tokens it has (<= 0: none)
-    size_t place;
-    __device__ RetChunk(const int* seq_new, const int* cu_new, int b, int c)
-        : row0(cu_new[b] + c * RET_CHUNK), n(min(RET_CHUNK, seq_new[b] - c * RET_CHUNK)), place(cu_new[b] / RET_CHUNK + b + c) {}
+    int row0, n;                 // the first row of a place's chunk and how many tokens it has (<= 0: none)
+    __device__ RetChunk(const int* seq_new, const int* cu_new, int n_seqs, int place) {
+        const int lane = threadIdx.x % WAVE;
+        row0 = n = 0;            // of the last sequence whose first place is not beyond this one
+        for (int s0 = 0; s0 < n_seqs; s0 += WAVE) {
+            const int s = s0 + lane, first = cu_new[min(s, n_seqs - 1)], count = seq_new[min(s, n_seqs - 1)];
+            const unsigned long long at_or_before = __ballot(s < n_seqs && first / RET_CHUNK + s <= place);
+            if (!at_or_before) break;
+            const int at = __popcll(at_or_before) - 1, done = (place - (s0 + at) - __shfl(first, at, WAVE) / RET_CHUNK) * RET_CHUNK;
+            row0 = __shfl(first, at, WAVE) + done;
+            n = min(RET_CHUNK, __shfl(count, at, WAVE) - done);
+        }
+    }
 };
 
 template <typename T, int DIM, int VT>
 __global__ __launch_bounds__(256) void retention_local_kernel(const T* __restrict__ rows, int row_stride, int v_off, const float* __restrict__ qk,
                                                               const float* __restrict__ decay, const int* __restrict__ seq_new,
-                                                              const int* __restrict__ cu_new, int heads, int act, float* __restrict__ starts) {
+                                                              const int* __restrict__ cu_new, int n_seqs, int place0, int heads, int act,
+                                                              float* __restrict__ starts) {
     constexpr int VDIM = 64 * VT, DQ = DIM / 64;
     __shared__ float power[RET_CHUNK];
     const int h = blockIdx.x;
-    const RetChunk chunk(seq_new, cu_new, blockIdx.z, blockIdx.y);
+    const RetChunk chunk(seq_new, cu_new, n_seqs, place0 + blockIdx.y);
     const int n = chunk.n;
     if (n <= 0) return;
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, r = lane % 16, g = lane / 16, v0 = wave * 16 * VT;
@@ -151,7 +164,7 @@ __global__ __launch_bounds__(256) void retention_local_kernel(const T* __restric
                 for (int ve = 0; ve < VT; ++ve) acc[q][e][ve] = ret_mfma(vv.v[ve], t < n ? kv.v[e] * w : 0.f, acc[q][e][ve]);
         }
     }
-    float* out = starts + (chunk.place * heads + h) * DIM * VDIM + v0 + 4 * VT * g;
+    float* out = starts + ((size_t)blockIdx.y * heads + h) * DIM * VDIM + v0 + 4 * VT * g;
 #pragma unroll
     for (int q = 0; q < DQ; ++q)
 #pragma unroll
@@ -163,19 +176,21 @@ __global__ __launch_bounds__(256) void retention_local_kernel(const T* __restric
             }
 }
 
-// One thread for four elements of (sequence, head, dim, vdim): starts holds L_c and leaves as S_c; the next L is on its way.
+// One thread for four elements of (sequence, head, dim, vdim): starts holds L_c of the window's places and leaves as S_c, the state is
+// left as it is behind the window's last chunk; the next L is on its way.
 __global__ void retention_starts_kernel(float* __restrict__ starts, float* __restrict__ state, const float* __restrict__ decay,
                                         const int* __restrict__ seq_slot, const int* __restrict__ seq_new, const int* __restrict__ cu_new,
-                                        int heads, int per_head) {
+                                        int place0, int places, int heads, int per_head) {
     const int e = (blockIdx.x * blockDim.x + threadIdx.x) * 4, b = blockIdx.y;
     if (e >= heads * per_head) return;
-    const int n_new = seq_new[b];
-    if (n_new <= 0) return;
+    const int first = cu_new[b] / RET_CHUNK + b;         // the sequence's first place
+    const int before = max(place0 - first, 0);            // chunks of earlier windows
+    const int n_new = seq_new[b] - before * RET_CHUNK, chunks = min((n_new + RET_CHUNK - 1) / RET_CHUNK, place0 + places - first - before);
+    if (n_new <= 0 || chunks <= 0) return;
     const float g = decay[e / per_head], whole = powf(g, (float)RET_CHUNK);
     const size_t stride = (size_t)heads * per_head;
     float4* st = reinterpret_cast<float4*>(state + (size_t)seq_slot[b] * stride + e);
-    float* at = starts + (cu_new[b] / RET_CHUNK + b) * stride + e;
-    const int chunks = (n_new + RET_CHUNK - 1) / RET_CHUNK;
+    float* at = starts + (first + before - place0) * stride + e;
     constexpr int AHEAD = 4;
     float4 s = *st, local[AHEAD];
 #pragma unroll
@@ -199,14 +214,15 @@ __global__ void retention_starts_kernel(float* __restrict__ starts, float* __res
 template <typename T, int DIM, int VT>
 __global__ __launch_bounds__(256) void retention_out_kernel(const T* __restrict__ rows, int row_stride, int v_off, int g_off,
                                                             const float* __restrict__ qk, const float* __restrict__ decay, float eps,
-                                                            const int* __restrict__ seq_new, const int* __restrict__ cu_new, int heads, int act,
-                                                            const float* __restrict__ starts, T* __restrict__ out, int joined, float* __restrict__ raw) {
+                                                            const int* __restrict__ seq_new, const int* __restrict__ cu_new, int n_seqs, int place0,
+                                                            int heads, int act, const float* __restrict__ starts, T* __restrict__ out, int joined,
+                                                            float* __restrict__ raw) {
     constexpr int VDIM = 64 * VT, TT = RET_CHUNK / 16;
     __shared__ float power[RET_CHUNK + 1];
     __shared__ __attribute__((aligned(16))) float P[RET_CHUNK][RET_CHUNK + 4];
     __shared__ float squares[4][RET_CHUNK];
     const int h = blockIdx.x;
-    const RetChunk chunk(seq_new, cu_new, blockIdx.z, blockIdx.y);
+    const RetChunk chunk(seq_new, cu_new, n_seqs, place0 + blockIdx.y);
     const int n = chunk.n;
     if (n <= 0) return;
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, r = lane % 16, g = lane / 16, v0 = wave * 16 * VT;
@@ -241,7 +257,7 @@ __global__ __launch_bounds__(256) void retention_out_kernel(const T* __restrict_
     float from_start[TT];
 #pragma unroll
     for (int i = 0; i < TT; ++i) from_start[i] = power[16 * i + r + 1];
-    const float* start = starts + (chunk.place * heads + h) * DIM * VDIM + v0 + VT * r;
+    const float* start = starts + ((size_t)blockIdx.y * heads + h) * DIM * VDIM + v0 + VT * r;
 #pragma unroll 2
     for (int d = 0; d < DIM; d += 16) {
         RetRun<4> qv[TT];
@@ -348,23 +364,31 @@ PALM_API int palm_retention_matrix_chunk(int dim, int vdim, int max_new) {
     return (dim == 64 || dim == 128) && (vdim == 128 || vdim == 256) && max_new >= 16 ? RET_CHUNK : 0;
 }
 
+// Places of chunks that the starts have room for (as many as n_tokens tokens of n_seqs sequences need, up to RET_ROOM bytes).
+PALM_API int palm_retention_places(int heads, int dim, int vdim, int n_tokens, int n_seqs) {
+    const long long room = max(1ll, RET_ROOM / ((long long)heads * dim * vdim * (long long)sizeof(float)));
+    return (int)min(min(room, 65535ll), (long long)n_tokens / RET_CHUNK + n_seqs);
+}
+
 template <typename T, int DIM, int VT>
 static void launch_retention_chunks(hipStream_t stream, const T* rows, int row_stride, int v_off, int g_off, const float* qk, const float* decay,
-                                    float eps, float* state, const int* seq_slot, const int* seq_new, const int* cu_new, int n_seqs, int max_new,
+                                    float eps, float* state, const int* seq_slot, const int* seq_new, const int* cu_new, int n_seqs, int n_tokens,
                                     int heads, float* starts, T* out, int act, int joined, float* raw) {
-    const dim3 grid(heads, (max_new + RET_CHUNK - 1) / RET_CHUNK, n_seqs);
-    retention_local_kernel<T, DIM, VT><<<grid, 256, 0, stream>>>(rows, row_stride, v_off, qk, decay, seq_new, cu_new, heads, act, starts);
-    const int per_head = DIM * 64 * VT;
-    retention_starts_kernel<<<dim3((heads * per_head / 4 + 255) / 256, n_seqs), 256, 0, stream>>>(starts, state, decay, seq_slot, seq_new, cu_new,
-                                                                                                   heads, per_head);
-    retention_out_kernel<T, DIM, VT><<<grid, 256, 0, stream>>>(rows, row_stride, v_off, g_off, qk, decay, eps, seq_new, cu_new, heads, act, starts,
-                                                               out, joined, raw);
+    const int per_head = DIM * 64 * VT, all = n_tokens / RET_CHUNK + n_seqs, window = palm_retention_places(heads, DIM, 64 * VT, n_tokens, n_seqs);
+    for (int place0 = 0; place0 < all; place0 += window) {
+        const int places = min(window, all - place0);
+        const dim3 grid(heads, places);
+        retention_local_kernel<T, DIM, VT><<<grid, 256, 0, stream>>>(rows, row_stride, v_off, qk, decay, seq_new, cu_new, n_seqs, place0, heads, act, starts);
+        retention_starts_kernel<<<dim3((heads * per_head / 4 + 255) / 256, n_seqs), 256, 0, stream>>>(starts, state, decay, seq_slot, seq_new, cu_new,
+                                                                                                       place0, places, heads, per_head);
+        retention_out_kernel<T, DIM, VT><<<grid, 256, 0, stream>>>(rows, row_stride, v_off, g_off, qk, decay, eps, seq_new, cu_new, n_seqs, place0, heads,
+                                                                   act, starts, out, joined, raw);
+    }
 }
 
 // qk: room for n_tokens * heads * 2 * pad floats (the rotated q and k; pad = palm_retention_pad(dim)).  chunk == 0: every sequence's run in one block
 // per head.  Else `starts` holds n_seqs * max_chunks * heads * dim * vdim floats, max_chunks = ceil(max_new / chunk); with
-// matrix != 0 (chunk = palm_retention_matrix_chunk, rows and offsets of whole 16-byte pieces) (n_tokens / chunk + n_seqs) *
-// heads * dim * vdim.
+// matrix != 0 (chunk = palm_retention_matrix_chunk, rows and offsets of whole 16-byte pieces) palm_retention_places * heads * dim * vdim.
 PALM_API int palm_retention_pad(int dim) { return dim <= 32 ? 32 : dim <= 64 ? 64 : dim <= 128 ? 128 : 256; }
 
 PALM_API int palm_retention(hipStream_t stream, const void* qkvg, int dtype, int row_stride, int q_off, int k_off, int v_off,
@@ -387,7 +411,7 @@ PALM_API int palm_retention(hipStream_t stream, const void* qkvg, int dtype, int
     const int pad = palm_retention_pad(dim);
     const long long rot_threads = (long long)n_tokens * heads * pad;
 #define RET_MATRIX(D, V) launch_retention_chunks<T, D, V / 64>(stream, (const T*)qkvg, row_stride, v_off, g_off, qk, decay, eps, state, seq_slot, seq_new, \
-            cu_new, n_seqs, max_new, heads, starts, (T*)out, act, joined, raw)
+            cu_new, n_seqs, n_tokens, heads, starts, (T*)out, act, joined, raw)
 #define RET_CASE(D) linear_recurrence_sized<T, D, false>(stream, n_seqs, max_new, chunk, starts, nullptr, (const T*)qkvg, row_stride, v_off, g_off, \
             PreparedRows<D, 2>{qk, heads}, \
             decay, nullptr, eps, state, seq_slot, seq_new, cu_new, heads, dim, vdim, (T*)out, act, joined, raw)

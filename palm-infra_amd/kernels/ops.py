@@ -889,6 +889,7 @@ _RECURRENT_SIGNATURES = {
                        c_float, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
                        c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int],
     "palm_retention_matrix_chunk": [c_int, c_int, c_int],
+    "palm_retention_places": [c_int, c_int, c_int, c_int, c_int],
     "palm_retention_pad": [c_int],
     "palm_joined_norm_gate": [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
 }
@@ -1097,7 +1098,7 @@ def retention(qkvg: torch.Tensor, heads: int, dim: int, vdim: int, decay: torch.
     rotated = torch.empty((n, heads, 2, recurrent().palm_retention_pad(dim)), dtype=F32, device=qkvg.device)
     starts = None
     if chunk:
-        places = n // chunk + ctx.n_seqs if matrix else ctx.n_seqs * -(-ctx.max_new // chunk)
+        places = recurrent().palm_retention_places(heads, dim, vdim, n, ctx.n_seqs) if matrix else ctx.n_seqs * -(-ctx.max_new // chunk)
         starts = torch.empty((places, heads, dim, vdim), dtype=F32, device=qkvg.device)
     g_off = col0 + 2 * heads * dim + heads * vdim
     library.call(recurrent(), "palm_retention", _stream(), _p(qkvg), _code(qkvg, "retention"), qkvg.shape[1], col0, col0 + heads * dim,

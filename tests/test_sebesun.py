@@ -366,6 +366,35 @@ def test_retention_in_chunks_on_the_matrix_cores(dtype, dk, dv):
         assert (results[0].float() - results[1].float()).abs().max() < tol * max(1.0, float(want[kind].abs().max()))
 
 
+def test_retention_starts_have_bounded_room():
+    from palm_infra_amd.kernels import ops
+    places = ops.recurrent().palm_retention_places
+    assert places(16, 128, 256, 32768, 1) * 16 * 128 * 256 * 4 <= 128 << 20
+    assert places(16, 128, 256, 700, 3) == 700 // 64 + 3 and places(1, 64, 128, 5, 1) == 1
+    assert places(4096, 128, 256, 300, 2) == 1
+
+
+@gpu
+@pytest.mark.parametrize("lengths", [[700, 1, 500, 130], [1500], [20] * 70 + [1, 200]])
+def test_retention_in_windows_of_chunks(lengths):
+    """More chunks than the starts have room for: the state crosses from one window to the next, within a sequence and between
+    sequences; against the walk token by token."""
+    from palm_infra_amd.kernels import ops
+    torch.manual_seed(len(lengths))
+    H, dk, dv, T = 64, 128, 256, sum(lengths)
+    assert ops.recurrent().palm_retention_places(H, dk, dv, T, len(lengths)) == 16 < T // 64 + len(lengths)
+    rows = (torch.randn(T, H * (2 * dk + 2 * dv)) * 0.5).bfloat16().cuda()
+    decay, state0 = torch.linspace(0.9, 0.999, H).cuda(), torch.randn(len(lengths), H, dk, dv).cuda()
+    results = []
+    for chunk in (None, 0):
+        state = state0.clone()
+        y = ops.retention(rows, H, dk, dv, decay, dk ** -0.5, 1e-6, state, _step_context([0] * len(lengths), lengths), chunk=chunk)
+        results.append((y.float(), state))
+    (got, left), (want, walked) = results
+    # one rounding to bfloat16 each; 32-bit sums in another order
+    assert (got - want).abs().max() < 2.0 ** -7 * float(want.abs().max()) and (left - walked).abs().max() < 1e-4
+
+
 @gpu
 @pytest.mark.parametrize("dk,dv", [(64, 128), (128, 256)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
