@@ -679,6 +679,35 @@ def test_top_k_in_slices_draws_what_one_block_draws(ops, V, k):
         assert ops.sample(lg, u, T, k, top_p, min_p).tolist() == want.tolist(), (T, top_p, min_p)
 
 
+@pytest.mark.parametrize("V,k", [(16384, 2), (16388, 128), (151936, 50), (151936, 128)])
+def test_top_k_in_slices_where_logits_are_equal(ops, V, k):
+    """Rows whose cut by value alone leaves more candidates than there is room for: all equal, all masked but a few (one, fewer than
+    k, more than k), two values, sorted both ways.  The same tokens as the kernel that takes a row whole, every slice within its
+    room."""
+    from palm_infra_amd.kernels import library
+    masked = torch.full((3, V), float("-inf"))
+    for r, allowed in enumerate((1, 40, 1000)):
+        where = torch.randperm(V, generator=torch.Generator().manual_seed(r))[:allowed]
+        masked[r, where] = rand(1, V, seed=r)[0, where]
+    two = (rand(1, V, seed=9) > 0).float()
+    rising = torch.arange(V, dtype=torch.float32)[None] / V
+    lg = torch.cat([masked, torch.zeros(1, V), torch.full((1, V), float("-inf")), two, rising, rising.flip(1)]).to(DEV)
+    n = lg.shape[0]
+    u = torch.rand(n, generator=torch.Generator().manual_seed(k)).to(DEV)
+
+    def whole(lg, u):
+        out = torch.empty(lg.shape[0], dtype=torch.int32, device=DEV)
+        library.call(ops.core(), "palm_sample", ops._stream(), lg.data_ptr(), lg.shape[0], V, u.data_ptr(), 0.7, k, 0.95, 0.0, out.data_ptr(), None)
+        return out.tolist()
+    needed = ops.core().palm_sample_sliced_work(n, V, 0.7, k)
+    work, out = torch.empty(needed, dtype=torch.uint8, device=DEV), torch.empty(n, dtype=torch.int32, device=DEV)
+    library.call(ops.core(), "palm_sample_sliced", ops._stream(), lg.data_ptr(), n, V, u.data_ptr(), 0.7, k, 0.95, 0.0, out.data_ptr(), work.data_ptr(), needed)
+    assert out.tolist() == whole(lg, u)
+    slices = -(-(V // 4) // 1024)
+    counts = work[n * slices * 512 * 8:].view(torch.int32)
+    assert counts.numel() == n * slices and counts.min() >= min(k, 4) and counts.max() <= 512
+
+
 def test_rows_are_sampled_independently(ops):
     lg = rand(4, 2000, seed=8)
     u = torch.tensor([0.1, 0.5, 0.9, 0.3])
