@@ -788,6 +788,7 @@ constexpr int SLICE_QUADS = 4;                                       // 16-byte 
 constexpr int SLICE = SLICE_THREADS * SLICE_QUADS * 4;
 constexpr int SLICED_TOPK_MAX = 128;                                 // half a slice's threads: the cut stays a tail of the slice
 constexpr int SLICE_CAP = 4 * SLICED_TOPK_MAX;                       // candidates that a slice can hand on (equal or sorted logits: four a thread)
+constexpr int SLICED_ROWS = 512;                                     // rows that share the workspace (80 MB for 151,936 logits)
 constexpr int SLICED_MIN_VOCAB = 16384;                              // (below, the row is a few slices: one block does as well)
 constexpr int SURVIVORS = 1024;
 
@@ -1088,7 +1089,7 @@ PALM_API int palm_sample(hipStream_t stream, const float* logits, int n_rows, in
 // pieces; and the bytes of workspace that it needs then (0: it does not).  From SLICED_MIN_VOCAB on the slices win at any batch.
 PALM_API long long palm_sample_sliced_work(int n_rows, int V, float temperature, int top_k) {
     if (temperature <= 0.f || top_k <= 1 || top_k > SLICED_TOPK_MAX || V < SLICED_MIN_VOCAB || V % 4 != 0 || n_rows < 1 || n_rows > 65535) return 0;
-    return (long long)n_rows * slices_of(V) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int));
+    return (long long)min(n_rows, SLICED_ROWS) * slices_of(V) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int));
 }
 
 PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, float temperature,
@@ -1102,10 +1103,14 @@ PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_r
     PALM_CHECK(uniforms, "sample: a draw needs the uniform numbers");
     const int slices = slices_of(V);
     uint2* cands = (uint2*)work;
-    int* counts = (int*)(cands + (size_t)n_rows * slices * SLICE_CAP);
-    topk_slice_kernel<<<dim3(slices, n_rows), SLICE_THREADS, 0, stream>>>(logits, V, top_k, counts, cands);
-    PALM_LAUNCHED();
-    topk_draw_kernel<<<n_rows, SAMPLE_THREADS, 0, stream>>>(logits, V, uniforms, temperature, top_k, top_p, min_p, counts, cands, slices, out);
-    PALM_LAUNCHED();
+    int* counts = (int*)(cands + (size_t)min(n_rows, SLICED_ROWS) * slices * SLICE_CAP);
+    for (int r0 = 0; r0 < n_rows; r0 += SLICED_ROWS) {
+        const int rows = min(SLICED_ROWS, n_rows - r0);
+        const float* at = logits + (size_t)r0 * V;
+        topk_slice_kernel<<<dim3(slices, rows), SLICE_THREADS, 0, stream>>>(at, V, top_k, counts, cands);
+        PALM_LAUNCHED();
+        topk_draw_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(at, V, uniforms + r0, temperature, top_k, top_p, min_p, counts, cands, slices, out + r0);
+        PALM_LAUNCHED();
+    }
     return 0;
 }

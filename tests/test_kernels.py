@@ -683,7 +683,7 @@ def test_top_k_in_slices_draws_what_one_block_draws(ops, V, k):
 def test_top_k_in_slices_where_logits_are_equal(ops, V, k):
     """Rows whose cut by value alone leaves more candidates than there is room for: all equal, all masked but a few (one, fewer than
     k, more than k), two values, sorted both ways.  The same tokens as the kernel that takes a row whole, every slice within its
-    room."""
+    room, and more rows than share the workspace."""
     from palm_infra_amd.kernels import library
     masked = torch.full((3, V), float("-inf"))
     for r, allowed in enumerate((1, 40, 1000)):
@@ -706,6 +706,11 @@ def test_top_k_in_slices_where_logits_are_equal(ops, V, k):
     slices = -(-(V // 4) // 1024)
     counts = work[n * slices * 512 * 8:].view(torch.int32)
     assert counts.numel() == n * slices and counts.min() >= min(k, 4) and counts.max() <= 512
+    if V == 16388:
+        many = lg.repeat(600 // n + 1, 1)
+        assert ops.core().palm_sample_sliced_work(len(many), V, 0.7, k) == ops.core().palm_sample_sliced_work(512, V, 0.7, k)
+        u = torch.rand(len(many), generator=torch.Generator().manual_seed(5)).to(DEV)
+        assert ops.sample(many, u, 0.7, k, 0.95).tolist() == whole(many, u)
 
 
 def test_rows_are_sampled_independently(ops):
