@@ -167,6 +167,12 @@ static bool big_takes(int M, int N, int K, bool gated) {
            (long long)N * K < (1ll << 31) - 8 * K;
 }
 PALM_API int palm_linear_big_takes(int M, int N, int K, int gated) { return big_takes(M, N, K, gated != 0); }
+// 64-token pieces of a tile, times 16, and into how many ranges of K the last tiles are cut (1: not); 0 where it does not take the product
+PALM_API int palm_linear_big_plan(int M, int N, int K, int gated) {
+    if (!big_takes(M, N, K, gated != 0)) return 0;
+    const BigPlan p = big_plan(M, N, K, gated != 0);
+    return p.nt * 16 + p.shape.split;
+}
 // bytes of workspace for the tiles that are cut (0: none are)
 PALM_API long long palm_linear_big_work(int M, int N, int K, int gated) {
     if (!big_takes(M, N, K, gated != 0)) return 0;

@@ -49,6 +49,7 @@ _SIGNATURES = {
     "palm_linear_big": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_longlong],
     "palm_linear_big_work": [c_int, c_int, c_int, c_int],
     "palm_linear_big_takes": [c_int, c_int, c_int, c_int],
+    "palm_linear_big_plan": [c_int, c_int, c_int, c_int],
     "palm_linear_tile": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int],
     "palm_linear_tile_parts": [c_int, c_int, c_int],
     "palm_argmax": [c_void_p, c_void_p, c_int, c_int, c_void_p],

@@ -306,10 +306,26 @@ def test_linear_tile_against_the_plain_product(ops, M, N, K):
 
 # tiles of 128, 192 and 256 tokens, whole and cut along K; odd and even numbers of stages, the fewest; rows, weight rows and
 # features that end inside a tile; grids that are no multiple of the dies
-@pytest.mark.parametrize("M,N,K,gated", [
+LARGE_TILES = [
     (1, 8, 128, False), (300, 136, 192, False), (257, 264, 320, False), (70, 1040, 1088, False), (190, 520, 4160, False), (250, 2400, 8192, False),
     (570, 4096, 8192, False), (2500, 8200, 192, False), (4096, 4096, 192, False), (4309, 4104, 4160, False),
-    (300, 160, 192, True), (900, 160, 8192, True), (520, 4000, 2048, True), (3000, 5504, 320, True), (4096, 8192, 128, True), (4309, 8208, 4160, True)])
+    (300, 160, 192, True), (900, 160, 8192, True), (520, 4000, 2048, True), (3000, 5504, 320, True), (4096, 8192, 128, True), (4309, 8208, 4160, True),
+    (2073, 8192, 4096, True), (2703, 6144, 2048, True)]
+
+
+def test_every_large_tile_is_among_the_products_below(ops):
+    """Whole and cut, both epilogues, and cut behind a full round of whole tiles."""
+    plans = set()
+    for M, N, K, gated in LARGE_TILES:
+        p = ops.core().palm_linear_big_plan(M, N, K, int(gated))
+        nt, cut = p // 16, p % 16 > 1
+        tiles = -(-M // (64 * nt)) * -(-(N // 2 if gated else N) // (128 if gated else 256))
+        plans |= {(nt, cut, gated), (nt, cut, gated, "behind whole tiles")} if cut and tiles > 256 else {(nt, cut, gated)}
+    assert plans >= {(nt, cut, gated) for nt in (2, 3, 4) for cut in (False, True) for gated in (False, True)}
+    assert plans >= {(3, True, True, "behind whole tiles"), (4, True, True, "behind whole tiles"), (4, True, False, "behind whole tiles")}
+
+
+@pytest.mark.parametrize("M,N,K,gated", LARGE_TILES)
 def test_products_in_large_tiles_against_the_plain_product(ops, M, N, K, gated):
     a, w = rand(M, K, seed=M + K).to(DEV), rand(N, K, seed=N, scale=K ** -0.5).to(DEV)
     ref = a.double() @ w.double().t()
