@@ -429,7 +429,7 @@ def test_attention_kernel_far_keys_page_borders_window_edges_and_the_sink(dtype,
 
 @gpu
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("H,d,dv", [(3, 16, 24), (1, 40, 72), (2, 8, 130), (2, 128, 64), (4, 32, 16)])
+@pytest.mark.parametrize("H,d,dv", [(3, 16, 24), (1, 40, 72), (2, 8, 130), (2, 128, 64), (4, 32, 16), (2, 64, 128), (2, 128, 256)])
 def test_recurrence_options_keep_a_far_write_whole_in_portions_and_in_chunks(dtype, H, d, dv):
     """silu'd inputs, the joined heads normed together with a weight, a sigmoid gate: the kernel against the plain steps.  The
     first token writes a large value under a key that only the last token asks for, through a head that hardly decays; a
