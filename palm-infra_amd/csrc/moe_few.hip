@@ -58,6 +58,11 @@ __device__ inline void few_piece(const bf16_t* w_row, const bf16_t* const (&xr)[
 // (The matrices come in order through one counter of loads: activations read from memory between them would make every wait for
 // them a wait for the rows asked for ahead.)
 constexpr int few_segment(int max_ct) { return max_ct == 1 ? 2048 : 512; }
+// Whether blocks begin their walks at chunks of their own: in step they meet on a few of memory's channels, out of step they share
+// less of what they read.  Us in step and apart, 32 experts of 2,048 x 4,096: 4 rows 118 and 125, 8 rows 156 and 156, 12 187 and 173, 16
+// 198 and 189; 16 gated ones of 2,752 x 4,096: 4 172 and 173, 12 201 and 203, 16 218 and 205; with more rows the sizes that come here
+// (few tiles) are 0 to 3 % faster in step.
+template <int MAX_CT> __device__ inline bool few_apart(int n) { return MAX_CT == 1 && n > 8; }
 constexpr int FEW_PAD = 8;                         // elements between a segment's end and the next row: rows begin in different banks
 
 template <bool GATED, int MAX_CT>
@@ -103,9 +108,7 @@ __global__ __launch_bounds__(FEW_UP_WAVES * WAVE) void moe_few_up_kernel(const b
             const int k1 = min(width, k0 + segment), len = k1 - k0;
             // the first chunk's matrix rows are on their way while the activations go to LDS
             constexpr int CHUNK = 32 * FEW_STEPS;
-            // blocks begin at chunks of their own: in step they meet on a few of memory's channels (16 rows, 32 experts of 2,048 x
-            // 4,096, a layer: 206 -> 196 us)
-            const int chunks = (len + CHUNK - 1) / CHUNK, turn = (3 * e + blockIdx.y + 2 * wave) % chunks;
+            const int chunks = (len + CHUNK - 1) / CHUNK, turn = few_apart<MAX_CT>(ch.n) ? (3 * e + blockIdx.y + 2 * wave) % chunks : 0;
             auto chunk_at = [&](int i) { i += turn; return k0 + (i < chunks ? i : i - chunks) * CHUNK; };
             bf16x8 wf[MATS][FEW_STEPS];
             auto read = [&](int k, bf16x8 (&to)[MATS][FEW_STEPS]) {
@@ -249,7 +252,7 @@ __global__ __launch_bounds__(FEW_DOWN_WAVES * WAVE) void moe_few_down_kernel(con
     const int items = of_experts + (shared_ff + FEW_PIECE - 1) / FEW_PIECE;
     float* mine = sums + wave * n * 16;
     // (the pieces in a turn of the block's own, as above)
-    const int turn = (int)((5u * blockIdx.x) % (unsigned)items);
+    const int turn = few_apart<MAX_CT>(n) ? (int)((5u * blockIdx.x) % (unsigned)items) : 0;
     for (int at = plane + planes * wave; at < items; at += planes * FEW_DOWN_WAVES) {
         const int i = at + turn < items ? at + turn : at + turn - items;
         const bool is_shared = i >= of_experts;
