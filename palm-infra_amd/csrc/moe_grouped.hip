@@ -262,41 +262,52 @@ __global__ void moe_combine_kernel(const TY* __restrict__ y, const int* __restri
     }
 }
 
+struct MoeSizes {
+    long long n_pairs;
+    int experts, width, ff;
+    bool gated, aligned;         // aligned: h, gate_up and down start on 16 bytes
+};
+
 // Rows of a tile for experts with n_pairs / experts rows each: what takes the fewest stages' time (0.75, 0.87, 1.13 and 1.42 us
-// for 64 to 256 rows, a full chip) for an expert with somewhat more rows than the mean, a second tile for a few experts costing
-// almost a whole round.  Measured, us, 32 experts of 2,048 x 4,096, tiles of 64 / 128 / 192 / 256 rows: mean 25: 212 / 230 / 272 /
+// for 64 to 256 rows) for an expert with somewhat more rows than the mean, a second tile for a few experts costing
+// almost a whole round.  Tiles that do not fill the chip run side by side, so few or small experts take low ones: 16 experts of 256 x
+// 512 with 125 rows each 43 us in tiles of 192 rows, 29 in tiles of 64.  Measured with a full chip, us, 32 experts of 2,048 x 4,096, tiles of 64 / 128 / 192 / 256 rows: mean 25: 212 / 230 / 272 /
 // 317, 75: 288 / 231 / 244 / 275, 106: - / 308 / 262 / 312, 187: - / 363 / 378 / 303, 256: - / 484 / 440 / 454, 625: 1,247 / 909 /
 // 849 / 831.
-static int big_tile_of(long long n_pairs, int experts) {
-    const double mean = (double)n_pairs / experts, rows = mean + 2.25 * sqrt(mean);
+static int big_tile_of(const MoeSizes& s) {
+    const double mean = (double)s.n_pairs / s.experts, rows = mean + 2.25 * sqrt(mean), in_use = (double)min((long long)s.experts, s.n_pairs);
     const double stage_us[4] = {0.75, 0.87, 1.13, 1.42};
     int best = 64;
     double best_cost = 1e300;
     for (int nt = 1; nt <= 4; ++nt) {
-        const double cost = ceil(rows / (64 * nt)) * stage_us[nt - 1];
+        const double tiles = in_use * ceil(rows / (64 * nt));
+        auto rounds = [&](int features, int of_tile) { return ceil(tiles * ((features + of_tile - 1) / of_tile) / 256.0); };
+        const double cost = (rounds(s.ff, s.gated ? BIG_FEAT / 2 : BIG_FEAT) * s.width + rounds(s.width, BIG_FEAT) * s.ff) * stage_us[nt - 1];
         if (cost < best_cost) { best_cost = cost; best = 64 * nt; }
     }
     return best;
 }
-// Whether the tiles cross LDS: rows in whole stages that start on 16 bytes, offsets from a matrix's first row of 32 bits.
-static bool big_tiles(long long n_pairs, int experts, int width, int ff, bool aligned) {
-    const long long rows = n_pairs + 256ll * (experts + 1), inner = max(width, ff);
-    return aligned && width % BIG_K == 0 && ff % BIG_K == 0 && rows * inner < (1ll << 31) && 2ll * ff * width < (1ll << 31);
+// Whether the tiles cross LDS: rows in whole stages that start on 16 bytes, offsets from a matrix's first row of 32 bits, and, for
+// few rows an expert, first matrices that fill half a tile (512 experts of 64 x 512, four a row, 300 rows: 59 us through LDS, 50 by
+// fragments).
+static bool big_tiles(const MoeSizes& s) {
+    const long long rows = s.n_pairs + 256ll * (s.experts + 1), inner = max(s.width, s.ff);
+    return s.aligned && s.width % BIG_K == 0 && s.ff % BIG_K == 0 && rows * inner < (1ll << 31) && 2ll * s.ff * s.width < (1ll << 31) &&
+           ((s.gated ? 2 : 1) * s.ff >= BIG_FEAT / 2 || s.n_pairs >= 40ll * s.experts);
 }
-static int tile_of(long long n_pairs, int experts, int width, int ff, bool aligned) {
-    return big_tiles(n_pairs, experts, width, ff, aligned) ? big_tile_of(n_pairs, experts) : GT_TOKENS;
+static int tile_of(const MoeSizes& s) { return big_tiles(s) ? big_tile_of(s) : GT_TOKENS; }
+PALM_API int palm_moe_tile_tokens(int n_pairs, int experts, int width, int ff, int gated, int aligned) {
+    return tile_of(MoeSizes{n_pairs, experts, width, ff, gated != 0, aligned != 0});
 }
-// aligned: h, gate_up and down start on 16 bytes
-PALM_API int palm_moe_tile_tokens(int n_pairs, int experts, int width, int ff, int aligned) { return tile_of(n_pairs, experts, width, ff, aligned != 0); }
 
 // chosen, weight [n, top]; h bfloat16 [n, width]; gate_up bfloat16 [experts, 2 ff, width] (the plain forms: [experts, ff, width], up
 // rows alone); add0, add1: null or bfloat16 rows [n, width]; down bfloat16 [experts, width, ff].
 // With ids [n] chosen is a table [vocab, top] of which every token takes its id's row, and weight may be null (1 / top).
-// Room, with tile = palm_moe_tile_tokens(n top, experts, width, ff, aligned), max_tiles = ceil(n top / tile) + experts and
+// Room, with tile = palm_moe_tile_tokens(n top, experts, width, ff, gated, aligned), max_tiles = ceil(n top / tile) + experts and
 // slots = max_tiles * tile: plan: (max_tiles + slots + n top + 1) ints; mid: slots * ff bfloat16; y: slots * width, bfloat16 or with y32
 // (for tiles that cross LDS) float32.  planes: n_planes float32 rows [n, width] to add.  out float32 [n, width].
-PALM_API int palm_moe_grouped_in_tiles(long long n_pairs, int experts, int width, int ff, int aligned) {
-    return experts <= PLAN_MAX_EXPERTS && big_tiles(n_pairs, experts, width, ff, aligned != 0);
+PALM_API int palm_moe_grouped_in_tiles(int n_pairs, int experts, int width, int ff, int gated, int aligned) {
+    return experts <= PLAN_MAX_EXPERTS && big_tiles(MoeSizes{n_pairs, experts, width, ff, gated != 0, aligned != 0});
 }
 PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gate_up, const void* down, const int* chosen,
                               const float* weight, int n_tokens, int top, int experts, int width, int ff, int* plan, void* mid, void* y,
@@ -313,10 +324,11 @@ PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gat
     if (n_tokens == 0) return 0;
     const long long n_pairs = (long long)n_tokens * top;
     PALM_CHECK(n_pairs < (1ll << 30), "moe_grouped: %lld pairs are more than one launch takes", n_pairs);
-    const bool aligned = ((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down) % 16 == 0, big = big_tiles(n_pairs, experts, width, ff, aligned);
+    const MoeSizes sizes{n_pairs, experts, width, ff, expert_is_gated(form), ((uintptr_t)h | (uintptr_t)gate_up | (uintptr_t)down) % 16 == 0};
+    const bool big = big_tiles(sizes);
     PALM_CHECK(big || !y32, "moe_grouped: 32-bit results come from tiles that cross LDS (sizes of whole stages, rows that start on 16 bytes)");
     PALM_CHECK(n_planes == 0 || (n_planes > 0 && planes && (uintptr_t)planes % 16 == 0), "moe_grouped: %d planes to add", n_planes);
-    const int tile = tile_of(n_pairs, experts, width, ff, aligned);
+    const int tile = tile_of(sizes);
     const int max_tiles = (int)((n_pairs + tile - 1) / tile) + experts;
     int* tile_expert = plan;
     int* slot_pair = tile_expert + max_tiles;

@@ -912,10 +912,10 @@ _FEEDFORWARD_SIGNATURES = {
                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "palm_moe_few_planes": [c_int],
     "palm_moe_route_table": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p],
-    "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int, c_int],
+    "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int, c_int, c_int],
     "palm_moe_grouped": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                          c_void_p, c_void_p, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int],
-    "palm_moe_grouped_in_tiles": [c_longlong, c_int, c_int, c_int, c_int],
+    "palm_moe_grouped_in_tiles": [c_int, c_int, c_int, c_int, c_int, c_int],
     "palm_gather_rows": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
     "palm_scatter_add": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p],
     "palm_activation": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_longlong],
@@ -2008,7 +2008,7 @@ def moe_grouped_pays(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
     if n <= GROUPED_FROM or not moe_grouped_serves(h, gate_up, ff) or down.dtype != BF16:
         return False
     experts = down.shape[0] // width
-    if not feedforward().palm_moe_grouped_in_tiles(n * top, experts, width, ff, _starts_on_16(h, gate_up, down)):
+    if not feedforward().palm_moe_grouped_in_tiles(n * top, experts, width, ff, expert_rows(form) > 1, _starts_on_16(h, gate_up, down)):
         return False
     tiles = min(experts, n * top) * (-(-expert_rows(form) * ff // 256) + -(-width // 256))
     return n > GROUPED_SURELY_FROM or tiles >= (GROUPED_TILES_SHARED if shared else GROUPED_TILES)
@@ -2037,7 +2037,7 @@ def moe_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chos
         n_planes = planes.shape[0] if planes.dim() == 3 else 1
         _need(planes.shape[-2:] == h.shape and planes.dim() in (2, 3) and planes.dtype == F32 and planes.is_contiguous(), f"{what}: planes {planes.dtype} "
               f"{tuple(planes.shape)} for rows {tuple(h.shape)}")
-    tile = feedforward().palm_moe_tile_tokens(n * top, experts, width, ff, aligned)
+    tile = feedforward().palm_moe_tile_tokens(n * top, experts, width, ff, expert_rows(form) > 1, aligned)
     max_tiles = (n * top + tile - 1) // tile + experts
     slots = max_tiles * tile
     plan = torch.empty((max_tiles + slots + n * top + 1,), dtype=torch.int32, device=h.device)

@@ -165,11 +165,22 @@ def test_which_steps_go_through_the_grouped_products():
         h = torch.empty(n * W + 8, dtype=dt)[offset:offset + n * W].view(n, W)
         return ops.moe_grouped_pays(h, torch.empty(E * ops.expert_rows(form) * F, W, dtype=dt), torch.empty(E * W, F, dtype=dt), F, top, form, shared)
     assert pays(97, 64, 128) and pays(128, 4096, 64) and not pays(96, 64, 128)
-    assert pays(17, 2048, 64, E=22, top=4) and not pays(17, 2048, 64, E=21, top=4)          # 198 and 189 tiles
-    assert not pays(17, 2048, 64, E=22, top=1)                                               # at most seventeen experts in use
-    assert not pays(17, 2048, 64, E=22, top=4, shared=True) and pays(17, 2048, 64, E=36, top=4, shared=True)
+    assert pays(17, 2048, 128, E=22, top=4) and not pays(17, 2048, 128, E=21, top=4)          # 198 and 189 tiles
+    assert not pays(17, 2048, 128, E=22, top=1)                                               # at most seventeen experts in use
+    assert not pays(17, 2048, 128, E=22, top=4, shared=True) and pays(17, 2048, 128, E=36, top=4, shared=True)
     assert pays(17, 1024, 512, E=32, top=4) and pays(17, 1024, 512, E=32, top=4, form="gated_silu")
-    assert not pays(16, 2048, 64, E=22, top=4) and not pays(97, 72, 128) and not pays(97, 64, 40) and not pays(97, 64, 128, dt=torch.float32)
+    assert not pays(16, 2048, 128, E=22, top=4) and not pays(97, 72, 128) and not pays(97, 64, 40) and not pays(97, 64, 128, dt=torch.float32)
     # what the grouped products refuse or do from memory stays with the kernels for few rows: more experts, rows that start on no 16 bytes
-    assert pays(97, 64, 64, E=512, top=4) and not pays(97, 64, 64, E=513, top=4)
+    assert pays(97, 64, 128, E=512, top=4) and not pays(97, 64, 128, E=513, top=4)
+    assert not pays(97, 64, 64, E=512, top=4) and pays(97, 64, 64, E=512, top=4, form="gated_silu")      # first matrices of a quarter of a tile
     assert not pays(97, 64, 128, offset=1) and pays(97, 64, 128, offset=8)
+
+
+def test_tiles_of_the_grouped_products():
+    """Low tiles as long as all run side by side, one tile an expert where the chip is full, fragments for narrow first matrices of few rows."""
+    from palm_infra_amd.kernels import ops
+    tile = lambda pairs, E, W, F, gated=0, aligned=1: ops.feedforward().palm_moe_tile_tokens(pairs, E, W, F, gated, aligned)
+    assert tile(2000, 16, 512, 256) == 64 and tile(4000, 16, 512, 256) == 64          # 125 and 250 rows each
+    assert [tile(4 * n, 32, 4096, 2048) for n in (200, 600, 850, 1500)] == [64, 128, 192, 256]
+    assert tile(1200, 512, 512, 64) == tile(1200, 512, 512, 64, aligned=0) == 64 and not ops.feedforward().palm_moe_grouped_in_tiles(1200, 512, 512, 64, 0, 1)
+    assert ops.feedforward().palm_moe_grouped_in_tiles(1200, 512, 512, 64, 1, 1) and ops.feedforward().palm_moe_grouped_in_tiles(320, 8, 512, 64, 0, 1)

@@ -586,7 +586,7 @@ def test_direct_queries_through_the_key_matrix_and_cache_rows_in_one_launch(dtyp
 @gpu
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,top,W,F,shared", [(6, 2, 48, 24, 40), (5, 1, 64, 32, 32), (4, 4, 40, 16, None), (9, 5, 50, 7, 11), (33, 3, 72, 40, 8), (7, 2, 264, 136, 64),
-                                             (6, 2, 64, 128, 192), (36, 4, 2048, 64, 128)])
+                                             (6, 2, 64, 128, 192), (36, 4, 2048, 128, 128)])
 def test_table_experts_for_few_rows_and_many(dtype, E, top, W, F, shared):
     """The part alone, with the step's token ids choosing: one row, a few (the shared expert rides along), a decode batch's
     and a prompt's; also when all tokens choose the same experts and when an expert is chosen by nobody."""
@@ -818,8 +818,8 @@ def test_a_recorded_step_whose_experts_are_grouped(tmp_path):
     """Nineteen sequences decode together, padded to twenty-four rows, through experts whose tiles take the grouped products in a
     recorded step, the shared expert beside them: several replays, with other work between them, against the plain implementation."""
     from palm_infra_amd.engine import Engine, StepEntry
-    raw = S.model(97, 2048, 1e-5, [S.layer(S.attention(4, 2, 32, 32, 0.2, window=37, rot=(16, 500.0)), S.moe(36, 4, 64, shared=128)),
-                                   S.layer(S.attention(2, 2, 32, 32, 0.2), S.moe(40, 2, 64))])
+    raw = S.model(97, 2048, 1e-5, [S.layer(S.attention(4, 2, 32, 32, 0.2, window=37, rot=(16, 500.0)), S.moe(36, 4, 128, shared=128)),
+                                   S.layer(S.attention(2, 2, 32, 32, 0.2), S.moe(40, 2, 128))])
     eng = Engine.from_dir(S.write_model(raw, 31, tmp_path, "bfloat16"), dtype="bfloat16", max_tokens=4096)
     rows = torch.empty((24, 2048), dtype=torch.bfloat16, device="cuda")
     assert not any(b.feed_forward.takes_few(rows, b.feed_forward.shared is not None) for b in eng.model.layers)
