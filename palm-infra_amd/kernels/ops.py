@@ -486,26 +486,33 @@ def linear_mid(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: 
 
 BIG_FROM = 320              # rows from which the kernel of large tiles may serve a product
 BIG_GATED_FROM = 500
-BIG_LONG_K = 8192
-BIG_REST = 90               # tiles
+BIG_LONG_K, BIG_LONGEST_K = 8192, 16384
+BIG_ROUNDS = 8
 
 
 def big_pays(M: int, N: int, K: int, gated: bool = False) -> bool:
     """Whether a prompt's product of bfloat16 operands goes through the kernel of large tiles (linear_big.hip) instead of the
-    library.  Measured from 260 to 13,331 rows at the shapes of the named models (the kernel some 1.35 PFLOP/s where the chip is full,
-    the library 0.7 to 1.5):
+    library.  Measured at 24 shapes of 2,048 to 51,200 weight rows, K from 2,048 to 28,672, each with 25 to 32 numbers of rows from 257
+    to 13,331 (own time over the library's; where tiles fill whole rounds of the compute units the library is the faster one by 2 to
+    12 %, elsewhere it often takes a poor tile).
 
-    gated (the activation in the kernel, against the library and the activation's pass): from 500 rows on, 0.95 to 1.40 times as
-    fast, 1.08 in the geometric mean; below 0.88 to 0.96.
-    inner sizes from 8,192 on: 0.94 to 1.97 times as fast, 1.17 in the mean (4,309 x 4,096, K = 12,288: 316 us and 623): the
-    library's choice of tile is often a poor one there.  (At 260 rows 0.81 to 1.54.)
-    other products: 0.89 to 1.40, 0.99 in the mean, so the library keeps them, but where tiles of 256 x 256 would fill the chip once
-    or more and then leave up to a third of it busy: those last tiles are cut along K here (7,000 x 7,168, K = 5,120: 372 us and
-    494; 1.08 in the mean of such sizes)."""
+    gated (the activation in the kernel, against the library and the activation's pass): from 500 rows on, 0.92 in the geometric mean,
+    1.05 at worst.
+    other products, by the rounds that tiles of 256 x 256 make on 256 compute units:
+      one to eight full rounds and up to 0.3 of another (inner sizes from 8,192 on: 0.68), whose tiles are cut along K here: 4,309 x
+      4,096, K = 12,288 (1.06 rounds) 0.49, 7,000 x 7,168, K = 5,120 (3.06) 0.79; 0.89 in the mean, 1.18 at worst
+      0.55 to 0.72 of a round with an inner size from 8,192 on: a third of the chip is idle there, the tiles are smaller or cut here
+      (2,603 x 4,096, K = 16,384: 0.51); 0.97 in the mean, 1.07 at worst
+      inner sizes beyond 16,384 whatever the rounds: 0.47 to 1.21, 0.76 in the mean
+    0.84 in the mean where this says yes (243 of 766 products); 45 lose more than 2 % to the library."""
     if M < (BIG_GATED_FROM if gated else BIG_FROM) or not core().palm_linear_big_takes(M, N, K, int(gated)):
         return False
-    tiles = -(-M // 256) * -(-N // 256)
-    return gated or K >= BIG_LONG_K or (tiles > COMPUTE_UNITS and 0 < tiles % COMPUTE_UNITS <= BIG_REST)
+    rounds = -(-M // 256) * -(-N // 256) / COMPUTE_UNITS
+    if gated or K > BIG_LONGEST_K:
+        return True
+    if rounds <= 1:
+        return K >= BIG_LONG_K and 0.55 < rounds <= 0.72
+    return rounds <= BIG_ROUNDS and 0 < rounds % 1 <= (0.68 if K >= BIG_LONG_K else 0.3)
 
 
 def linear_big(a: torch.Tensor, w: torch.Tensor, gated: bool = False) -> torch.Tensor:

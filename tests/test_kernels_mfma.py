@@ -345,6 +345,18 @@ def test_products_in_large_tiles_refuse_what_does_not_fit(ops):
             ops.linear_big(rand(M, K).to(DEV), rand(N, K).to(DEV), gated=gated)
 
 
+def test_which_products_of_prompts_take_large_tiles(ops):
+    pays = ops.big_pays
+    assert pays(500, 24576, 4096, True) and not pays(499, 24576, 4096, True)
+    # a part of a round behind whole ones, short of whole rounds, whole rounds, many rounds
+    assert pays(4309, 4096, 4096) and pays(4309, 4096, 12288) and pays(7000, 7168, 5120)
+    assert not pays(7885, 4096, 4096) and not pays(4096, 4096, 4096) and not pays(8192, 4096, 16384) and not pays(8941, 24576, 4096)
+    assert pays(10000, 4096, 12288) and not pays(10000, 4096, 4096)                     # half of a round: for long inner sizes
+    # less than a round: long inner sizes that leave a third of the chip idle; the longest whatever the rounds
+    assert pays(2603, 4096, 16384) and not pays(2603, 4096, 4096) and not pays(600, 4096, 16384) and not pays(320, 4096, 12288)
+    assert pays(320, 5120, 17408) and not pays(319, 5120, 17408)
+
+
 @pytest.mark.parametrize("M", [70, 256, 300])
 @pytest.mark.parametrize("N,K,cut", [(4096, 12288, True), (4096, 4096, True), (1000, 3072, True), (24576, 4096, False),
                                      (4096, 1024, False)])
