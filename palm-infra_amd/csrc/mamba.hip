@@ -101,17 +101,24 @@ __global__ void causal_conv_run_kernel(const T* __restrict__ x, int x_stride, co
     }
 }
 
+// A run takes its 10 us whatever the work, a thread for every token and channel a launch's 6 and then what the work asks (us, one
+// at a time and in runs, four taps, 2,048 channels: 300 tokens 8.6 and 10.5, 600 11 and 11, 2,600 29 and 17; 8,192 channels: 64 tokens
+// 7.7 and 10.5, 200 13 and 11).  The blocks of short sequences beside a long one cost a little too (41 sequences, one of 2,000 tokens,
+// 1,000 channels: 147 and 12).
+constexpr long long CONV_RUN_WORK = 5ll << 18, CONV_RUN_GRID = 8ll << 20;       // elements of the step, and of its grid
+
 PALM_API int palm_causal_conv(hipStream_t stream, const void* x, int dtype, int x_stride, const float* w, const float* bias,
                               float* conv_state, const int* seq_slot, const int* seq_new, const int* cu_new, int n_seqs,
-                              int max_new, int channels, int taps, void* out) {
+                              int max_new, int n_tokens, int channels, int taps, void* out) {
     PALM_CHECK(n_seqs >= 0 && max_new >= 0 && channels > 0, "causal_conv: seqs=%d max_new=%d channels=%d", n_seqs, max_new, channels);
     PALM_CHECK(taps >= 1 && taps <= CONV_MAX_TAPS, "causal_conv: %d taps (1 to %d)", taps, CONV_MAX_TAPS);
     PALM_CHECK(n_seqs <= 65535 && max_new <= 65535, "causal_conv: %d sequences / %d tokens are more than one launch takes", n_seqs, max_new);
     if (n_seqs == 0 || max_new == 0) return 0;
     const int threads = 256, cb = (channels + threads - 1) / threads;
-    // runs of tokens where a sequence has a run's, for the tap counts that models use, rows that start on whole reads
+    // runs of tokens where there is work for them, for the tap counts that models use, rows that start on whole reads
     const size_t read = dtype == PALM_F32 ? 16 : 8;
-    const bool runs = max_new >= CONV_RUN && (taps == 3 || taps == 4) && channels % 4 == 0 && x_stride % 4 == 0 &&
+    const bool much = (long long)n_tokens * channels >= CONV_RUN_WORK || (long long)max_new * n_seqs * channels >= CONV_RUN_GRID;
+    const bool runs = much && max_new >= CONV_RUN && (taps == 3 || taps == 4) && channels % 4 == 0 && x_stride % 4 == 0 &&
                       ((uintptr_t)x | (uintptr_t)out) % read == 0;
     const dim3 run_grid((channels / 4 + threads - 1) / threads, (max_new + CONV_RUN - 1) / CONV_RUN, n_seqs);
     PALM_DTYPE_SWITCH(dtype, T, {

@@ -846,7 +846,7 @@ _MIXER_SIGNATURES = {
                         c_longlong, c_void_p, c_int],
     "palm_xielu": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_longlong],
     "palm_causal_conv": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
-                         c_int, c_int, c_int, c_void_p],
+                         c_int, c_int, c_int, c_int, c_void_p],
     "palm_selective_scan": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "palm_diff_qkv_store": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
@@ -1170,7 +1170,7 @@ def causal_conv(xz: torch.Tensor, channels: int, weight: torch.Tensor, bias: tor
           f"causal_conv: state {tuple(conv_state.shape)} is not float32 [slots, {taps - 1}, {channels}]")
     out = torch.empty((xz.shape[0], channels), dtype=xz.dtype, device=xz.device)
     library.call(mixers(), "palm_causal_conv", _stream(), _p(xz), _code(xz, "causal_conv"), xz.shape[1], _p(weight), _p(bias),
-                 _p(conv_state), _p(ctx.seq_slot), _p(ctx.seq_new), _p(ctx.cu_new), ctx.n_seqs, ctx.max_new, channels, taps, _p(out))
+                 _p(conv_state), _p(ctx.seq_slot), _p(ctx.seq_new), _p(ctx.cu_new), ctx.n_seqs, ctx.max_new, xz.shape[0], channels, taps, _p(out))
     return out
 
 

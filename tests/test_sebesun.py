@@ -236,7 +236,8 @@ def test_averages_over_many_planes(W, J):
 @gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("taps", [2, 3, 4, 5])
-@pytest.mark.parametrize("lens,C,wide", [([16], 64, 64), ([1, 15, 47], 1028, 2060), ([33, 2, 130], 260, 264), ([40, 3], 66, 66), ([20, 16], 64, 67)])
+@pytest.mark.parametrize("lens,C,wide", [([16], 64, 64), ([1, 15, 47], 1028, 2060), ([33, 2, 130], 260, 264), ([40, 3], 66, 66), ([20, 16], 64, 67),
+                                         ([1, 15, 47, 16, 33], 11800, 11804), ([16, 130], 9204, 18408), ([47] + [1] * 20, 8500, 8504), ([60, 50], 12000, 12001)])
 def test_causal_conv_in_runs_is_the_convolution_token_by_token(dtype, taps, lens, C, wide):
     """Runs of tokens a thread, their remainders, and the sizes that go a token a thread: bit for bit the steps of one token each."""
     from palm_infra_amd.kernels import ops
