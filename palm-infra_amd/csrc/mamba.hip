@@ -206,8 +206,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     constexpr int NB = (SCAN_TILE * NP + SCAN_THREADS - 1) / SCAN_THREADS, NC = (SCAN_TILE * CH + SCAN_THREADS - 1) / SCAN_THREADS;
     // of B and C at a time: all, but where that costs blocks a compute unit (128 states, eight at a time: 88 registers and five waves a
     // SIMD; 2,048 channels, 717 + 572 + 1,314 tokens 694 us, in halves 617; one token each of 64 sequences 84 and 65).  (256 states:
-    // LDS sets the number of blocks.)
+    // LDS sets the number of blocks; in quarters 1,139 us, 981 all together.)  A tile of few tokens does not go through the rest: 64
+    // sequences of one token, with it and without, 128 states 64 us and 59, 256 states, a token an element, 143 and 122.
     constexpr int HELD = PER == 2 ? 4 : NB;
+    constexpr bool BY_TOKEN = NP == SCAN_THREADS;      // element first + i of every thread is of token first + i
     __shared__ float b_s[SCAN_TILE][NP], c_s[SCAN_TILE][NP];
     __shared__ float dt_s[SCAN_TILE][CH], u_s[SCAN_TILE][CH], y_s[SCAN_TILE][CH];
     const int j = threadIdx.x % G, ch = threadIdx.x / G;
@@ -241,6 +243,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 #pragma unroll
         for (int i = 0; i < HELD; ++i) {
             const int idx = threadIdx.x + (first + i) * SCAN_THREADS, n = idx % NP;
+            if (BY_TOKEN && t0 + first + i >= n_new) break;
             b_r[i] = c_r[i] = T{};
             if (n >= n_state || t0 + idx / NP >= n_new) continue;
             const T* r = bc + (row0 + t0 + idx / NP) * bc_stride;
@@ -252,6 +255,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 #pragma unroll
         for (int i = 0; i < HELD; ++i) {
             const int idx = threadIdx.x + (first + i) * SCAN_THREADS;
+            if (BY_TOKEN && first + i >= tt) break;
             if (idx / NP < tt) { b_s[idx / NP][idx % NP] = to_float(b_r[i]); c_s[idx / NP][idx % NP] = to_float(c_r[i]); }
         }
     };
@@ -276,7 +280,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
         if (!AHEAD) ask_channels(t0);
         float u_t[NC], z_t[NC];
 #pragma unroll 1
-        for (int first = 0; first < NB; first += HELD) {
+        for (int first = 0; first < NB && (HELD == NB || first * SCAN_THREADS < tt * NP); first += HELD) {
             if (!AHEAD) ask_states(t0, first);
             keep_states(tt, first);
         }
