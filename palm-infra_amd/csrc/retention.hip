@@ -358,10 +358,23 @@ __global__ __launch_bounds__(256) void retention_out_kernel(const T* __restrict_
     }
 }
 
-// The chunk with which a step's runs go through the kernels above, or 0: sizes that fill the waves' tiles, and runs longer than
+// The chunk with which a step's runs can go through the kernels above, or 0: sizes that fill the waves' tiles, and runs longer than
 // one walk should take (16 heads of 128 x 256: 8 tokens 30 us and 25 walked, 16 tokens 32 and 45, 2,048 tokens 138 and 535).
 PALM_API int palm_retention_matrix_chunk(int dim, int vdim, int max_new) {
     return (dim == 64 || dim == 128) && (vdim == 128 || vdim == 256) && max_new >= 16 ? RET_CHUNK : 0;
+}
+
+// Whether they should.  In chunks a sequence's state crosses memory six times, once a single token as well, in the walk twice; the
+// walk is the longest run's chain, slower with more blocks a compute unit (as many as all tokens make in runs of that length).  In
+// us, what chunks spare of that against what they cost.  16 heads of 128 x 256, walked and in chunks: 63 single tokens beside 16
+// new ones 77 and 190, beside 512 1,280 and 312, 17 tokens of each of 64 sequences 152 and 271, 30 of 32 139 and 137.
+// Drawn from 1,196 steps timed both ways (2 to 64 heads, 1 to 128 sequences; equal runs, one or some among single tokens, ragged); at
+// 500 others 0.4 % from the better way in the mean, 8 % behind the walk at worst, 49 % behind chunks (92 of 16 tokens, four heads).
+PALM_API int palm_retention_matrix_pays(int heads, int dim, int vdim, int n_seqs, int n_tokens, int max_new) {
+    if (!palm_retention_matrix_chunk(dim, vdim, max_new)) return 0;
+    const double a_unit = (double)heads * n_tokens / max_new / 256, mb = (double)n_seqs * heads * dim * vdim * sizeof(float) / (1 << 20);
+    const double few = min(ceil(a_unit), 3.0), crowded = vdim == 128 ? max(0.72 * few, 0.22 * a_unit) : max(0.56 * few, 0.37 * a_unit);
+    return (0.41 + 0.0105 * dim) * max_new * max(1.0, crowded) > 7.1 + 0.92 * mb + 0.44 * max(mb - 128.0, 0.0);
 }
 
 // Places of chunks that the starts have room for (as many as n_tokens tokens of n_seqs sequences need, up to RET_ROOM bytes).

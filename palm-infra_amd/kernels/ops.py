@@ -897,6 +897,7 @@ _RECURRENT_SIGNATURES = {
                        c_float, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
                        c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int],
     "palm_retention_matrix_chunk": [c_int, c_int, c_int],
+    "palm_retention_matrix_pays": [c_int, c_int, c_int, c_int, c_int, c_int],
     "palm_retention_places": [c_int, c_int, c_int, c_int, c_int],
     "palm_retention_pad": [c_int],
     "palm_joined_norm_gate": [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
@@ -1097,9 +1098,10 @@ def retention(qkvg: torch.Tensor, heads: int, dim: int, vdim: int, decay: torch.
         raw = torch.empty((n, heads * vdim), dtype=F32, device=qkvg.device)
     else:
         _need(not gate_sigmoid, "retention: the per-head unit norm comes with a silu gate")
-    # runs in chunks on the matrix cores where the sizes and the rows' alignment allow, else walked over token by token
+    # runs in chunks on the matrix cores where the sizes and the rows' alignment allow and it pays, else walked over token by token
     matrix = 0
-    if chunk is None and col0 % 8 == 0 and qkvg.shape[1] % 8 == 0 and (qkvg.data_ptr() | state.data_ptr()) % 16 == 0:
+    if (chunk is None and col0 % 8 == 0 and qkvg.shape[1] % 8 == 0 and (qkvg.data_ptr() | state.data_ptr()) % 16 == 0
+            and recurrent().palm_retention_matrix_pays(heads, dim, vdim, ctx.n_seqs, n, ctx.max_new)):
         matrix = recurrent().palm_retention_matrix_chunk(dim, vdim, ctx.max_new)
     chunk = matrix or (retention_chunk(ctx.n_seqs, heads, ctx.max_new) if chunk is None else int(chunk))
     # q and k after the rotation, 32-bit, in rows padded to the key size that the kernel is compiled for

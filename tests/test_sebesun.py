@@ -352,7 +352,7 @@ def test_retention_in_chunks_on_the_matrix_cores(dtype, dk, dv):
     want = {"head": P.unit_rms(o, 1e-6).reshape(T, H * dv) * P.silu(g), "joined": P.unit_rms(flat, 1e-6) * weight.double() * torch.sigmoid(g)}
     # outputs of unit scale: 32-bit sums of up to 130 * dk terms, then one rounding to the type
     tol = 1e-4 if dtype == torch.float32 else 3e-2
-    assert ops.recurrent().palm_retention_matrix_chunk(dk, dv, max(lengths)) == 64
+    assert ops.recurrent().palm_retention_matrix_pays(H, dk, dv, len(lengths), T, max(lengths))
     for kind in ("head", "joined"):
         results = []
         for chunk in (None, 0):
@@ -367,6 +367,36 @@ def test_retention_in_chunks_on_the_matrix_cores(dtype, dk, dv):
         assert (results[0].float() - results[1].float()).abs().max() < tol * max(1.0, float(want[kind].abs().max()))
 
 
+def test_which_steps_of_retention_go_in_chunks():
+    """Not where many states would move for a few short runs: there the walk, which touches a state once, is the faster one."""
+    from palm_infra_amd.kernels import ops
+    pays = lambda lengths, heads=16, dim=128, vdim=256: bool(ops.recurrent().palm_retention_matrix_pays(heads, dim, vdim, len(lengths), sum(lengths), max(lengths)))
+    assert pays([16]) and not pays([15]) and pays([2048]) and pays([1] * 8 + [300]) and pays([300] * 8) and pays([1] * 63 + [512])
+    assert not pays([1] * 63 + [16]) and not pays([1] * 63 + [64]) and not pays([17] * 64) and not pays([24] * 128)
+    assert pays([16] * 8, 32, 64, 128) and not pays([1] * 127 + [40], 32, 64, 128) and pays([24] * 32, 20, 128, 128)
+    assert pays([700, 1], 1, 64, 256) and not pays([700, 1], 1, 64, 192) and not pays([700, 1], 1, 72, 128)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths", [[1] * 40 + [20], [1] * 40 + [90]])
+def test_retention_of_many_single_tokens_beside_a_run(dtype, lengths):
+    """A run short enough that the step is walked over and one long enough that it goes in chunks: both against the walk."""
+    from palm_infra_amd.kernels import ops
+    torch.manual_seed(len(lengths))
+    H, dk, dv, n, T = 16, 128, 256, len(lengths), sum(lengths)
+    assert bool(ops.recurrent().palm_retention_matrix_pays(H, dk, dv, n, T, max(lengths))) == (lengths[-1] > 64)
+    rows, decay, state0 = (torch.randn(T, H * (2 * dk + 2 * dv)) * 0.5).to(dtype).cuda(), torch.linspace(0.9, 0.999, H).cuda(), torch.randn(n, H, dk, dv).cuda()
+    got, walked = [], []
+    for results, chunk in ((got, None), (walked, 0)):
+        state = state0.clone()
+        results += [ops.retention(rows, H, dk, dv, decay, dk ** -0.5, 1e-6, state, _step_context([0] * n, lengths), chunk=chunk).float(), state]
+    # 32-bit sums in another order, then one rounding to the type
+    assert (got[0] - walked[0]).abs().max() < (1e-4 if dtype == torch.float32 else 2.0 ** -7) * float(walked[0].abs().max())
+    assert (got[1] - walked[1]).abs().max() < 1e-4
+    assert lengths[-1] > 64 or (torch.equal(got[0], walked[0]) and torch.equal(got[1], walked[1]))
+
+
 def test_retention_starts_have_bounded_room():
     from palm_infra_amd.kernels import ops
     places = ops.recurrent().palm_retention_places
@@ -376,7 +406,7 @@ def test_retention_starts_have_bounded_room():
 
 
 @gpu
-@pytest.mark.parametrize("lengths", [[700, 1, 500, 130], [1500], [20] * 70 + [1, 200]])
+@pytest.mark.parametrize("lengths", [[700, 1, 500, 130], [1500], [20] * 70 + [1, 900]])
 def test_retention_in_windows_of_chunks(lengths):
     """More chunks than the starts have room for: the state crosses from one window to the next, within a sequence and between
     sequences; against the walk token by token."""
@@ -384,6 +414,7 @@ def test_retention_in_windows_of_chunks(lengths):
     torch.manual_seed(len(lengths))
     H, dk, dv, T = 64, 128, 256, sum(lengths)
     assert ops.recurrent().palm_retention_places(H, dk, dv, T, len(lengths)) == 16 < T // 64 + len(lengths)
+    assert ops.recurrent().palm_retention_matrix_pays(H, dk, dv, len(lengths), T, max(lengths))
     rows = (torch.randn(T, H * (2 * dk + 2 * dv)) * 0.5).bfloat16().cuda()
     decay, state0 = torch.linspace(0.9, 0.999, H).cuda(), torch.randn(len(lengths), H, dk, dv).cuda()
     results = []
