@@ -792,7 +792,10 @@ constexpr int SLICED_ROWS = 512;                                     // rows tha
 constexpr int SLICED_MIN_VOCAB = 16384;                              // (below, the row is a few slices: one block does as well)
 constexpr int SURVIVORS = 1024;
 
-static int slices_of(int V) { return (V / 4 + SLICE / 4 - 1) / (SLICE / 4); }
+// As few as hold the row, but one for every eight of the k at least: the second kernel's cut is made of the maxima of 16 groups a
+// slice, and with fewer groups than k it lets every candidate through to be ranked (k = 128, 16,384 logits: 81 us with four slices,
+// 35 with sixteen, 58 as one block; 32,000 logits 62, 36 and 59).  A slice has a group of four for every thread at least.
+static int slices_of(int V, int k) { return max((V / 4 + SLICE / 4 - 1) / (SLICE / 4), (k + 7) / 8); }
 
 // how many of the 256 keys are larger
 __device__ inline int larger_keys(const uint32_t* keys, uint32_t own) {
@@ -1089,7 +1092,7 @@ PALM_API int palm_sample(hipStream_t stream, const float* logits, int n_rows, in
 // pieces; and the bytes of workspace that it needs then (0: it does not).  From SLICED_MIN_VOCAB on the slices win at any batch.
 PALM_API long long palm_sample_sliced_work(int n_rows, int V, float temperature, int top_k) {
     if (temperature <= 0.f || top_k <= 1 || top_k > SLICED_TOPK_MAX || V < SLICED_MIN_VOCAB || V % 4 != 0 || n_rows < 1 || n_rows > 65535) return 0;
-    return (long long)min(n_rows, SLICED_ROWS) * slices_of(V) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int));
+    return (long long)min(n_rows, SLICED_ROWS) * slices_of(V, top_k) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int));
 }
 
 PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, float temperature,
@@ -1101,7 +1104,7 @@ PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_r
     PALM_CHECK(top_p >= 0.f && top_p <= 1.f, "sample: top_p must be between 0 and 1");
     PALM_CHECK(min_p >= 0.f && min_p <= 1.f, "sample: min_p must be between 0 and 1");
     PALM_CHECK(uniforms, "sample: a draw needs the uniform numbers");
-    const int slices = slices_of(V);
+    const int slices = slices_of(V, top_k);
     uint2* cands = (uint2*)work;
     int* counts = (int*)(cands + (size_t)min(n_rows, SLICED_ROWS) * slices * SLICE_CAP);
     for (int r0 = 0; r0 < n_rows; r0 += SLICED_ROWS) {

@@ -703,7 +703,7 @@ def test_top_k_in_slices_where_logits_are_equal(ops, V, k):
     work, out = torch.empty(needed, dtype=torch.uint8, device=DEV), torch.empty(n, dtype=torch.int32, device=DEV)
     library.call(ops.core(), "palm_sample_sliced", ops._stream(), lg.data_ptr(), n, V, u.data_ptr(), 0.7, k, 0.95, 0.0, out.data_ptr(), work.data_ptr(), needed)
     assert out.tolist() == whole(lg, u)
-    slices = -(-(V // 4) // 1024)
+    slices = max(-(-(V // 4) // 1024), -(-k // 8))
     counts = work[n * slices * 512 * 8:].view(torch.int32)
     assert counts.numel() == n * slices and counts.min() >= min(k, 4) and counts.max() <= 512
     if V == 16388:
