@@ -788,7 +788,7 @@ constexpr int SLICE_QUADS = 4;                                       // 16-byte 
 constexpr int SLICE = SLICE_THREADS * SLICE_QUADS * 4;
 constexpr int SLICED_TOPK_MAX = 128;                                 // half a slice's threads: the cut stays a tail of the slice
 constexpr int SLICE_CAP = 4 * SLICED_TOPK_MAX;                       // candidates that a slice can hand on (equal or sorted logits: four a thread)
-constexpr int SLICED_ROWS = 512;                                     // rows that share the workspace (80 MB for 151,936 logits)
+constexpr long long SLICED_ROOM = 128ll << 20;                       // workspace that rows share, group after group (151,936 logits: 861 rows)
 constexpr int SLICED_MIN_VOCAB = 16384;                              // (below, the row is a few slices: one block does as well)
 constexpr int SURVIVORS = 1024;
 
@@ -1088,11 +1088,15 @@ PALM_API int palm_sample(hipStream_t stream, const float* logits, int n_rows, in
     return 0;
 }
 
+// Rows of a group (two more launches for each further one: 600 rows of 50,304 logits, k = 128, 129 us in one group and 147 in two).
+static long long row_room(int V, int k) { return slices_of(V, k) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int)); }
+static int sliced_rows(int n_rows, int V, int k) { return (int)min((long long)n_rows, max(1ll, SLICED_ROOM / row_room(V, k))); }
+
 // Whether palm_sample_sliced serves these rows: one to SLICED_TOPK_MAX candidates of a large vocabulary, rows of whole 16-byte
 // pieces; and the bytes of workspace that it needs then (0: it does not).  From SLICED_MIN_VOCAB on the slices win at any batch.
 PALM_API long long palm_sample_sliced_work(int n_rows, int V, float temperature, int top_k) {
     if (temperature <= 0.f || top_k <= 1 || top_k > SLICED_TOPK_MAX || V < SLICED_MIN_VOCAB || V % 4 != 0 || n_rows < 1 || n_rows > 65535) return 0;
-    return (long long)min(n_rows, SLICED_ROWS) * slices_of(V, top_k) * (long long)(SLICE_CAP * sizeof(uint2) + sizeof(int));
+    return sliced_rows(n_rows, V, top_k) * row_room(V, top_k);
 }
 
 PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, float temperature,
@@ -1104,11 +1108,11 @@ PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_r
     PALM_CHECK(top_p >= 0.f && top_p <= 1.f, "sample: top_p must be between 0 and 1");
     PALM_CHECK(min_p >= 0.f && min_p <= 1.f, "sample: min_p must be between 0 and 1");
     PALM_CHECK(uniforms, "sample: a draw needs the uniform numbers");
-    const int slices = slices_of(V, top_k);
+    const int slices = slices_of(V, top_k), group = sliced_rows(n_rows, V, top_k);
     uint2* cands = (uint2*)work;
-    int* counts = (int*)(cands + (size_t)min(n_rows, SLICED_ROWS) * slices * SLICE_CAP);
-    for (int r0 = 0; r0 < n_rows; r0 += SLICED_ROWS) {
-        const int rows = min(SLICED_ROWS, n_rows - r0);
+    int* counts = (int*)(cands + (size_t)group * slices * SLICE_CAP);
+    for (int r0 = 0; r0 < n_rows; r0 += group) {
+        const int rows = min(group, n_rows - r0);
         const float* at = logits + (size_t)r0 * V;
         topk_slice_kernel<<<dim3(slices, rows), SLICE_THREADS, 0, stream>>>(at, V, top_k, counts, cands);
         PALM_LAUNCHED();

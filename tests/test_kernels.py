@@ -707,8 +707,8 @@ def test_top_k_in_slices_where_logits_are_equal(ops, V, k):
     counts = work[n * slices * 512 * 8:].view(torch.int32)
     assert counts.numel() == n * slices and counts.min() >= min(k, 4) and counts.max() <= 512
     if V == 16388:
-        many = lg.repeat(600 // n + 1, 1)
-        assert ops.core().palm_sample_sliced_work(len(many), V, 0.7, k) == ops.core().palm_sample_sliced_work(512, V, 0.7, k)
+        many = lg.repeat(2100 // n + 1, 1)
+        assert ops.core().palm_sample_sliced_work(len(many), V, 0.7, k) <= 128 << 20 < len(many) * (needed // n)
         u = torch.rand(len(many), generator=torch.Generator().manual_seed(5)).to(DEV)
         assert ops.sample(many, u, 0.7, k, 0.95).tolist() == whole(many, u)
 
