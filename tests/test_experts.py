@@ -164,9 +164,10 @@ def test_which_steps_go_through_the_grouped_products():
     def pays(n, W, F, E=1, top=1, dt=torch.bfloat16, form="gelu", shared=False, offset=0):
         h = torch.empty(n * W + 8, dtype=dt)[offset:offset + n * W].view(n, W)
         return ops.moe_grouped_pays(h, torch.empty(E * ops.expert_rows(form) * F, W, dtype=dt), torch.empty(E * W, F, dtype=dt), F, top, form, shared)
-    assert pays(97, 64, 128) and pays(128, 4096, 64) and not pays(96, 64, 128)
-    assert pays(17, 2048, 128, E=22, top=4) and not pays(17, 2048, 128, E=21, top=4)          # 198 and 189 tiles
-    assert not pays(17, 2048, 128, E=22, top=1)                                               # at most seventeen experts in use
+    assert pays(97, 64, 128, E=16) and pays(128, 4096, 64) and not pays(96, 64, 128, E=16)
+    assert pays(48, 64, 128, E=8, top=2) and not pays(47, 64, 128, E=8, top=2) and pays(17, 64, 128)      # twelve rows an expert
+    assert pays(17, 2048, 128, E=15, top=4) and not pays(17, 2048, 128, E=14, top=4)          # 135 and 126 tiles
+    assert pays(17, 1792, 128, E=64, top=1) and not pays(17, 1536, 128, E=64, top=1)          # at most seventeen experts in use: 136 and 119
     assert not pays(17, 2048, 128, E=22, top=4, shared=True) and pays(17, 2048, 128, E=36, top=4, shared=True)
     assert pays(17, 1024, 512, E=32, top=4) and pays(17, 1024, 512, E=32, top=4, form="gated_silu")
     assert not pays(16, 2048, 128, E=22, top=4) and not pays(97, 72, 128) and not pays(97, 64, 40) and not pays(97, 64, 128, dt=torch.float32)
