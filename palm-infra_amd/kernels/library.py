@@ -27,8 +27,8 @@ Libraries:
   ``mlstm``             a matrix memory with input and forget gates per head and token
   ``latent_attention_k<K>_v<V>``  attention over compressed rows on the matrix cores, compiled for rows up to 32 K and
                         latents up to 16 V
-  ``attention_diff_k<K>_v<V>_q<Q>``  differential attention for prompts on the matrix cores, compiled for key sizes up to
-                        32 K, value sizes up to 16 V and Q tiles of 16 queries a wave
+  ``attention_diff_k<K>_v<V>``  differential attention for prompts on the matrix cores, compiled for key sizes up to
+                        32 K and value sizes up to 16 V
 """
 from __future__ import annotations
 
@@ -76,7 +76,7 @@ HEADERS = ["common.h", "mfma.h", "linear_thin.h", "linear_wide.h", "attention_ap
 # headers of a few sources only: a change of one rebuilds the libraries of the sources that include it
 OWN_HEADERS = {"retention.hip": ["linear_recurrence.h"], "gla.hip": ["linear_recurrence.h"], "delta_rule.hip": ["delta_rule.h"],
                "delta_head.hip": ["delta_rule.h", "conv_state.h"], "mamba.hip": ["conv_state.h"], "moe.hip": ["expert_form.h"], "moe_few.hip": ["expert_form.h"],
-               "moe_grouped.hip": ["big_walk.h", "expert_form.h", "lds_stage.h"], "linear_tile.hip": ["lds_stage.h"], "linear_big.hip": ["big_walk.h", "lds_stage.h"], "attention_sink_mfma.hip": ["lds_stage.h"],
+               "moe_grouped.hip": ["big_walk.h", "expert_form.h", "lds_stage.h"], "linear_tile.hip": ["lds_stage.h"], "linear_big.hip": ["big_walk.h", "lds_stage.h"], "attention_sink_mfma.hip": ["lds_stage.h"], "attention_diff_mfma.hip": ["lds_stage.h"],
                "branch_scaled.hip": ["expert_form.h"]}
 
 
@@ -232,9 +232,8 @@ def _spec(name: str):
         kk, vt = name[len("sink_attention_k"):].split("_v")
         return SINK_ATTENTION_MFMA_SOURCES, (f"PALM_SINK_KK={int(kk)}", f"PALM_SINK_VT={int(vt)}")
     if name.startswith("attention_diff_k"):
-        kk, rest = name[len("attention_diff_k"):].split("_v")
-        vt, qt = rest.split("_q")
-        return DIFF_ATTENTION_SOURCES, (f"PALM_DIFF_KK={int(kk)}", f"PALM_DIFF_VT={int(vt)}", f"PALM_DIFF_QT={int(qt)}")
+        kk, vt = name[len("attention_diff_k"):].split("_v")
+        return DIFF_ATTENTION_SOURCES, (f"PALM_DIFF_KK={int(kk)}", f"PALM_DIFF_VT={int(vt)}")
     if name.startswith("latent_attention_k"):
         kk, vt = name[len("latent_attention_k"):].split("_v")
         return LATENT_ATTENTION_SOURCES, (f"PALM_LAT_KK={int(kk)}", f"PALM_LAT_VT={int(vt)}")

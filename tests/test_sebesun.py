@@ -580,6 +580,57 @@ def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge
     cache.check()
 
 
+@gpu
+@pytest.mark.parametrize("heads,kv_heads,dk,dv", [(4, 1, 64, 128), (8, 2, 128, 256), (6, 3, 40, 72), (3, 3, 96, 64), (8, 2, 256, 256), (4, 1, 32, 20)])
+@pytest.mark.parametrize("lengths", [(1, 15), (16, 17, 64), (65, 129, 33), (700, 300, 513, 64)])
+def test_differential_attention_of_prompts_at_the_edges_of_its_blocks(heads, kv_heads, dk, dv, lengths):
+    """Prompts on the matrix cores (four or eight waves a block, one or two pages in LDS, heads of a block that share keys or do
+    not) against 64 bits, over pages whose places beyond the sequences hold NaN, and with keys already there."""
+    from palm_infra_amd.kernels import ops
+    torch.manual_seed(sum(lengths) + dk)
+    scale, lam, gain, eps = dk ** -0.5, 0.4, 0.6, 1e-6
+    starts = [70 * (b % 2) for b in range(len(lengths))]
+    ends = [s + n for s, n in zip(starts, lengths)]
+    pages = [(e + 63) // 64 for e in ends]
+    table = torch.zeros(len(lengths), max(pages), dtype=torch.int32)
+    order = torch.randperm(sum(pages)).int()
+    for b, n in enumerate(pages):
+        table[b, :n] = order[sum(pages[:b]):sum(pages[:b + 1])]
+    k_cache = torch.full((sum(pages), 2 * kv_heads, 64, dk), math.nan).bfloat16()
+    v_cache = torch.full((sum(pages), kv_heads, dv, 64), math.nan).bfloat16()
+    q = torch.randn(sum(lengths), heads, 2, dk).bfloat16()
+    want, at = [], 0
+    for b, end in enumerate(ends):
+        k, v = (torch.randn(end, 2 * kv_heads, dk) * 2).bfloat16(), torch.randn(end, kv_heads, dv).bfloat16()
+        for p in range(pages[b]):
+            here = slice(64 * p, min(end, 64 * p + 64))
+            k_cache[table[b, p], :, :here.stop - here.start] = k[here].transpose(0, 1)
+            v_cache[table[b, p], :, :, :here.stop - here.start] = v[here].permute(1, 2, 0)
+        mine = q[at:at + lengths[b]].double()
+        at += lengths[b]
+        hidden = torch.arange(end) > starts[b] + torch.arange(lengths[b])[:, None]
+        out = torch.empty(lengths[b], heads, dv, dtype=P.F64)
+        for h in range(heads):
+            g = h // (heads // kv_heads)
+            a = [torch.softmax((mine[:, h, m] @ k[:, 2 * g + m].double().T * scale).masked_fill(hidden, -math.inf), -1) @ v[:, g].double() for m in range(2)]
+            out[:, h] = P.unit_rms(a[0] - lam * a[1], eps) * gain
+        want.append(out.reshape(lengths[b], -1))
+    cum = [0]
+    for n in lengths:
+        cum.append(cum[-1] + n)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    class Ctx:
+        seq_slot, seq_start, seq_new, cu_new = ints(list(range(len(lengths)))), ints(starts), ints(list(lengths)), ints(cum)
+        n_tokens, n_seqs, max_new, is_decode = cum[-1], len(lengths), max(lengths), False
+
+    got = ops.attention_diff_mfma(q.view(cum[-1], -1).cuda(), k_cache.cuda(), v_cache.cuda(), table.cuda(), Ctx, heads, kv_heads, dk, dv, scale, lam, gain, eps)
+    # a weight is rounded to bfloat16 once (2^-9 of it), the result once more, and a1 - lambda a2 is shorter than its terms
+    err = (got.double().cpu() - torch.cat(want)).norm() / torch.cat(want).norm()
+    assert err < 6e-3, f"{err}"
+    assert (got.double().cpu() - torch.cat(want)).abs().max() < 0.1 * float(torch.cat(want).abs().max())
+
+
 # ---- whole models ----------------------------------------------------------------------------------------
 
 @gpu
