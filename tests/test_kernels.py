@@ -231,6 +231,18 @@ def test_float32_products_on_the_matrix_cores(ops, M, N, K):
     assert torch.equal(out.cpu(), got + c)
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 12300, 4096), (16, 12288, 4128), (47, 12290, 64), (64, 72, 8192), (161, 392, 128), (250, 4100, 288)])
+def test_float32_products_of_every_width_of_a_block(ops, M, N, K):
+    """Blocks of 16 to 64 weight rows, rings of two to four stages, fewer stages of K than the ring has and than there are waves; a
+    row's result is the same whatever tile it lies in."""
+    a, w = rand(M, K, seed=M), rand(N, K, seed=N + 1)
+    got = ops.linear_exact(a.to(DEV), w.to(DEV)).cpu()
+    assert (got.double() - P.linear(a, w)).abs().max() < 8 * 2.0 ** -24 * K ** 0.5 * 4        # as above
+    part = slice(0, N // 2 + 5)
+    for rows in (slice(0, 1), slice(M // 2, M // 2 + 2), slice(M // 3, M)):
+        assert torch.equal(ops.linear_exact(a[rows].contiguous().to(DEV), w[part].contiguous().to(DEV)).cpu(), got[rows, part])
+
+
 def test_linear_refuses_what_does_not_fit(ops):
     from palm_infra_amd.kernels import KernelError
     with pytest.raises(KernelError, match="inner size"):
