@@ -80,7 +80,9 @@ def core():
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """torch's current stream on the current device (``torch.cuda.current_stream()`` makes an object for it: 2.9 us against 0.2, at
+    every launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t):
@@ -110,6 +112,8 @@ def _dev(what: str, *tensors) -> None:
 
 
 def _need(cond: bool, msg: str) -> None:
+    """For messages that are there: one that tells sizes is put together only where it is raised (a check's text took a microsecond
+    at every launch)."""
     if not cond:
         raise KernelError(msg)
 
@@ -126,12 +130,14 @@ def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor | None = Non
     """out[t, :] = table[ids[t], :] * scale as float32."""
     _dev("embed", table, ids, out)
     _i32("embed", ids)
-    _need(table.dim() == 2 and ids.dim() == 1, f"embed: table {tuple(table.shape)}, ids {tuple(ids.shape)}")
+    if not (table.dim() == 2 and ids.dim() == 1):
+        raise KernelError(f"embed: table {tuple(table.shape)}, ids {tuple(ids.shape)}")
     vocab, hidden = table.shape
     n = ids.shape[0]
     if out is None:
         out = torch.empty((n, hidden), dtype=F32, device=table.device)
-    _need(out.shape == (n, hidden) and out.dtype == F32, f"embed: out {tuple(out.shape)} {out.dtype}")
+    if not (out.shape == (n, hidden) and out.dtype == F32):
+        raise KernelError(f"embed: out {tuple(out.shape)} {out.dtype}")
     library.call(core(), "palm_embed", _stream(), _p(table), _code(table, "embed table"), _p(ids), n, hidden, vocab, _p(out),
                  float(scale))
     return out
@@ -144,15 +150,17 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.
     planes [P, n, width], which are added one after the other."""
     _dev("rmsnorm", x, weight, delta, rows)
     _i32("rmsnorm", rows)
-    _need(x.dim() == 2, f"rmsnorm: x {tuple(x.shape)} is not [rows, width]")
+    if not (x.dim() == 2):
+        raise KernelError(f"rmsnorm: x {tuple(x.shape)} is not [rows, width]")
     n, width = x.shape
-    _need(weight.shape == (width,) and weight.dtype == F32, f"rmsnorm: weight {tuple(weight.shape)} {weight.dtype}, "
-          f"width {width} (norm weights are float32)")
+    if not (weight.shape == (width,) and weight.dtype == F32):
+        raise KernelError(f"rmsnorm: weight {tuple(weight.shape)} {weight.dtype}, "
+                          f"width {width} (norm weights are float32)")
     planes = 1
     if delta is not None and delta.dim() == 3:
         planes = delta.shape[0]
-        _need(delta.dtype == F32 and delta.shape[1:] == x.shape and delta.is_contiguous(),
-              f"rmsnorm: delta planes {tuple(delta.shape)} {delta.dtype} for x {tuple(x.shape)} (planes are contiguous float32)")
+        if not (delta.dtype == F32 and delta.shape[1:] == x.shape and delta.is_contiguous()):
+            raise KernelError(f"rmsnorm: delta planes {tuple(delta.shape)} {delta.dtype} for x {tuple(x.shape)} (planes are contiguous float32)")
     else:
         _need(delta is None or delta.shape == x.shape, "rmsnorm: delta and x differ in shape")
     _need(not update_x or (delta is not None and rows is None), "rmsnorm: update_x needs a delta and no row selection")
@@ -167,7 +175,8 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.
 def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     """[n, 2I] -> [n, I]: silu(first half) * second half."""
     _dev("swiglu", gate_up)
-    _need(gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0, f"swiglu: input {tuple(gate_up.shape)}")
+    if not (gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0):
+        raise KernelError(f"swiglu: input {tuple(gate_up.shape)}")
     n, two_i = gate_up.shape
     out = torch.empty((n, two_i // 2), dtype=gate_up.dtype, device=gate_up.device)
     library.call(core(), "palm_swiglu", _stream(), _p(gate_up), _code(gate_up, "swiglu"), _p(out), n, two_i // 2)
@@ -177,8 +186,8 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
 def add_bias(y: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     """y[r, :] += bias, in place; y [n, out] float32 or bfloat16, bias [out] float32.  Returns y."""
     _dev("add_bias", y, bias)
-    _need(y.dim() == 2 and y.is_contiguous() and bias.shape == (y.shape[1],) and bias.dtype == F32 and bias.is_contiguous(),
-          f"add_bias: y {tuple(y.shape)}, bias {tuple(bias.shape)} {bias.dtype} is not float32 [{y.shape[-1]}]")
+    if not (y.dim() == 2 and y.is_contiguous() and bias.shape == (y.shape[1],) and bias.dtype == F32 and bias.is_contiguous()):
+        raise KernelError(f"add_bias: y {tuple(y.shape)}, bias {tuple(bias.shape)} {bias.dtype} is not float32 [{y.shape[-1]}]")
     library.call(core(), "palm_add_bias", _stream(), _p(y), _code(y, "add_bias"), _p(bias), y.shape[0], y.shape[1])
     return y
 
@@ -191,8 +200,10 @@ def convert_into(src: torch.Tensor, dst: torch.Tensor) -> None:
     float16 or float64).  One rounding to nearest where dst is narrower.  dst may be a run of rows of a larger
     tensor: what a checkpoint's tensors go through when they are joined into one parameter."""
     _dev("convert", src, dst)
-    _need(src.dtype in _STORED_CODES, f"convert: a tensor stored as {src.dtype} is not float32, bfloat16, float16 or float64")
-    _need(src.numel() == dst.numel(), f"convert: {tuple(src.shape)} into {tuple(dst.shape)}")
+    if not (src.dtype in _STORED_CODES):
+        raise KernelError(f"convert: a tensor stored as {src.dtype} is not float32, bfloat16, float16 or float64")
+    if not (src.numel() == dst.numel()):
+        raise KernelError(f"convert: {tuple(src.shape)} into {tuple(dst.shape)}")
     library.call(core(), "palm_convert", _stream(), _p(src), _STORED_CODES[src.dtype], _p(dst), _code(dst, "convert dst"),
                  src.numel())
 
@@ -211,14 +222,15 @@ def linear_exact(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None
                  accumulate: bool = False) -> torch.Tensor:
     """a [M, K] . w [N, K]^T with plain 32-bit FMA; any mix of float32 and bfloat16 operands."""
     _dev("linear", a, w, out)
-    _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1],
-          f"linear: a {tuple(a.shape)} and w {tuple(w.shape)} do not share the inner size")
+    if not (a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]):
+        raise KernelError(f"linear: a {tuple(a.shape)} and w {tuple(w.shape)} do not share the inner size")
     M, K = a.shape
     N = w.shape[0]
     if out is None:
         _need(not accumulate, "linear: accumulate needs an output to add to")
         out = torch.empty((M, N), dtype=out_dtype or a.dtype, device=a.device)
-    _need(out.shape == (M, N), f"linear: out {tuple(out.shape)} is not {(M, N)}")
+    if not (out.shape == (M, N)):
+        raise KernelError(f"linear: out {tuple(out.shape)} is not {(M, N)}")
     library.call(core(), "palm_linear", _stream(), _p(a), _code(a, "linear a"), _p(w), _code(w, "linear w"), _p(out),
                  _code(out, "linear out"), M, N, K, int(accumulate))
     return out
@@ -227,11 +239,12 @@ def linear_exact(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None
 # ---- attention ------------------------------------------------------------------------------------
 
 def _check_cache(what, k_cache, v_cache, block_table, nkv, hd):
-    _need(k_cache.dim() == 4 and k_cache.shape[1:] == (nkv, PAGE_TOKENS, hd),
-          f"{what}: key cache {tuple(k_cache.shape)} is not [pages, {nkv}, {PAGE_TOKENS}, {hd}]")
-    _need(v_cache.shape == (k_cache.shape[0], nkv, hd, PAGE_TOKENS) and v_cache.dtype == k_cache.dtype,
-          f"{what}: value cache {tuple(v_cache.shape)} is not [pages, {nkv}, {hd}, {PAGE_TOKENS}] (values are kept transposed)")
-    _need(block_table.dim() == 2, f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
+    if not (k_cache.dim() == 4 and k_cache.shape[1:] == (nkv, PAGE_TOKENS, hd)):
+        raise KernelError(f"{what}: key cache {tuple(k_cache.shape)} is not [pages, {nkv}, {PAGE_TOKENS}, {hd}]")
+    if not (v_cache.shape == (k_cache.shape[0], nkv, hd, PAGE_TOKENS) and v_cache.dtype == k_cache.dtype):
+        raise KernelError(f"{what}: value cache {tuple(v_cache.shape)} is not [pages, {nkv}, {hd}, {PAGE_TOKENS}] (values are kept transposed)")
+    if not (block_table.dim() == 2):
+        raise KernelError(f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
 
 
 def qk_norm_rope_store(qkv: torch.Tensor, nh: int, nkv: int, hd: int, positions: torch.Tensor, *, q_norm_w=None,
@@ -252,27 +265,32 @@ def qk_norm_rope_store(qkv: torch.Tensor, nh: int, nkv: int, hd: int, positions:
         _need(planes >= 2 or out_dtype == F32, "qk_norm_rope_store: a single plane comes as rows of the result's type")
         n = qkv.shape[1]
     else:
-        _need(qkv.dim() == 2, f"qk_norm_rope_store: qkv {tuple(qkv.shape)}")
+        if not (qkv.dim() == 2):
+            raise KernelError(f"qk_norm_rope_store: qkv {tuple(qkv.shape)}")
         n = qkv.shape[0]
         out_dtype = out_dtype or qkv.dtype
         _need(out_dtype == qkv.dtype, "qk_norm_rope_store: q and the cache have the type of qkv unless qkv comes in planes")
-    _need(qkv.shape[-1] == (nh + 2 * nkv) * hd, f"qk_norm_rope_store: qkv {tuple(qkv.shape)} is not "
-          f"[n, ({nh} + 2*{nkv}) * {hd}]")
+    if not (qkv.shape[-1] == (nh + 2 * nkv) * hd):
+        raise KernelError(f"qk_norm_rope_store: qkv {tuple(qkv.shape)} is not "
+                          f"[n, ({nh} + 2*{nkv}) * {hd}]")
     _need(positions.shape == (n,), "qk_norm_rope_store: one position for each token")
     for w, nm in ((q_norm_w, "q"), (k_norm_w, "k")):
-        _need(w is None or (w.shape == (hd,) and w.dtype == F32), f"qk_norm_rope_store: {nm} norm weight must be float32 [{hd}]")
+        if not (w is None or (w.shape == (hd,) and w.dtype == F32)):
+            raise KernelError(f"qk_norm_rope_store: {nm} norm weight must be float32 [{hd}]")
     _need((cos is None) == (sin is None), "qk_norm_rope_store: cos and sin come together")
     if cos is not None:
-        _need(0 < rotary_dim <= hd and rotary_dim % 2 == 0, f"qk_norm_rope_store: rotary_dim {rotary_dim}, head_dim {hd}")
+        if not (0 < rotary_dim <= hd and rotary_dim % 2 == 0):
+            raise KernelError(f"qk_norm_rope_store: rotary_dim {rotary_dim}, head_dim {hd}")
         for tab in (cos, sin):
-            _need(tab.dtype == F32 and tab.shape == (n, rotary_dim // 2),
-                  f"qk_norm_rope_store: rotation table {tuple(tab.shape)} {tab.dtype} is not float32 [{n}, {rotary_dim // 2}]")
+            if not (tab.dtype == F32 and tab.shape == (n, rotary_dim // 2)):
+                raise KernelError(f"qk_norm_rope_store: rotation table {tuple(tab.shape)} {tab.dtype} is not float32 [{n}, {rotary_dim // 2}]")
     max_pages = 0
     if write_cache:
         _need(k_cache is not None and v_cache is not None and block_table is not None and tok_slot is not None,
               "qk_norm_rope_store: writing the cache needs cache, page table and slots")
         _check_cache("qk_norm_rope_store", k_cache, v_cache, block_table, nkv, hd)
-        _need(k_cache.dtype == out_dtype, f"qk_norm_rope_store: cache is {k_cache.dtype}, activations are {out_dtype}")
+        if not (k_cache.dtype == out_dtype):
+            raise KernelError(f"qk_norm_rope_store: cache is {k_cache.dtype}, activations are {out_dtype}")
         _need(tok_slot.shape == (n,), "qk_norm_rope_store: one slot for each token")
         max_pages = block_table.shape[1]
     q_out = torch.empty((n, nh * hd), dtype=out_dtype, device=qkv.device)
@@ -302,9 +320,11 @@ def attention_exact(q: torch.Tensor, k_cache, v_cache, block_table, seq_slot, se
     _dev("attention", q, k_cache, v_cache, block_table, seq_slot, seq_start, seq_new, cu_new)
     _i32("attention", block_table, seq_slot, seq_start, seq_new, cu_new)
     n = q.shape[0]
-    _need(q.dim() == 2 and q.shape[1] == nh * hd, f"attention: q {tuple(q.shape)} is not [n, {nh}*{hd}]")
+    if not (q.dim() == 2 and q.shape[1] == nh * hd):
+        raise KernelError(f"attention: q {tuple(q.shape)} is not [n, {nh}*{hd}]")
     _check_cache("attention", k_cache, v_cache, block_table, nkv, hd)
-    _need(k_cache.dtype == q.dtype, f"attention: cache is {k_cache.dtype}, queries are {q.dtype}")
+    if not (k_cache.dtype == q.dtype):
+        raise KernelError(f"attention: cache is {k_cache.dtype}, queries are {q.dtype}")
     B = seq_slot.shape[0]
     _need(seq_start.shape == (B,) and seq_new.shape == (B,) and cu_new.shape == (B + 1,),
           "attention: per-sequence arrays differ in length")
@@ -319,7 +339,8 @@ def attention_exact(q: torch.Tensor, k_cache, v_cache, block_table, seq_slot, se
 
 def argmax(logits: torch.Tensor) -> torch.Tensor:
     _dev("argmax", logits)
-    _need(logits.dim() == 2 and logits.dtype == F32, f"argmax: logits {tuple(logits.shape)} {logits.dtype}")
+    if not (logits.dim() == 2 and logits.dtype == F32):
+        raise KernelError(f"argmax: logits {tuple(logits.shape)} {logits.dtype}")
     out = torch.empty((logits.shape[0],), dtype=torch.int32, device=logits.device)
     library.call(core(), "palm_argmax", _stream(), _p(logits), logits.shape[0], logits.shape[1], _p(out))
     return out
@@ -339,8 +360,8 @@ def uniforms_into(out: torch.Tensor, seed: int, streams, draws) -> None:
     """out[i], a float32 in host memory, = the uniform number of (seed, streams[i], draws[i]), as ``sampling.uniform`` makes one
     (one by one in Python 33 of them took some 60 us, longer than the draw itself)."""
     s, d = _u64(streams), _u64(draws)
-    _need(out.device.type == "cpu" and out.dtype == F32 and out.is_contiguous() and out.shape == (len(s),) and len(s) == len(d),
-          f"uniforms: {out.dtype} {tuple(out.shape)} on {out.device} for {len(s)} streams and {len(d)} draws")
+    if not (out.device.type == "cpu" and out.dtype == F32 and out.is_contiguous() and out.shape == (len(s),) and len(s) == len(d)):
+        raise KernelError(f"uniforms: {out.dtype} {tuple(out.shape)} on {out.device} for {len(s)} streams and {len(d)} draws")
     library.call(core(), "palm_uniforms", int(seed) & _U64, s.buffer_info()[0], d.buffer_info()[0], len(s), out.data_ptr())
 
 
@@ -359,7 +380,8 @@ def sample(logits: torch.Tensor, uniforms: torch.Tensor | None, temperature: flo
     """One token for each row.  ``uniforms`` [rows] float32 in [0, 1).  With want_probs also the
     distribution that was drawn from, [rows, vocab]."""
     _dev("sample", logits, uniforms)
-    _need(logits.dim() == 2 and logits.dtype == F32, f"sample: logits {tuple(logits.shape)} {logits.dtype}")
+    if not (logits.dim() == 2 and logits.dtype == F32):
+        raise KernelError(f"sample: logits {tuple(logits.shape)} {logits.dtype}")
     n, V = logits.shape
     _need(uniforms is None or (uniforms.shape == (n,) and uniforms.dtype == F32), "sample: uniforms must be float32 [rows]")
     out = torch.empty((n,), dtype=torch.int32, device=logits.device)
@@ -383,8 +405,8 @@ def linear_library(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     accumulation, bfloat16 result: the one place where a library computes on the product path."""
     _dev("linear", a, w)
     _need(a.dtype == BF16 and w.dtype == BF16, "linear_library serves bfloat16 operands only")
-    _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1],
-          f"linear: a {tuple(a.shape)} and w {tuple(w.shape)} do not share the inner size")
+    if not (a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]):
+        raise KernelError(f"linear: a {tuple(a.shape)} and w {tuple(w.shape)} do not share the inner size")
     recorder = profile.active()
     if recorder is not None:
         return recorder.around("library_matmul", lambda: torch.matmul(a, w.t()))
@@ -467,12 +489,13 @@ def linear_mid(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: 
     float32 ([M, N/2] bfloat16 when ``gated``), or, if ``planes_ok`` and the weight rows are few, float32 planes
     [P, M, N] over ranges of K."""
     _dev("linear_mid", a, w)
-    _need(a.dtype == BF16 and w.dtype == BF16 and a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]
-          and a.is_contiguous() and w.is_contiguous(),
-          f"linear_mid: a {tuple(a.shape)} {a.dtype} and w {tuple(w.shape)} {w.dtype} (bfloat16, one inner size)")
+    if not (a.dtype == BF16 and w.dtype == BF16 and a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]
+            and a.is_contiguous() and w.is_contiguous()):
+        raise KernelError(f"linear_mid: a {tuple(a.shape)} {a.dtype} and w {tuple(w.shape)} {w.dtype} (bfloat16, one inner size)")
     M, K = a.shape
     N = w.shape[0]
-    _need(K % MID_CHUNK == 0, f"linear_mid: K = {K} is no multiple of {MID_CHUNK}")
+    if not (K % MID_CHUNK == 0):
+        raise KernelError(f"linear_mid: K = {K} is no multiple of {MID_CHUNK}")
     _need(not gated or (N % 2 == 0 and out_dtype == BF16), "linear_mid: a gated product has an even number of weight rows and a bfloat16 result")
     planes = core().palm_linear_mid_parts(M, N, K, 0) if planes_ok and not gated else 1
     if planes > 1:
@@ -519,8 +542,8 @@ def linear_big(a: torch.Tensor, w: torch.Tensor, gated: bool = False) -> torch.T
     """bfloat16 a [M, K] . w [N, K]^T for a prompt's rows in tiles of up to 256 x 256; [M, N] in bfloat16, or with ``gated`` (w: gate
     rows over up rows) silu(gate) * up, [M, N / 2]."""
     _dev("linear_big", a, w)
-    _need(a.dtype == BF16 and w.dtype == BF16 and a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1],
-          f"linear_big: a {tuple(a.shape)} {a.dtype} and w {tuple(w.shape)} {w.dtype} (bfloat16, one inner size)")
+    if not (a.dtype == BF16 and w.dtype == BF16 and a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]):
+        raise KernelError(f"linear_big: a {tuple(a.shape)} {a.dtype} and w {tuple(w.shape)} {w.dtype} (bfloat16, one inner size)")
     M, K = a.shape
     N = w.shape[0]
     out = torch.empty((M, N // 2 if gated else N), dtype=BF16, device=a.device)
@@ -540,17 +563,20 @@ def _row_ss(what: str, a: torch.Tensor, row_ss) -> int:
     if row_ss is None:
         return 0
     _dev(what, a, row_ss)
-    _need(row_ss.dim() == 2 and row_ss.shape[0] == a.shape[0] and row_ss.dtype == F32 and row_ss.is_contiguous()
-          and row_ss.shape[1] > 0, f"{what}: sums of squares {tuple(row_ss.shape)} {row_ss.dtype} for {a.shape[0]} rows")
-    _need(a.shape[0] <= THIN_TOKENS and thin_serves(a, a), f"{what}: a norm is folded into products of at most {THIN_TOKENS} bfloat16 rows")
+    if not (row_ss.dim() == 2 and row_ss.shape[0] == a.shape[0] and row_ss.dtype == F32 and row_ss.is_contiguous()
+            and row_ss.shape[1] > 0):
+        raise KernelError(f"{what}: sums of squares {tuple(row_ss.shape)} {row_ss.dtype} for {a.shape[0]} rows")
+    if not (a.shape[0] <= THIN_TOKENS and thin_serves(a, a)):
+        raise KernelError(f"{what}: a norm is folded into products of at most {THIN_TOKENS} bfloat16 rows")
     return row_ss.shape[1]
 
 
 def scale_rows(a: torch.Tensor, row_ss: torch.Tensor, eps: float) -> torch.Tensor:
     """a[r] / sqrt(sum of row_ss[r, :] / width + eps): rows that lack their norm's factor, made whole."""
     _dev("scale_rows", a, row_ss)
-    _need(a.dim() == 2 and row_ss.dim() == 2 and row_ss.shape[0] == a.shape[0] and row_ss.dtype == F32 and row_ss.is_contiguous()
-          and row_ss.shape[1] > 0, f"scale_rows: rows {tuple(a.shape)}, sums of squares {tuple(row_ss.shape)} {row_ss.dtype}")
+    if not (a.dim() == 2 and row_ss.dim() == 2 and row_ss.shape[0] == a.shape[0] and row_ss.dtype == F32 and row_ss.is_contiguous()
+            and row_ss.shape[1] > 0):
+        raise KernelError(f"scale_rows: rows {tuple(a.shape)}, sums of squares {tuple(row_ss.shape)} {row_ss.dtype}")
     out = torch.empty_like(a)
     library.call(core(), "palm_scale_rows", _stream(), _p(a), _code(a, "scale_rows"), _p(row_ss), row_ss.shape[1], a.shape[0],
                  float(eps), a.shape[1], _p(out))
@@ -565,9 +591,11 @@ def linear_thin_into_residual(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor,
     _dev("linear_thin_into_residual", a, w, x, norm_w)
     M, K = a.shape
     N = w.shape[0]
-    _need(thin_serves(a, w) and M <= THIN_TOKENS and w.shape[1] == K, f"linear_thin_into_residual: a {tuple(a.shape)} {a.dtype}, "
-          f"w {tuple(w.shape)} {w.dtype} (bfloat16, at most {THIN_TOKENS} rows, K a multiple of 8)")
-    _need(x.shape == (M, N) and x.dtype == F32 and x.is_contiguous(), f"linear_thin_into_residual: residual {tuple(x.shape)} {x.dtype}")
+    if not (thin_serves(a, w) and M <= THIN_TOKENS and w.shape[1] == K):
+        raise KernelError(f"linear_thin_into_residual: a {tuple(a.shape)} {a.dtype}, "
+                          f"w {tuple(w.shape)} {w.dtype} (bfloat16, at most {THIN_TOKENS} rows, K a multiple of 8)")
+    if not (x.shape == (M, N) and x.dtype == F32 and x.is_contiguous()):
+        raise KernelError(f"linear_thin_into_residual: residual {tuple(x.shape)} {x.dtype}")
     _need(norm_w.shape == (N,) and norm_w.dtype == F32, "linear_thin_into_residual: the norm's weight is float32 [N]")
     pieces = _row_ss("linear_thin_into_residual", a, row_ss)
     values = torch.empty((M, N), dtype=BF16, device=a.device)
@@ -594,11 +622,12 @@ def linear_thin(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated:
         out = linear_exact(a, w, out_dtype)
         return swiglu(out) if gated else out
     _dev("linear_thin", a, w)
-    _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1],
-          f"linear: a {tuple(a.shape)} and w {tuple(w.shape)} do not share the inner size")
+    if not (a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]):
+        raise KernelError(f"linear: a {tuple(a.shape)} and w {tuple(w.shape)} do not share the inner size")
     M, K = a.shape
     N = w.shape[0]
-    _need(not gated or N % 2 == 0, f"linear_thin: a gated product needs an even number of weight rows, got {N}")
+    if not (not gated or N % 2 == 0):
+        raise KernelError(f"linear_thin: a gated product needs an even number of weight rows, got {N}")
     out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=a.device)
     if M <= THIN_TOKENS:
         planes = core().palm_linear_thin_parts(M, N, K) if planes_ok and not gated else 1
@@ -607,7 +636,8 @@ def linear_thin(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated:
         library.call(core(), "palm_linear_thin", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_thin out"), M, N, K,
                      1 if gated else 0, planes, _p(row_ss), pieces, float(row_eps), None, None, None)
         return out
-    _need(row_ss is None, f"linear_thin: rows that lack their norm's factor come at most {THIN_TOKENS} at a time, not {M}")
+    if not (row_ss is None):
+        raise KernelError(f"linear_thin: rows that lack their norm's factor come at most {THIN_TOKENS} at a time, not {M}")
     if M > WIDE_TOKENS or (M > WIDE_FLOAT32_TOKENS and out_dtype == F32 and not planes_ok):
         # a float32 result for many rows (logits at many places): the tiled kernel, which reads the weight once for
         # every 256 rows; where K is no whole number of its stages, 64 rows at a time
@@ -639,8 +669,9 @@ def linear_tile(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, planes
     ``planes_ok``: the caller takes float32 planes [P, M, N] of partial sums (see linear_thin); the kernel then
     cuts K into ranges where the tiles alone would leave most of the chip without work."""
     _dev("linear_tile", a, w)
-    _need(a.dim() == 2 and w.dim() == 2 and tile_serves(a, w), f"linear_tile: a {tuple(a.shape)} {a.dtype}, w {tuple(w.shape)} "
-          f"{w.dtype} (bfloat16, one inner size, a multiple of {TILE_K})")
+    if not (a.dim() == 2 and w.dim() == 2 and tile_serves(a, w)):
+        raise KernelError(f"linear_tile: a {tuple(a.shape)} {a.dtype}, w {tuple(w.shape)} "
+                          f"{w.dtype} (bfloat16, one inner size, a multiple of {TILE_K})")
     M, K = a.shape
     N = w.shape[0]
     parts = core().palm_linear_tile_parts(M, N, K) if planes_ok else 1
@@ -701,10 +732,13 @@ def decode_slices(n_seqs: int, nh: int, nkv: int, max_keys: int) -> int:
 def _attention_checks(what, q, k_cache, v_cache, block_table, nh, nkv, hd, *index):
     _dev(what, q, k_cache, v_cache, block_table, *index)
     _i32(what, block_table, *index)
-    _need(q.dim() == 2 and q.shape[1] == nh * hd and q.dtype == BF16, f"{what}: q {tuple(q.shape)} {q.dtype} is not bfloat16 [n, {nh}*{hd}]")
-    _need(nh % nkv == 0, f"{what}: {nh} heads are not a multiple of {nkv} kv heads")
+    if not (q.dim() == 2 and q.shape[1] == nh * hd and q.dtype == BF16):
+        raise KernelError(f"{what}: q {tuple(q.shape)} {q.dtype} is not bfloat16 [n, {nh}*{hd}]")
+    if not (nh % nkv == 0):
+        raise KernelError(f"{what}: {nh} heads are not a multiple of {nkv} kv heads")
     _check_cache(what, k_cache, v_cache, block_table, nkv, hd)
-    _need(k_cache.dtype == BF16, f"{what}: the cache is {k_cache.dtype}, not bfloat16")
+    if not (k_cache.dtype == BF16):
+        raise KernelError(f"{what}: the cache is {k_cache.dtype}, not bfloat16")
 
 
 def _slices_workspace(what: str, work, B: int, nh: int, n_slices: int, hd: int, device):
@@ -715,8 +749,9 @@ def _slices_workspace(what: str, work, B: int, nh: int, n_slices: int, hd: int, 
     if work is None:
         return torch.empty((need,), dtype=F32, device=device)
     _dev(what, work)
-    _need(work.dtype == F32 and work.numel() >= need, f"{what}: the workspace holds {work.numel()} {work.dtype}, "
-          f"{B} sequences x {nh} heads x {n_slices} slices need {need} float32")
+    if not (work.dtype == F32 and work.numel() >= need):
+        raise KernelError(f"{what}: the workspace holds {work.numel()} {work.dtype}, "
+                          f"{B} sequences x {nh} heads x {n_slices} slices need {need} float32")
     return work
 
 
@@ -763,20 +798,24 @@ def attention_decode_fused(qkv, k_cache, v_cache, block_table, seq_slot, seq_sta
     _dev(what, qkv, k_cache, v_cache, block_table, seq_slot, seq_start, q_norm_w, k_norm_w, cos, sin)
     _i32(what, block_table, seq_slot, seq_start)
     as_planes = qkv.dim() == 3
-    _need(qkv.is_contiguous() and (as_planes and qkv.dtype == F32 or qkv.dim() == 2 and qkv.dtype == BF16),
-          f"{what}: qkv {tuple(qkv.shape)} {qkv.dtype} is neither bfloat16 rows nor float32 planes")
+    if not (qkv.is_contiguous() and (as_planes and qkv.dtype == F32 or qkv.dim() == 2 and qkv.dtype == BF16)):
+        raise KernelError(f"{what}: qkv {tuple(qkv.shape)} {qkv.dtype} is neither bfloat16 rows nor float32 planes")
     B = seq_slot.shape[0]
-    _need(qkv.shape[-2] == B and qkv.shape[-1] == (nh + 2 * nkv) * hd and seq_start.shape == (B,),
-          f"{what}: qkv {tuple(qkv.shape)} is not [.., {B}, ({nh} + 2*{nkv}) * {hd}]")
-    _need(nh % nkv == 0, f"{what}: {nh} heads are not a multiple of {nkv} kv heads")
+    if not (qkv.shape[-2] == B and qkv.shape[-1] == (nh + 2 * nkv) * hd and seq_start.shape == (B,)):
+        raise KernelError(f"{what}: qkv {tuple(qkv.shape)} is not [.., {B}, ({nh} + 2*{nkv}) * {hd}]")
+    if not (nh % nkv == 0):
+        raise KernelError(f"{what}: {nh} heads are not a multiple of {nkv} kv heads")
     _check_cache(what, k_cache, v_cache, block_table, nkv, hd)
-    _need(k_cache.dtype == BF16, f"{what}: the cache is {k_cache.dtype}, not bfloat16")
+    if not (k_cache.dtype == BF16):
+        raise KernelError(f"{what}: the cache is {k_cache.dtype}, not bfloat16")
     for w, nm in ((q_norm_w, "q"), (k_norm_w, "k")):
-        _need(w is None or (w.shape == (hd,) and w.dtype == F32), f"{what}: {nm} norm weight must be float32 [{hd}]")
-    _need((cos is None) == (sin is None), f"{what}: cos and sin come together")
+        if not (w is None or (w.shape == (hd,) and w.dtype == F32)):
+            raise KernelError(f"{what}: {nm} norm weight must be float32 [{hd}]")
+    if not ((cos is None) == (sin is None)):
+        raise KernelError(f"{what}: cos and sin come together")
     for tab in (cos, sin):
-        _need(tab is None or (tab.dtype == F32 and tab.shape == (B, hd // 2) and tab.is_contiguous() and rotary_dim == hd),
-              f"{what}: a rotation table is float32 [{B}, {hd // 2}] over the whole head")
+        if not (tab is None or (tab.dtype == F32 and tab.shape == (B, hd // 2) and tab.is_contiguous() and rotary_dim == hd)):
+            raise KernelError(f"{what}: a rotation table is float32 [{B}, {hd // 2}] over the whole head")
     out = torch.empty((B, nh * hd), dtype=BF16, device=qkv.device)
     work = _slices_workspace(what, work, B, nh, n_slices, hd, qkv.device)
     library.call(attention_lib(hd), "palm_attention_decode_fused", _stream(), _p(qkv), int(as_planes),
@@ -1002,7 +1041,8 @@ def mlstm_lib():
 
 def padded_key_size(dim: int) -> int:
     """The key size that a recurrence over keys of ``dim`` is compiled for."""
-    _need(1 <= dim <= 256, f"a key size of {dim} lies outside 1 to 256")
+    if not (1 <= dim <= 256):
+        raise KernelError(f"a key size of {dim} lies outside 1 to 256")
     return 32 if dim <= 32 else 64 if dim <= 64 else 128 if dim <= 128 else 256
 
 
@@ -1025,14 +1065,16 @@ def add_normed(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps: 
     Returns x in ``out_dtype`` for the branch that reads it next: x itself if that is float32, else a rounded copy
     made in the same pass."""
     _dev("add_normed", x, delta, weight, results, mix)
-    _need(x.dim() == 2 and x.dtype == F32 and delta.shape == x.shape, f"add_normed: x {tuple(x.shape)} {x.dtype}, delta {tuple(delta.shape)}")
+    if not (x.dim() == 2 and x.dtype == F32 and delta.shape == x.shape):
+        raise KernelError(f"add_normed: x {tuple(x.shape)} {x.dtype}, delta {tuple(delta.shape)}")
     n, width = x.shape
-    _need(weight.shape == (width,) and weight.dtype == F32, f"add_normed: the norm's weight is float32 [{width}]")
+    if not (weight.shape == (width,) and weight.dtype == F32):
+        raise KernelError(f"add_normed: the norm's weight is float32 [{width}]")
     planes, stride = 0, 0
     if results is not None:
-        _need(mix is not None and mix.dtype == F32 and mix.dim() == 1 and results.dtype == F32 and results.dim() == 3
-              and results.shape[1:] == x.shape and 1 <= mix.shape[0] <= results.shape[0],
-              f"add_normed: results {tuple(results.shape)} {results.dtype} and {None if mix is None else tuple(mix.shape)} weights")
+        if not (mix is not None and mix.dtype == F32 and mix.dim() == 1 and results.dtype == F32 and results.dim() == 3
+                and results.shape[1:] == x.shape and 1 <= mix.shape[0] <= results.shape[0]):
+            raise KernelError(f"add_normed: results {tuple(results.shape)} {results.dtype} and {None if mix is None else tuple(mix.shape)} weights")
         planes, stride = mix.shape[0], n * width
     else:
         _need(mix is None, "add_normed: weights without results")
@@ -1045,7 +1087,8 @@ def add_normed(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps: 
 def xielu(z: torch.Tensor, pq: torch.Tensor) -> torch.Tensor:
     """z > 0: softplus(p) z^2 + z/2;  z <= 0: (1/2 + softplus(q)) (exp(z) - 1 - z) + z/2, with pq = [p, q] float32."""
     _dev("xielu", z, pq)
-    _need(pq.shape == (2,) and pq.dtype == F32, f"xielu: the two numbers are float32 [2], not {pq.dtype} {tuple(pq.shape)}")
+    if not (pq.shape == (2,) and pq.dtype == F32):
+        raise KernelError(f"xielu: the two numbers are float32 [2], not {pq.dtype} {tuple(pq.shape)}")
     out = torch.empty_like(z)
     library.call(mixers(), "palm_xielu", _stream(), _p(z), _p(out), _code(z, "xielu"), _p(pq), z.numel())
     return out
@@ -1081,20 +1124,23 @@ def retention(qkvg: torch.Tensor, heads: int, dim: int, vdim: int, decay: torch.
     _dev("retention", qkvg, decay, state, cos, sin, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     _i32("retention", ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     n = qkvg.shape[0]
-    _need(qkvg.dim() == 2 and col0 >= 0 and qkvg.shape[1] >= col0 + heads * (2 * dim + 2 * vdim) and (col0 or qkvg.shape[1] == heads * (2 * dim + 2 * vdim)),
-          f"retention: rows {tuple(qkvg.shape)} from column {col0} are not [n, {heads} * (2*{dim} + 2*{vdim})]")
-    _need(decay.shape == (heads,) and decay.dtype == F32, f"retention: one float32 decay for each of {heads} heads")
-    _need(state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32,
-          f"retention: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
+    if not (qkvg.dim() == 2 and col0 >= 0 and qkvg.shape[1] >= col0 + heads * (2 * dim + 2 * vdim) and (col0 or qkvg.shape[1] == heads * (2 * dim + 2 * vdim))):
+        raise KernelError(f"retention: rows {tuple(qkvg.shape)} from column {col0} are not [n, {heads} * (2*{dim} + 2*{vdim})]")
+    if not (decay.shape == (heads,) and decay.dtype == F32):
+        raise KernelError(f"retention: one float32 decay for each of {heads} heads")
+    if not (state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32):
+        raise KernelError(f"retention: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
     _need(n == ctx.n_tokens, "retention: one row for each token of the step")
     if rot:
         for tab in (cos, sin):
-            _need(tab is not None and tab.dtype == F32 and tab.shape == (n, rot // 2), f"retention: rotation rows are float32 [{n}, {rot // 2}]")
+            if not (tab is not None and tab.dtype == F32 and tab.shape == (n, rot // 2)):
+                raise KernelError(f"retention: rotation rows are float32 [{n}, {rot // 2}]")
     out = torch.empty((n, heads * vdim), dtype=qkvg.dtype, device=qkvg.device)
     raw = None
     if joined_norm is not None:
         _dev("retention", joined_norm)
-        _need(joined_norm.shape == (heads * vdim,) and joined_norm.dtype == F32, f"retention: the joined heads' norm weight is float32 [{heads * vdim}]")
+        if not (joined_norm.shape == (heads * vdim,) and joined_norm.dtype == F32):
+            raise KernelError(f"retention: the joined heads' norm weight is float32 [{heads * vdim}]")
         raw = torch.empty((n, heads * vdim), dtype=F32, device=qkvg.device)
     else:
         _need(not gate_sigmoid, "retention: the per-head unit norm comes with a silu gate")
@@ -1133,14 +1179,15 @@ def gla(rows: torch.Tensor, low: torch.Tensor, w2: torch.Tensor, bias: torch.Ten
     _dev(what, rows, w2, bias, norm_w, state, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     _i32(what, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     n, rank = rows.shape[0], w2.shape[0]
-    _need(rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + heads * (2 * dim + 2 * vdim) and n == ctx.n_tokens,
-          f"{what}: rows {tuple(rows.shape)} from column {col0} are not [{ctx.n_tokens}, {heads} * (2*{dim} + 2*{vdim})]")
-    _need(low.is_cuda and low.dtype == F32 and low.shape == (n, rank) and (n == 0 or low.stride(1) == 1),
-          f"{what}: the decays' inputs are float32 [{n}, {rank}] with contiguous rows, not {low.dtype} {tuple(low.shape)}")
-    _need(w2.shape == (rank, heads * dim) and w2.dtype == F32 and bias.shape == (heads * dim,) and bias.dtype == F32 and norm_w.shape == (vdim,)
-          and norm_w.dtype == F32, f"{what}: the decays' weights [{rank}, {heads * dim}] and bias and the norm's weight [{vdim}] are float32")
-    _need(state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32,
-          f"{what}: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
+    if not (rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + heads * (2 * dim + 2 * vdim) and n == ctx.n_tokens):
+        raise KernelError(f"{what}: rows {tuple(rows.shape)} from column {col0} are not [{ctx.n_tokens}, {heads} * (2*{dim} + 2*{vdim})]")
+    if not (low.is_cuda and low.dtype == F32 and low.shape == (n, rank) and (n == 0 or low.stride(1) == 1)):
+        raise KernelError(f"{what}: the decays' inputs are float32 [{n}, {rank}] with contiguous rows, not {low.dtype} {tuple(low.shape)}")
+    if not (w2.shape == (rank, heads * dim) and w2.dtype == F32 and bias.shape == (heads * dim,) and bias.dtype == F32 and norm_w.shape == (vdim,)
+            and norm_w.dtype == F32):
+        raise KernelError(f"{what}: the decays' weights [{rank}, {heads * dim}] and bias and the norm's weight [{vdim}] are float32")
+    if not (state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32):
+        raise KernelError(f"{what}: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
     lib = gla_lib(dim)
     out = torch.empty((n, heads * vdim), dtype=rows.dtype, device=rows.device)
     prep = torch.empty((n, heads, 3, lib.palm_gla_pad()), dtype=F32, device=rows.device) if ctx.max_new > 1 else None
@@ -1165,11 +1212,12 @@ def causal_conv(xz: torch.Tensor, channels: int, weight: torch.Tensor, bias: tor
     _dev("causal_conv", xz, weight, bias, conv_state, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     _i32("causal_conv", ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     taps = weight.shape[1]
-    _need(xz.dim() == 2 and xz.shape[1] >= channels and xz.shape[0] == ctx.n_tokens, f"causal_conv: input {tuple(xz.shape)}")
-    _need(weight.shape == (channels, taps) and weight.dtype == F32 and (bias is None or (bias.shape == (channels,) and bias.dtype == F32)),
-          f"causal_conv: weight {tuple(weight.shape)} {weight.dtype}, bias {None if bias is None else tuple(bias.shape)}")
-    _need(conv_state.dim() == 3 and conv_state.shape[1:] == (max(taps - 1, 0), channels) and conv_state.dtype == F32,
-          f"causal_conv: state {tuple(conv_state.shape)} is not float32 [slots, {taps - 1}, {channels}]")
+    if not (xz.dim() == 2 and xz.shape[1] >= channels and xz.shape[0] == ctx.n_tokens):
+        raise KernelError(f"causal_conv: input {tuple(xz.shape)}")
+    if not (weight.shape == (channels, taps) and weight.dtype == F32 and (bias is None or (bias.shape == (channels,) and bias.dtype == F32))):
+        raise KernelError(f"causal_conv: weight {tuple(weight.shape)} {weight.dtype}, bias {None if bias is None else tuple(bias.shape)}")
+    if not (conv_state.dim() == 3 and conv_state.shape[1:] == (max(taps - 1, 0), channels) and conv_state.dtype == F32):
+        raise KernelError(f"causal_conv: state {tuple(conv_state.shape)} is not float32 [slots, {taps - 1}, {channels}]")
     out = torch.empty((xz.shape[0], channels), dtype=xz.dtype, device=xz.device)
     library.call(mixers(), "palm_causal_conv", _stream(), _p(xz), _code(xz, "causal_conv"), xz.shape[1], _p(weight), _p(bias),
                  _p(conv_state), _p(ctx.seq_slot), _p(ctx.seq_new), _p(ctx.cu_new), ctx.n_seqs, ctx.max_new, xz.shape[0], channels, taps, _p(out))
@@ -1185,14 +1233,18 @@ def selective_scan(u: torch.Tensor, xz: torch.Tensor, bc: torch.Tensor, b_off: i
     _i32("selective_scan", ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     n, C = u.shape
     N = a_log.shape[1]
-    _need(xz.shape == (n, 2 * C) and xz.dtype == u.dtype and bc.dtype == u.dtype and bc.dim() == 2 and bc.shape[0] == n
-          and 0 <= b_off and b_off + N <= bc.shape[1] and 0 <= c_off and c_off + N <= bc.shape[1],
-          f"selective_scan: u {tuple(u.shape)}, xz {tuple(xz.shape)}, bc {tuple(bc.shape)}")
-    _need(dt_linear.shape == (n, C) and dt_linear.dtype == F32, f"selective_scan: step sizes {tuple(dt_linear.shape)} {dt_linear.dtype} are float32 [{n}, {C}]")
+    if not (xz.shape == (n, 2 * C) and xz.dtype == u.dtype and bc.dtype == u.dtype and bc.dim() == 2 and bc.shape[0] == n
+            and 0 <= b_off and b_off + N <= bc.shape[1] and 0 <= c_off and c_off + N <= bc.shape[1]):
+        raise KernelError(f"selective_scan: u {tuple(u.shape)}, xz {tuple(xz.shape)}, bc {tuple(bc.shape)}")
+    if not (dt_linear.shape == (n, C) and dt_linear.dtype == F32):
+        raise KernelError(f"selective_scan: step sizes {tuple(dt_linear.shape)} {dt_linear.dtype} are float32 [{n}, {C}]")
     for v, nm in ((dt_bias, "dt bias"), (d_skip, "D")):
-        _need(v.shape == (C,) and v.dtype == F32, f"selective_scan: {nm} is float32 [{C}]")
-    _need(a_log.shape == (C, N) and a_log.dtype == F32, f"selective_scan: A_log {tuple(a_log.shape)} {a_log.dtype}")
-    _need(state.dim() == 3 and state.shape[1:] == (C, N) and state.dtype == F32, f"selective_scan: state {tuple(state.shape)} {state.dtype}")
+        if not (v.shape == (C,) and v.dtype == F32):
+            raise KernelError(f"selective_scan: {nm} is float32 [{C}]")
+    if not (a_log.shape == (C, N) and a_log.dtype == F32):
+        raise KernelError(f"selective_scan: A_log {tuple(a_log.shape)} {a_log.dtype}")
+    if not (state.dim() == 3 and state.shape[1:] == (C, N) and state.dtype == F32):
+        raise KernelError(f"selective_scan: state {tuple(state.shape)} {state.dtype}")
     _need(n == ctx.n_tokens, "selective_scan: one row for each token of the step")
     out = torch.empty((n, C), dtype=u.dtype, device=u.device)
     library.call(mixers(), "palm_selective_scan", _stream(), _p(u), xz.data_ptr() + C * xz.element_size(), 2 * C, _p(bc), bc.shape[1],
@@ -1202,11 +1254,12 @@ def selective_scan(u: torch.Tensor, xz: torch.Tensor, bc: torch.Tensor, b_off: i
 
 
 def _check_diff_cache(what, k_cache, v_cache, block_table, kv_heads, dim, vdim):
-    _need(k_cache.dim() == 4 and k_cache.shape[1:] == (2 * kv_heads, PAGE_TOKENS, dim),
-          f"{what}: key cache {tuple(k_cache.shape)} is not [pages, 2*{kv_heads}, {PAGE_TOKENS}, {dim}]")
-    _need(v_cache.shape == (k_cache.shape[0], kv_heads, vdim, PAGE_TOKENS) and v_cache.dtype == k_cache.dtype,
-          f"{what}: value cache {tuple(v_cache.shape)} is not [pages, {kv_heads}, {vdim}, {PAGE_TOKENS}]")
-    _need(block_table.dim() == 2, f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
+    if not (k_cache.dim() == 4 and k_cache.shape[1:] == (2 * kv_heads, PAGE_TOKENS, dim)):
+        raise KernelError(f"{what}: key cache {tuple(k_cache.shape)} is not [pages, 2*{kv_heads}, {PAGE_TOKENS}, {dim}]")
+    if not (v_cache.shape == (k_cache.shape[0], kv_heads, vdim, PAGE_TOKENS) and v_cache.dtype == k_cache.dtype):
+        raise KernelError(f"{what}: value cache {tuple(v_cache.shape)} is not [pages, {kv_heads}, {vdim}, {PAGE_TOKENS}]")
+    if not (block_table.dim() == 2):
+        raise KernelError(f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
 
 
 def diff_qkv_store(qkv: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, q_norm_w, k_norm_w, eps: float,
@@ -1217,12 +1270,16 @@ def diff_qkv_store(qkv: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim:
     _dev(what, qkv, q_norm_w, k_norm_w, k_cache, v_cache, block_table, ctx.tok_slot, ctx.positions)
     _i32(what, block_table, ctx.tok_slot, ctx.positions)
     n = qkv.shape[0]
-    _need(qkv.dim() == 2 and qkv.shape[1] == 2 * (heads + kv_heads) * dim + kv_heads * vdim, f"{what}: rows {tuple(qkv.shape)}")
+    if not (qkv.dim() == 2 and qkv.shape[1] == 2 * (heads + kv_heads) * dim + kv_heads * vdim):
+        raise KernelError(f"{what}: rows {tuple(qkv.shape)}")
     for w in (q_norm_w, k_norm_w):
-        _need(w.shape == (dim,) and w.dtype == F32, f"{what}: a norm weight is float32 [{dim}]")
+        if not (w.shape == (dim,) and w.dtype == F32):
+            raise KernelError(f"{what}: a norm weight is float32 [{dim}]")
     _check_diff_cache(what, k_cache, v_cache, block_table, kv_heads, dim, vdim)
-    _need(k_cache.dtype == qkv.dtype, f"{what}: cache is {k_cache.dtype}, activations are {qkv.dtype}")
-    _need(n == ctx.n_tokens, f"{what}: one row for each token of the step")
+    if not (k_cache.dtype == qkv.dtype):
+        raise KernelError(f"{what}: cache is {k_cache.dtype}, activations are {qkv.dtype}")
+    if not (n == ctx.n_tokens):
+        raise KernelError(f"{what}: one row for each token of the step")
     q = torch.empty((n, 2 * heads * dim), dtype=qkv.dtype, device=qkv.device)
     library.call(mixers(), "palm_diff_qkv_store", _stream(), _p(qkv), _code(qkv, what), _p(q), _p(k_cache), _p(v_cache), _p(block_table),
                  block_table.shape[1], _p(ctx.tok_slot), _p(ctx.positions), _p(q_norm_w), _p(k_norm_w), float(eps), n, heads, kv_heads,
@@ -1249,12 +1306,15 @@ def attention_diff_exact(q: torch.Tensor, k_cache, v_cache, block_table, ctx, he
     _dev(what, q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     _i32(what, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     n = q.shape[0]
-    _need(q.dim() == 2 and q.shape[1] == 2 * heads * dim and n == ctx.n_tokens, f"{what}: q {tuple(q.shape)} is not [n, 2*{heads}*{dim}]")
+    if not (q.dim() == 2 and q.shape[1] == 2 * heads * dim and n == ctx.n_tokens):
+        raise KernelError(f"{what}: q {tuple(q.shape)} is not [n, 2*{heads}*{dim}]")
     _check_diff_cache(what, k_cache, v_cache, block_table, kv_heads, dim, vdim)
-    _need(k_cache.dtype == q.dtype, f"{what}: cache is {k_cache.dtype}, queries are {q.dtype}")
+    if not (k_cache.dtype == q.dtype):
+        raise KernelError(f"{what}: cache is {k_cache.dtype}, queries are {q.dtype}")
     out = torch.empty((n, heads * vdim), dtype=q.dtype, device=q.device)
     n_slices = diff_slices(ctx, heads) if n_slices is None else int(n_slices)
-    _need(n_slices == 1 or ctx.is_decode, f"{what}: only a decode step's key ranges are cut into slices")
+    if not (n_slices == 1 or ctx.is_decode):
+        raise KernelError(f"{what}: only a decode step's key ranges are cut into slices")
     work = torch.empty((n * heads * n_slices * 2 * (vdim + 2),), dtype=F32, device=q.device) if n_slices > 1 else None
     library.call(mixers(), "palm_attention_diff", _stream(), _p(q), _code(q, what), _p(k_cache), _p(v_cache), _p(block_table),
                  block_table.shape[1], _p(ctx.seq_slot), _p(ctx.seq_start), _p(ctx.seq_new), _p(ctx.cu_new), ctx.n_seqs, int(ctx.max_new),
@@ -1292,10 +1352,13 @@ def attention_diff_mfma(q: torch.Tensor, k_cache, v_cache, block_table, ctx, hea
     _dev(what, q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     _i32(what, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     n = q.shape[0]
-    _need(diff_mfma_serves(q, dim, vdim), f"{what}: {q.dtype}, key size {dim}, value size {vdim}")
-    _need(q.dim() == 2 and q.shape[1] == 2 * heads * dim and n == ctx.n_tokens, f"{what}: q {tuple(q.shape)} is not [n, 2*{heads}*{dim}]")
+    if not diff_mfma_serves(q, dim, vdim):
+        raise KernelError(f"{what}: {q.dtype}, key size {dim}, value size {vdim}")
+    if not (q.dim() == 2 and q.shape[1] == 2 * heads * dim and n == ctx.n_tokens):
+        raise KernelError(f"{what}: q {tuple(q.shape)} is not [n, 2*{heads}*{dim}]")
     _check_diff_cache(what, k_cache, v_cache, block_table, kv_heads, dim, vdim)
-    _need(k_cache.dtype == BF16, f"{what}: the cache is {k_cache.dtype}, not bfloat16")
+    if not (k_cache.dtype == BF16):
+        raise KernelError(f"{what}: the cache is {k_cache.dtype}, not bfloat16")
     out = torch.empty((n, heads * vdim), dtype=BF16, device=q.device)
     library.call(attention_diff_lib(dim, vdim), "palm_attention_diff_mfma", _stream(), _p(q), _p(k_cache), _p(v_cache), _p(block_table),
                  block_table.shape[1], _p(ctx.seq_slot), _p(ctx.seq_start), _p(ctx.seq_new), _p(ctx.cu_new), ctx.n_seqs, int(ctx.max_new),
@@ -1319,10 +1382,12 @@ def add_normed_scaled(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor
     ``next_weight``: also returns x / sqrt(mean(x^2) + next_eps) * next_weight in ``out_dtype``, made in the same pass
     (what the norm that reads the stream next would give); else returns None."""
     _dev("add_normed_scaled", x, delta, weight, next_weight)
-    _need(x.dim() == 2 and x.dtype == F32 and delta.shape == x.shape, f"add_normed_scaled: x {tuple(x.shape)} {x.dtype}, delta {tuple(delta.shape)}")
+    if not (x.dim() == 2 and x.dtype == F32 and delta.shape == x.shape):
+        raise KernelError(f"add_normed_scaled: x {tuple(x.shape)} {x.dtype}, delta {tuple(delta.shape)}")
     n, width = x.shape
     for w in (weight, next_weight):
-        _need(w is None or (w.shape == (width,) and w.dtype == F32), f"add_normed_scaled: a norm's weight is float32 [{width}]")
+        if not (w is None or (w.shape == (width,) and w.dtype == F32)):
+            raise KernelError(f"add_normed_scaled: a norm's weight is float32 [{width}]")
     out = None
     if next_weight is not None:
         out = torch.empty((n, width), dtype=out_dtype or F32, device=x.device)
@@ -1335,7 +1400,8 @@ def add_normed_scaled(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor
 def softcap(logits: torch.Tensor, cap: float) -> torch.Tensor:
     """logits <- cap * tanh(logits / cap), in place (float32).  Returns logits."""
     _dev("softcap", logits)
-    _need(logits.dtype == F32 and cap > 0, f"softcap: float32 logits and a positive cap, not {logits.dtype} and {cap}")
+    if not (logits.dtype == F32 and cap > 0):
+        raise KernelError(f"softcap: float32 logits and a positive cap, not {logits.dtype} and {cap}")
     library.call(mixers(), "palm_softcap", _stream(), _p(logits), float(cap), logits.numel())
     return logits
 
@@ -1374,15 +1440,16 @@ def delta_rule(u: torch.Tensor, offsets: tuple, b: torch.Tensor, a: torch.Tensor
     _i32(what, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     n = u.shape[0]
     q_off, k_off, v_off = (int(o) for o in offsets)
-    _need(u.dim() == 2 and n == ctx.n_tokens and max(q_off, k_off) + kv_heads * dim <= u.shape[1] and v_off + heads * vdim <= u.shape[1],
-          f"{what}: rows {tuple(u.shape)} do not hold q, k ({kv_heads} x {dim}) and v ({heads} x {vdim}) at {offsets}")
+    if not (u.dim() == 2 and n == ctx.n_tokens and max(q_off, k_off) + kv_heads * dim <= u.shape[1] and v_off + heads * vdim <= u.shape[1]):
+        raise KernelError(f"{what}: rows {tuple(u.shape)} do not hold q, k ({kv_heads} x {dim}) and v ({heads} x {vdim}) at {offsets}")
     for t, cols, dt, nm in ((b, heads, u.dtype, "write strengths"), (a, heads * dim, F32, "decay rows"), (gate, heads * vdim, F32, "gate rows")):
-        _need(t.is_cuda and t.dim() == 2 and t.shape == (n, cols) and t.dtype == dt and (n == 0 or t.stride(1) == 1),
-              f"{what}: the {nm} are {dt} [{n}, {cols}] with contiguous rows, not {t.dtype} {tuple(t.shape)}")
-    _need(a_log.shape == (heads,) and a_log.dtype == F32 and dt_bias.shape == (heads * dim,) and dt_bias.dtype == F32
-          and norm_w.shape == (vdim,) and norm_w.dtype == F32, f"{what}: A_log [{heads}], dt_bias [{heads * dim}] and the norm's weight [{vdim}] are float32")
-    _need(state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32,
-          f"{what}: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
+        if not (t.is_cuda and t.dim() == 2 and t.shape == (n, cols) and t.dtype == dt and (n == 0 or t.stride(1) == 1)):
+            raise KernelError(f"{what}: the {nm} are {dt} [{n}, {cols}] with contiguous rows, not {t.dtype} {tuple(t.shape)}")
+    if not (a_log.shape == (heads,) and a_log.dtype == F32 and dt_bias.shape == (heads * dim,) and dt_bias.dtype == F32
+            and norm_w.shape == (vdim,) and norm_w.dtype == F32):
+        raise KernelError(f"{what}: A_log [{heads}], dt_bias [{heads * dim}] and the norm's weight [{vdim}] are float32")
+    if not (state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32):
+        raise KernelError(f"{what}: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
     out = torch.empty((n, heads * vdim), dtype=u.dtype, device=u.device)
     prep = torch.empty((n, heads, 3, mixers().palm_delta_pad(dim)), dtype=F32, device=u.device)
     beta = torch.empty((n, heads), dtype=F32, device=u.device)
@@ -1414,16 +1481,18 @@ def delta_head(rows: torch.Tensor, ab: torch.Tensor, conv_w: torch.Tensor, conv_
     _i32(what, ctx.tok_slot, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     n, channels = rows.shape[0], 2 * kv_heads * dim + heads * vdim
     taps = conv_w.shape[1]
-    _need(rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + channels + heads * vdim and n == ctx.n_tokens,
-          f"{what}: rows {tuple(rows.shape)} from column {col0} do not hold q, k ({kv_heads} x {dim}), v and gate ({heads} x {vdim}) of {ctx.n_tokens} tokens")
-    _need(ab.is_cuda and ab.dtype == F32 and ab.shape == (n, 2 * heads) and (n == 0 or ab.stride(1) == 1),
-          f"{what}: write strengths and decays are float32 [{n}, {2 * heads}] with contiguous rows, not {ab.dtype} {tuple(ab.shape)}")
-    _need(conv_w.shape == (channels, taps) and conv_w.dtype == F32 and conv_state.dim() == 3 and conv_state.shape[1:] == (taps - 1, channels)
-          and conv_state.dtype == F32, f"{what}: convolution {tuple(conv_w.shape)} with kept inputs {tuple(conv_state.shape)} for {channels} channels")
+    if not (rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + channels + heads * vdim and n == ctx.n_tokens):
+        raise KernelError(f"{what}: rows {tuple(rows.shape)} from column {col0} do not hold q, k ({kv_heads} x {dim}), v and gate ({heads} x {vdim}) of {ctx.n_tokens} tokens")
+    if not (ab.is_cuda and ab.dtype == F32 and ab.shape == (n, 2 * heads) and (n == 0 or ab.stride(1) == 1)):
+        raise KernelError(f"{what}: write strengths and decays are float32 [{n}, {2 * heads}] with contiguous rows, not {ab.dtype} {tuple(ab.shape)}")
+    if not (conv_w.shape == (channels, taps) and conv_w.dtype == F32 and conv_state.dim() == 3 and conv_state.shape[1:] == (taps - 1, channels)
+            and conv_state.dtype == F32):
+        raise KernelError(f"{what}: convolution {tuple(conv_w.shape)} with kept inputs {tuple(conv_state.shape)} for {channels} channels")
     for t, shape, nm in ((a_log, (heads,), "A_log"), (dt_bias, (heads,), "dt_bias"), (norm_w, (vdim,), "the norm's weight")):
-        _need(tuple(t.shape) == shape and t.dtype == F32, f"{what}: {nm} is float32 {shape}, not {t.dtype} {tuple(t.shape)}")
-    _need(state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32,
-          f"{what}: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
+        if not (tuple(t.shape) == shape and t.dtype == F32):
+            raise KernelError(f"{what}: {nm} is float32 {shape}, not {t.dtype} {tuple(t.shape)}")
+    if not (state.dim() == 4 and state.shape[1:] == (heads, dim, vdim) and state.dtype == F32):
+        raise KernelError(f"{what}: state {tuple(state.shape)} {state.dtype} is not float32 [slots, {heads}, {dim}, {vdim}]")
     lib, dev = delta_head_lib(dim), rows.device
     out = torch.empty((n, heads * vdim), dtype=rows.dtype, device=dev)
     prep = torch.empty((n, kv_heads, 2, lib.palm_delta_head_pad()), dtype=F32, device=dev)
@@ -1455,8 +1524,10 @@ def latent_prep(down: torch.Tensor, q_rank: int, kv_off: int, kv_rank: int, rot_
     _dev(what, down, q_norm_w)
     _latent_rows(what, down.dtype, kv_rank, rot_dim, kv_norm_w, rows_cache, block_table, ctx, rows_t, table_t, pairing)
     n = down.shape[0]
-    _need(down.dim() == 2 and n == ctx.n_tokens, f"{what}: rows {tuple(down.shape)} for {ctx.n_tokens} tokens")
-    _need(q_norm_w.shape == (q_rank,) and q_norm_w.dtype == F32, f"{what}: the query norm's weight is float32 [{q_rank}]")
+    if not (down.dim() == 2 and n == ctx.n_tokens):
+        raise KernelError(f"{what}: rows {tuple(down.shape)} for {ctx.n_tokens} tokens")
+    if not (q_norm_w.shape == (q_rank,) and q_norm_w.dtype == F32):
+        raise KernelError(f"{what}: the query norm's weight is float32 [{q_rank}]")
     _latent_rotation(what, cos, sin, n, rot_dim)
     cq = torch.empty((n, q_rank), dtype=down.dtype, device=down.device)
     library.call(latent_lib(), "palm_latent_prep", _stream(), _p(down), _code(down, what), down.shape[1], q_rank, kv_off, kv_rank, rot_dim,
@@ -1469,21 +1540,25 @@ def _latent_rotation(what: str, cos, sin, n: int, rot_dim: int) -> None:
     if rot_dim:
         _dev(what, cos, sin)
         for tab in (cos, sin):
-            _need(tab is not None and tab.dtype == F32 and tab.shape == (n, rot_dim // 2), f"{what}: rotation rows are float32 [{n}, {rot_dim // 2}]")
+            if not (tab is not None and tab.dtype == F32 and tab.shape == (n, rot_dim // 2)):
+                raise KernelError(f"{what}: rotation rows are float32 [{n}, {rot_dim // 2}]")
 
 
 def _latent_rows(what: str, dtype, kv_rank: int, rot_dim: int, kv_norm_w, rows_cache, block_table, ctx, rows_t, table_t, pairing: str) -> None:
     """The checks of whatever writes cache rows of latents."""
     _dev(what, kv_norm_w, rows_cache, block_table, ctx.positions, ctx.tok_slot, rows_t, table_t)
     _i32(what, block_table, ctx.positions, ctx.tok_slot, table_t)
-    _need(pairing in ROTARY_PAIRINGS, f"{what}: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
-    _need(rows_t is None or (table_t is not None and rows_t.dtype == BF16 and rows_t.dim() == 3 and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS)
-                             and table_t.shape == block_table.shape),
-          f"{what}: the transposed copy is bfloat16 [pages, {kv_rank}, {PAGE_TOKENS}] with a page table like the rows'")
-    _need(kv_norm_w.shape == (kv_rank,) and kv_norm_w.dtype == F32, f"{what}: the latent norm's weight is float32 [{kv_rank}]")
-    _need(rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and rows_cache.dtype == dtype,
-          f"{what}: the cache {tuple(rows_cache.shape)} {rows_cache.dtype} is not {dtype} [pages, {PAGE_TOKENS}, {kv_rank + rot_dim}]")
-    _need(block_table.dim() == 2, f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
+    if not (pairing in ROTARY_PAIRINGS):
+        raise KernelError(f"{what}: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
+    if not (rows_t is None or (table_t is not None and rows_t.dtype == BF16 and rows_t.dim() == 3 and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS)
+            and table_t.shape == block_table.shape)):
+        raise KernelError(f"{what}: the transposed copy is bfloat16 [pages, {kv_rank}, {PAGE_TOKENS}] with a page table like the rows'")
+    if not (kv_norm_w.shape == (kv_rank,) and kv_norm_w.dtype == F32):
+        raise KernelError(f"{what}: the latent norm's weight is float32 [{kv_rank}]")
+    if not (rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and rows_cache.dtype == dtype):
+        raise KernelError(f"{what}: the cache {tuple(rows_cache.shape)} {rows_cache.dtype} is not {dtype} [pages, {PAGE_TOKENS}, {kv_rank + rot_dim}]")
+    if not (block_table.dim() == 2):
+        raise KernelError(f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
 
 
 @dataclass
@@ -1516,15 +1591,17 @@ def latent_query(q: torch.Tensor, uk: torch.Tensor, cos, sin, heads: int, dim: i
     what = "latent_query"
     _dev(what, uk)
     n = q.shape[0]
-    _need(q.is_cuda and q.dim() == 2 and q.shape[1] == heads * (dim + rot_dim) and (n == 0 or q.stride(1) == 1) and uk.shape == (heads * dim, kv_rank),
-          f"{what}: q {tuple(q.shape)}, key matrix {tuple(uk.shape)} for {heads} heads of {dim} + {rot_dim} and a latent of {kv_rank}")
-    _need(pairing in ROTARY_PAIRINGS, f"{what}: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
+    if not (q.is_cuda and q.dim() == 2 and q.shape[1] == heads * (dim + rot_dim) and (n == 0 or q.stride(1) == 1) and uk.shape == (heads * dim, kv_rank)):
+        raise KernelError(f"{what}: q {tuple(q.shape)}, key matrix {tuple(uk.shape)} for {heads} heads of {dim} + {rot_dim} and a latent of {kv_rank}")
+    if not (pairing in ROTARY_PAIRINGS):
+        raise KernelError(f"{what}: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
     _latent_rotation(what, cos, sin, n, rot_dim)
     keep = _latent_store(what, store, q, kv_rank, rot_dim, ctx, pairing)
     qa = torch.empty((n, heads, kv_rank + rot_dim), dtype=F32, device=q.device)
     if uk_t is not None and q.dtype == BF16 and rot_dim % 8 == 0 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0:
         _dev(what, uk_t)
-        _need(uk_t.shape == (heads, kv_rank, dim) and uk_t.dtype == BF16, f"{what}: transposed key matrices {tuple(uk_t.shape)} {uk_t.dtype}")
+        if not (uk_t.shape == (heads, kv_rank, dim) and uk_t.dtype == BF16):
+            raise KernelError(f"{what}: transposed key matrices {tuple(uk_t.shape)} {uk_t.dtype}")
         library.call(latent_lib(), "palm_latent_query_mfma", _stream(), _p(q), q.stride(0), _p(uk_t), _p(cos), _p(sin), n, heads, dim, rot_dim, kv_rank,
                      ROTARY_PAIRINGS[pairing], _p(qa), *keep)
         return qa
@@ -1539,8 +1616,9 @@ def _latent_store(what: str, store: LatentStore | None, q: torch.Tensor, kv_rank
         return [None, 0, None, 0.0, None, None, None, 0, None, None, None]
     src, n = store.src, q.shape[0]
     _latent_rows(what, q.dtype, kv_rank, rot_dim, store.norm_w, store.rows_cache, store.block_table, ctx, store.rows_t, store.table_t, pairing)
-    _need(src.is_cuda and src.dtype == q.dtype and src.dim() == 2 and src.shape[0] == n == ctx.n_tokens and src.shape[1] >= kv_rank + rot_dim
-          and (n == 0 or src.stride(1) == 1), f"{what}: latents {tuple(src.shape)} {src.dtype} for {ctx.n_tokens} tokens")
+    if not (src.is_cuda and src.dtype == q.dtype and src.dim() == 2 and src.shape[0] == n == ctx.n_tokens and src.shape[1] >= kv_rank + rot_dim
+            and (n == 0 or src.stride(1) == 1)):
+        raise KernelError(f"{what}: latents {tuple(src.shape)} {src.dtype} for {ctx.n_tokens} tokens")
     return [_p(src), src.stride(0), _p(store.norm_w), float(store.eps), _p(ctx.positions), _p(ctx.tok_slot), _p(store.block_table),
             store.block_table.shape[1], _p(store.rows_cache), _p(store.rows_t), _p(store.table_t)]
 
@@ -1590,14 +1668,17 @@ def latent_attention_expanded(q: torch.Tensor, uk: torch.Tensor, uv: torch.Tenso
     _dev(what, uk, uv, rows_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     _i32(what, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     n = q.shape[0]
-    _need(latent_expanded_serves(q, rows_cache, uk, uv, ctx, heads, dim, rot_dim, kv_rank, vdim, window), f"{what}: a long prompt in bfloat16 with "
-          "sizes the kernels take")
-    _need(q.is_cuda and q.shape == (ctx.n_tokens, heads * (dim + rot_dim)) and q.stride(1) == 1, f"{what}: queries {tuple(q.shape)}")
-    _need(uk.shape == (heads * dim, kv_rank) and uv.shape == (heads * vdim, kv_rank), f"{what}: matrices {tuple(uk.shape)}, {tuple(uv.shape)}")
-    _need(rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and block_table.dim() == 2,
-          f"{what}: the cache {tuple(rows_cache.shape)}, page table {tuple(block_table.shape)}")
-    _need(gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == BF16 and gate.stride(1) == 1),
-          f"{what}: the gate is bfloat16 [{n}, {heads}] with contiguous rows")
+    if not latent_expanded_serves(q, rows_cache, uk, uv, ctx, heads, dim, rot_dim, kv_rank, vdim, window):
+        raise KernelError(f"{what}: a long prompt in bfloat16 with "
+                          "sizes the kernels take")
+    if not (q.is_cuda and q.shape == (ctx.n_tokens, heads * (dim + rot_dim)) and q.stride(1) == 1):
+        raise KernelError(f"{what}: queries {tuple(q.shape)}")
+    if not (uk.shape == (heads * dim, kv_rank) and uv.shape == (heads * vdim, kv_rank)):
+        raise KernelError(f"{what}: matrices {tuple(uk.shape)}, {tuple(uv.shape)}")
+    if not (rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and block_table.dim() == 2):
+        raise KernelError(f"{what}: the cache {tuple(rows_cache.shape)}, page table {tuple(block_table.shape)}")
+    if not (gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == BF16 and gate.stride(1) == 1)):
+        raise KernelError(f"{what}: the gate is bfloat16 [{n}, {heads}] with contiguous rows")
     _latent_sink(what, sink, heads)
     _latent_rotation(what, cos, sin, n, rot_dim)
     key = ("latent_pages", window)
@@ -1669,16 +1750,19 @@ def latent_attention(qa: torch.Tensor, rows_cache: torch.Tensor, block_table: to
     _dev(what, qa, rows_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new, rows_t, table_t)
     _i32(what, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new, table_t)
     n = qa.shape[0]
-    _need(qa.shape == (n, heads, kv_rank + rot_dim) and qa.dtype == F32 and n == ctx.n_tokens, f"{what}: queries {tuple(qa.shape)} {qa.dtype}")
-    _need(rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim),
-          f"{what}: the cache {tuple(rows_cache.shape)} is not [pages, {PAGE_TOKENS}, {kv_rank + rot_dim}]")
-    _need(block_table.dim() == 2, f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
+    if not (qa.shape == (n, heads, kv_rank + rot_dim) and qa.dtype == F32 and n == ctx.n_tokens):
+        raise KernelError(f"{what}: queries {tuple(qa.shape)} {qa.dtype}")
+    if not (rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim)):
+        raise KernelError(f"{what}: the cache {tuple(rows_cache.shape)} is not [pages, {PAGE_TOKENS}, {kv_rank + rot_dim}]")
+    if not (block_table.dim() == 2):
+        raise KernelError(f"{what}: page table {tuple(block_table.shape)} is not [slots, pages]")
     _latent_sink(what, sink, heads)
     out = torch.empty((n, heads, kv_rank), dtype=F32, device=qa.device)
     if rows_t is not None and not ctx.is_decode and latent_mfma_serves(rows_cache, kv_rank, rot_dim):
-        _need(table_t is not None and rows_t.dtype == BF16 and rows_t.dim() == 3 and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS)
-              and table_t.shape == block_table.shape, f"{what}: the transposed copy is bfloat16 [pages, {kv_rank}, {PAGE_TOKENS}] with a page "
-              "table like the rows'")
+        if not (table_t is not None and rows_t.dtype == BF16 and rows_t.dim() == 3 and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS)
+                and table_t.shape == block_table.shape):
+            raise KernelError(f"{what}: the transposed copy is bfloat16 [pages, {kv_rank}, {PAGE_TOKENS}] with a page "
+                              "table like the rows'")
         library.call(latent_attention_lib(kv_rank, rot_dim), "palm_latent_attention_mfma", _stream(), _p(qa), _p(rows_cache), _p(rows_t),
                      _p(block_table), _p(table_t), block_table.shape[1], _p(ctx.seq_slot), _p(ctx.seq_start), _p(ctx.seq_new), _p(ctx.cu_new),
                      ctx.n_seqs, int(ctx.max_new), heads, kv_rank, rot_dim, float(scale), int(window or 0), _p(sink), _p(out), None, None, 0, 0, None)
@@ -1692,7 +1776,8 @@ def latent_attention(qa: torch.Tensor, rows_cache: torch.Tensor, block_table: to
 def _latent_sink(what: str, sink, heads: int) -> None:
     if sink is not None:
         _dev(what, sink)
-        _need(sink.shape == (heads,) and sink.dtype == F32, f"{what}: learned sink scores are float32 [{heads}], not {sink.dtype} {tuple(sink.shape)}")
+        if not (sink.shape == (heads,) and sink.dtype == F32):
+            raise KernelError(f"{what}: learned sink scores are float32 [{heads}], not {sink.dtype} {tuple(sink.shape)}")
 
 
 # a decode step's key ranges are cut into slices until about this many blocks run (measured with 8 sequences of 2,048 tokens,
@@ -1723,14 +1808,17 @@ def latent_attention_decode(qa: torch.Tensor, rows_cache: torch.Tensor, block_ta
     _dev(what, qa, rows_cache, block_table, ctx.seq_slot, ctx.seq_start, rows_t, table_t, uv)
     _i32(what, block_table, ctx.seq_slot, ctx.seq_start, table_t)
     n = qa.shape[0]
-    _need(latent_decode_serves(rows_cache, rows_t, uv, ctx, kv_rank, rot_dim), f"{what}: single tokens in bfloat16 with sizes the kernel takes")
-    _need(qa.shape == (n, heads, kv_rank + rot_dim) and qa.dtype == F32 and n == ctx.n_tokens == ctx.n_seqs, f"{what}: queries {tuple(qa.shape)} {qa.dtype}")
-    _need(rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and rows_t.dtype == BF16 and rows_t.dim() == 3
-          and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS) and block_table.dim() == 2 and table_t.shape == block_table.shape,
-          f"{what}: the cache {tuple(rows_cache.shape)}, its transposed copy {tuple(rows_t.shape)}, page tables {tuple(block_table.shape)}")
-    _need(uv.shape == (heads * vdim, kv_rank), f"{what}: value matrix {tuple(uv.shape)} for {heads} heads of {vdim} over a latent of {kv_rank}")
-    _need(gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == BF16 and (n == 0 or gate.stride(1) == 1)),
-          f"{what}: the gate is bfloat16 [{n}, {heads}] with contiguous rows")
+    if not latent_decode_serves(rows_cache, rows_t, uv, ctx, kv_rank, rot_dim):
+        raise KernelError(f"{what}: single tokens in bfloat16 with sizes the kernel takes")
+    if not (qa.shape == (n, heads, kv_rank + rot_dim) and qa.dtype == F32 and n == ctx.n_tokens == ctx.n_seqs):
+        raise KernelError(f"{what}: queries {tuple(qa.shape)} {qa.dtype}")
+    if not (rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and rows_t.dtype == BF16 and rows_t.dim() == 3
+            and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS) and block_table.dim() == 2 and table_t.shape == block_table.shape):
+        raise KernelError(f"{what}: the cache {tuple(rows_cache.shape)}, its transposed copy {tuple(rows_t.shape)}, page tables {tuple(block_table.shape)}")
+    if not (uv.shape == (heads * vdim, kv_rank)):
+        raise KernelError(f"{what}: value matrix {tuple(uv.shape)} for {heads} heads of {vdim} over a latent of {kv_rank}")
+    if not (gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == BF16 and (n == 0 or gate.stride(1) == 1))):
+        raise KernelError(f"{what}: the gate is bfloat16 [{n}, {heads}] with contiguous rows")
     _latent_sink(what, sink, heads)
     slices = latent_slices(ctx, heads, window) if slices is None else int(slices)
     work_ml = torch.empty((n * heads * slices * 2,), dtype=F32, device=qa.device)
@@ -1757,14 +1845,17 @@ def latent_attention_fused(qa: torch.Tensor, rows_cache: torch.Tensor, block_tab
     _dev(what, qa, rows_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new, rows_t, table_t, uv)
     _i32(what, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new, table_t)
     n = qa.shape[0]
-    _need(latent_fused_serves(qa, rows_cache, rows_t, uv, ctx, kv_rank, rot_dim, vdim), f"{what}: a prompt in bfloat16 with sizes the kernel takes")
-    _need(qa.shape == (n, heads, kv_rank + rot_dim) and qa.dtype == F32 and n == ctx.n_tokens, f"{what}: queries {tuple(qa.shape)} {qa.dtype}")
-    _need(rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and rows_t.dtype == BF16 and rows_t.dim() == 3
-          and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS) and block_table.dim() == 2 and table_t.shape == block_table.shape,
-          f"{what}: the cache {tuple(rows_cache.shape)}, its transposed copy {tuple(rows_t.shape)}, page tables {tuple(block_table.shape)}")
-    _need(uv.shape == (heads * vdim, kv_rank), f"{what}: value matrix {tuple(uv.shape)} for {heads} heads of {vdim} over a latent of {kv_rank}")
-    _need(gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == BF16 and (n == 0 or gate.stride(1) == 1)),
-          f"{what}: the gate is bfloat16 [{n}, {heads}] with contiguous rows")
+    if not latent_fused_serves(qa, rows_cache, rows_t, uv, ctx, kv_rank, rot_dim, vdim):
+        raise KernelError(f"{what}: a prompt in bfloat16 with sizes the kernel takes")
+    if not (qa.shape == (n, heads, kv_rank + rot_dim) and qa.dtype == F32 and n == ctx.n_tokens):
+        raise KernelError(f"{what}: queries {tuple(qa.shape)} {qa.dtype}")
+    if not (rows_cache.dim() == 3 and rows_cache.shape[1:] == (PAGE_TOKENS, kv_rank + rot_dim) and rows_t.dtype == BF16 and rows_t.dim() == 3
+            and rows_t.shape[1:] == (kv_rank, PAGE_TOKENS) and block_table.dim() == 2 and table_t.shape == block_table.shape):
+        raise KernelError(f"{what}: the cache {tuple(rows_cache.shape)}, its transposed copy {tuple(rows_t.shape)}, page tables {tuple(block_table.shape)}")
+    if not (uv.shape == (heads * vdim, kv_rank)):
+        raise KernelError(f"{what}: value matrix {tuple(uv.shape)} for {heads} heads of {vdim} over a latent of {kv_rank}")
+    if not (gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == BF16 and (n == 0 or gate.stride(1) == 1))):
+        raise KernelError(f"{what}: the gate is bfloat16 [{n}, {heads}] with contiguous rows")
     _latent_sink(what, sink, heads)
     out = torch.empty((n, heads * vdim), dtype=BF16, device=qa.device)
     library.call(latent_attention_lib(kv_rank, rot_dim), "palm_latent_attention_mfma", _stream(), _p(qa), _p(rows_cache), _p(rows_t),
@@ -1781,10 +1872,10 @@ def latent_output(o_lat: torch.Tensor, uv: torch.Tensor, gate: torch.Tensor | No
     what = "latent_output"
     _dev(what, o_lat, uv)
     n = o_lat.shape[0]
-    _need(o_lat.shape == (n, heads, kv_rank) and o_lat.dtype == F32 and uv.shape == (heads * vdim, kv_rank),
-          f"{what}: sums {tuple(o_lat.shape)} {o_lat.dtype}, value matrix {tuple(uv.shape)}")
-    _need(gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == out_dtype and (n == 0 or gate.stride(1) == 1)),
-          f"{what}: the gate is {out_dtype} [{n}, {heads}] with contiguous rows")
+    if not (o_lat.shape == (n, heads, kv_rank) and o_lat.dtype == F32 and uv.shape == (heads * vdim, kv_rank)):
+        raise KernelError(f"{what}: sums {tuple(o_lat.shape)} {o_lat.dtype}, value matrix {tuple(uv.shape)}")
+    if not (gate is None or (gate.is_cuda and gate.shape == (n, heads) and gate.dtype == out_dtype and (n == 0 or gate.stride(1) == 1))):
+        raise KernelError(f"{what}: the gate is {out_dtype} [{n}, {heads}] with contiguous rows")
     out = torch.empty((n, heads * vdim), dtype=out_dtype, device=o_lat.device)
     library.call(latent_lib(), "palm_latent_output", _stream(), _p(o_lat), _p(uv), _code(uv, what + " value matrix"), _p(gate),
                  gate.stride(0) if gate is not None else 0, _code(out, what), n, heads, kv_rank, vdim, _p(out))
@@ -1797,7 +1888,8 @@ def moe_route(logits: torch.Tensor, top: int):
     """logits float32 [n, experts] -> (chosen int32 [n, top], weight float32 [n, top]): the ``top`` largest logits of each
     row, largest first (the lower index wins a tie), and the softmax over them alone."""
     _dev("moe_route", logits)
-    _need(logits.dim() == 2 and logits.dtype == F32, f"moe_route: router logits are float32 [n, experts], not {logits.dtype} {tuple(logits.shape)}")
+    if not (logits.dim() == 2 and logits.dtype == F32):
+        raise KernelError(f"moe_route: router logits are float32 [n, experts], not {logits.dtype} {tuple(logits.shape)}")
     n, experts = logits.shape
     chosen = torch.empty((n, top), dtype=torch.int32, device=logits.device)
     weight = torch.empty((n, top), dtype=F32, device=logits.device)
@@ -1818,20 +1910,24 @@ def expert_rows(form: str) -> int:
 
 def _addends(what: str, add, h):
     """Up to two tensors of rows that other branches made, as addresses (None where there is none)."""
-    _need(len(add) <= 2, f"{what}: {len(add)} rows to add (at most two)")
+    if not (len(add) <= 2):
+        raise KernelError(f"{what}: {len(add)} rows to add (at most two)")
     for y in add:
         _dev(what, y)
-        _need(y.shape == h.shape and y.dtype == h.dtype, f"{what}: rows to add are {h.dtype} {tuple(h.shape)}, not {y.dtype} {tuple(y.shape)}")
+        if not (y.shape == h.shape and y.dtype == h.dtype):
+            raise KernelError(f"{what}: rows to add are {h.dtype} {tuple(h.shape)}, not {y.dtype} {tuple(y.shape)}")
     return [_p(y) for y in add] + [None] * (2 - len(add))
 
 
 def _expert_shapes(what, h, up, down, ff, form):
     """-> (experts, rows of an expert's first matrix): gated experts keep their gate rows before their up rows."""
-    _need(form in EXPERT_FORMS, f"{what}: an expert's form {form!r} is not one of {sorted(EXPERT_FORMS)}")
+    if not (form in EXPERT_FORMS):
+        raise KernelError(f"{what}: an expert's form {form!r} is not one of {sorted(EXPERT_FORMS)}")
     per = expert_rows(form) * ff
     width = h.shape[1]
-    _need(up.dim() == 2 and up.shape[1] == width and up.shape[0] % per == 0 and down.shape == (up.shape[0] // per * width, ff)
-          and up.dtype == down.dtype, f"{what}: first matrices {tuple(up.shape)}, down {tuple(down.shape)} for width {width}, inner size {ff}")
+    if not (up.dim() == 2 and up.shape[1] == width and up.shape[0] % per == 0 and down.shape == (up.shape[0] // per * width, ff)
+            and up.dtype == down.dtype):
+        raise KernelError(f"{what}: first matrices {tuple(up.shape)}, down {tuple(down.shape)} for width {width}, inner size {ff}")
     return up.shape[0] // per
 
 
@@ -1847,11 +1943,14 @@ def moe_route_scored(logits: torch.Tensor, experts: int, top: int, correction: t
     two largest corrected scores (``group_score`` "largest": by its largest), and only experts of the best ``keep`` groups can
     be chosen (the lower index wins a tie); the weights are the chosen scores over their sum (+ 1e-20), times ``scale``."""
     _dev("moe_route_scored", correction)
-    _need(logits.is_cuda and logits.dim() == 2 and (logits.shape[0] == 0 or logits.stride(1) == 1) and logits.dtype == F32 and logits.shape[1] >= experts, f"moe_route_scored: router logits are float32 [n, >= {experts}], "
-          f"not {logits.dtype} {tuple(logits.shape)}")
-    _need(score in ROUTER_SCORES and group_score in GROUP_SCORES, f"moe_route_scored: score {score!r} is one of {sorted(ROUTER_SCORES)}, group_score "
-          f"{group_score!r} one of {sorted(GROUP_SCORES)}")
-    _need(correction is None or (correction.shape == (experts,) and correction.dtype == F32), f"moe_route_scored: the correction is float32 [{experts}]")
+    if not (logits.is_cuda and logits.dim() == 2 and (logits.shape[0] == 0 or logits.stride(1) == 1) and logits.dtype == F32 and logits.shape[1] >= experts):
+        raise KernelError(f"moe_route_scored: router logits are float32 [n, >= {experts}], "
+                          f"not {logits.dtype} {tuple(logits.shape)}")
+    if not (score in ROUTER_SCORES and group_score in GROUP_SCORES):
+        raise KernelError(f"moe_route_scored: score {score!r} is one of {sorted(ROUTER_SCORES)}, group_score "
+                          f"{group_score!r} one of {sorted(GROUP_SCORES)}")
+    if not (correction is None or (correction.shape == (experts,) and correction.dtype == F32)):
+        raise KernelError(f"moe_route_scored: the correction is float32 [{experts}]")
     n = logits.shape[0]
     chosen = torch.empty((n, top), dtype=torch.int32, device=logits.device)
     weight = torch.empty((n, top), dtype=F32, device=logits.device)
@@ -1864,9 +1963,9 @@ def add_gated_rows(out: torch.Tensor, y: torch.Tensor, logits: torch.Tensor, col
     """out[t] += sigmoid(logits[t, column]) * y[t]: out float32 [n, width] in place, logits float32 [n, *]."""
     _dev("add_gated_rows", out, y)
     _need(logits.is_cuda and (logits.shape[0] == 0 or logits.stride(1) == 1), "add_gated_rows: the gate's rows are contiguous and on the GPU")
-    _need(out.dim() == 2 and out.dtype == F32 and y.shape == out.shape and logits.dim() == 2 and logits.dtype == F32
-          and logits.shape[0] == out.shape[0] and 0 <= column < logits.shape[1],
-          f"add_gated_rows: out {tuple(out.shape)} {out.dtype}, y {tuple(y.shape)}, gate column {column} of {tuple(logits.shape)} {logits.dtype}")
+    if not (out.dim() == 2 and out.dtype == F32 and y.shape == out.shape and logits.dim() == 2 and logits.dtype == F32
+            and logits.shape[0] == out.shape[0] and 0 <= column < logits.shape[1]):
+        raise KernelError(f"add_gated_rows: out {tuple(out.shape)} {out.dtype}, y {tuple(y.shape)}, gate column {column} of {tuple(logits.shape)} {logits.dtype}")
     library.call(feedforward(), "palm_add_gated_rows", _stream(), _p(out), _p(y), _code(y, "add_gated_rows"),
                  logits.data_ptr() + column * 4, logits.stride(0), out.shape[0], out.shape[1])
     return out
@@ -1878,7 +1977,8 @@ ACTIVATIONS = {"relu_squared": 0, "gelu_erf": 1, "gelu_tanh": 2}
 def activation(z: torch.Tensor, kind: str) -> torch.Tensor:
     """max(z, 0)^2, or the gelu with erf, or the gelu with tanh, elementwise, 32-bit inside."""
     _dev("activation", z)
-    _need(kind in ACTIVATIONS, f"activation: {kind!r} is not one of {sorted(ACTIVATIONS)}")
+    if not (kind in ACTIVATIONS):
+        raise KernelError(f"activation: {kind!r} is not one of {sorted(ACTIVATIONS)}")
     out = torch.empty_like(z)
     library.call(feedforward(), "palm_activation", _stream(), _p(z), _p(out), _code(z, "activation"), ACTIVATIONS[kind], z.numel())
     return out
@@ -1887,8 +1987,10 @@ def activation(z: torch.Tensor, kind: str) -> torch.Tensor:
 def activation_of_planes(z: torch.Tensor, kind: str, out_dtype: torch.dtype) -> torch.Tensor:
     """``activation`` of a product in float32, [n, m] or planes [P, n, m] of partial sums (see ``linear_thin``); rounded once, to ``out_dtype``."""
     _dev("activation", z)
-    _need(kind in ACTIVATIONS, f"activation: {kind!r} is not one of {sorted(ACTIVATIONS)}")
-    _need(z.dtype == F32 and z.dim() in (2, 3) and z.is_contiguous(), f"activation: {z.dtype} {tuple(z.shape)} are no float32 planes")
+    if not (kind in ACTIVATIONS):
+        raise KernelError(f"activation: {kind!r} is not one of {sorted(ACTIVATIONS)}")
+    if not (z.dtype == F32 and z.dim() in (2, 3) and z.is_contiguous()):
+        raise KernelError(f"activation: {z.dtype} {tuple(z.shape)} are no float32 planes")
     out = torch.empty(z.shape[-2:], dtype=out_dtype, device=z.device)
     library.call(feedforward(), "palm_activation_planes", _stream(), _p(z), z.shape[0] if z.dim() == 3 else 1, _p(out), _code(out, "activation"),
                  ACTIVATIONS[kind], out.numel())
@@ -1900,7 +2002,8 @@ def moe_route_table(ids: torch.Tensor, table: torch.Tensor):
     and 1 / top for each choice.  (An id outside the table takes its nearest row: such a token's logits are no numbers anyway.)"""
     _dev("moe_route_table", ids, table)
     _i32("moe_route_table", ids, table)
-    _need(ids.dim() == 1 and table.dim() == 2, f"moe_route_table: ids {tuple(ids.shape)}, table {tuple(table.shape)}")
+    if not (ids.dim() == 1 and table.dim() == 2):
+        raise KernelError(f"moe_route_table: ids {tuple(ids.shape)}, table {tuple(table.shape)}")
     n, top = ids.shape[0], table.shape[1]
     chosen = torch.empty((n, top), dtype=torch.int32, device=ids.device)
     weight = torch.empty((n, top), dtype=F32, device=ids.device)
@@ -1945,7 +2048,8 @@ def moe_few(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: 
     n, width = h.shape
     top = chosen.shape[1]
     experts, shared_up, shared_down, shared_ff = _check_experts(what, h, gate_up, down, chosen, weight, ff, form, ids, shared)
-    _need(moe_few_serves(h, gate_up, ff, experts, top, shared), f"{what}: at most {FEW_ROWS} bfloat16 rows, bfloat16 weights, sizes in multiples of eight")
+    if not moe_few_serves(h, gate_up, ff, experts, top, shared):
+        raise KernelError(f"{what}: at most {FEW_ROWS} bfloat16 rows, bfloat16 weights, sizes in multiples of eight")
     planes = feedforward().palm_moe_few_planes(width) if planes_ok else 1
     mid = torch.empty((n, top * ff + shared_ff), dtype=BF16, device=h.device)
     out = torch.empty((planes, n, width), dtype=F32, device=h.device)
@@ -1963,16 +2067,18 @@ def _check_experts(what: str, h, gate_up, down, chosen, weight, ff: int, form: s
     top = chosen.shape[1]
     experts = _expert_shapes(what, h, gate_up, down, ff, form)
     if ids is None:
-        _need(chosen.shape == (n, top) and weight is not None and weight.shape == (n, top) and weight.dtype == F32,
-              f"{what}: choices {tuple(chosen.shape)}, weights {None if weight is None else tuple(weight.shape)}")
+        if not (chosen.shape == (n, top) and weight is not None and weight.shape == (n, top) and weight.dtype == F32):
+            raise KernelError(f"{what}: choices {tuple(chosen.shape)}, weights {None if weight is None else tuple(weight.shape)}")
     else:
-        _need(chosen.dim() == 2 and weight is None and ids.shape == (n,), f"{what}: a table of choices {tuple(chosen.shape)} with ids {tuple(ids.shape)} and no weights")
+        if not (chosen.dim() == 2 and weight is None and ids.shape == (n,)):
+            raise KernelError(f"{what}: a table of choices {tuple(chosen.shape)} with ids {tuple(ids.shape)} and no weights")
     shared_up, shared_down = shared if shared is not None else (None, None)
     shared_ff = shared_down.shape[1] if shared is not None else 0
     if shared is not None:
         _dev(what, shared_up, shared_down)
-        _need(shared_up.shape == (expert_rows(form) * shared_ff, width) and shared_down.shape == (width, shared_ff) and shared_up.dtype == gate_up.dtype
-              and shared_down.dtype == gate_up.dtype, f"{what}: the shared expert's matrices {tuple(shared_up.shape)}, {tuple(shared_down.shape)}")
+        if not (shared_up.shape == (expert_rows(form) * shared_ff, width) and shared_down.shape == (width, shared_ff) and shared_up.dtype == gate_up.dtype
+                and shared_down.dtype == gate_up.dtype):
+            raise KernelError(f"{what}: the shared expert's matrices {tuple(shared_up.shape)}, {tuple(shared_down.shape)}")
     return experts, shared_up, shared_down, shared_ff
 
 
@@ -2031,14 +2137,16 @@ def moe_grouped(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chos
     n, width = h.shape
     top = chosen.shape[1]
     experts = _check_experts(what, h, gate_up, down, chosen, weight, ff, form, ids, None)[0]
-    _need(moe_grouped_serves(h, gate_up, ff) and down.dtype == BF16, f"{what}: bfloat16 rows and weights, sizes in multiples of eight")
+    if not (moe_grouped_serves(h, gate_up, ff) and down.dtype == BF16):
+        raise KernelError(f"{what}: bfloat16 rows and weights, sizes in multiples of eight")
     aligned = _starts_on_16(h, gate_up, down)
     n_planes = 0
     if planes is not None:
         _dev(what, planes)
         n_planes = planes.shape[0] if planes.dim() == 3 else 1
-        _need(planes.shape[-2:] == h.shape and planes.dim() in (2, 3) and planes.dtype == F32 and planes.is_contiguous(), f"{what}: planes {planes.dtype} "
-              f"{tuple(planes.shape)} for rows {tuple(h.shape)}")
+        if not (planes.shape[-2:] == h.shape and planes.dim() in (2, 3) and planes.dtype == F32 and planes.is_contiguous()):
+            raise KernelError(f"{what}: planes {planes.dtype} "
+                              f"{tuple(planes.shape)} for rows {tuple(h.shape)}")
     tile = feedforward().palm_moe_tile_tokens(n * top, experts, width, ff, expert_rows(form) > 1, aligned)
     max_tiles = (n * top + tile - 1) // tile + experts
     slots = max_tiles * tile
@@ -2056,7 +2164,8 @@ def gather_rows(h: torch.Tensor, src: torch.Tensor) -> torch.Tensor:
     """xs[p] = h[src[p]] (src int32)."""
     _dev("gather_rows", h, src)
     _i32("gather_rows", src)
-    _need(h.dim() == 2 and src.dim() == 1, f"gather_rows: rows {tuple(h.shape)}, indices {tuple(src.shape)}")
+    if not (h.dim() == 2 and src.dim() == 1):
+        raise KernelError(f"gather_rows: rows {tuple(h.shape)}, indices {tuple(src.shape)}")
     xs = torch.empty((src.shape[0], h.shape[1]), dtype=h.dtype, device=h.device)
     library.call(feedforward(), "palm_gather_rows", _stream(), _p(h), _code(h, "gather_rows"), _p(src), src.shape[0], h.shape[1], _p(xs))
     return xs
@@ -2066,9 +2175,10 @@ def scatter_add(out: torch.Tensor, y: torch.Tensor, rows: torch.Tensor, weight: 
     """out[rows[i]] += weight[i] * y[i]; out float32; the rows must be distinct."""
     _dev("scatter_add", out, y, rows, weight)
     _i32("scatter_add", rows)
-    _need(out.dtype == F32 and out.dim() == 2 and y.dim() == 2 and y.shape[1] == out.shape[1] and rows.shape == (y.shape[0],)
-          and weight.shape == (y.shape[0],) and weight.dtype == F32, f"scatter_add: out {tuple(out.shape)} {out.dtype}, y {tuple(y.shape)}, "
-          f"rows {tuple(rows.shape)}, weights {tuple(weight.shape)} {weight.dtype}")
+    if not (out.dtype == F32 and out.dim() == 2 and y.dim() == 2 and y.shape[1] == out.shape[1] and rows.shape == (y.shape[0],)
+            and weight.shape == (y.shape[0],) and weight.dtype == F32):
+        raise KernelError(f"scatter_add: out {tuple(out.shape)} {out.dtype}, y {tuple(y.shape)}, "
+                          f"rows {tuple(rows.shape)}, weights {tuple(weight.shape)} {weight.dtype}")
     library.call(feedforward(), "palm_scatter_add", _stream(), _p(y), _code(y, "scatter_add"), _p(rows), _p(weight), y.shape[0], out.shape[1], _p(out))
 
 
@@ -2100,33 +2210,39 @@ def sink_qkv_store(rows: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim
     q_size = heads * dim
     k_size, v_size = (kv_heads * dim, kv_heads * vdim) if write_cache else (0, 0)
     channels = q_size + k_size + v_size
-    _need(rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + channels and n == ctx.n_tokens,
-          f"sink_qkv_store: rows {tuple(rows.shape)} for {ctx.n_tokens} tokens of {q_size} + {k_size} + {v_size}")
-    _need(norm in SINK_NORMS, f"sink_qkv_store: norm {norm!r} is not one of {sorted(map(str, SINK_NORMS))}")
-    _need(pairing in ROTARY_PAIRINGS, f"sink_qkv_store: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
+    if not (rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + channels and n == ctx.n_tokens):
+        raise KernelError(f"sink_qkv_store: rows {tuple(rows.shape)} for {ctx.n_tokens} tokens of {q_size} + {k_size} + {v_size}")
+    if not (norm in SINK_NORMS):
+        raise KernelError(f"sink_qkv_store: norm {norm!r} is not one of {sorted(map(str, SINK_NORMS))}")
+    if not (pairing in ROTARY_PAIRINGS):
+        raise KernelError(f"sink_qkv_store: pairing {pairing!r} is not one of {sorted(ROTARY_PAIRINGS)}")
     if bias is not None:
-        _need(bias.shape == (channels,) and bias.dtype == F32, f"sink_qkv_store: the bias is float32 [{channels}]")
+        if not (bias.shape == (channels,) and bias.dtype == F32):
+            raise KernelError(f"sink_qkv_store: the bias is float32 [{channels}]")
     if norm == "head_unit":
         _need(q_w is None and k_w is None, "sink_qkv_store: unit heads have no weights")
     elif norm is not None:
         want = (q_size, kv_heads * dim) if norm == "projection" else (dim, dim)
-        _need(q_w is not None and k_w is not None and q_w.shape == (want[0],) and k_w.shape == (want[1],) and q_w.dtype == F32
-              and k_w.dtype == F32, f"sink_qkv_store: the norm weights are float32 [{want[0]}] and [{want[1]}]")
+        if not (q_w is not None and k_w is not None and q_w.shape == (want[0],) and k_w.shape == (want[1],) and q_w.dtype == F32
+                and k_w.dtype == F32):
+            raise KernelError(f"sink_qkv_store: the norm weights are float32 [{want[0]}] and [{want[1]}]")
     if rot:
         for tab in (cos, sin):
-            _need(tab is not None and tab.dtype == F32 and tab.shape == (n, rot // 2), f"sink_qkv_store: rotation rows are float32 [{n}, {rot // 2}]")
+            if not (tab is not None and tab.dtype == F32 and tab.shape == (n, rot // 2)):
+                raise KernelError(f"sink_qkv_store: rotation rows are float32 [{n}, {rot // 2}]")
     if write_cache:
         _dev("sink_qkv_store", k_cache, v_cache)
-        _need(k_cache.dtype == rows.dtype and v_cache.dtype == rows.dtype and k_cache.shape[1:] == (kv_heads, PAGE_TOKENS, dim)
-              and v_cache.shape[1:] == (kv_heads, vdim, PAGE_TOKENS) and block_table.dim() == 2,
-              f"sink_qkv_store: cache {tuple(k_cache.shape)} / {tuple(v_cache.shape)} {k_cache.dtype} for rows of {rows.dtype}")
+        if not (k_cache.dtype == rows.dtype and v_cache.dtype == rows.dtype and k_cache.shape[1:] == (kv_heads, PAGE_TOKENS, dim)
+                and v_cache.shape[1:] == (kv_heads, vdim, PAGE_TOKENS) and block_table.dim() == 2):
+            raise KernelError(f"sink_qkv_store: cache {tuple(k_cache.shape)} / {tuple(v_cache.shape)} {k_cache.dtype} for rows of {rows.dtype}")
     taps = 0
     if conv is not None:
         taps = conv.shape[1] if conv.dim() == 2 else -1
-        _need(conv.shape == (channels, taps) and conv.dtype == F32 and taps >= 1, f"sink_qkv_store: the convolution is float32 [{channels}, taps], not {tuple(conv.shape)}")
+        if not (conv.shape == (channels, taps) and conv.dtype == F32 and taps >= 1):
+            raise KernelError(f"sink_qkv_store: the convolution is float32 [{channels}, taps], not {tuple(conv.shape)}")
         if taps > 1:
-            _need(conv_state is not None and conv_state.dim() == 3 and conv_state.shape[1:] == (taps - 1, channels) and conv_state.dtype == F32,
-                  f"sink_qkv_store: the convolution's state is float32 [slots, {taps - 1}, {channels}]")
+            if not (conv_state is not None and conv_state.dim() == 3 and conv_state.shape[1:] == (taps - 1, channels) and conv_state.dtype == F32):
+                raise KernelError(f"sink_qkv_store: the convolution's state is float32 [slots, {taps - 1}, {channels}]")
             _dev("sink_qkv_store", ctx.seq_slot, ctx.seq_new, ctx.cu_new)
             _i32("sink_qkv_store", ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     q = torch.empty((n, heads, dim), dtype=rows.dtype, device=rows.device)
@@ -2163,9 +2279,11 @@ def sink_attention_exact(q: torch.Tensor, k_cache, v_cache, block_table, ctx, he
     _dev("sink_attention", q, k_cache, v_cache, block_table, gate, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     _i32("sink_attention", block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     n = q.shape[0]
-    _need(q.shape == (ctx.n_tokens, heads, dim), f"sink_attention: q {tuple(q.shape)} is not [{ctx.n_tokens}, {heads}, {dim}]")
-    _need(k_cache.dtype == q.dtype and v_cache.dtype == q.dtype and k_cache.shape[1:] == (kv_heads, PAGE_TOKENS, dim)
-          and v_cache.shape[1:] == (kv_heads, vdim, PAGE_TOKENS), f"sink_attention: cache {tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
+    if not (q.shape == (ctx.n_tokens, heads, dim)):
+        raise KernelError(f"sink_attention: q {tuple(q.shape)} is not [{ctx.n_tokens}, {heads}, {dim}]")
+    if not (k_cache.dtype == q.dtype and v_cache.dtype == q.dtype and k_cache.shape[1:] == (kv_heads, PAGE_TOKENS, dim)
+            and v_cache.shape[1:] == (kv_heads, vdim, PAGE_TOKENS)):
+        raise KernelError(f"sink_attention: cache {tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
     gate_ptr, gate_stride = _sink_gate("sink_attention", gate, gate_off, n, heads, vdim, q.dtype, gate_per_head)
     sink_score, sink_scores = _sink_scores("sink_attention", sink, heads, q.device)
     _sink_slopes("sink_attention", slopes, heads, window, chunked)
@@ -2184,8 +2302,8 @@ def _sink_gate(what: str, gate, gate_off: int, n: int, heads: int, vdim: int, dt
     if gate is None:
         return None, 0
     cols = heads if per_head else heads * vdim
-    _need(gate.dim() == 2 and gate.shape[0] == n and gate.shape[1] >= gate_off + cols and gate.dtype == dtype,
-          f"{what}: gate rows {tuple(gate.shape)} {gate.dtype} with {cols} columns from column {gate_off}")
+    if not (gate.dim() == 2 and gate.shape[0] == n and gate.shape[1] >= gate_off + cols and gate.dtype == dtype):
+        raise KernelError(f"{what}: gate rows {tuple(gate.shape)} {gate.dtype} with {cols} columns from column {gate_off}")
     return gate.data_ptr() + gate_off * gate.element_size(), gate.shape[1]
 
 
@@ -2193,7 +2311,8 @@ def _sink_scores(what: str, sink, heads: int, device):
     """(one score for all heads, a tensor of one for each or None)."""
     if isinstance(sink, torch.Tensor):
         _dev(what, sink)
-        _need(sink.shape == (heads,) and sink.dtype == F32, f"{what}: learned sink scores are float32 [{heads}], not {sink.dtype} {tuple(sink.shape)}")
+        if not (sink.shape == (heads,) and sink.dtype == F32):
+            raise KernelError(f"{what}: learned sink scores are float32 [{heads}], not {sink.dtype} {tuple(sink.shape)}")
         return 0.0, sink
     return float(sink or 0.0), None
 
@@ -2201,8 +2320,10 @@ def _sink_scores(what: str, sink, heads: int, device):
 def _sink_slopes(what: str, slopes, heads: int, window, chunked: bool) -> None:
     if slopes is not None:
         _dev(what, slopes)
-        _need(slopes.shape == (heads,) and slopes.dtype == F32, f"{what}: the distance bias's slopes are float32 [{heads}], not {slopes.dtype} {tuple(slopes.shape)}")
-    _need(window or not chunked, f"{what}: chunks need their size")
+        if not (slopes.shape == (heads,) and slopes.dtype == F32):
+            raise KernelError(f"{what}: the distance bias's slopes are float32 [{heads}], not {slopes.dtype} {tuple(slopes.shape)}")
+    if not (window or not chunked):
+        raise KernelError(f"{what}: chunks need their size")
 
 
 _SINK_MFMA_SIGNATURE = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
@@ -2236,10 +2357,13 @@ def sink_attention_mfma(q: torch.Tensor, k_cache, v_cache, block_table, ctx, hea
     _dev("sink_attention_mfma", q, k_cache, v_cache, block_table, gate, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     _i32("sink_attention_mfma", block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new)
     n = q.shape[0]
-    _need(sink_mfma_serves(q, dim, vdim), f"sink_attention_mfma: {q.dtype} queries of key size {dim} and value size {vdim} are not served")
-    _need(q.shape == (ctx.n_tokens, heads, dim), f"sink_attention_mfma: q {tuple(q.shape)} is not [{ctx.n_tokens}, {heads}, {dim}]")
-    _need(k_cache.dtype == BF16 and v_cache.dtype == BF16 and k_cache.shape[1:] == (kv_heads, PAGE_TOKENS, dim)
-          and v_cache.shape[1:] == (kv_heads, vdim, PAGE_TOKENS), f"sink_attention_mfma: cache {tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
+    if not sink_mfma_serves(q, dim, vdim):
+        raise KernelError(f"sink_attention_mfma: {q.dtype} queries of key size {dim} and value size {vdim} are not served")
+    if not (q.shape == (ctx.n_tokens, heads, dim)):
+        raise KernelError(f"sink_attention_mfma: q {tuple(q.shape)} is not [{ctx.n_tokens}, {heads}, {dim}]")
+    if not (k_cache.dtype == BF16 and v_cache.dtype == BF16 and k_cache.shape[1:] == (kv_heads, PAGE_TOKENS, dim)
+            and v_cache.shape[1:] == (kv_heads, vdim, PAGE_TOKENS)):
+        raise KernelError(f"sink_attention_mfma: cache {tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
     gate_ptr, gate_stride = _sink_gate("sink_attention_mfma", gate, gate_off, n, heads, vdim, BF16, gate_per_head)
     sink_score, sink_scores = _sink_scores("sink_attention_mfma", sink, heads, q.device)
     _sink_slopes("sink_attention_mfma", slopes, heads, window, chunked)
@@ -2270,14 +2394,16 @@ def add_scaled_normed(x: torch.Tensor, terms, weights, scale: torch.Tensor | Non
     None; the sum in 32-bit, x float32 in place), and what the norm with weight ``norm_w`` makes of the sum, in
     ``out_dtype``.  With ``rows`` only those rows are summed and normed and x stays as it is.  ``norm_w`` None: the sum
     alone is made, and nothing is returned."""
-    _need(1 <= len(terms) <= 2 and len(weights) == len(terms), f"add_scaled_normed: {len(terms)} terms with {len(weights)} weights (one or two)")
+    if not (1 <= len(terms) <= 2 and len(weights) == len(terms)):
+        raise KernelError(f"add_scaled_normed: {len(terms)} terms with {len(weights)} weights (one or two)")
     _dev("add_scaled_normed", x, *terms, scale, norm_w, rows)
     _i32("add_scaled_normed", rows)
     n, width = x.shape
-    _need(x.dtype == F32 and all(t.shape == x.shape and t.dtype == terms[0].dtype for t in terms),
-          f"add_scaled_normed: x {tuple(x.shape)} {x.dtype}, terms {[tuple(t.shape) for t in terms]}")
+    if not (x.dtype == F32 and all(t.shape == x.shape and t.dtype == terms[0].dtype for t in terms)):
+        raise KernelError(f"add_scaled_normed: x {tuple(x.shape)} {x.dtype}, terms {[tuple(t.shape) for t in terms]}")
     for v in (scale, norm_w):
-        _need(v is None or (v.shape == (width,) and v.dtype == F32), f"add_scaled_normed: vectors are float32 [{width}]")
+        if not (v is None or (v.shape == (width,) and v.dtype == F32)):
+            raise KernelError(f"add_scaled_normed: vectors are float32 [{width}]")
     _need(norm_w is not None or rows is None, "add_scaled_normed: a selection of rows is for the norm that reads them")
     n_out = n if rows is None else rows.shape[0]
     out = torch.empty((n_out, width), dtype=out_dtype or F32, device=x.device) if norm_w is not None else None
@@ -2291,8 +2417,8 @@ def add_scaled_normed(x: torch.Tensor, terms, weights, scale: torch.Tensor | Non
 def capped_gate(gate_up: torch.Tensor, limit: float, slope: float, shift: float) -> torch.Tensor:
     """[n, 2 ff] (gate | up; a view of wider rows is fine) -> [n, ff]: g * sigmoid(slope * g) * (u + shift), g = min(gate, limit),
     u = clamp(up, -limit, limit)."""
-    _need(gate_up.is_cuda and gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0 and (gate_up.shape[0] == 0 or gate_up.stride(1) == 1),
-          f"capped_gate: rows {tuple(gate_up.shape)} on {gate_up.device} are not [n, 2 ff] with contiguous rows")
+    if not (gate_up.is_cuda and gate_up.dim() == 2 and gate_up.shape[1] % 2 == 0 and (gate_up.shape[0] == 0 or gate_up.stride(1) == 1)):
+        raise KernelError(f"capped_gate: rows {tuple(gate_up.shape)} on {gate_up.device} are not [n, 2 ff] with contiguous rows")
     n, ff = gate_up.shape[0], gate_up.shape[1] // 2
     out = torch.empty((n, ff), dtype=gate_up.dtype, device=gate_up.device)
     library.call(branches(), "palm_capped_gate", _stream(), _p(gate_up), gate_up.stride(0), _p(out), _code(gate_up, "capped_gate"), n, ff, float(limit),
@@ -2308,7 +2434,8 @@ STREAM_NORMS = {None: 0, "dyt": 1, "rms": 2}
 def streams_spread(x: torch.Tensor, streams: int) -> torch.Tensor:
     """x float32 [n, width] -> [n, streams, width]: every stream starts as a copy of x."""
     _dev("streams_spread", x)
-    _need(x.dim() == 2 and x.dtype == F32 and streams >= 1, f"streams_spread: x {tuple(x.shape)} {x.dtype}, {streams} streams")
+    if not (x.dim() == 2 and x.dtype == F32 and streams >= 1):
+        raise KernelError(f"streams_spread: x {tuple(x.shape)} {x.dtype}, {streams} streams")
     xs = torch.empty((x.shape[0], streams, x.shape[1]), dtype=F32, device=x.device)
     library.call(streams_lib(), "palm_streams_spread", _stream(), _p(x), x.shape[0], int(streams), x.shape[1], _p(xs))
     return xs
@@ -2326,21 +2453,26 @@ def streams_mix_norm(xs: torch.Tensor, y: torch.Tensor | None, mix: torch.Tensor
     what = "streams_mix_norm"
     _dev(what, xs, y, mix, out_w, in_w, norm_w, norm_b, rows)
     _i32(what, rows)
-    _need(xs.dim() == 3 and xs.dtype == F32, f"{what}: the streams are float32 [n, S, width], not {xs.dtype} {tuple(xs.shape)}")
+    if not (xs.dim() == 3 and xs.dtype == F32):
+        raise KernelError(f"{what}: the streams are float32 [n, S, width], not {xs.dtype} {tuple(xs.shape)}")
     n, S, width = xs.shape
-    _need(norm in STREAM_NORMS, f"{what}: norm {norm!r} is not one of {sorted(map(str, STREAM_NORMS))}")
+    if not (norm in STREAM_NORMS):
+        raise KernelError(f"{what}: norm {norm!r} is not one of {sorted(map(str, STREAM_NORMS))}")
     if y is not None:
-        _need(y.shape == (n, width) and mix is not None and mix.shape == (S, S) and mix.dtype == F32 and out_w is not None
-              and out_w.shape == (S,) and out_w.dtype == F32, f"{what}: output {tuple(y.shape)} with weights {None if mix is None else tuple(mix.shape)}, "
-              f"{None if out_w is None else tuple(out_w.shape)} for {S} streams of width {width}")
-    _need(in_w is None or (in_w.shape == (S,) and in_w.dtype == F32), f"{what}: the reader's weights are float32 [{S}]")
-    _need(y is not None or read, f"{what}: neither a write nor a read")
+        if not (y.shape == (n, width) and mix is not None and mix.shape == (S, S) and mix.dtype == F32 and out_w is not None
+                and out_w.shape == (S,) and out_w.dtype == F32):
+            raise KernelError(f"{what}: output {tuple(y.shape)} with weights {None if mix is None else tuple(mix.shape)}, "
+                              f"{None if out_w is None else tuple(out_w.shape)} for {S} streams of width {width}")
+    if not (in_w is None or (in_w.shape == (S,) and in_w.dtype == F32)):
+        raise KernelError(f"{what}: the reader's weights are float32 [{S}]")
+    if not (y is not None or read):
+        raise KernelError(f"{what}: neither a write nor a read")
     out = None
     n_rows = n if rows is None else rows.shape[0]
     if read:
         if norm is not None:
-            _need(norm_w is not None and norm_w.shape == (width,) and norm_w.dtype == F32 and (norm_b is None or (norm_b.shape == (width,) and norm_b.dtype == F32)),
-                  f"{what}: the norm's vectors are float32 [{width}]")
+            if not (norm_w is not None and norm_w.shape == (width,) and norm_w.dtype == F32 and (norm_b is None or (norm_b.shape == (width,) and norm_b.dtype == F32))):
+                raise KernelError(f"{what}: the norm's vectors are float32 [{width}]")
         out = torch.empty((n_rows, width), dtype=out_dtype or F32, device=xs.device)
     if rows is not None and n_rows == 0:
         return out                                  # nothing is read, and a selection leaves the streams as they are
@@ -2381,14 +2513,18 @@ def mlstm(rows: torch.Tensor, gates: torch.Tensor, gate_bias: torch.Tensor | Non
     _i32(what, ctx.seq_slot, ctx.seq_new, ctx.cu_new)
     n = rows.shape[0]
     in_rows = heads * (2 * dim + 2 * vdim)
-    _need(rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + in_rows and n == ctx.n_tokens, f"{what}: rows {tuple(rows.shape)} from column {col0} "
-          f"are not [{ctx.n_tokens}, {heads} * (2*{dim} + 2*{vdim})]")
-    _need(gates.shape == (n, 2 * heads) and gates.dtype == F32, f"{what}: the gates' rows are float32 [{n}, {2 * heads}], not {gates.dtype} {tuple(gates.shape)}")
-    _need(gate_bias is None or (gate_bias.shape == (2 * heads,) and gate_bias.dtype == F32), f"{what}: the gates' bias is float32 [{2 * heads}]")
-    _need(norm_w.shape == (heads * vdim,) and norm_w.dtype == F32, f"{what}: the norm's weight is float32 [{heads * vdim}]")
-    _need(state.dim() == 4 and state.shape[1:] == (heads, dim, vdim + 1) and state.dtype == F32 and m_state.dim() == 2
-          and m_state.shape == (state.shape[0], heads) and m_state.dtype == F32,
-          f"{what}: state {tuple(state.shape)} {state.dtype} / {tuple(m_state.shape)} is not float32 [slots, {heads}, {dim}, {vdim + 1}] / [slots, {heads}]")
+    if not (rows.dim() == 2 and col0 >= 0 and rows.shape[1] >= col0 + in_rows and n == ctx.n_tokens):
+        raise KernelError(f"{what}: rows {tuple(rows.shape)} from column {col0} "
+                          f"are not [{ctx.n_tokens}, {heads} * (2*{dim} + 2*{vdim})]")
+    if not (gates.shape == (n, 2 * heads) and gates.dtype == F32):
+        raise KernelError(f"{what}: the gates' rows are float32 [{n}, {2 * heads}], not {gates.dtype} {tuple(gates.shape)}")
+    if not (gate_bias is None or (gate_bias.shape == (2 * heads,) and gate_bias.dtype == F32)):
+        raise KernelError(f"{what}: the gates' bias is float32 [{2 * heads}]")
+    if not (norm_w.shape == (heads * vdim,) and norm_w.dtype == F32):
+        raise KernelError(f"{what}: the norm's weight is float32 [{heads * vdim}]")
+    if not (state.dim() == 4 and state.shape[1:] == (heads, dim, vdim + 1) and state.dtype == F32 and m_state.dim() == 2
+            and m_state.shape == (state.shape[0], heads) and m_state.dtype == F32):
+        raise KernelError(f"{what}: state {tuple(state.shape)} {state.dtype} / {tuple(m_state.shape)} is not float32 [slots, {heads}, {dim}, {vdim + 1}] / [slots, {heads}]")
     lib = mlstm_lib()
     out = torch.empty((n, heads * vdim), dtype=rows.dtype, device=rows.device)
     chunk = mlstm_chunk(ctx.n_seqs, heads, ctx.max_new) if chunk is None else int(chunk)
