@@ -437,6 +437,8 @@ def _mixer_rooflines(raw: dict, tokens: int, batch: int, context: int) -> dict:
         out["palm_attention_prefill"] = (4.0 * nh * hd * pairs, mfma, None, None)
         kv = 2.0 * batch * context * 2 * nkv * hd
         out["palm_attention_decode_fused"] = out["palm_attention_decode"] = (None, None, kv, hbm)
+    if "palm_moe_few" in out:                       # a step of up to 16 rows, in the sizes that the stream takes
+        out["palm_moe_ring"] = out["palm_moe_few"]
     return out
 
 

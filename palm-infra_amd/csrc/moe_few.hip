@@ -9,6 +9,7 @@
 //          values of the experts in use are dealt to the planes' waves in turn; a piece's products go, weighted, into the wave's
 //          own sums [row, 16 features] in LDS, and the waves' sums are added in their order
 //
+// Steps of up to 16 rows come here only in sizes that the stream of whole lines (moe_ring.hip) does not take.
 // Both kernels are made for up to 16 rows (one column tile) and for more (up to four that share every matrix fragment): the steps
 // of more rows that the grouped products (moe_grouped.hip) do not serve, or whose few tiles there leave the chip idle.
 //

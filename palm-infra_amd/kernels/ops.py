@@ -958,6 +958,9 @@ _FEEDFORWARD_SIGNATURES = {
     "palm_moe_few": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "palm_moe_few_planes": [c_int],
+    "palm_moe_ring": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+    "palm_moe_ring_planes": [c_int],
     "palm_moe_route_table": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p],
     "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int, c_int, c_int],
     "palm_moe_grouped": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
@@ -2040,6 +2043,24 @@ def moe_few_serves(h: torch.Tensor, gate_up: torch.Tensor, ff: int, experts: int
             and h.shape[1] % 8 == 0 and ff % 8 == 0 and (shared is None or (shared[1].shape[1] % 8 == 0 and shared[0].dtype == BF16)))
 
 
+RING_ROWS, RING_EXPERTS, RING_TOP, RING_WIDTH, RING_STEP = 16, 256, 32, 8192, 128
+
+
+def moe_ring_serves(h, gate_up, down, top: int, experts: int, width: int, ff: int, shared_ff: int, shared) -> bool:
+    """Whether a step of few rows goes through the stream of whole lines (``moe_ring.hip``): up to 16 rows (one tile of columns), sizes
+    in whole steps of 128, operands on 16 bytes.  It is the faster way at every size measured that it takes.  Us, blocks by expert and
+    the stream, 1 / 4 / 8 / 16 rows, both products:
+      32 experts of 2,048 x 4,096, four a row, a shared one of 4,096    78 116 182 189    42  95 143 166
+      32 capped experts of 1,536 x 4,096, four a row                   117 142 168 186    35  94 149 174
+      16 gated experts of 1,408 x 2,048, four a row                     46  61  67  69    21  43  52  58
+      128 gated experts of 512 x 2,560, eight a row                     64 107 138 167    21  52  80 137
+      8 experts of 1,024 x 2,048, two a row                             18  24  25  28    11  19  20  23
+      16 experts of 256 x 512, two a row                                11  12  12  13     8   9  10  11"""
+    return (h.shape[0] <= RING_ROWS and experts <= RING_EXPERTS and top <= RING_TOP and width <= RING_WIDTH and width % RING_STEP == 0
+            and ff % RING_STEP == 0 and shared_ff % RING_STEP == 0
+            and all(t.data_ptr() % 16 == 0 for t in (h, gate_up, down, *(shared or ()))))
+
+
 def moe_few(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor | None, ff: int,
             form: str = "gated_silu", cap=NO_CAP, add=(), ids: torch.Tensor | None = None, shared=None, planes_ok: bool = False) -> torch.Tensor:
     """``moe_experts`` on the matrix cores (its arguments): every expert in use is read once for all its rows.  Returns float32
@@ -2050,10 +2071,11 @@ def moe_few(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: 
     experts, shared_up, shared_down, shared_ff = _check_experts(what, h, gate_up, down, chosen, weight, ff, form, ids, shared)
     if not moe_few_serves(h, gate_up, ff, experts, top, shared):
         raise KernelError(f"{what}: at most {FEW_ROWS} bfloat16 rows, bfloat16 weights, sizes in multiples of eight")
-    planes = feedforward().palm_moe_few_planes(width) if planes_ok else 1
+    entry = "palm_moe_ring" if moe_ring_serves(h, gate_up, down, top, experts, width, ff, shared_ff, shared) else "palm_moe_few"
+    planes = getattr(feedforward(), entry + "_planes")(width) if planes_ok else 1
     mid = torch.empty((n, top * ff + shared_ff), dtype=BF16, device=h.device)
     out = torch.empty((planes, n, width), dtype=F32, device=h.device)
-    library.call(feedforward(), "palm_moe_few", _stream(), _p(h), _p(gate_up), _p(down), _p(chosen), _p(weight), _p(ids),
+    library.call(feedforward(), entry, _stream(), _p(h), _p(gate_up), _p(down), _p(chosen), _p(weight), _p(ids),
                  chosen.shape[0] if ids is not None else 0, n, top, experts, width, ff, _p(shared_up), _p(shared_down), shared_ff,
                  EXPERT_FORMS[form], *(float(c) for c in cap), *_addends(what, add, h), _p(mid), planes, _p(out))
     return out if planes > 1 else out[0]

@@ -121,6 +121,41 @@ def test_few_rows(form, E, top, W, F, shared):
 
 
 @gpu
+@pytest.mark.parametrize("form", ["gated_silu", "gelu", "capped_gated", "relu_squared"])
+@pytest.mark.parametrize("E,top,W,F,shared", [(1, 1, 128, 128, None), (4, 2, 128, 384, 128), (33, 4, 1152, 256, None), (256, 32, 384, 128, 256),
+                                              (6, 2, 2048, 640, 1280), (5, 5, 8192, 128, None), (40, 3, 4096, 128, 1152)])
+def test_few_rows_as_one_stream(form, E, top, W, F, shared):
+    """The kernels for up to 16 rows in whole lines: one step of a row of activations and all that a wave holds, waves without any,
+    strips and steps that do not fill the blocks, eight rows and more, choices that repeat an expert, experts that nobody or everybody
+    chose.  The inner rows and the result are rounded where the sum in float64 is not: as in the test above."""
+    from palm_infra_amd.kernels import ops
+    cap = CAP if form == "capped_gated" else ops.NO_CAP
+    for n, uneven, repeats in ((1, False, False), (3, True, True), (8, False, False), (9, True, False), (16, False, True)):
+        h, up, down, chosen, weight = case(form, E, top, W, F, n, uneven, E + F + n, torch.bfloat16)
+        if repeats and top > 1:
+            chosen[0, 1] = chosen[0, 0]
+            chosen[n - 1, top - 1] = chosen[n - 1, 0]
+        want = plain_mixture(form, h, up, down, chosen, weight, F)
+        extra = None
+        if shared:
+            g = torch.Generator().manual_seed(n)
+            per = (2 if form in ("gated_silu", "capped_gated") else 1) * shared
+            extra = ((torch.randn(per, W, generator=g) * W ** -0.5).to(torch.bfloat16), (torch.randn(W, shared, generator=g) * shared ** -0.5).to(torch.bfloat16))
+            want += plain_expert(form, h.double() @ extra[0].double().T, shared) @ extra[1].double().T
+            extra = tuple(t.cuda() for t in extra)
+        args = [t.cuda() for t in (h, up, down, chosen, weight)]
+        assert ops.moe_ring_serves(*args[:3], top, E, W, F, shared or 0, extra)
+        tol = 0.02 * float(want.abs().max())
+        got = ops.moe_few(*args, F, form, cap, shared=extra)
+        assert float((got.cpu().double() - want).abs().max()) <= tol, (n, uneven)
+        assert torch.equal(ops.moe_few(*args, F, form, cap, shared=extra), got)
+        y = [torch.randn(n, W).to(torch.bfloat16).cuda() for _ in range(2)]
+        planes = ops.moe_few(*args, F, form, cap, add=y, shared=extra, planes_ok=True)
+        planes = planes if planes.dim() == 2 else planes.sum(0)
+        assert torch.allclose(planes, got + y[0].float() + y[1].float(), atol=1e-4 * float(want.abs().max()) + 1e-5, rtol=1e-4)
+
+
+@gpu
 @pytest.mark.parametrize("form,E,top,W,F", [("relu_squared", 6, 2, 256, 128), ("gated_silu", 4, 3, 1088, 64), ("capped_gated", 33, 4, 320, 192), ("gelu", 2, 1, 64, 704)])
 def test_grouped_products_in_32_bits_are_as_near_as_the_kernels_for_few_rows(form, E, top, W, F):
     """A step of few rows may take either way: both round the inner rows to bfloat16 and nothing behind them, so their errors against
