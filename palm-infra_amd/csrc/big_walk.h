@@ -1,109 +1,172 @@
-// The walk over K of a tile of a product X . W^T that a block of eight waves owns: 64 NT tokens (rows of X) x 256 rows of W,
+// The walk over K of tiles of a product X . W^T that a block of four waves owns: 64 NT tokens (rows of X) x 256 rows of W,
 // bfloat16, 32-bit sums, for the products of a prompt's rows and of many experts' rows.
 //
+// What bounds it is power: the chip's clock falls as its matrix cores are kept busy (8,192 cubed: 1.6 to 1.7 GHz at 1.2 million
+// cycles, 87 % of which the matrix cores work).  So a wave owns 128 x 32 NT of a tile, 128 x 128 of the largest (its sums are the 256
+// accumulator registers), which reads a third less from LDS than eight waves of 128 x 64 would; and since each wave is alone on its SIMD,
+// it keeps its own matrix cores busy: an instruction goes out every four clocks, a product takes sixteen, and reads of LDS and
+// loads stand between the products one at a time.  (8,192 cubed, on one card: eight waves in two fours that read and multiply in
+// turn 742 us, this walk 717; with four reads or loads in a row between four products and four 790.)
+//
 // K goes by in stages of 64: rows of 128 bytes, a whole cache line, straight from memory into LDS (16 bytes a lane, an
-// instruction fills 8 rows), two stages, features first, then tokens.  A row's eight 16-byte chunks are permuted by the row's
-// number so that the lanes that LDS serves together hit different banks; the lane that fills a place fetches the chunk that
-// belongs there.
-// Waves: 2 (features) x 4 (tokens), a wave owns 128 x 16 NT.  A stage has two halves: the wave's tokens (both k-steps) and
-// its first 64 features are read and multiplied, then its other 64 features.  So three quarters of a stage's rows (set P)
-// are free again after the first half, the rest (set Q) after the second, and each is asked for again at once: a load has one
-// and a half stages to arrive.
-// The waves 0 .. 3 and 4 .. 7, one of each on a SIMD, work half a step apart: while one four read LDS and ask memory, the
-// other four multiply, and a barrier swaps them.  All waits are counted by hand; the loads are not seen by the compiler.
+// instruction fills 8 rows): two stages of W and three of X for the high tiles (160 KB), one more of each for the low ones, whose
+// stages are over sooner (16 experts of 1,024 x 2,048, 17 rows: 65 us with two and three, 55).  A row's eight 16-byte chunks are permuted by
+// the row's number so that the lanes that LDS serves together hit different banks; the lane that fills a place fetches the chunk
+// that belongs there.
+// A stage is four quarters of 4 x 2 NT products: features' first half and second half in the first k-step of 32, both again in the
+// second.  Its operands of the second k-step are read in the first two quarters, those of the next stage's first k-step in the last
+// two, each into the registers of the k-step that is not being multiplied.  So one barrier a stage, between them, is enough: before
+// it a wave has read all of this stage and waited for its share of the next; behind it the places of this stage's W are asked
+// for again at once (quarters three and four), those of X, which has a stage more, in the next stage's first two.
+//
+// Tiles follow each other without a stop: the loads run two (three) stages ahead, into the next tile's where a tile ends, and are on
+// their way while its sums are stored.
 #pragma once
 #include "lds_stage.h"
 #include "mfma.h"
 
-constexpr int BIG_K = 64, BIG_ROW = BIG_K * 2, BIG_WAVES = 8, BIG_THREADS = BIG_WAVES * WAVE;
+#include <type_traits>
+
+constexpr int BIG_K = 64, BIG_ROW = BIG_K * 2, BIG_WAVES = 4, BIG_THREADS = BIG_WAVES * WAVE;
 constexpr int BIG_FEAT = 256, BIG_DIES = 8;
+// stages that the loads run ahead: W has as many places in LDS, X one more
+constexpr int big_ahead(int nt) { return nt <= 2 ? 3 : 2; }
+constexpr int big_lds_bytes(int nt) { return (big_ahead(nt) * BIG_FEAT + (big_ahead(nt) + 1) * 64 * nt) * BIG_ROW; }
 
 __device__ __forceinline__ void big_load(const char* base, uint32_t offset, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds) : "m0", "memory");
 }
-__device__ __forceinline__ void big_swap() {               // the barrier between the two fours of waves
+__device__ __forceinline__ void big_swap() {               // the block's barrier; loads stay on their way
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
 __device__ __forceinline__ void big_lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+__device__ __forceinline__ void big_multiply(f32x4& acc, bf16x8 a, bf16x8 b) {
+    asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+template <int N, int I = 0, class F> __device__ __forceinline__ void big_each(F f) {
+    if constexpr (I < N) { f(std::integral_constant<int, I>{}); big_each<N, I + 1>(f); }
+}
 // A lane of a result tile holds four features of one token.  Row 4 g + v of a wave's f-th of four tiles is feature
 // 16 g + 4 f + v of their 64, so that a lane's four tiles are 16 features side by side.
 __device__ __forceinline__ int big_feature_row(int f, int r) { return 16 * (r / 4) + 4 * f + r % 4; }
 __device__ __forceinline__ int big_w_swizzle(int row) { return ((row >> 1) & 1) | ((row >> 3) & 6); }      // rows big_feature_row(f, 0 .. 15)
 __device__ __forceinline__ int big_x_swizzle(int row) { return (row >> 1) & 7; }                           // 16 rows side by side
 
-// 16 features of one token's row of the result, from feature `at`
+// 16 features of one token's row of the result, from feature `at`; rows are a multiple of eight long
 __device__ __forceinline__ void big_store(bf16_t* __restrict__ row, int at, int width, const float (&v)[16]) {
-    if (at + 16 <= width) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t w[4];
+    for (int h = 0; h < 2; ++h) {
+        uint32_t w[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = (uint32_t)f32_to_bf16(v[8 * h + 2 * i]).bits | ((uint32_t)f32_to_bf16(v[8 * h + 2 * i + 1]).bits << 16);
-            *reinterpret_cast<uint4*>(row + at + 8 * h) = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (at + i < width) row[at + i] = f32_to_bf16(v[i]);
+        for (int i = 0; i < 4; ++i) w[i] = (uint32_t)f32_to_bf16(v[8 * h + 2 * i]).bits | ((uint32_t)f32_to_bf16(v[8 * h + 2 * i + 1]).bits << 16);
+        if (at + 8 * h < width) *reinterpret_cast<uint4*>(row + at + 8 * h) = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
-
 __device__ __forceinline__ void big_store(float* __restrict__ row, int at, int width, const float (&v)[16]) {
-    if (at + 16 <= width) {
 #pragma unroll
-        for (int h = 0; h < 4; ++h) *reinterpret_cast<float4*>(row + at + 4 * h) = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
-    } else {
+    for (int h = 0; h < 4; ++h)
+        if (at + 4 * h < width) *reinterpret_cast<float4*>(row + at + 4 * h) = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+}
+
+// The sums of token tile t, taken from their registers no sooner than here (a tile's all at once would not fit the others).
+template <int TT> __device__ __forceinline__ void big_column(f32x4 (&acc)[8][TT], int t, f32x4 (&a)[8]) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (at + i < width) row[at + i] = v[i];
+    for (int f = 0; f < 8; ++f) {
+        asm volatile("" : "+a"(acc[f][t]));
+        a[f] = acc[f][t];
     }
 }
 
-// x, w: the matrices' first rows and first column of the walk; x_row(i), w_row(i): the rows that are row i of the tile (of 64 NT
-// and of 256); row_bytes from row to row in both.  acc[4 half + f][t][v], lane (r, g) of wave (wave_f, wave_t): token
-// wave_t * 16 NT + 16 t + r, tile row 128 wave_f + 64 half + 16 g + 4 f + v.  TURNED: the walk begins at stage `turn` and wraps.
-template <int NT, bool TURNED, class XRow, class WRow>
-__device__ __forceinline__ void big_walk(char* lds, const void* x, const void* w, uint32_t row_bytes, int stages, int turn, XRow x_row, WRow w_row,
-                                         f32x4 (&acc)[8][NT]) {
-    constexpr int ROWS = BIG_FEAT + 64 * NT, STAGE = ROWS * BIG_ROW;
-    constexpr int P = (64 * NT + 128) / 8 / BIG_WAVES, Q = 128 / 8 / BIG_WAVES;          // a wave's loads of each set
-    static_assert(2 * STAGE <= 160 * 1024 && P * BIG_WAVES * 8 == 64 * NT + 128, "the stages fit LDS, the sets the waves");
+// silu(gate) * up by the hardware's own 2^x and reciprocal, 32-bit and within some units of the last place: a wave alone on its SIMD has
+// nothing to hide the library's 25 instructions behind (13,331 x 24,576 x 4,096 gated: 1,876 us with them, 1,805).  The bfloat16 results'
+// error against 64 bits is the same to six digits, 0.00166.
+__device__ __forceinline__ float big_silu_gated(float gate, float up) {
+    return gate * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gate * -1.4426950408889634f)) * up;
+}
+
+// One tile's walk: where its rows begin (first column of the walk), its stages, and the stage it begins with (it wraps around).
+struct BigItem {
+    const char* x;
+    const char* w;
+    int stages, turn;
+    int x_rows, w_rows;           // rows that there are (beyond them the last one again)
+};
+
+// items: how many tiles the block owns; make(i): the i-th's BigItem, the same in every lane; x_row(item, i), w_row(item, i): where row i
+// of the tile lies, in rows from item.x or item.w (for tiles with the same x_rows and w_rows the same); row_bytes from row to row
+// in both.  finish(i, acc): acc[4 half + f][t][v], lane (r, g) of wave (wave_f, wave_t) = (wave % 2, wave / 2): token
+// wave_t * 32 NT + 16 t + r, tile row 128 wave_f + 64 half + 16 g + 4 f + v.
+template <int NT, bool TURNED, class Make, class XRow, class WRow, class Finish>
+__device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int items, Make make, XRow x_row, WRow w_row, Finish finish) {
+    constexpr int TT = 2 * NT, W_STAGE = BIG_FEAT * BIG_ROW, X_STAGE = 64 * NT * BIG_ROW, GAPS = 4 * TT, A = big_ahead(NT);
+    constexpr int XL = 2 * NT, WL = 8;                       // a wave's loads of a stage, 8 rows each
+    static_assert(A * W_STAGE + (A + 1) * X_STAGE == big_lds_bytes(NT) && big_lds_bytes(NT) <= 160 * 1024, "the stages fit LDS");
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int wave_f = wave % 2, wave_t = wave / 2, r = lane % 16, g = lane / 16;
-    const bool second = wave >= BIG_WAVES / 2;
 
-    // ---- this wave's loads, 8 rows each: of set P the tokens and the first 64 features of each wave_f, of set Q the others
-    uint32_t offset[P + Q], to[P + Q];
-    const char* base[P + Q];
+    // ---- the loads: a cursor that runs A stages ahead of the products
+    uint32_t w_off[WL], x_off[XL];
+    auto offsets_of = [&](const BigItem& item) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < P + Q; ++q) {
-        const int id = q < P ? wave * P + q : wave * Q + q - P, w_id = q < P ? id - 8 * NT : id;
-        const bool tokens = q < P && id < 8 * NT;
-        const int R = tokens ? id * 8 : w_id / 8 * 128 + (q < P ? 0 : 64) + w_id % 8 * 8, row = R + lane / 8;
-        const int chunk = (lane % 8) ^ (tokens ? big_x_swizzle(row) : big_w_swizzle(row));
-        base[q] = reinterpret_cast<const char*>(tokens ? x : w);
-        offset[q] = (uint32_t)(tokens ? x_row(row) : w_row(row)) * row_bytes + chunk * 16;
-        to[q] = (uint32_t)((tokens ? BIG_FEAT : 0) + R) * BIG_ROW;
-    }
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds);
-    // (beyond the last stage the last one's rows again, for nobody: the waits count every wave's loads alike)
-    auto stage_at = [&](int kt) __attribute__((always_inline)) {
-        kt = min(kt, stages - 1);
-        if (TURNED) kt = kt + turn < stages ? kt + turn : kt + turn - stages;
-        return (size_t)kt * BIG_ROW;
+        for (int q = 0; q < WL; ++q) {
+            const int row = (q * BIG_WAVES + wave) * 8 + lane / 8;
+            w_off[q] = (uint32_t)w_row(item, row) * row_bytes + ((lane % 8) ^ big_w_swizzle(row)) * 16;
+        }
+#pragma unroll
+        for (int q = 0; q < XL; ++q) {
+            const int row = (q * BIG_WAVES + wave) * 8 + lane / 8;
+            x_off[q] = (uint32_t)x_row(item, row) * row_bytes + ((lane % 8) ^ big_x_swizzle(row)) * 16;
+        }
     };
-    auto bring_p = [&](int kt, int slot) __attribute__((always_inline)) {
-        const size_t at = stage_at(kt);
-#pragma unroll
-        for (int q = 0; q < P; ++q) big_load(base[q] + at, offset[q], lds0 + slot * STAGE + to[q]);
+    BigItem ahead = make(0);
+    int ahead_item = 0, ahead_left = ahead.stages, ahead_wrap = ahead.stages - ahead.turn;
+    size_t ahead_at = (size_t)ahead.turn * BIG_ROW;
+    offsets_of(ahead);
+    auto advance = [&]() __attribute__((always_inline)) {
+        ahead_at += BIG_ROW;
+        if (TURNED && --ahead_wrap == 0) ahead_at = 0;
+        if (--ahead_left == 0) {
+            if (ahead_item + 1 < items) {
+                const int x_rows = ahead.x_rows, w_rows = ahead.w_rows;
+                ahead = make(++ahead_item);
+                ahead_left = ahead.stages;
+                ahead_wrap = ahead.stages - ahead.turn;
+                ahead_at = (size_t)ahead.turn * BIG_ROW;
+                if (ahead.x_rows != x_rows || ahead.w_rows != w_rows) offsets_of(ahead);
+            } else {                                         // beyond the last: its first stage again, for nobody
+                ahead_left = 1;
+                ahead_wrap = 0;
+                ahead_at = 0;
+            }
+        }
     };
-    auto bring_q = [&](int kt, int slot) __attribute__((always_inline)) {
-        const size_t at = stage_at(kt);
-#pragma unroll
-        for (int q = P; q < P + Q; ++q) big_load(base[q] + at, offset[q], lds0 + slot * STAGE + to[q]);
+    // A load in two parts, with a product between them: where in LDS (m0 stands for an instruction before it is used), and the load.
+    const uint32_t lds_w = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds) + wave * 8 * BIG_ROW;
+    const uint32_t lds_x = lds_w + A * W_STAGE;
+    auto place = [&](uint32_t stage, auto q) __attribute__((always_inline)) {
+        asm volatile("s_add_u32 m0, %0, %1" : : "s"(stage), "i"(decltype(q)::value * BIG_WAVES * 8 * BIG_ROW) : "m0", "scc", "memory");
+    };
+    auto fetch = [&](const char* from, uint32_t offset) __attribute__((always_inline)) {
+        asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(from) : "memory");
+    };
+    // loads FROM .. FROM + COUNT of a stage's, over the gaps of a quarter
+    auto w_loads = [&](int n, auto from, auto count, uint32_t stage) __attribute__((always_inline)) {
+        big_each<decltype(count)::value>([&](auto j) __attribute__((always_inline)) {
+            constexpr int q = decltype(from)::value + decltype(j)::value, gap = decltype(j)::value * GAPS / decltype(count)::value;
+            if (n == gap) place(stage, std::integral_constant<int, q>{});
+            if (n == gap + 1) fetch(ahead.w + ahead_at, w_off[q]);
+        });
+    };
+    auto x_loads = [&](int n, auto from, auto count, uint32_t stage) __attribute__((always_inline)) {
+        big_each<decltype(count)::value>([&](auto j) __attribute__((always_inline)) {
+            constexpr int q = decltype(from)::value + decltype(j)::value, gap = decltype(j)::value * GAPS / decltype(count)::value;
+            if (n == gap) place(stage, std::integral_constant<int, q>{});
+            if (n == gap + 1) fetch(ahead.x + ahead_at, x_off[q]);
+        });
     };
 
     // ---- the operands this lane reads: k-step i, chunk 4 i + g of its rows
@@ -116,66 +179,92 @@ __device__ __forceinline__ void big_walk(char* lds, const void* x, const void* w
             wc[f][i] = row * BIG_ROW + ((4 * i + g) ^ big_w_swizzle(row)) * 16;
         }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) xc[i] = (BIG_FEAT + wave_t * 16 * NT + r) * BIG_ROW + ((4 * i + g) ^ big_x_swizzle(r)) * 16;
-#pragma unroll
-    for (int f = 0; f < 8; ++f)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 wf[2][4], xf[2][NT];
-    auto read_tokens = [&](const char* stage) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int t = 0; t < NT; ++t) xf[i][t] = *reinterpret_cast<const bf16x8*>(stage + xc[i] + t * 16 * BIG_ROW);
+    for (int i = 0; i < 2; ++i) xc[i] = (A * BIG_FEAT + wave_t * 32 * NT + r) * BIG_ROW + ((4 * i + g) ^ big_x_swizzle(r)) * 16;
+    f32x4 acc[8][TT];
+    bf16x8 wf[2][2][4], xf[2][TT];                           // [half][k-step][tile], [k-step][tile]
+    auto read_w = [&](const char* stage, int i, int f) __attribute__((always_inline)) {
+        wf[f / 4][i][f % 4] = *reinterpret_cast<const bf16x8*>(stage + wc[f % 4][i] + f / 4 * 64 * BIG_ROW);
     };
-    auto read_features = [&](const char* stage, int half) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) wf[i][f] = *reinterpret_cast<const bf16x8*>(stage + wc[f][i] + half * 64 * BIG_ROW);
+    auto read_x = [&](const char* stage, int i, int t) __attribute__((always_inline)) {
+        xf[i][t] = *reinterpret_cast<const bf16x8*>(stage + xc[i] + t * 16 * BIG_ROW);
     };
-    auto multiply = [&](int half) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_setprio(1);
+    // a stage's reads, not before the first product (where the last quarter's are waited for) and not in the last few gaps
+    auto w_reads = [&](int n, const char* stage, int i) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int f = 0; f < 4; ++f)
-#pragma unroll
-                for (int t = 0; t < NT; ++t) acc[4 * half + f][t] = mfma_16x16x32(wf[i][f], xf[i][t], acc[4 * half + f][t]);
-        __builtin_amdgcn_s_setprio(0);
+        for (int f = 0; f < 8; ++f)
+            if (n == 1 + f * GAPS * 3 / 32) read_w(stage, i, f);
     };
+    auto x_reads = [&](int n, const char* stage, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+            if (n == 1 + t * GAPS * 7 / (8 * TT)) read_x(stage, i, t);
+    };
+    auto quarter = [&](int half, int i, auto between) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                between(4 * t + f);
+                big_multiply(acc[4 * half + f][t], wf[half][i][f], xf[i][t]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+#define BIG_C(v) std::integral_constant<int, (v)>{}
 
-    // ---- the walk over K.  In steps of the first four waves (the others are one step later): 4 kt reads P of stage kt and asks
-    // for Q of kt + 1 (whose place the others left at step 4 kt - 1), 4 kt + 1 multiplies, 4 kt + 2 reads Q of kt and asks for P
-    // of kt + 2 (left at 4 kt + 1), 4 kt + 3 multiplies.  P of kt is read from step 4 kt on, Q from 4 kt + 2: each wave has waited
-    // for its share, asked for six or four steps earlier with P + Q loads after it, before the barrier that ends the step before.
-    bring_p(0, 0);
-    bring_q(0, 0);
-    bring_p(1, 1);
-    all_but_the_youngest_have_arrived<P + Q>();
-    big_swap();
-    if (second) big_swap();
-    for (int kt = 0; kt < stages; ++kt) {
-        const int slot = kt & 1;
-        const char* stage = lds + slot * STAGE;
-        read_tokens(stage);
-        read_features(stage, 0);
-        bring_q(kt + 1, slot ^ 1);
-        if (second) all_but_the_youngest_have_arrived<P + Q>();
-        big_lds_reads_done();
-        big_swap();
-        multiply(0);
-        if (!second) all_but_the_youngest_have_arrived<P + Q>();
-        big_swap();
-        read_features(stage, 1);
-        bring_p(kt + 2, slot);
-        if (second) all_but_the_youngest_have_arrived<P + Q>();
-        big_lds_reads_done();
-        big_swap();
-        multiply(1);
-        if (!second) all_but_the_youngest_have_arrived<P + Q>();
-        big_swap();
+#pragma unroll
+    for (int s = 0; s < A; ++s) {
+        big_each<XL>([&](auto q) __attribute__((always_inline)) { place(lds_x + s * X_STAGE, q); asm volatile("s_nop 0"); fetch(ahead.x + ahead_at, x_off[q]); });
+        big_each<WL>([&](auto q) __attribute__((always_inline)) { place(lds_w + s * W_STAGE, q); asm volatile("s_nop 0"); fetch(ahead.w + ahead_at, w_off[q]); });
+        advance();
     }
-    if (!second) big_swap();
+    all_but_the_youngest_have_arrived<(A - 1) * (XL + WL)>();
+    big_swap();
+    uint32_t xs_before = A * X_STAGE, xs = 0, xs_next = X_STAGE, ws = 0, ws_next = W_STAGE;
+    for (int item = 0; item < items; ++item) {
+#pragma unroll
+        for (int f = 0; f < 8; ++f)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                asm volatile("" : "+a"(acc[f][t]));
+            }
+        asm volatile("s_nop 7" ::: "memory");                // (the products are written out: their distance to what writes or reads the sums is kept here)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) read_x(lds + xs, 0, t); // (read again behind another tile's end, which has better use for the registers)
+#pragma unroll
+        for (int f = 0; f < 8; ++f) read_w(lds + ws, 0, f);
+        const int stages = make(item).stages;
+        for (int kt = 0; kt < stages; ++kt) {
+            quarter(0, 0, [&](int n) __attribute__((always_inline)) {
+                w_reads(n, lds + ws, 1);
+                x_loads(n, BIG_C(0), BIG_C(XL / 2), lds_x + xs_before);
+            });
+            quarter(1, 0, [&](int n) __attribute__((always_inline)) {
+                x_reads(n, lds + xs, 1);
+                x_loads(n, BIG_C(XL / 2), BIG_C(XL - XL / 2), lds_x + xs_before);
+            });
+            all_but_the_youngest_have_arrived<(A - 1) * XL + (A - 2) * WL>();
+            big_lds_reads_done();
+            big_swap();
+            quarter(0, 1, [&](int n) __attribute__((always_inline)) {
+                x_reads(n, lds + xs_next, 0);
+                w_loads(n, BIG_C(0), BIG_C(WL / 2), lds_w + ws);
+            });
+            quarter(1, 1, [&](int n) __attribute__((always_inline)) {
+                w_reads(n, lds + ws_next, 0);
+                w_loads(n, BIG_C(WL / 2), BIG_C(WL / 2), lds_w + ws);
+            });
+            advance();
+            xs_before = xs; xs = xs_next; ws = ws_next;
+            xs_next = xs_next == A * X_STAGE ? 0 : xs_next + X_STAGE;
+            ws_next = ws_next == (A - 1) * W_STAGE ? 0 : ws_next + W_STAGE;
+        }
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        finish(item, acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#undef BIG_C
     all_but_the_youngest_have_arrived<0>();                  // nothing may land in LDS after the block's end
 }

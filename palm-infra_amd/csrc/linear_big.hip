@@ -2,18 +2,17 @@
 // result; or, with the gated epilogue (W = gate rows over up rows), C[M, N / 2] = silu(X G^T) * (X U^T).  The product is the
 // reference's matmul (kernels/matmul_dense.cpp:939-953), which its GPU path hands to a library (engine/cuda_matmul.cu:245-260).
 //
-// What bounds it is power: with the matrix cores three quarters busy the chip's clock falls (8,192 cubed: 1.37 million cycles
-// at 1.6 GHz), so what counts beside the products is what they cost to feed.  Tried on the way, 8,192 cubed: 32 x 32 x 16
-// instructions 850 us, 16 x 16 x 32 787 (half the accumulator traffic); operands in 64-byte pieces 800, in whole cache lines
-// (half the L2 requests) 750; the library 685 (its waves of 128 x 128 read a third less from LDS).
+// What bounds it is power (big_walk.h); 32 x 32 x 16 instructions cost more of it than 16 x 16 x 32 (twice the accumulator traffic),
+// operands in 64-byte pieces more than in whole cache lines (twice the L2 requests).  8,192 cubed 705 us (736 with eight waves a
+// block), the library 684; 13,331 x 24,576 x 4,096 gated 1,805 (1,959), the library and the activation's pass 1,952.
 //
-// A block owns a tile of 64 NT tokens x 256 features (big_walk.h).  Blocks are numbered so that the 32 blocks that run on one
+// A block owns tiles of 64 NT tokens x 256 features (big_walk.h), one after the other.  They are numbered so that the 32 blocks that run on one
 // die at a time (blocks go to the eight dies in turn) own neighbouring tiles, 4 tiles of tokens x 8 of features: a die's L2
 // reads a fifth of what the blocks ask for.
 //
 // The last round.  256 compute units take 256 tiles at a time; the tiles beyond the last full round are cut along K into
 // ranges where that fills the chip, whose float32 tiles a second kernel adds up in their order (4,309 x 4,096, K = 12,288:
-// 272 tiles, 316 us, 478 with whole tiles alone, the library 623).
+// 272 tiles, 305 us, the library 620).
 #include "big_walk.h"
 
 #include <hip/hip_runtime.h>
@@ -48,7 +47,7 @@ __device__ __forceinline__ void big_finish(const BigShape& s, bf16_t* __restrict
 #pragma unroll
         for (int f = 0; f < 4; ++f)
 #pragma unroll
-            for (int x = 0; x < 4; ++x) { const float gate = a[f][x]; v[4 * f + x] = gate / (1.0f + expf(-gate)) * a[4 + f][x]; }
+            for (int x = 0; x < 4; ++x) v[4 * f + x] = big_silu_gated(a[f][x], a[4 + f][x]);
         big_store(C + (size_t)token * s.inter, f0 * 128 + wave_f * 64 + 16 * g, s.inter, v);
     } else {
 #pragma unroll
@@ -63,75 +62,87 @@ __device__ __forceinline__ void big_finish(const BigShape& s, bf16_t* __restrict
     }
 }
 
+// Blocks: one for each compute unit.  A block takes every 32nd of its die's whole tiles, and one range of a cut tile if there is one left
+// for it.
 template <int NT, bool GATED>
-__global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void linear_big_kernel(
+__global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void linear_big_kernel(
     const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, bf16_t* __restrict__ C, const BigShape s, f32x4* __restrict__ partial) {
-    __shared__ __attribute__((aligned(1024))) char lds[2 * (BIG_FEAT + 64 * NT) * BIG_ROW];
-
-    // which tile, and which of its stages
-    int tile, stage0 = 0, stages = s.K / BIG_K;
-    const int block = blockIdx.x;
-    const bool owns = s.split == 1 || block < s.whole;      // a whole tile (without cut tiles the grid is rounded up to the dies)
-    if (owns) {
-        const int per_die = (s.whole + BIG_DIES - 1) / BIG_DIES;
-        tile = block % BIG_DIES * per_die + block / BIG_DIES;
-        if (tile >= s.whole) return;
-    } else {
-        const int j = block - s.whole, per = (stages + s.split - 1) / s.split;
-        tile = s.whole + j / s.split;
-        stage0 = j % s.split * per;
-        stages = min(per, stages - stage0);
-    }
-    const BigPlace place = BigPlace::of<NT>(s, tile);
-    const int t0 = place.t0, f0 = place.f0;
+    __shared__ __attribute__((aligned(1024))) char lds[big_lds_bytes(NT)];
+    const int block = blockIdx.x, stride = max(1, (int)gridDim.x / BIG_DIES), stages = s.K / BIG_K;
+    const int per_die = (s.whole + BIG_DIES - 1) / BIG_DIES, first = block % BIG_DIES * per_die + block / BIG_DIES;
+    const int last = min(s.whole, (block % BIG_DIES + 1) * per_die), mine = first < last ? (last - first + stride - 1) / stride : 0;
+    const bool cut = block < (s.tiles_t * s.tiles_f - s.whole) * s.split;
+    const int items = mine + cut;
+    if (items == 0) return;
+    auto tile_of = [&](int item) __attribute__((always_inline)) { return item < mine ? first + item * stride : s.whole + block / s.split; };
+    const uint32_t row_bytes = (uint32_t)(s.K * 2);
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int wave_f = wave % 2, wave_t = wave / 2, r = lane % 16, g = lane / 16;
-    f32x4 acc[8][NT];
-    big_walk<NT, false>(lds, X + (size_t)stage0 * BIG_K, W + (size_t)stage0 * BIG_K, (uint32_t)(s.K * 2), stages, 0,
-                        [&](int row) { return min(t0 + row, s.M - 1); },
-                        [&](int row) {
-                            return GATED ? (row & 64 ? s.inter : 0) + min(f0 * 128 + row / 128 * 64 + row % 64, s.inter - 1) : min(f0 * 256 + row, s.N - 1);
-                        },
-                        acc);
-
-    if (owns) {
+    big_walk<NT, false>(lds, row_bytes, items,
+        [&](int item) __attribute__((always_inline)) {
+            const BigPlace place = BigPlace::of<NT>(s, tile_of(item));
+            const int from = place.f0 * (GATED ? 128 : BIG_FEAT);
+            BigItem it{reinterpret_cast<const char*>(X + (size_t)place.t0 * s.K), reinterpret_cast<const char*>(W + (size_t)from * s.K), stages, 0,
+                       min(64 * NT, s.M - place.t0), min(GATED ? 128 : BIG_FEAT, (GATED ? s.inter : s.N) - from)};
+            if (item >= mine) {
+                const int per = (stages + s.split - 1) / s.split, stage0 = block % s.split * per;
+                it.x += (size_t)stage0 * BIG_ROW;
+                it.w += (size_t)stage0 * BIG_ROW;
+                it.stages = min(per, stages - stage0);
+            }
+            return it;
+        },
+        [&](const BigItem& it, int row) __attribute__((always_inline)) { return min(row, it.x_rows - 1); },
+        [&](const BigItem& it, int row) __attribute__((always_inline)) {
+            return GATED ? (row & 64 ? s.inter : 0) + min(row / 128 * 64 + row % 64, it.w_rows - 1) : min(row, it.w_rows - 1);
+        },
+        [&](int item, f32x4 (&acc)[8][2 * NT]) __attribute__((always_inline)) {
+            f32x4 a[8];
+            if (item < mine) {
+                const BigPlace place = BigPlace::of<NT>(s, tile_of(item));
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const f32x4 a[8] = {acc[0][t], acc[1][t], acc[2][t], acc[3][t], acc[4][t], acc[5][t], acc[6][t], acc[7][t]};
-            big_finish<GATED>(s, C, f0, t0 + wave_t * 16 * NT + t * 16 + r, wave_f, g, a);
-        }
-    } else {                                                 // the sums as they lie in the lanes: [block][t][f][thread]
-        f32x4* out = partial + (size_t)(block - s.whole) * NT * 8 * BIG_THREADS + threadIdx.x;
+                for (int t = 0; t < 2 * NT; ++t) {
+                    big_column(acc, t, a);
+                    big_finish<GATED>(s, C, place.f0, place.t0 + wave_t * 32 * NT + t * 16 + r, wave_f, g, a);
+                }
+            } else {                                         // the sums as they lie in the lanes: [block][t][f][thread]
+                uint32_t at = block * 2 * NT * 8 * BIG_THREADS + threadIdx.x;
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+                for (int t = 0; t < 2 * NT; ++t) {
+                    asm volatile("" : "+v"(at));             // (or the addresses of all of them are kept over the walk)
+                    big_column(acc, t, a);
 #pragma unroll
-            for (int f = 0; f < 8; ++f) out[(t * 8 + f) * BIG_THREADS] = acc[f][t];
-    }
+                    for (int f = 0; f < 8; ++f) partial[at + (t * 8 + f) * BIG_THREADS] = a[f];
+                }
+            }
+        });
 }
 
 // A block for each (tile that was cut, token tile of its waves): the ranges' sums in their order, then as above.
 template <int NT, bool GATED>
 __global__ __launch_bounds__(BIG_THREADS) void linear_big_sum_kernel(bf16_t* __restrict__ C, const BigShape s, const f32x4* __restrict__ partial) {
-    const int j = blockIdx.x / NT, t = blockIdx.x % NT;
+    const int j = blockIdx.x / (2 * NT), t = blockIdx.x % (2 * NT);
     const BigPlace place = BigPlace::of<NT>(s, s.whole + j);
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     f32x4 a[8];
 #pragma unroll
     for (int f = 0; f < 8; ++f) a[f] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int p = 0; p < s.split; ++p) {
-        const f32x4* from = partial + ((size_t)(j * s.split + p) * NT + t) * 8 * BIG_THREADS + threadIdx.x;
+        const f32x4* from = partial + ((size_t)(j * s.split + p) * 2 * NT + t) * 8 * BIG_THREADS + threadIdx.x;
 #pragma unroll
         for (int f = 0; f < 8; ++f) a[f] += from[f * BIG_THREADS];
     }
-    big_finish<GATED>(s, C, place.f0, place.t0 + wave / 2 * 16 * NT + t * 16 + lane % 16, wave % 2, lane / 16, a);
+    big_finish<GATED>(s, C, place.f0, place.t0 + wave / 2 * 32 * NT + t * 16 + lane % 16, wave % 2, lane / 16, a);
 }
 
 // ---- launch -----------------------------------------------------------------------------------------
 struct BigPlan { int nt; BigShape shape; double cost; };
 
 // Tiles of 256, 192 or 128 tokens, and into how many ranges of K the tiles beyond the last full round are cut: what takes least by
-// this count of microseconds.  With the chip full a stage of a tile of 256 tokens takes 1.42 us, of 192 1.13, of 128 0.87; a
-// block's start and end 3; a sum kernel 6, and the float32 tiles cross memory twice, at 4 TB/s.
+// this count of microseconds.  With the chip full a stage of a tile of 256 tokens takes 1.37 us (64 stages 95 us, 256 stages 362, a
+// second tile of 64 stages 89), of 192 1.11, of 128 0.83 and, in some sizes, 1.0; the beginning and end of a tile that are not hidden 2.6;
+// a sum kernel 6, and the float32 tiles cross memory twice, at 4.1 TB/s.  (At 360 products of 330 to 13,331 rows the tiles so chosen are
+// 1.1 % behind the best of the three in the mean.)
 static BigPlan big_plan(int M, int N, int K, bool gated) {
     BigPlan best{};
     best.cost = 1e300;
@@ -144,13 +155,13 @@ static BigPlan big_plan(int M, int N, int K, bool gated) {
         const long long tiles = (long long)s.tiles_t * s.tiles_f;
         if (tiles > 1 << 24) continue;
         const int rounds = (int)(tiles / BIG_UNITS), rest = (int)(tiles % BIG_UNITS);
-        const double stage_us = nt == 4 ? 1.42 : nt == 3 ? 1.13 : 0.87;
+        const double stage_us = nt == 4 ? 1.37 : nt == 3 ? 1.11 : 0.97;
         for (int split = 1; split <= 8; ++split) {
             if (split > 1 && (rest == 0 || rest * split > BIG_UNITS || stages / split < 8)) break;
             if (split > 1 && (split - 1) * ((stages + split - 1) / split) >= stages) continue;      // a range without stages
-            const double last = rest == 0 ? 0.0 : (double)((stages + split - 1) / split) * stage_us + 3.0;
-            const double sums = split == 1 ? 0.0 : 6.0 + (double)rest * split * nt * 8 * BIG_THREADS * 16 * 2 / 4e6;
-            const double cost = rounds * (stages * stage_us + 3.0) + last + sums;
+            const double last = rest == 0 ? 0.0 : (double)((stages + split - 1) / split) * stage_us + 2.6;
+            const double sums = split == 1 ? 0.0 : 6.0 + (double)rest * split * nt * 16 * BIG_THREADS * 16 * 2 / 4.1e6;
+            const double cost = rounds * (stages * stage_us + 2.6) + last + sums;
             if (cost < best.cost) {
                 s.split = split;
                 s.whole = split == 1 ? (int)tiles : rounds * BIG_UNITS;
@@ -178,18 +189,18 @@ PALM_API long long palm_linear_big_work(int M, int N, int K, int gated) {
     if (!big_takes(M, N, K, gated != 0)) return 0;
     const BigPlan p = big_plan(M, N, K, gated != 0);
     const long long tiles = (long long)p.shape.tiles_t * p.shape.tiles_f;
-    return p.shape.split == 1 ? 0 : (tiles - p.shape.whole) * p.shape.split * p.nt * 8 * BIG_THREADS * 16;
+    return p.shape.split == 1 ? 0 : (tiles - p.shape.whole) * p.shape.split * p.nt * 16 * BIG_THREADS * 16;
 }
 
 template <int NT, bool GATED>
 static int launch_big(hipStream_t stream, const void* x, const void* w, void* c, const BigShape& s, void* work) {
     const int tiles = s.tiles_t * s.tiles_f, cut = tiles - s.whole;
-    const int blocks = cut ? s.whole + cut * s.split : (s.whole + BIG_DIES - 1) / BIG_DIES * BIG_DIES;
+    const int blocks = min(BIG_UNITS, max((s.whole + BIG_DIES - 1) / BIG_DIES * BIG_DIES, cut * s.split));
     BigShape shape = s;
     linear_big_kernel<NT, GATED><<<blocks, BIG_THREADS, 0, stream>>>((const bf16_t*)x, (const bf16_t*)w, (bf16_t*)c, shape, (f32x4*)work);
     PALM_LAUNCHED();
     if (cut) {
-        linear_big_sum_kernel<NT, GATED><<<cut * NT, BIG_THREADS, 0, stream>>>((bf16_t*)c, shape, (const f32x4*)work);
+        linear_big_sum_kernel<NT, GATED><<<cut * 2 * NT, BIG_THREADS, 0, stream>>>((bf16_t*)c, shape, (const f32x4*)work);
         PALM_LAUNCHED();
     }
     return 0;

@@ -180,48 +180,55 @@ __global__ __launch_bounds__(GT_WAVES * WAVE) void moe_grouped_kernel(const bf16
 // Us with plan and sum, squared relu, rows of four choices over 32 experts: 130 rows 484 -> 211 (fragments from memory before),
 // 352: 347 -> 212, 852: 372 -> 262, 2,048: 590 -> 440 (a ring of three stages of 32 x 32 x 16 instructions before).
 template <int NT, int FORM, typename TO>
-__global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_big_kernel(
+__global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void moe_big_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ slot_pair, int top, const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
     const int* __restrict__ used, int feature_tiles, int n_features, int k_dim, ExpertCap cap, TO* __restrict__ out) {
     constexpr bool GATED = FORM == 1 || FORM == 3;
-    __shared__ __attribute__((aligned(1024))) char lds[2 * (BIG_FEAT + 64 * NT) * BIG_ROW];
-    const int total = *used * feature_tiles, per_die = (total + BIG_DIES - 1) / BIG_DIES;
-    const int pid = (blockIdx.x % BIG_DIES) * per_die + blockIdx.x / BIG_DIES;
-    if ((int)blockIdx.x / BIG_DIES >= per_die || pid >= total) return;
-    const int tile = pid / feature_tiles, ft = pid % feature_tiles;
-    const int e = __builtin_amdgcn_readfirstlane(tile_expert[tile]);
-    const int stages = k_dim / BIG_K;
-    f32x4 acc[8][NT];
-    big_walk<NT, true>(lds, a, w + (size_t)e * (GATED ? 2 : 1) * n_features * k_dim, (uint32_t)(k_dim * 2), stages, (5 * e + 2 * ft) % stages,
-                       [&](int row) {
-                           const int slot = tile * 64 * NT + row;
-                           return FORM == 0 ? slot : max(slot_pair[slot], 0) / top;      // a slot that pads the run reads row 0; nobody reads its result
-                       },
-                       [&](int row) {
-                           return GATED ? (row & 64 ? n_features : 0) + min(ft * 128 + row / 128 * 64 + row % 64, n_features - 1)
-                                        : min(ft * 256 + row, n_features - 1);
-                       },
-                       acc);
+    __shared__ __attribute__((aligned(1024))) char lds[big_lds_bytes(NT)];
+    const int total = *used * feature_tiles, per_die = (total + BIG_DIES - 1) / BIG_DIES, stages = k_dim / BIG_K;
+    const int first = (blockIdx.x % BIG_DIES) * per_die + blockIdx.x / BIG_DIES, stride = gridDim.x / BIG_DIES;
+    const int last = min(total, (int)(blockIdx.x % BIG_DIES + 1) * per_die), items = first < last ? (last - first + stride - 1) / stride : 0;
+    if (items == 0) return;
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, wave_f = wave % 2, wave_t = wave / 2;
+    big_walk<NT, true>(lds, (uint32_t)(k_dim * 2), items,
+        [&](int item) __attribute__((always_inline)) {
+            const int pid = first + item * stride, tile = pid / feature_tiles, ft = pid % feature_tiles;
+            const int e = __builtin_amdgcn_readfirstlane(tile_expert[tile]), from = ft * (GATED ? 128 : BIG_FEAT);
+            // (x_rows names the tile of slots: the rows of another are others)
+            return BigItem{reinterpret_cast<const char*>(a), reinterpret_cast<const char*>(w + ((size_t)e * (GATED ? 2 : 1) * n_features + from) * k_dim), stages,
+                           (5 * e + 2 * ft) % stages, tile, min(GATED ? 128 : BIG_FEAT, n_features - from)};
+        },
+        [&](const BigItem& it, int row) __attribute__((always_inline)) {
+            const int slot = it.x_rows * 64 * NT + row;
+            return FORM == 0 ? slot : max(slot_pair[slot], 0) / top;      // a slot that pads the run reads row 0; nobody reads its result
+        },
+        [&](const BigItem& it, int row) __attribute__((always_inline)) {
+            return GATED ? (row & 64 ? n_features : 0) + min(row / 128 * 64 + row % 64, it.w_rows - 1) : min(row, it.w_rows - 1);
+        },
+        [&](int item, f32x4 (&acc)[8][2 * NT]) __attribute__((always_inline)) {
+            const int pid = first + item * stride, tile = pid / feature_tiles, ft = pid % feature_tiles;
+            f32x4 z[8];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int slot = tile * 64 * NT + wave_t * 16 * NT + 16 * t + lane % 16;
-        if (sizeof(TO) == 4 && slot_pair[slot] < 0) continue;          // (few rows: most of a tile pads its run)
-        TO* row = out + (size_t)slot * n_features;
+            for (int t = 0; t < 2 * NT; ++t) {
+                big_column(acc, t, z);
+                const int slot = tile * 64 * NT + wave_t * 32 * NT + 16 * t + lane % 16;
+                if (sizeof(TO) == 4 && slot_pair[slot] < 0) continue;          // (few rows: most of a tile pads its run)
+                TO* row = out + (size_t)slot * n_features;
 #pragma unroll
-        for (int half = 0; half < (GATED ? 1 : 2); ++half) {
-            float v[16];
+                for (int half = 0; half < (GATED ? 1 : 2); ++half) {
+                    float v[16];
 #pragma unroll
-            for (int f = 0; f < 4; ++f)
+                    for (int f = 0; f < 4; ++f)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float z = acc[4 * half + f][t][i];
-                    v[4 * f + i] = FORM == 1 ? expert_silu_gated(z, acc[4 + f][t][i]) : FORM == 3 ? expert_capped(z, acc[4 + f][t][i], cap)
-                                   : FORM == 2 ? expert_gelu(z) : FORM == 4 ? expert_relu_squared(z) : z;
+                        for (int i = 0; i < 4; ++i) {
+                            const float x = z[4 * half + f][i];
+                            v[4 * f + i] = FORM == 1 ? big_silu_gated(x, z[4 + f][i]) : FORM == 3 ? expert_capped(x, z[4 + f][i], cap)
+                                           : FORM == 2 ? expert_gelu(x) : FORM == 4 ? expert_relu_squared(x) : x;
+                        }
+                    big_store(row, (GATED ? ft * 128 + wave_f * 64 : ft * 256 + wave_f * 128 + half * 64) + 16 * (lane / 16), n_features, v);
                 }
-            big_store(row, (GATED ? ft * 128 + wave_f * 64 : ft * 256 + wave_f * 128 + half * 64) + 16 * (lane / 16), n_features, v);
-        }
-    }
+            }
+        });
 }
 
 __device__ inline void combine_load8(const bf16_t* p, float (&v)[8]) {
@@ -340,7 +347,7 @@ PALM_API int palm_moe_grouped(hipStream_t stream, const void* h, const void* gat
         (const bf16_t*)add0, (const bf16_t*)add1, planes, n_planes, out)
     const ExpertCap cap{limit, slope, shift};
     if (big) {
-        auto blocks = [&](int feature_tiles) { return dim3((max_tiles * feature_tiles + BIG_DIES - 1) / BIG_DIES * BIG_DIES); };
+        auto blocks = [&](int feature_tiles) { return dim3(min(256, (max_tiles * feature_tiles + BIG_DIES - 1) / BIG_DIES * BIG_DIES)); };
         const int up_features = expert_is_gated(form) ? BIG_FEAT / 2 : BIG_FEAT;
         const int up_tiles = (ff + up_features - 1) / up_features, down_tiles = (width + BIG_FEAT - 1) / BIG_FEAT;
         PALM_CHECK((long long)max_tiles * max(up_tiles, down_tiles) < (1ll << 30), "moe_grouped: %d tiles of rows are more than one launch takes", max_tiles);

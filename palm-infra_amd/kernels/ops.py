@@ -509,33 +509,37 @@ def linear_mid(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: 
 
 BIG_FROM = 320              # rows from which the kernel of large tiles may serve a product
 BIG_GATED_FROM = 500
-BIG_LONG_K, BIG_LONGEST_K = 8192, 16384
+BIG_SHORT_K, BIG_LONG_K, BIG_LONGEST_K = 8192, 12288, 16384
 BIG_ROUNDS = 8
 
 
 def big_pays(M: int, N: int, K: int, gated: bool = False) -> bool:
     """Whether a prompt's product of bfloat16 operands goes through the kernel of large tiles (linear_big.hip) instead of the
-    library.  Measured at 24 shapes of 2,048 to 51,200 weight rows, K from 2,048 to 28,672, each with 25 to 32 numbers of rows from 257
-    to 13,331 (own time over the library's; where tiles fill whole rounds of the compute units the library is the faster one by 2 to
-    12 %, elsewhere it often takes a poor tile).
+    library.  Measured at 834 products: 2,048 to 34,816 weight rows, K from 2,048 to 17,408, 320 to 13,331 rows (own time over the
+    library's; where tiles of 256 x 256 fill whole rounds of the compute units the library is the faster one by some 4 %, elsewhere it
+    often takes a poor tile).
 
-    gated (the activation in the kernel, against the library and the activation's pass): from 500 rows on, 0.92 in the geometric mean,
-    1.05 at worst.
+    gated (the activation in the kernel, against the library and the activation's pass): from 500 rows on, 0.84 in the geometric mean,
+    0.96 at worst.
     other products, by the rounds that tiles of 256 x 256 make on 256 compute units:
-      one to eight full rounds and up to 0.3 of another (inner sizes from 8,192 on: 0.68), whose tiles are cut along K here: 4,309 x
-      4,096, K = 12,288 (1.06 rounds) 0.49, 7,000 x 7,168, K = 5,120 (3.06) 0.79; 0.89 in the mean, 1.18 at worst
-      0.55 to 0.72 of a round with an inner size from 8,192 on: a third of the chip is idle there, the tiles are smaller or cut here
-      (2,603 x 4,096, K = 16,384: 0.51); 0.97 in the mean, 1.07 at worst
-      inner sizes beyond 16,384 whatever the rounds: 0.47 to 1.21, 0.76 in the mean
-    0.84 in the mean where this says yes (243 of 766 products); 45 lose more than 2 % to the library."""
+      up to one: from 0.55 to 0.85 with an inner size from 8,192 on, from 0.2 with one from 12,288 on (K is cut there); 0.93
+      up to eight: not where the rounds are whole (1.04), and with inner sizes under 8,192 not from 1.5 to 2, 2.3 to 2.6 and 3.3 to 4 (1.03);
+      elsewhere 0.86 (2,603 x 16,384, K = 4,096: 2.75 rounds, 0.70; 13,331 x 6,144: 4.97, 0.77; 2.6 to 2.8 rounds 0.67 to 1.10)
+      beyond: in the upper half of a round (0.90; the lower 1.02)
+      inner sizes beyond 16,384 whatever the rounds
+    0.83 in the mean where this says yes (312 of 786); 32 lose more than 2 % to the library."""
     if M < (BIG_GATED_FROM if gated else BIG_FROM) or not core().palm_linear_big_takes(M, N, K, int(gated)):
         return False
-    rounds = -(-M // 256) * -(-N // 256) / COMPUTE_UNITS
     if gated or K > BIG_LONGEST_K:
         return True
-    if rounds <= 1:
-        return K >= BIG_LONG_K and 0.55 < rounds <= 0.72
-    return rounds <= BIG_ROUNDS and 0 < rounds % 1 <= (0.68 if K >= BIG_LONG_K else 0.3)
+    rounds = -(-M // 256) * -(-N // 256) / COMPUTE_UNITS
+    if rounds < 1:
+        return (K >= BIG_SHORT_K and 0.55 < rounds <= 0.85) or (K >= BIG_LONG_K and 0.2 < rounds <= 0.55)
+    if K >= BIG_SHORT_K:
+        return rounds % 1 > 0
+    if rounds > BIG_ROUNDS:
+        return rounds % 1 >= 0.5
+    return rounds % 1 > 0 and not (1.5 <= rounds < 2 or 2.3 <= rounds < 2.6 or 3.3 <= rounds < 4)
 
 
 def linear_big(a: torch.Tensor, w: torch.Tensor, gated: bool = False) -> torch.Tensor:

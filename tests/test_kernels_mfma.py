@@ -1,6 +1,8 @@
 """The matrix-core kernels alone against their plain references: the thin linear product (with and
 without the gated epilogue) and the bfloat16 attention kernels, at sizes other than the tiny models'."""
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -355,6 +357,29 @@ def test_which_products_of_prompts_take_large_tiles(ops):
     # less than a round: long inner sizes that leave a third of the chip idle; the longest whatever the rounds
     assert pays(2603, 4096, 16384) and not pays(2603, 4096, 4096) and not pays(600, 4096, 16384) and not pays(320, 4096, 12288)
     assert pays(320, 5120, 17408) and not pays(319, 5120, 17408)
+    # the rounds between: short inner sizes where the library's tiles are poor, long ones wherever they are not whole
+    assert pays(2603, 16384, 4096) and pays(13331, 6144, 4096) and pays(5000, 4096, 4096) and not pays(6400, 4096, 4096)
+    assert pays(1700, 4096, 12288) and not pays(1700, 4096, 8192) and pays(13000, 16384, 4096) == (51 * 64 / 256 % 1 >= 0.5)
+
+
+@pytest.mark.parametrize("gate", [0.0, -0.0, 30.0, -30.0, 87.5, -87.5, 88.8, -88.8, 200.0, -200.0, 3e38, -3e38, float("inf"), float("-inf"), float("nan")])
+def test_gated_products_in_large_tiles_at_the_activations_limits(ops, gate):
+    """silu at gates that saturate it, at the ends of 2^x's range, infinite and not a number: as the activation's own pass gives it
+    (what is smaller than bfloat16's least normal number aside, 1.2e-38 times the up value)."""
+    M, N, K = 600, 512, 128
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
+    x[:, 0] = 1.0
+    w[:N // 2, 0] = gate
+    w[N // 2:, 0] = torch.linspace(-3.0, 3.0, N // 2).to(torch.bfloat16)
+    if not math.isfinite(gate):                                # (zeros elsewhere would make it NaN in every sum)
+        x[:, 1:], w[:, 1:] = 0.0, 0.0
+    g, u = x[:, :1].float() * w[:N // 2, 0].float(), x[:, :1].float() * w[N // 2:, 0].float()
+    want = ops.swiglu(torch.cat([g, u], dim=1).to(torch.bfloat16))
+    got = ops.linear_big(x, w, gated=True)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    ok = ~torch.isnan(want)
+    assert torch.allclose(got[ok].float(), want[ok].float(), rtol=2.0 ** -7, atol=1e-36)
 
 
 @pytest.mark.parametrize("M", [70, 256, 300])
