@@ -509,6 +509,33 @@ def test_attention_exact_takes_nothing_from_what_lies_beyond_a_sequence(ops, dty
     assert torch.isfinite(got).all() and torch.allclose(got, ref, atol=1e-5 if dtype == F32 else 2e-2)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (4, 2, 64), (6, 2, 72), (10, 2, 40), (5, 1, 128), (3, 3, 96), (4, 1, 30), (4, 2, 200)])
+def test_attention_exact_is_the_same_bits_whatever_the_heads_that_share_a_block(ops, dtype, nh, nkv, hd):
+    """Launches of many queries share a page among the heads of a group, launches of few do not: a query's result is the same bits in
+    both, with a window too, and with keys beyond it that are no numbers."""
+    for window, lens in ((None, [1040 // nh + 3, 1, 65, 130]), (50, [1040 // nh + 3, 64, 100])):
+        mp = max((n + 63) // 64 for n in lens)
+        g = torch.Generator().manual_seed(nh + hd)
+        kc, vc = (torch.full(shape, float("nan")).to(dtype) for shape in ((len(lens) * mp, nkv, 64, hd), (len(lens) * mp, nkv, hd, 64)))
+        table = torch.arange(len(lens) * mp, dtype=torch.int32).view(len(lens), mp)
+        for b, n in enumerate(lens):
+            _fill_cache(kc, vc, table, b, torch.randn(n, nkv, hd, generator=g), torch.randn(n, nkv, hd, generator=g))
+        q = torch.randn(sum(lens), nh * hd, generator=g).to(dtype).to(DEV)
+        kc, vc, table = kc.to(DEV), vc.to(DEV), table.to(DEV)
+        i32 = lambda xs: torch.tensor(xs, dtype=torch.int32, device=DEV)
+        cu = [sum(lens[:b]) for b in range(len(lens) + 1)]
+        assert max(lens) * nh * len(lens) >= 1024
+        got = ops.attention_exact(q, kc, vc, table, i32(list(range(len(lens)))), i32([0] * len(lens)), i32(lens), i32(cu), max(lens), nh, nkv, hd, hd ** -0.5, window)
+        assert torch.isfinite(got).all()
+        for b, n in enumerate(lens):
+            few = 1000 // nh
+            for at in range(0, n, few):
+                new = min(few, n - at)
+                part = ops.attention_exact(q[cu[b] + at:cu[b] + at + new].contiguous(), kc, vc, table, i32([b]), i32([at]), i32([new]), i32([0, new]), new, nh, nkv, hd, hd ** -0.5, window)
+                assert torch.equal(part, got[cu[b] + at:cu[b] + at + new]), (window, b, at)
+
+
 def test_attention_exact_over_thousands_of_keys(ops):
     """The float32 path's attention keeps its 1e-5 where a query sees thousands of keys (a prompt's continuation
     far into a sequence, single queries)."""
