@@ -106,7 +106,7 @@ __device__ inline void mr_plan(RingPlan& plan, const RingChoices& ch, const Ring
 }
 
 // What a lane asks for in an instruction: 16 bytes of row (lane / 8) of eight, piece (lane % 8) ^ (lane / 8) of a line's eight; and
-// where it finds its fragment of 32 values j: row r, pieces 4 (j % 2) + g of half j / 2 (linear_ring.hip).
+// where it finds its fragment of 32 values j: row r, pieces 4 (j % 2) + g of half j / 2 (linear_ring.h).
 __device__ __forceinline__ uint32_t mr_fragment(int j, int r, int g) {
     return ((r / 8) + 2 * (j / 2)) * 1024 + (r % 8) * 128 + ((((j % 2) * 4 + g) ^ (r % 8)) * 16);
 }

@@ -7,6 +7,7 @@ are memory here; the one computation that torch does on the product path is the 
 """
 from __future__ import annotations
 
+import functools
 from array import array
 from ctypes import c_float, c_int, c_longlong, c_ulonglong, c_void_p
 from dataclasses import dataclass
@@ -38,6 +39,9 @@ _SIGNATURES = {
                               c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
     "palm_linear_thin": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p],
+    "palm_linear_ring": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                         c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p],
+    "palm_linear_ring_parts": [c_int, c_int, c_int, c_int, c_int],
     "palm_scale_rows": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_int, c_void_p],
     "palm_linear_thin_parts": [c_int, c_int, c_int],
     "palm_linear_wide": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int],
@@ -422,7 +426,8 @@ COMPUTE_UNITS = 256     # of an MI355X; a folded product's blocks come in rounds
 
 
 def fold_pays(M: int, N: int, K: int) -> bool:
-    """Whether a product of M <= 16 rows that is a branch's output should fold the residual add and the next norm
+    """Whether a product of M <= 16 rows (or up to 48 that ``ring_serves`` takes whole: 4,096 x 4,096 10.2 to 13.0 us, 9.7 to 10.3 and
+    the norm's 5.2 apart) that is a branch's output should fold the residual add and the next norm
     in, or rather be cut along K into planes that the norm's own kernel adds up.  A fold needs all of K in one
     block.  Up to K = 8192 the block keeps the activations in registers and the fold won at every width measured
     (N 1024 to 5120: 8 to 28 us against 8 to 36).  Beyond that it reads them beside the weights and wins only
@@ -562,7 +567,54 @@ def thin_serves(a: torch.Tensor, w: torch.Tensor) -> bool:
     return a.dtype == BF16 and w.dtype == BF16 and a.shape[1] % 8 == 0
 
 
-def _row_ss(what: str, a: torch.Tensor, row_ss) -> int:
+RING_STEP_K = 1024    # of one super-step of all waves
+RING_TOKENS = 48      # rows that the stream of whole lines takes with its activations in registers (above THIN_TOKENS)
+
+
+@functools.lru_cache(maxsize=4096)
+def ring_parts(M: int, N: int, K: int, gated: bool, planes_ok: bool) -> int:
+    """The library's plan for a product of 17 to 48 rows, 0 where it does not take it (a launch asks several times: remembered by the
+    sizes, which are all it depends on)."""
+    return core().palm_linear_ring_parts(M, N, K, int(gated), int(planes_ok))
+
+
+def ring_serves(M: int, N: int, K: int, gated: bool = False, planes_ok: bool = False) -> bool:
+    """Whether the stream of whole lines (linear_ring.hip) takes this product of 17 to 48 rows."""
+    return THIN_TOKENS < M <= RING_TOKENS and ring_parts(M, N, K, gated, planes_ok) > 0
+
+
+def ring_pays(M: int, N: int, K: int, gated: bool = False, planes_ok: bool = False) -> bool:
+    """Whether it is also the faster way, against the kernel with both operands in LDS (linear_mid.hip; us, 17, 32 and 48 rows):
+    gate/up of 24,576 x 4,096 gated 40.6 38.9 39.2 and 37.0 37.3 39.0, of 34,816 x 5,120 (up to 32 rows) 85 88 and 65 67, q/k/v of 6,144 x 4,096 15.1 15.5 16.2
+    and 11.9 12.2 13.3, down of 4,096 x 12,288 22.3 23.5 24.0 and 21.2 22.1 21.7, the head 230 231 237 and 219 228 237.  Not where one round of
+    whole strips is all there is (4,096 x 4,096: 9.9 9.5 10.3 and 9.7 10.6 11.9): there every block reads all rows for one strip."""
+    if K < 2 * RING_STEP_K or not ring_serves(M, N, K, gated, planes_ok):       # (K of one step: not measured)
+        return False
+    return gated or ring_parts(M, N, K, False, planes_ok) > 1 or (N + 15) // 16 > 1.25 * COMPUTE_UNITS
+
+
+def linear_ring(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: bool = False, planes_ok: bool = False, row_ss=None,
+                row_eps: float = 0.0) -> torch.Tensor:
+    """``linear_thin`` (its arguments) for 17 to 48 rows where ``ring_serves`` says so: the weight streamed once for all rows."""
+    _dev("linear_ring", a, w)
+    if not (a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1] and thin_serves(a, w) and a.is_contiguous() and w.is_contiguous()):
+        raise KernelError(f"linear_ring: a {tuple(a.shape)} {a.dtype} and w {tuple(w.shape)} {w.dtype} (bfloat16, one inner size)")
+    M, K = a.shape
+    N = w.shape[0]
+    if not ring_serves(M, N, K, gated, planes_ok):
+        raise KernelError(f"linear_ring: {M} rows of {K} times {N} weight rows are not served")
+    pieces = _row_ss("linear_ring", a, row_ss, RING_TOKENS)
+    planes = ring_parts(M, N, K, gated, planes_ok)
+    if planes > 1:
+        out = torch.empty((planes, M, N), dtype=F32, device=a.device)
+    else:
+        out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=a.device)
+    library.call(core(), "palm_linear_ring", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_ring out"), M, N, K, int(gated), planes,
+                 _p(row_ss), pieces, float(row_eps), None, None, None)
+    return out
+
+
+def _row_ss(what: str, a: torch.Tensor, row_ss, rows: int = THIN_TOKENS) -> int:
     """Checks the pieces of the rows' sums of squares that come with rows lacking their norm's factor."""
     if row_ss is None:
         return 0
@@ -570,8 +622,8 @@ def _row_ss(what: str, a: torch.Tensor, row_ss) -> int:
     if not (row_ss.dim() == 2 and row_ss.shape[0] == a.shape[0] and row_ss.dtype == F32 and row_ss.is_contiguous()
             and row_ss.shape[1] > 0):
         raise KernelError(f"{what}: sums of squares {tuple(row_ss.shape)} {row_ss.dtype} for {a.shape[0]} rows")
-    if not (a.shape[0] <= THIN_TOKENS and thin_serves(a, a)):
-        raise KernelError(f"{what}: a norm is folded into products of at most {THIN_TOKENS} bfloat16 rows")
+    if not (a.shape[0] <= rows and thin_serves(a, a)):
+        raise KernelError(f"{what}: a norm is folded into products of at most {rows} bfloat16 rows")
     return row_ss.shape[1]
 
 
@@ -589,22 +641,23 @@ def scale_rows(a: torch.Tensor, row_ss: torch.Tensor, eps: float) -> torch.Tenso
 
 def linear_thin_into_residual(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor, row_ss=None,
                               row_eps: float = 0.0):
-    """A branch's last product and what follows it, for up to 16 rows: x += a . w^T (x float32 [M, N], in
+    """A branch's last product and what follows it, for up to 16 rows, or as many as ``ring_serves`` takes whole: x += a . w^T (x float32 [M, N], in
     place); returns (x * norm_w rounded to bfloat16, the pieces [M, N/16] of each row's sum of squares of x):
     the next norm's output but for the row factor.  row_ss / row_eps: a itself lacks a row factor."""
     _dev("linear_thin_into_residual", a, w, x, norm_w)
     M, K = a.shape
     N = w.shape[0]
-    if not (thin_serves(a, w) and M <= THIN_TOKENS and w.shape[1] == K):
+    many = M > THIN_TOKENS
+    if not (thin_serves(a, w) and w.shape[1] == K and (not many or (ring_serves(M, N, K) and a.is_contiguous() and w.is_contiguous()))):
         raise KernelError(f"linear_thin_into_residual: a {tuple(a.shape)} {a.dtype}, "
                           f"w {tuple(w.shape)} {w.dtype} (bfloat16, at most {THIN_TOKENS} rows, K a multiple of 8)")
     if not (x.shape == (M, N) and x.dtype == F32 and x.is_contiguous()):
         raise KernelError(f"linear_thin_into_residual: residual {tuple(x.shape)} {x.dtype}")
     _need(norm_w.shape == (N,) and norm_w.dtype == F32, "linear_thin_into_residual: the norm's weight is float32 [N]")
-    pieces = _row_ss("linear_thin_into_residual", a, row_ss)
+    pieces = _row_ss("linear_thin_into_residual", a, row_ss, RING_TOKENS if many else THIN_TOKENS)
     values = torch.empty((M, N), dtype=BF16, device=a.device)
     ss = torch.empty((M, (N + 15) // 16), dtype=F32, device=a.device)
-    library.call(core(), "palm_linear_thin", _stream(), _p(a), _p(w), _p(values), _code(values, "values"), M, N, K, 0, 1,
+    library.call(core(), "palm_linear_ring" if many else "palm_linear_thin", _stream(), _p(a), _p(w), _p(values), _code(values, "values"), M, N, K, 0, 1,
                  _p(row_ss), pieces, float(row_eps), _p(x), _p(norm_w), _p(ss))
     return values, ss
 

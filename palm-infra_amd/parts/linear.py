@@ -3,6 +3,9 @@
   float32 run, or a 32-bit weight under bfloat16 activations   the exact FMA kernel
   bfloat16 x bfloat16, an inner size that is no multiple of 8    the exact FMA kernel (rows do not start on 16 bytes)
   bfloat16 x bfloat16, up to 16 rows (decode)                   the matrix-core kernel for thin products
+  bfloat16 x bfloat16, 17 to 48 rows                             the stream of whole lines with two or three tiles of rows
+                                                                (ops.ring_pays: inner sizes in steps of 1,024 up to 6,144 or
+                                                                4,096 a range), else as follows
   bfloat16 x bfloat16, 17 to 256 rows (decode batches, short    the kernel that brings both operands through rings in
   prompts)                                                      LDS, where it beats the others (ops.mid_pays); where
                                                                 it does not serve (K no multiple of 64, few weight
@@ -24,8 +27,8 @@ import torch
 from ..kernels import ops
 from .residual import Prenormed
 
-# Up to this many rows the kernel that streams the weight past one block of 16 rows serves; from 17 to 256 rows the
-# kernel with rings in LDS where it pays (ops.mid_pays); else, up to 128 rows, the kernel that shares the rows through
+# Up to this many rows the kernel that streams the weight past one block of 16 rows serves; from 17 to 48 rows the same stream past
+# two or three (ops.ring_pays); from 17 to 256 rows the kernel with rings in LDS where it pays (ops.mid_pays); else, up to 128 rows, the kernel that shares the rows through
 # LDS, where it has blocks enough to fill the chip (ops.wide_pays), and for every product with a float32 result; else
 # the library.
 THIN_ROWS = 16
@@ -66,12 +69,15 @@ class Linear:
     def _product(self, x, out_dtype, planes_ok):
         w = self.weight
         if isinstance(x, Prenormed):
-            if self._folds(x.values):
-                return ops.linear_thin(x.values, w, out_dtype or x.dtype, planes_ok=planes_ok, row_ss=x.ss, row_eps=x.eps)
+            if self._folds(x.values, planes_ok=planes_ok):
+                product = ops.linear_thin if x.shape[0] <= ops.THIN_TOKENS else ops.linear_ring
+                return product(x.values, w, out_dtype or x.dtype, planes_ok=planes_ok, row_ss=x.ss, row_eps=x.eps)
             x = x.materialize()
         out_dtype = out_dtype or x.dtype
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.in_features % 8 == 0:
             rows = x.shape[0]
+            if ops.ring_pays(rows, self.out_features, self.in_features, planes_ok=planes_ok) and self._whole_pieces(x):
+                return ops.linear_ring(x, w, out_dtype, planes_ok=planes_ok)
             if x.is_contiguous() and ops.mid_pays(rows, self.out_features, self.in_features, planes_ok=planes_ok, out_dtype=out_dtype):
                 return ops.linear_mid(x, w, out_dtype, planes_ok=planes_ok)
             if (rows <= THIN_ROWS or out_dtype != torch.bfloat16
@@ -84,13 +90,18 @@ class Linear:
 
     def _big(self, x, gated: bool = False) -> bool:
         """Whether the kernel of large tiles serves these rows (its reads are of 16 bytes)."""
-        return (x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and x.is_contiguous() and self.weight.is_contiguous()
-                and (x.data_ptr() | self.weight.data_ptr()) % 16 == 0
-                and ops.big_pays(x.shape[0], self.out_features, self.in_features, gated=gated))
+        return self._whole_pieces(x) and ops.big_pays(x.shape[0], self.out_features, self.in_features, gated=gated)
 
-    def _folds(self, rows: torch.Tensor) -> bool:
-        """Whether the kernel that folds a norm into the product serves these rows."""
-        return rows.shape[0] <= ops.THIN_TOKENS and ops.thin_serves(rows, self.weight)
+    def _whole_pieces(self, x) -> bool:
+        """Whether rows and weight are bfloat16 that can be read 16 bytes at a time."""
+        return (x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and x.is_contiguous() and self.weight.is_contiguous()
+                and (x.data_ptr() | self.weight.data_ptr()) % 16 == 0)
+
+    def _folds(self, rows: torch.Tensor, gated: bool = False, planes_ok: bool = False) -> bool:
+        """Whether a kernel that folds a norm into the product serves these rows."""
+        if rows.shape[0] <= ops.THIN_TOKENS:
+            return ops.thin_serves(rows, self.weight)
+        return ops.ring_serves(rows.shape[0], self.out_features, self.in_features, gated, planes_ok) and self._whole_pieces(rows)
 
     def _into(self, x, sink):
         rows = x.values if isinstance(x, Prenormed) else x
@@ -107,9 +118,12 @@ class Linear:
         if self.bias is not None:
             return ops.swiglu(self(x))
         if isinstance(x, Prenormed):
-            if self._folds(x.values):
-                return ops.linear_thin(x.values, self.weight, x.dtype, gated=True, row_ss=x.ss, row_eps=x.eps)
+            if self._folds(x.values, gated=True):
+                product = ops.linear_thin if x.shape[0] <= ops.THIN_TOKENS else ops.linear_ring
+                return product(x.values, self.weight, x.dtype, gated=True, row_ss=x.ss, row_eps=x.eps)
             x = x.materialize()
+        if ops.ring_pays(x.shape[0], self.out_features, self.in_features, gated=True) and self._whole_pieces(x):
+            return ops.linear_ring(x, self.weight, x.dtype, gated=True)
         if (x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and x.is_contiguous()
                 and ops.mid_pays(x.shape[0], self.out_features, self.in_features, gated=True)):
             return ops.linear_mid(x, self.weight, x.dtype, gated=True)

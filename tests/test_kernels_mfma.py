@@ -121,6 +121,51 @@ def test_linear_thin_into_the_residual_stream_and_on_with_the_row_factor(ops, M,
         assert torch.allclose(ss2.cpu().double().sum(1), (x1.cpu().double() ** 2).sum(1), rtol=1e-4)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 48])
+@pytest.mark.parametrize("N,K,planes", [(7, 1024, 1), (4096, 4096, 1), (6144, 4096, 2), (4096, 12288, 0), (1000, 3072, 0), (9000, 2048, 2), (515, 8192, 0)])
+def test_products_of_17_to_48_rows_as_one_stream(ops, M, N, K, planes):
+    """Two and three column tiles: whole results in both types, planes of partial sums, one rounding, the same bits every time."""
+    a, w = rand(M, K, seed=M + K).to(DEV), rand(N, K, seed=N, scale=0.5).to(DEV)
+    ref = a.double() @ w.double().t()
+    if ops.ring_serves(M, N, K):
+        got32 = ops.linear_ring(a, w, F32)
+        assert torch.allclose(got32.double(), ref, atol=2e-4 * (K ** 0.5), rtol=1e-5)
+        assert torch.equal(ops.linear_ring(a, w, BF16), got32.to(BF16)) and torch.equal(ops.linear_ring(a, w, F32), got32)
+    else:
+        assert K > 4096
+    got = ops.linear_ring(a, w, BF16, planes_ok=True)
+    assert got.dtype == (F32 if got.dim() == 3 else BF16) and (planes == 0 or ops.core().palm_linear_ring_parts(M, N, K, 0, 1) == planes)
+    if got.dim() == 3:
+        assert all(float(p.abs().max()) > 0 for p in got)
+        assert torch.allclose(got.double().sum(0), ref, atol=2e-4 * (K ** 0.5), rtol=1e-5)
+
+
+@pytest.mark.parametrize("M", [17, 31, 32, 40, 48])
+@pytest.mark.parametrize("N,K", [(1024, 2048), (4096, 4096), (2056, 1024)])
+def test_the_stream_of_17_to_48_rows_into_the_residual_and_on_with_the_row_factor(ops, M, N, K):
+    """As the kernel for up to 16 rows folds a norm in: x += a W1^T, then rows that lack their factor, into a plain product and a gated one."""
+    eps = 1e-5
+    a, w1 = rand(M, K, seed=M).to(DEV), rand(N, K, seed=N, scale=0.1).to(DEV)
+    x0, nw = (rand(M, N, seed=3, dtype=F32) * 3).to(DEV), (rand(N, seed=4, dtype=F32) + 1.0).to(DEV)
+    x = x0.clone()
+    values, ss = ops.linear_thin_into_residual(a, w1, x, nw)
+    x_ref = x0.double() + a.double() @ w1.double().t()
+    assert torch.allclose(x.double(), x_ref, atol=2e-4 * (K ** 0.5), rtol=1e-5) and ss.shape == (M, (N + 15) // 16)
+    assert torch.allclose(ss.double().sum(1), (x_ref ** 2).sum(1), rtol=1e-4)
+    assert torch.equal(values, (x * nw).to(BF16))
+    for N2, gated, planes_ok in ((96, False, False), (6144, False, True), (2 * 176, True, False)):
+        w2 = rand(N2, N, seed=N2, scale=0.2).to(DEV)
+        if not ops.ring_serves(M, N2, N, gated, planes_ok):
+            assert N % 1024 != 0
+            continue
+        got = ops.linear_ring(values, w2, F32, gated=gated, planes_ok=planes_ok, row_ss=ss, row_eps=eps).double()
+        got = got.sum(0) if got.dim() == 3 else got
+        y = values.double() / torch.sqrt(ss.double().sum(1, keepdim=True) / N + eps) @ w2.double().t()
+        want = torch.nn.functional.silu(y[:, :N2 // 2]) * y[:, N2 // 2:] if gated else y
+        # 32-bit sums of exact products and a factor known to some 2^-23
+        assert torch.allclose(got, want, atol=2e-4 * (N ** 0.5), rtol=2e-5), (N2, gated, float((got - want).abs().max()))
+
+
 def test_the_folded_norm_refuses_what_it_does_not_serve(ops):
     from palm_infra_amd.kernels import KernelError
     a, w, x, nw = rand(17, 64).to(DEV), rand(32, 64).to(DEV), torch.zeros(17, 32, device=DEV), torch.ones(32, device=DEV)
