@@ -271,6 +271,28 @@ def test_xielu_on_both_sides_of_zero():
     assert float(ops.xielu(torch.zeros(1, device="cuda"), torch.tensor([0.3, 0.2], device="cuda"))) == 0.0
 
 
+@gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 7, 8, 4095, 4100, 70001])
+def test_xielu_in_pieces_of_sixteen_bytes(dtype, n):
+    """Every remainder and operands that do not start on 16 bytes, around zero, where the series ends and far out: 32-bit arithmetic
+    of some roundings, and one to the type."""
+    from palm_infra_amd.kernels import ops
+    g = torch.Generator().manual_seed(n)
+    z = torch.randn(n + 1, generator=g) * torch.tensor([1e-4, 0.5, 1.0, 30.0, 3000.0])[torch.randint(0, 5, (n + 1,), generator=g)]
+    z[:4] = torch.tensor([-0.5, -0.49999, -0.50001, 0.0])[:n + 1]
+    z, pq = z.to(dtype).cuda(), torch.tensor([0.3, -0.7], device="cuda")
+    for part in (z[:n], z[1:]):
+        want = P.xielu(part.double().cpu(), torch.tensor(0.3, dtype=P.F64), torch.tensor(-0.7, dtype=P.F64))
+        got = ops.xielu(part, pq)
+        # the two terms below zero cancel where they meet: some roundings of 2^-24 of the larger, |z| at most, and of the result
+        bound = 16 * 2.0 ** -24 * (want.abs() + part.double().cpu().abs()) + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)
+        assert bool(((got.double().cpu() - want).abs() <= bound).all()), float(((got.double().cpu() - want).abs() / bound).max())
+    odd = torch.tensor([float("nan"), float("inf"), float("-inf"), -3e38, -0.0], device="cuda")
+    got = ops.xielu(odd, pq).cpu()
+    assert torch.isnan(got[0]) and got[1] == float("inf") and torch.isnan(got[2]) and bool(torch.isfinite(got[3])) and got[4] == 0.0
+
+
 def _step_context(lengths_before, new_counts, n_slots=None):
     """A cache-less context for kernels that only need the packed layout: slots 0.., given starts."""
     from palm_infra_amd.parts import make_context
