@@ -8,7 +8,7 @@
 // about sqrt(K) roundings, which at K = 12288 and 36 layers adds up to more than 1e-4 on logits of order one; two levels
 // leave sqrt(SUM_RUN) + sqrt(K / SUM_RUN).  Two kernels: linear_f32_kernel for float32 throughout, the float32 mode's
 // products, on the matrix cores' 32-bit instruction; linear_tiled_kernel (plain FMA) for every mix of element types (a
-// 32-bit matrix under bfloat16 activations) and for inner sizes that are not whole stages of it.
+// 32-bit matrix under bfloat16 activations) and for inner sizes that are not whole stages of it or beyond its offsets.
 #include "lds_stage.h"
 
 constexpr int TILE_M = 64, TILE_N = 64, TILE_K = 16;
@@ -209,6 +209,9 @@ static void launch_f32(hipStream_t stream, const float* a, const float* w, float
 }
 
 constexpr int F32_MAX_TILES = 5;                     // 16-row tiles of a block: 80 rows
+// A lane's row is an offset of 32 bits from its tile's first.  The limit is the highest tile's, whatever the tile of a call: a row's
+// result does not depend on how many rows are computed with it.
+constexpr int F32_MAX_K = (int)((1ll << 32) / (16 * F32_MAX_TILES * 4));
 
 // The rows go in the fewest blocks of up to 80, of equal height (157 rows: two of 80).  How wide a block is: what takes the
 // fewest rounds of 256 blocks times the work of one, its products and (0.7 of a product each) the operands it reads (157 x 6,144, K =
@@ -245,7 +248,8 @@ PALM_API int palm_linear(hipStream_t stream, const void* a, int a_dtype, const v
                          int c_dtype, int M, int N, int K, int accumulate) {
     PALM_CHECK(M >= 0 && N > 0 && K > 0, "linear: M=%d N=%d K=%d", M, N, K);
     if (M == 0) return 0;
-    if (a_dtype == PALM_F32 && w_dtype == PALM_F32 && c_dtype == PALM_F32 && K % F32_STAGE == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0 && M <= 65535 * 16) {
+    if (a_dtype == PALM_F32 && w_dtype == PALM_F32 && c_dtype == PALM_F32 && K % F32_STAGE == 0 && K <= F32_MAX_K &&
+        ((uintptr_t)a | (uintptr_t)w) % 16 == 0 && M <= 65535 * 16) {
         dispatch_f32(stream, (const float*)a, (const float*)w, (float*)c, M, N, K, accumulate);
         PALM_LAUNCHED();
         return 0;

@@ -243,6 +243,17 @@ def test_float32_products_of_every_width_of_a_block(ops, M, N, K):
         assert torch.equal(ops.linear_exact(a[rows].contiguous().to(DEV), w[part].contiguous().to(DEV)).cpu(), got[rows, part])
 
 
+@pytest.mark.parametrize("K", [13_421_760, 13_600_000])
+def test_float32_products_whose_rows_lie_far_apart(ops, K):
+    """80 rows on both sides of the inner size at which the last one begins 4 GiB behind the first.  Small whole numbers: exact sums."""
+    M, N = 80, 16
+    a, w = torch.zeros(M, K, device=DEV), torch.ones(N, K, device=DEV)
+    value = torch.arange(1.0, M + 1, device=DEV)
+    for k in (0, K // 2, K - 1):
+        a[:, k] = value
+    assert torch.equal(ops.linear_exact(a, w), (3 * value)[:, None].expand(M, N))
+
+
 def test_linear_refuses_what_does_not_fit(ops):
     from palm_infra_amd.kernels import KernelError
     with pytest.raises(KernelError, match="inner size"):
