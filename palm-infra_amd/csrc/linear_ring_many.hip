@@ -15,6 +15,8 @@ static int ring_many_steps(int M) { return M <= 32 ? 6 : 4; }
 // blocks the fewest steps, then the fewest ranges; only one where the result has to come whole.  0: not served.
 PALM_API int palm_linear_ring_parts(int M, int N, int K, int epilogue, int planes_ok) {
     if (M <= 16 || M > RING_MANY_ROWS || N <= 0 || K <= 0 || K % (SUPER_K * RING_WAVES) != 0) return 0;
+    if (epilogue == EPI_SWIGLU && N % 2 != 0) return 0;
+    if ((double)RING_MANY_ROWS * K * 2 >= 2.0e9 || (double)RING_MANY_ROWS * N * 4 >= 2.0e9) return 0;          // (offsets of 32 bits)
     const int steps = K / (SUPER_K * RING_WAVES), strips = epilogue == EPI_SWIGLU ? (N / 2 + 7) / 8 : (N + 15) / 16;
     int best = 0, best_work = 1 << 30;
     for (int parts = 1; parts <= (planes_ok && epilogue == EPI_STORE ? 4 : 1); ++parts) {
@@ -55,8 +57,6 @@ PALM_API int palm_linear_ring(hipStream_t stream, const void* a, const void* w, 
                "linear_ring: adding to the residual stream needs a plain bfloat16 product in one plane, the next norm's weight and room for the "
                "sums of squares");
     PALM_CHECK(parts == 1 || c_dtype == PALM_F32, "linear_ring: planes of partial sums are float32");
-    PALM_CHECK((double)RING_MANY_ROWS * K * 2 < 2.0e9 && (double)RING_MANY_ROWS * N * 4 < 2.0e9, "linear_ring: N=%d K=%d is beyond 32-bit offsets", N, K);
-    PALM_CHECK(epilogue != EPI_SWIGLU || N % 16 == 0, "linear_ring: a gated product needs whole strips, N = %d", N);
     PALM_CHECK(((uintptr_t)a | (uintptr_t)w) % 16 == 0, "linear_ring: operands must be 16-byte aligned");
     if (epilogue == EPI_SWIGLU) {
         PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_ring_tiles<TC, EPI_SWIGLU>(stream, a, w, c, M, N, K, parts, norm));

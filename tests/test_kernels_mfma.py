@@ -166,6 +166,25 @@ def test_the_stream_of_17_to_48_rows_into_the_residual_and_on_with_the_row_facto
         assert torch.allclose(got, want, atol=2e-4 * (N ** 0.5), rtol=2e-5), (N2, gated, float((got - want).abs().max()))
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 48])
+@pytest.mark.parametrize("N,K", [(2008, 2048), (2 * 1001, 4096), (2 * 3, 2048), (22008, 4096)])
+def test_gated_products_of_17_to_48_rows_whose_last_strip_is_not_whole(ops, M, N, K):
+    """Feed-forward sizes that are no multiple of eight, through the linear part, of rows as they are and of rows that lack their norm's
+    factor."""
+    from palm_infra_amd.parts.linear import Linear
+    from palm_infra_amd.parts.residual import Prenormed
+    x, w = rand(M, K, seed=M).to(DEV), rand(N, K, seed=N, scale=K ** -0.5).to(DEV)
+    ss, eps = (rand(M, K // 16, seed=2, dtype=F32) ** 2 * 16).to(DEV), 1e-5
+    factor = 1.0 / torch.sqrt(ss.double().sum(1, keepdim=True) / K + eps)
+    for rows, f in ((x, 1.0), (Prenormed(x, ss, eps), factor)):
+        got = Linear(w).gated(rows)
+        y = f * (x.double() @ w.double().t())
+        want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+        assert got.dtype == BF16 and got.shape == (M, N // 2)
+        # 32-bit sums of exact products, their activation, and one rounding
+        assert torch.allclose(got.double(), want, atol=1e-4, rtol=2.0 ** -8), float((got.double() - want).abs().max())
+
+
 def test_the_folded_norm_refuses_what_it_does_not_serve(ops):
     from palm_infra_amd.kernels import KernelError
     a, w, x, nw = rand(17, 64).to(DEV), rand(32, 64).to(DEV), torch.zeros(17, 32, device=DEV), torch.ones(32, device=DEV)
