@@ -116,14 +116,18 @@ __global__ __launch_bounds__(ATT_WAVES * WAVE) void attention_simple_kernel(
         const int j_first = max(lo, pg * PAGE_TOKENS) - pg * PAGE_TOKENS;
         const int j_last = min(pos, pg * PAGE_TOKENS + PAGE_TOKENS - 1) - pg * PAGE_TOKENS;
         // keys that are not seen have weight 0, and what lies at their places is not read; jj is the same in every lane
+        // (the weights come from all lanes, so before a lane leaves one out)
         auto one_key = [&](int jj) {
+            float w[HEADS];
+#pragma unroll
+            for (int x = 0; x < HEADS; ++x) w[x] = of_lane(p[x], jj);
 #pragma unroll
             for (int i = 0; i < ACC; ++i) {
                 const int d = lane + i * WAVE;
                 if (d >= hd) continue;
                 const float vd = to_float(vp[(size_t)d * PAGE_TOKENS + jj]);
 #pragma unroll
-                for (int x = 0; x < HEADS; ++x) acc[x][i] = fmaf(of_lane(p[x], jj), vd, acc[x][i]);
+                for (int x = 0; x < HEADS; ++x) acc[x][i] = fmaf(w[x], vd, acc[x][i]);
             }
         };
         int jj = j_first;
