@@ -151,25 +151,9 @@ PALM_API int palm_add_normed(hipStream_t stream, float* x, const void* delta, in
 // ---- xIELU ------------------------------------------------------------------------------------------
 __device__ inline float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 
-// exp(z) - 1 - z for z <= 0: near zero by its series, whose terms beyond the eighth are below 2^-28 of the sum there (and where
-// expm1f(z) - z would cancel), else by the hardware's 2^x, whose error is small against a sum of a tenth and more.
-__device__ inline float exp_beyond_line(float z) {
-    float s = 1.f / 362880.f;
-    s = fmaf(s, z, 1.f / 40320.f);
-    s = fmaf(s, z, 1.f / 5040.f);
-    s = fmaf(s, z, 1.f / 720.f);
-    s = fmaf(s, z, 1.f / 120.f);
-    s = fmaf(s, z, 1.f / 24.f);
-    s = fmaf(s, z, 1.f / 6.f);
-    s = fmaf(s, z, 0.5f) * z * z;
-    // (z / ln 2 in two parts: its rounding would be the largest error; below -104 exp(z) is nothing beside 1)
-    const float near = fmaxf(z, -104.f), t = near * 1.4426950408889634f, power = __builtin_amdgcn_exp2f(t);
-    const float e = fmaf(power, 0.69314718055994531f * fmaf(near, 1.4426950408889634f, -t), power) - 1.0f - z;
-    return z > -0.5f ? s : e;
-}
-
-// What bounds it is memory, once an element costs no library call (two bytes a lane and expm1f: 54 us for 2,603 x 16,384 in
-// bfloat16 among a prompt's launches, 46 alone; so 31 alone).  EACH elements a lane and turn, 16 bytes where the operands start on them.
+// What bounds it is memory, once operands come 16 bytes a lane (two bytes: 46 us for 2,603 x 16,384 in bfloat16, so 35; float32 92 and 63).
+// EACH elements a lane and turn, 16 bytes where the operands start on them.  The library's expm1f costs nothing there: with a series
+// near zero and the hardware's 2^x beyond it took 35 us too, and up to twice the error from -1 to -0.5 (1 - e^z cancels against z).
 template <typename T, int EACH>
 __global__ void xielu_kernel(const T* __restrict__ in, T* __restrict__ out, const float* __restrict__ pq, long long n) {
     const float a_pos = softplus_f(pq[0]), a_neg = 0.5f + softplus_f(pq[1]);
@@ -177,7 +161,7 @@ __global__ void xielu_kernel(const T* __restrict__ in, T* __restrict__ out, cons
     const long long pieces = n / EACH;
     auto one = [&](T v) {
         const float z = to_float(v);
-        return from_float<T>(z > 0.f ? fmaf(a_pos * z, z, 0.5f * z) : fmaf(a_neg, exp_beyond_line(z), 0.5f * z));
+        return from_float<T>(z > 0.f ? fmaf(a_pos * z, z, 0.5f * z) : fmaf(a_neg, expm1f(z) - z, 0.5f * z));
     };
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < pieces; i += (long long)gridDim.x * blockDim.x) {
         Piece v = reinterpret_cast<const Piece*>(in)[i];

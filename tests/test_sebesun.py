@@ -8,6 +8,7 @@ first tokens of a sequence, and greedy generation through ``generate``.  In floa
 """
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -275,8 +276,8 @@ def test_xielu_on_both_sides_of_zero():
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n", [1, 7, 8, 4095, 4100, 70001])
 def test_xielu_in_pieces_of_sixteen_bytes(dtype, n):
-    """Every remainder and operands that do not start on 16 bytes, around zero, where the series ends and far out: 32-bit arithmetic
-    of some roundings, and one to the type."""
+    """Every remainder and operands that do not start on 16 bytes, around zero, at a half and far out: 32-bit arithmetic of some
+    roundings, and one to the type."""
     from palm_infra_amd.kernels import ops
     g = torch.Generator().manual_seed(n)
     z = torch.randn(n + 1, generator=g) * torch.tensor([1e-4, 0.5, 1.0, 30.0, 3000.0])[torch.randint(0, 5, (n + 1,), generator=g)]
@@ -291,6 +292,22 @@ def test_xielu_in_pieces_of_sixteen_bytes(dtype, n):
     odd = torch.tensor([float("nan"), float("inf"), float("-inf"), -3e38, -0.0], device="cuda")
     got = ops.xielu(odd, pq).cpu()
     assert torch.isnan(got[0]) and got[1] == float("inf") and torch.isnan(got[2]) and bool(torch.isfinite(got[3])) and got[4] == 0.0
+
+
+@gpu
+def test_xielu_below_zero_is_as_exact_as_its_exponential():
+    """A steep negative side shows exp(z) - 1 - z itself: off by the exponential's last place, the difference's and the result's rounding."""
+    from palm_infra_amd.kernels import ops
+    g = torch.Generator().manual_seed(0)
+    z = -torch.cat([torch.rand(1 << 18, generator=g) * top for top in (0.5, 1.0, 2.0, 20.0)])
+    steep = 100.5                                             # 0.5 + softplus(100)
+    got = ops.xielu(z.cuda(), torch.tensor([0.0, 100.0], device="cuda")).double().cpu().numpy()
+    d = z.double().numpy()
+    near = np.expm1(d)
+    want = steep * (near - d) + 0.5 * d
+    ulp = lambda x: np.spacing(np.abs(x).astype(np.float32)).astype(np.float64)
+    bound = steep * (ulp(near) + 0.5 * ulp(near - d)) + 0.5 * ulp(want)
+    assert (np.abs(got - want) <= bound).all(), float((np.abs(got - want) / bound).max())
 
 
 def _step_context(lengths_before, new_counts, n_slots=None):
