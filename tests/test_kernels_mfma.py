@@ -428,8 +428,8 @@ def test_which_products_of_prompts_take_large_tiles(ops):
 
 @pytest.mark.parametrize("gate", [0.0, -0.0, 30.0, -30.0, 87.5, -87.5, 88.8, -88.8, 200.0, -200.0, 3e38, -3e38, float("inf"), float("-inf"), float("nan")])
 def test_gated_products_in_large_tiles_at_the_activations_limits(ops, gate):
-    """silu at gates that saturate it, at the ends of 2^x's range, infinite and not a number: as the activation's own pass gives it
-    (what is smaller than bfloat16's least normal number aside, 1.2e-38 times the up value)."""
+    """silu at gates that saturate it, at the ends of 2^x's range, infinite and not a number, against 64 bits (what is smaller than
+    bfloat16's least normal number aside, 1.2e-38 times the up value)."""
     M, N, K = 600, 512, 128
     x = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
@@ -438,12 +438,43 @@ def test_gated_products_in_large_tiles_at_the_activations_limits(ops, gate):
     w[N // 2:, 0] = torch.linspace(-3.0, 3.0, N // 2).to(torch.bfloat16)
     if not math.isfinite(gate):                                # (zeros elsewhere would make it NaN in every sum)
         x[:, 1:], w[:, 1:] = 0.0, 0.0
-    g, u = x[:, :1].float() * w[:N // 2, 0].float(), x[:, :1].float() * w[N // 2:, 0].float()
-    want = ops.swiglu(torch.cat([g, u], dim=1).to(torch.bfloat16))
+    g, u = x[:, :1].double() * w[:N // 2, 0].double(), x[:, :1].double() * w[N // 2:, 0].double()
+    want = (g / (1.0 + torch.exp(-g)) * u).to(torch.bfloat16)
     got = ops.linear_big(x, w, gated=True)
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     ok = ~torch.isnan(want)
     assert torch.allclose(got[ok].float(), want[ok].float(), rtol=2.0 ** -7, atol=1e-36)
+
+
+@pytest.mark.parametrize("gate", [-87.5, -88.0, -88.5])
+def test_gated_products_in_large_tiles_whose_activation_is_the_smallest(ops, gate):
+    """e^-gate close to 2^128: gate / (1 + e^-gate) is still a normal number, and shows beside a large up value."""
+    M, N, K = 500, 256, 128
+    x, w = torch.zeros(M, K, dtype=torch.bfloat16, device=DEV), torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
+    x[:, 0] = 1.0
+    w[:N // 2, 0], w[N // 2:, 0] = gate, 1e30
+    want = gate / (1.0 + math.exp(-gate)) * float(w[N // 2, 0])
+    got = ops.linear_big(x, w, gated=True).double()
+    assert float((got - want).abs().max()) <= 2.0 ** -8 * abs(want), (float(got[0, 0]), want)
+
+
+def test_gated_products_in_large_tiles_round_their_activation_once(ops):
+    """Gates and up values that are exact sums: how many results are not the bfloat16 nearest to silu(gate) * up tells the error before
+    that rounding.  A 32-bit value off by 2.4e-7 of itself at most is on another side of the middle between two bfloat16 numbers in
+    2.4e-7 / 2^-8 of all cases, 38 of 614,400; and five deviations more."""
+    M, N, K = 600, 2048, 128
+    g = torch.Generator().manual_seed(0)
+    x, w = torch.zeros(M, K), torch.zeros(N, K)
+    x[:, 0], x[:, 1] = 1.0, torch.arange(1, M + 1) % 128 / 128.0
+    w[:N // 2, 0], w[:N // 2, 1] = -torch.randint(56, 84, (N // 2,), generator=g).float(), torch.randint(-127, 128, (N // 2,), generator=g) / 1024.0
+    w[N // 2:, 0], w[N // 2:, 1] = 1.0, torch.randint(-127, 128, (N // 2,), generator=g) / 1024.0
+    x, w = x.to(torch.bfloat16).to(DEV), w.to(torch.bfloat16).to(DEV)
+    y = x.double() @ w.double().t()
+    assert torch.equal(y, y.float().double())
+    gate, up = y[:, :N // 2], y[:, N // 2:]
+    want = (gate / (1.0 + torch.exp(-gate)) * up).to(torch.bfloat16)
+    missed = int((ops.linear_big(x, w, gated=True) != want).sum())
+    assert missed <= 70, missed
 
 
 @pytest.mark.parametrize("M", [70, 256, 300])
