@@ -263,6 +263,26 @@ __global__ __launch_bounds__(DM_WAVES * WAVE) void attention_diff_mfma_kernel(
     }
 }
 
+struct DiffPlan {
+    int heads_a_block, waves;
+    long long lists;                          // groups of heads of all sequences
+    int tiles;                                // of queries
+};
+// Eight waves a block bring a page for twice as many queries, and two waves a SIMD take turns; four leave more blocks.  Eight win where
+// their blocks fill the compute units: in more than one round where a unit holds one block of either kind (128 and 256 elements, 16
+// heads: 3,000 tokens 144 us against 224 with four, 7,600: 691 and 1,209, 8 prompts of 300: 30 and 40; 1,000 tokens 55 and 50), in
+// two where it holds two of four waves (64 and 128: 4,096 tokens 131 us against 151, 3,000: 90 and 87, 300: 15 and 13).  Key sizes
+// beyond 128 keep four: the registers of a lane.
+static DiffPlan diff_plan(int n_seqs, int max_new, int heads, int kv_heads) {
+    const int per_kv = heads / kv_heads, heads_a_block = per_kv % 4 == 0 ? 4 : per_kv % 2 == 0 ? 2 : 1;
+    const long long lists = (long long)n_seqs * (heads / heads_a_block);
+    auto tiles = [&](int waves) { const int run = waves / heads_a_block * 16; return (max_new + run - 1) / run; };
+    const bool eight = KK <= 4 && lists * tiles(8) >= (2 * STAGES * DM_STAGE > 160 * 1024 ? COMPUTE_UNITS + 1 : 2 * COMPUTE_UNITS);
+    const int waves = eight ? 8 : 4;
+    return DiffPlan{heads_a_block, waves, lists, tiles(waves)};
+}
+PALM_API int palm_attention_diff_mfma_waves(int n_seqs, int max_new, int heads, int kv_heads) { return diff_plan(n_seqs, max_new, heads, kv_heads).waves; }
+
 PALM_API int palm_attention_diff_mfma(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
                                       const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
                                       const int* seq_new, const int* cu_new, int n_seqs, int max_new, int heads, int kv_heads,
@@ -276,20 +296,13 @@ PALM_API int palm_attention_diff_mfma(hipStream_t stream, const void* q, const v
                (VT - 1) * 16 + 4, VT * 16, vdim);
     PALM_CHECK(max_pages > 0, "attention_diff_mfma: max_pages %d", max_pages);
     if (n_seqs == 0 || max_new == 0) return 0;
-    const int per_kv = heads / kv_heads, heads_a_block = per_kv % 4 == 0 ? 4 : per_kv % 2 == 0 ? 2 : 1;
-    const long long lists = (long long)n_seqs * (heads / heads_a_block);
-    auto tiles = [&](int waves) { const int run = waves / heads_a_block * 16; return (max_new + run - 1) / run; };
-    PALM_CHECK(lists * tiles(4) < (1ll << 31), "attention_diff_mfma: %d heads / %d sequences of %d tokens are more than one launch takes", heads, n_seqs, max_new);
-#define DIFF_LAUNCH(WAVES) attention_diff_mfma_kernel<WAVES><<<(unsigned)(lists * tiles(WAVES)), WAVES * WAVE, 0, stream>>>( \
+    const DiffPlan p = diff_plan(n_seqs, max_new, heads, kv_heads);
+    PALM_CHECK(p.lists * p.tiles < (1ll << 31), "attention_diff_mfma: %d heads / %d sequences of %d tokens are more than one launch takes", heads, n_seqs, max_new);
+#define DIFF_LAUNCH(WAVES) attention_diff_mfma_kernel<WAVES><<<(unsigned)(p.lists * p.tiles), WAVES * WAVE, 0, stream>>>( \
         (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, max_pages, seq_slot, seq_start, seq_new, cu_new, \
-        n_seqs, tiles(WAVES), heads, kv_heads, heads_a_block, dim, vdim, scale, lambda, gain, eps, (bf16_t*)out)
-    // Eight waves a block bring a page for twice as many queries, and two waves a SIMD take turns; four leave more blocks.  Eight win where
-    // their blocks fill the compute units: in more than one round where a unit holds one block of either kind (128 and 256 elements, 16
-    // heads: 3,000 tokens 144 us against 224 with four, 7,600: 691 and 1,209, 8 prompts of 300: 30 and 40; 1,000 tokens 55 and 50), in
-    // two where it holds two of four waves (64 and 128: 4,096 tokens 131 us against 151, 3,000: 90 and 87, 300: 15 and 13).  Key sizes
-    // beyond 128 keep four: the registers of a lane.
+        n_seqs, p.tiles, heads, kv_heads, p.heads_a_block, dim, vdim, scale, lambda, gain, eps, (bf16_t*)out)
     if constexpr (KK <= 4) {
-        if (lists * tiles(8) >= (2 * STAGES * DM_STAGE > 160 * 1024 ? COMPUTE_UNITS + 1 : 2 * COMPUTE_UNITS)) {
+        if (p.waves == 8) {
             DIFF_LAUNCH(8);
             PALM_LAUNCHED();
             return 0;

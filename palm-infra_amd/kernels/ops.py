@@ -1399,6 +1399,7 @@ def attention_diff_lib(dim: int, vdim: int):
         lib = library.load(f"attention_diff_k{key[0]}_v{key[1]}")
         lib.palm_attention_diff_mfma.argtypes, lib.palm_attention_diff_mfma.restype = _DIFF_MFMA_SIGNATURE, c_int
         lib.palm_attention_diff_mfma_sizes.argtypes, lib.palm_attention_diff_mfma_sizes.restype = [c_int], c_int
+        lib.palm_attention_diff_mfma_waves.argtypes, lib.palm_attention_diff_mfma_waves.restype = [c_int] * 4, c_int
         if tuple(lib.palm_attention_diff_mfma_sizes(i) for i in range(2)) != (key[0] * 32, key[1] * 16):
             raise KernelError(f"library attention_diff_k{key[0]}_v{key[1]} was built for other sizes")
         _diff_libs[key] = lib

@@ -623,9 +623,25 @@ def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge
 @pytest.mark.parametrize("heads,kv_heads,dk,dv", [(4, 1, 64, 128), (8, 2, 128, 256), (6, 3, 40, 72), (3, 3, 96, 64), (8, 2, 256, 256), (4, 1, 32, 20)])
 @pytest.mark.parametrize("lengths", [(1, 15), (16, 17, 64), (65, 129, 33), (700, 300, 513, 64)])
 def test_differential_attention_of_prompts_at_the_edges_of_its_blocks(heads, kv_heads, dk, dv, lengths):
-    """Prompts on the matrix cores (four or eight waves a block, one or two pages in LDS, heads of a block that share keys or do
-    not) against 64 bits, over pages whose places beyond the sequences hold NaN, and with keys already there."""
+    """Prompts on the matrix cores in blocks of four waves (one or two pages in LDS, heads of a block that share keys or do not) against
+    64 bits, over pages whose places beyond the sequences hold NaN, and with keys already there."""
+    check_differential_prompts(heads, kv_heads, dk, dv, lengths, waves=4)
+
+
+@gpu
+@pytest.mark.parametrize("heads,kv_heads,dk,dv,lengths,waves", [
+    (16, 4, 128, 256, (1100, 1037, 63), 8), (16, 4, 128, 256, (2048, 17), 8), (16, 4, 128, 256, (1000,), 4),          # one page of either kind in LDS
+    (16, 4, 64, 128, (1100, 1037, 63, 700), 8), (16, 4, 64, 128, (1100, 1037, 63), 4), (8, 2, 40, 72, (513,) * 16, 8),
+    (12, 6, 64, 128, (1100, 1037, 63, 700, 129), 8), (12, 12, 96, 64, (1100, 1037, 63, 700, 129), 8)])                # two heads a block, and one
+def test_differential_attention_of_prompts_in_blocks_of_eight_waves(heads, kv_heads, dk, dv, lengths, waves):
+    """Prompts on both sides of where the blocks of eight waves begin: heads and runs of queries that they share a page for, ends of
+    sequences inside a block, waves without a query."""
+    check_differential_prompts(heads, kv_heads, dk, dv, lengths, waves)
+
+
+def check_differential_prompts(heads, kv_heads, dk, dv, lengths, waves):
     from palm_infra_amd.kernels import ops
+    assert ops.attention_diff_lib(dk, dv).palm_attention_diff_mfma_waves(len(lengths), max(lengths), heads, kv_heads) == waves
     torch.manual_seed(sum(lengths) + dk)
     scale, lam, gain, eps = dk ** -0.5, 0.4, 0.6, 1e-6
     starts = [70 * (b % 2) for b in range(len(lengths))]
