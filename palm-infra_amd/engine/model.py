@@ -69,9 +69,10 @@ class DecoderModel:
                 # the sum is made in 32-bit in the pass that norms it for this entry
                 h = self.layers[call.layer].entry_norm(x, delta=x0, update=True)
             if i + 1 < len(self.order):
-                sink = ResidualSink(x, self.layers[self.order[i + 1].layer].entry_norm)
+                after = self.layers[self.order[i + 1].layer]
+                sink = ResidualSink(x, after.entry_norm, reader=getattr(after, "entry_reader", None))
             else:
-                sink = ResidualSink(x, self.final_norm, rows=want_rows)
+                sink = ResidualSink(x, self.final_norm, rows=want_rows, reader=self.head)
             h = self.layers[call.layer].forward(x, h, ctx, sink)
         ctx.layer_cache = None
         ctx.results = None

@@ -423,17 +423,27 @@ WIDE_FLOAT32_TOKENS = 64   # a float32 result (logits) of more rows than this go
 
 
 COMPUTE_UNITS = 256     # of an MI355X; a folded product's blocks come in rounds of this many
+FOLD_MANY_K = 5120
 
 
 def fold_pays(M: int, N: int, K: int) -> bool:
-    """Whether a product of M <= 16 rows (or up to 48 that ``ring_serves`` takes whole: 4,096 x 4,096 10.2 to 13.0 us, 9.7 to 10.3 and
-    the norm's 5.2 apart) that is a branch's output should fold the residual add and the next norm
+    """Whether a product of M <= 16 rows that is a branch's output should fold the residual add and the next norm
     in, or rather be cut along K into planes that the norm's own kernel adds up.  A fold needs all of K in one
     block.  Up to K = 8192 the block keeps the activations in registers and the fold won at every width measured
     (N 1024 to 5120: 8 to 28 us against 8 to 36).  Beyond that it reads them beside the weights and wins only
     where whole rounds of blocks fill the compute units: N 4096 at K 12288 and 14336 (25 to 42 us against 32 to
     41), not N 2560 or 5120 (a quarter of a second round: 55 to 125 us against 40 to 66), and nowhere measured
-    beyond K 14336."""
+    beyond K 14336.
+
+    17 to 48 rows (that ``ring_serves`` takes whole): inner sizes up to FOLD_MANY_K, and only where the same stream serves
+    what reads the rows, so N a whole number of its steps; else they get their factor in a pass of their own.  Us with the
+    next product, folded and apart, 17 and 48 rows: N 1,024, K 1,024, gate/up of 6,144 9.9 11.6 and 19.4 22.6; 2,048, 2,048, 12,288
+    18.4 20.7 and 19.9 21.5; 4,096, 4,096, 24,576 47.5 53.3 and 49.9 52.7; 3,072, 3,072, 16,384 28.4 32.1 and 31.0 33.9; 5,120, 5,120, 34,816
+    (17 and 32 rows) 82.2 85.7 and 84.2 85.6.  K beyond: 2,048, 6,144, q/k/v of 4,096 18.7 and 18.1.  Readers that the stream does not
+    serve: 1,536, 2,048, 17,920 27.2 28.1 and 24.2 25.9; 2,560, 4,096, 19,456 41.8 44.6 and 39.2 41.3; 5,120, 4,096, 34,816 (33 and 48 rows)
+    110 117 and 104 112; 8,192, 4,096, 16,384 74.8 76.1 and 69.5 71.0."""
+    if M > THIN_TOKENS:
+        return K <= FOLD_MANY_K and ring_serves(M, N, K) and ring_serves(M, 16, N)
     if K <= 8192:
         return True
     strips = (N + 15) // 16

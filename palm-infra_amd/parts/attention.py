@@ -53,6 +53,7 @@ class Attention:
         return [KVNeed(int(p["num_kv_heads"]), int(p["head_dim"]), int(p["window"]) if p.get("window") else None)]
 
     takes_sink = True
+    takes_prenormed = True
 
     def forward(self, h, ctx, sink=None):
         lc = ctx.layer_cache

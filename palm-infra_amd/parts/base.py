@@ -15,11 +15,13 @@ which model it is in.  Interfaces, by category:
                 A mixer or feed-forward may set ``takes_sink = True`` and have ``forward(h, ctx, sink=None)``: h
                 may then be ``Prenormed`` rows, and with a sink the part returns what the sink's norm makes of
                 the residual stream after its output is added (parts/residual.py), usually by handing the sink
-                to its last ``Linear``.
+                to its last ``Linear``.  ``takes_prenormed = True``: all that it does with ``Prenormed`` rows are products
+                that apply the row factor themselves (also for a head).
   block         ``entry_norm``: the norm applied to the residual stream before the block's first branch;
                 ``forward(x, h, ctx, sink)`` -> normed rows: x is the residual stream (updated in place), h is
                 ``entry_norm`` of x (a tensor or ``Prenormed`` rows), sink names the norm that reads x after the
-                block and the rows it wants; what that norm gives is returned.
+                block and the rows it wants; what that norm gives is returned.  ``entry_reader`` (where there is
+                one): the part that reads h.
   embedding     ``forward(token_ids)`` -> float32 [n, hidden].
   head          ``forward(h)`` -> float32 logits [rows, vocab].
 """

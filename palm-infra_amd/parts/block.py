@@ -67,10 +67,14 @@ class PreNormBlock:
     def entry_norm(self):
         return self.mixer_norm
 
+    @property
+    def entry_reader(self):
+        return self.mixer
+
     def forward(self, x, h, ctx, sink):
         if self.feed_forward is None:
             return run_branch(self.mixer, h, ctx, sink)
-        h = run_branch(self.mixer, h, ctx, ResidualSink(x, self.feed_forward_norm))
+        h = run_branch(self.mixer, h, ctx, ResidualSink(x, self.feed_forward_norm, reader=self.feed_forward))
         return run_branch(self.feed_forward, h, ctx, sink)
 
 

@@ -29,6 +29,7 @@ class TokenEmbedding:
 @register_part("head", "linear")
 class LinearHead:
     capturable = True
+    takes_prenormed = True
 
     """logits = h W^T in float32; W is lm_head.weight, or the embedding table when the head is tied
     (models/qwen3.py:89-95, 162-165; engine/engine.cpp:403-485).  With ``softcap`` c the logits are c * tanh(logits / c)."""

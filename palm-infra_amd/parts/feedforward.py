@@ -63,6 +63,7 @@ class GatedSiluFeedForward:
                              f"do not fit hidden {self.hidden}, intermediate {self.inter}")
 
     takes_sink = True
+    takes_prenormed = True
 
     def forward(self, h, ctx, sink=None):
         return self.down(self.gate_up.gated(h), sink=sink)

@@ -106,7 +106,7 @@ class Linear:
     def _into(self, x, sink):
         rows = x.values if isinstance(x, Prenormed) else x
         if (self.bias is None and sink.foldable and self._folds(rows) and sink.x.shape == (rows.shape[0], self.out_features)
-                and rows.dtype == torch.bfloat16 and ops.fold_pays(rows.shape[0], self.out_features, self.in_features)):
+                and rows.dtype == torch.bfloat16 and sink.fold_pays(rows.shape[0], self.out_features, self.in_features)):
             ss_in, eps_in = (x.ss, x.eps) if isinstance(x, Prenormed) else (None, 0.0)
             values, ss = ops.linear_thin_into_residual(rows, self.weight, sink.x, sink.norm.weight, row_ss=ss_in, row_eps=eps_in)
             return Prenormed(values, ss, sink.norm.eps)

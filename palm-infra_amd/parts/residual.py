@@ -58,10 +58,11 @@ def as_tensor(h) -> torch.Tensor:
 
 class ResidualSink:
     """x: the float32 residual stream [n, width], updated in place; norm: the part that reads it next;
-    rows: the rows that reader wants (None: all, and x is updated)."""
+    rows: the rows that reader wants (None: all, and x is updated); reader: the part that reads the norm's rows, where the
+    block or the model knows it."""
 
-    def __init__(self, x: torch.Tensor, norm, rows: torch.Tensor | None = None):
-        self.x, self.norm, self.rows = x, norm, rows
+    def __init__(self, x: torch.Tensor, norm, rows: torch.Tensor | None = None, reader=None):
+        self.x, self.norm, self.rows, self.reader = x, norm, rows, reader
 
     @property
     def takes_planes(self) -> bool:
@@ -72,6 +73,13 @@ class ResidualSink:
         """Whether a product may do the add and this norm's elementwise part itself: a norm of the form
         x * f(row) * weight with f from the mean square (it says so), over all rows."""
         return self.rows is None and bool(getattr(self.norm, "folds_into_products", False))
+
+    def fold_pays(self, n: int, width: int, inner: int) -> bool:
+        """Whether a product of n rows should use that.  More rows than the thin products take: only where what reads the rows
+        next takes them without their factor (a pass of its own costs more than the norm's pass did)."""
+        if n > ops.THIN_TOKENS and not getattr(self.reader, "takes_prenormed", False):
+            return False
+        return ops.fold_pays(n, width, inner)
 
     def finish(self, delta: torch.Tensor) -> torch.Tensor:
         if self.rows is None:
