@@ -73,7 +73,7 @@ def test_grouped_products(form, E, top, W, F, n, uneven):
 @pytest.mark.parametrize("E,top,W,F,n,uneven", [(7, 3, 64, 128, 1, False), (4, 1, 1088, 64, 129, True), (3, 1, 192, 320, 200, False), (2, 2, 640, 576, 97, False),
                                                 (2, 1, 128, 704, 290, True), (2, 1, 256, 64, 430, False)])
 def test_grouped_tiles(form, E, top, W, F, n, uneven):
-    """Tiles of 64 to 256 rows, with one stage and many, part tiles of features and of rows, and rows that start on no 16 bytes
+    """Tiles of 64 rows, with one stage and many, part tiles of features and of rows, and rows that start on no 16 bytes
     (which take the fragments' kernel): 32-bit sums of the same products, one rounding of the inner rows and one of the experts'."""
     from palm_infra_amd.kernels import ops
     h, up, down, chosen, weight = case(form, E, top, W, F, n, uneven, E * n + F, torch.bfloat16)
@@ -85,6 +85,30 @@ def test_grouped_tiles(form, E, top, W, F, n, uneven):
     assert torch.equal(ops.moe_grouped(*args, F, form), first)
     odd = torch.empty(n * W + 1, dtype=torch.bfloat16, device="cuda")[1:].view(n, W).copy_(args[0])
     assert float((ops.moe_grouped(odd, *args[1:], F, form).cpu().double() - want).abs().max()) <= tol
+
+
+@gpu
+@pytest.mark.parametrize("form,E,top,W,F,n,uneven,tile", [
+    ("gated_silu", 64, 2, 320, 1088, 640, True, 64), ("gated_silu", 64, 2, 1088, 320, 1920, True, 128), ("gated_silu", 64, 2, 320, 1088, 3520, False, 192),
+    ("capped_gated", 64, 2, 1088, 320, 3520, True, 192), ("gated_silu", 64, 2, 1088, 320, 5440, True, 256), ("capped_gated", 36, 2, 1088, 1088, 3060, False, 256),
+    ("relu_squared", 64, 2, 1088, 320, 1920, False, 128), ("gelu", 64, 2, 320, 1088, 7360, True, 192), ("relu_squared", 80, 2, 1088, 320, 6800, True, 256)])
+def test_grouped_tiles_of_every_height_one_after_the_other(form, E, top, W, F, n, uneven, tile):
+    """More tiles than compute units, so that blocks go on into another expert's, 5 and 17 stages that the walk begins inside and wraps
+    around, an expert of many tiles and one that nobody chose."""
+    from palm_infra_amd.kernels import ops
+    gated = ops.expert_rows(form) > 1
+    assert ops.feedforward().palm_moe_tile_tokens(n * top, E, W, F, int(gated), 1) == tile
+    assert E * max(-(-F // (128 if gated else 256)), -(-W // 256)) > 256
+    cap = CAP if form == "capped_gated" else ops.NO_CAP
+    h, up, down, chosen, weight = case(form, E, top, W, F, n, uneven, E * n + F, torch.bfloat16)
+    want = plain_mixture(form, h, up, down, chosen, weight, F)
+    args = [t.cuda() for t in (h, up, down, chosen, weight)]
+    for exact in (False, True):
+        got = ops.moe_grouped(*args, F, form, cap, exact=exact)
+        # the inner rows are rounded to bfloat16, 0.0017 of them in the mean square; so are the experts' results, unless they stay in 32 bits
+        assert float((got.cpu().double() - want).norm() / want.norm()) < (0.003 if exact else 0.004)
+        assert float((got.cpu().double() - want).abs().max()) <= 0.02 * float(want.abs().max())
+        assert torch.equal(ops.moe_grouped(*args, F, form, cap, exact=exact), got)
 
 
 @gpu
