@@ -220,14 +220,15 @@ constexpr int F32_MAX_K = (int)((1ll << 32) / (16 * F32_MAX_TILES * 4));
 // (16 rows, 24,576 x 4,096: 75 us against 86, one row 75 and 78).
 static void dispatch_f32(hipStream_t stream, const float* a, const float* w, float* c, int M, int N, int K, int accumulate) {
     const int tiles = (M + 15) / 16, blocks_m = (tiles + F32_MAX_TILES - 1) / F32_MAX_TILES, mt = (tiles + blocks_m - 1) / blocks_m;
-    int nt = 1;
-    double least = 1e300;
-    for (int candidate : {4, 3, 2, 1}) {
-        const long long blocks = (long long)((N + 16 * candidate - 1) / (16 * candidate)) * blocks_m;
-        const double cost = (double)((blocks + 255) / 256) * (mt * candidate + 0.7 * (mt + candidate));
-        if (cost < least) { least = cost; nt = candidate; }
+    int nt = N >= 256 * 48 && K >= 4096 ? 3 : 1;
+    if (mt > 1) {
+        double least = 1e300;
+        for (int candidate : {4, 3, 2, 1}) {
+            const long long blocks = (long long)((N + 16 * candidate - 1) / (16 * candidate)) * blocks_m;
+            const double cost = (double)((blocks + 255) / 256) * (mt * candidate + 0.7 * (mt + candidate));
+            if (cost < least) { least = cost; nt = candidate; }
+        }
     }
-    if (mt == 1) nt = N >= 256 * 48 && K >= 4096 ? 3 : 1;
 #define PALM_F32_CASE(MT) case MT: \
         if (nt == 4) launch_f32<MT, 4>(stream, a, w, c, M, N, K, accumulate); \
         else if (nt == 3) launch_f32<MT, 3>(stream, a, w, c, M, N, K, accumulate); \
@@ -235,7 +236,10 @@ static void dispatch_f32(hipStream_t stream, const float* a, const float* w, flo
         else launch_f32<MT, 1>(stream, a, w, c, M, N, K, accumulate); \
         break
     switch (mt) {
-        PALM_F32_CASE(1);
+        case 1:
+            if (nt == 3) launch_f32<1, 3>(stream, a, w, c, M, N, K, accumulate);
+            else launch_f32<1, 1>(stream, a, w, c, M, N, K, accumulate);
+            break;
         PALM_F32_CASE(2);
         PALM_F32_CASE(3);
         PALM_F32_CASE(4);
