@@ -15,8 +15,12 @@
 
 constexpr int ATT_WAVES = 4;
 constexpr int ATT_MAX_HD = 512;
-// (query, head) pairs from which a block takes four heads: below, the chip has room for a block each.  Us, one and four heads a block, 32
-// heads of 128 on eight: 544 pairs 6.0 and 9.2 (17 queries of a prompt), 1,024 476 and 57 (32 sequences of 900), 1,280 12.5 and 10.4, 5,024 64 and 31
+// (query, head) pairs, every sequence counted as the longest, from which a block takes four heads: below, the chip has room for a block
+// each.  Us, one and four heads a block, 32 heads of 128 on eight: 544 pairs 6.0 and 9.2 (17 queries of a prompt), 1,024 448 and 57 (32 sequences
+// of 900), 1,280 12.2 and 10.6, 5,024 64 and 30.  Groups of three heads (24 on eight), whose fourth is computed for nobody: 960 pairs 8.8 and 10.1, 1,536
+// 17.8 and 11.7, 3,768 51 and 29; of five (40 on eight), two blocks: 1,280 13.3 and 10.2, 1,600 13.5 and 11.2, 6,280 77 and 44.  Ragged steps: a prompt of 20 beside
+// seven sequences of 500 101 and 51, of 8 beside fifteen 315 and 176; where all is short a few microseconds either way (17, 1 and 1 tokens 6.1 and 9.4;
+// 40, 7, 7, 7 and 7 16.1 and 10.7).
 constexpr long long SIMPLE_SHARED_FROM = 1024;
 
 // Four consecutive elements, widened.

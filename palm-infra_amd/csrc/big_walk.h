@@ -33,9 +33,6 @@ constexpr int BIG_FEAT = 256, BIG_DIES = 8;
 constexpr int big_ahead(int nt) { return nt <= 2 ? 3 : 2; }
 constexpr int big_lds_bytes(int nt) { return (big_ahead(nt) * BIG_FEAT + (big_ahead(nt) + 1) * 64 * nt) * BIG_ROW; }
 
-__device__ __forceinline__ void big_load(const char* base, uint32_t offset, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds) : "m0", "memory");
-}
 __device__ __forceinline__ void big_swap() {               // the block's barrier; loads stay on their way
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_barrier" ::: "memory");

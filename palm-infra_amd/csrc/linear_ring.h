@@ -1,4 +1,4 @@
-// C[M, N] = A[M, K] . W[N, K]^T for up to 16 rows and a long K (decode steps), the weights crossing LDS.
+// C[M, N] = A[M, K] . W[N, K]^T for up to 48 rows, in tiles of 16, and a long K (decode steps), the weights crossing LDS.
 //
 // The matrix instruction wants a lane to hold 16 bytes of weight row (lane % 16); a wave's read of that shape touches
 // 16 cache lines 64 bytes at a time, and the vector cache takes such an instruction at a quarter of the rate of one

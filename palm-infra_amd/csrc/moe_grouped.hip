@@ -177,8 +177,8 @@ __global__ __launch_bounds__(GT_WAVES * WAVE) void moe_grouped_kernel(const bf16
 //   - an expert's features begin their walk at stages of their own: rows lie 4 or 8 KB apart, and blocks that walk in step ask
 //     all for the same few of memory's channels (352 rows: 288 us in step, 234 so, tiles of 128 rows)
 //   - the tile is as high as an expert's rows need, as long as that spares another tile (see big_tile_of).
-// Us with plan and sum, squared relu, rows of four choices over 32 experts: 130 rows 484 -> 211 (fragments from memory before),
-// 352: 347 -> 212, 852: 372 -> 262, 2,048: 590 -> 440 (a ring of three stages of 32 x 32 x 16 instructions before).
+// Us with plan and sum, squared relu, rows of four choices over 32 experts: 130 rows 484 -> 209 (fragments from memory before),
+// 852: 372 -> 251, 2,048: 590 -> 388 (a ring of three stages of 32 x 32 x 16 instructions before; this walk with eight waves 262 and 440).
 template <int NT, int FORM, typename TO>
 __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void moe_big_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ slot_pair, int top, const bf16_t* __restrict__ w, const int* __restrict__ tile_expert,
@@ -278,9 +278,11 @@ struct MoeSizes {
 // Rows of a tile for experts with n_pairs / experts rows each: what takes the fewest stages' time (0.75, 0.87, 1.13 and 1.42 us
 // for 64 to 256 rows) for an expert with somewhat more rows than the mean, a second tile for a few experts costing
 // almost a whole round.  Tiles that do not fill the chip run side by side, so few or small experts take low ones: 16 experts of 256 x
-// 512 with 125 rows each 43 us in tiles of 192 rows, 29 in tiles of 64.  Measured with a full chip, us, 32 experts of 2,048 x 4,096, tiles of 64 / 128 / 192 / 256 rows: mean 25: 212 / 230 / 272 /
-// 317, 75: 288 / 231 / 244 / 275, 106: - / 308 / 262 / 312, 187: - / 363 / 378 / 303, 256: - / 484 / 440 / 454, 625: 1,247 / 909 /
-// 849 / 831.
+// 512 with 250 rows each 51 us in tiles of 192 rows, 30 in tiles of 64.  Measured with a full chip, us, 32 experts of 2,048 x 4,096, tiles of
+// 64 / 128 / 192 / 256 rows: mean 25: 210 / 222 / 242 / 271, 75: 291 / 230 / 247 / 268, 106: 345 / 294 / 251 / 279, 150: 390 / 314 / 257 / 281,
+// 181: 439 / 323 / 345 / 288, 256: 571 / 438 / 388 / 450, 375: 752 / 549 / 519 / 472, 625: 1,125 / 794 / 724 / 709.  At 49 sizes (8 to 128 experts of 256
+// to 2,048 x 512 to 4,096, means of 8 to 2,000 rows) it takes the best tile at 40 and is 1.0 % behind it in the mean, 10 % at worst (1,000 rows for each of
+// 16 small experts); with the times that a fit over those sizes gives (0.65, 0.77, 1.04, 1.46) it chooses otherwise at three of them, no better.
 static int big_tile_of(const MoeSizes& s) {
     const double mean = (double)s.n_pairs / s.experts, rows = mean + 2.25 * sqrt(mean), in_use = (double)min((long long)s.experts, s.n_pairs);
     const double stage_us[4] = {0.75, 0.87, 1.13, 1.42};

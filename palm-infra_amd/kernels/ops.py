@@ -542,6 +542,10 @@ def big_pays(M: int, N: int, K: int, gated: bool = False) -> bool:
       elsewhere 0.86 (2,603 x 16,384, K = 4,096: 2.75 rounds, 0.70; 13,331 x 6,144: 4.97, 0.77; 2.6 to 2.8 rounds 0.67 to 1.10)
       beyond: in the upper half of a round (0.90; the lower 1.02)
       inner sizes beyond 16,384 whatever the rounds
+    Why the lines lie there: the library's kernels for these sizes have tiles of 256 x 256 too (by their names; 256 x 160 or 192 up to half a
+    round beyond a whole one) and are even with these where the last round is mostly full (8,192 weight rows, K = 2,048, 3.4 to 4 rounds: 1.02 to
+    1.06 of its time), but just beyond a whole round, and in some sizes anywhere, take a quarter to a half longer (3.1 rounds 0.86, 4.1
+    0.79; 2.75 and 2.88 0.82 and 0.67 between 1.09 at 2.62 and 3.0): the ranges are where it does so at most sizes.
     0.83 in the mean where this says yes (312 of 786); 32 lose more than 2 % to the library."""
     if M < (BIG_GATED_FROM if gated else BIG_FROM) or not core().palm_linear_big_takes(M, N, K, int(gated)):
         return False
