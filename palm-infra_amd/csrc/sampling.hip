@@ -342,7 +342,7 @@ __device__ void write_probabilities(const float* __restrict__ row, int V, float 
 }
 
 // One row by the whole block.  *out = the token; probs_out (optional, [V]) = the distribution drawn from.
-__device__ __forceinline__ void sample_row(const float* __restrict__ row, int V, const float* __restrict__ uniform, float temperature, int top_k,
+__device__ __forceinline__ void sample_row(const float* __restrict__ row, int V, float u, float temperature, int top_k,
                                            float top_p, float min_p, int* __restrict__ out, float* __restrict__ probs_out, SampleShared& sh) {
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const BestPair best = block_argmax(row, V, sh.best);
@@ -353,7 +353,6 @@ __device__ __forceinline__ void sample_row(const float* __restrict__ row, int V,
     }
     const float l_max = best.v, inv_t = 1.0f / temperature;
     const float min_w = min_p > 0.f ? min_p : 0.f;          // w_best = exp(0) = 1
-    const float u = *uniform;
     const bool use_top_p = top_p > 0.f && top_p < 1.f;
     const Range mine = wave_range(V);
 
@@ -766,7 +765,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const float* __restrict__ logits, int V, const float* __restrict__ uniforms, float temperature, int top_k,
     float top_p, float min_p, int* __restrict__ out, float* __restrict__ probs_all) {
     __shared__ SampleShared sh;
-    sample_row(logits + (size_t)blockIdx.x * V, V, uniforms + blockIdx.x, temperature, top_k, top_p, min_p, out + blockIdx.x,
+    sample_row(logits + (size_t)blockIdx.x * V, V, uniforms ? uniforms[blockIdx.x] : 0.f, temperature, top_k, top_p, min_p, out + blockIdx.x,
                probs_all ? probs_all + (size_t)blockIdx.x * V : nullptr, sh);
 }
 
@@ -775,14 +774,15 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
 // 110 us for 151,936 logits whatever the batch.  Here the row is cut into slices of up to SLICE elements, a block each,
 // which stay in registers: a slice hands on what may belong to the row's k largest, and a second kernel (a block a row)
 // takes the exact k of the slices' candidates, sorts them and draws as sample_row does, in the same order of operations.
-// A slice's cut is the k-th largest of its threads' maxima (the least that fewer than k of them exceed): k elements of the slice are at least that large, so no element
-// below it belongs to the k; for k = 50 some 55 of 4,096 elements are not below it.  The second kernel narrows the 2,000
+// A slice's cut is made of its threads' maxima: its waves share the k out, and the least of the lines that so many maxima of a wave
+// reach is one that k elements of the slice reach, so no element below it belongs to the k; for k = 50 some 60 of 4,096 elements are not below it.  The second kernel narrows the 2,000
 // candidates of a row down the same way before it ranks what is left, each against each.  Where that leaves more candidates than
 // there is room for (many equal logits, as of a row with most of its vocabulary masked) the slice or the row is cut once more by key
 // and index together, lower indices first: no two elements are equal then.  A row that still does not go this way, or has a NaN in
 // it, is done by sample_row.  (33 rows of 151,936 logits of which all but some 40 are masked: 767 us when sample_row did them, now 67.)
-// Measured with k = 50 and 151,936 logits, both kernels: 21 us for one row (110 as one block), 26 us for 33 (117).  What is left
-// is latency: two launches, and in the second a chain of two trips to memory, five barriers and the k dependent additions.
+// Measured with k = 50 and 151,936 logits, 33 rows, both kernels in a recorded run: 17 us (25 with a count of larger keys for every
+// key; 117 as one block a row).  What is left is latency: two launches, 6.6 us for the slices, and in the second, 10.7 us, a chain of two
+// trips to memory, three barriers and the k dependent additions.
 constexpr int SLICE_THREADS = 256;
 constexpr int SLICE_QUADS = 4;                                       // 16-byte pieces of a slice that a thread holds
 constexpr int SLICE = SLICE_THREADS * SLICE_QUADS * 4;
@@ -797,16 +797,21 @@ constexpr int SURVIVORS = 1024;
 // 35 with sixteen, 58 as one block; 32,000 logits 62, 36 and 59).  A slice has a group of four for every thread at least.
 static int slices_of(int V, int k) { return max((V / 4 + SLICE / 4 - 1) / (SLICE / 4), (k + 7) / 8); }
 
-// how many of the 256 keys are larger
-__device__ inline int larger_keys(const uint32_t* keys, uint32_t own) {
-    int n = 0;
-    const uint4* four = reinterpret_cast<const uint4*>(keys);
-#pragma unroll 8
-    for (int j = 0; j < 64; ++j) {
-        const uint4 q = four[j];
-        n += (q.x > own) + (q.y > own) + (q.z > own) + (q.w > own);
+// A key that at least m of the wave's keys, N a lane, reach: the m-th largest, or a smaller one that as many reach (0: there are not m
+// beside the keys 0).  A bit of it at a time, by counting lanes: some 18 steps, which no other wave waits for.  (Counting for each of
+// a block's 256 keys how many are larger, 256 reads of LDS a thread, was half of both kernels' time.)
+template <int N>
+__device__ inline uint32_t reached_by(const uint32_t (&key)[N], int m) {
+    uint32_t line = 0u;
+    for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t trial = line | (1u << bit);
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) n += __popcll(__ballot(key[i] >= trial));
+        if (n >= m) line = trial;
+        if (n == m) break;
     }
-    return n;
+    return line;
 }
 
 // elements in the order of the draw's candidates: larger keys first, equal ones by their lower index (0: none)
@@ -815,54 +820,56 @@ __device__ inline unsigned long long key_and_index(uint32_t key, uint32_t index)
 // counts [rows, slices]: how many candidates (-1: the row does not go this way); cands [rows, slices, SLICE_CAP]: key, index
 __global__ __launch_bounds__(SLICE_THREADS) void topk_slice_kernel(const float* __restrict__ logits, int V, int k, int* __restrict__ counts,
                                                                    uint2* __restrict__ cands) {
-    __shared__ __attribute__((aligned(16))) uint32_t top[SLICE_THREADS];
-    __shared__ uint32_t cut;
-    __shared__ int n, bad;
-    const int slices = gridDim.x, tid = threadIdx.x;
+    constexpr int WAVES = SLICE_THREADS / WAVE;
+    __shared__ uint32_t cut[WAVES];
+    __shared__ bool has_nan[WAVES];
+    __shared__ int n;
+    const int slices = gridDim.x, tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const float4* row = reinterpret_cast<const float4*>(logits + (size_t)blockIdx.y * V);
     const int per = (V / 4 + slices - 1) / slices;                   // the slices are of one length, or nearly
     const int begin = blockIdx.x * per, end = min(V / 4, begin + per);
-    if (tid == 0) { n = 0; bad = 0; cut = 0xffffffffu; }
-    float e[SLICE_QUADS * 4];
+    uint32_t e[SLICE_QUADS * 4];                                     // keys; 0 beyond the slice's end
+    uint32_t best[1] = {0u};
+    bool nan = false;
+    float4 q[SLICE_QUADS];
+#pragma unroll
+    for (int u = 0; u < SLICE_QUADS; ++u) q[u] = row[max(0, min(begin + u * SLICE_THREADS + tid, end - 1))];
 #pragma unroll
     for (int u = 0; u < SLICE_QUADS; ++u) {
-        const int i = begin + u * SLICE_THREADS + tid;
-        const float4 q = i < end ? row[i] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-        e[4 * u] = q.x; e[4 * u + 1] = q.y; e[4 * u + 2] = q.z; e[4 * u + 3] = q.w;
+        const bool there = begin + u * SLICE_THREADS + tid < end;
+        const float l[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            nan |= there && l[c] != l[c];
+            e[4 * u + c] = there ? ordered_key(l[c]) : 0u;
+            best[0] = max(best[0], e[4 * u + c]);
+        }
     }
-    uint32_t best = 0u;
-    bool nan = false;
+    // The cut: the waves whose every lane holds elements share the k out, and the least of their lines is one that k elements reach
+    const int whole = min(WAVES, max(0, end - begin) / WAVE), share = whole ? (k + whole - 1) / whole : k;
+    const uint32_t own_cut = wave < max(whole, 1) ? reached_by(best, share) : 0xffffffffu;
+    const bool any_nan = __ballot(nan) != 0ull;
+    if (lane == 0) { cut[wave] = own_cut; has_nan[wave] = any_nan; }
+    if (tid == 0) n = 0;
+    __syncthreads();
+    uint32_t least = 0xffffffffu;
+    bool bad = false;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) { least = min(least, cut[w]); bad |= has_nan[w]; }
+    least = max(least, 1u);
+    uint2* mine = cands + ((size_t)blockIdx.y * slices + blockIdx.x) * SLICE_CAP;
+    int hits = 0;                                                    // of the wave
+#pragma unroll
+    for (int u = 0; u < SLICE_QUADS * 4; ++u) hits += __popcll(__ballot(e[u] >= least));
+    int at = 0;
+    if (lane == 0 && hits) at = atomicAdd(&n, hits);
+    at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
     for (int u = 0; u < SLICE_QUADS * 4; ++u) {
-        nan |= e[u] != e[u];
-        best = max(best, ordered_key(e[u]));
-    }
-    top[tid] = best;
-    __syncthreads();
-    if (nan) bad = 1;
-    if (larger_keys(top, best) < k) atomicMin(&cut, best);           // the k-th largest is the least of those
-    __syncthreads();
-    const uint32_t least = cut;
-    uint2* mine = cands + ((size_t)blockIdx.y * slices + blockIdx.x) * SLICE_CAP;
-    int hits = 0;
-#pragma unroll
-    for (int u = 0; u < SLICE_QUADS * 4; ++u) hits += begin + (u / 4) * SLICE_THREADS + tid < end && ordered_key(e[u]) >= least;
-    int upto = hits;                                                 // with those of the lanes before
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) { const int o = __shfl_up(upto, off, WAVE); if (tid % WAVE >= off) upto += o; }
-    int at = 0;
-    if (tid % WAVE == WAVE - 1) at = atomicAdd(&n, upto);
-    at = __shfl(at, WAVE - 1, WAVE) + upto - hits;
-    if (hits) {
-#pragma unroll
-        for (int u = 0; u < SLICE_QUADS * 4; ++u) {
-            const int i = begin + (u / 4) * SLICE_THREADS + tid;
-            const uint32_t key = ordered_key(e[u]);
-            if (i < end && key >= least) {
-                if (at < SLICE_CAP) mine[at] = make_uint2(key, 4u * i + u % 4);
-                ++at;
-            }
-        }
+        const bool hit = e[u] >= least;
+        const int place = at + lanes_before(hit);
+        if (hit && place < SLICE_CAP) mine[place] = make_uint2(e[u], 4u * (begin + (u / 4) * SLICE_THREADS + tid) + u % 4);
+        at += __popcll(__ballot(hit));
     }
     __syncthreads();
     int handed_on = n;
@@ -872,7 +879,7 @@ __global__ __launch_bounds__(SLICE_THREADS) void topk_slice_kernel(const float* 
 #pragma unroll
             for (int u = 0; u < SLICE_QUADS * 4; ++u) {
                 const int i = begin + (u / 4) * SLICE_THREADS + tid;
-                if (i < end) f(ordered_key(e[u]), (uint32_t)(4 * i + u % 4));
+                if (i < end) f(e[u], (uint32_t)(4 * i + u % 4));
             }
         };
         unsigned long long own = 0;
@@ -899,7 +906,6 @@ __global__ __launch_bounds__(SLICE_THREADS) void topk_slice_kernel(const float* 
 
 struct DrawShared {
     __attribute__((aligned(16))) uint32_t top[256];
-    uint32_t cut;
     unsigned long long line;
     int n, bad, zeros;
     unsigned long long most[SAMPLE_THREADS];
@@ -908,15 +914,23 @@ struct DrawShared {
     int i[SLICED_TOPK_MAX];
 };
 
+// The rows' uniform numbers: in memory, or with the launch's arguments.
+constexpr int GIVEN_ROWS = 256;
+struct GivenUniforms { float u[GIVEN_ROWS]; };
+__device__ inline float uniform_of(const float* uniforms) { return uniforms[blockIdx.x]; }
+__device__ inline float uniform_of(const GivenUniforms& uniforms) { return uniforms.u[blockIdx.x]; }
+
+template <typename UNIFORMS>
 __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
-    const float* __restrict__ logits, int V, const float* __restrict__ uniforms, float temperature, int k, float top_p, float min_p,
-    const int* __restrict__ counts, const uint2* __restrict__ cands, int slices, int* __restrict__ out) {
+    const float* __restrict__ logits, int V, float temperature, int k, float top_p, float min_p,
+    const int* __restrict__ counts, const uint2* __restrict__ cands, int slices, int* __restrict__ out, const UNIFORMS uniforms) {
     __shared__ union { SampleShared row; DrawShared draw; } shared;
     DrawShared& sh = shared.draw;
     const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     counts += (size_t)blockIdx.x * slices;
     cands += (size_t)blockIdx.x * slices * SLICE_CAP;
-    if (tid == 0) { sh.n = 0; sh.bad = 0; sh.zeros = 0; sh.cut = 0xffffffffu; }
+    if (tid == 0) { sh.n = 0; sh.bad = 0; sh.zeros = 0; }
+    const float u = uniform_of(uniforms);
     __syncthreads();
     // the counts of the first slices a wave takes and the first places a lane takes are asked for together and kept (a place
     // beyond its slice's count holds nothing, and nothing is made of it)
@@ -957,18 +971,34 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
     best = max(best, (uint32_t)__shfl_xor((int)best, 2, WAVE));
     if (tid % 4 == 0) sh.top[tid / 4] = best;
     __syncthreads();
-    if (tid < 256 && larger_keys(sh.top, sh.top[tid]) < k) atomicMin(&sh.cut, sh.top[tid]);
-    __syncthreads();
-    const uint32_t least = max(sh.cut, 1u);
+    // every wave finds the cut for itself: the k-th largest of the groups' maxima
+    const uint4 four = reinterpret_cast<const uint4*>(sh.top)[lane];
+    const uint32_t tops[4] = {four.x, four.y, four.z, four.w};
+    const uint32_t least = max(reached_by(tops, k), 1u);
+    int hits = 0;                                                    // of the wave
+#pragma unroll
+    for (int h = 0; h < HELD; ++h)
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) hits += __popcll(__ballot(held[h][r].x >= least));
+    if (hits) {
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&sh.n, hits);
+        at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+        for (int h = 0; h < HELD; ++h)
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                const bool hit = held[h][r].x >= least;
+                const int place = at + lanes_before(hit);
+                if (hit && place < SURVIVORS) sh.survivor[place] = held[h][r];
+                at += __popcll(__ballot(hit));
+            }
+    }
     auto survives = [&](uint2 one) {
         if (one.x < least) return;
         const int at = atomicAdd(&sh.n, 1);
         if (at < SURVIVORS) sh.survivor[at] = one;
     };
-#pragma unroll
-    for (int h = 0; h < HELD; ++h)
-#pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) survives(held[h][r]);
     rest(survives);
     __syncthreads();
     int n = sh.n;
@@ -1003,19 +1033,23 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
     }
     if (sh.bad || n > SURVIVORS || n < k) {                          // (n < k: fewer than k elements in the row; not with k < V)
         __syncthreads();
-        sample_row(logits + (size_t)blockIdx.x * V, V, uniforms + blockIdx.x, temperature, k, top_p, min_p, out + blockIdx.x, nullptr, shared.row);
+        sample_row(logits + (size_t)blockIdx.x * V, V, u, temperature, k, top_p, min_p, out + blockIdx.x, nullptr, shared.row);
         return;
     }
-    // the k largest by key, ties to the lower index, each to the place that its rank names
-    if (tid < n) {
-        const uint2 own = sh.survivor[tid];
+    // the k largest by key, ties to the lower index, each to the place that its rank names; as many threads as there are for
+    // each (16 where 64 are left) count those before it
+    int sharing = 16;
+    while (sharing > 1 && n * sharing > SAMPLE_THREADS) sharing /= 2;
+    if (wave * WAVE < n * sharing) {
+        const uint2 own = sh.survivor[min(tid / sharing, n - 1)];
         int rank = 0;
-#pragma unroll 8
-        for (int j = 0; j < n; ++j) {
+#pragma unroll 4
+        for (int j = tid % sharing; j < n; j += sharing) {
             const uint2 o = sh.survivor[j];
             rank += o.x > own.x || (o.x == own.x && o.y < own.y);
         }
-        if (rank < k) {
+        for (int off = sharing / 2; off > 0; off /= 2) rank += __shfl_xor(rank, off, WAVE);
+        if (rank < k && tid % sharing == 0 && tid / sharing < n) {
             sh.v[rank] = key_value(own.x);
             sh.i[rank] = (int)own.y;
             if (key_value(own.x) == 0.f) sh.zeros = 1;
@@ -1066,7 +1100,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
         const int last = first_place([&](int h) { return sum_to[h] >= cutoff; }, active, -1);
         if (last >= 0) { active = last + 1; sum = prefix(last); }
     }
-    const float target = uniforms[blockIdx.x] * sum;
+    const float target = u * sum;
     const int pick = first_place([&](int h) { return target <= sum_to[h]; }, active, active - 1);
     if (lane == 0) out[blockIdx.x] = sh.i[pick];
 }
@@ -1099,15 +1133,19 @@ PALM_API long long palm_sample_sliced_work(int n_rows, int V, float temperature,
     return sliced_rows(n_rows, V, top_k) * row_room(V, top_k);
 }
 
-PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, float temperature,
-                                int top_k, float top_p, float min_p, int* out, void* work, long long work_bytes) {
+// uniforms: in device memory; or null, and then made here from (seed, streams[i], draws[i]), arrays in host memory, and handed to the
+// kernel with its arguments, 256 rows a launch.  (Through pinned memory they took a copy of their own on the stream, 3.4 us and the
+// gap behind it, and the host an allocation and a copy: half of its time for a draw.)
+static int sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, unsigned long long seed,
+                         const uint64_t* streams, const uint64_t* draws, float temperature, int top_k, float top_p, float min_p, int* out,
+                         void* work, long long work_bytes) {
     const long long needed = palm_sample_sliced_work(n_rows, V, temperature, top_k);
     PALM_CHECK(needed > 0 && (uintptr_t)logits % 16 == 0, "sample: %d rows of %d logits with top_k = %d do not go in slices", n_rows, V, top_k);
     PALM_CHECK(work_bytes >= needed && (uintptr_t)work % 8 == 0, "sample: %lld bytes of workspace where %lld are needed", work_bytes, needed);
     PALM_CHECK(temperature <= 2.f, "sample: temperature must be between 0 and 2");
     PALM_CHECK(top_p >= 0.f && top_p <= 1.f, "sample: top_p must be between 0 and 1");
     PALM_CHECK(min_p >= 0.f && min_p <= 1.f, "sample: min_p must be between 0 and 1");
-    PALM_CHECK(uniforms, "sample: a draw needs the uniform numbers");
+    PALM_CHECK(uniforms || (streams && draws), "sample: a draw needs the uniform numbers");
     const int slices = slices_of(V, top_k), group = sliced_rows(n_rows, V, top_k);
     uint2* cands = (uint2*)work;
     int* counts = (int*)(cands + (size_t)group * slices * SLICE_CAP);
@@ -1116,8 +1154,31 @@ PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_r
         const float* at = logits + (size_t)r0 * V;
         topk_slice_kernel<<<dim3(slices, rows), SLICE_THREADS, 0, stream>>>(at, V, top_k, counts, cands);
         PALM_LAUNCHED();
-        topk_draw_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(at, V, uniforms + r0, temperature, top_k, top_p, min_p, counts, cands, slices, out + r0);
-        PALM_LAUNCHED();
+        if (uniforms) {
+            topk_draw_kernel<const float*><<<rows, SAMPLE_THREADS, 0, stream>>>(at, V, temperature, top_k, top_p, min_p, counts, cands, slices, out + r0,
+                                                                               uniforms + r0);
+            PALM_LAUNCHED();
+            continue;
+        }
+        for (int r = 0; r < rows; r += GIVEN_ROWS) {
+            const int now = min(GIVEN_ROWS, rows - r);
+            GivenUniforms given{};
+            if (palm_uniforms(seed, streams + r0 + r, draws + r0 + r, now, given.u) != 0) return 1;
+            topk_draw_kernel<GivenUniforms><<<now, SAMPLE_THREADS, 0, stream>>>(
+                at + (size_t)r * V, V, temperature, top_k, top_p, min_p, counts + (size_t)r * slices, cands + (size_t)r * slices * SLICE_CAP, slices,
+                out + r0 + r, given);
+            PALM_LAUNCHED();
+        }
     }
     return 0;
+}
+PALM_API int palm_sample_sliced(hipStream_t stream, const float* logits, int n_rows, int V, const float* uniforms, float temperature,
+                                int top_k, float top_p, float min_p, int* out, void* work, long long work_bytes) {
+    PALM_CHECK(uniforms, "sample: a draw needs the uniform numbers");
+    return sample_sliced(stream, logits, n_rows, V, uniforms, 0ull, nullptr, nullptr, temperature, top_k, top_p, min_p, out, work, work_bytes);
+}
+PALM_API int palm_sample_sliced_drawn(hipStream_t stream, const float* logits, int n_rows, int V, unsigned long long seed, const uint64_t* streams,
+                                      const uint64_t* draws, float temperature, int top_k, float top_p, float min_p, int* out, void* work,
+                                      long long work_bytes) {
+    return sample_sliced(stream, logits, n_rows, V, nullptr, seed, streams, draws, temperature, top_k, top_p, min_p, out, work, work_bytes);
 }

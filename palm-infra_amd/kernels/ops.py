@@ -61,6 +61,8 @@ _SIGNATURES = {
     "palm_uniforms": [c_ulonglong, c_void_p, c_void_p, c_int, c_void_p],
     "palm_sample": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_float, c_int, c_float, c_float, c_void_p, c_void_p],
     "palm_sample_sliced": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_float, c_int, c_float, c_float, c_void_p, c_void_p, c_longlong],
+    "palm_sample_sliced_drawn": [c_void_p, c_void_p, c_int, c_int, c_ulonglong, c_void_p, c_void_p, c_float, c_int, c_float, c_float, c_void_p, c_void_p,
+                                 c_longlong],
     "palm_sample_sliced_work": [c_int, c_int, c_float, c_int],
 }
 
@@ -400,6 +402,27 @@ def sample(logits: torch.Tensor, uniforms: torch.Tensor | None, temperature: flo
     library.call(core(), "palm_sample", _stream(), _p(logits), n, V, _p(uniforms), float(temperature), int(top_k), float(top_p),
                  float(min_p), _p(out), _p(probs))
     return (out, probs) if want_probs else out
+
+
+def sample_drawn(logits: torch.Tensor, seed: int, streams, draws, temperature: float, top_k: int = 0, top_p: float = 0.0,
+                 min_p: float = 0.0) -> torch.Tensor:
+    """``sample`` with the uniform numbers of (seed, streams[i], draws[i]).  Where the rows go in slices the numbers reach the kernel
+    with its arguments; else through pinned memory, so that the host does not wait for the device."""
+    n = logits.shape[0]
+    if logits.is_cuda and logits.dim() == 2 and logits.dtype == F32 and logits.is_contiguous() and logits.data_ptr() % 16 == 0:
+        V = logits.shape[1]
+        needed = core().palm_sample_sliced_work(n, V, temperature, top_k)
+        if needed:
+            s, d = _u64(streams), _u64(draws)
+            _need(len(s) == n and len(d) == n, "sample: a stream and a draw's number for each row")
+            out = torch.empty((n,), dtype=torch.int32, device=logits.device)
+            work = torch.empty((needed,), dtype=torch.uint8, device=logits.device)
+            library.call(core(), "palm_sample_sliced_drawn", _stream(), logits.data_ptr(), n, V, int(seed) & _U64, s.buffer_info()[0],
+                         d.buffer_info()[0], temperature, top_k, top_p, min_p, out.data_ptr(), work.data_ptr(), needed)
+            return out
+    u = torch.empty((n,), dtype=F32, pin_memory=True)
+    uniforms_into(u, seed, streams, draws)
+    return sample(logits, u.to(logits.device, non_blocking=True), temperature, top_k, top_p, min_p)
 
 
 # ---- dispatch: which kernel serves a call -----------------------------------------------------------

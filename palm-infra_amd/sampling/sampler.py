@@ -92,14 +92,11 @@ class DeviceSampler:
                                     p.frequency_penalty)
         if p.greedy:
             return ops.argmax(logits)
-        # through pinned memory: the host does not wait for the device here
-        u = torch.empty((len(states),), dtype=torch.float32, pin_memory=True)
-        ops.uniforms_into(u, p.seed, [st.stream for st in states], [st.draws for st in states])
-        u = u.to(logits.device, non_blocking=True)
+        streams, draws = [st.stream for st in states], [st.draws for st in states]
         for st in states:
             st.draws += 1
         top_k = p.top_k if 0 < p.top_k < V else 0
-        return ops.sample(logits, u, p.temperature, top_k, p.top_p, p.min_p)
+        return ops.sample_drawn(logits, p.seed, streams, draws, p.temperature, top_k, p.top_p, p.min_p)
 
     def probabilities(self, logits: torch.Tensor, states) -> torch.Tensor:
         """The distribution a draw would come from, [B, vocab]; changes no state

@@ -763,6 +763,17 @@ def test_top_k_in_slices_where_logits_are_equal(ops, V, k):
         assert ops.sample(many, u, 0.7, k, 0.95).tolist() == whole(many, u)
 
 
+@pytest.mark.parametrize("n,V,k", [(1, 151936, 50), (256, 16388, 128), (257, 32000, 7), (600, 16384, 50), (5, 16385, 50), (3, 151936, 0)])
+def test_draws_by_streams_are_draws_by_their_uniform_numbers(ops, n, V, k):
+    """Rows in one launch, in several, and where the numbers go through memory (odd vocabularies, no top-k)."""
+    lg = rand(n, V, seed=n, scale=3.0).to(DEV)
+    streams, draws = [3 * i + (1 << 40) for i in range(n)], [i % 5 for i in range(n)]
+    u = torch.empty(n)
+    ops.uniforms_into(u, 42, streams, draws)
+    want = ops.sample(lg, u.to(DEV), 0.8, k, 0.95, 0.0)
+    assert ops.sample_drawn(lg, 42, streams, draws, 0.8, k, 0.95, 0.0).tolist() == want.tolist()
+
+
 def test_rows_are_sampled_independently(ops):
     lg = rand(4, 2000, seed=8)
     u = torch.tensor([0.1, 0.5, 0.9, 0.3])
