@@ -311,6 +311,14 @@ class ModelCache:
                 raise CacheFull(f"the step needs {need} more pages of {PAGE_TOKENS} tokens; "
                                 f"{g.table.pages.free_count} of {g.n_pages} are free")
 
+    def has_room(self, growth: list[tuple[int, int]]) -> bool:
+        """Whether the whole step fits as it is."""
+        try:
+            self.check_room(growth)
+        except CacheFull:
+            return False
+        return True
+
     def reserve(self, growth: list[tuple[int, int]]) -> None:
         """Make room for ``n_new`` more tokens in each ``(slot, n_new)``; nothing is taken if the
         whole step does not fit."""

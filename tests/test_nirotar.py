@@ -878,6 +878,34 @@ def test_a_prompt_longer_than_a_step_takes_at_once(tmp_path_factory, name, dtype
 
 
 @gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_a_long_prompt_takes_smaller_pieces_where_the_window_has_no_room(tmp_path_factory, dtype):
+    """All layers keep a window: a prompt that does not fit at once goes through in the least pieces, one that fits goes at once."""
+    from palm_infra_amd.engine import Engine, StepEntry
+    eng = Engine.from_dir(model_dir(tmp_path_factory, "attention", dtype), dtype=dtype, max_tokens=64 * 18)
+    assert (eng.step_tokens_per_seq, eng.step_tokens_least) == (1024, 1024)
+    eng.step_tokens_least = 100
+    steps = []
+    run = eng._run
+    eng._run = lambda entries: steps.append([len(e.tokens) for e in entries]) or run(entries)
+    a, b, c = S.prompts(raw_of("attention"), [90, 90, 1000], seed=31)
+    sa, sb = eng.open(), eng.open()
+    eng.step([StepEntry(sa, a, []), StepEntry(sb, b, [])])
+    want = [0, 99, 100, 511, 999]
+    for room in (False, True):
+        del steps[:]
+        if room:
+            eng.close(sa), eng.close(sb)
+        sc = eng.open()
+        got = eng.step([StepEntry(sc, c, want)])
+        # (what lies behind the window goes back after each piece: the later ones may have room)
+        assert steps == [[1000]] if room else steps[0] == [100] and sum(n for n, in steps) == 1000
+        assert_close(got, reference(tmp_path_factory, "attention", dtype, c)[want], dtype, "pieces")
+        eng.close(sc)
+    eng.cache.check()
+
+
+@gpu
 @pytest.mark.parametrize("name", ["A", "D"])
 def test_recorded_and_launched_steps_agree(tmp_path_factory, name):
     """Decode steps replayed from a HIP graph against the same steps launched kernel by kernel, several replays with other
