@@ -49,3 +49,10 @@ PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const voi
                                     const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
                                     int hd, float scale, int window, int q_prescaled, void* out);
 PALM_API int palm_attention_prefill_takes_prescaled();
+
+// The same by the kernel whose waves hold 64 columns each (head size 128: palm_attention_prefill_wide_serves()).
+PALM_API int palm_attention_prefill_wide(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
+                                         const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
+                                         const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
+                                         int hd, float scale, int window, int q_prescaled, void* out);
+PALM_API int palm_attention_prefill_wide_serves();

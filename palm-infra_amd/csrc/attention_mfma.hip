@@ -24,6 +24,7 @@
 
 #include "mfma.h"
 #include "attention_api.h"
+#include "lds_stage.h"
 
 #ifndef PALM_HEAD_DIM
 #error "compile with -DPALM_HEAD_DIM=<head size>"
@@ -1496,6 +1497,348 @@ __global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefil
     }
 }
 
+// ---- prefill of long prompts: 64 columns a wave -----------------------------------------------------
+// The kernel above reads every fragment of a page from LDS for two units of 16 columns: 32 KB a wave and page, 1,024 clocks of a
+// compute unit's LDS for its four waves (128 bytes a clock) beside 1,088 clocks of matrix instructions a wave, and the two hardly
+// overlapped (2,300 clocks a page and wave).  Here a wave has four units, so a fragment feeds four products, and is alone on its
+// SIMD; what hides a unit's arithmetic is the wave's own other units.  A product takes 16 clocks and its issue four of them: in the
+// other twelve an exponential (eight) and one or two other instructions run for nothing, more do not (16 products alone 145 ns, with 16
+// exponentials in turn 148, two of each in turn 172).  So every instruction of a page has its place between two products:
+// P and Q are the wave's two pairs of units, a page four runs of products, and between them stand
+//     scores of P           the last keys, half of V^T's fragments, the loads of V^T two pages on, the first maxima of P
+//     scores of Q           P's maxima and most of its weights, the other half of V^T
+//     values by P's weights the rest of them, Q's maxima and half of its weights, the next page's first keys
+//     values by Q's weights the rest of Q's weights, the next page's keys, the loads of the keys three pages on
+// A page's fragments are read once and it takes one barrier (behind the first run); four pages of K and of V^T lie in LDS.  What
+// reads or loads stand at least three products apart (four waves of 8 clocks of LDS, or of 16 of the load's way, each).
+// The maxima decide by one vote, as above, whether any column has to be masked or its reference moved; that is settled aside.
+//
+// Measured, us, the kernel above and this one: 32 heads of 8, 13,331 tokens 1,281 and 1,134 (1.28 PFLOP/s), 2,048 behind 30,720
+// 949 and 780 (1.36), 4,096 142 and 124, 2,048 51 and 58; 40 heads of 8 (the kernel above uses five of its eight units) 8,192 tokens 939 and
+// 590; in the middle of a whole prompt of 13,331, where the chip's clock is lower, 1,511 and 1,358.  A block's start and end (its first keys' way from memory, masks on its first and last page) are some 9 us that no second block
+// hides, so few pages a block, or few blocks, are better served above: ops.wide_prompt_attention.  Tried: sums of the weights by dot
+// products instead of a row of ones on the matrix cores (13,331 tokens 1,200 us); exponentials written out too (1,156).
+constexpr bool PF_WIDE = PF_DMA && HD == 128;
+constexpr int WIDE_UNITS = 4, WIDE_STAGES = 4;
+
+// The products are written out, so that sums and queries stay in the accumulator registers and the scores where vector instructions
+// read them.  The distances that the compiler would keep for its own products are kept by their order: a score is read five
+// products or more behind its last one, a sum is added to again four behind, weights are read behind an s_nop.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void wide_score_first(f32x4& s, bf16x8 k, bf16x8 q, f32x4 from) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %3" : "=&v"(s) : "v"(k), "a"(q), "v"(from));
+}
+__device__ __forceinline__ void wide_score(f32x4& s, bf16x8 k, bf16x8 q) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "a"(q));
+}
+__device__ __forceinline__ void wide_weigh(f32x4& o, bf16x8 v, u32x4 p) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(o) : "v"(v), "v"(p));
+}
+__device__ __forceinline__ float wide_max(float a, float b, float c) {         // (fmaxf would first make each of them quiet)
+    float most;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(most) : "v"(a), "v"(b), "v"(c));
+    return most;
+}
+
+template <bool PRESCALED>
+__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void attention_prefill_wide_kernel(
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+    const int* __restrict__ block_table, int max_pages, const int* __restrict__ seq_slot,
+    const int* __restrict__ seq_start, const int* __restrict__ seq_new, const int* __restrict__ cu_new, int nh,
+    int nkv, float scale_log2, int window, int qb, int hg, bf16_t* __restrict__ out) {
+    if constexpr (PF_WIDE) {
+        constexpr int K_TILE = PAGE_TOKENS * K_STRIDE, V_TILE = HD * V_STRIDE, PAGE_LOADS = 2 * PF_LOADS;
+        constexpr int QK = 8 * KSTEPS, PV = 4 * DTILES + 4;         // products of a pair of units
+        static_assert(QK == 32 && PV == 36 && PAGE_LOADS == 8, "what goes between which products below is laid out for heads of 128");
+        __shared__ __attribute__((aligned(16))) bf16_t k_lds[WIDE_STAGES * K_TILE];
+        __shared__ __attribute__((aligned(16))) bf16_t v_lds[WIDE_STAGES * V_TILE];
+
+        const int b = blockIdx.z;
+        const int G = nh / nkv, n_hg = (G + hg - 1) / hg;
+        const int kvh = blockIdx.x / n_hg, hgi = blockIdx.x % n_hg;   // the kv head runs fastest over the blocks, see the launch
+        const int n_new = seq_new[b];
+        const int subs = qb / 16, n_q = (n_new + qb - 1) / qb;        // tiles of qb queries in this sequence
+        if ((int)blockIdx.y >= n_q) return;
+        const int tile_first = (n_q - 1 - (int)blockIdx.y) * qb;      // the tile's first query: the tiles with the most pages go first
+        const int lane = threadIdx.x % WAVE, r = lane % 16, g = lane / 16;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+        const int start = seq_start[b];
+        const int seq_tail = start + n_new - 1;                       // the sequence's last key
+        const int heads_here = min(hg, G - hgi * hg);
+        const int n_units = heads_here * subs;
+        const int* pages = block_table + (size_t)seq_slot[b] * max_pages;
+        const PageSources sources = page_sources();
+
+        // unit x of the wave: its first query within the step, its head, whether there is one
+        auto first_query = [&](int x) { return tile_first + (wave + x * PF_WAVES) / heads_here * 16; };
+        auto head_of = [&](int x) { return kvh * G + hgi * hg + (wave + x * PF_WAVES) % heads_here; };
+        auto live = [&](int x) { return wave + x * PF_WAVES < n_units && first_query(x) < n_new; };
+        auto first_key = [&](int pos) { return window > 0 ? max(0, pos - window + 1) : 0; };
+        bf16x8 qv[WIDE_UNITS][KSTEPS];
+        f32x4 o[WIDE_UNITS][DTILES], weights[WIDE_UNITS], minus_m[WIDE_UNITS];       // minus the reference of the lane's column, four times
+        unsigned fresh = 0;                                           // bit x: the column has seen no key yet
+        int least_pos = 0x7fffffff, last_first = 0;                   // over the columns of live units: every key between is seen by all
+#pragma unroll
+        for (int x = 0; x < WIDE_UNITS; ++x) {
+            const size_t row = (size_t)cu_new[b] + min(first_query(x) + r, n_new - 1);
+            load_query(q + (row * nh + head_of(x)) * HD, true, g, qv[x]);
+            minus_m[x] = weights[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int dt = 0; dt < DTILES; ++dt) o[x][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int dt = 0; dt < DTILES; ++dt) asm volatile("" : "+a"(o[x][dt]));
+            asm volatile("" : "+a"(weights[x]));
+            fresh |= 1u << x;
+            if (live(x)) {
+                least_pos = min(least_pos, start + first_query(x));
+                last_first = max(last_first, first_key(start + min(first_query(x) + 15, n_new - 1)));
+            }
+        }
+        const int tile_last = min(tile_first + qb - 1, n_new - 1);
+        const int p_hi = (start + tile_last) / PAGE_TOKENS;
+        const int p_lo = first_key(start + tile_first) / PAGE_TOKENS;
+
+        const uint32_t k_at = lds_address(k_lds) + wave * 1024, v_at = lds_address(v_lds) + wave * 1024;
+        auto page_offset = [&](int page) { return ((size_t)page * nkv + kvh) * (PAGE_TOKENS * HD * sizeof(bf16_t)); };
+        // where the lane finds its fragments in a page: key tile t, k-step j; value tile dt, half h
+        int k_frag[KSTEPS], v_frag[2];
+#pragma unroll
+        for (int j = 0; j < KSTEPS; ++j) k_frag[j] = tile_key(0, r) * K_STRIDE + ((j * 4 + g) ^ k_swizzle(tile_key(0, r))) * 8;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) v_frag[h] = r * V_STRIDE + ((h * 4 + g) ^ v_swizzle(r)) * 8;
+        // (tiles of a half lie 4 rows apart and halves 32, value tiles 16: neither changes a row's permutation)
+        static_assert(K_STRIDE == HD, "rows of whole chunks");
+        bf16x8 kf[4][KSTEPS], vf[DTILES][2];
+        auto read_k = [&](int stage, int t, int j) __attribute__((always_inline)) {
+            kf[t][j] = *reinterpret_cast<const bf16x8*>(k_lds + stage * K_TILE + k_frag[j] + (tile_key(t, 0)) * K_STRIDE);
+        };
+        auto read_v = [&](int stage, int dt, int h) __attribute__((always_inline)) {
+            vf[dt][h] = *reinterpret_cast<const bf16x8*>(v_lds + stage * V_TILE + v_frag[h] + dt * 16 * V_STRIDE);
+        };
+
+        f32x4 s[2][2][4];                                             // scores of the two pairs
+        float top[2], e[4];
+        u32x4 pv[2][2][2];                                            // weights: [pair][unit][half]
+        bf16x8 ones;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+        f32x4 zeros = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+v"(ones), "+v"(zeros));                   // (kept: a product reads nothing that was written just before it)
+
+        auto score = [&](int pair, int n) __attribute__((always_inline)) {
+            const int j = n / 8, t = n % 8 / 2, x = n % 2;
+            if (j == 0) wide_score_first(s[pair][x][t], kf[t][j], qv[2 * pair + x][j], PRESCALED ? minus_m[2 * pair + x] : zeros);
+            else wide_score(s[pair][x][t], kf[t][j], qv[2 * pair + x][j]);
+        };
+        auto weigh = [&](int pair, int n) __attribute__((always_inline)) {
+            const int h = n / (PV / 2), m = n % (PV / 2), x = m % 2;
+            if (m / 2 < DTILES) wide_weigh(o[2 * pair + x][m / 2], vf[m / 2][h], pv[pair][x][h]);
+            else wide_weigh(weights[2 * pair + x], ones, pv[pair][x][h]);      // the sum of a column's weights: a row of ones
+        };
+        auto maximum = [&](int pair, int n) __attribute__((always_inline)) {         // n-th of eight parts
+            const int x = n % 2, t = n / 2;
+            f32x4 v = s[pair][x][t];
+            if (!PRESCALED) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = fmaf(v[i], scale_log2, minus_m[2 * pair + x][i]);
+                s[pair][x][t] = v;
+            }
+            top[x] = t == 0 ? wide_max(v[0], v[1], v[1]) : wide_max(top[x], v[0], v[1]);
+            top[x] = wide_max(top[x], v[2], v[3]);
+        };
+        // masks, moved references, rescaled outputs: off the usual path
+        auto settle = [&](int pair, int page_first_key, bool masked) __attribute__((always_inline)) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                const int u = 2 * pair + x;
+                if (masked) {
+                    int row = r, quad = 4 * g;                        // (made anew: kept for this rare path, what follows from them would cost the others registers)
+                    asm volatile("" : "+v"(row), "+v"(quad));
+                    const int pos = start + min(first_query(u) + row, n_new - 1);
+                    const int lo = first_key(pos) - page_first_key, hi = pos - page_first_key;
+                    top[x] = -INFINITY;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int key = tile_key(t, 0) + quad / 4 * 8 + i;
+                            s[pair][x][t][i] = (key >= lo && key <= hi) ? s[pair][x][t][i] : -INFINITY;
+                            top[x] = fmaxf(top[x], s[pair][x][t][i]);
+                        }
+                }
+                float most = top[x];                                  // of the column: its four lanes agree
+                most = fmaxf(most, __shfl_xor(most, 16, WAVE));
+                most = fmaxf(most, __shfl_xor(most, 32, WAVE));
+                const bool is_fresh = (fresh >> u) & 1u;              // no key yet: outputs and sums are still zero
+                const bool jump = most > PF_LAZY_LOG2 || (is_fresh && most > -INFINITY);
+                const float shift = jump ? most : 0.f;
+                const float alpha = jump && !is_fresh ? exp2_weight(-most) : 1.0f;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[pair][x][t][i] -= shift;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) minus_m[u][i] -= shift;
+                asm volatile("" : "+v"(minus_m[u]));                  // (whole again, so that no path to here takes it apart)
+                if (jump) fresh &= ~(1u << u);
+                if (__any(alpha != 1.0f)) {
+#pragma unroll
+                    for (int dt = 0; dt < DTILES; ++dt) {
+                        asm volatile("" : "+a"(o[u][dt]));            // (taken from its registers no sooner than here)
+                        o[u][dt] = o[u][dt] * alpha;
+                        asm volatile("" : "+a"(o[u][dt]));
+                    }
+                    asm volatile("" : "+a"(weights[u]));
+                    weights[u] = weights[u] * alpha;
+                    asm volatile("" : "+a"(weights[u]));
+                }
+            }
+        };
+        auto vote = [&](int pair, bool masked) __attribute__((always_inline)) {
+            return masked || __any(top[0] > PF_LAZY_LOG2 || top[1] > PF_LAZY_LOG2 || (fresh >> (2 * pair) & 3u) != 0u);
+        };
+        // i-th of the pair's 32 weights, first halves first; two are rounded together, one step behind.  (Each is made where it
+        // stands here: left to itself the compiler makes them all where the first of them is used.)
+        auto round_two = [&](int pair, int i) __attribute__((always_inline)) {       // weights i and i + 1
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            const bf16x2 two = {(__bf16)e[i % 4], (__bf16)e[i % 4 + 1]};
+            uint32_t bits = __builtin_bit_cast(uint32_t, two);
+            asm volatile("" : "+v"(bits));
+            pv[pair][i % 16 / 8][i / 16][i % 8 / 2] = bits;
+        };
+        auto weight = [&](int pair, int i) __attribute__((always_inline)) {
+            const int h = i / 16, x = i % 16 / 8, k = i % 8;
+            if (i >= 2 && i % 2 == 0) round_two(pair, i - 2);
+            if (i < 32) {
+                e[i % 4] = exp2_weight(s[pair][x][2 * h + k / 4][k % 4]);
+                asm volatile("" : "+v"(e[i % 4]));
+            }
+        };
+#define WIDE_FENCE __builtin_amdgcn_sched_barrier(0)
+#define WIDE_NOP asm volatile("s_nop 3")
+
+        wait_for_all_but_the_youngest_loads<0>();                     // the queries
+        // 64 entries of the page table, a lane each (read through the scalar unit, each would be waited for together with all reads of LDS)
+        int ids = pages[min(p_lo + lane, p_hi)];
+        auto load_k = [&](size_t page, int stage, int i) __attribute__((always_inline)) {
+            row_chunk_into_lds(reinterpret_cast<const char*>(k_cache) + page, sources.k[i], k_at + stage * (K_TILE * 2) + i * PF_WAVES * 1024);
+        };
+        auto load_v = [&](size_t page, int stage, int i) __attribute__((always_inline)) {
+            row_chunk_into_lds(reinterpret_cast<const char*>(v_cache) + page, sources.v[i], v_at + stage * (V_TILE * 2) + i * PF_WAVES * 1024);
+        };
+        size_t from = 0;                                              // the page whose keys were asked for last
+        auto page_bytes = [&](int p) { return page_offset(__builtin_amdgcn_readlane(ids, (p - p_lo) & 63)); };
+#pragma unroll
+        for (int ahead = 0; ahead < 3; ++ahead) {                     // (beyond the last page the last one again, for nobody: every page has its loads)
+            from = page_bytes(min(p_lo + ahead, p_hi));
+#pragma unroll
+            for (int i = 0; i < PF_LOADS; ++i) load_k(from, ahead, i);
+#pragma unroll
+            for (int i = 0; i < PF_LOADS; ++i)
+                if (ahead < 2) load_v(from, ahead, i);
+        }
+        wait_for_all_but_the_youngest_loads<3 * PF_LOADS>();
+        page_barrier();
+#pragma unroll
+        for (int i = 0; i < 14; ++i) read_k(0, i % 4, i / 4);
+        int stage = 0;
+        for (int p = p_lo; p <= p_hi; ++p) {
+            const int next = (stage + 1) % WIDE_STAGES, free_stage = (stage + 3) % WIDE_STAGES;
+            const int first = p * PAGE_TOKENS;
+            const bool masked = last_first > first || least_pos < first + PAGE_TOKENS - 1;
+            if (seq_tail - first < PAGE_TOKENS - 1) {                 // the sequence's last page: no page follows it
+                blank_values_after(v_lds + stage * V_TILE, seq_tail - first);
+                __syncthreads();
+            }
+            if (((p + 3 - p_lo) & 63) == 0) ids = pages[min(p + 3 + lane, p_hi)];
+            WIDE_FENCE;
+#pragma unroll
+            for (int n = 0; n < QK; ++n) {
+                score(0, n);
+                if (n == 1 || n == 5) read_k(stage, 2 + n / 4, 3);
+                if (n >= 8 && n % 3 == 2) read_v(stage, (n - 8) / 3, 0);
+                if (n % 4 == 3 && n < 16) load_v(from, (stage + 2) % WIDE_STAGES, n / 4);
+                if (n >= 28) maximum(0, n - 28);
+                WIDE_FENCE;
+            }
+            // the next page has landed when at most the one after it is on its way; behind the barrier no wave reads the page before this one
+            wait_for_all_but_the_youngest_loads<PAGE_LOADS>();
+            asm volatile("s_barrier" ::: "memory");
+            WIDE_FENCE;
+            bool unsettled = false;
+#pragma unroll
+            for (int n = 0; n < 7; ++n) {
+                score(1, n);
+                if (n < 4) maximum(0, 4 + n);
+                if (n == 4) unsettled = vote(0, masked);
+                if (n % 4 == 3) read_v(stage, n / 4, 1);
+                WIDE_FENCE;
+            }
+            if (unsettled) settle(0, first, masked);
+            WIDE_FENCE;
+#pragma unroll
+            for (int n = 7; n < QK; ++n) {
+                score(1, n);
+                weight(0, n - 7);
+                if (n % 4 == 3) read_v(stage, n / 4, 1);
+                WIDE_FENCE;
+            }
+            WIDE_NOP;
+            WIDE_FENCE;
+#pragma unroll
+            for (int n = 0; n < 18; ++n) {
+                weigh(0, n);
+                if (n < 8) weight(0, 25 + n);
+                if (n >= 7 && n < 15) maximum(1, n - 7);
+                if (n == 15) unsettled = vote(1, masked);
+                if (n == 17) read_k(next, 0, 0);
+                WIDE_FENCE;
+            }
+            if (unsettled) settle(1, first, masked);
+            WIDE_FENCE;
+#pragma unroll
+            for (int n = 18; n < PV; ++n) {
+                weigh(0, n);
+                weight(1, n - 18);
+                if (n % 4 == 1) read_k(next, (n - 17) / 4 % 4, (n - 17) / 4 / 4);
+                WIDE_FENCE;
+            }
+#pragma unroll
+            for (int n = 0; n < PV; ++n) {
+                weigh(1, n);
+                if (n < 15) weight(1, 18 + n);
+                if (n % 4 == 1) read_k(next, (n / 4 + 5) % 4, (n / 4 + 5) / 4);
+                if (n == 15) from = page_bytes(min(p + 3, p_hi));
+                if (n >= 16 && n < 32 && n % 4 == 0) {
+                    load_k(from, free_stage, (n - 16) / 4);
+                }
+                WIDE_FENCE;
+            }
+            stage = next;
+        }
+        wait_for_all_but_the_youngest_loads<0>();                     // nothing may land in LDS after the block's end
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        WIDE_FENCE;
+#undef WIDE_FENCE
+#undef WIDE_NOP
+#pragma unroll
+        for (int x = 0; x < WIDE_UNITS; ++x) {
+            const int qi = first_query(x) + r;
+            if (live(x) && qi < n_new) {
+                const float inv = 1.0f / weights[x][0];
+                bf16_t* to = out + (((size_t)cu_new[b] + qi) * nh + head_of(x)) * HD;
+#pragma unroll
+                for (int dt = 0; dt < DTILES; ++dt) {           // the lane's four elements of a tile lie side by side: one store
+                    uint2 four;
+                    four.x = (uint32_t)f32_to_bf16(o[x][dt][0] * inv).bits | ((uint32_t)f32_to_bf16(o[x][dt][1] * inv).bits << 16);
+                    four.y = (uint32_t)f32_to_bf16(o[x][dt][2] * inv).bits | ((uint32_t)f32_to_bf16(o[x][dt][3] * inv).bits << 16);
+                    *reinterpret_cast<uint2*>(to + dt * 16 + 4 * g) = four;
+                }
+            }
+        }
+    }
+}
+
 // q_prescaled: the queries come multiplied by scale * log2(e) already (by the pass that rounds them), so a score is
 // the exponent of its weight as it leaves the matrix cores; `scale` is then not applied again.
 PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
@@ -1547,3 +1890,29 @@ PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const voi
 }
 
 PALM_API int palm_attention_prefill_takes_prescaled() { return PF_DMA ? 1 : 0; }
+
+// The same by the kernel for long prompts, where palm_attention_prefill_wide_serves() says so.
+PALM_API int palm_attention_prefill_wide(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
+                                         const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
+                                         const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
+                                         int hd, float scale, int window, int q_prescaled, void* out) {
+    PALM_CHECK(PF_WIDE && hd == HD, "attention_prefill_wide: not for head size %d (this library's is %d)", hd, HD);
+    PALM_CHECK(n_seqs >= 0 && max_new >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0,
+               "attention_prefill_wide: seqs=%d max_new=%d heads=%d kv=%d", n_seqs, max_new, nh, nkv);
+    PALM_CHECK(window >= 0 && max_pages > 0, "attention_prefill_wide: window=%d max_pages=%d", window, max_pages);
+    if (n_seqs == 0 || max_new == 0) return 0;
+    constexpr int UNITS = WIDE_UNITS * PF_WAVES;
+    const int G = nh / nkv, hg = min(G, UNITS), qb = 16 * (UNITS / hg), n_hg = (G + hg - 1) / hg;
+    PALM_CHECK(nkv * n_hg <= 65535 && n_seqs <= 65535 && (max_new + qb - 1) / qb <= 65535, "attention_prefill_wide: grid too large");
+    const dim3 grid(nkv * n_hg, (max_new + qb - 1) / qb, n_seqs);       // (the kv head fastest: see palm_attention_prefill)
+    const float scale_log2 = q_prescaled ? 1.0f : scale * LOG2E;
+#define PALM_WIDE(PRE) attention_prefill_wide_kernel<PRE><<<grid, PF_THREADS, 0, stream>>>( \
+        (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, max_pages, seq_slot, seq_start, seq_new, \
+        cu_new, nh, nkv, scale_log2, window, qb, hg, (bf16_t*)out)
+    if (q_prescaled) PALM_WIDE(true); else PALM_WIDE(false);
+#undef PALM_WIDE
+    PALM_LAUNCHED();
+    return 0;
+}
+PALM_API int palm_attention_prefill_wide_serves() { return PF_WIDE ? 1 : 0; }
+

@@ -785,6 +785,9 @@ _ATTENTION_SIGNATURES = {
     "palm_attention_prefill": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p],
     "palm_attention_prefill_takes_prescaled": [],
+    "palm_attention_prefill_wide": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                    c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p],
+    "palm_attention_prefill_wide_serves": [],
     "palm_attention_decode_fused": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
                                     c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int,
                                     c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p],
@@ -933,18 +936,44 @@ def prefill_q_scale(hd: int, dtype, scale: float) -> float:
 
 
 def attention_prefill(q, k_cache, v_cache, block_table, seq_slot, seq_start, seq_new, cu_new, max_new: int, nh: int,
-                      nkv: int, hd: int, scale: float, window: int | None, q_prescaled: bool = False) -> torch.Tensor:
+                      nkv: int, hd: int, scale: float, window: int | None, q_prescaled: bool = False, wide: bool = False) -> torch.Tensor:
     """The step's queries (several for each sequence) over the cache, on the matrix cores.  ``q_prescaled``: the
-    queries come multiplied by ``prefill_q_scale`` already, and ``scale`` is not applied again."""
+    queries come multiplied by ``prefill_q_scale`` already, and ``scale`` is not applied again.  ``wide``: by the kernel for long
+    prompts (head size 128), see ``wide_prompt_attention``."""
     _attention_checks("attention_prefill", q, k_cache, v_cache, block_table, nh, nkv, hd, seq_slot, seq_start, seq_new, cu_new)
     B = seq_slot.shape[0]
     _need(seq_start.shape == (B,) and seq_new.shape == (B,) and cu_new.shape == (B + 1,),
           "attention_prefill: per-sequence arrays differ in length")
     out = torch.empty_like(q)
-    library.call(attention_lib(hd), "palm_attention_prefill", _stream(), _p(q), _p(k_cache), _p(v_cache), _p(block_table),
+    library.call(attention_lib(hd), "palm_attention_prefill_wide" if wide else "palm_attention_prefill", _stream(), _p(q), _p(k_cache), _p(v_cache), _p(block_table),
                  block_table.shape[1], _p(seq_slot), _p(seq_start), _p(seq_new), _p(cu_new), B, int(max_new), nh, nkv, hd,
                  float(scale), int(window or 0), int(bool(q_prescaled)), _p(out))
     return out
+
+
+def wide_prompt_attention(starts, counts, nh: int, nkv: int) -> bool:
+    """Whether a step's prompts (``counts`` new tokens behind ``starts`` earlier ones) are sooner through the kernel whose waves hold 64
+    columns.  Both kernels' times in microseconds from the pages that their blocks walk over: the wide one has a block of 16 units (one
+    head's 16 queries) a compute unit, some 9 us of start and end that nothing hides, and 1.6 us a page with all units at work; the other two blocks
+    of eight units, 2 us a page each.  Measured (32 heads of 8 unless said otherwise; the other's time and this one's): 2,048 tokens 51 58,
+    3,072 82 82, 3,500 106 97, 4,096 142 125, 13,331 1,281 1,134, four of 2,048 151 156, four of 3,072 318 312, 64 behind 1,000 34 38, behind 2,000 58 58, 1,000
+    behind 3,000 112 102; 40 heads of 8 (five of eight units used, fifteen of sixteen) 1,024 tokens 31 38, 2,048 87 67, 8,192 939 590, five of 45 to 2,000 125 106;
+    64 heads of 8 3,072 150 157, 4,096 253 241; 16 heads of 8 4,096 92 102, 8,192 266 224.  The numbers below are fitted to 64 such steps: the slower one is taken at four of
+    them (16 heads of 8 at 4,096 tokens by 11 %, 8 of 8 at 8,192 by 8 %, two by less than 3 %)."""
+    G = nh // nkv
+
+    def tiles_and_pages(units):
+        heads = min(G, units)
+        rows, groups = 16 * (units // heads), nkv * -(-G // heads)
+        tiles = [-(-n // rows) for n in counts]
+        # the mean tile of a sequence ends half way through its new tokens, in the middle of a page
+        return groups * sum(tiles), groups * sum(t * ((s + (n + rows) / 2) / PAGE_TOKENS + 0.5) for t, s, n in zip(tiles, starts, counts))
+    longest = max((s + n + PAGE_TOKENS - 1) // PAGE_TOKENS for s, n in zip(starts, counts))
+    blocks, pages = tiles_and_pages(16)
+    wide_us = 9.2 + max(5 + 1.35 * longest, (9.6 * blocks + 1.61 * pages) / COMPUTE_UNITS)
+    blocks, pages = tiles_and_pages(8)
+    other_us = 6.8 + max(1.57 * longest, (2.2 * blocks + 1.95 * pages) / (2 * COMPUTE_UNITS))
+    return wide_us < other_us
 
 
 def slices_of_step(ctx, nh: int, nkv: int, window: int | None) -> int:
@@ -957,17 +986,25 @@ def attention(q, k_cache, v_cache, block_table, ctx, nh: int, nkv: int, hd: int,
               q_prescaled: bool = False):
     """The step's queries over the cache; picks the kernel by element type, head size and step shape.
     ``q_prescaled``: see ``attention_prefill`` (only a prompt step on the matrix cores takes such queries)."""
+    def wide():
+        if window or not ctx.host or not attention_lib(hd).palm_attention_prefill_wide_serves():
+            return False
+        key = ("wide_prompt_attention", nh, nkv)
+        if key not in ctx.memo:
+            ctx.memo[key] = wide_prompt_attention(ctx.host["starts"], ctx.host["counts"], nh, nkv)
+        return ctx.memo[key]
+
     if q_prescaled:
         _need(mfma_attention_serves(q, hd) and not ctx.is_decode, "attention: only the prompt kernel takes scaled queries")
         return attention_prefill(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new,
-                                 ctx.max_new, nh, nkv, hd, scale, window, q_prescaled=True)
+                                 ctx.max_new, nh, nkv, hd, scale, window, q_prescaled=True, wide=wide())
     if mfma_attention_serves(q, hd):
         if ctx.is_decode:
             n_slices = slices_of_step(ctx, nh, nkv, window)
             return attention_decode(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, nh, nkv, hd, scale,
                                     window, n_slices)
         return attention_prefill(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new,
-                                 ctx.max_new, nh, nkv, hd, scale, window)
+                                 ctx.max_new, nh, nkv, hd, scale, window, wide=wide())
     return attention_exact(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new,
                            ctx.max_new, nh, nkv, hd, scale, window)
 

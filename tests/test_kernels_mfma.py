@@ -582,6 +582,31 @@ def test_attention_prefill_with_the_scale_folded_into_the_queries(ops, nh, nkv, 
             q, kc, vc, table, slots, starts, news, cu, max_new, 6, 1, 80, scale, window, q_prescaled=True), BF16, 6, 1, 80, [(20, 20)], None)
 
 
+@pytest.mark.parametrize("nh,nkv", [(32, 8), (5, 1), (3, 3), (16, 1), (18, 1), (16, 2)])
+@pytest.mark.parametrize("prescaled", [True, False])
+def test_attention_prefill_wide(ops, nh, nkv, prescaled):
+    """The kernel whose waves hold 64 columns: tiles that are full, cut and of one query, pages before the prompt, windows below, at and
+    above a page, more than 64 pages of the table, maxima that rise late, pages that hold what earlier owners left."""
+    def wide(q, kc, vc, table, slots, starts, news, cu, max_new, nh_, nkv_, hd, scale, window):
+        qs = (q.float() * ops.prefill_q_scale(hd, BF16, scale)).to(BF16) if prescaled else q
+        return ops.attention_prefill(qs, kc, vc, table, slots, starts, news, cu, max_new, nh, nkv, hd, scale, window, q_prescaled=prescaled, wide=True)
+    for window in (None, 1, 64, 100):
+        for lens in ([(1, 1)], [(64, 64)], [(129, 129)], [(300, 44)], [(64, 64), (65, 1), (130, 70), (7, 7), (200, 17)], [(1100, 1100)], [(4300, 300), (70, 70)]):
+            got, ref = _attention_case(ops, wide, BF16, nh, nkv, 128, lens, window, seed=len(lens) + nh, poison=True)
+            # (queries and weights rounded to 8 bits, 2^-9 of outputs of unit scale, each twice: as for the kernel above)
+            assert torch.isfinite(got).all() and torch.allclose(got, ref, atol=3e-2), (lens, window, float((got - ref).abs().max()))
+
+
+def test_wide_prompt_attention_is_taken_for_long_prompts(ops):
+    from palm_infra_amd.kernels import KernelError
+    assert ops.wide_prompt_attention([0], [13331], 32, 8) and ops.wide_prompt_attention([30720], [2048], 32, 8)
+    assert not ops.wide_prompt_attention([0], [2048], 32, 8) and not ops.wide_prompt_attention([0], [91], 32, 8)
+    assert ops.wide_prompt_attention([0], [2048], 40, 8) and not ops.wide_prompt_attention([0] * 64, [20] * 64, 40, 8)
+    with pytest.raises(KernelError, match="not for head size 64"):
+        _attention_case(ops, lambda q, kc, vc, table, slots, starts, news, cu, max_new, a, b, c, scale, window: ops.attention_prefill(
+            q, kc, vc, table, slots, starts, news, cu, max_new, 4, 2, 64, scale, window, wide=True), BF16, 4, 2, 64, [(20, 20)], None)
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (4, 2, 64), (6, 1, 80)])
 def test_attention_mfma_long_sequences(ops, nh, nkv, hd):
     """The measured lengths and beyond: a 2,048-token prompt (32 pages, query tiles paired from both ends, a
