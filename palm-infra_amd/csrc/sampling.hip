@@ -780,9 +780,9 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
 // there is room for (many equal logits, as of a row with most of its vocabulary masked) the slice or the row is cut once more by key
 // and index together, lower indices first: no two elements are equal then.  A row that still does not go this way, or has a NaN in
 // it, is done by sample_row.  (33 rows of 151,936 logits of which all but some 40 are masked: 767 us when sample_row did them, now 67.)
-// Measured with k = 50 and 151,936 logits, 33 rows, both kernels in a recorded run: 17 us (25 with a count of larger keys for every
-// key; 117 as one block a row).  What is left is latency: two launches, 6.6 us for the slices, and in the second, 10.7 us, a chain of two
-// trips to memory, three barriers and the k dependent additions.
+// Measured with k = 50 and 151,936 logits, 33 rows, both kernels in a recorded run: 15.4 us (25 with a count of larger keys for every
+// key; 117 as one block a row).  What is left is latency: two launches, 7 us for the slices, and in the second, 9.4 us (10.7 with the k
+// additions by handing weights around), a chain of two trips to memory, three barriers and the k dependent additions.
 constexpr int SLICE_THREADS = 256;
 constexpr int SLICE_QUADS = 4;                                       // 16-byte pieces of a slice that a thread holds
 constexpr int SLICE = SLICE_THREADS * SLICE_QUADS * 4;
@@ -907,7 +907,8 @@ __global__ __launch_bounds__(SLICE_THREADS) void topk_slice_kernel(const float* 
 struct DrawShared {
     __attribute__((aligned(16))) uint32_t top[256];
     unsigned long long line;
-    int n, bad, zeros;
+    int n, zeros;
+    bool bad[SAMPLE_WAVES];
     unsigned long long most[SAMPLE_THREADS];
     uint2 survivor[SURVIVORS];
     float v[SLICED_TOPK_MAX];
@@ -929,9 +930,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
     const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     counts += (size_t)blockIdx.x * slices;
     cands += (size_t)blockIdx.x * slices * SLICE_CAP;
-    if (tid == 0) { sh.n = 0; sh.bad = 0; sh.zeros = 0; }
+    if (tid == 0) { sh.n = 0; sh.zeros = 0; }
     const float u = uniform_of(uniforms);
-    __syncthreads();
     // the counts of the first slices a wave takes and the first places a lane takes are asked for together and kept (a place
     // beyond its slice's count holds nothing, and nothing is made of it)
     constexpr int HELD = 3, ROUNDS = 2;
@@ -951,10 +951,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
         for (int r = 0; r < ROUNDS; ++r)
             if (lane + r * WAVE >= held_n[h]) held[h][r] = make_uint2(0u, 0u);
     }
+    bool refused = false;                                            // a slice that does not go this way (the same in every lane)
     // f(key, index) for the others: few, or a vocabulary of more than HELD x SAMPLE_WAVES slices
     auto rest = [&](auto&& f) {
         auto slice = [&](int s, int c, int first) {
-            if (c < 0) sh.bad = 1;
+            refused |= c < 0;
             for (int j = first; j < c; j += WAVE) f(cands[(size_t)s * SLICE_CAP + j]);
         };
 #pragma unroll
@@ -970,7 +971,9 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
     best = max(best, (uint32_t)__shfl_xor((int)best, 1, WAVE));
     best = max(best, (uint32_t)__shfl_xor((int)best, 2, WAVE));
     if (tid % 4 == 0) sh.top[tid / 4] = best;
+    if (lane == 0) sh.bad[wave] = refused;
     __syncthreads();
+    const bool bad = __ballot(sh.bad[lane % SAMPLE_WAVES]) != 0ull;
     // every wave finds the cut for itself: the k-th largest of the groups' maxima
     const uint4 four = reinterpret_cast<const uint4*>(sh.top)[lane];
     const uint32_t tops[4] = {four.x, four.y, four.z, four.w};
@@ -1002,7 +1005,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
     rest(survives);
     __syncthreads();
     int n = sh.n;
-    if (n > SURVIVORS && !sh.bad) {
+    if (n > SURVIVORS && !bad) {
         auto each = [&](auto&& f) {
             auto real = [&](uint2 one) { if (one.x) f(one); };
 #pragma unroll
@@ -1031,7 +1034,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
         __syncthreads();
         n = sh.n;
     }
-    if (sh.bad || n > SURVIVORS || n < k) {                          // (n < k: fewer than k elements in the row; not with k < V)
+    if (bad || n > SURVIVORS || n < k) {                          // (n < k: fewer than k elements in the row; not with k < V)
         __syncthreads();
         sample_row(logits + (size_t)blockIdx.x * V, V, u, temperature, k, top_p, min_p, out + blockIdx.x, nullptr, shared.row);
         return;
@@ -1070,17 +1073,19 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void topk_draw_kernel(
     // sample_row's walk.  Its three sums are prefixes of one, added up in the same order: a place each, lane l of this wave
     // holds the weights and the prefix sums l and 64 + l.
     const float l_max = sh.v[0], inv_t = 1.0f / temperature;
+    // (Lane l's sum is lane l - 1's plus its own weight; taken so of all lanes at once, lane l has its sum after l steps and keeps it.
+    // Handing every weight to all lanes in turn took four instructions a place.)
     float w[2], sum_to[2];
-    float run = 0.f;
+    float before = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         w[h] = lane + h * WAVE < k ? expf((sh.v[min(lane + h * WAVE, k - 1)] - l_max) * inv_t) : 0.f;
-        sum_to[h] = 0.f;
-#pragma unroll 8
-        for (int i = 0; i < min(k - h * WAVE, WAVE); ++i) {
-            run += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[h]), i));
-            if (lane == i) sum_to[h] = run;
-        }
+        const float own = lane == 0 ? before + w[h] : w[h];          // (0 + w is w)
+        float run = own;
+        for (int i = 1; i < min(k - h * WAVE, WAVE); ++i)
+            run = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(run), 0x138, 0xf, 0xf, true)) + own;          // wave_shr:1, 0 into lane 0
+        sum_to[h] = run;
+        before = __shfl(run, WAVE - 1, WAVE);
     }
     // the first of the `active` places for which the flag is set, `otherwise` if there is none
     auto first_place = [&](auto&& flag, int active, int otherwise) {

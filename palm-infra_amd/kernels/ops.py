@@ -404,21 +404,28 @@ def sample(logits: torch.Tensor, uniforms: torch.Tensor | None, temperature: flo
     return (out, probs) if want_probs else out
 
 
+@functools.lru_cache(maxsize=256)
+def _sliced_work(n: int, V: int, draws: bool, top_k: int) -> int:
+    """Bytes of workspace for rows that go in slices; 0: they do not."""
+    return core().palm_sample_sliced_work(n, V, 1.0 if draws else 0.0, top_k)
+
+
 def sample_drawn(logits: torch.Tensor, seed: int, streams, draws, temperature: float, top_k: int = 0, top_p: float = 0.0,
                  min_p: float = 0.0) -> torch.Tensor:
     """``sample`` with the uniform numbers of (seed, streams[i], draws[i]).  Where the rows go in slices the numbers reach the kernel
     with its arguments; else through pinned memory, so that the host does not wait for the device."""
     n = logits.shape[0]
-    if logits.is_cuda and logits.dim() == 2 and logits.dtype == F32 and logits.is_contiguous() and logits.data_ptr() % 16 == 0:
-        V = logits.shape[1]
-        needed = core().palm_sample_sliced_work(n, V, temperature, top_k)
+    if logits.is_cuda and logits.dim() == 2 and logits.dtype == F32 and logits.is_contiguous():
+        V, at = logits.shape[1], logits.data_ptr()
+        needed = _sliced_work(n, V, temperature > 0.0, top_k) if at % 16 == 0 else 0
         if needed:
             s, d = _u64(streams), _u64(draws)
             _need(len(s) == n and len(d) == n, "sample: a stream and a draw's number for each row")
-            out = torch.empty((n,), dtype=torch.int32, device=logits.device)
-            work = torch.empty((needed,), dtype=torch.uint8, device=logits.device)
-            library.call(core(), "palm_sample_sliced_drawn", _stream(), logits.data_ptr(), n, V, int(seed) & _U64, s.buffer_info()[0],
-                         d.buffer_info()[0], temperature, top_k, top_p, min_p, out.data_ptr(), work.data_ptr(), needed)
+            device = logits.device
+            out = torch.empty((n,), dtype=torch.int32, device=device)
+            work = torch.empty((needed,), dtype=torch.uint8, device=device)
+            library.call(core(), "palm_sample_sliced_drawn", _stream(), at, n, V, int(seed) & _U64, s.buffer_info()[0], d.buffer_info()[0],
+                         temperature, top_k, top_p, min_p, out.data_ptr(), work.data_ptr(), needed)
             return out
     u = torch.empty((n,), dtype=F32, pin_memory=True)
     uniforms_into(u, seed, streams, draws)

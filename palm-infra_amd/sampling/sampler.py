@@ -13,6 +13,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from ..kernels import ops
 from .params import SamplingParams
 
 _MASK = (1 << 64) - 1
@@ -75,7 +76,6 @@ class DeviceSampler:
         return bool(self.params.penalties_enabled)
 
     def sample(self, logits: torch.Tensor, states) -> torch.Tensor:
-        from ..kernels import ops
         p = self.params
         if len(states) != logits.shape[0]:
             raise ValueError(f"{logits.shape[0]} rows of logits for {len(states)} sequences")
@@ -101,7 +101,6 @@ class DeviceSampler:
     def probabilities(self, logits: torch.Tensor, states) -> torch.Tensor:
         """The distribution a draw would come from, [B, vocab]; changes no state
         (engine/sampler.cpp:352-395)."""
-        from ..kernels import ops
         p = self.params
         V = logits.shape[1]
         if p.penalties_enabled:
