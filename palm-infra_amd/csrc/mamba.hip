@@ -140,21 +140,23 @@ PALM_API int palm_causal_conv(hipStream_t stream, const void* x, int dtype, int 
 }
 
 // ---- the scan ---------------------------------------------------------------------------------------
-// A channel's row of S is spread over a group of G lanes (G a power of two, at most 64, chosen from the state
-// size): lane j of the group holds states j, j + G, ..; a block of four waves serves 256 / G channels.  The block
-// walks over a sequence's new tokens a tile at a time, in three phases with a barrier between them:
+// A channel's row of S is spread over a group of G lanes (G a power of two, at most 64): lane j of the group holds the PER states
+// from j PER on; a block of four waves serves 256 / G channels.  The block walks over a sequence's new tokens a tile at a time,
+// in three phases with a barrier between them:
 //   in     all threads bring the tile's inputs into LDS with reads that follow the memory's rows: B_t and C_t (the
-//          same for all channels), and for the block's channels u_t and the step size softplus(dtl_t + bias),
-//          computed once for each (token, channel)
-//   scan   for every token a lane updates its states from LDS and the group adds up its part of y with shuffles;
-//          nothing but the multiply-add on S waits for the token before it, so the exponentials of a tile overlap
+//          same for all channels), and for the block's channels the step size softplus(dtl_t + bias) and its product
+//          with u_t, computed once for each (token, channel)
+//   scan   for every token a lane updates its states from LDS; nothing but the multiply-add on S waits for the token
+//          before it.  A whole tile's sums over the groups are made together (group_sums), without a branch between tokens
 //   out    all threads add the skip term, gate with silu(z_t) and store the tile's outputs row by row
-// Up to 16 states the next tile's inputs are asked for before the scan and wait in registers (with more states a thread has more of
-// them to hold, and fewer blocks fit: 64 states, many sequences, 10 to 20 % slower).  A part tile goes token by token: unrolled, it
-// costs the registers of another wave a SIMD.  What bounds it is the vector unit (some 30 instructions a token and state) and, once
-// the short sequences are done, the chain of tiles.  8,192 channels x 16 states, us, before (each tile's inputs waited for, the
-// library's exponential, three barriers a tile) and now: 2,603 tokens 580 and 415, 717 + 572 + 1,314 405 and 335, 8 x 300 264 and
-// 235, one token each of 64 sequences 51 and 41.
+// Up to 64 states the next tile's inputs are asked for before the scan and wait in registers (with more a thread has more of
+// them to hold, and fewer blocks fit).  A part tile goes token by token: unrolled, it costs the registers of another wave a SIMD.
+// What bounds it is the vector unit (11 instructions a token and state, beside those of a token) and, once the short sequences are
+// done, the chain of tiles.  8,192 channels x 16 states, us, with sums and a branch a token, one state a lane and the library's softplus
+// and silu, and now: 2,603 tokens 417 and 253, 717 + 572 + 1,314 330 and 218, 8 x 300 245 and 135, one token each of 64 sequences 38.6
+// and 32.6; 2,048 channels x 64 states, 717 + 572 + 1,314, 437 and 203.  (A token's operands read from LDS four tokens ahead: a chain of
+// 2,603 233 and 202, but 64 single tokens 32.6 and 37.5, 128 states 438 and 539; outputs stored a tile later, so that the wait for
+// the next inputs is none for stores: 3 % slower.)
 constexpr int SCAN_TILE = 16;
 
 // Sum over groups of G consecutive lanes (G a power of two), every lane gets its group's sum.  Within a row of 16
@@ -173,24 +175,85 @@ template <int G> __device__ inline float group_sum(float y) {
     if constexpr (G >= 64) y += __shfl_xor(y, 32, WAVE);
     return y;
 }
+// The sums over a group's lanes of TG values at once, TG the group's size or 16 of it: lane j (j + 16, ..) gets the sum of y[j].  A step
+// halves the values, each lane keeping those of its half and handing on the others': 15 additions and 30 selections for 16 values and
+// lanes, where one after the other they take 64 additions and a write of one lane each, with a branch around it.  The
+// widest step comes first, so that mirrored partners hold the same values.
+template <int H> __device__ inline void fold_half(float* y, int j) {
+    constexpr int CTRL = H == 8 ? 0x140 : H == 4 ? 0x141 : H == 2 ? 0x4E : 0xB1;
+    const bool upper = j & H;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+        const float keep = upper ? y[i + H] : y[i], give = upper ? y[i] : y[i + H];
+        y[i] = keep + dpp_move<CTRL>(give);
+    }
+}
+template <int G> __device__ inline float group_sums(float* y, int j) {
+    if constexpr (G >= 16) fold_half<8>(y, j);
+    if constexpr (G >= 8) fold_half<4>(y, j);
+    fold_half<2>(y, j);
+    fold_half<1>(y, j);
+    float sum = y[0];
+    if constexpr (G >= 32) sum += __shfl_xor(sum, 16, WAVE);
+    if constexpr (G >= 64) sum += __shfl_xor(sum, 32, WAVE);
+    return sum;
+}
 // exp(dt A) for an A that stays: 2^(dt A log2 e) with the product's rounding and that of A log2 e made up for in first order, so that
 // the error is the exponential unit's own and not that of a rounded argument.  Below 2^-150: 0, as any 32-bit exponential.
 struct ScanDecay {
     float hi, lo;                                       // A log2 e and, times ln 2, what hi leaves of it
+    float most;                                         // the step from which on nothing is left
     __device__ static ScanDecay of(float a) {
         constexpr float LOG2E = 1.44269504f, LOG2E_REST = 1.92596299e-8f, LN2 = 0.693147181f;
         if (a < -2e38f) a = -2e38f;                     // (hi stays finite; no number stays none)
         ScanDecay d;
         d.hi = a * LOG2E;
         d.lo = (fmaf(a, LOG2E, -d.hi) + a * LOG2E_REST) * LN2;
+        d.most = a < 0.f ? -150.f / d.hi : __builtin_inff();
         return d;
     }
     __device__ float over(float dt) const {
         constexpr float LN2 = 0.693147181f;
+        dt = fminf(dt, most);
         const float p = dt * hi, rest = fmaf(fmaf(dt, hi, -p), LN2, dt * lo), e = __builtin_amdgcn_exp2f(p);
-        return p < -150.f ? 0.f : fmaf(e, rest, e);
+        return fmaf(e, rest, e);
     }
 };
+// What a (token, channel) of the scan needs once, its softplus and its silu: 119 and 33 instructions of the library's, where a token's
+// sixteen states take some 200 between them.  Arguments for which a step leaves the normal numbers, and what is no number, go to the
+// library (behind a branch: the compiler would go both ways).
+__device__ inline float scan_exp(float x) {             // |x| < 87: 2^f of the fraction, the whole powers exact
+    constexpr float LOG2E = 1.44269504f, LOG2E_REST = 1.92596299e-8f;
+    const float n = rintf(x * LOG2E);
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(x, LOG2E_REST, fmaf(x, LOG2E, -n))), (int)n);
+}
+// log(1 + e^z) = max(z, 0) + log(1 + e), e = e^-|z|, and log(1 + e) = 2 artanh(s) with s = e / (2 + e), where 2 s = e - e s: what is
+// rounded in s is small beside e.  s^2 <= 1/9: the series' terms from the ninth on are below 2^-29.
+__device__ inline float scan_softplus(float z) {
+    if (!(fabsf(z) < 87.f)) {
+        asm volatile("" : "+v"(z));
+        return softplus_dt(z);
+    }
+    const float e = scan_exp(-fabsf(z)), d = 2.f + e, d_rest = e - (d - 2.f), r = __builtin_amdgcn_rcpf(d), q = e * r;
+    const float s = fmaf(fmaf(-d_rest, q, fmaf(-d, q, e)), r, q), t = s * s;
+    float sum = 2.f / 17;
+    sum = fmaf(sum, t, 2.f / 15);
+    sum = fmaf(sum, t, 2.f / 13);
+    sum = fmaf(sum, t, 2.f / 11);
+    sum = fmaf(sum, t, 2.f / 9);
+    sum = fmaf(sum, t, 2.f / 7);
+    sum = fmaf(sum, t, 2.f / 5);
+    sum = fmaf(sum, t, 2.f / 3);
+    return fmaxf(z, 0.f) + fmaf(s, fmaf(t, sum, -e), e);
+}
+__device__ inline float scan_silu(float z) {
+    if (!(fabsf(z) < 87.f)) {
+        asm volatile("" : "+v"(z));
+        return silu_f(z);
+    }
+    const float d = 1.f + scan_exp(-z), r = __builtin_amdgcn_rcpf(d), q = z * r;
+    return fmaf(fmaf(-d, q, z), r, q);
+}
 constexpr int SCAN_WAVES = 4;
 constexpr int SCAN_THREADS = SCAN_WAVES * WAVE;
 
@@ -200,7 +263,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     const float* __restrict__ dtl, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
     const float* __restrict__ d_skip, float* __restrict__ state, const int* __restrict__ seq_slot,
     const int* __restrict__ seq_new, const int* __restrict__ cu_new, int channels, int n_state, T* __restrict__ out) {
-    constexpr bool AHEAD = G <= 16;
+    constexpr bool AHEAD = G * PER <= 64;
     constexpr int CH = SCAN_THREADS / G;               // channels of a block
     constexpr int NP = G * PER;                        // the state size, padded
     constexpr int NB = (SCAN_TILE * NP + SCAN_THREADS - 1) / SCAN_THREADS, NC = (SCAN_TILE * CH + SCAN_THREADS - 1) / SCAN_THREADS;
@@ -208,10 +271,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     // SIMD; 2,048 channels, 717 + 572 + 1,314 tokens 694 us, in halves 617; one token each of 64 sequences 84 and 65).  (256 states:
     // LDS sets the number of blocks; in quarters 1,139 us, 981 all together.)  A tile of few tokens does not go through the rest: 64
     // sequences of one token, with it and without, 128 states 64 us and 59, 256 states, a token an element, 143 and 122.
-    constexpr int HELD = PER == 2 ? 4 : NB;
+    constexpr int HELD = NP == 128 ? 4 : NB;
     constexpr bool BY_TOKEN = NP == SCAN_THREADS;      // element first + i of every thread is of token first + i
-    __shared__ float b_s[SCAN_TILE][NP], c_s[SCAN_TILE][NP];
-    __shared__ float dt_s[SCAN_TILE][CH], u_s[SCAN_TILE][CH], y_s[SCAN_TILE][CH];
+    constexpr int TG = G < 16 ? G : 16;                // tokens whose sums are made at once
+    __shared__ __attribute__((aligned(16))) float2 bc_s[SCAN_TILE][NP];        // B_t and C_t
+    __shared__ float2 in_s[SCAN_TILE][CH];             // the step size, and times u_t
+    __shared__ float y_s[SCAN_TILE][CH];
     const int j = threadIdx.x % G, ch = threadIdx.x / G;
     const int c0 = blockIdx.x * CH, b = blockIdx.y;
     const int c = c0 + ch;
@@ -224,7 +289,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     ScanDecay A[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        const int n = j + k * G;
+        const int n = j * PER + k;
         S[k] = n < n_state ? sp[n] : 0.f;
         A[k] = ScanDecay::of(n < n_state ? -expf(a_log[(size_t)cc * n_state + n]) : 0.f);
     }
@@ -256,7 +321,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
         for (int i = 0; i < HELD; ++i) {
             const int idx = threadIdx.x + (first + i) * SCAN_THREADS;
             if (BY_TOKEN && first + i >= tt) break;
-            if (idx / NP < tt) { b_s[idx / NP][idx % NP] = to_float(b_r[i]); c_s[idx / NP][idx % NP] = to_float(c_r[i]); }
+            if (idx / NP < tt) bc_s[idx / NP][idx % NP] = make_float2(to_float(b_r[i]), to_float(c_r[i]));
         }
     };
     // (where a tile has fewer elements than the block threads, the threads beyond it read the next tiles': nearer when their turn
@@ -287,31 +352,42 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
             const int idx = threadIdx.x + i * SCAN_THREADS;
-            if (idx / CH < tt) { dt_s[idx / CH][idx % CH] = softplus_dt(dt_r[i] + bias[i]); u_s[idx / CH][idx % CH] = to_float(u_r[i]); }
+            if (idx / CH < tt) {
+                const float dt = scan_softplus(dt_r[i] + bias[i]);
+                in_s[idx / CH][idx % CH] = make_float2(dt, dt * to_float(u_r[i]));
+            }
             u_t[i] = to_float(u_r[i]);
             z_t[i] = to_float(z_r[i]);
         }
         __syncthreads();
         if (AHEAD && t0 + SCAN_TILE < n_new) { ask_states(t0 + SCAN_TILE, 0); ask_channels(t0 + SCAN_TILE); }        // on their way while this tile is scanned
-#define SCAN_TOKEN(ti) { \
-            const float dt = dt_s[ti][ch]; \
-            const float du = dt * u_s[ti][ch]; \
-            float y = 0.f; \
-            _Pragma("unroll") for (int k = 0; k < PER; ++k) { \
-                const int n = j + k * G; \
-                S[k] = fmaf(A[k].over(dt), S[k], du * b_s[ti][n]);          /* beyond the state size A, B and C are zero */ \
-                y = fmaf(S[k], c_s[ti][n], y); \
-            } \
-            y = group_sum<G>(y); \
-            if (j == 0) y_s[ti][ch] = y; }
+        auto token = [&](int ti) __attribute__((always_inline)) {
+            const float2 in = in_s[ti][ch];
+            float y = 0.f;
+#pragma unroll
+            for (int k = 0; k < PER; ++k) {
+                const float2 v = bc_s[ti][j * PER + k];
+                S[k] = fmaf(A[k].over(in.x), S[k], in.y * v.x);              // beyond the state size A, B and C are zero
+                y = fmaf(S[k], v.y, y);
+            }
+            return y;
+        };
         if (tt == SCAN_TILE) {                                  // a whole tile: no test between its tokens
 #pragma unroll
-            for (int ti = 0; ti < SCAN_TILE; ++ti) SCAN_TOKEN(ti)
+            for (int t = 0; t < SCAN_TILE; t += TG) {
+                float y[TG];
+#pragma unroll
+                for (int i = 0; i < TG; ++i) y[i] = token(t + i);
+                const float sum = group_sums<G>(y, j);
+                if (G == TG || j < TG) y_s[t + j % TG][ch] = sum;
+            }
         } else {
 #pragma unroll 1
-            for (int ti = 0; ti < tt; ++ti) SCAN_TOKEN(ti)
+            for (int ti = 0; ti < tt; ++ti) {
+                const float y = group_sum<G>(token(ti));
+                if (j == 0) y_s[ti][ch] = y;
+            }
         }
-#undef SCAN_TOKEN
         __syncthreads();
         // the next tile's elements may go to LDS while these are read: y_s is written behind the next barrier only
 #pragma unroll
@@ -319,14 +395,14 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
             const int idx = threadIdx.x + i * SCAN_THREADS, ti = idx / CH, k = idx % CH;
             if (ti < tt && c0 + k < channels) {
                 const float y = fmaf(skip[i], u_t[i], y_s[ti][k]);
-                out[(row0 + t0 + ti) * channels + c0 + k] = from_float<T>(y * silu_f(z_t[i]));
+                out[(row0 + t0 + ti) * channels + c0 + k] = from_float<T>(y * scan_silu(z_t[i]));
             }
         }
     }
     if (mine && n_new > 0) {
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const int n = j + k * G;
+            const int n = j * PER + k;
             if (n < n_state) sp[n] = S[k];
         }
     }
@@ -345,12 +421,24 @@ PALM_API int palm_selective_scan(hipStream_t stream, const void* u, const void* 
         dim3 grid((channels + per_block - 1) / per_block, n_seqs); \
         selective_scan_kernel<T, G, PER><<<grid, SCAN_THREADS, 0, stream>>>((const T*)u, (const T*)z, z_stride, \
             (const T*)bc, bc_stride, b_off, c_off, dtl, dt_bias, a_log, d_skip, state, seq_slot, seq_new, cu_new, channels, n_state, (T*)out); }
+    // States a lane: one, while that leaves each SIMD no more than four waves (a long sequence is a chain of its tokens, and a lane with
+    // more states takes longer over each); else two or four, which share a token's reads and the sums over the group.  us with one,
+    // two and four: 8,192 channels x 16 states, 2,603 tokens (2,048 waves) 253, 337, 548; 717 + 572 + 1,314 (6,144) 229, 218, 308;
+    // 8 x 300 155, 135, 132; 2,048 channels x 64 states, 717 + 572 + 1,314 (6,144) 240, 203, 251; 8 x 300 (16,384) 179, 130, 113;
+    // 128 states, two and four, 6,144 waves 438 and 456, 16,384 waves 302 and 243.  Up to eight states one is always the fastest.
+    const long long lanes = n_state <= 8 ? 8 : n_state <= 16 ? 16 : n_state <= 32 ? 32 : 64, waves = lanes * n_seqs * channels / WAVE;
+    const bool many = waves > 4096, more = waves > 8192;
     PALM_DTYPE_SWITCH(dtype, T, {
         if (n_state <= 4) SCAN_CASE(4, 1)
         else if (n_state <= 8) SCAN_CASE(8, 1)
+        else if (n_state <= 16 && many) SCAN_CASE(8, 2)
         else if (n_state <= 16) SCAN_CASE(16, 1)
+        else if (n_state <= 32 && many) SCAN_CASE(16, 2)
         else if (n_state <= 32) SCAN_CASE(32, 1)
+        else if (n_state <= 64 && more) SCAN_CASE(16, 4)
+        else if (n_state <= 64 && many) SCAN_CASE(32, 2)
         else if (n_state <= 64) SCAN_CASE(64, 1)
+        else if (n_state <= 128 && more) SCAN_CASE(32, 4)
         else if (n_state <= 128) SCAN_CASE(64, 2)
         else SCAN_CASE(64, 4)
     });

@@ -541,6 +541,39 @@ def test_selective_scan_alone(dtype, C, N):
 
 
 @gpu
+@pytest.mark.parametrize("C,N", [(2740, 9), (2740, 16), (1370, 32), (700, 64), (1370, 64), (1370, 100)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_selective_scan_of_many_channels(dtype, C, N):
+    """Channels enough that a lane holds two or four states, to the same bounds."""
+    test_selective_scan_alone(dtype, C, N)
+
+
+@gpu
+def test_selective_scan_at_the_ends_of_its_step_sizes_and_gates():
+    """Step sizes and gates around where the kernel's own softplus and silu hand over to the library, and what is no finite number."""
+    from palm_infra_amd.kernels import ops
+    ends = torch.tensor([0.0, -0.0, 1e-3, -1e-3, 1.0, -1.0, 20.0, 20.1, 86.9, -86.9, 87.1, -87.1, 200.0, -200.0, float("inf"), -float("inf"), float("nan")])
+    C, N, T = len(ends), 5, 33
+    g = torch.Generator().manual_seed(3)
+    u, bc, a_log = torch.randn(T, C, generator=g), torch.randn(T, 2 * N, generator=g), torch.zeros(C, N)
+    for gates in (False, True):
+        dtl, z = (torch.randn(T, C, generator=g), ends.repeat(T, 1)) if gates else (ends.repeat(T, 1), torch.randn(T, C, generator=g))
+        dt, S, want = torch.nn.functional.softplus(dtl.double(), threshold=1e9), torch.zeros(C, N, dtype=P.F64), []
+        dt = torch.where(dtl > 500, dtl.double(), dt)
+        for t in range(T):
+            S = torch.exp(-dt[t][:, None]) * S + (dt[t] * u[t].double())[:, None] * bc[t, :N].double()
+            want.append((S * bc[t, N:].double()).sum(1) * z[t].double() / (1 + torch.exp(-z[t].double())))
+        want, state = torch.stack(want), torch.zeros(1, C, N).cuda()
+        got = ops.selective_scan(u.cuda(), torch.cat([u, z], 1).cuda(), bc.cuda(), 0, N, dtl.cuda(), torch.zeros(C).cuda(), a_log.cuda(),
+                                 torch.zeros(C).cuda(), state, _step_context([0], [T])).double().cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        # each channel against its own size: sums of 32-bit terms over 33 tokens (and below 2^-126 nothing is compared)
+        keep = torch.isfinite(want)
+        size = torch.where(keep, want, 0.0).abs().amax(0)
+        assert (torch.where(keep, got - want, 0.0).abs().amax(0) <= 1e-5 * size + 1e-37).all()
+
+
+@gpu
 @pytest.mark.parametrize("dk,dv", [(12, 28), (40, 72)])      # the second pair is one that the matrix-core kernel takes in bfloat16
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge(dtype, dk, dv):
