@@ -849,7 +849,7 @@ __device__ inline void stage_values(const PagePrefetch& pf, bf16_t* v_lds) {
 struct PageSources { uint32_t k[PF_LOADS], v[PF_LOADS]; };       // byte offsets into a page of K and of V^T
 __device__ inline PageSources page_sources() {
     PageSources src;
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE % PF_WAVES;
     static_assert(!PF_DMA || WAVE % CHUNKS == 0, "an instruction's 64 chunks must be whole key rows");
     constexpr int K_ROWS = WAVE / CHUNKS;                        // key rows an instruction covers
 #pragma unroll
@@ -876,7 +876,7 @@ __device__ __forceinline__ uint32_t lds_address(const bf16_t* p) {       // the 
 }
 __device__ inline void page_into_lds(const bf16_t* __restrict__ kp, const bf16_t* __restrict__ vp, const PageSources& src,
                                      bf16_t* k_lds, bf16_t* v_lds) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) % PF_WAVES;
     constexpr int KB = 1024 / sizeof(bf16_t);                    // elements of 1 KB
 #pragma unroll
     for (int i = 0; i < PF_LOADS; ++i)
@@ -891,7 +891,7 @@ __device__ inline void page_into_lds(const bf16_t* __restrict__ kp, const bf16_t
 // multiplied all the same, and zero times a NaN or an infinity is NaN: they are made zero in LDS, once, before the
 // page is used.  `tail`: the last key of the sequence, as an index into the page.  (A barrier must follow.)
 __device__ inline void blank_values_after(bf16_t* v_lds, int tail) {
-    for (int idx = threadIdx.x; idx < HD * (PAGE_TOKENS / 8); idx += PF_THREADS) {
+    for (int idx = threadIdx.x % PF_THREADS; idx < HD * (PAGE_TOKENS / 8); idx += PF_THREADS) {
         const int d = idx / (PAGE_TOKENS / 8), chunk = idx % (PAGE_TOKENS / 8);
         if (chunk * 8 + 7 <= tail) continue;
         bf16x8* at = reinterpret_cast<bf16x8*>(v_lds + d * V_STRIDE + (chunk ^ v_swizzle(d)) * 8);
@@ -1237,9 +1237,12 @@ __global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefil
 //    it.  Whether any column of the wave has to move is one vote over the lanes' own sixteen scores; the exchange
 //    between the four lanes of a column, the shift and the rescaling of the outputs stand behind that vote, off the
 //    usual path;
-//  * STAGES pages of K and V^T lie in LDS, STAGES - 1 of them on their way while one is used: two where many blocks
-//    share a compute unit, four where a short prompt leaves a unit one block, whose loads then need a longer lead.
-//    The barrier between pages waits for LDS and for the one page that is needed next, not for the younger loads.
+//  * two pages of K and V^T lie in LDS, one of them on its way while the other is used;
+//  * where the launch has a compute unit no second block (HALVES = 2), a block has eight waves instead: two halves of four that hold
+//    the same queries and take every other page each, with two pages of LDS a half.  A block alone walks its pages one after the other,
+//    some 2 us each, whatever else the unit could do meanwhile; at the end the second half's sums go to the first through LDS.  us, with
+//    four waves and four pages in LDS, and now (32 heads of 8): 1,024 tokens 34.1 and 25.1, 512 20.7 and 16.4, 256 13.8 and 12.3, 64 behind 2,000 60
+//    and 39, behind 8,000 205 and 120, 1,000 behind 3,000 115 and 77, 91 10.6 and 10.5; one page 9.0 and 9.3.
 template <int N> __device__ __forceinline__ void wait_for_all_but_the_youngest_loads() {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));          // s_waitcnt vmcnt(N)
 }
@@ -1375,17 +1378,16 @@ __device__ __forceinline__ void paired_page(const bf16_t* k_lds, const bf16_t* v
             for (int x = 0; x < PF_UNITS; ++x) u[x].o[dt] = mfma_16x16x32(vf[dt][h], pv[x][h], u[x].o[dt]);
 }
 
-template <int STAGES, bool PRESCALED>
-__global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefill_paired_kernel(
+template <int HALVES, bool PRESCALED>
+__global__ __launch_bounds__(HALVES * PF_THREADS) PF_WAVES_PER_SIMD void attention_prefill_paired_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ block_table, int max_pages, const int* __restrict__ seq_slot,
     const int* __restrict__ seq_start, const int* __restrict__ seq_new, const int* __restrict__ cu_new, int nh,
     int nkv, float scale_log2, int window, int qb, int hg, int partners_follow, bf16_t* __restrict__ out) {
     if constexpr (PF_DMA) {
         constexpr int K_TILE = PAGE_TOKENS * K_STRIDE, V_TILE = HD * V_STRIDE;
-        constexpr int PAGE_LOADS = 2 * PF_LOADS;                    // a wave's instructions for one page of K and V^T
-        __shared__ __attribute__((aligned(16))) bf16_t k_lds[STAGES * K_TILE];
-        __shared__ __attribute__((aligned(16))) bf16_t v_lds[STAGES * V_TILE];
+        __shared__ __attribute__((aligned(16))) bf16_t k_lds[HALVES * 2 * K_TILE];
+        __shared__ __attribute__((aligned(16))) bf16_t v_lds[HALVES * 2 * V_TILE];
 
         const int b = blockIdx.z;
         const int G = nh / nkv, n_hg = (G + hg - 1) / hg;
@@ -1395,10 +1397,11 @@ __global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefil
         if ((int)blockIdx.y >= n_q) return;
         // first the tiles from the back (the long ones), the last first; then, where the launch asks for it, their
         // partners from the front in the same order, else the rest from the back too
-        const int half = (n_q + 1) / 2, y = blockIdx.y;
-        const int tile = y < half || !partners_follow ? n_q - 1 - y : y - half;
+        const int from_back = (n_q + 1) / 2, y = blockIdx.y;
+        const int tile = y < from_back || !partners_follow ? n_q - 1 - y : y - from_back;
         const int lane = threadIdx.x % WAVE, r = lane % 16, g = lane / 16;
-        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) % PF_WAVES;
+        const int half = HALVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / PF_THREADS) : 0;
         const int start = seq_start[b];
         const int seq_tail = start + n_new - 1;                       // the sequence's last key
         const int heads_here = min(hg, G - hgi * hg);
@@ -1432,10 +1435,11 @@ __global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefil
             const int tile_last = min(tile_first + qb - 1, n_new - 1);
             const int p_hi = (start + tile_last) / PAGE_TOKENS;
             const int p_lo = window > 0 ? max(0, start + tile_first - window + 1) / PAGE_TOKENS : 0;
-            auto load_page = [&](int p) {
+            // of every HALVES pages in turn each half takes one, into two places of its own
+            bf16_t *k_half = k_lds + half * 2 * K_TILE, *v_half = v_lds + half * 2 * V_TILE;
+            auto load_page = [&](int p, int step) {
                 const size_t at = ((size_t)pages[p] * nkv + kvh) * PAGE_TOKENS * HD;
-                const int stage = (p - p_lo) % STAGES;
-                page_into_lds(k_cache + at, v_cache + at, sources, k_lds + stage * K_TILE, v_lds + stage * V_TILE);
+                page_into_lds(k_cache + at, v_cache + at, sources, k_half + step % 2 * K_TILE, v_half + step % 2 * V_TILE);
             };
             // is every key of page p visible to every column of this wave?
             auto interior = [&](int p) -> bool {
@@ -1446,38 +1450,53 @@ __global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefil
                 return __all(inside);
             };
             wait_for_all_but_the_youngest_loads<0>();                 // the queries
-#pragma unroll
-            for (int ahead = 0; ahead < STAGES - 1; ++ahead)
-                if (p_lo + ahead <= p_hi) load_page(p_lo + ahead);
-            // the first page has landed when at most the pages after it are on their way
-            if constexpr (STAGES > 2) {
-                const int young = min(p_hi - p_lo, STAGES - 2);
-                if (young >= 2) wait_for_all_but_the_youngest_loads<2 * PAGE_LOADS>();
-                else if (young == 1) wait_for_all_but_the_youngest_loads<PAGE_LOADS>();
-                else wait_for_all_but_the_youngest_loads<0>();
-            } else {
-                wait_for_all_but_the_youngest_loads<0>();
-            }
+            if (p_lo + half <= p_hi) load_page(p_lo + half, 0);
+            wait_for_all_but_the_youngest_loads<0>();
             page_barrier();
-            for (int p = p_lo; p <= p_hi; ++p) {
-                const int stage = (p - p_lo) % STAGES;
-                if (p + STAGES - 1 <= p_hi) load_page(p + STAGES - 1);      // into the stage whose readers passed the barrier a page ago
-                bf16_t* v_page = v_lds + stage * V_TILE;
-                if (seq_tail - p * PAGE_TOKENS < PAGE_TOKENS - 1) {          // the sequence's last page: no page follows it
-                    blank_values_after(v_page, seq_tail - p * PAGE_TOKENS);
+            for (int step = 0; p_lo + step * HALVES <= p_hi; ++step) {    // the same number of steps for all waves
+                const int p_step = p_lo + step * HALVES, p = p_step + half;
+                if (p + HALVES <= p_hi) load_page(p + HALVES, step + 1);    // into the place whose readers passed the barrier a step ago
+                bf16_t* v_page = v_half + step % 2 * V_TILE;
+                const int tail_page = seq_tail / PAGE_TOKENS, tail = seq_tail % PAGE_TOKENS;
+                if (tail < PAGE_TOKENS - 1 && p_step <= tail_page && tail_page < p_step + HALVES) {   // the sequence's last page: none follows it
+                    if (p == tail_page) blank_values_after(v_page, tail);
                     __syncthreads();
                 }
-                paired_page<PRESCALED>(k_lds + stage * K_TILE, v_page, u, p * PAGE_TOKENS, scale_log2, r, g, !interior(p));
-                // the next page has landed when at most the pages after it are on their way
-                if constexpr (STAGES > 2) {
-                    const int young = min(p_hi, p + STAGES - 1) - (p + 1);
-                    if (young >= 2) wait_for_all_but_the_youngest_loads<2 * PAGE_LOADS>();
-                    else if (young == 1) wait_for_all_but_the_youngest_loads<PAGE_LOADS>();
-                    else wait_for_all_but_the_youngest_loads<0>();
-                } else {
-                    wait_for_all_but_the_youngest_loads<0>();
-                }
+                if (p <= p_hi) paired_page<PRESCALED>(k_half + step % 2 * K_TILE, v_page, u, p * PAGE_TOKENS, scale_log2, r, g, !interior(p));
+                wait_for_all_but_the_youngest_loads<0>();             // the half's next page has landed
                 page_barrier();
+            }
+            if (HALVES > 1 && p_lo == p_hi) {                         // one page: the first half had it
+                if (half == 1) return;
+            } else if constexpr (HALVES > 1) {
+                // the second half's sums go through LDS (nobody reads pages any more, none is on its way) to the same lanes of the first
+                float4* o_lds = reinterpret_cast<float4*>(k_lds);
+                float2* m_lds = reinterpret_cast<float2*>(v_lds);
+                static_assert(PF_WAVES * PF_UNITS * DTILES * WAVE * 16 <= sizeof(k_lds) && PF_WAVES * PF_UNITS * WAVE * 8 <= sizeof(v_lds));
+                if (half == 1) {
+#pragma unroll
+                    for (int x = 0; x < PF_UNITS; ++x) {
+#pragma unroll
+                        for (int dt = 0; dt < DTILES; ++dt)
+                            o_lds[((wave * PF_UNITS + x) * DTILES + dt) * WAVE + lane] =
+                                make_float4(u[x].o[dt][0], u[x].o[dt][1], u[x].o[dt][2], u[x].o[dt][3]);
+                        m_lds[(wave * PF_UNITS + x) * WAVE + lane] = make_float2(u[x].m, u[x].weights[0]);
+                    }
+                }
+                __syncthreads();
+                if (half == 1) return;
+#pragma unroll
+                for (int x = 0; x < PF_UNITS; ++x) {
+                    const float2 other = m_lds[(wave * PF_UNITS + x) * WAVE + lane];
+                    const float top = fmaxf(u[x].m, other.x), from = top == -INFINITY ? 0.f : top;   // (a half may have seen none of the column's keys)
+                    const float mine = exp2_weight(u[x].m - from), its = exp2_weight(other.x - from);
+                    u[x].weights[0] = u[x].weights[0] * mine + other.y * its;
+#pragma unroll
+                    for (int dt = 0; dt < DTILES; ++dt) {
+                        const float4 o = o_lds[((wave * PF_UNITS + x) * DTILES + dt) * WAVE + lane];
+                        u[x].o[dt] = u[x].o[dt] * mine + f32x4{o.x, o.y, o.z, o.w} * its;
+                    }
+                }
             }
 #pragma unroll
             for (int x = 0; x < PF_UNITS; ++x) {
@@ -1865,14 +1884,17 @@ PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const voi
         PALM_CHECK(n_q <= 65535, "attention_prefill: %d new tokens are more than one launch takes", max_new);
         dim3 grid(nkv * n_hg, n_q, n_seqs);
         const long long blocks = (long long)grid.x * grid.y * grid.z;
-        // four pages in LDS leave a compute unit room for one block: where the launch has no second block for it anyway
-        const bool few = blocks <= 256;
-        const int partners_follow = blocks <= 512 && n_seqs == 1;     // all blocks run at once, two a unit
-#define PALM_PAIRED(STAGES, PRE) attention_prefill_paired_kernel<STAGES, PRE><<<grid, PF_THREADS, 0, stream>>>( \
+        // Two halves a block where every compute unit has one block at most, and for one sequence while the shortest tiles, which go last,
+        // are all that a second round has: 1,300 tokens (328 blocks) 38 and 30 us, 1,800 (456) 48 and 44, 64 heads of 8, 600 tokens
+        // (304) 23.1 and 21.8, 40 heads of 8, 800 (400) 26.2 and 25.8, 1,024 (512) 30.4 and 32.0.  Several sequences fill the rounds with long
+        // tiles and empty ones: four of 512 (512 blocks) 25 and 30, 700 + 500 + 300 (528) 25 and 28.
+        const bool few = blocks <= (n_seqs == 1 ? 448 : 256);
+        const int partners_follow = !few && blocks <= 512 && n_seqs == 1;     // all blocks run at once, two a unit
+#define PALM_PAIRED(HALVES, PRE) attention_prefill_paired_kernel<HALVES, PRE><<<grid, HALVES * PF_THREADS, 0, stream>>>( \
         (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, max_pages, seq_slot, seq_start, seq_new, \
         cu_new, nh, nkv, scale_log2, window, qb, hg, partners_follow, (bf16_t*)out)
-        if (few) { if (q_prescaled) PALM_PAIRED(4, true); else PALM_PAIRED(4, false); }
-        else { if (q_prescaled) PALM_PAIRED(2, true); else PALM_PAIRED(2, false); }
+        if (few) { if (q_prescaled) PALM_PAIRED(2, true); else PALM_PAIRED(2, false); }
+        else { if (q_prescaled) PALM_PAIRED(1, true); else PALM_PAIRED(1, false); }
 #undef PALM_PAIRED
         PALM_LAUNCHED();
         return 0;

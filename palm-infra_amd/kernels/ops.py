@@ -962,11 +962,13 @@ def wide_prompt_attention(starts, counts, nh: int, nkv: int) -> bool:
     """Whether a step's prompts (``counts`` new tokens behind ``starts`` earlier ones) are sooner through the kernel whose waves hold 64
     columns.  Both kernels' times in microseconds from the pages that their blocks walk over: the wide one has a block of 16 units (one
     head's 16 queries) a compute unit, some 9 us of start and end that nothing hides, and 1.6 us a page with all units at work; the other two blocks
-    of eight units, 2 us a page each.  Measured (32 heads of 8 unless said otherwise; the other's time and this one's): 2,048 tokens 51 58,
-    3,072 82 82, 3,500 106 97, 4,096 142 125, 13,331 1,281 1,134, four of 2,048 151 156, four of 3,072 318 312, 64 behind 1,000 34 38, behind 2,000 58 58, 1,000
-    behind 3,000 112 102; 40 heads of 8 (five of eight units used, fifteen of sixteen) 1,024 tokens 31 38, 2,048 87 67, 8,192 939 590, five of 45 to 2,000 125 106;
-    64 heads of 8 3,072 150 157, 4,096 253 241; 16 heads of 8 4,096 92 102, 8,192 266 224.  The numbers below are fitted to 64 such steps: the slower one is taken at four of
-    them (16 heads of 8 at 4,096 tokens by 11 %, 8 of 8 at 8,192 by 8 %, two by less than 3 %)."""
+    of eight units, 2 us a page each, or, where its blocks are few, one of two halves that take 1.9 us for two pages (then the other is the
+    sooner one but for second rounds of long blocks: 1,100 behind 2,000 79 83, 1,000 behind 3,000 77 102, 1,024 behind 30,000 458 675).
+    Measured (32 heads of 8 unless said otherwise; the other's time and this one's): 2,048 tokens 51 58, 3,072 82 82, 3,500 106 97, 4,096
+    142 125, 13,331 1,281 1,134, four of 2,048 151 156, four of 3,072 318 312; 40 heads of 8 (five of eight units used, fifteen of sixteen)
+    1,024 tokens 31 38, 2,048 87 67, 8,192 939 590, five of 45 to 2,000 125 106; 64 heads of 8 3,072 150 157, 4,096 253 241; 16 heads of 8
+    4,096 92 102, 8,192 266 224.  The numbers below are fitted to 64 such steps: the slower one is taken at four of them (16 heads of 8 at
+    4,096 tokens by 11 %, 8 of 8 at 8,192 by 8 %, two by less than 3 %)."""
     G = nh // nkv
 
     def tiles_and_pages(units):
@@ -979,6 +981,13 @@ def wide_prompt_attention(starts, counts, nh: int, nkv: int) -> bool:
     blocks, pages = tiles_and_pages(16)
     wide_us = 9.2 + max(5 + 1.35 * longest, (9.6 * blocks + 1.61 * pages) / COMPUTE_UNITS)
     blocks, pages = tiles_and_pages(8)
+    heads = min(G, 8)
+    launched = nkv * -(-G // heads) * -(-max(counts) // (16 * (8 // heads))) * len(counts)
+    if launched <= COMPUTE_UNITS or len(counts) == 1 and launched <= 448:       # as palm_attention_prefill takes halves
+        in_turn = longest
+        if launched > COMPUTE_UNITS:        # the last of the first round and the first of the second
+            in_turn = max(longest, 2 * (starts[0] + counts[0] * (1 - COMPUTE_UNITS / launched)) / PAGE_TOKENS)
+        return wide_us < 9 + 0.95 * in_turn
     other_us = 6.8 + max(1.57 * longest, (2.2 * blocks + 1.95 * pages) / (2 * COMPUTE_UNITS))
     return wide_us < other_us
 

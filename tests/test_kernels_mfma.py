@@ -602,9 +602,22 @@ def test_wide_prompt_attention_is_taken_for_long_prompts(ops):
     assert ops.wide_prompt_attention([0], [13331], 32, 8) and ops.wide_prompt_attention([30720], [2048], 32, 8)
     assert not ops.wide_prompt_attention([0], [2048], 32, 8) and not ops.wide_prompt_attention([0], [91], 32, 8)
     assert ops.wide_prompt_attention([0], [2048], 40, 8) and not ops.wide_prompt_attention([0] * 64, [20] * 64, 40, 8)
+    assert not ops.wide_prompt_attention([30000], [1024], 32, 8) and ops.wide_prompt_attention([30000], [1500], 32, 8)
     with pytest.raises(KernelError, match="not for head size 64"):
         _attention_case(ops, lambda q, kc, vc, table, slots, starts, news, cu, max_new, a, b, c, scale, window: ops.attention_prefill(
             q, kc, vc, table, slots, starts, news, cu, max_new, 4, 2, 64, scale, window, wide=True), BF16, 4, 2, 64, [(20, 20)], None)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (40, 8, 128), (4, 2, 64), (3, 3, 128)])
+@pytest.mark.parametrize("window", [None, 1, 64, 200])
+def test_attention_of_few_blocks_takes_pages_by_halves(ops, nh, nkv, hd, window):
+    """Prompts of few blocks, whose pages go to two halves of a block in turn: one page, an odd and an even number of them, a last page that is
+    full or holds one key, a half that sees none of a column's keys (a window, a second page that most queries do not reach), sequences of
+    unequal length together, and the first sizes beyond, which one half takes."""
+    for lens in ([(1, 1)], [(64, 64)], [(65, 65)], [(128, 100)], [(129, 2)], [(192, 192)], [(513, 70)], [(700, 1), (65, 65), (64, 3), (130, 130)],
+                 [(1300, 1300)], [(1100, 1100), (30, 30)]):
+        got, ref = _attention_case(ops, ops.attention_prefill, BF16, nh, nkv, hd, lens, window, seed=hd + len(lens))
+        assert torch.isfinite(got).all() and torch.allclose(got, ref, atol=2e-2), (lens, float((got - ref).abs().max()))
 
 
 @pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (4, 2, 64), (6, 1, 80)])
