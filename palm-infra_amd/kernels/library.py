@@ -57,6 +57,10 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-fno-gpu-rdc",
          # and 3,645 us; Nirotar, 6 sequences 1,560 and 1,544).  Structs among the arguments end the run: they stand last.
          "-mllvm", "-amdgpu-kernarg-preload-count=16",
          "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option"]
+# Sources that are compiled without some of them.  The large tiles run for hundreds of microseconds, a launch's start is nothing to
+# them, and their loop comes out a little slower behind preloaded arguments (gated, 4,309 rows 615.6 us and 613.5 without, 13,331
+# rows 1,872 and 1,860; a prompt of 13,331 tokens against the code without preloading 1.022 and 1.042 times as fast).
+FLAGS_LEFT_OUT = {"linear_big.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
 
 CORE_SOURCES = ["elementwise.hip", "linear.hip", "rope_store.hip", "attention_simple.hip", "sampling.hip",
                 "linear_mfma.hip", "linear_ring.hip", "linear_ring_many.hip", "linear_wide.hip", "linear_wide_store_32.hip", "linear_wide_store_64.hip",
@@ -132,7 +136,7 @@ def _digest(sources, defines) -> str:
     h.update(" ".join(FLAGS + sorted(defines)).encode())
     own = {h for s in sources for h in OWN_HEADERS.get(s, ())}
     for name in sorted(_existing(list(sources) + HEADERS + sorted(own))):
-        h.update(name.encode())
+        h.update(" ".join([name, *FLAGS_LEFT_OUT.get(name, ())]).encode())
         h.update((CSRC / name).read_bytes())
     return h.hexdigest()[:16]
 
@@ -169,7 +173,8 @@ def _compile(name: str, sources, defines, force: bool) -> Path:
 
     def one(src: str) -> Path:
         obj = work / (src.replace(".hip", "") + ".o")
-        cmd = [hipcc, *FLAGS, *[f"-D{d}" for d in defines], "-c", str(CSRC / src), "-o", str(obj)]
+        left_out = FLAGS_LEFT_OUT.get(src, ())
+        cmd = [hipcc, *[f for f in FLAGS if f not in left_out], *[f"-D{d}" for d in defines], "-c", str(CSRC / src), "-o", str(obj)]
         r = subprocess.run(cmd, capture_output=True, text=True, env=env)
         if r.returncode != 0:
             raise KernelBuildError(f"hipcc failed on {src}:\n{r.stderr[-4000:]}")
