@@ -1836,7 +1836,15 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
             stage = next;
         }
         wait_for_all_but_the_youngest_loads<0>();                     // nothing may land in LDS after the block's end
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        // The last products' sums are whole a few clocks from here.  All sums go through the wait or stand behind it: without operands of its own
+        // it would hold back none of their reads.
+        asm volatile("s_nop 15" : "+a"(weights[2]), "+a"(weights[3]), "+a"(o[2][DTILES - 1]), "+a"(o[3][DTILES - 1]));
+#pragma unroll
+        for (int x = 0; x < WIDE_UNITS; ++x) {
+#pragma unroll
+            for (int dt = 0; dt < DTILES; ++dt) asm volatile("" : "+a"(o[x][dt]));
+            asm volatile("" : "+a"(weights[x]));
+        }
         WIDE_FENCE;
 #undef WIDE_FENCE
 #undef WIDE_NOP
