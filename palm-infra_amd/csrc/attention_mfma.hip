@@ -1541,8 +1541,10 @@ constexpr bool PF_WIDE = PF_DMA && HD == 128;
 constexpr int WIDE_UNITS = 4, WIDE_STAGES = 4;
 
 // The products are written out, so that sums and queries stay in the accumulator registers and the scores where vector instructions
-// read them.  The distances that the compiler would keep for its own products are kept by their order: a score is read five
-// products or more behind its last one, a sum is added to again four behind, weights are read behind an s_nop.
+// read them.  The compiler keeps no distances between them and what reads their results (eight issue slots, two products, for its own
+// ones); the order of what stands between the products does: four products follow a score's last one before the score is read,
+// a sum is added to again PV / 2 products later, weights lie two instructions before the product that takes them, and the
+// sums are read behind a wait at the end.  (tests/test_written_out_products.py follows them through the assembly.)
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void wide_score_first(f32x4& s, bf16x8 k, bf16x8 q, f32x4 from) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %3" : "=&v"(s) : "v"(k), "a"(q), "v"(from));
@@ -1553,9 +1555,9 @@ __device__ __forceinline__ void wide_score(f32x4& s, bf16x8 k, bf16x8 q) {
 __device__ __forceinline__ void wide_weigh(f32x4& o, bf16x8 v, u32x4 p) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(o) : "v"(v), "v"(p));
 }
-__device__ __forceinline__ float wide_max(float a, float b, float c) {         // (fmaxf would first make each of them quiet)
+__device__ __forceinline__ float wide_max(float a, float b, float c) {         // (fmaxf would first make each of them quiet; volatile: not before the product in front of it)
     float most;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(most) : "v"(a), "v"(b), "v"(c));
+    asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(most) : "v"(a), "v"(b), "v"(c));
     return most;
 }
 
@@ -1569,6 +1571,8 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         constexpr int K_TILE = PAGE_TOKENS * K_STRIDE, V_TILE = HD * V_STRIDE, PAGE_LOADS = 2 * PF_LOADS;
         constexpr int QK = 8 * KSTEPS, PV = 4 * DTILES + 4;         // products of a pair of units
         static_assert(QK == 32 && PV == 36 && PAGE_LOADS == 8, "what goes between which products below is laid out for heads of 128");
+        constexpr int MAX_FROM = 28;                                // P's maxima begin behind this product of its scores; QK - 8 ends the first score
+        static_assert(MAX_FROM - (QK - 8) >= 4 && MAX_FROM < QK && PV / 2 >= 4, "four products between a result's last one and what reads it");
         __shared__ __attribute__((aligned(16))) bf16_t k_lds[WIDE_STAGES * K_TILE];
         __shared__ __attribute__((aligned(16))) bf16_t v_lds[WIDE_STAGES * V_TILE];
 
@@ -1656,6 +1660,7 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         };
         auto maximum = [&](int pair, int n) __attribute__((always_inline)) {         // n-th of eight parts
             const int x = n % 2, t = n / 2;
+            if (!PRESCALED) asm volatile("" : "+v"(s[pair][x][t]));   // (read behind the product that stands before this, not before it)
             f32x4 v = s[pair][x][t];
             if (!PRESCALED) {
 #pragma unroll
@@ -1777,7 +1782,7 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                 if (n == 1 || n == 5) read_k(stage, 2 + n / 4, 3);
                 if (n >= 8 && n % 3 == 2) read_v(stage, (n - 8) / 3, 0);
                 if (n % 4 == 3 && n < 16) load_v(from, (stage + 2) % WIDE_STAGES, n / 4);
-                if (n >= 28) maximum(0, n - 28);
+                if (n >= MAX_FROM) maximum(0, n - MAX_FROM);
                 WIDE_FENCE;
             }
             // the next page has landed when at most the one after it is on its way; behind the barrier no wave reads the page before this one
@@ -1788,8 +1793,8 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
 #pragma unroll
             for (int n = 0; n < 7; ++n) {
                 score(1, n);
-                if (n < 4) maximum(0, 4 + n);
-                if (n == 4) unsettled = vote(0, masked);
+                if (n < 8 - (QK - MAX_FROM)) maximum(0, QK - MAX_FROM + n);
+                if (n == 8 - (QK - MAX_FROM)) unsettled = vote(0, masked);
                 if (n % 4 == 3) read_v(stage, n / 4, 1);
                 WIDE_FENCE;
             }
