@@ -1765,8 +1765,8 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
         page_barrier();
 #pragma unroll
         for (int i = 0; i < 14; ++i) read_k(0, i % 4, i / 4);
-        int stage = 0;
-        for (int p = p_lo; p <= p_hi; ++p) {
+        int stage = 0, p = p_lo;
+        do {                                                          // (there is a first page: a test before it would keep the sums of a way past the loop)
             const int next = (stage + 1) % WIDE_STAGES, free_stage = (stage + 3) % WIDE_STAGES;
             const int first = p * PAGE_TOKENS;
             const bool masked = last_first > first || least_pos < first + PAGE_TOKENS - 1;
@@ -1774,7 +1774,10 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                 blank_values_after(v_lds + stage * V_TILE, seq_tail - first);
                 __syncthreads();
             }
-            if (((p + 3 - p_lo) & 63) == 0) ids = pages[min(p + 3 + lane, p_hi)];
+            if (((p + 3 - p_lo) & 63) == 0) {
+                ids = pages[min(p + 3 + lane, p_hi)];
+                asm volatile("" : "+v"(ids));                         // (waited for here: where it is used, every page would wait for all loads)
+            }
             WIDE_FENCE;
 #pragma unroll
             for (int n = 0; n < QK; ++n) {
@@ -1839,7 +1842,7 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                 WIDE_FENCE;
             }
             stage = next;
-        }
+        } while (++p <= p_hi);
         wait_for_all_but_the_youngest_loads<0>();                     // nothing may land in LDS after the block's end
         // The last products' sums are whole a few clocks from here.  All sums go through the wait or stand behind it: without operands of its own
         // it would hold back none of their reads.
