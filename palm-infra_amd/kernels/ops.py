@@ -406,7 +406,8 @@ def sample(logits: torch.Tensor, uniforms: torch.Tensor | None, temperature: flo
 
 @functools.lru_cache(maxsize=256)
 def _sliced_work(n: int, V: int, draws: bool, top_k: int) -> int:
-    """Bytes of workspace for rows that go in slices; 0: they do not."""
+    """Bytes of workspace for rows that go in slices; 0: they do not.  ``draws``: whether the temperature is above zero as the 32-bit number
+    that the launch gets."""
     return core().palm_sample_sliced_work(n, V, 1.0 if draws else 0.0, top_k)
 
 
@@ -417,7 +418,7 @@ def sample_drawn(logits: torch.Tensor, seed: int, streams, draws, temperature: f
     n = logits.shape[0]
     if logits.is_cuda and logits.dim() == 2 and logits.dtype == F32 and logits.is_contiguous():
         V, at = logits.shape[1], logits.data_ptr()
-        needed = _sliced_work(n, V, temperature > 0.0, top_k) if at % 16 == 0 else 0
+        needed = _sliced_work(n, V, c_float(temperature).value > 0.0, top_k) if at % 16 == 0 else 0
         if needed:
             s, d = _u64(streams), _u64(draws)
             _need(len(s) == n and len(d) == n, "sample: a stream and a draw's number for each row")

@@ -774,6 +774,13 @@ def test_draws_by_streams_are_draws_by_their_uniform_numbers(ops, n, V, k):
     assert ops.sample_drawn(lg, 42, streams, draws, 0.8, k, 0.95, 0.0).tolist() == want.tolist()
 
 
+@pytest.mark.parametrize("temperature", [1e-46, 7e-46, 2e-38])
+def test_draws_at_temperatures_around_the_smallest_32_bit_number(ops, temperature):
+    """A temperature that is zero as the kernel's 32-bit number draws as zero does; one above it goes in slices."""
+    lg = rand(3, 16384, seed=9, scale=3.0).to(DEV)
+    assert ops.sample_drawn(lg, 42, [1, 2, 3], [0, 1, 2], temperature, 50, 0.95, 0.0).tolist() == lg.argmax(1).tolist()
+
+
 def test_rows_are_sampled_independently(ops):
     lg = rand(4, 2000, seed=8)
     u = torch.tensor([0.1, 0.5, 0.9, 0.3])
