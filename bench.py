@@ -434,7 +434,7 @@ def _mixer_rooflines(raw: dict, tokens: int, batch: int, context: int) -> dict:
                 out["palm_moe_grouped"] = (2.0 * tokens * f["router"]["top"] * 3 * f["expert"]["ff"] * raw["width"], mfma, None, None)
     else:
         nh, nkv, hd = raw["num_attention_heads"], raw["num_key_value_heads"], raw["head_dim"]
-        out["palm_attention_prefill"] = (4.0 * nh * hd * pairs, mfma, None, None)
+        out["palm_attention_prefill_in"] = out["palm_attention_prefill_wide"] = (4.0 * nh * hd * pairs, mfma, None, None)
         kv = 2.0 * batch * context * 2 * nkv * hd
         out["palm_attention_decode_fused"] = out["palm_attention_decode"] = (None, None, kv, hbm)
     if "palm_moe_few" in out:                       # a step of up to 16 rows, in the sizes that the stream takes

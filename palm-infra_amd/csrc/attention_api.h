@@ -50,6 +50,14 @@ PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const voi
                                     int hd, float scale, int window, int q_prescaled, void* out);
 PALM_API int palm_attention_prefill_takes_prescaled();
 
+// The same by a caller who knows more: max_keys, the keys of the step's longest sequence (0: not known), and halves, whether a block's pages go to two
+// halves of it (1: no, 2: yes, 0: by the sizes, which palm_attention_prefill_halves tells; head sizes 64 and 128 only).
+PALM_API int palm_attention_prefill_in(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
+                                       const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
+                                       const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
+                                       int hd, float scale, int window, int q_prescaled, int max_keys, int halves, void* out);
+PALM_API int palm_attention_prefill_halves(int n_seqs, int max_new, int max_keys, int nh, int nkv, int window);
+
 // The same by the kernel whose waves hold 64 columns each (head size 128: palm_attention_prefill_wide_serves()).
 PALM_API int palm_attention_prefill_wide(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
                                          const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,

@@ -1238,11 +1238,12 @@ __global__ __launch_bounds__(PF_THREADS) PF_WAVES_PER_SIMD void attention_prefil
 //    between the four lanes of a column, the shift and the rescaling of the outputs stand behind that vote, off the
 //    usual path;
 //  * two pages of K and V^T lie in LDS, one of them on its way while the other is used;
-//  * where the launch has a compute unit no second block (HALVES = 2), a block has eight waves instead: two halves of four that hold
+//  * where the launch leaves a compute unit one block, or few second ones that are over soon, and a block's pages are many
+//    (prefill_takes_halves), a block has eight waves instead (HALVES = 2): two halves of four that hold
 //    the same queries and take every other page each, with two pages of LDS a half.  A block alone walks its pages one after the other,
 //    some 2 us each, whatever else the unit could do meanwhile; at the end the second half's sums go to the first through LDS.  us, with
-//    four waves and four pages in LDS, and now (32 heads of 8): 1,024 tokens 34.1 and 25.1, 512 20.7 and 16.4, 256 13.8 and 12.3, 64 behind 2,000 60
-//    and 39, behind 8,000 205 and 120, 1,000 behind 3,000 115 and 77, 91 10.6 and 10.5; one page 9.0 and 9.3.
+//    four waves and four pages in LDS, and so (32 heads of 8): 1,024 tokens 34.1 and 25.1, 512 20.7 and 16.4, 64 behind 2,000 60
+//    and 39, behind 8,000 205 and 120, 1,000 behind 3,000 115 and 77.
 template <int N> __device__ __forceinline__ void wait_for_all_but_the_youngest_loads() {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));          // s_waitcnt vmcnt(N)
 }
@@ -1874,16 +1875,53 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     }
 }
 
+// Whether a block's pages go to two halves of it (see the kernel).  max_keys: the longest sequence's keys, 0 where they are not known (the
+// new tokens alone then say how many pages there are at least).
+// From the pages that the longest tile walks over one after the other, us: 6.8 + 1.45 a page by one half with a second block on the unit,
+// 9 + 1.07 by two.  Blocks beyond the 256 units wait for the first round to end: their pages come on top of it, few for one
+// sequence from its start (the shortest tiles go last), as many as the first round's behind a long one or in a window.  A page with masks costs
+// twice more: the rest of a tile of 128 queries' own pages, and a window's first one.  One half and two, heads of 128, 32 of 8: one page 7.6 8.7 us,
+// two 9.1 9.9, four 11.8 12.1, five 13.0 13.1, six 14.4 13.9, nine 18.1 16.9; 1,000 tokens 28.8 25.0; 1,100 (280 blocks) 31.4 25.9, behind 2,000 79.7 79.2;
+// 1,400 (352) behind 1,500 71.5 71.7; 1,792 (448) 45.6 40.4, behind 1,000 69.4 68.6, behind 2,000 93.3 97.1; 1,300 in a window of 64 13.6 19.6, of
+// 512 26.6 28.8; 64 behind 2,000 in one of 64 12.0 12.5, of 128 14.2 13.0, of 512 21.6 18.5.  Heads of 64 divide alike (four pages 8.8 8.7, six
+// 10.8 10.0, 1,792 behind 1,000 48.3 47.0, 1,300 in a window of 64 9.6 12.7).  40 heads of 8, 1,024 tokens (512 blocks) 30.4 32.0.  Several sequences
+// fill the rounds with long tiles and empty ones: four of 512 (512 blocks) 25 30, 700 + 500 + 300 (528) 25 28.
+static bool prefill_takes_halves(int n_seqs, int max_new, int max_keys, int nh, int nkv, int window) {
+    const int G = nh / nkv, hg = min(G, PF_UNITS * PF_WAVES), qb = 16 * (PF_UNITS * PF_WAVES / hg), keys = max(max_keys, max_new);
+    const long long blocks = (long long)nkv * ((G + hg - 1) / hg) * ((max_new + qb - 1) / qb) * n_seqs;
+    constexpr int UNITS_OF_CHIP = 256;
+    if (!PF_DMA || (blocks > UNITS_OF_CHIP && (n_seqs > 1 || blocks > 448))) return false;
+    const bool windowed = window > 0 && window < keys;
+    int pages = (keys + PAGE_TOKENS - 1) / PAGE_TOKENS;
+    if (windowed) {         // a tile from a prompt's start lies within a page, any other one where it may
+        const long long most = keys > max_new ? (window + qb - 2ll) / PAGE_TOKENS + 2 : (window + 62ll) / PAGE_TOKENS + 1 + (qb - 1) / PAGE_TOKENS;
+        pages = (int)min((long long)pages, most) + 2;
+    }
+    pages += 2 * ((qb - 1) / PAGE_TOKENS);
+    double in_turn = pages;
+    if (blocks > UNITS_OF_CHIP) {
+        const double rest = 1.0 - (double)UNITS_OF_CHIP / blocks;      // the tokens whose tiles are the second round
+        in_turn = windowed ? 2.0 * pages : max(in_turn, 2.0 * (keys - max_new + max_new * rest) / PAGE_TOKENS);
+    }
+    return 9.0 + 1.07 * in_turn < 6.8 + 1.45 * pages;
+}
+PALM_API int palm_attention_prefill_halves(int n_seqs, int max_new, int max_keys, int nh, int nkv, int window) {
+    PALM_CHECK(n_seqs > 0 && max_new > 0 && max_keys >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0 && window >= 0,
+               "attention_prefill_halves: seqs=%d max_new=%d max_keys=%d heads=%d kv=%d window=%d", n_seqs, max_new, max_keys, nh, nkv, window);
+    return prefill_takes_halves(n_seqs, max_new, max_keys, nh, nkv, window) ? 2 : 1;
+}
+
 // q_prescaled: the queries come multiplied by scale * log2(e) already (by the pass that rounds them), so a score is
-// the exponent of its weight as it leaves the matrix cores; `scale` is then not applied again.
-PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
-                                    const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
-                                    const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
-                                    int hd, float scale, int window, int q_prescaled, void* out) {
+// the exponent of its weight as it leaves the matrix cores; `scale` is then not applied again.  halves: 1 or 2, 0: by the rule above
+PALM_API int palm_attention_prefill_in(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
+                                       const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
+                                       const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
+                                       int hd, float scale, int window, int q_prescaled, int max_keys, int halves, void* out) {
     PALM_CHECK(hd == HD, "attention_prefill: this library was built for head size %d, not %d", HD, hd);
     PALM_CHECK(n_seqs >= 0 && max_new >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0,
                "attention_prefill: seqs=%d max_new=%d heads=%d kv=%d", n_seqs, max_new, nh, nkv);
     PALM_CHECK(window >= 0 && max_pages > 0, "attention_prefill: window=%d max_pages=%d", window, max_pages);
+    PALM_CHECK(max_keys >= 0 && halves >= 0 && halves <= (PF_DMA ? 2 : 0), "attention_prefill: max_keys=%d halves=%d", max_keys, halves);
     if (n_seqs == 0 || max_new == 0) return 0;
     const int G = nh / nkv;
     constexpr int UNITS = PF_UNITS * PF_WAVES;                 // (head, 16 queries) units a block holds
@@ -1900,11 +1938,7 @@ PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const voi
         PALM_CHECK(n_q <= 65535, "attention_prefill: %d new tokens are more than one launch takes", max_new);
         dim3 grid(nkv * n_hg, n_q, n_seqs);
         const long long blocks = (long long)grid.x * grid.y * grid.z;
-        // Two halves a block where every compute unit has one block at most, and for one sequence while the shortest tiles, which go last,
-        // are all that a second round has: 1,300 tokens (328 blocks) 38 and 30 us, 1,800 (456) 48 and 44, 64 heads of 8, 600 tokens
-        // (304) 23.1 and 21.8, 40 heads of 8, 800 (400) 26.2 and 25.8, 1,024 (512) 30.4 and 32.0.  Several sequences fill the rounds with long
-        // tiles and empty ones: four of 512 (512 blocks) 25 and 30, 700 + 500 + 300 (528) 25 and 28.
-        const bool few = blocks <= (n_seqs == 1 ? 448 : 256);
+        const bool few = halves ? halves == 2 : prefill_takes_halves(n_seqs, max_new, max_keys, nh, nkv, window);
         const int partners_follow = !few && blocks <= 512 && n_seqs == 1;     // all blocks run at once, two a unit
 #define PALM_PAIRED(HALVES, PRE) attention_prefill_paired_kernel<HALVES, PRE><<<grid, HALVES * PF_THREADS, 0, stream>>>( \
         (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, max_pages, seq_slot, seq_start, seq_new, \
@@ -1925,6 +1959,14 @@ PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const voi
                                                              nkv, scale_log2, window, qb, hg, (bf16_t*)out);
     PALM_LAUNCHED();
     return 0;
+}
+
+PALM_API int palm_attention_prefill(hipStream_t stream, const void* q, const void* k_cache, const void* v_cache,
+                                    const int* block_table, int max_pages, const int* seq_slot, const int* seq_start,
+                                    const int* seq_new, const int* cu_new, int n_seqs, int max_new, int nh, int nkv,
+                                    int hd, float scale, int window, int q_prescaled, void* out) {
+    return palm_attention_prefill_in(stream, q, k_cache, v_cache, block_table, max_pages, seq_slot, seq_start, seq_new, cu_new, n_seqs, max_new,
+                                     nh, nkv, hd, scale, window, q_prescaled, 0, 0, out);
 }
 
 PALM_API int palm_attention_prefill_takes_prescaled() { return PF_DMA ? 1 : 0; }

@@ -792,6 +792,9 @@ _ATTENTION_SIGNATURES = {
                               c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p],
     "palm_attention_prefill": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p],
+    "palm_attention_prefill_in": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                  c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_void_p],
+    "palm_attention_prefill_halves": [c_int, c_int, c_int, c_int, c_int, c_int],
     "palm_attention_prefill_takes_prescaled": [],
     "palm_attention_prefill_wide": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p],
@@ -944,18 +947,21 @@ def prefill_q_scale(hd: int, dtype, scale: float) -> float:
 
 
 def attention_prefill(q, k_cache, v_cache, block_table, seq_slot, seq_start, seq_new, cu_new, max_new: int, nh: int,
-                      nkv: int, hd: int, scale: float, window: int | None, q_prescaled: bool = False, wide: bool = False) -> torch.Tensor:
+                      nkv: int, hd: int, scale: float, window: int | None, q_prescaled: bool = False, wide: bool = False,
+                      max_keys: int = 0, halves: int = 0) -> torch.Tensor:
     """The step's queries (several for each sequence) over the cache, on the matrix cores.  ``q_prescaled``: the
     queries come multiplied by ``prefill_q_scale`` already, and ``scale`` is not applied again.  ``wide``: by the kernel for long
-    prompts (head size 128), see ``wide_prompt_attention``."""
+    prompts (head size 128), see ``wide_prompt_attention``.  Else, for the head sizes 64 and 128, ``halves``: a block's pages go to one
+    half of it or to two (0: by the sizes; ``max_keys``: the longest sequence's keys, if known)."""
     _attention_checks("attention_prefill", q, k_cache, v_cache, block_table, nh, nkv, hd, seq_slot, seq_start, seq_new, cu_new)
     B = seq_slot.shape[0]
     _need(seq_start.shape == (B,) and seq_new.shape == (B,) and cu_new.shape == (B + 1,),
           "attention_prefill: per-sequence arrays differ in length")
     out = torch.empty_like(q)
-    library.call(attention_lib(hd), "palm_attention_prefill_wide" if wide else "palm_attention_prefill", _stream(), _p(q), _p(k_cache), _p(v_cache), _p(block_table),
-                 block_table.shape[1], _p(seq_slot), _p(seq_start), _p(seq_new), _p(cu_new), B, int(max_new), nh, nkv, hd,
-                 float(scale), int(window or 0), int(bool(q_prescaled)), _p(out))
+    more = () if wide else (int(max_keys), int(halves))
+    library.call(attention_lib(hd), "palm_attention_prefill_wide" if wide else "palm_attention_prefill_in", _stream(), _p(q), _p(k_cache), _p(v_cache),
+                 _p(block_table), block_table.shape[1], _p(seq_slot), _p(seq_start), _p(seq_new), _p(cu_new), B, int(max_new), nh, nkv, hd,
+                 float(scale), int(window or 0), int(bool(q_prescaled)), *more, _p(out))
     return out
 
 
@@ -982,9 +988,9 @@ def wide_prompt_attention(starts, counts, nh: int, nkv: int) -> bool:
     blocks, pages = tiles_and_pages(16)
     wide_us = 9.2 + max(5 + 1.35 * longest, (9.6 * blocks + 1.61 * pages) / COMPUTE_UNITS)
     blocks, pages = tiles_and_pages(8)
-    heads = min(G, 8)
-    launched = nkv * -(-G // heads) * -(-max(counts) // (16 * (8 // heads))) * len(counts)
-    if launched <= COMPUTE_UNITS or len(counts) == 1 and launched <= 448:       # as palm_attention_prefill takes halves
+    if attention_lib(128).palm_attention_prefill_halves(len(counts), max(counts), max(s + n for s, n in zip(starts, counts)), nh, nkv, 0) == 2:
+        heads = min(G, 8)
+        launched = nkv * -(-G // heads) * -(-max(counts) // (16 * (8 // heads))) * len(counts)
         in_turn = longest
         if launched > COMPUTE_UNITS:        # the last of the first round and the first of the second
             in_turn = max(longest, 2 * (starts[0] + counts[0] * (1 - COMPUTE_UNITS / launched)) / PAGE_TOKENS)
@@ -1014,14 +1020,14 @@ def attention(q, k_cache, v_cache, block_table, ctx, nh: int, nkv: int, hd: int,
     if q_prescaled:
         _need(mfma_attention_serves(q, hd) and not ctx.is_decode, "attention: only the prompt kernel takes scaled queries")
         return attention_prefill(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new,
-                                 ctx.max_new, nh, nkv, hd, scale, window, q_prescaled=True, wide=wide())
+                                 ctx.max_new, nh, nkv, hd, scale, window, q_prescaled=True, wide=wide(), max_keys=ctx.max_total)
     if mfma_attention_serves(q, hd):
         if ctx.is_decode:
             n_slices = slices_of_step(ctx, nh, nkv, window)
             return attention_decode(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, nh, nkv, hd, scale,
                                     window, n_slices)
         return attention_prefill(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new,
-                                 ctx.max_new, nh, nkv, hd, scale, window, wide=wide())
+                                 ctx.max_new, nh, nkv, hd, scale, window, wide=wide(), max_keys=ctx.max_total)
     return attention_exact(q, k_cache, v_cache, block_table, ctx.seq_slot, ctx.seq_start, ctx.seq_new, ctx.cu_new,
                            ctx.max_new, nh, nkv, hd, scale, window)
 

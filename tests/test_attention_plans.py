@@ -1,0 +1,25 @@
+"""Which of its builds the prompt attention takes for a launch, which is known without running it."""
+
+import pytest
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("n_seqs,max_new,max_keys,nh,nkv,window,halves", [
+    (1, 1, 64, 32, 8, 0, 1), (1, 320, 320, 32, 8, 0, 1), (1, 321, 321, 32, 8, 0, 2), (1, 20, 5000, 32, 8, 0, 2),        # few pages, many
+    (1, 1024, 1024, 32, 8, 0, 2), (1, 1792, 1792, 32, 8, 0, 2), (1, 1793, 1793, 32, 8, 0, 1), (1, 1024, 1024, 40, 8, 0, 1),   # up to 448 blocks
+    (1, 1792, 2792, 32, 8, 0, 2), (1, 1792, 3292, 32, 8, 0, 1), (1, 1100, 5000, 32, 8, 0, 1),       # a second round as long as the first
+    (1, 1024, 5000, 32, 8, 0, 2), (4, 250, 250, 32, 8, 0, 1), (4, 250, 550, 32, 8, 0, 2), (4, 512, 512, 32, 8, 0, 1),
+    (1, 1300, 1300, 32, 8, 64, 1), (1, 1300, 1300, 32, 8, 512, 1), (1, 1300, 1300, 32, 8, 1300, 2),  # windows: the second round is no shorter
+    (1, 64, 2064, 32, 8, 64, 1), (1, 64, 2064, 32, 8, 128, 2), (1, 1000, 1000, 32, 8, 128, 1), (1, 1000, 3000, 32, 8, 2 ** 31 - 1, 2),
+    (1, 300, 0, 32, 8, 0, 1), (1, 400, 0, 32, 8, 0, 2)])                                               # the keys not known: the new ones count
+def test_prompt_attention_takes_halves_where_a_block_has_many_pages_to_itself(hd, n_seqs, max_new, max_keys, nh, nkv, window, halves):
+    from palm_infra_amd.kernels import ops
+    assert ops.attention_lib(hd).palm_attention_prefill_halves(n_seqs, max_new, max_keys, nh, nkv, window) == halves
+
+
+def test_prompt_attention_of_other_head_sizes_has_no_halves():
+    from palm_infra_amd.kernels import ops
+    lib = ops.attention_lib(80)
+    assert lib.palm_attention_prefill_halves(1, 1000, 1000, 32, 8, 0) == 1
+    assert lib.palm_attention_prefill_in(None, None, None, None, None, 1, None, None, None, None, 1, 1, 1, 1, 80, 1.0, 0, 0, 1, 2, None) != 0
+    assert "halves=2" in lib.palm_last_error().decode()

@@ -620,6 +620,21 @@ def test_attention_of_few_blocks_takes_pages_by_halves(ops, nh, nkv, hd, window)
         assert torch.isfinite(got).all() and torch.allclose(got, ref, atol=2e-2), (lens, float((got - ref).abs().max()))
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (40, 8, 64), (6, 3, 64), (3, 3, 128)])
+@pytest.mark.parametrize("prescaled", [True, False])
+@pytest.mark.parametrize("halves", [1, 2])
+def test_attention_by_one_half_and_by_two_takes_nothing_from_beyond_a_sequence(ops, nh, nkv, hd, prescaled, halves):
+    """Both builds of the prompt kernel by name, whatever the rule would take: few blocks and many, pages that hold what earlier owners left."""
+    def fn(q, kc, vc, table, slots, starts, news, cu, max_new, nh_, nkv_, hd_, scale, window):
+        qs = (q.float() * ops.prefill_q_scale(hd, BF16, scale)).to(BF16) if prescaled else q
+        return ops.attention_prefill(qs, kc, vc, table, slots, starts, news, cu, max_new, nh, nkv, hd, scale, window, q_prescaled=prescaled, halves=halves)
+    for window in (None, 70):
+        for lens in ([(1, 1)], [(64, 64)], [(300, 44)], [(64, 64), (65, 1), (130, 70), (7, 7), (200, 17)], [(1100, 1100)], [(2304, 300), (70, 70)], [(2100, 2048)]):
+            got, ref = _attention_case(ops, fn, BF16, nh, nkv, hd, lens, window, seed=len(lens) + hd, poison=True)
+            # (rounded queries of the prescaled kind: as in the tests above)
+            assert torch.isfinite(got).all() and torch.allclose(got, ref, atol=3e-2 if prescaled else 2e-2), (lens, window, float((got - ref).abs().max()))
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (4, 2, 64), (6, 1, 80)])
 def test_attention_mfma_long_sequences(ops, nh, nkv, hd):
     """The measured lengths and beyond: a 2,048-token prompt (32 pages, query tiles paired from both ends, a
