@@ -968,14 +968,14 @@ def attention_prefill(q, k_cache, v_cache, block_table, seq_slot, seq_start, seq
 def wide_prompt_attention(starts, counts, nh: int, nkv: int) -> bool:
     """Whether a step's prompts (``counts`` new tokens behind ``starts`` earlier ones) are sooner through the kernel whose waves hold 64
     columns.  Both kernels' times in microseconds from the pages that their blocks walk over: the wide one has a block of 16 units (one
-    head's 16 queries) a compute unit, some 9 us of start and end that nothing hides, and 1.6 us a page with all units at work; the other two blocks
-    of eight units, 2 us a page each, or, where its blocks are few, one of two halves that take 1.9 us for two pages (then the other is the
-    sooner one but for second rounds of long blocks: 1,100 behind 2,000 79 83, 1,000 behind 3,000 77 102, 1,024 behind 30,000 458 675).
-    Measured (32 heads of 8 unless said otherwise; the other's time and this one's): 2,048 tokens 51 58, 3,072 82 82, 3,500 106 97, 4,096
-    142 125, 13,331 1,281 1,134, four of 2,048 151 156, four of 3,072 318 312; 40 heads of 8 (five of eight units used, fifteen of sixteen)
-    1,024 tokens 31 38, 2,048 87 67, 8,192 939 590, five of 45 to 2,000 125 106; 64 heads of 8 3,072 150 157, 4,096 253 241; 16 heads of 8
-    4,096 92 102, 8,192 266 224.  The numbers below are fitted to 64 such steps: the slower one is taken at four of them (16 heads of 8 at
-    4,096 tokens by 11 %, 8 of 8 at 8,192 by 8 %, two by less than 3 %)."""
+    head's 16 queries) a compute unit, some 12 us of start and end that nothing hides, and 1.45 us a page with all units at work; the other two blocks
+    of eight units, 1.25 us a page alone and 1.65 to 1.8 beside another one, or, where its blocks are few and their pages many, one of two halves that
+    take 1.74 us for two pages (then the pages of the last block of the first round and of the first of the second come one after the other).
+    Measured (32 heads of 8 unless said otherwise; the other's time and this one's): 2,048 tokens 54 58, 3,000 80 82, 3,500 108 96, 4,096
+    141 122, 13,331 1,250 1,124, four of 2,048 156 159, four of 3,072 302 295, 1,000 behind 3,000 71 99, 1,024 behind 30,000 484 680; 40 heads of 8
+    (five of eight units used, fifteen of sixteen) 1,300 tokens 41 45, 2,048 78 61, 8,192 937 593; 64 heads of 8 2,048 78 72; 16 heads of 8 4,096 93
+    104, 8,192 263 223; 8 of 8 8,192 179 194.  The numbers below are fitted to 450 such steps: the slower one is taken at 15 of them by more than
+    2 %, this one at four of those (3,000 tokens and 24, 48 or 64 heads of 8 by 2 to 5, eight of 512 and 40 heads by 4)."""
     G = nh // nkv
 
     def tiles_and_pages(units):
@@ -984,18 +984,25 @@ def wide_prompt_attention(starts, counts, nh: int, nkv: int) -> bool:
         tiles = [-(-n // rows) for n in counts]
         # the mean tile of a sequence ends half way through its new tokens, in the middle of a page
         return groups * sum(tiles), groups * sum(t * ((s + (n + rows) / 2) / PAGE_TOKENS + 0.5) for t, s, n in zip(tiles, starts, counts))
-    longest = max((s + n + PAGE_TOKENS - 1) // PAGE_TOKENS for s, n in zip(starts, counts))
+    totals = [s + n for s, n in zip(starts, counts)]
+    longest = (max(totals) + PAGE_TOKENS - 1) // PAGE_TOKENS
     blocks, pages = tiles_and_pages(16)
-    wide_us = 9.2 + max(5 + 1.35 * longest, (9.6 * blocks + 1.61 * pages) / COMPUTE_UNITS)
-    blocks, pages = tiles_and_pages(8)
-    if attention_lib(128).palm_attention_prefill_halves(len(counts), max(counts), max(s + n for s, n in zip(starts, counts)), nh, nkv, 0) == 2:
+    wide_us = 12.3 + max(1.44 * longest, (11 * blocks + 1.45 * pages) / COMPUTE_UNITS)
+    if attention_lib(128).palm_attention_prefill_halves(len(counts), max(counts), max(totals), nh, nkv, 0) == 2:
         heads = min(G, 8)
         launched = nkv * -(-G // heads) * -(-max(counts) // (16 * (8 // heads))) * len(counts)
         in_turn = longest
         if launched > COMPUTE_UNITS:        # the last of the first round and the first of the second
             in_turn = max(longest, 2 * (starts[0] + counts[0] * (1 - COMPUTE_UNITS / launched)) / PAGE_TOKENS)
-        return wide_us < 9 + 0.95 * in_turn
-    other_us = 6.8 + max(1.57 * longest, (2.2 * blocks + 1.95 * pages) / (2 * COMPUTE_UNITS))
+        return wide_us < 10.9 + 0.87 * in_turn
+    blocks, pages = tiles_and_pages(8)
+    slots = 2 * COMPUTE_UNITS
+    # The longest block shares its unit while the others last; where two sequences are the longest and all blocks run at once, to its end.  (One
+    # sequence's blocks run at once with the shortest beside the longest, or the longest first.)
+    shared = min(longest, pages / slots) if len(counts) > 1 else 0.0
+    if COMPUTE_UNITS < blocks <= slots and sum(10 * t >= 9 * max(totals) for t in totals) > 1:
+        shared = longest
+    other_us = 9.5 + max(1.25 * longest + 0.4 * shared, (4.9 * blocks + 1.79 * pages) / min(max(blocks, COMPUTE_UNITS), slots))
     return wide_us < other_us
 
 

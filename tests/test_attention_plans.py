@@ -23,3 +23,13 @@ def test_prompt_attention_of_other_head_sizes_has_no_halves():
     assert lib.palm_attention_prefill_halves(1, 1000, 1000, 32, 8, 0) == 1
     assert lib.palm_attention_prefill_in(None, None, None, None, None, 1, None, None, None, None, 1, 1, 1, 1, 80, 1.0, 0, 0, 1, 2, None) != 0
     assert "halves=2" in lib.palm_last_error().decode()
+
+
+@pytest.mark.parametrize("starts,counts,nh,nkv,wide", [
+    ([0], [13331], 32, 8, True), ([0], [3500], 32, 8, True), ([0], [2500], 32, 8, False), ([8000], [2048], 32, 8, True), ([3000], [1000], 32, 8, False),
+    ([0], [4096], 16, 8, False), ([0], [8192], 16, 8, True), ([0], [4096], 16, 2, False), ([0], [8192], 8, 8, False), ([0], [13331], 8, 8, True),
+    ([0], [2048], 40, 8, True), ([0], [1300], 40, 8, False), ([0], [4096], 24, 8, True),
+    ([0] * 3, [3000, 1000, 100], 8, 8, False), ([0] * 3, [3000, 1000, 100], 16, 8, False), ([0] * 2, [4096] * 2, 8, 8, True), ([3000] * 6, [100] * 6, 64, 8, True)])
+def test_wide_prompt_attention_is_taken_where_it_was_measured_to_be_sooner(starts, counts, nh, nkv, wide):
+    from palm_infra_amd.kernels import ops
+    assert ops.wide_prompt_attention(starts, counts, nh, nkv) == wide
