@@ -52,15 +52,21 @@ ARCH = "gfx950"
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-fno-gpu-rdc",
          # packed 32-bit float instructions are kept out of generated code on purpose
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-         # a kernel's first arguments (pointers and sizes, up to 16 registers of them) are in scalar registers when its waves
-         # start, not behind a read of memory: a decode step of 220 to 290 launches 0.6 % faster (Qwen3-8B, 8 sequences 3,669
-         # and 3,645 us; Nirotar, 6 sequences 1,560 and 1,544).  Structs among the arguments end the run: they stand last.
-         "-mllvm", "-amdgpu-kernarg-preload-count=16",
          "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option"]
-# Sources that are compiled without some of them.  The large tiles run for hundreds of microseconds, a launch's start is nothing to
-# them, and their loop comes out a little slower behind preloaded arguments (gated, 4,309 rows 615.6 us and 613.5 without, 13,331
-# rows 1,872 and 1,860; a prompt of 13,331 tokens against the code without preloading 1.022 and 1.042 times as fast).
-FLAGS_LEFT_OUT = {"linear_big.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
+# A kernel's first arguments (pointers and sizes, up to 16 registers of them) are in scalar registers when its waves start, not behind a
+# read of memory: a decode step of 220 to 290 launches some 0.6 % faster (Qwen3-8B, 8 sequences 3,669 and 3,645 us; Nirotar, 6 sequences
+# 1,560 and 1,544).  Structs among the arguments end the run: they stand last.
+PRELOADED_ARGUMENTS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+# Without it: the large tiles run for hundreds of microseconds, a launch's start is nothing to them, and their loop comes out a little slower
+# behind preloaded arguments (gated, 24,576 x 4,096, 13,331 rows 1,861 us and 1,851 without, the quarters of 30 pairs 4 to 13 apart; 4,309 rows 613 and
+# 608; products that are not gated the same).  The experts' grouped products, the same walk, do not differ (32 experts, 2,900 rows 473 and 471, 64 of
+# 1,408, 3,000 rows 447 and 449).
+NOT_PRELOADED = ("linear_big.hip",)
+
+
+def flags_of(source: str) -> list[str]:
+    return FLAGS if source in NOT_PRELOADED else FLAGS + PRELOADED_ARGUMENTS
+
 
 CORE_SOURCES = ["elementwise.hip", "linear.hip", "rope_store.hip", "attention_simple.hip", "sampling.hip",
                 "linear_mfma.hip", "linear_ring.hip", "linear_ring_many.hip", "linear_wide.hip", "linear_wide_store_32.hip", "linear_wide_store_64.hip",
@@ -133,10 +139,10 @@ def _existing(names) -> list[str]:
 
 def _digest(sources, defines) -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + sorted(defines)).encode())
+    h.update(" ".join(sorted(defines)).encode())
     own = {h for s in sources for h in OWN_HEADERS.get(s, ())}
     for name in sorted(_existing(list(sources) + HEADERS + sorted(own))):
-        h.update(" ".join([name, *FLAGS_LEFT_OUT.get(name, ())]).encode())
+        h.update(" ".join([name, *(flags_of(name) if name in sources else ())]).encode())
         h.update((CSRC / name).read_bytes())
     return h.hexdigest()[:16]
 
@@ -173,8 +179,7 @@ def _compile(name: str, sources, defines, force: bool) -> Path:
 
     def one(src: str) -> Path:
         obj = work / (src.replace(".hip", "") + ".o")
-        left_out = FLAGS_LEFT_OUT.get(src, ())
-        cmd = [hipcc, *[f for f in FLAGS if f not in left_out], *[f"-D{d}" for d in defines], "-c", str(CSRC / src), "-o", str(obj)]
+        cmd = [hipcc, *flags_of(src), *[f"-D{d}" for d in defines], "-c", str(CSRC / src), "-o", str(obj)]
         r = subprocess.run(cmd, capture_output=True, text=True, env=env)
         if r.returncode != 0:
             raise KernelBuildError(f"hipcc failed on {src}:\n{r.stderr[-4000:]}")

@@ -176,3 +176,16 @@ def test_a_rebuilt_library_removes_its_own_older_builds_only(tmp_path):
         (tmp_path / n).write_text("")
     remove_older_builds(tmp_path / names[1], "sink_attention")
     assert sorted(p.name for p in tmp_path.iterdir()) == sorted(names[1:])
+
+
+def test_an_option_that_comes_in_two_words_reaches_every_source_whole(monkeypatch):
+    from palm_infra_amd.kernels import library
+    option = ["-mllvm", "-another-option"]
+    before = library._digest(["linear_big.hip"], ())
+    monkeypatch.setattr(library, "FLAGS", library.FLAGS + option)
+    for source in ("linear_big.hip", "linear.hip"):
+        flags = library.flags_of(source)
+        assert any(flags[i:i + 2] == option for i in range(len(flags)))
+        # (every -mllvm has its option behind it)
+        assert all(flags[i + 1].startswith("-a") for i, f in enumerate(flags) if f == "-mllvm")
+    assert library._digest(["linear_big.hip"], ()) != before

@@ -14,9 +14,7 @@ PRODUCT, SLOTS, RESULT, OPERAND = "v_mfma_f32_16x16x32_bf16", 4, 1 + 4 * 4, 2
 
 
 def assembly(source, defines, out):
-    left_out = ["-shared", "-fPIC"]
-    cmd = [library._hipcc(), *[f for f in library.FLAGS if f not in left_out], *[f"-D{d}" for d in defines], "--cuda-device-only", "-S",
-           str(library.CSRC / source), "-o", str(out)]
+    cmd = [library._hipcc(), *library.flags_of(source), *[f"-D{d}" for d in defines], "--cuda-device-only", "-S", str(library.CSRC / source), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, text=True)
     return out.read_text()
 
