@@ -141,7 +141,7 @@ PALM_API int palm_causal_conv(hipStream_t stream, const void* x, int dtype, int 
 
 // ---- the scan ---------------------------------------------------------------------------------------
 // A channel's row of S is spread over a group of G lanes (G a power of two, at most 64): lane j of the group holds the PER states
-// from j PER on; a block of four waves serves 256 / G channels.  The block walks over a sequence's new tokens a tile at a time,
+// from j PER on, of 128 states and more j, j + G, ..; a block of four waves serves 256 / G channels.  The block walks over a sequence's new tokens a tile at a time,
 // in three phases with a barrier between them:
 //   in     all threads bring the tile's inputs into LDS with reads that follow the memory's rows: B_t and C_t (the
 //          same for all channels), and for the block's channels the step size softplus(dtl_t + bias) and its product
@@ -278,6 +278,11 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     __shared__ float2 in_s[SCAN_TILE][CH];             // the step size, and times u_t
     __shared__ float y_s[SCAN_TILE][CH];
     const int j = threadIdx.x % G, ch = threadIdx.x / G;
+    // The states of lane j.  Side by side, a token's B and C come in one read of LDS; but the lanes' reads of S and of a_log then lie PER numbers
+    // apart, and with rows of 128 states and more those are most of a single token's time: side by side and G apart, us, one token each of 16
+    // and 64 sequences, 2,048 channels x 128 states 19.0 14.4 and 60.0 49.7, 1,024 x 256 19.7 16.5 and 66.2 62.3; 200 of 200 states (2,048)
+    // 422 442; prompts the same to 2 %.
+    auto state_of = [&](int k) { return NP >= 128 ? j + k * G : j * PER + k; };
     const int c0 = blockIdx.x * CH, b = blockIdx.y;
     const int c = c0 + ch;
     const bool mine = c < channels;
@@ -289,7 +294,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     ScanDecay A[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        const int n = j * PER + k;
+        const int n = state_of(k);
         S[k] = n < n_state ? sp[n] : 0.f;
         A[k] = ScanDecay::of(n < n_state ? -expf(a_log[(size_t)cc * n_state + n]) : 0.f);
     }
@@ -366,7 +371,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
             float y = 0.f;
 #pragma unroll
             for (int k = 0; k < PER; ++k) {
-                const float2 v = bc_s[ti][j * PER + k];
+                const float2 v = bc_s[ti][state_of(k)];
                 S[k] = fmaf(A[k].over(in.x), S[k], in.y * v.x);              // beyond the state size A, B and C are zero
                 y = fmaf(S[k], v.y, y);
             }
@@ -402,7 +407,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void selective_scan_kernel(
     if (mine && n_new > 0) {
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const int n = j * PER + k;
+            const int n = state_of(k);
             if (n < n_state) sp[n] = S[k];
         }
     }
