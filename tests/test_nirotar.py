@@ -906,6 +906,35 @@ def test_a_long_prompt_takes_smaller_pieces_where_the_window_has_no_room(tmp_pat
 
 
 @gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_long_prompts_go_in_pieces_of_five_windows_or_of_two(tmp_path, dtype):
+    """A window at which the two sizes differ (2,600 and 1,040 tokens): several sequences fall back together where their pages do not fit
+    at once, one goes on in large pieces, and the tokens of either way are the plain implementation's."""
+    from palm_infra_amd.engine import Engine, StepEntry
+    raw = S.model(90, 32, 1e-6, [S.layer(S.attention(4, 2, 12, 20, 0.3, window=520, rot=(8, 60.0, (4.0, 1.0, 4.0, 128))))])
+    path = S.write_model(raw, 121, tmp_path / "model", dtype)
+    cfg, w = P.read_model(path)
+    a, b, c = S.prompts(raw, [1300, 1290, 2700], seed=37)
+    refs = {len(ids): P.forward(cfg, w, ids) for ids in (a, b, c)}
+    for pages, pieces in ((36, {2: [[1040, 1040], [260, 250]]}), (44, {2: [[1300, 1290]], 1: [[2600], [100]]})):
+        eng = Engine.from_dir(path, dtype=dtype, max_tokens=64 * pages)
+        assert (eng.step_tokens_per_seq, eng.step_tokens_least) == (2600, 1040)
+        steps = []
+        run = eng._run
+        eng._run = lambda entries: steps.append([len(e.tokens) for e in entries]) or run(entries)
+        for prompts in ((a, b), (c,))[:len(pieces)]:
+            del steps[:]
+            slots = [eng.open() for _ in prompts]
+            want = [[0, 519, 520, 1039, 1040, len(ids) - 1] for ids in prompts]
+            got = eng.step([StepEntry(slot, ids, at) for slot, ids, at in zip(slots, prompts, want)])
+            assert steps == pieces[len(prompts)], (pages, steps)
+            assert_close(got, torch.cat([refs[len(ids)][at] for ids, at in zip(prompts, want)]), dtype, f"{pages} pages")
+            for slot in slots:
+                eng.close(slot)
+        eng.cache.check()
+
+
+@gpu
 @pytest.mark.parametrize("name", ["A", "D"])
 def test_recorded_and_launched_steps_agree(tmp_path_factory, name):
     """Decode steps replayed from a HIP graph against the same steps launched kernel by kernel, several replays with other

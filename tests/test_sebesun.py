@@ -574,6 +574,25 @@ def test_selective_scan_at_the_ends_of_its_step_sizes_and_gates():
 
 
 @gpu
+def test_selective_scan_softplus_and_silu_to_the_last_places():
+    """One token from an empty state with inputs of one is softplus(step) times silu(gate): both within some halves of the last place of
+    64 bits, between the points where the library's functions take over."""
+    from palm_infra_amd.kernels import ops
+    small = torch.logspace(-7, 0, 500)
+    x = torch.cat([torch.linspace(-86.9, 86.9, 6001), small, -small])
+    C, one = len(x), torch.ones(1, len(x))
+    for gates in (False, True):
+        dtl, z = (one, x[None]) if gates else (x[None], one)
+        got = ops.selective_scan(one.cuda(), torch.cat([one, z], 1).cuda(), torch.ones(1, 2).cuda(), 0, 1, dtl.contiguous().cuda(), torch.zeros(C).cuda(),
+                                 torch.zeros(C, 1).cuda(), torch.zeros(C).cuda(), torch.zeros(1, C, 1).cuda(), _step_context([0], [1])).double().cpu()[0]
+        step, gate = dtl[0].double(), z[0].double()
+        want = (step.clamp(min=0) + torch.log1p(torch.exp(-step.abs()))) * gate / (1 + torch.exp(-gate))
+        # 2.3 and 3.1 halves of a place (2^-24) were measured for the two functions over all such arguments, one more is the last product's
+        worst = float(((got - want) / want).abs().max()) * 2 ** 24
+        assert worst <= 2.3 + 3.1 + 1 + 0.5, (gates, worst)
+
+
+@gpu
 @pytest.mark.parametrize("dk,dv", [(12, 28), (40, 72)])      # the second pair is one that the matrix-core kernel takes in bfloat16
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_differential_attention_kernel_far_keys_page_borders_and_the_causal_edge(dtype, dk, dv):
