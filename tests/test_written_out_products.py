@@ -116,3 +116,16 @@ def test_wide_attention_keeps_its_products_distances(attention_of_heads_of_128, 
     code, following = kernel(attention_of_heads_of_128, f"attention_prefill_wide_kernelILb{prescaled}E")
     assert sum(one.written_out for one in code) == 4 * 34
     assert too_near(code, following) == []
+
+
+@pytest.mark.parametrize("prescaled", [1, 0])
+def test_wide_attention_waits_for_loads_where_it_says_so_and_keeps_nothing_in_memory(attention_of_heads_of_128, prescaled):
+    """Between the first product and the last the loads into LDS, which the compiler does not know, stay on their way: all of them are waited
+    for behind a read of the page table only, once in 64 pages."""
+    name = f"attention_prefill_wide_kernelILb{prescaled}E"
+    code, _ = kernel(attention_of_heads_of_128, name)
+    assert not any(one.name.startswith("scratch_") for one in code)
+    products = [i for i, one in enumerate(code) if one.written_out]
+    waits = [i for i, one in enumerate(code) if one.name == "s_waitcnt" and "vmcnt" in one.text and products[0] < i < products[-1]]
+    of_the_table = [i for i in waits if "vmcnt(0)" in code[i].text and code[i - 1].name == "global_load_dword"]
+    assert len(of_the_table) <= 1 and ["vmcnt(8)" in code[i].text for i in waits if i not in of_the_table] == [True]
