@@ -1533,11 +1533,12 @@ __global__ __launch_bounds__(HALVES * PF_THREADS) PF_WAVES_PER_SIMD void attenti
 // reads or loads stand at least three products apart (four waves of 8 clocks of LDS, or of 16 of the load's way, each).
 // The maxima decide by one vote, as above, whether any column has to be masked or its reference moved; that is settled aside.
 //
-// Measured, us, the kernel above and this one: 32 heads of 8, 13,331 tokens 1,281 and 1,134 (1.28 PFLOP/s), 2,048 behind 30,720
-// 949 and 780 (1.36), 4,096 142 and 124, 2,048 51 and 58; 40 heads of 8 (the kernel above uses five of its eight units) 8,192 tokens 939 and
-// 590; in the middle of a whole prompt of 13,331, where the chip's clock is lower, 1,511 and 1,358.  A block's start and end (its first keys' way from memory, masks on its first and last page) are some 9 us that no second block
-// hides, so few pages a block, or few blocks, are better served above: ops.wide_prompt_attention.  Tried: sums of the weights by dot
-// products instead of a row of ones on the matrix cores (13,331 tokens 1,200 us); exponentials written out too (1,156).
+// Measured, us, the kernel above and this one: 32 heads of 8, 13,331 tokens 1,250 and 1,100 (1.32 PFLOP/s), 2,048 behind 30,720
+// 911 and 757 (1.41), 4,096 141 and 120, 2,048 54 and 58; 40 heads of 8 (the kernel above uses five of its eight units) 8,192 tokens 937 and
+// 576; in the middle of a whole prompt of 13,331, where the chip's clock is lower, 1,511 and 1,380 (1.06 PFLOP/s).  A block's start and end (its
+// first keys' way from memory, masks on its first and last page) are some 12 us that no second block hides, so few pages a block, or few
+// blocks, are better served above: ops.wide_prompt_attention.  Tried: sums of the weights by dot products instead of a row of ones on the
+// matrix cores (13,331 tokens 1,134 -> 1,200 us); exponentials written out too (1,156); all loads waited for in every page (1,113 where this takes 1,100).
 constexpr bool PF_WIDE = PF_DMA && HD == 128;
 constexpr int WIDE_UNITS = 4, WIDE_STAGES = 4;
 

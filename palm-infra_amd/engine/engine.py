@@ -77,7 +77,8 @@ class Engine:
         self._graph_pool_handle = None
         # A windowed group gives pages back only between steps, so long prompts go through it in pieces: of five windows, or of
         # two where the group has no room for more.  (Every piece reads all weights again: a Nirotar prompt of 2,900 tokens, 4,096
-        # wide, in pieces of two windows 11.1 ms, in one 8.5.)
+        # wide, in pieces of two windows 11.3 ms, in one 8.6, of 12,000 43.6 and 37.3; Biguzen, Vovalix, Pazilorn, Matalix and Nirotar,
+        # windows of 1,024 and 1,088, 2,048 and 4,096 wide, 2,900 to 12,000 tokens and three prompts at once: 2 to 27 % sooner.)
         windows = [g.table.window for g in self.cache.paged_groups if g.table.window]
         self.step_tokens_per_seq = max(1024, 5 * max(windows)) if windows else None
         self.step_tokens_least = max(1024, 2 * max(windows)) if windows else None

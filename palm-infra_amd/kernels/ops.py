@@ -1017,6 +1017,7 @@ def attention(q, k_cache, v_cache, block_table, ctx, nh: int, nkv: int, hd: int,
     """The step's queries over the cache; picks the kernel by element type, head size and step shape.
     ``q_prescaled``: see ``attention_prefill`` (only a prompt step on the matrix cores takes such queries)."""
     def wide():
+        # (a window leaves a block few pages, which the wide kernel's start and end outweigh: not measured)
         if window or not ctx.host or not attention_lib(hd).palm_attention_prefill_wide_serves():
             return False
         key = ("wide_prompt_attention", nh, nkv)
