@@ -55,7 +55,9 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-fno-gpu-rdc",
          "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option"]
 # A kernel's first arguments (pointers and sizes, up to 16 registers of them) are in scalar registers when its waves start, not behind a
 # read of memory: a decode step of 220 to 290 launches some 0.6 % faster (Qwen3-8B, 8 sequences 3,669 and 3,645 us; Nirotar, 6 sequences
-# 1,560 and 1,544).  Structs among the arguments end the run: they stand last.
+# 1,560 and 1,544).  Structs among the arguments end the run: they stand last.  Not every kernel gains: decode attention over rows in bfloat16
+# takes 24.0 us with it and 23.2 without (Qwen3-14B, 16 sequences: 6,584 and 6,546 us a step), over planes of partial sums less (8B, 8
+# sequences: 3,650 and 3,666); both are of one source.
 PRELOADED_ARGUMENTS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 # Without it: the large tiles run for hundreds of microseconds, a launch's start is nothing to them, and their loop comes out a little slower
 # behind preloaded arguments (gated, 24,576 x 4,096, 13,331 rows 1,861 us and 1,851 without, the quarters of 30 pairs 4 to 13 apart; 4,309 rows 613 and
