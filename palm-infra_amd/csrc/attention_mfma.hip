@@ -26,6 +26,8 @@
 #include "attention_api.h"
 #include "lds_stage.h"
 
+#include <type_traits>
+
 #ifndef PALM_HEAD_DIM
 #error "compile with -DPALM_HEAD_DIM=<head size>"
 #endif
@@ -716,6 +718,49 @@ PALM_API int palm_attention_decode_fused(hipStream_t stream, const void* qkv, in
         launch_merge(stream, work, n_slices, n_seqs, nh, seq_start, window, (bf16_t*)out);
         PALM_LAUNCHED();
     }
+    return 0;
+}
+
+// ---- decode cut by pages ------------------------------------------------------------------------------
+#include "attention_decode_pages.h"
+
+PALM_API int palm_attention_decode_pages_serves(int nh, int nkv, int n_seqs) {
+    return PAGES_SERVE_HEAD && nkv > 0 && nkv <= 65535 && nh / nkv <= DP_HEADS && n_seqs <= DP_SEQS;
+}
+
+// What `work` has to hold, in floats.
+PALM_API int palm_attention_decode_pages_work(int nh, int nkv) { return 2 * max(DP_BLOCKS, nkv) * (nh / nkv) * WORK_STRIDE; }
+
+// palm_attention_decode_fused by the kernel that is cut by pages.  arrivals: n_seqs * nh counters, zero before the call and after it; calls
+// that overlap in time need counters and a workspace of their own.
+PALM_API int palm_attention_decode_pages(hipStream_t stream, const void* qkv, int qkv_is_planes, int planes,
+                                         const float* q_norm_w, const float* k_norm_w, float eps, const float* cos_t,
+                                         const float* sin_t, int rotary_dim, int pairing, int write_cache, void* k_cache,
+                                         void* v_cache, const int* block_table, int max_pages, const int* seq_slot,
+                                         const int* seq_start, int n_seqs, int nh, int nkv, int hd, float scale,
+                                         int window, float* work, int* arrivals, void* out) {
+    PALM_CHECK(hd == HD, "attention_decode_pages: this library was built for head size %d, not %d", HD, hd);
+    PALM_CHECK((cos_t == nullptr) == (sin_t == nullptr), "attention_decode_pages: cos and sin tables come together");
+    PALM_CHECK(palm_attention_decode_fused_serves(cos_t ? rotary_dim : 0, pairing),
+               "attention_decode_pages: head size %d with rotation over %d (pairing %d) is not served", HD, rotary_dim, pairing);
+    PALM_CHECK((q_norm_w == nullptr) == (k_norm_w == nullptr), "attention_decode_pages: q and k norm weights come together");
+    PALM_CHECK(n_seqs >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0, "attention_decode_pages: seqs=%d heads=%d kv=%d", n_seqs, nh, nkv);
+    PALM_CHECK(palm_attention_decode_pages_serves(nh, nkv, n_seqs), "attention_decode_pages: head size %d, %d heads of %d, %d sequences are not served",
+               HD, nh, nkv, n_seqs);
+    PALM_CHECK(window >= 0 && max_pages > 0 && max_pages < (1 << 24) / DP_SEQS, "attention_decode_pages: window=%d max_pages=%d", window, max_pages);
+    PALM_CHECK(planes >= 1 && (qkv_is_planes || planes == 1), "attention_decode_pages: %d planes of whole rows", planes);
+    if (n_seqs == 0) return 0;
+    PALM_CHECK(work && arrivals, "attention_decode_pages: a workspace and counters are needed");
+    const size_t plane_stride = (size_t)n_seqs * (nh + 2 * nkv) * HD;
+#define PALM_PAGES(TIN, P) attention_decode_pages_kernel<TIN, P><<<dim3(max(1, DP_BLOCKS / nkv), nkv), DP_THREADS, 0, stream>>>( \
+        (const TIN*)qkv, planes, plane_stride, q_norm_w, k_norm_w, eps, cos_t, sin_t, write_cache, (bf16_t*)k_cache, \
+        (bf16_t*)v_cache, block_table, max_pages, seq_slot, seq_start, n_seqs, nh, nkv, scale * LOG2E, window, work, arrivals, (bf16_t*)out)
+    if (!qkv_is_planes) PALM_PAGES(bf16_t, 1);
+    else if (planes == 1) PALM_PAGES(float, 1);
+    else if (planes == 2) PALM_PAGES(float, 2);
+    else PALM_PAGES(float, 0);
+#undef PALM_PAGES
+    PALM_LAUNCHED();
     return 0;
 }
 

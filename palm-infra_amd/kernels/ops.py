@@ -802,6 +802,11 @@ _ATTENTION_SIGNATURES = {
     "palm_attention_decode_fused": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
                                     c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int,
                                     c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p],
+    "palm_attention_decode_pages": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
+                                    c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
+                                    c_int, c_float, c_int, c_void_p, c_void_p, c_void_p],
+    "palm_attention_decode_pages_serves": [c_int, c_int, c_int],
+    "palm_attention_decode_pages_work": [c_int, c_int],
     "palm_attention_decode_fused_serves": [c_int, c_int],
 }
 _attention_libs: dict = {}
@@ -895,13 +900,35 @@ def decode_fused_serves(qkv: torch.Tensor, hd: int, out_dtype, rotary_dim: int, 
     return bool(attention_lib(hd).palm_attention_decode_fused_serves(int(rotary_dim), int(pairing)))
 
 
+def decode_pages_serves(n_seqs: int, nh: int, nkv: int, hd: int) -> bool:
+    """Whether a decode step's attention may be cut by pages: head sizes 64 and 128, up to eight query heads a kv head, 128 sequences."""
+    return bool(attention_lib(hd).palm_attention_decode_pages_serves(nh, nkv, n_seqs))
+
+
+def decode_pages_pays(n_seqs: int, nh: int, nkv: int, hd: int, longest: int) -> bool:
+    """Whether it should be: where sequences are many or long (``longest``: the longest one, or what a recorded step is sized for).  Its
+    blocks all read until the end, but they begin some 3 us later than a slice's wave (the cut, the queries through LDS) and add their
+    pieces across dies instead of in a launch of their own.  Us by slices and by pages, head size 128, 32 heads of 8, sequences of equal
+    length or spread evenly: 8 of 2,048 20.6 19.3; 8 of 700 11.5 13.1; 12 of 64 to 2,048 19.4 16.0; 16 of 200 10.2 11.8, of 30 to 600 12.3
+    13.0, of 70 to 1,500 20.2 18.3, of 64 to 2,048 23.9 20.5, of 2,000 32.1 31.2, of 300 to 8,000 76 63; 24 of 2,000 44.3 44.6; 40 of 700 30.7
+    32.5, of 70 to 1,500 34.2 27.8; 48 of 70 to 1,500 44.0 37.9; 64 of 200 23.9 20.8, of 64 to 2,048 75.7 62.4.  With more heads a block adds more
+    pieces: 40 heads of 8, 16 of 64 to 2,048 23.8 21.4 or 24.7 25.4 by their lengths, 24 of 70 to 1,500 26.0 26.6, 32 of them 33.1 30.7; 64 heads of
+    8, 32 of them 33.2 33.1, 64 55.2 52.7.  Four up to 8,000
+    tokens 24.9 23.6, eight 36.4 31.4, of 70 to 1,500 13.4 13.8."""
+    return n_seqs * longest >= (32768 if nh <= 4 * nkv and n_seqs >= 12 else 65536) and decode_pages_serves(n_seqs, nh, nkv, hd)
+
+
 def attention_decode_fused(qkv, k_cache, v_cache, block_table, seq_slot, seq_start, nh: int, nkv: int, hd: int, scale: float,
                            window: int | None, n_slices: int, *, q_norm_w=None, k_norm_w=None, eps: float = 0.0, cos=None,
                            sin=None, rotary_dim: int = 0, pairing: int = 0, write_cache: bool = True,
-                           work: torch.Tensor | None = None) -> torch.Tensor:
+                           work: torch.Tensor | None = None, pages: bool = False, arrivals: torch.Tensor | None = None) -> torch.Tensor:
     """A decode step's attention from the joined projection's rows: qk_norm_rope_store and attention_decode in one
     launch.  qkv is [B, (nh + 2 nkv) hd] bfloat16 or float32 planes [P, B, (nh + 2 nkv) hd]; sequence b's token is
-    row b, at position seq_start[b]; cos, sin are [B, hd / 2] rows of those positions.  Returns [B, nh hd] bfloat16."""
+    row b, at position seq_start[b]; cos, sin are [B, hd / 2] rows of those positions.  Returns [B, nh hd] bfloat16.
+
+    ``pages``: by the kernel whose work is cut by pages (attention_decode_pages.h), whatever ``n_slices``, where ``decode_pages_serves``.
+    ``arrivals``: its counters, int32 [B * nh] or more, zero before the call and left zero by it, not shared by calls that may overlap in
+    time (made here if None)."""
     what = "attention_decode_fused"
     _dev(what, qkv, k_cache, v_cache, block_table, seq_slot, seq_start, q_norm_w, k_norm_w, cos, sin)
     _i32(what, block_table, seq_slot, seq_start)
@@ -925,6 +952,21 @@ def attention_decode_fused(qkv, k_cache, v_cache, block_table, seq_slot, seq_sta
         if not (tab is None or (tab.dtype == F32 and tab.shape == (B, hd // 2) and tab.is_contiguous() and rotary_dim == hd)):
             raise KernelError(f"{what}: a rotation table is float32 [{B}, {hd // 2}] over the whole head")
     out = torch.empty((B, nh * hd), dtype=BF16, device=qkv.device)
+    if pages:
+        if arrivals is None:
+            arrivals = torch.zeros((B * nh,), dtype=torch.int32, device=qkv.device)
+        _dev(what, arrivals)
+        _i32(what, arrivals)
+        if not (arrivals.is_contiguous() and arrivals.numel() >= B * nh):
+            raise KernelError(f"{what}: {arrivals.numel()} counters for {B} sequences x {nh} heads")
+        lib = attention_lib(hd)
+        work = torch.empty((lib.palm_attention_decode_pages_work(nh, nkv),), dtype=F32, device=qkv.device)
+        library.call(lib, "palm_attention_decode_pages", _stream(), _p(qkv), int(as_planes),
+                     qkv.shape[0] if as_planes else 1, _p(q_norm_w), _p(k_norm_w), float(eps), _p(cos), _p(sin),
+                     int(rotary_dim if cos is not None else 0), int(pairing), int(write_cache), _p(k_cache), _p(v_cache),
+                     _p(block_table), block_table.shape[1], _p(seq_slot), _p(seq_start), B, nh, nkv, hd, float(scale),
+                     int(window or 0), _p(work), _p(arrivals), _p(out))
+        return out
     work = _slices_workspace(what, work, B, nh, n_slices, hd, qkv.device)
     library.call(attention_lib(hd), "palm_attention_decode_fused", _stream(), _p(qkv), int(as_planes),
                  qkv.shape[0] if as_planes else 1, _p(q_norm_w), _p(k_norm_w), float(eps), _p(cos), _p(sin),

@@ -72,7 +72,8 @@ class Attention:
                 self.window, ops.slices_of_step(ctx, self.nh, self.nkv, self.window),
                 q_norm_w=self.q_norm.weight if self.q_norm else None, k_norm_w=self.k_norm.weight if self.k_norm else None,
                 eps=self.q_norm.eps if self.q_norm else 0.0, cos=cos, sin=sin, rotary_dim=rotary_dim, pairing=pairing,
-                write_cache=lc.writes)
+                write_cache=lc.writes, arrivals=lc.kv.arrivals,
+                pages=ops.decode_pages_pays(ctx.n_seqs, self.nh, self.nkv, self.hd, min(ctx.max_total, self.window or ctx.max_total)))
             return self.out(o, sink=sink)
         # a prompt's queries carry the scale (times log2 e) into their one rounding where the prompt kernel of this
         # head size takes them so: a score then leaves the matrix cores as the exponent of its weight

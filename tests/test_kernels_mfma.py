@@ -757,7 +757,7 @@ def test_attention_mfma_refuses_what_it_was_not_built_for(ops):
 
 # ---- decode attention that starts from the joined projection's rows -----------------------------------
 
-def _fused_case(ops, nh, nkv, hd, lengths, n_slices, planes, window=None, norm=True, rotate=True, seed=0, poison=False):
+def _fused_case(ops, nh, nkv, hd, lengths, n_slices, planes, window=None, norm=True, rotate=True, seed=0, poison=False, **how):
     """Sequences whose last token is new: its q/k/v row goes (a) through qk_norm_rope_store and attention_decode and
     (b) through attention_decode_fused, each on its own copy of a cache that holds the earlier tokens and stale
     values elsewhere.  Returns both outputs and both pairs of caches."""
@@ -796,7 +796,7 @@ def _fused_case(ops, nh, nkv, hd, lengths, n_slices, planes, window=None, norm=T
     apart = torch.cat([qkv, torch.zeros_like(qkv)]) if planes == 1 else qkv          # the pass alone takes two planes or more
     q = ops.qk_norm_rope_store(apart, nh, nkv, hd, pos, k_cache=ka, v_cache=va, block_table=tab, tok_slot=slot, out_dtype=BF16, **kw)
     two = ops.attention_decode(q, ka, va, tab, slot, pos, nh, nkv, hd, hd ** -0.5, window, n_slices)
-    one = ops.attention_decode_fused(qkv, kb, vb, tab, slot, pos, nh, nkv, hd, hd ** -0.5, window, n_slices, **kw)
+    one = ops.attention_decode_fused(qkv, kb, vb, tab, slot, pos, nh, nkv, hd, hd ** -0.5, window, n_slices, **kw, **how)
     return one.float().cpu(), two.float().cpu(), (ka.cpu(), va.cpu()), (kb.cpu(), vb.cpu()), (kc.cpu(), vc.cpu())
 
 
@@ -879,6 +879,49 @@ def test_attention_decode_fused_sees_its_own_key_and_leaves_a_read_only_cache_al
                                                n_slices, write_cache=False)
             assert torch.allclose(again.float().cpu(), want, atol=1e-2)
             assert torch.equal(k2, kd) and torch.equal(v2, vd)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (40, 8, 128), (8, 1, 128), (3, 3, 128), (12, 4, 64), (7, 1, 64), (600, 300, 64)])
+def test_attention_decode_cut_by_pages_is_the_two_kernels_in_one(ops, nh, nkv, hd):
+    """Runs that end with a sequence, inside one and a page from either end; fewer pages than blocks; blocks that hold more sequences than make
+    their queries at once (a long one beside 70 of a token); more than 64 sequences; rows as bfloat16 and as planes; windows; stale values.
+    The counters are zero again, and a second call gives the same bits."""
+    if nkv > 8:
+        cases = [(2, [64, 1, 200], None)]                                # more kv heads than blocks
+    else:
+        cases = [(0, [300], None), (1, [1], None), (2, [64, 65, 700, 7, 128, 129, 1], None), (3, [193, 2], None), (2, [2049] * 3, None),
+                 (2, [5000] + [1] * 70 + [900], None), (1, [65] * 65, None), (2, [70 + 97 * i % 1431 for i in range(24)], None),
+                 (2, [300, 64, 65, 1], 70), (0, [200, 66, 3, 65], 1), (2, [1500, 90], 600)]
+    for i, (planes, lengths, window) in enumerate(cases):
+        counters = torch.zeros(128 * nh, dtype=torch.int32, device=DEV)
+        run = lambda: _fused_case(ops, nh, nkv, hd, lengths, 1, planes, window=window, seed=hd + i, poison=True, pages=True, arrivals=counters)
+        one, two, ca, cb, _ = run()
+        assert torch.isfinite(one).all() and _one_ulp(one, two), (planes, lengths, window, float((one - two).abs().max()))
+        finite = lambda cs: [torch.nan_to_num(c.float(), nan=0.0, posinf=0.0, neginf=0.0) for c in cs]
+        _same_caches(finite(ca), finite(cb))
+        assert not counters.any()
+        assert torch.equal(run()[0], one)
+
+
+def test_attention_decode_cut_by_pages_reads_a_cache_that_is_not_its_own(ops):
+    """Without writing: the same result as the writing call left the cache for, and the cache stays as it is; without norm and rotation."""
+    from palm_infra_amd.kernels import KernelError
+    nh, nkv, hd, i32 = 8, 2, 128, lambda xs: torch.tensor(xs, dtype=torch.int32).to(DEV)
+    for L in (1, 64, 65, 300):
+        table = torch.arange((L + 63) // 64 + 1, dtype=torch.int32).flip(0)[None, :].contiguous().to(DEV)
+        kc, vc = rand(table.shape[1], nkv, 64, hd, seed=1).to(DEV), rand(table.shape[1], nkv, hd, 64, seed=2).to(DEV)
+        row = rand(1, (nh + 2 * nkv) * hd, seed=3).to(DEV)
+        args = (table, i32([0]), i32([L - 1]), nh, nkv, hd, 0.1, None, 1)
+        got = ops.attention_decode_fused(row, kc, vc, *args, pages=True)
+        k2, v2 = kc.clone(), vc.clone()
+        again = ops.attention_decode_fused(row, k2, v2, *args, pages=True, write_cache=False)
+        assert torch.equal(k2, kc) and torch.equal(v2, vc) and _one_ulp(got.float().cpu(), again.float().cpu())
+        assert _one_ulp(got.float().cpu(), ops.attention_decode_fused(row, kc.clone(), vc.clone(), *args).float().cpu())
+    with pytest.raises(KernelError, match="not served"):
+        ops.attention_decode_fused(rand(1, 11 * 128, seed=3).to(DEV), *(torch.zeros(2, 1, *s, dtype=BF16, device=DEV) for s in ((64, 128), (128, 64))),
+                                   i32([[0, 1]]), i32([0]), i32([3]), 9, 1, 128, 1.0, None, 1, pages=True)
+    with pytest.raises(KernelError, match="counters"):
+        ops.attention_decode_fused(row, kc, vc, *args, pages=True, arrivals=torch.zeros(7, dtype=torch.int32, device=DEV))
 
 
 def test_attention_decode_fused_says_what_it_serves(ops):
