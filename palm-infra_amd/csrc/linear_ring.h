@@ -36,6 +36,15 @@ constexpr int RING_UNITS = 256;                 // compute units: a launch is on
 __device__ __forceinline__ void ring_load_16(const void* base, uint32_t offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
 }
+// The same for weights, which pass once: marked as a stream (nt), they don't push what is read again (the rows, the planes and the norms'
+// 32-bit values) out of the caches, nor wait for room among lines that are kept.  Us without and with it, weights of 4 GB in turn:
+// 24,576 x 4,096 gated 1 / 8 / 33 / 48 rows 34.6 35.1 37.7 39.4 and 32.4 32.7 35.6 37.1 (5.8 to 6.2 TB/s at one row), 34,816 x 5,120 gated
+// 60.9 62.2 (1, 8 rows) and 55.1 55.3, 5,120 x 17,408 32.3 33.4 and 29.4 29.6, 4,096 x 12,288 to planes 19.1 19.4 21.6 and 18.2 18.2 19.7,
+// 6,144 x 4,096 11.4 11.3 13.1 and 10.8 10.8 12.4, 151,936 x 4,096 198 206 229 236 and 184 190 207 212.  Matrices up to 20 MB: the same
+// within 1%, one of 50 to 200 MB that nothing else passes by before it is read again up to 10% slower (11.0 and 11.4, 18.5 and 20.0).
+__device__ __forceinline__ void ring_load_16_once(const void* base, uint32_t offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+}
 __device__ __forceinline__ void ring_load_4(const void* base, uint32_t offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
 }
@@ -143,7 +152,7 @@ __global__ __launch_bounds__(RING_THREADS) void linear_ring_kernel(const bf16_t*
             // K is a multiple of 8: a piece is whole or absent; an absent one reads the row's start and counts as zeros
             const bool ok = EXACT || k0 + (i / 2) * 64 + piece * 8 < K;
             const uint32_t in_row = ok ? (uint32_t)(k0 * 2 + (i / 2) * 128 + piece * 16) : 0u;
-            ring_load_16(ask_base[i % 2], w_off[i % 2] + in_row, to + i * 1024);
+            ring_load_16_once(ask_base[i % 2], w_off[i % 2] + in_row, to + i * 1024);
             if (!AREG) ring_load_16(A, x_off[i % 2] + in_row, to + 4096 + i * 1024);
         }
         ++n_asked;
