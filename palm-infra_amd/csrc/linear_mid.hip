@@ -46,6 +46,14 @@ constexpr int MID_UNITS = 256;                  // compute units of the chip
 __device__ __forceinline__ void mid_load_16_bytes_a_lane_into_lds(const void* base, uint32_t offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
 }
+// The same for the weights, which pass once (linear_ring.h: nt).  Us without and with it: 64 rows, 4,096 x 12,288 25.9 and 23.5,
+// 5,120 x 17,408 42.9 and 39.2, 24,576 x 4,096 gated 41.6 and 39.5, 6,144 x 4,096 16.6 and 15.2; 91 and 128 rows, the same 29.6 32.2 and
+// 28.6 31.5, 49.5 53.4 and 48.4 52.6, 44.0 46.7 and 42.0 43.4, 17.0 19.5 and 16.2 18.3; 4,096 x 4,096 12.6 14.1 and 13.0 14.2.
+// What is left is neither LDS nor the matrix cores (without their work the same time): the weights alone take 35 us of those 42 to 43
+// (5.7 TB/s), the rows alone, which every block reads again from L2, 29.
+__device__ __forceinline__ void mid_load_16_bytes_a_lane_into_lds_once(const void* base, uint32_t offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+}
 template <int N> __device__ __forceinline__ void mid_wait_for_all_but_the_youngest_loads() {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));          // s_waitcnt vmcnt(N)
 }
@@ -163,7 +171,7 @@ __global__ __launch_bounds__(MID_THREADS) void linear_mid_kernel(
         const char* base = reinterpret_cast<const char*>(W) + (size_t)turned(min(chunk, c1 - 1)) * MID_ROW_BYTES;
         const uint32_t to = w_lds0 + ((chunk - c0) % W_STAGES) * W_BYTES + wave * W_LOADS * 1024;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) mid_load_16_bytes_a_lane_into_lds(base, w_from[i], to + i * 1024);
+        for (int i = 0; i < W_LOADS; ++i) mid_load_16_bytes_a_lane_into_lds_once(base, w_from[i], to + i * 1024);
     };
 
     // fragments: lane l holds row l % 32 of a tile and the eight k-values 16 s + 8 (l / 32) .. of step s
