@@ -15,10 +15,10 @@
 // fence writes back or empties a die's cache for it, and no wave ever waits for another block.  The counters are zero between launches: the wave that
 // finds the last piece sets its counter back.
 //
-// What bounds it: the walk reads at 5.3 to 5.9 TB/s; before it lie 3 us (two round trips for the step's lengths and the page numbers, the queries through LDS;
+// What bounds it: the walk reads at 5.5 to 6.3 TB/s; before it lie 3 us (two round trips for the step's lengths and the page numbers, the queries through LDS;
 // 96 KB a unit are on their way meanwhile), behind it 2 to 4 (pieces to memory, the count, the last one's reads).  Us, 32 heads of 8 (by slices of every
-// sequence alike, and so): 45 sequences of 70 to 1,500 tokens 45.2 and 37.9 (3.7 TB/s with all of it), 64 of 64 to 2,048 75.7 and 62.4, 8 of 2,048 20.6 and 19.3, one of
-// 777 8.9 and 11.7: ops.decode_pages_pays.  Pages through LDS in whole lines against fragments read as the matrix cores want them, 16 rows by 64 bytes: 45
+// sequence alike, and so): 45 sequences of 70 to 1,500 tokens 44.9 and 35.2 (4.0 TB/s with all of it), 64 of 2,048 106.8 and 100.4, 8 of 2,048 20.8 and 17.7, one of
+// 777 8.9 and 12.0: ops.decode_pages_pays.  The pages pass once and are marked so (nt): without that 37.6 105.2 19.3 for the first three.  Pages through LDS in whole lines against fragments read as the matrix cores want them, 16 rows by 64 bytes: 45
 // sequences 39.6 and 37.9, one of 100 15.8 and 10.8.  Tried: rings of 16 KB (no change).
 constexpr bool PAGES_SERVE_HEAD = HD == 64 || HD == 128;
 constexpr int DP_WAVES = 8, DP_THREADS = DP_WAVES * WAVE;
@@ -207,8 +207,8 @@ struct RingPlaces {
         lds_reads_done();                                                  // the slot may be the one they read
 #pragma unroll
         for (int i = 0; i < DP_LOADS; ++i) {
-            if (part < 4) row_chunk_into_lds(in_scalars(keys + (part / 2 * 32 + part % 2 * 4) * (HD * 2)), ask_k[i], lds + i * 1024);
-            else row_chunk_into_lds(in_scalars(values + (part - 4) * DP_SLOT + i * 1024), ask_v, lds + i * 1024);
+            if (part < 4) row_chunk_into_lds_once(in_scalars(keys + (part / 2 * 32 + part % 2 * 4) * (HD * 2)), ask_k[i], lds + i * 1024);
+            else row_chunk_into_lds_once(in_scalars(values + (part - 4) * DP_SLOT + i * 1024), ask_v, lds + i * 1024);
         }
     }
 };

@@ -909,13 +909,22 @@ def decode_pages_pays(n_seqs: int, nh: int, nkv: int, hd: int, longest: int) -> 
     """Whether it should be: where sequences are many or long (``longest``: the longest one, or what a recorded step is sized for).  Its
     blocks all read until the end, but they begin some 3 us later than a slice's wave (the cut, the queries through LDS) and add their
     pieces across dies instead of in a launch of their own.  Us by slices and by pages, head size 128, 32 heads of 8, sequences of equal
-    length or spread evenly: 8 of 2,048 20.6 19.3; 8 of 700 11.5 13.1; 12 of 64 to 2,048 19.4 16.0; 16 of 200 10.2 11.8, of 30 to 600 12.3
-    13.0, of 70 to 1,500 20.2 18.3, of 64 to 2,048 23.9 20.5, of 2,000 32.1 31.2, of 300 to 8,000 76 63; 24 of 2,000 44.3 44.6; 40 of 700 30.7
-    32.5, of 70 to 1,500 34.2 27.8; 48 of 70 to 1,500 44.0 37.9; 64 of 200 23.9 20.8, of 64 to 2,048 75.7 62.4.  With more heads a block adds more
-    pieces: 40 heads of 8, 16 of 64 to 2,048 23.8 21.4 or 24.7 25.4 by their lengths, 24 of 70 to 1,500 26.0 26.6, 32 of them 33.1 30.7; 64 heads of
-    8, 32 of them 33.2 33.1, 64 55.2 52.7.  Four up to 8,000
-    tokens 24.9 23.6, eight 36.4 31.4, of 70 to 1,500 13.4 13.8."""
-    return n_seqs * longest >= (32768 if nh <= 4 * nkv and n_seqs >= 12 else 65536) and decode_pages_serves(n_seqs, nh, nkv, hd)
+    length or spread evenly.  16,384 keys (sequences times longest) and sequences of 2,048 and more, or 32 of them and more: 8 of 2,000
+    20.3 18.9, of 1,100 15.7 15.0, of 70 to 1,500 13.2 13.4; 4 of 4,000 21.1 19.8, of 2,100 14.8 15.6, of 300 to 4,000 18.9 17.0; 2 of 8,000 21.7
+    21.6; one of 16,000 26.3 23.2; 32 of 260 15.5 14.1, of 500 20.7 17.6; 64 of 130 to 250 21.6 21.6, of 20 to 60 14.0 11.9.  Fewer and shorter ones
+    no: 16 of 30 to 600 11.9 13.2, of 520 14.9 15.2 (of 1,000 20.5 19.2); 8 of 520 to 1,000 13.9 13.6, 48 of 10 to 250 16.6 17.7.  32,768 keys,
+    twelve sequences and more: 24 of 1,000 27.3 24.9, of 700 21.4 20.5, 16 of 70 to 1,500 20.9 20.4, 45 of them 44.9 35.2, 32 of 900 31.5 26.0,
+    64 of 2,048 106.8 100.4; of the shortest, 100 of 20 to 120 17.9 20.0.  A smaller head or fewer kv heads leave a block less to read: head size 64, 16
+    of 70 to 1,500 15.0 14.6, 8 of 1,100 10.0 11.9; 32 heads of 4, 16 of 1,000 14.7 14.9, 8 of 1,100 12.3 14.4.  With more heads a block adds more
+    pieces: 40 heads of 8, 16 of 70 to 1,500 21.3 21.3, 8 of 1,100 15.8 16.9, 16 of 4,000 55.4 50.5, 32 of 1,500 45.0 39.6; 64 heads of 8, 16 of 70 to
+    1,500 21.4 24.6, 40 of 30 to 600 22.3 23.2, 8 of 2,000 21.0 19.9."""
+    keys = 65536
+    if nh <= 4 * nkv:
+        if hd == 128 and nkv >= 8 and (longest >= 2048 or n_seqs >= 32):
+            keys = 16384
+        elif n_seqs >= 12:
+            keys = 32768
+    return n_seqs * longest >= keys and decode_pages_serves(n_seqs, nh, nkv, hd)
 
 
 def attention_decode_fused(qkv, k_cache, v_cache, block_table, seq_slot, seq_start, nh: int, nkv: int, hd: int, scale: float,
