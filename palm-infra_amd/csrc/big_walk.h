@@ -96,15 +96,18 @@ struct BigItem {
     const char* w;
     int stages, turn;
     int x_rows, w_rows;           // rows that there are (beyond them the last one again)
+    int live = 0;                 // (RAGGED) column tiles that a wave multiplies, of its TT
 };
 
 // items: how many tiles the block owns; make(i): the i-th's BigItem, the same in every lane; x_row(item, i), w_row(item, i): where row i
 // of the tile lies, in rows from item.x or item.w (for tiles with the same x_rows and w_rows the same); row_bytes from row to row
-// in both.  finish(i, acc): acc[4 half + f][t][v], lane (r, g) of wave (wave_f, wave_t) = (wave % 2, wave / 2): token
+// in both.  finish(i, acc, live): acc[4 half + f][t][v], lane (r, g) of wave (wave_f, wave_t) = (wave % 2, wave / 2): token
 // wave_t * 32 NT + 16 t + r, tile row 128 wave_f + 64 half + 16 g + 4 f + v.
-template <int NT, bool TURNED, class Make, class XRow, class WRow, class Finish>
+// RAGGED (of the high tiles): a tile's last column tiles may be nobody's.  They are neither read from LDS nor multiplied, each number of
+// them in a loop of its own, from half a tile on (below that the loads of a stage have no products left to stand between); their sums are zero.
+template <int NT, bool TURNED, bool RAGGED = false, class Make, class XRow, class WRow, class Finish>
 __device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int items, Make make, XRow x_row, WRow w_row, Finish finish) {
-    constexpr int TT = 2 * NT, W_STAGE = BIG_FEAT * BIG_ROW, X_STAGE = 64 * NT * BIG_ROW, GAPS = 4 * TT, A = big_ahead(NT);
+    constexpr int TT = 2 * NT, W_STAGE = BIG_FEAT * BIG_ROW, X_STAGE = 64 * NT * BIG_ROW, A = big_ahead(NT);
     constexpr int XL = 2 * NT, WL = 8;                       // a wave's loads of a stage, 8 rows each
     static_assert(A * W_STAGE + (A + 1) * X_STAGE == big_lds_bytes(NT) && big_lds_bytes(NT) <= 160 * 1024, "the stages fit LDS");
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -156,16 +159,16 @@ __device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int item
         asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(from) : "memory");
     };
     // loads FROM .. FROM + COUNT of a stage's, over the gaps of a quarter
-    auto w_loads = [&](int n, auto from, auto count, uint32_t stage) __attribute__((always_inline)) {
+    auto w_loads = [&](int n, auto from, auto count, uint32_t stage, auto live) __attribute__((always_inline)) {
         big_each<decltype(count)::value>([&](auto j) __attribute__((always_inline)) {
-            constexpr int q = decltype(from)::value + decltype(j)::value, gap = decltype(j)::value * GAPS / decltype(count)::value;
+            constexpr int q = decltype(from)::value + decltype(j)::value, gap = decltype(j)::value * (4 * decltype(live)::value) / decltype(count)::value;
             if (n == gap) place(stage, std::integral_constant<int, q>{});
             if (n == gap + 1) fetch(ahead.w + ahead_at, w_off[q]);
         });
     };
-    auto x_loads = [&](int n, auto from, auto count, uint32_t stage) __attribute__((always_inline)) {
+    auto x_loads = [&](int n, auto from, auto count, uint32_t stage, auto live) __attribute__((always_inline)) {
         big_each<decltype(count)::value>([&](auto j) __attribute__((always_inline)) {
-            constexpr int q = decltype(from)::value + decltype(j)::value, gap = decltype(j)::value * GAPS / decltype(count)::value;
+            constexpr int q = decltype(from)::value + decltype(j)::value, gap = decltype(j)::value * (4 * decltype(live)::value) / decltype(count)::value;
             if (n == gap) place(stage, std::integral_constant<int, q>{});
             if (n == gap + 1) fetch(ahead.x + ahead_at, x_off[q]);
         });
@@ -182,35 +185,6 @@ __device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int item
         }
 #pragma unroll
     for (int i = 0; i < 2; ++i) xc[i] = (A * BIG_FEAT + wave_t * 32 * NT + r) * BIG_ROW + ((4 * i + g) ^ big_x_swizzle(r)) * 16;
-    f32x4 acc[8][TT];
-    bf16x8 wf[2][2][4], xf[2][TT];                           // [half][k-step][tile], [k-step][tile]
-    auto read_w = [&](const char* stage, int i, int f) __attribute__((always_inline)) {
-        wf[f / 4][i][f % 4] = *reinterpret_cast<const bf16x8*>(stage + wc[f % 4][i] + f / 4 * 64 * BIG_ROW);
-    };
-    auto read_x = [&](const char* stage, int i, int t) __attribute__((always_inline)) {
-        xf[i][t] = *reinterpret_cast<const bf16x8*>(stage + xc[i] + t * 16 * BIG_ROW);
-    };
-    // a stage's reads, not before the first product (where the last quarter's are waited for) and not in the last few gaps
-    auto w_reads = [&](int n, const char* stage, int i) __attribute__((always_inline)) {
-#pragma unroll
-        for (int f = 0; f < 8; ++f)
-            if (n == 1 + f * GAPS * 3 / 32) read_w(stage, i, f);
-    };
-    auto x_reads = [&](int n, const char* stage, int i) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < TT; ++t)
-            if (n == 1 + t * GAPS * 7 / (8 * TT)) read_x(stage, i, t);
-    };
-    auto quarter = [&](int half, int i, auto between) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < TT; ++t)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                between(4 * t + f);
-                big_multiply(acc[4 * half + f][t], wf[half][i][f], xf[i][t]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-    };
 #define BIG_C(v) std::integral_constant<int, (v)>{}
 
 #pragma unroll
@@ -222,40 +196,71 @@ __device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int item
     all_but_the_youngest_have_arrived<(A - 1) * (XL + WL)>();
     big_swap();
     uint32_t xs_before = A * X_STAGE, xs = 0, xs_next = X_STAGE, ws = 0, ws_next = W_STAGE;
-    for (int item = 0; item < items; ++item) {
+    // (the sums and what is multiplied live inside: with RAGGED nothing but the cursor and the offsets is carried from one tile's walk to another's)
+    auto tile = [&](int item, auto live) __attribute__((always_inline)) {
+        f32x4 acc[8][TT];
+        bf16x8 wf[2][2][4], xf[2][TT];                       // [half][k-step][tile], [k-step][tile]
+        constexpr int LIVE = decltype(live)::value;
+        auto read_w = [&](const char* stage, int i, int f) __attribute__((always_inline)) {
+            wf[f / 4][i][f % 4] = *reinterpret_cast<const bf16x8*>(stage + wc[f % 4][i] + f / 4 * 64 * BIG_ROW);
+        };
+        auto read_x = [&](const char* stage, int i, int t) __attribute__((always_inline)) {
+            xf[i][t] = *reinterpret_cast<const bf16x8*>(stage + xc[i] + t * 16 * BIG_ROW);
+        };
+        // a stage's reads, not before the first product (where the last quarter's are waited for) and not in the last few gaps
+        auto w_reads = [&](int n, const char* stage, int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int f = 0; f < 8; ++f)
+                if (n == 1 + f * (4 * LIVE) * 3 / 32) read_w(stage, i, f);
+        };
+        auto x_reads = [&](int n, const char* stage, int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < LIVE; ++t)
+                if (n == 1 + t * 7 / 2) read_x(stage, i, t);
+        };
+        auto quarter = [&](int half, int i, auto between) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+                for (int f = 0; f < 4; ++f) {
+                    between(4 * t + f);
+                    big_multiply(acc[4 * half + f][t], wf[half][i][f], xf[i][t]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        };
 #pragma unroll
         for (int f = 0; f < 8; ++f)
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
+            for (int t = 0; t < LIVE; ++t) {
                 acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
                 asm volatile("" : "+a"(acc[f][t]));
             }
         asm volatile("s_nop 7" ::: "memory");                // (the products are written out: their distance to what writes or reads the sums is kept here)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < TT; ++t) read_x(lds + xs, 0, t); // (read again behind another tile's end, which has better use for the registers)
+        for (int t = 0; t < LIVE; ++t) read_x(lds + xs, 0, t); // (read again behind another tile's end, which has better use for the registers)
 #pragma unroll
         for (int f = 0; f < 8; ++f) read_w(lds + ws, 0, f);
         const int stages = make(item).stages;
         for (int kt = 0; kt < stages; ++kt) {
             quarter(0, 0, [&](int n) __attribute__((always_inline)) {
                 w_reads(n, lds + ws, 1);
-                x_loads(n, BIG_C(0), BIG_C(XL / 2), lds_x + xs_before);
+                x_loads(n, BIG_C(0), BIG_C(XL / 2), lds_x + xs_before, live);
             });
             quarter(1, 0, [&](int n) __attribute__((always_inline)) {
                 x_reads(n, lds + xs, 1);
-                x_loads(n, BIG_C(XL / 2), BIG_C(XL - XL / 2), lds_x + xs_before);
+                x_loads(n, BIG_C(XL / 2), BIG_C(XL - XL / 2), lds_x + xs_before, live);
             });
             all_but_the_youngest_have_arrived<(A - 1) * XL + (A - 2) * WL>();
             big_lds_reads_done();
             big_swap();
             quarter(0, 1, [&](int n) __attribute__((always_inline)) {
                 x_reads(n, lds + xs_next, 0);
-                w_loads(n, BIG_C(0), BIG_C(WL / 2), lds_w + ws);
+                w_loads(n, BIG_C(0), BIG_C(WL / 2), lds_w + ws, live);
             });
             quarter(1, 1, [&](int n) __attribute__((always_inline)) {
                 w_reads(n, lds + ws_next, 0);
-                w_loads(n, BIG_C(WL / 2), BIG_C(WL / 2), lds_w + ws);
+                w_loads(n, BIG_C(WL / 2), BIG_C(WL / 2), lds_w + ws, live);
             });
             advance();
             xs_before = xs; xs = xs_next; ws = ws_next;
@@ -264,8 +269,21 @@ __device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int item
         }
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        finish(item, acc);
+        finish(item, acc, live);
         __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int item = 0; item < items; ++item) {
+        if constexpr (RAGGED) {
+            static_assert(TT == 8, "tiles of 256 rows");
+            const int live = make(item).live;
+            if (live >= 8) tile(item, BIG_C(8));
+            else if (live == 7) tile(item, BIG_C(7));
+            else if (live == 6) tile(item, BIG_C(6));
+            else if (live == 5) tile(item, BIG_C(5));
+            else tile(item, BIG_C(4));
+        } else {
+            tile(item, BIG_C(TT));
+        }
     }
 #undef BIG_C
     all_but_the_youngest_have_arrived<0>();                  // nothing may land in LDS after the block's end

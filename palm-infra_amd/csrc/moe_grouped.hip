@@ -29,14 +29,26 @@ __device__ inline bf16x8 grouped_row8(const bf16_t* row, int col, int dim) {
     return col < dim ? v : zero_bf16x8();
 }
 
-// One block.  starts[e] = first slot of expert e's run (runs padded to whole tiles); tile_expert[i] = the expert of tile i, -1 beyond
-// the last tile; slot_pair[slot] = pair (-1 where a run is padded), pair_slot[pair] = slot.  The choices are rows [n, top], or with
+// What the plan says of a tile: its expert and how many of its slots are pairs, in one number; -1 beyond the last tile
+constexpr int TILE_EXPERT_BITS = 10;
+static_assert(PLAN_MAX_EXPERTS <= 1 << TILE_EXPERT_BITS, "an expert's number and a tile's rows in one int");
+__device__ __forceinline__ int tile_expert_of(int t) { return t & ((1 << TILE_EXPERT_BITS) - 1); }
+__device__ __forceinline__ int tile_rows_of(int t) { return t >> TILE_EXPERT_BITS; }
+// Rows of each of an expert's tiles but the last.  Tiles of 256 rows that may stop early (moe_big_kernel) share up to 768 rows evenly, in whole
+// steps of 32 (what a column tile of each of a tile's two waves of rows holds), so that no compute unit gets a full one and another little; other
+// tiles are filled one after the other.
+__device__ __forceinline__ int rows_per_tile(int rows, int tile) {
+    const int tiles = (rows + tile - 1) / tile;
+    return tile == 256 && tiles >= 1 && tiles <= 3 ? ((rows + tiles - 1) / tiles + 31) / 32 * 32 : tile;
+}
+
+// One block.  starts[e] = first slot of expert e's run (runs padded to whole tiles); tile_expert[i]: see above; slot_pair[slot] = pair (-1 where a run is padded), pair_slot[pair] = slot.  The choices are rows [n, top], or with
 // ids the rows of a table [vocab, top] that the tokens' ids pick.
 __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int* __restrict__ chosen, const int* __restrict__ ids, int vocab, int top,
                                                                 int n_pairs, int experts, int max_tiles, int tile,
                                                                 int* __restrict__ tile_expert, int* __restrict__ slot_pair,
                                                                 int* __restrict__ pair_slot, int* __restrict__ used) {
-    __shared__ int start_s[PLAN_MAX_EXPERTS + 1], cursor_s[PLAN_MAX_EXPERTS];
+    __shared__ int start_s[PLAN_MAX_EXPERTS + 1], cursor_s[PLAN_MAX_EXPERTS], per_s[PLAN_MAX_EXPERTS];
     const int lane = threadIdx.x % WAVE;
     auto choice = [&](int p) { return ids ? chosen[(size_t)min(max(ids[p / top], 0), vocab - 1) * top + p % top] : chosen[p]; };
     for (int e = threadIdx.x; e < experts; e += PLAN_THREADS) cursor_s[e] = 0;
@@ -72,17 +84,23 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int* __res
     }
     __syncthreads();
     for (int i = threadIdx.x; i < max_tiles; i += PLAN_THREADS) tile_expert[i] = -1;
-    // the slots that pad each run
-    for (int e = threadIdx.x / WAVE; e < experts; e += PLAN_THREADS / WAVE)
-        for (int s = start_s[e] + cursor_s[e] + lane; s < start_s[e + 1]; s += WAVE) slot_pair[s] = -1;
+    // the slots that pad each tile
+    for (int e = threadIdx.x / WAVE; e < experts; e += PLAN_THREADS / WAVE) {
+        const int rows = cursor_s[e], per = rows_per_tile(rows, tile);
+        for (int s = lane; s < start_s[e + 1] - start_s[e]; s += WAVE)
+            if (s % tile >= min(per, rows - s / tile * per)) slot_pair[start_s[e] + s] = -1;
+    }
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += PLAN_THREADS) {
-        for (int i = start_s[e] / tile; i < start_s[e + 1] / tile; ++i) tile_expert[i] = e;
-        cursor_s[e] = start_s[e];
+        const int rows = cursor_s[e], per = rows_per_tile(rows, tile), tiles = (start_s[e + 1] - start_s[e]) / tile;
+        for (int i = 0; i < tiles; ++i) tile_expert[start_s[e] / tile + i] = e | min(per, rows - i * per) << TILE_EXPERT_BITS;
+        cursor_s[e] = 0;
+        per_s[e] = per;
     }
     __syncthreads();
     for (int p = threadIdx.x; p < n_pairs; p += PLAN_THREADS) {
-        const int slot = atomicAdd(&cursor_s[choice(p)], 1);
+        const int e = choice(p), at = atomicAdd(&cursor_s[e], 1), per = per_s[e];
+        const int slot = start_s[e] + at / per * tile + at % per;
         slot_pair[slot] = p;
         pair_slot[p] = slot;
     }
@@ -98,8 +116,9 @@ __global__ __launch_bounds__(GT_WAVES * WAVE) void moe_grouped_kernel(const bf16
                                                                       int n_features, int k_dim, ExpertCap cap, bf16_t* __restrict__ out) {
     constexpr bool GATED = FORM == 1 || FORM == 3;
     const int tile = blockIdx.x;
-    const int e = tile_expert[tile];
-    if (e < 0) return;
+    const int planned = tile_expert[tile];
+    if (planned < 0) return;
+    const int e = tile_expert_of(planned);
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const int r = lane % 16, g = lane / 16;
     const int f0 = blockIdx.y * GT_FEATURES + wave * 32;
@@ -176,7 +195,10 @@ __global__ __launch_bounds__(GT_WAVES * WAVE) void moe_grouped_kernel(const bf16
 //     three of eight dies stood idle at 852 rows
 //   - an expert's features begin their walk at stages of their own: rows lie 4 or 8 KB apart, and blocks that walk in step ask
 //     all for the same few of memory's channels (352 rows: 288 us in step, 234 so, tiles of 128 rows)
-//   - the tile is as high as an expert's rows need, as long as that spares another tile (see big_tile_of).
+//   - the tile is as high as an expert's rows need, as long as that spares another tile (see big_tile_of)
+//   - a tile of 256 rows multiplies 128 to 256 of them, in steps of 32, and an expert's rows are shared out evenly over its tiles (experts of
+//     362 rows: two tiles of 192 and 170, not of 256 and 106): both products of 32 experts of 2,048 x 4,096 with 188 / 362 / 425 / 588 rows each 300 462
+//     462 696 -> 268 405 435 618.
 // Us with plan and sum, squared relu, rows of four choices over 32 experts: 130 rows 484 -> 209 (fragments from memory before),
 // 852: 372 -> 251, 2,048: 590 -> 388 (a ring of three stages of 32 x 32 x 16 instructions before; this walk with eight waves 262 and 440).
 template <int NT, int FORM, typename TO>
@@ -190,28 +212,31 @@ __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(1, 
     const int last = min(total, (int)(blockIdx.x % BIG_DIES + 1) * per_die), items = first < last ? (last - first + stride - 1) / stride : 0;
     if (items == 0) return;
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, wave_f = wave % 2, wave_t = wave / 2;
-    big_walk<NT, true>(lds, (uint32_t)(k_dim * 2), items,
+    // (RAGGED) A tile's rows, 32 at a time, are dealt to its two waves of rows: what a wave has lies in its first column tiles
+    constexpr bool RAGGED = NT == 4;
+    auto row_at = [&](int row) __attribute__((always_inline)) { return RAGGED ? row % (32 * NT) / 16 * 32 + row / (32 * NT) * 16 + row % 16 : row; };
+    big_walk<NT, true, RAGGED>(lds, (uint32_t)(k_dim * 2), items,
         [&](int item) __attribute__((always_inline)) {
             const int pid = first + item * stride, tile = pid / feature_tiles, ft = pid % feature_tiles;
-            const int e = __builtin_amdgcn_readfirstlane(tile_expert[tile]), from = ft * (GATED ? 128 : BIG_FEAT);
+            const int planned = __builtin_amdgcn_readfirstlane(tile_expert[tile]), e = tile_expert_of(planned), from = ft * (GATED ? 128 : BIG_FEAT);
             // (x_rows names the tile of slots: the rows of another are others)
             return BigItem{reinterpret_cast<const char*>(a), reinterpret_cast<const char*>(w + ((size_t)e * (GATED ? 2 : 1) * n_features + from) * k_dim), stages,
-                           (5 * e + 2 * ft) % stages, tile, min(GATED ? 128 : BIG_FEAT, n_features - from)};
+                           (5 * e + 2 * ft) % stages, tile, min(GATED ? 128 : BIG_FEAT, n_features - from), (tile_rows_of(planned) + 31) / 32};
         },
         [&](const BigItem& it, int row) __attribute__((always_inline)) {
-            const int slot = it.x_rows * 64 * NT + row;
+            const int slot = it.x_rows * 64 * NT + (RAGGED ? min(row_at(row), it.live * 32 - 1) : row);
             return FORM == 0 ? slot : max(slot_pair[slot], 0) / top;      // a slot that pads the run reads row 0; nobody reads its result
         },
         [&](const BigItem& it, int row) __attribute__((always_inline)) {
             return GATED ? (row & 64 ? n_features : 0) + min(row / 128 * 64 + row % 64, it.w_rows - 1) : min(row, it.w_rows - 1);
         },
-        [&](int item, f32x4 (&acc)[8][2 * NT]) __attribute__((always_inline)) {
+        [&](int item, f32x4 (&acc)[8][2 * NT], auto live) __attribute__((always_inline)) {
             const int pid = first + item * stride, tile = pid / feature_tiles, ft = pid % feature_tiles;
             f32x4 z[8];
 #pragma unroll
-            for (int t = 0; t < 2 * NT; ++t) {
+            for (int t = 0; t < decltype(live)::value; ++t) {
                 big_column(acc, t, z);
-                const int slot = tile * 64 * NT + wave_t * 32 * NT + 16 * t + lane % 16;
+                const int slot = tile * 64 * NT + row_at(wave_t * 32 * NT + 16 * t + lane % 16);
                 if (sizeof(TO) == 4 && slot_pair[slot] < 0) continue;          // (few rows: most of a tile pads its run)
                 TO* row = out + (size_t)slot * n_features;
 #pragma unroll
@@ -280,7 +305,7 @@ struct MoeSizes {
 // almost a whole round.  Tiles that do not fill the chip run side by side, so few or small experts take low ones: 16 experts of 256 x
 // 512 with 250 rows each 51 us in tiles of 192 rows, 30 in tiles of 64.  Measured with a full chip, us, 32 experts of 2,048 x 4,096, tiles of
 // 64 / 128 / 192 / 256 rows: mean 25: 210 / 222 / 242 / 271, 75: 291 / 230 / 247 / 268, 106: 345 / 294 / 251 / 279, 150: 390 / 314 / 257 / 281,
-// 181: 439 / 323 / 345 / 288, 256: 571 / 438 / 388 / 450, 375: 752 / 549 / 519 / 472, 625: 1,125 / 794 / 724 / 709.  At 49 sizes (8 to 128 experts of 256
+// 181: 439 / 323 / 345 / 288, 256: 571 / 438 / 388 / 450, 375: 752 / 549 / 519 / 472, 625: 1,125 / 794 / 724 / 709 (tiles of 256 before they could stop early).  At 49 sizes (8 to 128 experts of 256
 // to 2,048 x 512 to 4,096, means of 8 to 2,000 rows) it takes the best tile at 40 and is 1.0 % behind it in the mean, 10 % at worst (1,000 rows for each of
 // 16 small experts); with the times that a fit over those sizes gives (0.65, 0.77, 1.04, 1.46) it chooses otherwise at three of them, no better.
 static int big_tile_of(const MoeSizes& s) {
@@ -294,6 +319,10 @@ static int big_tile_of(const MoeSizes& s) {
         const double cost = (rounds(s.ff, s.gated ? BIG_FEAT / 2 : BIG_FEAT) * s.width + rounds(s.width, BIG_FEAT) * s.ff) * stage_us[nt - 1];
         if (cost < best_cost) { best_cost = cost; best = 64 * nt; }
     }
+    // Experts of many rows: tiles of 256 multiply no more than their rows need either, and read the weights less often.  Us, tiles of 192 and of
+    // 256 rows, 32 experts of 2,048 x 4,096: mean 256 386 and 398, 325 397 and 392, 512 599 and 586, 750 851 and 803, 1,000 1,093 and 1,003; 32 capped ones of
+    // 1,536 x 4,096, mean 512 718 and 670; 16 gated ones of 1,408 x 2,048, mean 500 195 and 187.
+    if (best == 192 && mean >= 448) best = 256;
     return best;
 }
 // Whether the tiles cross LDS: rows in whole stages that start on 16 bytes, offsets from a matrix's first row of 32 bits, and, for

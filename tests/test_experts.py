@@ -112,6 +112,32 @@ def test_grouped_tiles_of_every_height_one_after_the_other(form, E, top, W, F, n
 
 
 @gpu
+@pytest.mark.parametrize("form,E,W,F,rows", [("gated_silu", 40, 256, 320, (1, 31, 32, 33, 64, 127, 128, 129, 160, 161, 192, 193, 224, 225, 255, 256)),
+                                             ("relu_squared", 40, 256, 320, (257, 320, 321, 384, 385, 512, 513, 576, 577, 700, 768, 769, 0, 900, 1024, 1025))])
+def test_grouped_tiles_that_stop_early(form, E, W, F, rows):
+    """Experts of as many rows as fill one to five tiles of 256 and a little more or less, one choice a row, the experts after those chosen by 700 or 400 each."""
+    from palm_infra_amd.kernels import ops
+    per = ops.expert_rows(form) * F
+    g = torch.Generator().manual_seed(E + W)
+    counts = list(rows) + [700 if form == "gated_silu" else 400] * (E - len(rows))
+    chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)]).to(torch.int32)
+    chosen = chosen[torch.randperm(len(chosen), generator=g)][:, None]
+    n = len(chosen)
+    assert ops.feedforward().palm_moe_tile_tokens(n, E, W, F, int(ops.expert_rows(form) > 1), 1) == 256
+    up, down = (torch.randn(E * per, W, generator=g) * W ** -0.5).to(torch.bfloat16), (torch.randn(E * W, F, generator=g) * F ** -0.5).to(torch.bfloat16)
+    h, weight = torch.randn(n, W, generator=g).to(torch.bfloat16), torch.rand(n, 1, generator=g)
+    want = plain_mixture(form, h, up, down, chosen, weight, F)
+    args = [t.cuda() for t in (h, up, down, chosen, weight)]
+    for exact in (False, True):
+        got = ops.moe_grouped(*args, F, form, exact=exact).cpu().double()
+        # the inner rows' rounding to bfloat16, 0.0017 in the mean square, and the experts' results' unless they stay in 32 bits
+        assert float((got - want).norm() / want.norm()) < (0.003 if exact else 0.004)
+        for e in range(len(rows)):                           # and in no expert's rows more than in others'
+            of = chosen[:, 0] == e
+            assert not of.any() or float((got[of] - want[of]).norm() / want[of].norm()) < 0.006
+
+
+@gpu
 @pytest.mark.parametrize("form", ["gated_silu", "gelu", "capped_gated", "relu_squared"])
 @pytest.mark.parametrize("E,top,W,F,shared", [(4, 2, 64, 64, 40), (3, 1, 72, 24, None), (33, 4, 320, 264, 264), (5, 5, 8, 8, 16), (512, 3, 48, 16, None), (6, 2, 2056, 520, 1032)])
 def test_few_rows(form, E, top, W, F, shared):
