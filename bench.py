@@ -166,7 +166,8 @@ def kernel_table(engine, cfg, slots, batch: int, context: int) -> dict:
     kv = cache.layer_caches[0].kv           # the store of the first layer's group (all layers of this model share it)
     seq_slot = torch.tensor(slots, dtype=torch.int32, device=dev)
     seq_start = torch.tensor([cache.lengths[s] - 1 for s in slots], dtype=torch.int32, device=dev)
-    n_slices = ops.decode_slices(batch, nh, nkv, engine._length_bucket(context + 1))
+    bucket = engine._length_bucket(context + 1)
+    n_slices, by_pages = ops.decode_slices(batch, nh, nkv, bucket), ops.decode_pages_pays(batch, nh, nkv, hd, bucket)
     # what the attention part runs after its q/k/v projection in a decode step: the projection's planes of partial
     # sums in, per-head norms, rotation, the new key and value into the cache, attention, the merge of the slices
     mixer0 = layers[0].mixer
@@ -177,7 +178,7 @@ def kernel_table(engine, cfg, slots, batch: int, context: int) -> dict:
         m = layers[i].mixer
         return ops.attention_decode_fused(qkv, kv.k[i], kv.v[i], kv.table_dev, seq_slot, seq_start, nh, nkv, hd, m.scale, None,
                                           n_slices, q_norm_w=m.q_norm.weight, k_norm_w=m.k_norm.weight, eps=m.q_norm.eps,
-                                          cos=cos, sin=sin, rotary_dim=hd, pairing=0)
+                                          cos=cos, sin=sin, rotary_dim=hd, pairing=0, pages=by_pages, arrivals=kv.arrivals)
 
     def each_layer(fn):
         return lambda: [fn(i) for i in range(L)]
@@ -436,7 +437,7 @@ def _mixer_rooflines(raw: dict, tokens: int, batch: int, context: int) -> dict:
         nh, nkv, hd = raw["num_attention_heads"], raw["num_key_value_heads"], raw["head_dim"]
         out["palm_attention_prefill_in"] = out["palm_attention_prefill_wide"] = (4.0 * nh * hd * pairs, mfma, None, None)
         kv = 2.0 * batch * context * 2 * nkv * hd
-        out["palm_attention_decode_fused"] = out["palm_attention_decode"] = (None, None, kv, hbm)
+        out["palm_attention_decode_pages"] = out["palm_attention_decode_fused"] = out["palm_attention_decode"] = (None, None, kv, hbm)
     if "palm_moe_few" in out:                       # a step of up to 16 rows, in the sizes that the stream takes
         out["palm_moe_ring"] = out["palm_moe_few"]
     return out
