@@ -2,8 +2,9 @@
 // whose activations stay in registers (a tile takes 16 a super-step: three tiles hold four steps, two hold six).  They come through the
 // ring: read into registers 16 rows x 64 bytes at a time the 390 KB of 48 rows took a compute unit ten microseconds.  (linear_mid.hip
 // brings the rows through LDS beside the weights, for every 64 or 128 weight rows again.)
-// Us, that kernel and this one, 17 / 32 / 48 rows: 24,576 x 4,096 gated 41 39 39 and 37 37 39, 34,816 x 5,120 gated (up to 32 rows) 85 88
-// and 65 67, 6,144 x 4,096 15 16 16 and 12 12 13, 4,096 x 12,288 22 24 24 and 21 22 22; 4,096 x 4,096 with the norm after it 15 and 10 to 13.
+// Us, that kernel and this one, 17 / 32 / 48 rows: 24,576 x 4,096 gated 36 36 36 and 35 36 38, 34,816 x 5,120 gated (up to 32 rows) 81 84
+// and 58 60, 6,144 x 4,096 13 14 14 and 11 12 13, 4,096 x 12,288 20 21 22 and 20 20 20; 4,096 x 4,096 with the norm after it 15 and 10 to 13 (before the
+// weights' loads of both were marked as read once).
 // (In a file of its own: a program loads a file's kernels when it first runs one of them, which takes milliseconds for these.)
 #include "linear_ring.h"
 

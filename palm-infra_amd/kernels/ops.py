@@ -507,7 +507,8 @@ def mid_pays(M: int, N: int, K: int, planes_ok: bool = False, gated: bool = Fals
     """Whether the kernel that brings both operands through rings in LDS serves this product of bfloat16 operands.
 
     17 to 128 rows (decode steps of many sequences, short prompts): wherever its blocks fill the chip (for few weight
-    rows that needs a reader that takes planes).  Measured at Qwen3-8B's shapes (us, this kernel against that one): 64 rows gate/up gated 46
+    rows that needs a reader that takes planes).  Measured before the weights' loads were marked as read once (64 and 128 rows now: gate/up 38 and 46,
+    down 23 and 31, output projection 10 and 13, q/k/v 15 and 18, head 231 and 289) at Qwen3-8B's shapes (us, this kernel against that one): 64 rows gate/up gated 46
     and 49, down 25 and 27, output projection 11 and 14, q/k/v 16 and 17, head 231 and 275; 128 rows 47 and 67, 30 and
     36, 14 and 17, 19 and 21, 273 and 338 (the tiled kernel 289); 32 rows 42 and 40, 22 and 23, 10 and 11, 14 and 14,
     222 and 252 (a decode step of 32 sequences at Qwen3-32B's sizes 20.7 against 21.3 ms).
@@ -630,9 +631,9 @@ def ring_serves(M: int, N: int, K: int, gated: bool = False, planes_ok: bool = F
 
 def ring_pays(M: int, N: int, K: int, gated: bool = False, planes_ok: bool = False) -> bool:
     """Whether it is also the faster way, against the kernel with both operands in LDS (linear_mid.hip; us, 17, 32 and 48 rows):
-    gate/up of 24,576 x 4,096 gated 40.6 38.9 39.2 and 37.0 37.3 39.0, of 34,816 x 5,120 (up to 32 rows) 85 88 and 65 67, q/k/v of 6,144 x 4,096 15.1 15.5 16.2
-    and 11.9 12.2 13.3, down of 4,096 x 12,288 22.3 23.5 24.0 and 21.2 22.1 21.7, the head 230 231 237 and 219 228 237.  Not where one round of
-    whole strips is all there is (4,096 x 4,096: 9.9 9.5 10.3 and 9.7 10.6 11.9): there every block reads all rows for one strip."""
+    gate/up of 24,576 x 4,096 gated 36.0 35.6 35.8 and 34.6 35.6 37.6, of 34,816 x 5,120 (up to 32 rows) 81 84 and 58 60, q/k/v of 6,144 x 4,096 13.2 13.7 14.3
+    and 11.3 11.6 12.7, down of 4,096 x 12,288 20.3 20.9 21.9 and 19.7 20.4 20.2, the head 203 217 227 and 198 207 212.  Not where one round of
+    whole strips is all there is (4,096 x 4,096: 8.7 9.1 9.6 and 9.1 10.0 11.6): there every block reads all rows for one strip."""
     if K < 2 * RING_STEP_K or not ring_serves(M, N, K, gated, planes_ok):       # (K of one step: not measured)
         return False
     return gated or ring_parts(M, N, K, False, planes_ok) > 1 or (N + 15) // 16 > 1.25 * COMPUTE_UNITS
