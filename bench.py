@@ -167,7 +167,7 @@ def kernel_table(engine, cfg, slots, batch: int, context: int) -> dict:
     seq_slot = torch.tensor(slots, dtype=torch.int32, device=dev)
     seq_start = torch.tensor([cache.lengths[s] - 1 for s in slots], dtype=torch.int32, device=dev)
     bucket = engine._length_bucket(context + 1)
-    n_slices, by_pages = ops.decode_slices(batch, nh, nkv, bucket), ops.decode_pages_pays(batch, nh, nkv, hd, bucket)
+    n_slices, by_pages = ops.decode_slices(batch, nh, nkv, bucket), ops.decode_pages_pays([context + 1] * batch, nh, nkv, hd, bucket)
     # what the attention part runs after its q/k/v projection in a decode step: the projection's planes of partial
     # sums in, per-head norms, rotation, the new key and value into the cache, attention, the merge of the slices
     mixer0 = layers[0].mixer

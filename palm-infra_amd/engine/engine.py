@@ -73,7 +73,7 @@ class Engine:
         self.cache = ModelCache(needs, shares, max_tokens, max_seqs, spec.max_positions, dtype, self.device, page_slack=page_slack)
         self.vocab_size = spec.vocab_size
         self.graphs_enabled = bool(graphs)
-        self._decode_graphs: dict = {}            # (batch bucket, length bucket) -> recorded step, least recently used first
+        self._decode_graphs: dict = {}            # (batch bucket, length bucket, parts' choices) -> recorded step, least recently used first
         self._graph_pool_handle = None
         # A windowed group gives pages back only between steps, so long prompts go through it in pieces: of five windows, or of
         # two where the group has no room for more.  (Every piece reads all weights again: a Nirotar prompt of 2,900 tokens, 4,096
@@ -222,8 +222,9 @@ class Engine:
     # A decode step is some hundred small kernels; launched one by one the host is the bottleneck.  For a
     # batch of single tokens the whole forward pass is recorded once into a HIP graph and replayed with
     # new contents in the same buffers.  A graph is keyed by the batch size, rounded up (rows that pad it
-    # belong to a slot of their own and write into a page that is never read), and by the longest sequence,
-    # rounded up to a power of two (it only sizes how attention cuts the key range).
+    # belong to a slot of their own and write into a page that is never read), by the longest sequence,
+    # rounded up to a power of two (it only sizes how attention cuts the key range), and by what the lengths that
+    # the step really has choose among the parts' kernels (one long sequence beside short ones is not many long ones).
     GRAPH_MAX_BATCH = 128        # as many rows as the products' own kernels take: a recorded step of Qwen3 runs no library code
 
     @staticmethod
@@ -308,8 +309,9 @@ class Engine:
         starts = [cache.lengths[e.slot] for e in entries]
         B = len(entries)
         Bb = self._batch_bucket(B)
-        key = (Bb, self._length_bucket(max(starts) + 1))
         pad = Bb - B
+        longest = self._length_bucket(max(starts) + 1)
+        key = (Bb, longest, self.model.decode_forms(starts + [0] * pad, longest))
         state = self._recorded(key, Bb, Bb, None)
         # the step's arrays, laid out as for any step, at the addresses the recording reads; rows that pad the batch
         # belong to a slot of their own whose page is never read

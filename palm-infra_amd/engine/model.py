@@ -23,6 +23,7 @@ class DecoderModel:
         self.head = builder.build(spec.head)
         self.order = spec.order
         self.weights = weights
+        self._choosing = list(builder.choosing.values())
 
     @property
     def capturable(self) -> bool:
@@ -30,6 +31,10 @@ class DecoderModel:
         that it launches the same kernels whatever the step holds (a part that plans on the host does not)."""
         parts = [self.embedding, *self.layers, self.final_norm, self.head]
         return all(getattr(p, "capturable", False) for p in parts)
+
+    def decode_forms(self, starts: list[int], max_total: int) -> tuple:
+        """What the lengths of a decode step's sequences choose among the parts' kernels: a recorded step serves only steps that choose the same."""
+        return tuple(part.decode_form(starts, max_total) for part in self._choosing)
 
     def cache_plan(self):
         """For each entry of the run order: what it keeps per sequence, and whose cache it reads."""

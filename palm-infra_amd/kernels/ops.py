@@ -12,6 +12,7 @@ from array import array
 from ctypes import c_float, c_int, c_longlong, c_ulonglong, c_void_p
 from dataclasses import dataclass
 
+import numpy as np
 import torch
 
 from . import library, profile
@@ -906,26 +907,36 @@ def decode_pages_serves(n_seqs: int, nh: int, nkv: int, hd: int) -> bool:
     return bool(attention_lib(hd).palm_attention_decode_pages_serves(nh, nkv, n_seqs))
 
 
-def decode_pages_pays(n_seqs: int, nh: int, nkv: int, hd: int, longest: int) -> bool:
-    """Whether it should be: where sequences are many or long (``longest``: the longest one, or what a recorded step is sized for).  Its
-    blocks all read until the end, but they begin some 3 us later than a slice's wave (the cut, the queries through LDS) and add their
-    pieces across dies instead of in a launch of their own.  Us by slices and by pages, head size 128, 32 heads of 8, sequences of equal
-    length or spread evenly.  16,384 keys (sequences times longest) and sequences of 2,048 and more, or 32 of them and more: 8 of 2,000
-    20.3 18.9, of 1,100 15.7 15.0, of 70 to 1,500 13.2 13.4; 4 of 4,000 21.1 19.8, of 2,100 14.8 15.6, of 300 to 4,000 18.9 17.0; 2 of 8,000 21.7
-    21.6; one of 16,000 26.3 23.2; 32 of 260 15.5 14.1, of 500 20.7 17.6; 64 of 130 to 250 21.6 21.6, of 20 to 60 14.0 11.9.  Fewer and shorter ones
-    no: 16 of 30 to 600 11.9 13.2, of 520 14.9 15.2 (of 1,000 20.5 19.2); 8 of 520 to 1,000 13.9 13.6, 48 of 10 to 250 16.6 17.7.  32,768 keys,
-    twelve sequences and more: 24 of 1,000 27.3 24.9, of 700 21.4 20.5, 16 of 70 to 1,500 20.9 20.4, 45 of them 44.9 35.2, 32 of 900 31.5 26.0,
-    64 of 2,048 106.8 100.4; of the shortest, 100 of 20 to 120 17.9 20.0.  A smaller head or fewer kv heads leave a block less to read: head size 64, 16
-    of 70 to 1,500 15.0 14.6, 8 of 1,100 10.0 11.9; 32 heads of 4, 16 of 1,000 14.7 14.9, 8 of 1,100 12.3 14.4.  With more heads a block adds more
-    pieces: 40 heads of 8, 16 of 70 to 1,500 21.3 21.3, 8 of 1,100 15.8 16.9, 16 of 4,000 55.4 50.5, 32 of 1,500 45.0 39.6; 64 heads of 8, 16 of 70 to
-    1,500 21.4 24.6, 40 of 30 to 600 22.3 23.2, 8 of 2,000 21.0 19.9."""
-    keys = 65536
-    if nh <= 4 * nkv:
-        if hd == 128 and nkv >= 8 and (longest >= 2048 or n_seqs >= 32):
-            keys = 16384
-        elif n_seqs >= 12:
-            keys = 32768
-    return n_seqs * longest >= keys and decode_pages_serves(n_seqs, nh, nkv, hd)
+def decode_pages_pays(lengths, nh: int, nkv: int, hd: int, max_keys: int) -> bool:
+    """Whether it should be.  ``lengths``: the keys that each sequence of the step sees, its new one among them; ``max_keys``: what the slices are
+    cut for (the longest sequence, or in a recorded step what it is sized for).
+
+    By slices the step waits for its longest walk: 2.3 us a page, then the merge, 0.15 us for each slice of the longest sequence.  By pages it reads at 7.8
+    bytes a nanosecond at best, and hands pieces from block to block: whoever counts a head's last piece adds up eight records at a time, a round of
+    some 2.4 us, and a block makes the queries of eight sequences at a time, 5 us for each further eight.  So it pays where the longest walk is longer than
+    that (a long sequence in a large batch; not a long one beside few short ones), or where the bytes are many and come from all sequences alike.
+
+    Us by slices and by pages, 32 heads of 8, head size 128, the slices cut for the length rounded up to a power of two: one of 2,100 and three of 20 11.2 and 16.8, one
+    of 2,100 and seven of 100 13.0 14.4, one of 4,000 and seven of 400 22.1 14.8, one of 2,100 and 31 of 100 33.7 14.7; 4 of 2,100 14.8 16.0, of 4,000 20.6 20.2, 8
+    of 1,100 15.4 14.9, of 2,100 20.5 19.4, of 2,500 23.7 20.2, 16 of 30 to 600 11.9 13.2, of 70 to 1,500 20.9 20.4, 45 of them 44.9 35.2, 64 of 2,048 106.8 100.4; 32 of
+    4,000 before 32 of 20 103.7 113.0; one of 4,000 13.0 18.3, of 9,000 19.5 19.4, of 32,000 36.8 31.6.  Over 3,504 batches (1 to 96 sequences of 10 to 130,000 keys, 8 shapes of
+    heads) the way taken is 24.2 % sooner than slices alone in the geometric mean, the better of the two would be 24.6; at 47 it takes pages that are 3 % slower or more, 21 % at worst."""
+    n, group = len(lengths), nh // nkv
+    pages = np.maximum(1, (np.asarray(lengths, dtype=np.int64) + (PAGE_TOKENS - 2)) // PAGE_TOKENS)      # (the new key is no part of the walk)
+    total, longest = int(pages.sum()), int(pages.max())
+    walk = -(-longest // decode_slices(n, nh, nkv, max_keys))
+    runs = min(max(1, COMPUTE_UNITS // nkv), total)              # blocks of a kv head
+    rounds = -(-longest * runs // (8 * total))
+    eights = 1
+    if n > 8 and total > 8 * runs:                               # (a block with more than eight sequences has more than eight pages)
+        ends, cuts = np.cumsum(pages), np.arange(runs + 1) * (total // runs) + np.minimum(np.arange(runs + 1), total % runs)
+        eights = -(-int((np.searchsorted(ends, cuts[1:], "left") - np.searchsorted(ends, cuts[:-1], "right")).max() + 1) // 8)
+    mb = sum(lengths) * nkv * hd * 4e-6
+    late = 2.3 * (0.3 + 0.7 * hd / 128) * walk + 0.145 * -(-longest // walk)
+    if not (late >= 0.6 + 0.2 * group + (2.0 + 0.1 * group) * rounds + 5.0 * (eights - 1) + mb / 7.8
+            or (eights == 1 and mb >= (35 if group <= 4 else 112) * (0.5 + 0.5 * hd / 128) and mb >= 14 * (rounds - 1))):
+        return False
+    return decode_pages_serves(n, nh, nkv, hd)
 
 
 def attention_decode_fused(qkv, k_cache, v_cache, block_table, seq_slot, seq_start, nh: int, nkv: int, hd: int, scale: float,

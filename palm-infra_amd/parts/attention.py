@@ -10,6 +10,8 @@ bias; a specification that names tensors ``qkv_bias`` / ``out_bias`` (float32 ve
 """
 from __future__ import annotations
 
+import torch
+
 from ..cache import KVNeed
 from ..kernels import ops
 from .base import register_part
@@ -46,6 +48,15 @@ class Attention:
             raise ValueError("attention: q_norm and k_norm must be over head_dim with one eps")
         self.position = builder.build(spec.parts["position"]) if "position" in spec.parts else None
         self.dtype = builder.dtype
+        self.decode_shape = (self.nh, self.nkv, self.hd, self.window)
+
+    def decode_form(self, starts: list[int], max_total: int) -> bool:
+        """Whether the attention of a decode step of sequences that hold ``starts`` tokens is cut by pages; ``max_total``: the longest sequence that
+        the step is sized for."""
+        if self.dtype != torch.bfloat16 or self.hd not in ops.MFMA_HEAD_DIMS or len(starts) > ops.DECODE_FUSED_ROWS:
+            return False
+        most = self.window or max_total
+        return ops.decode_pages_pays([min(n + 1, most) for n in starts], self.nh, self.nkv, self.hd, min(max_total, most))
 
     @staticmethod
     def cache_needs(spec):
@@ -54,6 +65,12 @@ class Attention:
 
     takes_sink = True
     takes_prenormed = True
+
+    def _by_pages(self, ctx) -> bool:
+        key = ("by pages", self.decode_shape)                # (asked once for all layers of this shape)
+        if key not in ctx.memo:
+            ctx.memo[key] = self.decode_form(ctx.host["starts"], ctx.max_total)
+        return ctx.memo[key]
 
     def forward(self, h, ctx, sink=None):
         lc = ctx.layer_cache
@@ -72,8 +89,7 @@ class Attention:
                 self.window, ops.slices_of_step(ctx, self.nh, self.nkv, self.window),
                 q_norm_w=self.q_norm.weight if self.q_norm else None, k_norm_w=self.k_norm.weight if self.k_norm else None,
                 eps=self.q_norm.eps if self.q_norm else 0.0, cos=cos, sin=sin, rotary_dim=rotary_dim, pairing=pairing,
-                write_cache=lc.writes, arrivals=lc.kv.arrivals,
-                pages=ops.decode_pages_pays(ctx.n_seqs, self.nh, self.nkv, self.hd, min(ctx.max_total, self.window or ctx.max_total)))
+                write_cache=lc.writes, arrivals=lc.kv.arrivals, pages=self._by_pages(ctx))
             return self.out(o, sink=sink)
         # a prompt's queries carry the scale (times log2 e) into their one rounding where the prompt kernel of this
         # head size takes them so: a score then leaves the matrix cores as the exponent of its weight

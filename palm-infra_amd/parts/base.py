@@ -80,9 +80,13 @@ class Builder:
 
     def __init__(self, weights, dtype: torch.dtype, device):
         self.weights, self.dtype, self.device = weights, dtype, torch.device(device)
+        self.choosing: dict = {}     # parts whose kernels a decode step's lengths choose, one of each ``decode_shape`` (see ``decode_form``)
 
     def build(self, spec: PartSpec):
-        return part_class(spec.category, spec.kind)(spec, self)
+        part = part_class(spec.category, spec.kind)(spec, self)
+        if hasattr(part, "decode_form"):
+            self.choosing.setdefault(part.decode_shape, part)
+        return part
 
     def tensor(self, spec: PartSpec, name: str) -> torch.Tensor:
         return self.weights.get(spec.tensors[name])

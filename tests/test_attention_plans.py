@@ -33,3 +33,37 @@ def test_prompt_attention_of_other_head_sizes_has_no_halves():
 def test_wide_prompt_attention_is_taken_where_it_was_measured_to_be_sooner(starts, counts, nh, nkv, wide):
     from palm_infra_amd.kernels import ops
     assert ops.wide_prompt_attention(starts, counts, nh, nkv) == wide
+
+
+@pytest.mark.parametrize("lengths,nh,nkv,hd,pages", [
+    ([2100] + [20] * 3, 32, 8, 128, False), ([2100] + [100] * 7, 32, 8, 128, False), ([4000] + [20] * 3, 32, 8, 128, False),        # a long one beside few
+    ([2100] * 2 + [100] * 6, 32, 8, 128, False), ([8000] + [100] * 7, 8, 2, 128, False), ([4000] + [400] * 7, 32, 8, 128, True),
+    ([2100] + [100] * 31, 32, 8, 128, True), ([1100] + [20] * 63, 32, 8, 128, True), ([2100] * 4, 32, 8, 128, False), ([4000] * 4, 32, 8, 128, True),
+    ([2049] * 8, 32, 8, 128, True), ([2500] * 8, 32, 8, 128, True), ([4000] * 8, 32, 8, 128, True), ([300] * 8, 32, 8, 128, False), ([70 + 97 * i % 1431 for i in range(45)], 32, 8, 128, True),
+    ([4000] * 32 + [20] * 32, 32, 8, 128, False), ([4000, 20] * 32, 32, 8, 128, True),                    # blocks of many short sequences, or none
+    ([2500] * 8, 32, 8, 64, True), ([1100] * 8, 40, 8, 128, False), ([2048] * 64, 40, 8, 128, True), ([4000], 32, 8, 128, False), ([32000], 32, 8, 128, True),
+    ([1], 32, 8, 128, False), ([1] * 96, 32, 8, 128, False), ([70000] * 8, 32, 8, 80, False), ([70000] * 8, 32, 2, 128, False)])  # not served
+def test_decode_attention_is_cut_by_pages_where_the_keys_that_are_there_make_it_sooner(lengths, nh, nkv, hd, pages):
+    from palm_infra_amd.kernels import ops
+    longest = 256
+    while longest < max(lengths):
+        longest *= 2
+    assert ops.decode_pages_pays(lengths, nh, nkv, hd, longest) == pages
+
+
+def test_a_recorded_step_is_kept_apart_by_the_attention_that_its_lengths_choose():
+    import torch
+
+    from palm_infra_amd.config import config_from_dict
+    from palm_infra_amd.engine import DecoderModel
+    from palm_infra_amd.weights import Weights
+
+    spec = config_from_dict(dict(architectures=["Qwen3ForCausalLM"], vocab_size=64, hidden_size=64, num_hidden_layers=2, num_attention_heads=32,
+                                 num_key_value_heads=8, head_dim=128, intermediate_size=64, tie_word_embeddings=False, rope_theta=10000.0,
+                                 rms_norm_eps=1e-6, max_position_embeddings=8192)).spec()
+    weights = Weights({ref.key: torch.zeros(ref.shape, dtype=torch.float32 if ref.role == "vector" else torch.bfloat16) for ref in spec.tensor_refs()})
+    model = DecoderModel(spec, weights, torch.bfloat16, "cpu")
+    assert model.decode_forms([2099] * 8, 4096) == (True,)                       # one answer for the layers of one shape
+    assert model.decode_forms([2099] + [19] * 7, 4096) == (False,)
+    assert model.decode_forms([2099] * 97, 4096) == (False,)                      # more rows than start from the projection
+    assert DecoderModel(spec, weights, torch.float32, "cpu").decode_forms([2099] * 8, 4096) == (False,)

@@ -234,3 +234,38 @@ def test_short_prompts_of_one_sequence_are_recorded_too(model_dirs, name, dtype)
     g.step([StepEntry(s2, list(range(1, 65)), [63])])
     assert {k: st["calls"] for k, st in g._decode_graphs.items()} == before
     g.cache.check()
+
+
+def test_recorded_steps_whose_attention_is_cut_by_pages():
+    """A long sequence in a batch of short ones grows until its attention is cut by pages; the batch is padded, shrinks and grows again, so that
+    several recorded steps of either kind run in turn and each is replayed.  Against an engine that takes slices throughout: where the attention's last
+    rounding falls apart (2^-9 of an element, for some elements, in each of three layers) the logits differ by some 0.002."""
+    from palm_infra_amd.config import config_from_dict
+    from palm_infra_amd.engine import Engine, StepEntry
+    raw = dict(architectures=["Qwen3ForCausalLM"], vocab_size=300, hidden_size=256, num_hidden_layers=3, num_attention_heads=16, num_key_value_heads=8,
+               head_dim=128, intermediate_size=256, tie_word_embeddings=False, rope_theta=10000.0, rms_norm_eps=1e-6, max_position_embeddings=4096)
+    lengths = [379, 764] + [40 + i for i in range(10)]
+    g, e = (Engine.from_config(config_from_dict(raw), seed=5, max_tokens=64 * 64, max_seqs=16) for _ in range(2))
+    e.model.decode_forms = lambda starts, longest: (False,)
+    for mixer in (layer.mixer for layer in e.model.layers):
+        mixer.decode_form = lambda starts, longest: False
+    slots = [[eng.open() for _ in lengths] for eng in (g, e)]
+    for eng, held in zip((g, e), slots):
+        eng.step([StepEntry(s, [(7 * i + 3 * t) % 300 for t in range(n)], []) for i, (s, n) in enumerate(zip(held, lengths))])
+    seen, fed = [], 0
+    short = list(range(2, 12))
+    for t in range(40):
+        # the long one of 379 with ten others, without one of them and with it again; the one of 764 takes its place now and then
+        live = [1 if t % 5 == 3 else 0] + short[:10 - (t // 4) % 3]
+        a, b = (eng.step([StepEntry(held[i], [(11 * t + i) % 300], [0]) for i in live]) for eng, held in zip((g, e), slots))
+        seen.append(next(reversed(g._decode_graphs)))
+        assert float((a - b).norm() / b.norm()) < 0.01, (t, seen[-1])
+        if not seen[-1][2][0]:
+            assert torch.equal(a, b) or fed, (t, "the same kernels, from caches that steps by pages have not touched yet")
+        fed += seen[-1][2][0]
+        if t % 6 == 2:
+            torch.cuda.synchronize()
+    for by_pages in (True, False):                              # steps of both kinds, recorded and replayed
+        assert any(k[2] == (by_pages,) and st["graph"] is not None and st["calls"] > 2 for k, st in g._decode_graphs.items()), seen
+    assert len({k for k in seen if k[2] == (True,)}) >= 2 and all(k[2] == (False,) for k in e._decode_graphs)
+    g.cache.check()
