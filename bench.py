@@ -168,6 +168,7 @@ def kernel_table(engine, cfg, slots, batch: int, context: int) -> dict:
     seq_start = torch.tensor([cache.lengths[s] - 1 for s in slots], dtype=torch.int32, device=dev)
     bucket = engine._length_bucket(context + 1)
     n_slices, by_pages = ops.decode_slices(batch, nh, nkv, bucket), ops.decode_pages_pays([context + 1] * batch, nh, nkv, hd, bucket)
+    arrivals = torch.zeros((batch * nh,), dtype=torch.int32, device=dev)       # zero between launches
     # what the attention part runs after its q/k/v projection in a decode step: the projection's planes of partial
     # sums in, per-head norms, rotation, the new key and value into the cache, attention, the merge of the slices
     mixer0 = layers[0].mixer
@@ -178,7 +179,7 @@ def kernel_table(engine, cfg, slots, batch: int, context: int) -> dict:
         m = layers[i].mixer
         return ops.attention_decode_fused(qkv, kv.k[i], kv.v[i], kv.table_dev, seq_slot, seq_start, nh, nkv, hd, m.scale, None,
                                           n_slices, q_norm_w=m.q_norm.weight, k_norm_w=m.k_norm.weight, eps=m.q_norm.eps,
-                                          cos=cos, sin=sin, rotary_dim=hd, pairing=0, pages=by_pages, arrivals=kv.arrivals)
+                                          cos=cos, sin=sin, rotary_dim=hd, pairing=0, pages=by_pages, arrivals=arrivals)
 
     def each_layer(fn):
         return lambda: [fn(i) for i in range(L)]

@@ -144,9 +144,6 @@ class KVGroup(PagedGroup):
                              device=device)
         self.v = torch.zeros((n_entries, n_pages + 1, need.value_heads or need.num_kv_heads, need.value_dim or need.head_dim,
                               PAGE_TOKENS), dtype=dtype, device=device)
-        # Counters, zero between launches, by which the blocks of a decode step's attention tell whose piece of a (sequence, head) is the
-        # last: 128 sequences and eight query heads a kv head at most.  One set for all layers of the group, whose launches follow each other.
-        self.arrivals = torch.zeros((128 * 8 * need.num_kv_heads,), dtype=torch.int32, device=device)
 
     def nbytes(self) -> int:
         return (self.k.numel() + self.v.numel()) * self.k.element_size()

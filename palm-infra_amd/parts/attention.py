@@ -72,6 +72,14 @@ class Attention:
             ctx.memo[key] = self.decode_form(ctx.host["starts"], ctx.max_total)
         return ctx.memo[key]
 
+    def _arrivals(self, ctx) -> torch.Tensor:
+        """The counters of the attention cut by pages, zero before a launch and after it.  A step's layers follow each other and share them; another step
+        may run beside this one, on another stream, so each has its own."""
+        key = ("arrivals", self.nh)
+        if key not in ctx.memo:
+            ctx.memo[key] = torch.zeros((ctx.n_seqs * self.nh,), dtype=torch.int32, device=ctx.seq_slot.device)
+        return ctx.memo[key]
+
     def forward(self, h, ctx, sink=None):
         lc = ctx.layer_cache
         if lc is None or lc.kv is None:
@@ -84,12 +92,13 @@ class Attention:
         if ctx.is_decode and ops.decode_fused_serves(qkv, self.hd, self.dtype, rotary_dim, pairing):
             # one token a sequence: its slot and position are the sequence's, and the q/k/v pass rides in the
             # attention kernel
+            pages = self._by_pages(ctx)
             o = ops.attention_decode_fused(
                 qkv, lc.k, lc.v, lc.kv.table_dev, ctx.seq_slot, ctx.seq_start, self.nh, self.nkv, self.hd, self.scale,
                 self.window, ops.slices_of_step(ctx, self.nh, self.nkv, self.window),
                 q_norm_w=self.q_norm.weight if self.q_norm else None, k_norm_w=self.k_norm.weight if self.k_norm else None,
                 eps=self.q_norm.eps if self.q_norm else 0.0, cos=cos, sin=sin, rotary_dim=rotary_dim, pairing=pairing,
-                write_cache=lc.writes, arrivals=lc.kv.arrivals, pages=self._by_pages(ctx))
+                write_cache=lc.writes, pages=pages, arrivals=self._arrivals(ctx) if pages else None)
             return self.out(o, sink=sink)
         # a prompt's queries carry the scale (times log2 e) into their one rounding where the prompt kernel of this
         # head size takes them so: a score then leaves the matrix cores as the exponent of its weight

@@ -67,3 +67,18 @@ def test_a_recorded_step_is_kept_apart_by_the_attention_that_its_lengths_choose(
     assert model.decode_forms([2099] + [19] * 7, 4096) == (False,)
     assert model.decode_forms([2099] * 97, 4096) == (False,)                      # more rows than start from the projection
     assert DecoderModel(spec, weights, torch.float32, "cpu").decode_forms([2099] * 8, 4096) == (False,)
+
+
+def test_steps_beside_each_other_share_no_counters():
+    """The layers of a step follow each other and share the counters of the attention cut by pages; another step may run on another stream meanwhile."""
+    import torch
+
+    from palm_infra_amd.parts import make_context
+    from palm_infra_amd.parts.attention import Attention
+
+    part = Attention.__new__(Attention)
+    part.nh = 4
+    one, other = (make_context([0, 1, 2], [5, 6, 7], [[1]] * 3, torch.bfloat16, "cpu") for _ in range(2))
+    counters = part._arrivals(one)
+    assert counters.dtype == torch.int32 and counters.numel() == 12 and not counters.any()
+    assert part._arrivals(one) is counters and part._arrivals(other).data_ptr() != counters.data_ptr()
