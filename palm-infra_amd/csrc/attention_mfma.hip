@@ -724,8 +724,9 @@ PALM_API int palm_attention_decode_fused(hipStream_t stream, const void* qkv, in
 // ---- decode cut by pages ------------------------------------------------------------------------------
 #include "attention_decode_pages.h"
 
-PALM_API int palm_attention_decode_pages_serves(int nh, int nkv, int n_seqs) {
-    return PAGES_SERVE_HEAD && nkv > 0 && nkv <= 65535 && nh / nkv <= DP_HEADS && n_seqs <= DP_SEQS;
+// max_pages: of a slot, as the block table has them (the cut divides numbers of pages of a step that are exact as floats, see quotient)
+PALM_API int palm_attention_decode_pages_serves(int nh, int nkv, int n_seqs, int max_pages) {
+    return PAGES_SERVE_HEAD && nkv > 0 && nkv <= 65535 && nh / nkv <= DP_HEADS && n_seqs <= DP_SEQS && (long long)n_seqs * max_pages < 1 << 24;
 }
 
 // What `work` has to hold, in floats.
@@ -745,9 +746,9 @@ PALM_API int palm_attention_decode_pages(hipStream_t stream, const void* qkv, in
                "attention_decode_pages: head size %d with rotation over %d (pairing %d) is not served", HD, rotary_dim, pairing);
     PALM_CHECK((q_norm_w == nullptr) == (k_norm_w == nullptr), "attention_decode_pages: q and k norm weights come together");
     PALM_CHECK(n_seqs >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0, "attention_decode_pages: seqs=%d heads=%d kv=%d", n_seqs, nh, nkv);
-    PALM_CHECK(palm_attention_decode_pages_serves(nh, nkv, n_seqs), "attention_decode_pages: head size %d, %d heads of %d, %d sequences are not served",
-               HD, nh, nkv, n_seqs);
-    PALM_CHECK(window >= 0 && max_pages > 0 && max_pages < (1 << 24) / DP_SEQS, "attention_decode_pages: window=%d max_pages=%d", window, max_pages);
+    PALM_CHECK(palm_attention_decode_pages_serves(nh, nkv, n_seqs, max_pages),
+               "attention_decode_pages: head size %d, %d heads of %d, %d sequences of up to %d pages are not served", HD, nh, nkv, n_seqs, max_pages);
+    PALM_CHECK(window >= 0 && max_pages > 0, "attention_decode_pages: window=%d max_pages=%d", window, max_pages);
     PALM_CHECK(planes >= 1 && (qkv_is_planes || planes == 1), "attention_decode_pages: %d planes of whole rows", planes);
     if (n_seqs == 0) return 0;
     PALM_CHECK(work && arrivals, "attention_decode_pages: a workspace and counters are needed");

@@ -807,7 +807,7 @@ _ATTENTION_SIGNATURES = {
     "palm_attention_decode_pages": [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
                                     c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                                     c_int, c_float, c_int, c_void_p, c_void_p, c_void_p],
-    "palm_attention_decode_pages_serves": [c_int, c_int, c_int],
+    "palm_attention_decode_pages_serves": [c_int, c_int, c_int, c_int],
     "palm_attention_decode_pages_work": [c_int, c_int],
     "palm_attention_decode_fused_serves": [c_int, c_int],
 }
@@ -902,9 +902,10 @@ def decode_fused_serves(qkv: torch.Tensor, hd: int, out_dtype, rotary_dim: int, 
     return bool(attention_lib(hd).palm_attention_decode_fused_serves(int(rotary_dim), int(pairing)))
 
 
-def decode_pages_serves(n_seqs: int, nh: int, nkv: int, hd: int) -> bool:
-    """Whether a decode step's attention may be cut by pages: head sizes 64 and 128, up to eight query heads a kv head, 128 sequences."""
-    return bool(attention_lib(hd).palm_attention_decode_pages_serves(nh, nkv, n_seqs))
+def decode_pages_serves(n_seqs: int, nh: int, nkv: int, hd: int, max_pages: int) -> bool:
+    """Whether a decode step's attention may be cut by pages: head sizes 64 and 128, up to eight query heads a kv head, 128 sequences, and tables
+    (``max_pages``: a slot's pages) with which the step cannot hold 2^24 pages."""
+    return bool(attention_lib(hd).palm_attention_decode_pages_serves(nh, nkv, n_seqs, max_pages))
 
 
 def decode_pages_pays(lengths, nh: int, nkv: int, hd: int, max_keys: int) -> bool:
@@ -936,7 +937,7 @@ def decode_pages_pays(lengths, nh: int, nkv: int, hd: int, max_keys: int) -> boo
     if not (late >= 0.6 + 0.2 * group + (2.0 + 0.1 * group) * rounds + 5.0 * (eights - 1) + mb / 7.8
             or (eights == 1 and mb >= (35 if group <= 4 else 112) * (0.5 + 0.5 * hd / 128) and mb >= 14 * (rounds - 1))):
         return False
-    return decode_pages_serves(n, nh, nkv, hd)
+    return decode_pages_serves(n, nh, nkv, hd, longest)
 
 
 def attention_decode_fused(qkv, k_cache, v_cache, block_table, seq_slot, seq_start, nh: int, nkv: int, hd: int, scale: float,

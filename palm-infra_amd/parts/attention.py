@@ -92,7 +92,7 @@ class Attention:
         if ctx.is_decode and ops.decode_fused_serves(qkv, self.hd, self.dtype, rotary_dim, pairing):
             # one token a sequence: its slot and position are the sequence's, and the q/k/v pass rides in the
             # attention kernel
-            pages = self._by_pages(ctx)
+            pages = self._by_pages(ctx) and ops.decode_pages_serves(ctx.n_seqs, self.nh, self.nkv, self.hd, lc.kv.table_dev.shape[1])
             o = ops.attention_decode_fused(
                 qkv, lc.k, lc.v, lc.kv.table_dev, ctx.seq_slot, ctx.seq_start, self.nh, self.nkv, self.hd, self.scale,
                 self.window, ops.slices_of_step(ctx, self.nh, self.nkv, self.window),

@@ -82,3 +82,16 @@ def test_steps_beside_each_other_share_no_counters():
     counters = part._arrivals(one)
     assert counters.dtype == torch.int32 and counters.numel() == 12 and not counters.any()
     assert part._arrivals(one) is counters and part._arrivals(other).data_ptr() != counters.data_ptr()
+
+
+@pytest.mark.parametrize("n_seqs,max_pages,served", [(96, 174762, True), (96, 174763, False), (1, (1 << 24) - 1, True), (1, 1 << 24, False), (128, 131071, True), (128, 131072, False), (0, 4, True)])
+def test_decode_attention_by_pages_says_which_tables_it_takes(n_seqs, max_pages, served):
+    """What is not served is known before the launch, so that a step goes by slices instead of ending in an error."""
+    from palm_infra_amd.kernels import ops
+    assert ops.decode_pages_serves(n_seqs, 32, 8, 128, max_pages) == served
+    lib = ops.attention_lib(128)
+    # (the workspace is looked for last)
+    assert lib.palm_attention_decode_pages(None, None, 0, 1, None, None, 0.0, None, None, 0, 0, 1, None, None, None, max_pages, None, None, n_seqs, 32, 8, 128, 1.0, 0,
+                                           None, None, None) == (0 if n_seqs == 0 else -1)
+    if n_seqs:
+        assert ("a workspace and counters" if served else "not served") in lib.palm_last_error().decode()
