@@ -104,7 +104,8 @@ struct BigItem {
 // in both.  finish(i, acc, live): acc[4 half + f][t][v], lane (r, g) of wave (wave_f, wave_t) = (wave % 2, wave / 2): token
 // wave_t * 32 NT + 16 t + r, tile row 128 wave_f + 64 half + 16 g + 4 f + v.
 // RAGGED (of the high tiles): a tile's last column tiles may be nobody's.  They are neither read from LDS nor multiplied, each number of
-// them in a loop of its own, from half a tile on (below that the loads of a stage have no products left to stand between); their sums are zero.
+// them in a loop of its own, from half a tile on (below that the loads of a stage have no products left to stand between).  finish gets their
+// number as a constant, `live`: sums from acc[..][live] on were never set and are not to be read.
 template <int NT, bool TURNED, bool RAGGED = false, class Make, class XRow, class WRow, class Finish>
 __device__ __forceinline__ void big_walk(char* lds, uint32_t row_bytes, int items, Make make, XRow x_row, WRow w_row, Finish finish) {
     constexpr int TT = 2 * NT, W_STAGE = BIG_FEAT * BIG_ROW, X_STAGE = 64 * NT * BIG_ROW, A = big_ahead(NT);

@@ -97,6 +97,7 @@ __global__ __launch_bounds__(BIG_THREADS) __attribute__((amdgpu_waves_per_eu(1, 
             return GATED ? (row & 64 ? s.inter : 0) + min(row / 128 * 64 + row % 64, it.w_rows - 1) : min(row, it.w_rows - 1);
         },
         [&](int item, f32x4 (&acc)[8][2 * NT], auto live) __attribute__((always_inline)) {
+            static_assert(decltype(live)::value == 2 * NT, "every column's sums are there");
             f32x4 a[8];
             if (item < mine) {
                 const BigPlace place = BigPlace::of<NT>(s, tile_of(item));

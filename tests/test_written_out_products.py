@@ -107,6 +107,22 @@ def too_near(code, following):
 
 
 @pytest.fixture(scope="module")
+def large_tiles(tmp_path_factory):
+    return {source: assembly(source, [], tmp_path_factory.mktemp("assembly") / f"{source}.s") for source in ("linear_big.hip", "moe_grouped.hip")}
+
+
+@pytest.mark.parametrize("source,name,products", [("linear_big.hip", f"linear_big_kernelILi{nt}ELb{gated}E", 32 * nt) for nt in (2, 3, 4) for gated in (0, 1)]
+                         + [("moe_grouped.hip", f"moe_big_kernelILi{nt}ELi{form}E{to}", 32 * nt) for nt in (1, 2, 3) for form, to in ((0, "f"), (0, "6bf16_t"), (2, ""))]
+                         + [("moe_grouped.hip", f"moe_big_kernelILi4ELi{form}E{to}", 16 * (8 + 7 + 6 + 5 + 4))                # a walk for each number of columns
+                            for form, to in ((0, "f"), (0, "6bf16_t"), (1, ""), (2, ""), (3, ""), (4, ""))])
+def test_large_tiles_keep_their_products_distances_and_keep_nothing_in_memory(large_tiles, source, name, products):
+    code, following = kernel(large_tiles[source], name)
+    assert sum(one.written_out for one in code) == products
+    assert too_near(code, following) == []
+    assert not any(one.name.startswith("scratch_") for one in code)
+
+
+@pytest.fixture(scope="module")
 def attention_of_heads_of_128(tmp_path_factory):
     return assembly("attention_mfma.hip", ["PALM_HEAD_DIM=128"], tmp_path_factory.mktemp("assembly") / "attention.s")
 
