@@ -883,9 +883,9 @@ def test_attention_decode_fused_sees_its_own_key_and_leaves_a_read_only_cache_al
 
 @pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (40, 8, 128), (8, 1, 128), (3, 3, 128), (12, 4, 64), (7, 1, 64), (600, 300, 64)])
 def test_attention_decode_cut_by_pages_is_the_two_kernels_in_one(ops, nh, nkv, hd):
-    """Runs that end with a sequence, inside one and a page from either end; fewer pages than blocks; blocks that hold more sequences than make
-    their queries at once (a long one beside 70 of a token); more than 64 sequences; rows as bfloat16 and as planes; windows; stale values.
-    The counters are zero again, and a second call gives the same bits."""
+    """Runs that end with a sequence, inside one and a page from either end; fewer pages than blocks, and up to eight pages a block, one a wave; sequences
+    that all blocks share; more than 64 sequences; rows as bfloat16 and as planes; windows; stale values.  The counters are zero again, and
+    a second call gives the same bits.  (Longer runs: the test below.)"""
     if nkv > 8:
         cases = [(2, [64, 1, 200], None)]                                # more kv heads than blocks
     else:
@@ -901,6 +901,60 @@ def test_attention_decode_cut_by_pages_is_the_two_kernels_in_one(ops, nh, nkv, h
         _same_caches(finite(ca), finite(cb))
         assert not counters.any()
         assert torch.equal(run()[0], one)
+
+
+def _pages_cut(lengths, nkv, window):
+    """What the kernel's blocks and waves of one kv head get, cut as it cuts: for each wave the (sequence, pages of it, all of it) in its run, for each block its sequences."""
+    pages = []
+    for L in lengths:
+        first = max(0, L - window) if window else 0
+        pages.append(max(L - 2, first) // 64 - first // 64 + 1)
+    row = [b for b, n in enumerate(pages) for _ in range(n)]
+    even = lambda n, runs: [i * (n // runs) + min(i, n % runs) for i in range(runs + 1)]
+    ends = [sum(pages[:b + 1]) for b in range(len(pages))]
+    cuts = even(len(row), min(max(1, 256 // nkv), len(row)))
+    waves, blocks = [], []
+    for i0, i1 in zip(cuts, cuts[1:]):
+        blocks.append(sorted(set(row[i0:i1])))
+        while i0 < i1:
+            c1 = min(i1, ends[min(row[i0] + 7, len(ends) - 1)])                # as many sequences as make their queries at once
+            at = [i0 + w for w in even(c1 - i0, 8)]
+            for w0, w1 in zip(at, at[1:]):
+                held = row[w0:w1]
+                waves.append([(b, held.count(b), held.count(b) == pages[b]) for b in sorted(set(held))])
+            i0 = c1
+    return waves, blocks
+
+
+@pytest.mark.parametrize("nh,nkv,hd,cases", [
+    (32, 8, 128, [(2, [70 + 97 * i % 1431 for i in range(45)], None), (0, [2500] * 16, None)]),
+    (12, 4, 64, [(3, [3000] * 20 + [1 + 13 * i % 65 for i in range(60)], None)]),
+    (128, 64, 64, [(2, [1 + 97 * i % 401 for i in range(40)], None), (1, [130 + 7 * i for i in range(64)], 130), (0, [1 + 29 * i % 301 for i in range(128)], None),
+                   (2, [640] * 7 + [1] * 20 + [129], 200)]),
+    (32, 32, 128, [(2, [60] * 63 + [512], None), (0, [512] + [1] * 90 + [300], 64), (1, [70 + 97 * i % 431 for i in range(30)], None)]),
+    (600, 300, 64, [(2, [1] * 20, None), (0, [700] + [1] * 20 + [300], None), (1, [64, 65, 66, 200] * 6, 70)])])
+def test_attention_decode_cut_by_pages_in_runs_of_many_pages_and_sequences(ops, nh, nkv, hd, cases):
+    """Several pages a wave, across the ends of sequences; sequences that one wave finishes after several pages; blocks of more sequences than make their
+    queries at once, whose run goes piece by piece.  That the cases have all this is counted."""
+    waves, blocks = [], []
+    for i, (planes, lengths, window) in enumerate(cases):
+        of_case = _pages_cut(lengths, nkv, window)
+        waves += of_case[0]
+        blocks += of_case[1]
+        counters = torch.zeros(len(lengths) * nh, dtype=torch.int32, device=DEV)
+        run = lambda: _fused_case(ops, nh, nkv, hd, lengths, 1, planes, window=window, seed=hd + i, poison=True, pages=True, arrivals=counters)
+        one, two, ca, cb, _ = run()
+        assert torch.isfinite(one).all() and _one_ulp(one, two), (planes, lengths, window, float((one - two).abs().max()))
+        finite = lambda cs: [torch.nan_to_num(c.float(), nan=0.0, posinf=0.0, neginf=0.0) for c in cs]
+        _same_caches(finite(ca), finite(cb))
+        assert not counters.any()
+        assert torch.equal(run()[0], one)
+    reached = (max(sum(n for _, n, _ in w) for w in waves), max(len(w) for w in waves), max(len(b) for b in blocks))
+    assert reached == {8: (3, 2, 5), 4: (2, 2, 15), 64: (5, 3, 33), 32: (3, 2, 12), 300: (3, 2, 24)}[nkv]        # pages and sequences a wave, sequences a block
+    finished = [n for w in waves for _, n, whole in w if whole]
+    assert (max(finished) >= 2) == (nkv != 4)
+    if nkv in (8, 64, 32):
+        assert any(len(w) >= 2 and w[0][1] >= 2 for w in waves) and any(len(w) >= 2 and w[-1][1] >= 2 for w in waves)       # pages before and behind the switch
 
 
 def test_attention_decode_cut_by_pages_reads_a_cache_that_is_not_its_own(ops):
