@@ -207,8 +207,8 @@ struct RingPlaces {
         lds_reads_done();                                                  // the slot may be the one they read
 #pragma unroll
         for (int i = 0; i < DP_LOADS; ++i) {
-            if (part < 4) row_chunk_into_lds_once(in_scalars(keys + (part / 2 * 32 + part % 2 * 4) * (HD * 2)), ask_k[i], lds + i * 1024);
-            else row_chunk_into_lds_once(in_scalars(values + (part - 4) * DP_SLOT + i * 1024), ask_v, lds + i * 1024);
+            if (part < 4) row_chunk_into_lds<true>(in_scalars(keys + (part / 2 * 32 + part % 2 * 4) * (HD * 2)), ask_k[i], lds + i * 1024);
+            else row_chunk_into_lds<true>(in_scalars(values + (part - 4) * DP_SLOT + i * 1024), ask_v, lds + i * 1024);
         }
     }
 };

@@ -7,12 +7,12 @@ __device__ __forceinline__ void row_chunk_into_lds(const void* from, uint32_t ld
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds_base) : "m0", "memory");
 }
 // the same from a base that all lanes share and a lane's own offset
-__device__ __forceinline__ void row_chunk_into_lds(const char* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
-}
-// the same for what passes once: marked as a stream (nt), it does not push out of the caches what is read again
-__device__ __forceinline__ void row_chunk_into_lds_once(const char* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+// ONCE: for what passes once, marked as a stream (nt) that does not push out of the caches what is read again
+template <bool ONCE = false> __device__ __forceinline__ void row_chunk_into_lds(const char* base, uint32_t offset, uint32_t lds_base) {
+    if constexpr (ONCE)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
 }
 // For a ring that one wave fills and reads without a barrier: its reads of LDS are in registers; reads stay behind a wait.
 __device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }

@@ -385,7 +385,7 @@ static void dispatch_stream(hipStream_t stream, const void* a, const void* w, vo
 
 template <typename TC, int EPI>
 static void dispatch_thin(hipStream_t stream, const void* a, const void* w, void* c, int M, int N, int K, int parts,
-                          const RowNorm& norm) {
+                          const RowNorm& norm, bool once) {
     const int n_super = (K + SUPER_K - 1) / SUPER_K;
     const bool deep = n_super >= 16;                           // enough super-steps to feed a block's waves
     const bool folded = norm.ss_in || norm.resid;              // only the stream kernel folds a norm in
@@ -393,7 +393,7 @@ static void dispatch_thin(hipStream_t stream, const void* a, const void* w, void
         const int per_wave = stream_steps(n_super, parts);
         // eight waves: the stream whose weights cross LDS; four (a short K): the one that reads them into registers
         if (stream_waves(n_super) == 8)
-            launch_linear_ring(stream, a, w, c, sizeof(TC) == 2 ? PALM_BF16 : PALM_F32, M, N, K, EPI, parts, per_wave, norm);
+            (once ? launch_linear_ring_once : launch_linear_ring)(stream, a, w, c, sizeof(TC) == 2 ? PALM_BF16 : PALM_F32, M, N, K, EPI, parts, per_wave, norm);
         else
             dispatch_stream<4, TC, EPI>(stream, a, w, c, M, N, K, parts, norm, per_wave);
         return;
@@ -404,7 +404,7 @@ static void dispatch_thin(hipStream_t stream, const void* a, const void* w, void
 
 PALM_API int palm_linear_thin_parts(int M, int N, int K) { return stream_parts(M, N, K); }
 
-// a [M, K] bfloat16, w [N, K] bfloat16; c [M, N] (EPI_STORE) or [M, N/2] (EPI_SWIGLU) in bfloat16 or float32.
+// a [M, K] bfloat16, w [N, K] bfloat16; c [M, N] (EPI_STORE) or [M, N/2] (EPI_SWIGLU) in bfloat16 or float32.  EPI_ONCE may be added to the epilogue.
 // parts > 1 (at most palm_linear_thin_parts(M, N, K), float32, EPI_STORE): c is [parts, M, N] and the product is
 // the sum of its planes.
 // ss_in (with pieces_in, eps_in, width_in = K) and resid (with w_out, ss_out) fold a norm in, see RowNorm; both
@@ -413,6 +413,8 @@ PALM_API int palm_linear_thin(hipStream_t stream, const void* a, const void* w, 
                               int K, int epilogue, int parts, const float* ss_in, int pieces_in, float eps_in,
                               float* resid, const float* w_out, float* ss_out) {
     PALM_CHECK(parts >= 1, "linear_thin: parts = %d", parts);
+    const bool once = epilogue & EPI_ONCE;
+    epilogue &= ~EPI_ONCE;
     RowNorm norm{ss_in, pieces_in, eps_in, K, resid, w_out, ss_out};
     PALM_CHECK(!(ss_in || resid) || M <= 16, "linear_thin: a norm is folded in for at most 16 rows, not %d", M);
     PALM_CHECK(!ss_in || pieces_in > 0, "linear_thin: %d pieces of the rows' sums of squares", pieces_in);
@@ -431,9 +433,9 @@ PALM_API int palm_linear_thin(hipStream_t stream, const void* a, const void* w, 
     if (M == 0) return 0;
     PALM_CHECK(M <= 16, "linear_thin: %d rows are more than the 16 of one block of tokens (linear_wide takes up to 64)", M);
     if (epilogue == EPI_SWIGLU) {
-        PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_thin<TC, EPI_SWIGLU>(stream, a, w, c, M, N, K, 1, norm));
+        PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_thin<TC, EPI_SWIGLU>(stream, a, w, c, M, N, K, 1, norm, once));
     } else {
-        PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_thin<TC, EPI_STORE>(stream, a, w, c, M, N, K, parts, norm));
+        PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_thin<TC, EPI_STORE>(stream, a, w, c, M, N, K, parts, norm, once));
     }
     PALM_LAUNCHED();
     return 0;

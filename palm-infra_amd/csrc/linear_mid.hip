@@ -30,6 +30,7 @@
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 enum MidEpilogue : int { MID_STORE = 0, MID_SWIGLU = 1 };
+constexpr int MID_ONCE = 16;                    // added to the epilogue: the weights pass once (linear_thin.h's EPI_ONCE)
 
 constexpr int MID_MAX_ROWS = 256;               // rows of A a block holds: 64, 128 or 256
 constexpr int MID_WAVES = 4;
@@ -42,17 +43,18 @@ constexpr int MID_MAX_PARTS = 4;
 constexpr int MID_UNITS = 256;                  // compute units of the chip
 
 // 16 bytes a lane from memory into LDS, the 64 lanes' pieces side by side from lds_base on.  base is the same in every
-// lane (scalar registers), offset the lane's own.
-__device__ __forceinline__ void mid_load_16_bytes_a_lane_into_lds(const void* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
-}
-// The same for the weights, which pass once (linear_ring.h: nt).  Us without and with it: 64 rows, 4,096 x 12,288 25.9 and 23.5,
-// 5,120 x 17,408 42.9 and 39.2, 24,576 x 4,096 gated 41.6 and 39.5, 6,144 x 4,096 16.6 and 15.2; 91 and 128 rows, the same 29.6 32.2 and
-// 28.6 31.5, 49.5 53.4 and 48.4 52.6, 44.0 46.7 and 42.0 43.4, 17.0 19.5 and 16.2 18.3; 4,096 x 4,096 12.6 14.1 and 13.0 14.2.
-// What is left is neither LDS nor the matrix cores (without their work the same time): the weights alone take 35 us of those 42 to 43
+// lane (scalar registers), offset the lane's own.  ONCE: marked as a stream (nt), for weights that the memory-side cache does not hold until they are
+// read again (linear_ring.h).  Us, plain and marked, matrices read in turn, of 3 GB and of 96 to 240 MB together, 64 / 91 / 128 rows: 24,576 x 4,096
+// gated 39.2 45.6 47.0, 38.0 45.5 47.3 and 30.5 39.7 41.6, 38.5 45.4 46.6; 4,096 x 12,288 22.7 27.9 29.8, 22.0 27.3 29.2 and 20.0 24.7 26.0, 23.2 29.1 31.7; 6,144 x 4,096
+// 14.8 16.7 18.1, 14.7 16.2 17.7 and 13.0 15.5 17.2, 16.6 17.4 18.6; 4,096 x 4,096 9.5 11.9 13.3, 9.2 11.8 12.9 and 9.4 11.8 12.6, 10.4 12.9 13.4; 12,288 x 2,048 gated
+// 13.4 16.4 17.4, 13.3 16.3 17.4 and 12.4 15.9 15.9, 15.4 18.1 18.8.
+// With 3 GB in turn neither LDS nor the matrix cores bound it (without their work the same time): at 91 rows the gated product's weights alone take 35 us
 // (5.7 TB/s), the rows alone, which every block reads again from L2, 29.
-__device__ __forceinline__ void mid_load_16_bytes_a_lane_into_lds_once(const void* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+template <bool ONCE = false> __device__ __forceinline__ void mid_load_16_bytes_a_lane_into_lds(const void* base, uint32_t offset, uint32_t lds_base) {
+    if constexpr (ONCE)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
 }
 template <int N> __device__ __forceinline__ void mid_wait_for_all_but_the_youngest_loads() {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));          // s_waitcnt vmcnt(N)
@@ -75,10 +77,10 @@ __device__ inline f32x16 mfma_32x32x16(bf16x8 a, bf16x8 b, f32x16 acc) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
 }
 
-// R: rows of A a block holds.  TN: weight rows it holds (a multiple of 32; of 64 for 64 rows).  TC: element type of the
+// ONCE: see mid_load_16_bytes_a_lane_into_lds (a branch instead: kept weights, 64 rows, 5 % longer).  R: rows of A a block holds.  TN: weight rows it holds (a multiple of 32; of 64 for 64 rows).  TC: element type of the
 // result.  With 256 rows a wave has 64 of them (two tiles of 32) against all weight rows, with 128 rows 32 of them;
 // with 64 rows a wave has 32 rows against half of the weight rows.
-template <int R, int TN, typename TC, int EPI>
+template <int R, int TN, bool ONCE, typename TC, int EPI>
 __global__ __launch_bounds__(MID_THREADS) void linear_mid_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, TC* __restrict__ C, int M, int N, int K,
     int n_tiles, int m_tiles, int chunks_per_part, int turn_blocks) {
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(MID_THREADS) void linear_mid_kernel(
         const char* base = reinterpret_cast<const char*>(W) + (size_t)turned(min(chunk, c1 - 1)) * MID_ROW_BYTES;
         const uint32_t to = w_lds0 + ((chunk - c0) % W_STAGES) * W_BYTES + wave * W_LOADS * 1024;
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) mid_load_16_bytes_a_lane_into_lds_once(base, w_from[i], to + i * 1024);
+        for (int i = 0; i < W_LOADS; ++i) mid_load_16_bytes_a_lane_into_lds<ONCE>(base, w_from[i], to + i * 1024);
     };
 
     // fragments: lane l holds row l % 32 of a tile and the eight k-values 16 s + 8 (l / 32) .. of step s
@@ -361,28 +363,30 @@ PALM_API int palm_linear_mid_blocks(int M, int N, int K, int epilogue, int plane
     return plan.n_tiles * plan.parts * plan.m_tiles;
 }
 
-template <int R, int TN, typename TC, int EPI>
+template <int R, int TN, bool ONCE, typename TC, int EPI>
 static void launch_mid(hipStream_t stream, const void* a, const void* w, void* c, int M, int N, int K, MidPlan plan) {
     const int work = plan.n_tiles * plan.parts;
     const int groups = (work + 7) / 8;                          // whole groups of eight tiles of weights, a die each
-    linear_mid_kernel<R, TN, TC, EPI><<<groups * 8 * plan.m_tiles, MID_THREADS, 0, stream>>>(
+    linear_mid_kernel<R, TN, ONCE, TC, EPI><<<groups * 8 * plan.m_tiles, MID_THREADS, 0, stream>>>(
         (const bf16_t*)a, (const bf16_t*)w, (TC*)c, M, N, K, plan.n_tiles, plan.m_tiles, plan.chunks_per_part,
         plan.parts == 1 ? 1 : 0);
 }
 
-template <int R, int TN>
+template <int R, int TN, bool ONCE>
 static void launch_mid_as(hipStream_t stream, const void* a, const void* w, void* c, int c_dtype, int M, int N, int K,
                           int epilogue, MidPlan plan) {
-    if (epilogue == MID_SWIGLU) launch_mid<R, TN, bf16_t, MID_SWIGLU>(stream, a, w, c, M, N, K, plan);
-    else if (c_dtype == PALM_BF16) launch_mid<R, TN, bf16_t, MID_STORE>(stream, a, w, c, M, N, K, plan);
-    else launch_mid<R, TN, float, MID_STORE>(stream, a, w, c, M, N, K, plan);
+    if (epilogue == MID_SWIGLU) launch_mid<R, TN, ONCE, bf16_t, MID_SWIGLU>(stream, a, w, c, M, N, K, plan);
+    else if (c_dtype == PALM_BF16) launch_mid<R, TN, ONCE, bf16_t, MID_STORE>(stream, a, w, c, M, N, K, plan);
+    else launch_mid<R, TN, ONCE, float, MID_STORE>(stream, a, w, c, M, N, K, plan);
 }
 
 // a [M, K] bfloat16, w [N, K] bfloat16, K a multiple of 64; c [M, N] (store) or [M, N/2] (gated) in bfloat16, or, with
 // parts > 1 (as palm_linear_mid_parts says; store only), float32 planes [parts, M, N]; parts == 1 with c_dtype float32
-// is one float32 plane, the result itself.
+// is one float32 plane, the result itself.  MID_ONCE may be added to the epilogue.
 PALM_API int palm_linear_mid(hipStream_t stream, const void* a, const void* w, void* c, int c_dtype, int M, int N, int K,
                              int epilogue, int parts) {
+    const bool once = epilogue & MID_ONCE;
+    epilogue &= ~MID_ONCE;
     PALM_CHECK(M >= 0 && N > 0 && K > 0, "linear_mid: M=%d N=%d K=%d", M, N, K);
     PALM_CHECK(K % MID_CHUNK == 0, "linear_mid: K = %d is not a multiple of %d", K, MID_CHUNK);
     PALM_CHECK(epilogue == MID_STORE || epilogue == MID_SWIGLU, "linear_mid: epilogue %d", epilogue);
@@ -396,7 +400,7 @@ PALM_API int palm_linear_mid(hipStream_t stream, const void* a, const void* w, v
                "linear_mid: %d planes asked for, %d planned (planes are float32, not gated)", parts, plan.parts);
     PALM_CHECK(epilogue == MID_STORE || c_dtype == PALM_BF16, "linear_mid: a gated product comes in bfloat16");
     if (M == 0) return 0;
-#define PALM_MID(R, TN) launch_mid_as<R, TN>(stream, a, w, c, c_dtype, M, N, K, epilogue, plan)
+#define PALM_MID(R, TN) (once ? launch_mid_as<R, TN, true> : launch_mid_as<R, TN, false>)(stream, a, w, c, c_dtype, M, N, K, epilogue, plan)
     if (plan.rows == 64) { if (plan.tn == 128) PALM_MID(64, 128); else PALM_MID(64, 64); }
     else if (plan.rows == 128) { if (plan.tn == 128) PALM_MID(128, 128); else if (plan.tn == 96) PALM_MID(128, 96); else PALM_MID(128, 64); }
     else { if (plan.tn == 96) PALM_MID(256, 96); else PALM_MID(256, 64); }

@@ -33,17 +33,17 @@ constexpr int RING_UNITS = 256;                 // compute units: a launch is on
 // 16 (4) bytes a lane from memory into LDS, the 64 lanes' pieces side by side from lds_base on.  base is the same in
 // every lane (scalar registers), offset the lane's own.  LDS reads of the wave that are still out are waited for
 // first: the slot that is asked for may be the one they read.
-__device__ __forceinline__ void ring_load_16(const void* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
-}
-// The same for weights, which pass once: marked as a stream (nt), they don't push what is read again (the rows, the planes and the norms'
-// 32-bit values) out of the caches, nor wait for room among lines that are kept.  Us without and with it, weights of 4 GB in turn:
-// 24,576 x 4,096 gated 1 / 8 / 33 / 48 rows 34.6 35.1 37.7 39.4 and 32.4 32.7 35.6 37.1 (5.8 to 6.2 TB/s at one row), 34,816 x 5,120 gated
-// 60.9 62.2 (1, 8 rows) and 55.1 55.3, 5,120 x 17,408 32.3 33.4 and 29.4 29.6, 4,096 x 12,288 to planes 19.1 19.4 21.6 and 18.2 18.2 19.7,
-// 6,144 x 4,096 11.4 11.3 13.1 and 10.8 10.8 12.4, 151,936 x 4,096 198 206 229 236 and 184 190 207 212.  Matrices up to 20 MB: the same
-// within 1%, one of 50 to 200 MB that nothing else passes by before it is read again up to 10% slower (11.0 and 11.4, 18.5 and 20.0).
-__device__ __forceinline__ void ring_load_16_once(const void* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+// ONCE: marked as a stream (nt).  The memory-side cache holds 256 MB.  Weights that pass once, because more than that passes before they are
+// read again, don't push out what is read again (the rows, the planes and the norms' 32-bit values), nor wait for room among lines that
+// are kept; weights that stay there would be brought from memory each time.  So the caller says which (`once`).  Us, plain and
+// marked, matrices read in turn, of 3 GB and of 96 to 240 MB together, 1 / 8 / 33 rows: 24,576 x 4,096 gated 34.7 35.4 38.7, 32.7 33.0 36.6 and 31.6 31.9
+// 34.0, 31.4 31.8 35.7; 4,096 x 12,288 to planes 18.9 19.3 20.6, 18.2 18.2 19.0 and 16.4 16.7 18.7, 17.5 17.7 19.3; 6,144 x 4,096 11.4 11.0 12.8, 10.8 10.5 12.1 and
+// 10.3 10.1 11.8, 10.8 10.9 12.5; 4,096 x 4,096 8.6 8.7 8.4, 8.3 8.4 8.4 and 8.0 8.1 8.5, 8.6 8.6 9.4.  From 288 MB on marking is the faster way or the same.
+template <bool ONCE = false> __device__ __forceinline__ void ring_load_16(const void* base, uint32_t offset, uint32_t lds_base) {
+    if constexpr (ONCE)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
 }
 __device__ __forceinline__ void ring_load_4(const void* base, uint32_t offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(offset), "s"(base), "s"(lds_base) : "m0", "memory");
@@ -72,8 +72,9 @@ __device__ __forceinline__ uint32_t ring_lds_address(const void* p) {
 
 // U: slots of a wave's ring.  TREG: super-steps of activations a wave holds in registers (0: they cross LDS beside
 // the weights).  CT: column tiles, 16 rows of activations each, that share every fragment of weights.  T: steps a wave makes
-// for one strip.  XRING: the activations come through the ring, ahead of the weights.  EXACT: no step is beyond K.
-template <int U, int TREG, int CT, bool XRING, bool EXACT, typename TC, int EPI>
+// for one strip.  XRING: the activations come through the ring, ahead of the weights.  EXACT: no step is beyond K.  ONCE: see ring_load_16 (decided
+// by a branch in front of each slot's loads instead, kept weights took up to 3 % longer).
+template <int U, int TREG, int CT, bool XRING, bool EXACT, bool ONCE, typename TC, int EPI>
 __global__ __launch_bounds__(RING_THREADS) void linear_ring_kernel(const bf16_t* __restrict__ A,
                                                                     const bf16_t* __restrict__ W,
                                                                     TC* __restrict__ C, int M, int N, int K,
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(RING_THREADS) void linear_ring_kernel(const bf16_t*
             // K is a multiple of 8: a piece is whole or absent; an absent one reads the row's start and counts as zeros
             const bool ok = EXACT || k0 + (i / 2) * 64 + piece * 8 < K;
             const uint32_t in_row = ok ? (uint32_t)(k0 * 2 + (i / 2) * 128 + piece * 16) : 0u;
-            ring_load_16_once(ask_base[i % 2], w_off[i % 2] + in_row, to + i * 1024);
+            ring_load_16<ONCE>(ask_base[i % 2], w_off[i % 2] + in_row, to + i * 1024);
             if (!AREG) ring_load_16(A, x_off[i % 2] + in_row, to + 4096 + i * 1024);
         }
         ++n_asked;
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(RING_THREADS) void linear_ring_kernel(const bf16_t*
     }
 }
 
-template <int U, int TREG, int CT, typename TC, int EPI>
+template <int U, int TREG, int CT, bool ONCE, typename TC, int EPI>
 static void launch_ring(hipStream_t stream, const void* a, const void* w, void* c, int M, int N, int K, int parts, int steps,
                         const RowNorm& norm) {
     const int strips = EPI == EPI_SWIGLU ? (N / 2 + 7) / 8 : (N + 15) / 16;
@@ -378,7 +379,7 @@ static void launch_ring(hipStream_t stream, const void* a, const void* w, void* 
     const int rounds = (strips + slots - 1) / slots;
     const dim3 grid((strips + rounds - 1) / rounds, parts);
     const bool exact = K % SUPER_K == 0 && parts * T * RING_WAVES == n_super;
-#define RING_LAUNCH(XRING, EXACT) linear_ring_kernel<U, TREG, CT, XRING, EXACT, TC, EPI><<<grid, RING_THREADS, 0, stream>>>( \
+#define RING_LAUNCH(XRING, EXACT) linear_ring_kernel<U, TREG, CT, XRING, EXACT, ONCE, TC, EPI><<<grid, RING_THREADS, 0, stream>>>( \
         (const bf16_t*)a, (const bf16_t*)w, (TC*)c, M, N, K, strips, T, norm)
     if constexpr (CT > 1) RING_LAUNCH(true, true);
     else if constexpr (TREG > 0) {

@@ -28,29 +28,31 @@ PALM_API int palm_linear_ring_parts(int M, int N, int K, int epilogue, int plane
     return best;
 }
 
-template <int CT, typename TC, int EPI>
+template <int CT, bool ONCE, typename TC, int EPI>
 static void dispatch_ring_many(hipStream_t stream, const void* a, const void* w, void* c, int M, int N, int K, int parts, int steps,
                                const RowNorm& norm) {
-    if (steps == 1) launch_ring<3, 1, CT, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
-    else if (steps == 2) launch_ring<3, 2, CT, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
-    else if (steps == 3) launch_ring<3, 3, CT, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
-    else if (steps == 4) launch_ring<3, 4, CT, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+    if (steps == 1) launch_ring<3, 1, CT, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+    else if (steps == 2) launch_ring<3, 2, CT, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+    else if (steps == 3) launch_ring<3, 3, CT, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+    else if (steps == 4) launch_ring<3, 4, CT, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
     else if constexpr (CT == 2) {
-        if (steps == 5) launch_ring<3, 5, CT, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
-        else launch_ring<3, 6, CT, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+        if (steps == 5) launch_ring<3, 5, CT, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+        else launch_ring<3, 6, CT, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
     }
 }
-template <typename TC, int EPI>
+template <bool ONCE, typename TC, int EPI>
 static void dispatch_ring_tiles(hipStream_t stream, const void* a, const void* w, void* c, int M, int N, int K, int parts, const RowNorm& norm) {
     const int steps = K / (SUPER_K * RING_WAVES) / parts;
-    if (M <= 32) dispatch_ring_many<2, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
-    else dispatch_ring_many<3, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+    if (M <= 32) dispatch_ring_many<2, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
+    else dispatch_ring_many<3, ONCE, TC, EPI>(stream, a, w, c, M, N, K, parts, steps, norm);
 }
 
 // As palm_linear_thin, for 17 to 48 rows: parts as palm_linear_ring_parts says (1 with the gated epilogue or a norm that is folded into what follows).
 PALM_API int palm_linear_ring(hipStream_t stream, const void* a, const void* w, void* c, int c_dtype, int M, int N, int K, int epilogue,
                               int parts, const float* ss_in, int pieces_in, float eps_in, float* resid, const float* w_out, float* ss_out) {
     RowNorm norm{ss_in, pieces_in, eps_in, K, resid, w_out, ss_out};
+    const bool once = epilogue & EPI_ONCE;
+    epilogue &= ~EPI_ONCE;
     PALM_CHECK(epilogue == EPI_STORE || epilogue == EPI_SWIGLU, "linear_ring: epilogue %d", epilogue);
     PALM_CHECK(parts >= 1 && parts == palm_linear_ring_parts(M, N, K, epilogue, parts > 1), "linear_ring: %d rows, %d x %d in %d ranges are not served", M, N, K, parts);
     PALM_CHECK(!ss_in || pieces_in > 0, "linear_ring: %d pieces of the rows' sums of squares", pieces_in);
@@ -60,9 +62,9 @@ PALM_API int palm_linear_ring(hipStream_t stream, const void* a, const void* w, 
     PALM_CHECK(parts == 1 || c_dtype == PALM_F32, "linear_ring: planes of partial sums are float32");
     PALM_CHECK(((uintptr_t)a | (uintptr_t)w) % 16 == 0, "linear_ring: operands must be 16-byte aligned");
     if (epilogue == EPI_SWIGLU) {
-        PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_ring_tiles<TC, EPI_SWIGLU>(stream, a, w, c, M, N, K, parts, norm));
+        PALM_DTYPE_SWITCH(c_dtype, TC, (once ? dispatch_ring_tiles<true, TC, EPI_SWIGLU> : dispatch_ring_tiles<false, TC, EPI_SWIGLU>)(stream, a, w, c, M, N, K, parts, norm));
     } else {
-        PALM_DTYPE_SWITCH(c_dtype, TC, dispatch_ring_tiles<TC, EPI_STORE>(stream, a, w, c, M, N, K, parts, norm));
+        PALM_DTYPE_SWITCH(c_dtype, TC, (once ? dispatch_ring_tiles<true, TC, EPI_STORE> : dispatch_ring_tiles<false, TC, EPI_STORE>)(stream, a, w, c, M, N, K, parts, norm));
     }
     PALM_LAUNCHED();
     return 0;

@@ -4,6 +4,9 @@
 #include "mfma.h"
 
 enum ThinEpilogue : int { EPI_STORE = 0, EPI_SWIGLU = 1 };
+// Added to an entry point's epilogue: the weights pass once, more than the memory-side cache holds passes before they are read again
+// (see ring_load_16).
+constexpr int EPI_ONCE = 16;
 
 constexpr int SUPER_K = 128;         // k-values of a "super-step": four matrix instructions of 32
 
@@ -33,3 +36,5 @@ struct RowNorm {
 // the entry point checks.
 void launch_linear_ring(hipStream_t stream, const void* a, const void* w, void* c, int c_dtype, int M, int N, int K,
                         int epilogue, int parts, int steps, const RowNorm& norm);
+void launch_linear_ring_once(hipStream_t stream, const void* a, const void* w, void* c, int c_dtype, int M, int N, int K,
+                             int epilogue, int parts, int steps, const RowNorm& norm);

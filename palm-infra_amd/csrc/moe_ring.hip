@@ -15,7 +15,7 @@
 //
 // The shared expert's steps come first, because they are known before it is known who chose what.
 // 6 rows, 32 experts of 2,048 x 4,096 (17 in use) with a shared one of 4,096, both products: 127 -> 105 us, 5.7 TB/s; one row 78 -> 42;
-// 16 rows (27 in use) 189 -> 166.  The matrices pass once and their loads are marked so (nt): a decode step of six sequences through eight
+// 16 rows (27 in use) 189 -> 166.  Where the matrices pass once (ONCE) their loads are marked so (nt, linear_ring.h): a decode step of six sequences through eight
 // layers of 17 of 32 such experts 1,528 -> 1,447 us.
 #include "mfma.h"
 #include "expert_form.h"
@@ -112,7 +112,7 @@ __device__ __forceinline__ uint32_t mr_fragment(int j, int r, int g) {
     return ((r / 8) + 2 * (j / 2)) * 1024 + (r % 8) * 128 + ((((j % 2) * 4 + g) ^ (r % 8)) * 16);
 }
 
-template <int TREG, bool GATED>
+template <int TREG, bool GATED, bool ONCE>
 __global__ __launch_bounds__(MR_THREADS) void moe_ring_up_kernel(const bf16_t* __restrict__ h, const bf16_t* __restrict__ up, RingChoices ch,
                                                                  int width, int ff, const bf16_t* __restrict__ shared_up, int shared_ff,
                                                                  int form, ExpertCap cap, bf16_t* __restrict__ mid) {
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(MR_THREADS) void moe_ring_up_kernel(const bf16_t* _
         const uint32_t k0 = (uint32_t)(ask_t * MR_WAVES + wave) * (MR_K * 2);
         lds_reads_done();
 #pragma unroll
-        for (int i = 0; i < 4; ++i) row_chunk_into_lds_once(base[i % 2], in_line + k0 + (i / 2) * 128, to + i * 1024);
+        for (int i = 0; i < 4; ++i) row_chunk_into_lds<ONCE>(base[i % 2], in_line + k0 + (i / 2) * 128, to + i * 1024);
         ++n_asked;
         ++ask_t;
     };
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(MR_THREADS) void moe_ring_up_kernel(const bf16_t* _
 }
 
 // HALVES: eight (1) or sixteen (2) rows of inner values beside a step's weights.
-template <int HALVES>
+template <int HALVES, bool ONCE>
 __global__ __launch_bounds__(MR_THREADS) void moe_ring_down_kernel(const bf16_t* __restrict__ mid, const bf16_t* __restrict__ down, RingChoices ch,
                                                                    int width, int ff, const bf16_t* __restrict__ shared_down, int shared_ff,
                                                                    const bf16_t* __restrict__ add0, const bf16_t* __restrict__ add1,
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(MR_THREADS) void moe_ring_down_kernel(const bf16_t*
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            row_chunk_into_lds_once(base + (size_t)(i % 2) * 8 * row_bytes + (i / 2) * 128, row8 * row_bytes + piece * 16u, to + i * 1024);
+            row_chunk_into_lds<ONCE>(base + (size_t)(i % 2) * 8 * row_bytes + (i / 2) * 128, row8 * row_bytes + piece * 16u, to + i * 1024);
 #pragma unroll
         for (int i = 0; i < 2 * HALVES; ++i)
             row_chunk_into_lds(reinterpret_cast<const char*>(mid) + (i / HALVES) * 128, x_off[i % HALVES] + piece * 16u, to + 4096 + i * 1024);
@@ -328,11 +328,11 @@ PALM_API int palm_moe_ring_planes(int width) { return max(1, min(4, MR_UNITS / m
 
 // h bfloat16 [n, width]; up, down, shared_up, shared_down, forms as in moe.hip, all bfloat16; chosen, weight [n, top], or with ids [n]
 // the table [vocab, top] and no weight; add0, add1: null or bfloat16 rows [n, width]; mid: room for n * (top * ff + shared_ff) bfloat16;
-// out float32 [planes, n, width].
+// out float32 [planes, n, width].  once: the matrices pass once, more than the memory-side cache holds passes before they are read again (linear_ring.h).
 PALM_API int palm_moe_ring(hipStream_t stream, const void* h, const void* up, const void* down, const int* chosen, const float* weight,
                            const int* ids, int vocab, int n_tokens, int top, int experts, int width, int ff, const void* shared_up,
                            const void* shared_down, int shared_ff, int form, float limit, float slope, float shift, const void* add0,
-                           const void* add1, void* mid, int planes, float* out) {
+                           const void* add1, void* mid, int planes, float* out, int once) {
     PALM_CHECK(form >= EXPERT_GATED_SILU && form <= EXPERT_RELU_SQUARED, "moe_ring: form %d is neither gated silu (0) nor plain gelu (1) nor capped "
                "gated (2) nor squared relu (3)", form);
     PALM_CHECK(form != EXPERT_CAPPED || limit > 0.f, "moe_ring: the cap %g must be positive", (double)limit);
@@ -351,7 +351,7 @@ PALM_API int palm_moe_ring(hipStream_t stream, const void* h, const void* up, co
     const bool gated = expert_is_gated(form);
     const long long strips = ((long long)shared_ff + (long long)min(experts, n_tokens * top) * ff) / (gated ? 8 : 16);
     const int blocks = (int)min((long long)MR_UNITS, strips), steps = (width + MR_WAVES * MR_K - 1) / (MR_WAVES * MR_K);
-#define MR_UP(TREG, GATED) moe_ring_up_kernel<TREG, GATED><<<blocks, MR_THREADS, 0, stream>>>((const bf16_t*)h, (const bf16_t*)up, ch, width, ff, \
+#define MR_UP(TREG, GATED) (once ? moe_ring_up_kernel<TREG, GATED, true> : moe_ring_up_kernel<TREG, GATED, false>)<<<blocks, MR_THREADS, 0, stream>>>((const bf16_t*)h, (const bf16_t*)up, ch, width, ff, \
         (const bf16_t*)shared_up, shared_ff, form, cap, (bf16_t*)mid)
 #define MR_UP_STEPS(TREG) if (gated) MR_UP(TREG, true); else MR_UP(TREG, false)
     if (steps <= 1) { MR_UP_STEPS(1); }
@@ -361,7 +361,7 @@ PALM_API int palm_moe_ring(hipStream_t stream, const void* h, const void* up, co
 #undef MR_UP_STEPS
 #undef MR_UP
     PALM_LAUNCHED();
-#define MR_DOWN(HALVES) moe_ring_down_kernel<HALVES><<<dim3(width / 16, planes), MR_THREADS, 0, stream>>>((const bf16_t*)mid, (const bf16_t*)down, ch, \
+#define MR_DOWN(HALVES) (once ? moe_ring_down_kernel<HALVES, true> : moe_ring_down_kernel<HALVES, false>)<<<dim3(width / 16, planes), MR_THREADS, 0, stream>>>((const bf16_t*)mid, (const bf16_t*)down, ch, \
         width, ff, (const bf16_t*)shared_down, shared_ff, (const bf16_t*)add0, (const bf16_t*)add1, out)
     if (n_tokens <= 8) MR_DOWN(1); else MR_DOWN(2);
 #undef MR_DOWN

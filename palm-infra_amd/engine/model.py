@@ -21,6 +21,7 @@ class DecoderModel:
         self.layers = [builder.build(layer) for layer in spec.layers]
         self.final_norm = builder.build(spec.final_norm)
         self.head = builder.build(spec.head)
+        builder.finish()
         self.order = spec.order
         self.weights = weights
         self._choosing = list(builder.choosing.values())

@@ -71,7 +71,7 @@ def flags_of(source: str) -> list[str]:
 
 
 CORE_SOURCES = ["elementwise.hip", "linear.hip", "rope_store.hip", "attention_simple.hip", "sampling.hip",
-                "linear_mfma.hip", "linear_ring.hip", "linear_ring_many.hip", "linear_wide.hip", "linear_wide_store_32.hip", "linear_wide_store_64.hip",
+                "linear_mfma.hip", "linear_ring.hip", "linear_ring_once.hip", "linear_ring_many.hip", "linear_wide.hip", "linear_wide_store_32.hip", "linear_wide_store_64.hip",
                 "linear_wide_gated_32.hip", "linear_wide_gated_64.hip", "linear_wide_store_128.hip", "linear_wide_gated_128.hip", "linear_mid.hip",
                 "weights_prep.hip", "linear_tile.hip", "linear_big.hip"]
 ATTENTION_SOURCES = ["attention_mfma.hip"]
@@ -92,7 +92,7 @@ HEADERS = ["common.h", "mfma.h", "linear_thin.h", "linear_wide.h", "attention_ap
 # headers of a few sources only: a change of one rebuilds the libraries of the sources that include it
 OWN_HEADERS = {"retention.hip": ["linear_recurrence.h"], "gla.hip": ["linear_recurrence.h"], "delta_rule.hip": ["delta_rule.h"],
                "delta_head.hip": ["delta_rule.h", "conv_state.h"], "mamba.hip": ["conv_state.h"], "moe.hip": ["expert_form.h"], "moe_few.hip": ["expert_form.h"], "moe_ring.hip": ["expert_form.h", "lds_stage.h"],
-               "moe_grouped.hip": ["big_walk.h", "expert_form.h", "lds_stage.h"], "linear.hip": ["lds_stage.h"], "linear_ring.hip": ["linear_ring.h"], "linear_ring_many.hip": ["linear_ring.h"], "linear_tile.hip": ["lds_stage.h"], "linear_big.hip": ["big_walk.h", "lds_stage.h"], "attention_sink_mfma.hip": ["lds_stage.h"], "attention_mfma.hip": ["attention_decode_pages.h", "lds_stage.h"], "attention_diff_mfma.hip": ["lds_stage.h"],
+               "moe_grouped.hip": ["big_walk.h", "expert_form.h", "lds_stage.h"], "linear.hip": ["lds_stage.h"], "linear_ring.hip": ["linear_ring.h", "linear_ring_thin.h"], "linear_ring_once.hip": ["linear_ring.h", "linear_ring_thin.h"], "linear_ring_many.hip": ["linear_ring.h"], "linear_tile.hip": ["lds_stage.h"], "linear_big.hip": ["big_walk.h", "lds_stage.h"], "attention_sink_mfma.hip": ["lds_stage.h"], "attention_mfma.hip": ["attention_decode_pages.h", "lds_stage.h"], "attention_diff_mfma.hip": ["lds_stage.h"],
                "branch_scaled.hip": ["expert_form.h"]}
 
 

@@ -449,6 +449,19 @@ def linear_library(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.matmul(a, w.t())
 
 
+MEMORY_CACHE = 256 << 20      # bytes that the cache beside the memory holds
+EPI_ONCE = 16                 # added to a product's epilogue, see linear_thin.h
+
+
+def passes_once(once: bool | None, *weights: torch.Tensor) -> bool:
+    """Whether a launch's weights are read as a stream that no cache is to keep.  ``once`` is what the caller knows: whether more than MEMORY_CACHE
+    passes before they are read again (a model's weights are, step after step, read in turn).  If it does not know (None) the launch's own
+    matrices have to be more than that.  Us, kept and as a stream, matrices in turn of 144 to 240 MB, of 288 to 384 and of 3 GB together: 24,576 x 4,096 gated, 1
+    and 64 rows 31.6 30.5 and 31.4 38.5 (192 MB), 35.1 40.9 and 32.2 38.3 (384), 34.7 39.2 and 32.7 38.0; 4,096 x 12,288, 8 and 91 rows 16.7 24.7 and 17.7 29.1 (192), 18.5 27.9
+    and 17.8 28.6 (288), 19.3 27.9 and 18.2 27.3; 2,048 x 2,048, 64 rows 5.8 and 6.2 (160), 6.0 6.0 (320)."""
+    return once if once is not None else sum(w.numel() * w.element_size() for w in weights) > MEMORY_CACHE
+
+
 THIN_TOKENS = 16      # up to here every wave fetches its own activations; above, a block shares them through LDS
 WIDE_TOKENS = 128     # as many rows as that block holds
 WIDE_FLOAT32_TOKENS = 64   # a float32 result (logits) of more rows than this goes through the tiled kernel instead
@@ -531,11 +544,11 @@ def mid_pays(M: int, N: int, K: int, planes_ok: bool = False, gated: bool = Fals
 
 
 def linear_mid(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: bool = False,
-               planes_ok: bool = False) -> torch.Tensor:
+               planes_ok: bool = False, once: bool | None = None) -> torch.Tensor:
     """bfloat16 a [M, K] . w [N, K]^T for some hundred rows, K a multiple of 64: both operands go through rings in
     LDS, a block of four waves holding 256 rows against 96 or 64 weight rows.  The result is [M, N] in bfloat16 or
     float32 ([M, N/2] bfloat16 when ``gated``), or, if ``planes_ok`` and the weight rows are few, float32 planes
-    [P, M, N] over ranges of K."""
+    [P, M, N] over ranges of K.  ``once``: see ``passes_once``."""
     _dev("linear_mid", a, w)
     if not (a.dtype == BF16 and w.dtype == BF16 and a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1]
             and a.is_contiguous() and w.is_contiguous()):
@@ -551,7 +564,7 @@ def linear_mid(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: 
     else:
         out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=a.device)
     library.call(core(), "palm_linear_mid", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_mid out"), M, N, K,
-                 1 if gated else 0, planes)
+                 int(gated) + EPI_ONCE * passes_once(once, w), planes)
     return out
 
 
@@ -641,7 +654,7 @@ def ring_pays(M: int, N: int, K: int, gated: bool = False, planes_ok: bool = Fal
 
 
 def linear_ring(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: bool = False, planes_ok: bool = False, row_ss=None,
-                row_eps: float = 0.0) -> torch.Tensor:
+                row_eps: float = 0.0, once: bool | None = None) -> torch.Tensor:
     """``linear_thin`` (its arguments) for 17 to 48 rows where ``ring_serves`` says so: the weight streamed once for all rows."""
     _dev("linear_ring", a, w)
     if not (a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1] and thin_serves(a, w) and a.is_contiguous() and w.is_contiguous()):
@@ -656,7 +669,8 @@ def linear_ring(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated:
         out = torch.empty((planes, M, N), dtype=F32, device=a.device)
     else:
         out = torch.empty((M, N // 2 if gated else N), dtype=out_dtype, device=a.device)
-    library.call(core(), "palm_linear_ring", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_ring out"), M, N, K, int(gated), planes,
+    library.call(core(), "palm_linear_ring", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_ring out"), M, N, K,
+                 int(gated) + EPI_ONCE * passes_once(once, w), planes,
                  _p(row_ss), pieces, float(row_eps), None, None, None)
     return out
 
@@ -687,10 +701,10 @@ def scale_rows(a: torch.Tensor, row_ss: torch.Tensor, eps: float) -> torch.Tenso
 
 
 def linear_thin_into_residual(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor, row_ss=None,
-                              row_eps: float = 0.0):
+                              row_eps: float = 0.0, once: bool | None = None):
     """A branch's last product and what follows it, for up to 16 rows, or as many as ``ring_serves`` takes whole: x += a . w^T (x float32 [M, N], in
     place); returns (x * norm_w rounded to bfloat16, the pieces [M, N/16] of each row's sum of squares of x):
-    the next norm's output but for the row factor.  row_ss / row_eps: a itself lacks a row factor."""
+    the next norm's output but for the row factor.  row_ss / row_eps: a itself lacks a row factor.  ``once``: see ``passes_once``."""
     _dev("linear_thin_into_residual", a, w, x, norm_w)
     M, K = a.shape
     N = w.shape[0]
@@ -704,13 +718,13 @@ def linear_thin_into_residual(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor,
     pieces = _row_ss("linear_thin_into_residual", a, row_ss, RING_TOKENS if many else THIN_TOKENS)
     values = torch.empty((M, N), dtype=BF16, device=a.device)
     ss = torch.empty((M, (N + 15) // 16), dtype=F32, device=a.device)
-    library.call(core(), "palm_linear_ring" if many else "palm_linear_thin", _stream(), _p(a), _p(w), _p(values), _code(values, "values"), M, N, K, 0, 1,
-                 _p(row_ss), pieces, float(row_eps), _p(x), _p(norm_w), _p(ss))
+    library.call(core(), "palm_linear_ring" if many else "palm_linear_thin", _stream(), _p(a), _p(w), _p(values), _code(values, "values"), M, N, K,
+                 EPI_ONCE * passes_once(once, w), 1, _p(row_ss), pieces, float(row_eps), _p(x), _p(norm_w), _p(ss))
     return values, ss
 
 
 def linear_thin(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated: bool = False,
-                planes_ok: bool = False, row_ss=None, row_eps: float = 0.0) -> torch.Tensor:
+                planes_ok: bool = False, row_ss=None, row_eps: float = 0.0, once: bool | None = None) -> torch.Tensor:
     """bfloat16 a [M, K] . w [N, K]^T on the matrix cores, the weight streamed once per 16 rows of a (64 above 16);
     result [M, N] in bfloat16 or float32.  With ``gated`` w is [gate rows | up rows] and the result is
     silu(a gate^T) * (a up^T), [M, N/2].
@@ -720,7 +734,9 @@ def linear_thin(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated:
     rmsnorm's ``delta`` and qk_norm_rope_store's ``qkv`` take such planes.
 
     ``row_ss`` [M, pieces] float32 with ``row_eps``: the rows of a lack the factor 1 / sqrt(mean square + eps) of
-    their norm, whose sums of squares come in pieces; the result rows are multiplied by it (at most 16 rows)."""
+    their norm, whose sums of squares come in pieces; the result rows are multiplied by it (at most 16 rows).
+
+    ``once``: see ``passes_once``."""
     pieces = _row_ss("linear_thin", a, row_ss)
     if not thin_serves(a, w):
         out = linear_exact(a, w, out_dtype)
@@ -738,7 +754,7 @@ def linear_thin(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, gated:
         if planes > 1:
             out = torch.empty((planes, M, N), dtype=F32, device=a.device)
         library.call(core(), "palm_linear_thin", _stream(), _p(a), _p(w), _p(out), _code(out, "linear_thin out"), M, N, K,
-                     1 if gated else 0, planes, _p(row_ss), pieces, float(row_eps), None, None, None)
+                     int(gated) + EPI_ONCE * passes_once(once, w), planes, _p(row_ss), pieces, float(row_eps), None, None, None)
         return out
     if not (row_ss is None):
         raise KernelError(f"linear_thin: rows that lack their norm's factor come at most {THIN_TOKENS} at a time, not {M}")
@@ -1185,7 +1201,7 @@ _FEEDFORWARD_SIGNATURES = {
                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "palm_moe_few_planes": [c_int],
     "palm_moe_ring": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p,
-                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+                      c_void_p, c_int, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int],
     "palm_moe_ring_planes": [c_int],
     "palm_moe_route_table": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p],
     "palm_moe_tile_tokens": [c_int, c_int, c_int, c_int, c_int, c_int],
@@ -2289,22 +2305,25 @@ def moe_ring_serves(h, gate_up, down, top: int, experts: int, width: int, ff: in
 
 
 def moe_few(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, weight: torch.Tensor | None, ff: int,
-            form: str = "gated_silu", cap=NO_CAP, add=(), ids: torch.Tensor | None = None, shared=None, planes_ok: bool = False) -> torch.Tensor:
+            form: str = "gated_silu", cap=NO_CAP, add=(), ids: torch.Tensor | None = None, shared=None, planes_ok: bool = False,
+            once: bool | None = None) -> torch.Tensor:
     """``moe_experts`` on the matrix cores (its arguments): every expert in use is read once for all its rows.  Returns float32
-    [n, width], or with ``planes_ok`` possibly planes [P, n, width] for a reader that adds them."""
+    [n, width], or with ``planes_ok`` possibly planes [P, n, width] for a reader that adds them.  ``once``: see ``passes_once``."""
     what = "moe_few"
     n, width = h.shape
     top = chosen.shape[1]
     experts, shared_up, shared_down, shared_ff = _check_experts(what, h, gate_up, down, chosen, weight, ff, form, ids, shared)
     if not moe_few_serves(h, gate_up, ff, experts, top, shared):
         raise KernelError(f"{what}: at most {FEW_ROWS} bfloat16 rows, bfloat16 weights, sizes in multiples of eight")
-    entry = "palm_moe_ring" if moe_ring_serves(h, gate_up, down, top, experts, width, ff, shared_ff, shared) else "palm_moe_few"
+    ring = moe_ring_serves(h, gate_up, down, top, experts, width, ff, shared_ff, shared)
+    entry = "palm_moe_ring" if ring else "palm_moe_few"
     planes = getattr(feedforward(), entry + "_planes")(width) if planes_ok else 1
     mid = torch.empty((n, top * ff + shared_ff), dtype=BF16, device=h.device)
     out = torch.empty((planes, n, width), dtype=F32, device=h.device)
     library.call(feedforward(), entry, _stream(), _p(h), _p(gate_up), _p(down), _p(chosen), _p(weight), _p(ids),
                  chosen.shape[0] if ids is not None else 0, n, top, experts, width, ff, _p(shared_up), _p(shared_down), shared_ff,
-                 EXPERT_FORMS[form], *(float(c) for c in cap), *_addends(what, add, h), _p(mid), planes, _p(out))
+                 EXPERT_FORMS[form], *(float(c) for c in cap), *_addends(what, add, h), _p(mid), planes, _p(out),
+                 *((int(passes_once(once, gate_up, down, *(shared or ()))),) if ring else ()))
     return out if planes > 1 else out[0]
 
 

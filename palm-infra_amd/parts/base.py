@@ -33,6 +33,7 @@ import numpy as np
 import torch
 
 from ..config.spec import PartSpec
+from ..kernels import ops
 
 CATEGORIES = ("norm", "position", "mixer", "feed_forward", "block", "embedding", "head")
 _REGISTRY: dict[tuple[str, str], type] = {}
@@ -81,15 +82,32 @@ class Builder:
     def __init__(self, weights, dtype: torch.dtype, device):
         self.weights, self.dtype, self.device = weights, dtype, torch.device(device)
         self.choosing: dict = {}     # parts whose kernels a decode step's lengths choose, one of each ``decode_shape`` (see ``decode_form``)
+        self._streamed: list = []    # whatever streams weights in a decode step
+        self._read: dict = {}        # the tensors that parts read in whole, address -> bytes (an embedding's rows are looked up)
 
     def build(self, spec: PartSpec):
         part = part_class(spec.category, spec.kind)(spec, self)
+        self.note(part)
         if hasattr(part, "decode_form"):
             self.choosing.setdefault(part.decode_shape, part)
         return part
 
+    def note(self, part) -> None:
+        """The part, and what it holds, where it streams weights."""
+        for held in (part, *getattr(part, "__dict__", {}).values()):
+            self._streamed += [one for one in (held if isinstance(held, (list, tuple)) else (held,)) if hasattr(one, "passes_once")]
+
     def tensor(self, spec: PartSpec, name: str) -> torch.Tensor:
-        return self.weights.get(spec.tensors[name])
+        t = self.weights.get(spec.tensors[name])
+        if spec.category != "embedding":
+            self._read[t.data_ptr()] = t.numel() * t.element_size()
+        return t
+
+    def finish(self) -> None:
+        """When all parts of a model are built: its products learn whether a step's weights are more than the memory-side cache holds."""
+        once = sum(self._read.values()) > ops.MEMORY_CACHE
+        for one in self._streamed:
+            one.passes_once = once
 
 
 @dataclass

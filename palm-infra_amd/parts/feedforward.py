@@ -122,6 +122,7 @@ class RoutedExperts:
     "gated_silu" (an expert's first matrix holds its gate rows, then its up rows), "gelu" or "relu_squared" (up rows alone), or "capped_gated"
     (gate rows and up rows, capped as ``cap`` = (limit, slope, shift) says)."""
     DIRECT_ROWS = 128            # as many rows as a recorded step holds at most
+    passes_once: bool | None = None      # see Linear
 
     def _set_experts(self, first, down, experts: int, inter: int, hidden: int, form: str, cap=ops.NO_CAP):
         self.cap = cap
@@ -155,7 +156,7 @@ class RoutedExperts:
         reads its expert in.  ``ids``, ``shared``: see ``ops.moe_experts``; ``planes_ok``: float32 planes may come back."""
         args = (h, self.first, self.down_all, chosen, weight, self.inter, self.form, self.cap, add, ids, shared)
         if ops.moe_few_serves(h, self.first, self.inter, self.experts, chosen.shape[1], shared):
-            return ops.moe_few(*args, planes_ok=planes_ok)
+            return ops.moe_few(*args, planes_ok=planes_ok, once=self.passes_once)
         return ops.moe_experts(*args)
 
     def run_experts(self, h, chosen, weight, add=()):

@@ -43,6 +43,7 @@ class Linear:
         if bias is not None and (bias.shape != (self.out_features,) or bias.dtype != torch.float32):
             raise ValueError(f"a linear bias must be float32 [{self.out_features}], got {bias.dtype} {tuple(bias.shape)}")
         self.bias = bias
+        self.passes_once: bool | None = None        # whether a step reads more than the memory-side cache holds (ops.passes_once; the builder knows)
 
     def __call__(self, x, out_dtype: torch.dtype | None = None, planes_ok: bool = False, sink=None):
         """x: rows [n, in], or ``Prenormed`` rows (their row factor is applied to the result).
@@ -71,18 +72,18 @@ class Linear:
         if isinstance(x, Prenormed):
             if self._folds(x.values, planes_ok=planes_ok):
                 product = ops.linear_thin if x.shape[0] <= ops.THIN_TOKENS else ops.linear_ring
-                return product(x.values, w, out_dtype or x.dtype, planes_ok=planes_ok, row_ss=x.ss, row_eps=x.eps)
+                return product(x.values, w, out_dtype or x.dtype, planes_ok=planes_ok, row_ss=x.ss, row_eps=x.eps, once=self.passes_once)
             x = x.materialize()
         out_dtype = out_dtype or x.dtype
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.in_features % 8 == 0:
             rows = x.shape[0]
             if ops.ring_pays(rows, self.out_features, self.in_features, planes_ok=planes_ok) and self._whole_pieces(x):
-                return ops.linear_ring(x, w, out_dtype, planes_ok=planes_ok)
+                return ops.linear_ring(x, w, out_dtype, planes_ok=planes_ok, once=self.passes_once)
             if x.is_contiguous() and ops.mid_pays(rows, self.out_features, self.in_features, planes_ok=planes_ok, out_dtype=out_dtype):
-                return ops.linear_mid(x, w, out_dtype, planes_ok=planes_ok)
+                return ops.linear_mid(x, w, out_dtype, planes_ok=planes_ok, once=self.passes_once)
             if (rows <= THIN_ROWS or out_dtype != torch.bfloat16
                     or (ops.thin_serves(x, w) and ops.wide_pays(rows, self.out_features, self.in_features, planes_ok=planes_ok))):
-                return ops.linear_thin(x, w, out_dtype, planes_ok=planes_ok)
+                return ops.linear_thin(x, w, out_dtype, planes_ok=planes_ok, once=self.passes_once)
             if self._big(x):
                 return ops.linear_big(x, w)
             return ops.linear_library(x, w)
@@ -108,7 +109,7 @@ class Linear:
         if (self.bias is None and sink.foldable and self._folds(rows) and sink.x.shape == (rows.shape[0], self.out_features)
                 and rows.dtype == torch.bfloat16 and sink.fold_pays(rows.shape[0], self.out_features, self.in_features)):
             ss_in, eps_in = (x.ss, x.eps) if isinstance(x, Prenormed) else (None, 0.0)
-            values, ss = ops.linear_thin_into_residual(rows, self.weight, sink.x, sink.norm.weight, row_ss=ss_in, row_eps=eps_in)
+            values, ss = ops.linear_thin_into_residual(rows, self.weight, sink.x, sink.norm.weight, row_ss=ss_in, row_eps=eps_in, once=self.passes_once)
             return Prenormed(values, ss, sink.norm.eps)
         return sink.finish(self(x, planes_ok=sink.takes_planes))
 
@@ -120,16 +121,16 @@ class Linear:
         if isinstance(x, Prenormed):
             if self._folds(x.values, gated=True):
                 product = ops.linear_thin if x.shape[0] <= ops.THIN_TOKENS else ops.linear_ring
-                return product(x.values, self.weight, x.dtype, gated=True, row_ss=x.ss, row_eps=x.eps)
+                return product(x.values, self.weight, x.dtype, gated=True, row_ss=x.ss, row_eps=x.eps, once=self.passes_once)
             x = x.materialize()
         if ops.ring_pays(x.shape[0], self.out_features, self.in_features, gated=True) and self._whole_pieces(x):
-            return ops.linear_ring(x, self.weight, x.dtype, gated=True)
+            return ops.linear_ring(x, self.weight, x.dtype, gated=True, once=self.passes_once)
         if (x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and x.is_contiguous()
                 and ops.mid_pays(x.shape[0], self.out_features, self.in_features, gated=True)):
-            return ops.linear_mid(x, self.weight, x.dtype, gated=True)
+            return ops.linear_mid(x, self.weight, x.dtype, gated=True, once=self.passes_once)
         if ops.thin_serves(x, self.weight) and (
                 x.shape[0] <= THIN_ROWS or ops.wide_pays(x.shape[0], self.out_features, self.in_features, gated=True)):
-            return ops.linear_thin(x, self.weight, x.dtype, gated=True)
+            return ops.linear_thin(x, self.weight, x.dtype, gated=True, once=self.passes_once)
         if self._big(x, gated=True):
             return ops.linear_big(x, self.weight, gated=True)
         return ops.swiglu(self(x))

@@ -160,6 +160,7 @@ def test_few_rows(form, E, top, W, F, shared):
         assert float((got.cpu().double() - want).abs().max()) <= tol, (n, uneven)
         again = ops.moe_few(*args, F, form, cap, shared=extra)
         assert torch.equal(got, again)
+        assert torch.equal(ops.moe_few(*args, F, form, cap, shared=extra, once=True), got)          # (matrices marked as read once)
         planes = ops.moe_few(*args, F, form, cap, shared=extra, planes_ok=True)
         planes = planes if planes.dim() == 2 else planes.sum(0)
         assert torch.allclose(planes, got, atol=1e-4 * float(want.abs().max()), rtol=1e-4)
