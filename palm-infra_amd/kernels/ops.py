@@ -939,20 +939,23 @@ def decode_pages_pays(lengths, nh: int, nkv: int, hd: int, max_keys: int) -> boo
     4,000 before 32 of 20 103.7 113.0; one of 4,000 13.0 18.3, of 9,000 19.5 19.4, of 32,000 36.8 31.6.  Over 3,504 batches (1 to 96 sequences of 10 to 130,000 keys, 8 shapes of
     heads) the way taken is 24.2 % sooner than slices alone in the geometric mean, the better of the two would be 24.6; at 47 it takes pages that are 3 % slower or more, 21 % at worst."""
     n, group = len(lengths), nh // nkv
-    pages = np.maximum(1, (np.asarray(lengths, dtype=np.int64) + (PAGE_TOKENS - 2)) // PAGE_TOKENS)      # (the new key is no part of the walk)
-    total, longest = int(pages.sum()), int(pages.max())
+    pages = [(keys + (PAGE_TOKENS - 2)) // PAGE_TOKENS or 1 for keys in lengths]            # (the new key is no part of the walk)
+    total, longest = sum(pages), max(pages)
     walk = -(-longest // decode_slices(n, nh, nkv, max_keys))
     runs = min(max(1, COMPUTE_UNITS // nkv), total)              # blocks of a kv head
     rounds = -(-longest * runs // (8 * total))
-    eights = 1
-    if n > 8 and total > 8 * runs:                               # (a block with more than eight sequences has more than eight pages)
-        ends, cuts = np.cumsum(pages), np.arange(runs + 1) * (total // runs) + np.minimum(np.arange(runs + 1), total % runs)
-        eights = -(-int((np.searchsorted(ends, cuts[1:], "left") - np.searchsorted(ends, cuts[:-1], "right")).max() + 1) // 8)
     mb = sum(lengths) * nkv * hd * 4e-6
     late = 2.3 * (0.3 + 0.7 * hd / 128) * walk + 0.145 * -(-longest // walk)
-    if not (late >= 0.6 + 0.2 * group + (2.0 + 0.1 * group) * rounds + 5.0 * (eights - 1) + mb / 7.8
-            or (eights == 1 and mb >= (35 if group <= 4 else 112) * (0.5 + 0.5 * hd / 128) and mb >= 14 * (rounds - 1))):
+    spared = late - (0.6 + 0.2 * group + (2.0 + 0.1 * group) * rounds + mb / 7.8)
+    wide = mb >= (35 if group <= 4 else 112) * (0.5 + 0.5 * hd / 128) and mb >= 14 * (rounds - 1)
+    if spared < 0 and not wide:
         return False
+    if n > 8 and total > 8 * runs:                               # (a block with more than eight sequences has more than eight pages)
+        ends, at = np.cumsum(np.array(pages)), np.arange(runs + 1)
+        cuts = at * (total // runs) + np.minimum(at, total % runs)
+        eights = -(-int((ends.searchsorted(cuts[1:], "left") - ends.searchsorted(cuts[:-1], "right")).max() + 1) // 8)
+        if eights > 1 and spared < 5.0 * (eights - 1):
+            return False
     return decode_pages_serves(n, nh, nkv, hd, longest)
 
 
