@@ -3,7 +3,7 @@
 //
 // The pages of all sequences stand in one row, one sequence behind the other, and for each kv head the row is cut into equal runs, 256 blocks over all kv
 // heads, and a block's run into equal runs of its eight waves.  So a step of sequences of 70 to 1,500 tokens keeps every compute unit reading to the end, where
-// slices of every sequence alike leave the long ones' slices alone at the end, and the eight waves of a unit have up to 256 KB on their way.
+// slices of every sequence alike leave the long ones' slices alone at the end, and the eight waves of a unit have 96 KB on their way.
 // The cut follows from the step's lengths by arithmetic that every wave does for itself (a prefix sum over the sequences' pages).
 //
 // A block first makes the queries of its sequences from the projection's rows (a lane holds eight elements of a head, so a wave makes four
@@ -14,6 +14,9 @@
 // (an agent-scope store each), then counted; the wave that counts the last one adds them up in the order of the blocks.  No
 // fence writes back or empties a die's cache for it, and no wave ever waits for another block.  The counters are zero between launches: the wave that
 // finds the last piece sets its counter back.
+// Where a sequence is cut, and so in which order its pieces are added, follows from the pages of all sequences of the step: a step made again gives the
+// same bits, but a neighbour that is a page longer can change a sequence's last ones.  (Slices follow from the number of sequences and the
+// longest one, rounded up.)
 //
 // What bounds it: the walk reads at 5.5 to 6.3 TB/s; before it lie 3 us (two round trips for the step's lengths and the page numbers, the queries through LDS;
 // 96 KB a unit are on their way meanwhile), behind it 2 to 4 (pieces to memory, the count, the last one's reads).  Us, 32 heads of 8 (by slices of every

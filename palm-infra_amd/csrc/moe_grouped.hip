@@ -35,8 +35,9 @@ static_assert(PLAN_MAX_EXPERTS <= 1 << TILE_EXPERT_BITS, "an expert's number and
 __device__ __forceinline__ int tile_expert_of(int t) { return t & ((1 << TILE_EXPERT_BITS) - 1); }
 __device__ __forceinline__ int tile_rows_of(int t) { return t >> TILE_EXPERT_BITS; }
 // Rows of each of an expert's tiles but the last.  Tiles of 256 rows that may stop early (moe_big_kernel) share up to 768 rows evenly, in whole
-// steps of 32 (what a column tile of each of a tile's two waves of rows holds), so that no compute unit gets a full one and another little; other
-// tiles are filled one after the other.
+// steps of 32 (what a column tile of each of a tile's two waves of rows holds), so that no compute unit gets a full one and another little.  Filled one
+// after the other, two tiles multiply up to 33 % more (257 rows: 384 and 288), three up to 18 % (513: 640 and 544), four would up to 12, five 9: not
+// measured there.  Other tiles are filled one after the other.
 __device__ __forceinline__ int rows_per_tile(int rows, int tile) {
     const int tiles = (rows + tile - 1) / tile;
     return tile == 256 && tiles >= 1 && tiles <= 3 ? ((rows + tiles - 1) / tiles + 31) / 32 * 32 : tile;
@@ -304,8 +305,8 @@ struct MoeSizes {
 // for 64 to 256 rows) for an expert with somewhat more rows than the mean, a second tile for a few experts costing
 // almost a whole round.  Tiles that do not fill the chip run side by side, so few or small experts take low ones: 16 experts of 256 x
 // 512 with 250 rows each 51 us in tiles of 192 rows, 30 in tiles of 64.  Measured with a full chip, us, 32 experts of 2,048 x 4,096, tiles of
-// 64 / 128 / 192 / 256 rows: mean 25: 210 / 222 / 242 / 271, 75: 291 / 230 / 247 / 268, 106: 345 / 294 / 251 / 279, 150: 390 / 314 / 257 / 281,
-// 181: 439 / 323 / 345 / 288, 256: 571 / 438 / 388 / 450, 375: 752 / 549 / 519 / 472, 625: 1,125 / 794 / 724 / 709 (tiles of 256 before they could stop early).  At 49 sizes (8 to 128 experts of 256
+// 64 / 128 / 192 / 256 rows (before tiles of 256 could stop early): mean 25: 210 / 222 / 242 / 271, 75: 291 / 230 / 247 / 268, 106: 345 / 294 / 251 / 279, 150: 390 / 314 / 257 / 281,
+// 181: 439 / 323 / 345 / 288, 256: 571 / 438 / 388 / 450, 375: 752 / 549 / 519 / 472, 625: 1,125 / 794 / 724 / 709.  At 49 sizes (also before; 8 to 128 experts of 256
 // to 2,048 x 512 to 4,096, means of 8 to 2,000 rows) it takes the best tile at 40 and is 1.0 % behind it in the mean, 10 % at worst (1,000 rows for each of
 // 16 small experts); with the times that a fit over those sizes gives (0.65, 0.77, 1.04, 1.46) it chooses otherwise at three of them, no better.
 static int big_tile_of(const MoeSizes& s) {

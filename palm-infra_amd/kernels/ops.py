@@ -647,7 +647,10 @@ def ring_pays(M: int, N: int, K: int, gated: bool = False, planes_ok: bool = Fal
     """Whether it is also the faster way, against the kernel with both operands in LDS (linear_mid.hip; us, 17, 32 and 48 rows):
     gate/up of 24,576 x 4,096 gated 36.0 35.6 35.8 and 34.6 35.6 37.6, of 34,816 x 5,120 (up to 32 rows) 81 84 and 58 60, q/k/v of 6,144 x 4,096 13.2 13.7 14.3
     and 11.3 11.6 12.7, down of 4,096 x 12,288 20.3 20.9 21.9 and 19.7 20.4 20.2, the head 203 217 227 and 198 207 212.  Not where one round of
-    whole strips is all there is (4,096 x 4,096: 8.7 9.1 9.6 and 9.1 10.0 11.6): there every block reads all rows for one strip."""
+    whole strips is all there is (4,096 x 4,096: 8.7 9.1 9.6 and 9.1 10.0 11.6): there every block reads all rows for one strip.
+
+    Weights of 3 GB in turn, marked as read once (``passes_once``); with them the gated product of 48 rows is 5 % behind the other kernel, which
+    this rule does not look at: it is taken here all the same."""
     if K < 2 * RING_STEP_K or not ring_serves(M, N, K, gated, planes_ok):       # (K of one step: not measured)
         return False
     return gated or ring_parts(M, N, K, False, planes_ok) > 1 or (N + 15) // 16 > 1.25 * COMPUTE_UNITS
@@ -910,7 +913,8 @@ def decode_fused_serves(qkv: torch.Tensor, hd: int, out_dtype, rotary_dim: int, 
     size and a rotation for which a rotation pair lies in one lane, and not too many sequences: every wave of a
     sequence's slices makes the queries anew, which for many sequences costs more than the pass of its own that it
     saves (a step of Qwen3-8B's sizes, fused against apart: 64 sequences 7.80 and 7.93 ms, 96: 10.15 and 10.11,
-    128: 12.23 and 11.87)."""
+    128: 12.23 and 11.87; by slices: the kernel cut by pages makes them once, but is reached from here, and steps of 97 to 128 sequences
+    by it have not been measured)."""
     if out_dtype != BF16 or hd not in MFMA_HEAD_DIMS or qkv.shape[-2] > DECODE_FUSED_ROWS:
         return False
     if not (qkv.dim() == 3 and qkv.dtype == F32 or qkv.dim() == 2 and qkv.dtype == BF16):
