@@ -320,10 +320,14 @@ static int big_tile_of(const MoeSizes& s) {
         const double cost = (rounds(s.ff, s.gated ? BIG_FEAT / 2 : BIG_FEAT) * s.width + rounds(s.width, BIG_FEAT) * s.ff) * stage_us[nt - 1];
         if (cost < best_cost) { best_cost = cost; best = 64 * nt; }
     }
-    // Experts of many rows: tiles of 256 multiply no more than their rows need either, and read the weights less often.  Us, tiles of 192 and of
-    // 256 rows, 32 experts of 2,048 x 4,096: mean 256 386 and 398, 325 397 and 392, 512 599 and 586, 750 851 and 803, 1,000 1,093 and 1,003; 32 capped ones of
-    // 1,536 x 4,096, mean 512 718 and 670; 16 gated ones of 1,408 x 2,048, mean 500 195 and 187.
-    if (best == 192 && mean >= 448) best = 256;
+    // Experts of many rows: tiles of 256 multiply no more than their rows need either, and read the weights less often.  But each takes longer, so only
+    // where both products have enough that the compute units' last ones matter little: two rounds of them.  Us, tiles of 192 and of 256 rows: 32 experts of
+    // 2,048 x 4,096, mean 500 611 and 596, 850 955 and 895, 1,000 1,115 and 1,028; 16 of them, mean 500 333 and 361, 700 382 and 395; 4, mean 500 117 and 137; 32
+    // gated ones of 1,408 x 2,048, mean 600 434 and 373; 8, mean 700 125 and 143; 64 of 512 x 1,024, mean 500 166 and 182.  Over 364 sizes (4 to 128 experts, means of
+    // 450 to 1,800) at which the stages' time alone chooses 192: 0.5 % behind the better tile in the geometric mean (256 at all of them 5.0, 192 1.2), and 256
+    // taken where it is 3 % slower or more at 7 of them, 6 % at worst (at all of them: 194, 18 %).
+    auto tiles_of_256 = [&](int features, int of_tile) { return in_use * ceil(mean / 256) * ((features + of_tile - 1) / of_tile); };
+    if (best == 192 && mean >= 448 && fmin(tiles_of_256(s.ff, s.gated ? BIG_FEAT / 2 : BIG_FEAT), tiles_of_256(s.width, BIG_FEAT)) >= 512) best = 256;
     return best;
 }
 // Whether the tiles cross LDS: rows in whole stages that start on 16 bytes, offsets from a matrix's first row of 32 bits, and, for

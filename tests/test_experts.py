@@ -87,6 +87,14 @@ def test_grouped_tiles(form, E, top, W, F, n, uneven):
     assert float((ops.moe_grouped(odd, *args[1:], F, form).cpu().double() - want).abs().max()) <= tol
 
 
+@pytest.mark.parametrize("E,mean,W,F,gated,tile", [
+    (4, 500, 4096, 2048, 0, 192), (8, 700, 2048, 1408, 1, 192), (16, 1000, 2048, 1024, 0, 192), (16, 700, 4096, 2048, 0, 192), (64, 500, 1024, 512, 0, 192),
+    (16, 700, 2048, 1408, 1, 192), (32, 500, 4096, 2048, 0, 256), (32, 1000, 4096, 2048, 0, 256), (32, 600, 2048, 1408, 1, 256), (64, 1000, 2048, 768, 1, 256)])
+def test_experts_of_many_rows_take_high_tiles_only_where_those_fill_the_chip(E, mean, W, F, gated, tile):
+    from palm_infra_amd.kernels import ops
+    assert ops.feedforward().palm_moe_tile_tokens(E * mean, E, W, F, gated, 1) == tile
+
+
 @gpu
 @pytest.mark.parametrize("form,E,top,W,F,n,uneven,tile", [
     ("gated_silu", 64, 2, 320, 1088, 640, True, 64), ("gated_silu", 64, 2, 1088, 320, 1920, True, 128), ("gated_silu", 64, 2, 320, 1088, 3520, False, 192),
@@ -112,14 +120,15 @@ def test_grouped_tiles_of_every_height_one_after_the_other(form, E, top, W, F, n
 
 
 @gpu
-@pytest.mark.parametrize("form,E,W,F,rows", [("gated_silu", 40, 256, 320, (1, 31, 32, 33, 64, 127, 128, 129, 160, 161, 192, 193, 224, 225, 255, 256)),
-                                             ("relu_squared", 40, 256, 320, (257, 320, 321, 384, 385, 512, 513, 576, 577, 700, 768, 769, 0, 900, 1024, 1025))])
+@pytest.mark.parametrize("form,E,W,F,rows", [("gated_silu", 320, 256, 320, (1, 31, 32, 33, 64, 127, 128, 129, 160, 161, 192, 193, 224, 225, 255, 256)),
+                                             ("relu_squared", 320, 256, 320, (257, 320, 321, 384, 385, 512, 513, 576, 577, 700, 768, 769, 0, 900, 1024, 1025))])
 def test_grouped_tiles_that_stop_early(form, E, W, F, rows):
-    """Experts of as many rows as fill one to five tiles of 256 and a little more or less, one choice a row, the experts after those chosen by 700 or 400 each."""
+    """Experts of as many rows as fill one to five tiles of 256 and a little more or less, one choice a row, the experts after those chosen by 700 or 500 each, so
+    many that tiles of 256 rows are taken."""
     from palm_infra_amd.kernels import ops
     per = ops.expert_rows(form) * F
     g = torch.Generator().manual_seed(E + W)
-    counts = list(rows) + [700 if form == "gated_silu" else 400] * (E - len(rows))
+    counts = list(rows) + [700 if form == "gated_silu" else 500] * (E - len(rows))
     chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)]).to(torch.int32)
     chosen = chosen[torch.randperm(len(chosen), generator=g)][:, None]
     n = len(chosen)
